@@ -633,6 +633,31 @@ def test_one_row_filter_gradient_from_the_forward_pass_rows(shape, dtype):
     assert torch.equal(dw2, dw0) and torch.equal(db2, db0)
 
 
+@pytest.mark.parametrize("shape", [((3, 40, 1, 96), (64, 40, 1, 6), 1, 3),         # output rows of 97 positions: a last step of 1
+                                   ((2, 250, 1, 111), (250, 250, 1, 21), 1, 10),   # the speech window, filter and channel tails
+                                   ((3, 33, 2, 181), (150, 33, 1, 11), 2, 5),      # two rows per image, stride 2
+                                   ((1, 32, 1, 23), (32, 32, 1, 23), 1, 11),       # one row, shorter than a range
+                                   ((2, 96, 1, 998), (40, 96, 1, 16), 1, 8)])      # several ranges per row
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_one_row_filter_gradient_over_odd_rows(shape, dtype, shift):
+    """16-bit output gradients whose rows have an odd length (every other row starts on a 2-byte boundary), and, with
+    shift, whose first element does too.  Inputs exact in the storage type, fp32 sums: only their order differs."""
+    xs, ws_, stride, pad = shape
+    rng = np.random.default_rng(93)
+    d = flref.conv_desc(xs, ws_, (1, stride), (0, pad), (1, 1), 1)
+    x = round_to(rng.standard_normal(xs).astype(np.float32), dtype)
+    ys = (xs[0], ws_[0], xs[2], (xs[3] + 2 * pad - ws_[3]) // stride + 1)
+    assert ys[3] % 2 == 1
+    dy = round_to(rng.standard_normal(ys).astype(np.float32), dtype)
+    dw_ref, db_ref = flref.conv2d_bwd_filter(d, x, dy)
+    room = torch.empty(dy.size + 2, dtype=dtype, device="cuda")
+    dyd = room[shift:shift + dy.size].view(ys)
+    dyd.copy_(dev(dy, dtype))
+    dw, db = fa.conv2d_backward_filter_bias(dyd, dev(x, dtype), ws_, True, sx=stride, px=pad)
+    assert rel_l2(host(dw), dw_ref) <= 1e-5 and rel_l2(host(db), db_ref) <= 1e-5
+
+
 def _random_cases(n, seed):
     """Seeded random geometries biased towards the conditions the kernel families key on:
     1x1 and 3x3 windows, even / odd rows, planes of 4k positions, channel counts around the
