@@ -19,6 +19,7 @@
 
 #include "common.h"
 #include "conv2d.h"
+#include "conv2d_mfma.h"
 
 extern "C" int flhip_matmul(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
                             int trans_a, int trans_b, const float* bias_rows, int dtype, void* stream);
@@ -38,7 +39,10 @@ struct RnnGeom {
   uint32_t seed_lo, seed_hi;
 };
 
-inline int gates_of(int mode) { return mode == RNN_LSTM ? 4 : mode == RNN_GRU ? 3 : 1; }
+constexpr int gates_of(int mode) { return mode == RNN_LSTM ? 4 : mode == RNN_GRU ? 3 : 1; }
+
+// widest layer input, in whole 16-byte pieces so that what follows in the workspace stays aligned
+inline size_t widest_input(const RnnGeom& g) { return (std::max<size_t>(g.I, (size_t)g.D * g.H) + 3) & ~(size_t)3; }
 
 int make_geom(const flhip_rnn_desc* d, RnnGeom* g) {
   FLHIP_REQUIRE(d, "rnn: null descriptor");
@@ -156,7 +160,7 @@ int mm_sliced(const float* A, const float* B, float* C, size_t M, size_t N, size
 
 // ... and at the end the partial products of the sliced weight-gradient products
 size_t wgrad_scratch(const RnnGeom& g) {
-  const size_t TB = (size_t)g.T * g.B, inmax = std::max<size_t>(g.I, (size_t)g.D * g.H);
+  const size_t TB = (size_t)g.T * g.B, inmax = widest_input(g);
   size_t n = 0;
   for (size_t M : {(size_t)g.I, inmax, (size_t)g.H}) {
     const int ns = wgrad_slices(M, g.GH, TB);
@@ -166,7 +170,7 @@ size_t wgrad_scratch(const RnnGeom& g) {
 }
 
 size_t wgrad_scratch_offset(const RnnGeom& g) {
-  const size_t TB = (size_t)g.T * g.B, inmax = std::max<size_t>(g.I, (size_t)g.D * g.H);
+  const size_t TB = (size_t)g.T * g.B, inmax = widest_input(g);
   int k;
   const size_t sb = step_slices(g.H, g.B, g.GH, &k);
   return 2 * TB * g.GH + TB * g.D * g.H + 2 * TB * inmax + (3 + sb) * g.BH +
@@ -187,7 +191,10 @@ bool fused_applies(const RnnGeom& g) {
   return !options().rnn_unfused && g.H % 16 == 0 && g.B <= 64;
 }
 
-__device__ __forceinline__ float sigm(float v) { return 1.f / (1.f + expf(-v)); }
+__device__ __forceinline__ float sigm(float v) {
+#pragma clang fp contract(off)
+  return 1.f / (1.f + expf(-v));
+}
 
 // bsum[q] = bW[q] + bR[q], except the GRU n gate, whose recurrent bias stays inside
 // r * (R_n h + b_Rn)
@@ -247,6 +254,8 @@ struct CellFwd {
   int ldo;
 };
 
+// (The gate math below leaves no choice of fused or separate multiply-adds to the compiler: the step kernels of a captured
+// sequence and the sequence kernels give the same bits.)
 // gate math of one (batch b, hidden h) element, in two halves so that a kernel can issue
 // the loads before it computes the recurrent projections rp (one per gate)
 template <int MODE>
@@ -268,35 +277,52 @@ __device__ __forceinline__ CellFwdIn<MODE> cell_fwd_load(const CellFwd& a, int b
   return in;
 }
 
-template <int MODE>
-__device__ __forceinline__ void cell_fwd_finish(const CellFwd& a, int b, int h, int H, const CellFwdIn<MODE>& in,
-                                                const float* rp) {
+// Values that another workgroup of the same launch waits for (the sequence kernels below): every element starts as
+// RNN_UNSET, a NaN that no element is stored as, and is written once, past the caches that the readers do not share.
+constexpr uint32_t RNN_UNSET = 0xffffffffu;
+__device__ __forceinline__ float rnn_value(float v) { return __float_as_uint(v) == RNN_UNSET ? __uint_as_float(0x7fc00000u) : v; }
+__device__ __forceinline__ void rnn_publish(float* p, float v) {
+  __hip_atomic_store(p, rnn_value(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// SEQ: the state goes to the other workgroups of the launch; returns what the element's thread keeps for the next step
+// (LSTM: c, else h)
+template <int MODE, bool SEQ = false>
+__device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h, int H, const CellFwdIn<MODE>& in,
+                                                 const float* rp) {
+#pragma clang fp contract(off)
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
   const size_t e = (size_t)b * H + h, q = (size_t)b * G * H + h;
-  float hv;
+  float hv, keep = 0.f;
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float pre = in.xp[0] + rp[0];
     hv = MODE == RNN_RELU ? (pre > 0.f ? pre : 0.f) : tanhf(pre);
+    if (SEQ) rnn_publish(a.hn + e, hv);
     a.gt[q] = hv;
   } else if (MODE == RNN_LSTM) {
     const float ig = sigm(in.xp[0] + rp[0]), fg = sigm(in.xp[G > 1 ? 1 : 0] + rp[G > 1 ? 1 : 0]);
     const float gg = tanhf(in.xp[G > 2 ? 2 : 0] + rp[G > 2 ? 2 : 0]), og = sigm(in.xp[G > 3 ? 3 : 0] + rp[G > 3 ? 3 : 0]);
-    const float c = fg * in.prev + ig * gg;
+    const float c = fmaf(fg, in.prev, ig * gg);
+    keep = c;
+    hv = og * tanhf(c);
+    if (SEQ) rnn_publish(a.hn + e, hv);
     a.cn[e] = c;
     if (a.cy) a.cy[e] = c;
-    hv = og * tanhf(c);
     a.gt[q] = ig; a.gt[q + H] = fg; a.gt[q + 2 * H] = gg; a.gt[q + 3 * H] = og;
   } else {
     const float rg = sigm(in.xp[0] + rp[0]), zg = sigm(in.xp[G > 1 ? 1 : 0] + rp[G > 1 ? 1 : 0]);
     const float rn = rp[G > 2 ? 2 : 0] + in.bRn;
-    const float ng = tanhf(in.xp[G > 2 ? 2 : 0] + rg * rn);
+    const float ng = tanhf(fmaf(rg, rn, in.xp[G > 2 ? 2 : 0]));
+    hv = fmaf(1.f - zg, ng, zg * in.prev);
+    keep = hv;
+    if (SEQ) rnn_publish(a.hn + e, hv);
     a.rn[e] = rn;
-    hv = (1.f - zg) * ng + zg * in.prev;
     a.gt[q] = rg; a.gt[q + H] = zg; a.gt[q + 2 * H] = ng;
   }
-  a.hn[e] = hv;
+  if (!SEQ) a.hn[e] = hv;
   a.out[(size_t)b * a.ldo + h] = hv;
   if (a.hy) a.hy[e] = hv;
+  return keep;
 }
 
 template <int MODE>
@@ -321,8 +347,9 @@ __global__ void __launch_bounds__(256) rnn_cell_fwd(CellFwd a, int B, int H) {
 // One time step of up to two directions in one launch: recurrent product and gate math.
 // A workgroup owns four hidden units (blockIdx.x) of one direction (blockIdx.y): its
 // 16-row matrix-core tile is {gate g, unit hh} = row 4*g + hh of the recurrent
-// matrices, its columns are the batch (NBT tiles of 16, batch <= 64), and the four
-// waves split the contraction over the hidden state in interleaved chunks of 16.  A
+// matrices, its columns are the batch (NBT tiles of 16, batch <= 64), and the eight
+// waves split the contraction over the hidden state in interleaved chunks of 16 (as the sequence
+// kernels do: a captured launch sequence and an eager one add in the same order).  A
 // lane's 16-byte load supplies the operands of four 16x16x4 products (the k index of a
 // lane group is permuted the same way on both operands).  The partial tiles meet in
 // LDS, then one thread per (batch, unit) applies the gates; those threads issue the
@@ -332,11 +359,11 @@ struct StepFwd {
   CellFwd d[2];
   int B, H;
 };
-constexpr int STEP_FWD_WAVES = 4;
+constexpr int STEP_WAVES = 8;
 
 template <int MODE, int NBT>
-__global__ void __launch_bounds__(64 * STEP_FWD_WAVES) rnn_step_fwd(StepFwd p) {
-  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16, W = STEP_FWD_WAVES;
+__global__ void __launch_bounds__(64 * STEP_WAVES) rnn_step_fwd(StepFwd p) {
+  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16, W = STEP_WAVES;
   __shared__ float red[W][16][NB + 1];
   const CellFwd& a = p.d[blockIdx.y];
   const int H = p.H, B = p.B, h0 = blockIdx.x * 4;
@@ -428,6 +455,7 @@ struct CellBwd {
   float* dgw;         // [B][GH] pre-activation gradients seen by the input side
   float* dgr;         // [B][GH] ... by the recurrent side
   float* dh_dir;      // [B][H] direct gradient towards the previous state (GRU: go * z, else 0)
+  float* dhx;         // fused path: only the gradient of the initial state, no step (else null)
   int ldo;
 };
 
@@ -459,36 +487,45 @@ __device__ __forceinline__ CellBwdIn<MODE> cell_bwd_load(const CellBwd& a, int b
   return in;
 }
 
-template <int MODE>
+// SEQ: the recurrent-side gradients go to the other workgroups of the launch, and what the element's thread hands to its
+// next step stays in *dc and *dir
+template <int MODE, bool SEQ = false>
 __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, int H, const CellBwdIn<MODE>& in,
-                                                float rec) {
+                                                float rec, float* dc_out = nullptr, float* dir_out = nullptr) {
+#pragma clang fp contract(off)
+  auto put = [&](size_t i, float v) {
+    if (SEQ) rnn_publish(a.dgr + i, v);
+    else a.dgr[i] = v;
+  };
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
   const size_t e = (size_t)b * H + h, q = (size_t)b * G * H + h;
   const float go = in.go + rec;
   float direct = 0.f;
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float hv = in.gt[0];
-    const float gp = MODE == RNN_RELU ? (hv > 0.f ? go : 0.f) : go * (1.f - hv * hv);
+    const float gp = MODE == RNN_RELU ? (hv > 0.f ? go : 0.f) : go * fmaf(-hv, hv, 1.f);
+    put(q, gp);
     a.dgw[q] = gp;
-    a.dgr[q] = gp;
   } else if (MODE == RNN_LSTM) {
     const float ig = in.gt[0], fg = in.gt[G > 1 ? 1 : 0], gg = in.gt[G > 2 ? 2 : 0], og = in.gt[G > 3 ? 3 : 0];
     const float tc = tanhf(in.cn);
-    const float dc = in.dc + go * og * (1.f - tc * tc);
+    const float dc = fmaf(go * og, fmaf(-tc, tc, 1.f), in.dc);
     const float v0 = dc * gg * ig * (1.f - ig), v1 = dc * in.cp * fg * (1.f - fg);
-    const float v2 = dc * ig * (1.f - gg * gg), v3 = go * tc * og * (1.f - og);
+    const float v2 = dc * ig * fmaf(-gg, gg, 1.f), v3 = go * tc * og * (1.f - og);
+    put(q, v0); put(q + H, v1); put(q + 2 * H, v2); put(q + 3 * H, v3);
     a.dgw[q] = v0; a.dgw[q + H] = v1; a.dgw[q + 2 * H] = v2; a.dgw[q + 3 * H] = v3;
-    a.dgr[q] = v0; a.dgr[q + H] = v1; a.dgr[q + 2 * H] = v2; a.dgr[q + 3 * H] = v3;
-    a.dc[e] = dc * fg;
+    if (SEQ) *dc_out = dc * fg;
+    else a.dc[e] = dc * fg;
   } else {
     const float rg = in.gt[0], zg = in.gt[G > 1 ? 1 : 0], ng = in.gt[G > 2 ? 2 : 0], rn = in.rn;
-    const float dn = go * (1.f - zg) * (1.f - ng * ng);
+    const float dn = go * (1.f - zg) * fmaf(-ng, ng, 1.f);
     const float v0 = dn * rn * rg * (1.f - rg), v1 = go * (in.hp - ng) * zg * (1.f - zg);
+    put(q, v0); put(q + H, v1); put(q + 2 * H, dn * rg);
     a.dgw[q] = v0; a.dgw[q + H] = v1; a.dgw[q + 2 * H] = dn;
-    a.dgr[q] = v0; a.dgr[q + H] = v1; a.dgr[q + 2 * H] = dn * rg;
     direct = go * zg;
   }
-  a.dh_dir[e] = direct;
+  if (SEQ) *dir_out = direct;
+  else a.dh_dir[e] = direct;
 }
 
 template <int MODE>
@@ -506,21 +543,23 @@ __global__ void __launch_bounds__(256) rnn_cell_bwd(CellBwd a, int B, int H) {
 // One backward time step of up to two directions in one launch.  A workgroup owns 16
 // hidden units of one direction: rows of its matrix-core tile are the units (columns
 // of the recurrent matrices, 64 contiguous bytes per contraction index), columns the
-// batch.  Its sixteen waves split the contraction over the gate rows (G*H) in
+// batch.  Its eight waves split the contraction over the gate rows (G*H) in
 // interleaved chunks of 16 (with four batch tiles: eight groups of two waves, each wave
 // two of the tiles); the partial tiles meet in LDS and one thread per (unit, batch)
 // applies the gate gradients of the step, which become the next launch's operand.
 // Those threads issue their loads before the product.  H % 16 == 0.
+// A last launch with no step of its own (dhx) adds up the gradient of the initial state.
 struct StepBwd {
   CellBwd d[2];
   int B, H;
 };
+constexpr int step_bwd_waves(int nbt) { return nbt == 4 ? 2 * STEP_WAVES : STEP_WAVES; }
 
 template <int MODE, int NBT>
-__global__ void __launch_bounds__(1024) rnn_step_bwd(StepBwd p) {
+__global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16;
   constexpr int NW = NBT == 4 ? 2 : NBT;      // batch tiles per wave
-  constexpr int KG = 16 / (NBT / NW);         // wave groups along the contraction
+  constexpr int KG = STEP_WAVES;              // wave groups along the contraction
   __shared__ float red[KG][16][NB + 1];
   const CellBwd& a = p.d[blockIdx.y];
   const int H = p.H, B = p.B, h0 = blockIdx.x * 16, GH = G * H;
@@ -528,7 +567,7 @@ __global__ void __launch_bounds__(1024) rnn_step_bwd(StepBwd p) {
   const bool cell = tid < 16 * B;
   const int cb = tid >> 4, ch = h0 + (tid & 15);
   CellBwdIn<MODE> cin{};
-  if (cell) cin = cell_bwd_load<MODE>(a, cb, ch, H);
+  if (cell && !a.dhx) cin = cell_bwd_load<MODE>(a, cb, ch, H);
   const bool have = a.dgr_next != nullptr;
   if (have) {
     const int kg = wave % KG, nt0 = (wave / KG) * NW;
@@ -590,8 +629,290 @@ __global__ void __launch_bounds__(1024) rnn_step_bwd(StepBwd p) {
 #pragma unroll
       for (int k = 0; k < KG; ++k) rec += red[k][tid & 15][cb];
     }
-    cell_bwd_finish<MODE>(a, cb, ch, H, cin, rec);
+    if (a.dhx) a.dhx[(size_t)cb * H + ch] = a.dh_a[(size_t)cb * H + ch] + rec;
+    else cell_bwd_finish<MODE>(a, cb, ch, H, cin, rec);
   }
+}
+
+// ---- a layer's whole recurrence in one launch -----------------------------------------------------------------------
+// The steps of a sequence depend on each other, so a launch per step costs a launch's latency and one trip of the
+// recurrent matrices from the caches per step (LSTM of 512 units, two directions, 32 columns: 8.2 us forward, 12.4 us
+// backward per step, where the products need 0.9 and 1.7).  Here the workgroups stay: each keeps its part of the
+// recurrent matrices in registers for all steps, and only the state (forward) or the pre-activation gradients (backward)
+// of a step travel between workgroups.  Batch columns do not depend on each other: a cluster of workgroups is one
+// direction of 16 columns, and clusters never wait for one another.
+//
+// The exchange needs no flags and no barrier over the grid: the step's rows in the reserve buffer / workspace (which the
+// later products read anyway) are filled with RNN_UNSET before the launch, the owner of an element stores it once with
+// agent scope, and a reader repeats its 16-byte loads (agent scope as well: they pass by the caches that the eight dies
+// do not share) until none of its elements is unset.  Measured alone, 64 workgroups exchanging 32 / 128 KB per step:
+// 1.9 / 3.4 us, of which a load's trip is about 1.
+//
+// All workgroups of the launch have to be resident at once: the launch is cooperative, and a launch covers as many
+// clusters as the compute units hold, the rest follow in further launches.  A wait that does not end (it would take a
+// device that lost workgroups) stops after RNN_SPINS loads; the wave then goes on with NaN, which reaches every output.
+constexpr int SEQ_WAVES = STEP_WAVES, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
+constexpr int RNN_SPINS = 1 << 22;
+constexpr int RNN_OOB = (int)0x80000000;
+constexpr int AUX_AGENT = 16 | (int)0x80000000;      // buffer loads: sc1 (agent scope), and volatile: loaded every time
+
+struct SeqFwd {
+  struct Dir {
+    const float *xp, *R, *bRn;
+    float *HP, *CP, *GT, *RN, *out, *hy, *cy;
+  } d[2];
+  int B, H, T, ldo;
+  int groups;        // of 16 batch columns
+  int nwg;           // workgroups of a cluster
+  int cluster0;      // first cluster of this launch; cluster = direction * groups + group
+};
+
+// N 16-byte loads per lane at off[i], repeated until every element is set.  (A lane's loads that do not exist are out of
+// the buffer's range and read zero.)
+template <int N>
+__device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N]) {
+  asm volatile("" ::: "memory");       // memory may have changed since the last load
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, AUX_AGENT);
+}
+template <int N>
+__device__ __forceinline__ void seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], bool* dead) {
+  for (int spin = 0;; ++spin) {
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      ok = ok && v[i].x != RNN_UNSET && v[i].y != RNN_UNSET && v[i].z != RNN_UNSET && v[i].w != RNN_UNSET;
+    if (__all(ok) || *dead) return;
+    if (spin >= RNN_SPINS) {
+      *dead = true;
+      return;
+    }
+    seq_load(r, off, v);
+  }
+}
+
+// A workgroup owns HU hidden units of its cluster: row gate * HU + unit of its RT tiles of 16 rows.  The eight waves split
+// the contraction over the state in interleaved chunks of 16 (NC at most per wave, the recurrent matrices' fragments in
+// 4 RT NC registers); the partial tiles meet in LDS (two buffers in turn, so one barrier per step) and one thread per
+// (column, unit) applies the gates.  HU is the smallest for which a layer's clusters fit the compute units.
+template <int MODE, int HU, int NC>
+__global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
+  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, RT = (G * HU + 15) / 16, W = SEQ_WAVES;
+  extern __shared__ float seq_red[];      // [2][W][16 RT][17]
+  const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * HU;
+  const int dir = cluster / p.groups, b0 = (cluster - dir * p.groups) * SEQ_COLS;
+  const SeqFwd::Dir& q = p.d[dir];
+  const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  float a[RT][NC][4];
+  int off[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int k = (wave + W * i) * 16 + 4 * fg;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int row = rt * 16 + fr, gate = row / HU, h = h0 + row % HU;
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (gate < G && h < H && k < H) v = *reinterpret_cast<const float4*>(q.R + ((size_t)gate * H + h) * H + k);
+      a[rt][i][0] = v.x; a[rt][i][1] = v.y; a[rt][i][2] = v.z; a[rt][i][3] = v.w;
+    }
+    off[i] = (b0 + fr < B && k < H) ? ((b0 + fr) * H + k) * 4 : RNN_OOB;
+  }
+  const int unit = tid % HU, col = tid / HU, ch = h0 + unit, cb = b0 + col;
+  const bool cell = tid < HU * SEQ_COLS && cb < B && ch < H;
+  const size_t BH = (size_t)B * H, e = (size_t)cb * H + ch;
+  CellFwd c{};
+  c.bRn = q.bRn;
+  c.ldo = p.ldo;
+  float keep = 0.f;
+  if (cell) keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? q.HP[e] : 0.f;
+  bool dead = false;
+  for (int st = 0; st < T; ++st) {
+    const int t = dir ? T - 1 - st : st;
+    c.xp = q.xp + (size_t)t * B * GH;
+    CellFwdIn<MODE> in{};
+    if (cell) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) in.xp[g] = c.xp[(size_t)cb * GH + (size_t)g * H + ch];
+      in.bRn = MODE == RNN_GRU ? c.bRn[ch] : 0.f;
+      in.prev = keep;
+    }
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(q.HP + st * BH, (unsigned)(BH * 4));
+    uintx4_t v[NC];
+    seq_load(r, off, v);
+    seq_wait(r, off, v, &dead);
+    floatx4_t acc[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if ((wave + W * i) * 16 < H)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][i][m], __uint_as_float(v[i][m]), acc[rt], 0, 0, 0);
+    float* red = seq_red + (st & 1) * (W * RT * 16 * 17);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) red[(wave * RT * 16 + rt * 16 + 4 * fg + x) * 17 + fr] = acc[rt][x];
+    __syncthreads();
+    if (cell) {
+      float rp[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) sum += red[(w * RT * 16 + g * HU + unit) * 17 + col];
+        rp[g] = sum;
+      }
+      c.hn = q.HP + (st + 1) * BH;
+      c.cn = q.CP + (st + 1) * BH;
+      c.gt = q.GT + (size_t)st * B * GH;
+      c.rn = q.RN + st * BH;
+      c.out = q.out + (size_t)t * B * p.ldo;
+      c.hy = st == T - 1 ? q.hy : nullptr;
+      c.cy = st == T - 1 ? q.cy : nullptr;
+      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp);
+    }
+  }
+}
+
+struct SeqBwd {
+  struct Dir {
+    const float *gout, *dhy, *dcy, *R, *HP, *CP, *GT, *RN;
+    float *dGW, *dGR, *dhx, *dcx;
+  } d[2];
+  int B, H, T, ldo;
+  int groups, nwg, cluster0;
+};
+
+// The same for the backward pass: a workgroup owns 16 hidden units (rows of one tile: columns of the recurrent matrices,
+// 4 NC registers) and reads the gate gradients of all units of its cluster, U chunks in flight while U are multiplied.
+// After the last step the gradient of the initial state is one more product.
+template <int MODE, int NC>
+__global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
+  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, W = SEQ_WAVES, U = NC < 8 ? NC : 8, NB = NC / U;
+  __shared__ float red2[2][W][16][17];
+  const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * 16;
+  const int dir = cluster / p.groups, b0 = (cluster - dir * p.groups) * SEQ_COLS;
+  const SeqBwd::Dir& q = p.d[dir];
+  const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  float a[NC][4];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int k = (wave + W * i) * 16 + 4 * fg;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) a[i][m] = (h0 + fr < H && k < GH) ? q.R[(size_t)(k + m) * H + h0 + fr] : 0.f;
+  }
+  const int brow = b0 + fr < B ? (b0 + fr) * GH * 4 : RNN_OOB;
+  auto offsets_of = [&](int b, int (&off)[U]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (wave + W * (b * U + u)) * 16 + 4 * fg;
+      off[u] = k < GH ? brow + k * 4 : RNN_OOB;      // (brow out of range: so is the sum)
+    }
+  };
+  const int unit = tid & 15, col = tid >> 4, ch = h0 + unit, cb = b0 + col;
+  const bool cell = tid < 16 * SEQ_COLS && cb < B && ch < H;
+  const size_t BH = (size_t)B * H, e = (size_t)cb * H + ch;
+  CellBwd c{};
+  c.ldo = p.ldo;
+  float direct = cell && q.dhy ? q.dhy[e] : 0.f, dc = cell && MODE == RNN_LSTM && q.dcy ? q.dcy[e] : 0.f;
+  bool dead = false;
+  for (int st = T - 1; st >= (q.dhx ? -1 : 0); --st) {
+    const int t = dir ? T - 1 - st : st;
+    CellBwdIn<MODE> in{};
+    if (cell && st >= 0) {
+      const size_t qe = (size_t)cb * GH + ch;
+      in.go = q.gout ? q.gout[((size_t)t * B + cb) * p.ldo + ch] : 0.f;
+#pragma unroll
+      for (int g = 0; g < G; ++g) in.gt[g] = q.GT[(size_t)st * B * GH + qe + (size_t)g * H];
+      if (MODE == RNN_LSTM) {
+        in.cn = q.CP[(st + 1) * BH + e]; in.cp = q.CP[st * BH + e];
+      }
+      if (MODE == RNN_GRU) {
+        in.hp = q.HP[st * BH + e]; in.rn = q.RN[st * BH + e];
+      }
+    }
+    float (*red)[16][17] = red2[st & 1];
+    if (st < T - 1) {
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(q.dGR + (size_t)(st + 1) * B * GH, (unsigned)((size_t)B * GH * 4));
+      floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+      uintx4_t v[2][U];
+      {
+        int off[U];
+        offsets_of(0, off);
+        seq_load(r, off, v[0]);
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        int off[U];
+        if (b + 1 < NB) {
+          offsets_of(b + 1, off);
+          seq_load(r, off, v[(b + 1) & 1]);
+        }
+        offsets_of(b, off);
+        seq_wait(r, off, v[b & 1], &dead);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if ((wave + W * (b * U + u)) * 16 < GH)
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b * U + u][m], __uint_as_float(v[b & 1][u][m]), acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) red[wave][4 * fg + x][fr] = acc[x];
+      __syncthreads();
+    }
+    if (cell) {
+      float rec = 0.f;
+      if (st < T - 1) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) rec += red[w][unit][col];
+      }
+      if (st < 0) {
+        q.dhx[e] = direct + rec;
+      } else {
+        in.go += direct;
+        in.dc = dc;
+        c.dgw = q.dGW + (size_t)t * B * GH;
+        c.dgr = q.dGR + (size_t)st * B * GH;
+        cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct);
+      }
+    }
+  }
+  if (cell && MODE == RNN_LSTM && q.dcx) q.dcx[e] = dc;
+}
+
+// What a sequence launch finds in place: forward, per direction (blockIdx.y), the initial states, RNN_UNSET in the rows of
+// all steps' states, and the biases as rnn_bias_kernel makes them; backward, RNN_UNSET in all rows of dGR.
+struct SeqInit {
+  struct Dir {
+    const float *hx, *cx, *bW, *bR;
+    float *HP, *CP, *bsum;
+  } d[2];
+  size_t BH, n;       // elements of a state / of the rows to be filled
+  int GH, H, mode;
+};
+__global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
+  const SeqInit::Dir& q = p.d[blockIdx.y];
+  const size_t stride = (size_t)gridDim.x * 256, i0 = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const uintx4_t unset = {RNN_UNSET, RNN_UNSET, RNN_UNSET, RNN_UNSET};
+  for (size_t i = i0; i < p.n / 4; i += stride) reinterpret_cast<uintx4_t*>(q.HP + p.BH)[i] = unset;
+  if (p.BH == 0) return;                      // backward: nothing but the fill
+  for (size_t i = i0; i < p.BH; i += stride) {
+    q.HP[i] = q.hx ? rnn_value(q.hx[i]) : 0.f;
+    if (p.mode == RNN_LSTM) q.CP[i] = q.cx ? q.cx[i] : 0.f;
+  }
+  for (size_t i = i0; i < (size_t)p.GH; i += stride)
+    q.bsum[i] = (p.mode == RNN_GRU && i >= (size_t)2 * p.H) ? q.bW[i] : q.bW[i] + q.bR[i];
 }
 
 inline unsigned nblocks(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -655,18 +976,117 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
   return check_launch("rnn_fwd");
 }
 
-template <int MODE, int NBT>
-void launch_step_fwd(const StepFwd& p, int D, hipStream_t s) {
-  hipLaunchKernelGGL((rnn_step_fwd<MODE, NBT>), dim3(p.H / 4, D), dim3(64 * STEP_FWD_WAVES), 0, s, p);
+// ---- launching whole sequences: the hidden size a multiple of 4 (16-byte pieces of the state) and at most 1024
+// (registers), a stream that is not being captured (a cooperative launch is not recorded)
+bool seq_applies(const RnnGeom& g, hipStream_t s) {
+  if (options().rnn_unfused || g.H % 4 != 0 || g.H > 1024) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusNone;
 }
 
-// one layer, all directions: per direction the input projection of all steps, then one
-// launch per time step for both directions
+// FLHIP_DECLINED where the device does not hold the launch (nothing has run then)
+template <typename P>
+int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s) {
+  if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return FLHIP_DECLINED;
+  const int per = std::max(1, mfma_num_cus() / p.nwg);
+  for (p.cluster0 = 0; p.cluster0 < clusters; p.cluster0 += per) {
+    void* args[] = {&p};
+    const unsigned grid = (unsigned)(std::min(per, clusters - p.cluster0) * p.nwg);
+    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(grid), dim3(SEQ_THREADS), args,
+                                                    (unsigned)lds, s);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      if (p.cluster0 == 0 && e == hipErrorCooperativeLaunchTooLarge) return FLHIP_DECLINED;
+      return fail(FLHIP_RUNTIME_ERROR, std::string("rnn: ") + hipGetErrorString(e));
+    }
+  }
+  return FLHIP_OK;
+}
+
+template <int MODE, int HU>
+int seq_fwd_hu(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
+  constexpr int RT = (gates_of(MODE) * HU + 15) / 16;
+  p.nwg = (g.H + HU - 1) / HU;
+  const size_t lds = (size_t)2 * SEQ_WAVES * RT * 16 * 17 * sizeof(float);
+  const int nc = ((g.H + 15) / 16 + SEQ_WAVES - 1) / SEQ_WAVES;
+  if (nc <= 2) return seq_launch(rnn_seq_fwd<MODE, HU, 2>, p, g.D * p.groups, lds, s);
+  if (nc <= 4) return seq_launch(rnn_seq_fwd<MODE, HU, 4>, p, g.D * p.groups, lds, s);
+  return seq_launch(rnn_seq_fwd<MODE, HU, 8>, p, g.D * p.groups, lds, s);
+}
+template <int MODE>
+int seq_fwd(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
+  if constexpr (MODE == RNN_LSTM || MODE == RNN_GRU) {
+    const int cus = mfma_num_cus(), clusters = g.D * p.groups;
+    if (clusters * ((g.H + 3) / 4) <= cus) return seq_fwd_hu<MODE, 4>(g, p, s);
+    if (clusters * ((g.H + 7) / 8) <= cus) return seq_fwd_hu<MODE, 8>(g, p, s);
+  }
+  return seq_fwd_hu<MODE, 16>(g, p, s);
+}
+
+template <int MODE>
+int seq_bwd(const RnnGeom& g, SeqBwd& p, hipStream_t s) {
+  p.nwg = (g.H + 15) / 16;
+  const int nc = ((int)((g.GH + 15) / 16) + SEQ_WAVES - 1) / SEQ_WAVES, clusters = g.D * p.groups;
+  if (nc <= 4) return seq_launch(rnn_seq_bwd<MODE, 4>, p, clusters, 0, s);
+  if (nc <= 8) return seq_launch(rnn_seq_bwd<MODE, 8>, p, clusters, 0, s);
+  if constexpr (MODE == RNN_LSTM || MODE == RNN_GRU) {
+    if (nc <= 16) return seq_launch(rnn_seq_bwd<MODE, 16>, p, clusters, 0, s);
+    if (nc <= 24) return seq_launch(rnn_seq_bwd<MODE, 24>, p, clusters, 0, s);
+    if (MODE == RNN_LSTM && nc <= 32) return seq_launch(rnn_seq_bwd<MODE, MODE == RNN_LSTM ? 32 : 24>, p, clusters, 0, s);
+  }
+  return FLHIP_DECLINED;
+}
+
+template <int MODE, int NBT>
+void launch_step_fwd(const StepFwd& p, int D, hipStream_t s) {
+  hipLaunchKernelGGL((rnn_step_fwd<MODE, NBT>), dim3(p.H / 4, D), dim3(64 * STEP_WAVES), 0, s, p);
+}
+
+// one layer, all directions: per direction the input projection of all steps, then the recurrence: one launch for the whole
+// sequence (seq), or one per time step for both directions
 template <int MODE>
 int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, const float* w, const float* hx,
-                        const float* cx, float* out, float* hy, float* cy, float* res, float* ws, hipStream_t s) {
+                        const float* cx, float* out, float* hy, float* cy, float* res, float* ws, bool seq, hipStream_t s) {
   const Reserve r = reserve_layout(g);
   const size_t TB = (size_t)g.T * g.B;
+  if (seq) {
+    SeqInit ip{};
+    SeqFwd p{};
+    p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
+    p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+    ip.BH = g.BH; ip.n = (size_t)g.T * g.BH; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+    for (int dir = 0; dir < g.D; ++dir) {
+      const int pl = l * g.D + dir;
+      const Offsets o = offsets(g, pl);
+      float* base = res + (size_t)pl * r.per_pl;
+      SeqFwd::Dir& q = p.d[dir];
+      q.xp = ws + (size_t)dir * TB * g.GH;
+      q.R = w + o.R; q.bRn = w + o.bR + 2 * g.H;
+      q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
+      q.out = out + (size_t)dir * g.H;
+      q.hy = hy + (size_t)pl * g.BH;
+      q.cy = cy && MODE == RNN_LSTM ? cy + (size_t)pl * g.BH : nullptr;
+      SeqInit::Dir& i = ip.d[dir];
+      i.hx = hx ? hx + (size_t)pl * g.BH : nullptr;
+      i.cx = cx ? cx + (size_t)pl * g.BH : nullptr;
+      i.bW = w + o.bW; i.bR = w + o.bR;
+      i.HP = q.HP; i.CP = q.CP;
+      i.bsum = ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH;
+    }
+    const unsigned blocks = (unsigned)std::min<size_t>((ip.n / 4 + 255) / 256, 2048);
+    hipLaunchKernelGGL(rnn_seq_init_kernel, dim3(std::max(1u, blocks), g.D), dim3(256), 0, s, ip);
+    for (int dir = 0; dir < g.D; ++dir)
+      if (const int rc = mm(w + offsets(g, l * g.D + dir).W, in, const_cast<float*>(p.d[dir].xp), g.GH, TB, inl, 1, 0,
+                            ip.d[dir].bsum, s))
+        return rc;
+    const int rc = seq_fwd<MODE>(g, p, s);
+    if (rc != FLHIP_DECLINED) return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
+    if (!fused_applies(g)) return FLHIP_DECLINED;
+  }
   for (int dir = 0; dir < g.D; ++dir) {
     const int pl = l * g.D + dir;
     const Offsets o = offsets(g, pl);
@@ -719,7 +1139,7 @@ int backward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const flo
   const Reserve r = reserve_layout(g);
   const Offsets o = offsets(g, pl);
   const int dir = pl % g.D;
-  const size_t TB = (size_t)g.T * g.B, inmax = std::max<size_t>(g.I, (size_t)g.D * g.H);
+  const size_t TB = (size_t)g.T * g.B, inmax = widest_input(g);
   const float* HP = res + (size_t)pl * r.per_pl + r.hp;
   const float* CP = res + (size_t)pl * r.per_pl + r.cp;
   const float* GT = res + (size_t)pl * r.per_pl + r.gt;
@@ -781,15 +1201,15 @@ int backward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const flo
 
 template <int MODE, int NBT>
 void launch_step_bwd(const StepBwd& p, int D, hipStream_t s) {
-  hipLaunchKernelGGL((rnn_step_bwd<MODE, NBT>), dim3(p.H / 16, D), dim3(1024), 0, s, p);
+  hipLaunchKernelGGL((rnn_step_bwd<MODE, NBT>), dim3(p.H / 16, D), dim3(64 * step_bwd_waves(NBT)), 0, s, p);
 }
 
 template <int MODE>
 int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, const float* w, const float* gout,
                          const float* dhy, const float* dcy, float* gin, float* dhx, float* dcx, float* dw,
-                         const float* res, float* ws, hipStream_t s) {
+                         const float* res, float* ws, bool seq, hipStream_t s) {
   const Reserve r = reserve_layout(g);
-  const size_t TB = (size_t)g.T * g.B, inmax = std::max<size_t>(g.I, (size_t)g.D * g.H);
+  const size_t TB = (size_t)g.T * g.B, inmax = widest_input(g);
   int kdummy;
   const size_t sb = step_slices(g.H, g.B, g.GH, &kdummy);
   float* tmp = ws + 2 * TB * g.GH + TB * g.D * g.H + TB * inmax;
@@ -798,10 +1218,42 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
   float *dGW[2], *dGR[2], *dh_dir[2], *dc[2];
   dGW[0] = ws; dGR[0] = ws + TB * g.GH; dh_dir[0] = tmp + TB * inmax; dc[0] = dh_dir[0] + 2 * g.BH;
   dGW[1] = second; dGR[1] = second + TB * g.GH; dh_dir[1] = second + 2 * TB * g.GH; dc[1] = dh_dir[1] + 2 * g.BH;
+  if (seq) {
+    SeqInit ip{};
+    SeqBwd p{};
+    p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
+    p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+    ip.n = TB * g.GH;
+    for (int dir = 0; dir < g.D; ++dir) {
+      const int pl = l * g.D + dir;
+      const float* base = res + (size_t)pl * r.per_pl;
+      SeqBwd::Dir& q = p.d[dir];
+      q.gout = gout ? gout + (size_t)dir * g.H : nullptr;
+      q.dhy = dhy ? dhy + (size_t)pl * g.BH : nullptr;
+      q.dcy = dcy ? dcy + (size_t)pl * g.BH : nullptr;
+      q.R = w + offsets(g, pl).R;
+      q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
+      q.dGW = dGW[dir]; q.dGR = dGR[dir];
+      q.dhx = dhx ? dhx + (size_t)pl * g.BH : nullptr;
+      q.dcx = dcx ? dcx + (size_t)pl * g.BH : nullptr;
+      ip.d[dir].HP = dGR[dir];
+    }
+    hipLaunchKernelGGL(rnn_seq_init_kernel, dim3((unsigned)std::min<size_t>((ip.n / 4 + 255) / 256, 2048), g.D), dim3(256), 0, s, ip);
+    const int rc = seq_bwd<MODE>(g, p, s);
+    if (rc == FLHIP_DECLINED && !fused_applies(g)) return FLHIP_DECLINED;
+    if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
+    seq = rc == FLHIP_OK;
+  }
+  if (!seq) {
   if (MODE == RNN_LSTM)
     for (int dir = 0; dir < g.D; ++dir)
       hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s,
                          dcy ? dcy + (size_t)(l * g.D + dir) * g.BH : nullptr, dc[dir], g.BH);
+  auto step = [&](const StepBwd& p) {
+    if (g.B <= 16) launch_step_bwd<MODE, 1>(p, g.D, s);
+    else if (g.B <= 32) launch_step_bwd<MODE, 2>(p, g.D, s);
+    else launch_step_bwd<MODE, 4>(p, g.D, s);
+  };
   for (int st = g.T - 1; st >= 0; --st) {
     StepBwd p{};
     p.B = g.B;
@@ -827,23 +1279,30 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
       a.dgr = dGR[dir] + (size_t)st * g.B * g.GH;
       a.dh_dir = dh_dir[dir] + (size_t)(st & 1) * g.BH;
     }
-    if (g.B <= 16) launch_step_bwd<MODE, 1>(p, g.D, s);
-    else if (g.B <= 32) launch_step_bwd<MODE, 2>(p, g.D, s);
-    else launch_step_bwd<MODE, 4>(p, g.D, s);
+    step(p);
+  }
+  if (dhx) {
+    StepBwd p{};
+    p.B = g.B;
+    p.H = g.H;
+    for (int dir = 0; dir < g.D; ++dir) {
+      CellBwd& a = p.d[dir];
+      a.dhx = dhx + (size_t)(l * g.D + dir) * g.BH;
+      a.dh_a = dh_dir[dir];
+      a.R = w + offsets(g, l * g.D + dir).R;
+      a.dgr_next = dGR[dir];
+    }
+    step(p);
+  }
+  if (dcx && MODE == RNN_LSTM)
+    for (int dir = 0; dir < g.D; ++dir)
+      hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, dc[dir],
+                         dcx + (size_t)(l * g.D + dir) * g.BH, g.BH);
   }
   for (int dir = 0; dir < g.D; ++dir) {
     const int pl = l * g.D + dir;
     const Offsets o = offsets(g, pl);
     const float* HP = res + (size_t)pl * r.per_pl + r.hp;
-    if (dhx) {
-      int ndhb = 1;
-      if (const int rc = mm_sliced(w + o.R, dGR[dir], dh_rec, g.H, g.B, g.GH, 0, &ndhb, s)) return rc;
-      hipLaunchKernelGGL(rnn_add2_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, dh_dir[dir], dh_rec, ndhb,
-                         dhx + (size_t)pl * g.BH, g.BH);
-    }
-    if (dcx && MODE == RNN_LSTM)
-      hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, dc[dir], dcx + (size_t)pl * g.BH,
-                         g.BH);
     float* gdst = dir == 0 ? gin : tmp;
     if (const int rc = mm(w + o.W, dGW[dir], gdst, inl, TB, g.GH, 0, 0, nullptr, s)) return rc;
     if (dir)
@@ -889,15 +1348,16 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
+  const bool seq = seq_applies(g, s);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     float* out = l == g.L - 1 ? static_cast<float*>(y) : res + r.acts + (size_t)l * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;
-    if (fused_applies(g)) {
-      int rc;
+    int rc = FLHIP_DECLINED;
+    if (seq || fused_applies(g)) {
       auto args = [&](auto fn) {
         return fn(g, l, in, inl, wf, static_cast<const float*>(hx), static_cast<const float*>(cx), out,
-                  static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), s);
+                  static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), seq, s);
       };
       switch (g.mode) {
         case RNN_RELU: rc = args(forward_layer_fused<RNN_RELU>); break;
@@ -905,11 +1365,11 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
         case RNN_LSTM: rc = args(forward_layer_fused<RNN_LSTM>); break;
         default: rc = args(forward_layer_fused<RNN_GRU>);
       }
-      if (rc != FLHIP_OK) return rc;
-    } else {
+      if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
+    }
+    if (rc == FLHIP_DECLINED) {
       for (int dir = 0; dir < g.D; ++dir) {
         const int pl = l * g.D + dir;
-        int rc;
         auto args = [&](auto fn) {
           return fn(g, pl, in, inl, wf, static_cast<const float*>(hx), static_cast<const float*>(cx), out,
                     static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), s);
@@ -948,19 +1408,20 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   const float* res = static_cast<const float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   float* wsf = static_cast<float*>(ws);
-  const size_t TB = (size_t)g.T * g.B, act = TB * g.D * g.H, inmax = std::max<size_t>(g.I, (size_t)g.D * g.H);
+  const size_t TB = (size_t)g.T * g.B, act = TB * g.D * g.H, inmax = widest_input(g);
   float* goutbuf = wsf + 2 * TB * g.GH;
   float* ginbuf = goutbuf + act;
   const float* gout = static_cast<const float*>(dy);   // gradient of the top layer's output (may be null)
+  const bool seq = seq_applies(g, s);
   for (int l = g.L - 1; l >= 0; --l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;
     float* gin = l == 0 ? static_cast<float*>(dx) : ginbuf;
-    if (fused_applies(g)) {
-      int rc;
+    int rc = FLHIP_DECLINED;
+    if (seq || fused_applies(g)) {
       auto args = [&](auto fn) {
         return fn(g, l, in, inl, wf, gout, static_cast<const float*>(dhy), static_cast<const float*>(dcy), gin,
-                  static_cast<float*>(dhx), static_cast<float*>(dcx), static_cast<float*>(dw), res, wsf, s);
+                  static_cast<float*>(dhx), static_cast<float*>(dcx), static_cast<float*>(dw), res, wsf, seq, s);
       };
       switch (g.mode) {
         case RNN_RELU: rc = args(backward_layer_fused<RNN_RELU>); break;
@@ -968,11 +1429,11 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
         case RNN_LSTM: rc = args(backward_layer_fused<RNN_LSTM>); break;
         default: rc = args(backward_layer_fused<RNN_GRU>);
       }
-      if (rc != FLHIP_OK) return rc;
-    } else {
+      if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
+    }
+    if (rc == FLHIP_DECLINED) {
       for (int dir = 0; dir < g.D; ++dir) {
         const int pl = l * g.D + dir;
-        int rc;
         auto args = [&](auto fn) {
           return fn(g, pl, in, inl, wf, gout, static_cast<const float*>(dhy), static_cast<const float*>(dcy),
                     gin, dir == 0, static_cast<float*>(dhx), static_cast<float*>(dcx), static_cast<float*>(dw),
