@@ -7,7 +7,8 @@
 // GRU r, z, n with n = tanh(W_n x + b_Wn + r * (R_n h + b_Rn)), h' = (1-z)*n + z*h.
 //
 // Structure: the input projections of all time steps of a pseudo-layer are one matrix
-// product; the recurrence is a loop over time of (recurrent product, gate kernel).
+// product; the recurrence is one launch per layer where the hidden size allows, else a loop over
+// time of (recurrent product, gate kernel).
 // The products go through flhip_matmul (matrix cores where the shapes allow).  The
 // forward pass keeps, per pseudo-layer and in step order, the state before every step,
 // the gate activations and (GRU) R_n h + b_Rn in the reserve buffer; the backward pass
@@ -639,7 +640,9 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 // recurrent matrices from the caches per step (LSTM of 512 units, two directions, 32 columns: 8.2 us forward, 12.4 us
 // backward per step, where the products need 0.9 and 1.7).  Here the workgroups stay: each keeps its part of the
 // recurrent matrices in registers for all steps, and only the state (forward) or the pre-activation gradients (backward)
-// of a step travel between workgroups.  Batch columns do not depend on each other: a cluster of workgroups is one
+// of a step travel between workgroups.  Per step, forward / backward: that LSTM 8.2 -> 3.1 / 12.4 -> 5.9 us; GRU of 1024
+// units, 64 columns 16.2 -> 6.3 / 29.7 -> 7.3 us (products 2.6, exchange of 64 / 192 KB per workgroup); LSTM of 320 units,
+// 5 columns 5.1 -> 1.9 us forward.  What bounds them is the exchange's trip and its volume.  Batch columns do not depend on each other: a cluster of workgroups is one
 // direction of 16 columns, and clusters never wait for one another.
 //
 // The exchange needs no flags and no barrier over the grid: the step's rows in the reserve buffer / workspace (which the
@@ -654,7 +657,7 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 constexpr int SEQ_WAVES = STEP_WAVES, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
 constexpr int RNN_SPINS = 1 << 22;
 constexpr int RNN_OOB = (int)0x80000000;
-constexpr int AUX_AGENT = 16 | (int)0x80000000;      // buffer loads: sc1 (agent scope), and volatile: loaded every time
+constexpr int AUX_AGENT = 16;      // buffer loads: sc1, agent scope
 
 struct SeqFwd {
   struct Dir {
@@ -667,8 +670,21 @@ struct SeqFwd {
   int cluster0;      // first cluster of this launch; cluster = direction * groups + group
 };
 
-// N 16-byte loads per lane at off[i], repeated until every element is set.  (A lane's loads that do not exist are out of
-// the buffer's range and read zero.)
+// every load so far has arrived: what a loop carries from before it then needs no wait inside it (that wait would be one
+// for the stores of the step before)
+__device__ __forceinline__ void seq_drain() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
+// Between two steps: every wave waits until the workgroup's own elements are on their way, and as long again as such a
+// store travels (64 S cycles), before it asks for the others'.  Asked earlier, the loads come back unset and are repeated,
+// and their traffic holds up the very stores they wait for: LSTM of 512 units, 2 directions, 32 columns, forward, per step:
+// 6.2 us asking at once, 4.5 after the barrier, 4.0 / 3.6 / 3.7 with S = 8 / 12 / 16 (backward: 10.2, 9.9, 9.7, 9.6, 9.8).
+template <int S>
+__device__ __forceinline__ void seq_pause() {
+  __syncthreads();
+  __builtin_amdgcn_s_sleep(S);
+}
+
+// N 16-byte loads per lane at off[i].  (A lane's load that does not exist is out of the buffer's range and reads zero.)
 template <int N>
 __device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N]) {
   asm volatile("" ::: "memory");       // memory may have changed since the last load
@@ -676,19 +692,21 @@ __device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const int (&o
   for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, AUX_AGENT);
 }
 template <int N>
-__device__ __forceinline__ void seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], bool* dead) {
-  for (int spin = 0;; ++spin) {
-    bool ok = true;
+__device__ __forceinline__ bool seq_unset(const uintx4_t (&v)[N]) {
+  uint32_t m = 0;                    // (RNN_UNSET is the largest word)
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      ok = ok && v[i].x != RNN_UNSET && v[i].y != RNN_UNSET && v[i].z != RNN_UNSET && v[i].w != RNN_UNSET;
-    if (__all(ok) || *dead) return;
-    if (spin >= RNN_SPINS) {
-      *dead = true;
-      return;
-    }
+  for (int i = 0; i < N; ++i) m = max(max(m, max(v[i].x, v[i].y)), max(v[i].z, v[i].w));
+  return __builtin_amdgcn_ballot_w64(m == RNN_UNSET) != 0;
+}
+// Repeats the loads until every element is set.  -> whether the wave has given up, now or before (dead)
+template <int N>
+__device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], int dead) {
+  if (__builtin_amdgcn_readfirstlane(dead) || !seq_unset(v)) return dead;
+  for (int spin = 0; spin < RNN_SPINS; ++spin) {
     seq_load(r, off, v);
+    if (!seq_unset(v)) return 0;
   }
+  return 1;
 }
 
 // A workgroup owns HU hidden units of its cluster: row gate * HU + unit of its RT tiles of 16 rows.  The eight waves split
@@ -700,8 +718,9 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, RT = (G * HU + 15) / 16, W = SEQ_WAVES;
   extern __shared__ float seq_red[];      // [2][W][16 RT][17]
   const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * HU;
-  const int dir = cluster / p.groups, b0 = (cluster - dir * p.groups) * SEQ_COLS;
-  const SeqFwd::Dir& q = p.d[dir];
+  const int dir = __builtin_amdgcn_readfirstlane(cluster / p.groups), b0 = (cluster - dir * p.groups) * SEQ_COLS;
+  const SeqFwd::Dir q = dir ? p.d[1] : p.d[0];
+  float* const HP = q.HP;
   const int H = p.H, B = p.B, GH = G * H, T = p.T;
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -727,10 +746,11 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   c.bRn = q.bRn;
   c.ldo = p.ldo;
   float keep = 0.f;
-  if (cell) keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? q.HP[e] : 0.f;
-  bool dead = false;
-  for (int st = 0; st < T; ++st) {
-    const int t = dir ? T - 1 - st : st;
+  if (cell) keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? HP[e] : 0.f;
+  seq_drain();
+  int dead = 0;
+  for (int sv = 0; sv < T; ++sv) {
+    const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
     c.xp = q.xp + (size_t)t * B * GH;
     CellFwdIn<MODE> in{};
     if (cell) {
@@ -739,10 +759,12 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
       in.bRn = MODE == RNN_GRU ? c.bRn[ch] : 0.f;
       in.prev = keep;
     }
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(q.HP + st * BH, (unsigned)(BH * 4));
+    if (st > 0) seq_pause<12>();
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(HP + st * BH, (unsigned)(BH * 4));
     uintx4_t v[NC];
     seq_load(r, off, v);
-    seq_wait(r, off, v, &dead);
+    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v, dead));
+    seq_drain();
     floatx4_t acc[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) acc[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -769,7 +791,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
         for (int w = 0; w < W; ++w) sum += red[(w * RT * 16 + g * HU + unit) * 17 + col];
         rp[g] = sum;
       }
-      c.hn = q.HP + (st + 1) * BH;
+      c.hn = HP + (st + 1) * BH;
       c.cn = q.CP + (st + 1) * BH;
       c.gt = q.GT + (size_t)st * B * GH;
       c.rn = q.RN + st * BH;
@@ -798,8 +820,9 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, W = SEQ_WAVES, U = NC < 8 ? NC : 8, NB = NC / U;
   __shared__ float red2[2][W][16][17];
   const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * 16;
-  const int dir = cluster / p.groups, b0 = (cluster - dir * p.groups) * SEQ_COLS;
-  const SeqBwd::Dir& q = p.d[dir];
+  const int dir = __builtin_amdgcn_readfirstlane(cluster / p.groups), b0 = (cluster - dir * p.groups) * SEQ_COLS;
+  const SeqBwd::Dir q = dir ? p.d[1] : p.d[0];
+  float* const dGR = q.dGR;
   const int H = p.H, B = p.B, GH = G * H, T = p.T;
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -825,9 +848,10 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   CellBwd c{};
   c.ldo = p.ldo;
   float direct = cell && q.dhy ? q.dhy[e] : 0.f, dc = cell && MODE == RNN_LSTM && q.dcy ? q.dcy[e] : 0.f;
-  bool dead = false;
-  for (int st = T - 1; st >= (q.dhx ? -1 : 0); --st) {
-    const int t = dir ? T - 1 - st : st;
+  int dead = 0;
+  seq_drain();
+  for (int sv = T - 1; sv >= (q.dhx ? -1 : 0); --sv) {
+    const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
     CellBwdIn<MODE> in{};
     if (cell && st >= 0) {
       const size_t qe = (size_t)cb * GH + ch;
@@ -843,7 +867,8 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
     }
     float (*red)[16][17] = red2[st & 1];
     if (st < T - 1) {
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(q.dGR + (size_t)(st + 1) * B * GH, (unsigned)((size_t)B * GH * 4));
+      seq_pause<8>();
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(dGR + (size_t)(st + 1) * B * GH, (unsigned)((size_t)B * GH * 4));
       floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
       uintx4_t v[2][U];
       {
@@ -859,7 +884,8 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
           seq_load(r, off, v[(b + 1) & 1]);
         }
         offsets_of(b, off);
-        seq_wait(r, off, v[b & 1], &dead);
+        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v[b & 1], dead));
+        if (b == NB - 1) seq_drain();
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if ((wave + W * (b * U + u)) * 16 < GH)
@@ -883,7 +909,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
         in.go += direct;
         in.dc = dc;
         c.dgw = q.dGW + (size_t)t * B * GH;
-        c.dgr = q.dGR + (size_t)st * B * GH;
+        c.dgr = dGR + (size_t)st * B * GH;
         cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct);
       }
     }

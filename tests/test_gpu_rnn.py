@@ -64,6 +64,63 @@ def test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states):
         assert rel_l2(host(dcx), rdcx) <= 2e-4
 
 
+@pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
+    # whole sequences in one launch: hidden sizes that are multiples of 4 up to 1024.  4, 8 and 16 units per workgroup,
+    # a last workgroup with units to spare, a last contraction chunk with columns to spare, more waves than chunks
+    (flref.RNN_LSTM, 7, 20, 1, True, 5, 70, True),         # 5 column groups per direction
+    (flref.RNN_LSTM, 9, 500, 1, False, 4, 18, True),       # 4 units; 31 chunks + 4 columns
+    (flref.RNN_GRU, 130, 516, 1, True, 3, 20, True),       # 8 units (the last workgroup has 4), misaligned input width
+    (flref.RNN_LSTM, 8, 1024, 1, True, 2, 17, True),       # 16 units, the most registers
+    (flref.RNN_GRU, 8, 1000, 1, False, 3, 66, True),       # 5 clusters of 63 workgroups: two launches
+    (flref.RNN_TANH, 8, 1020, 2, False, 3, 5, False),
+    (flref.RNN_RELU, 8, 4, 2, True, 7, 16, True),          # one workgroup per cluster
+    (flref.RNN_LSTM, 8, 64, 1, False, 1, 1, True),         # one step, one column
+    (flref.RNN_GRU, 6, 1028, 1, False, 2, 3, True),        # too wide: a launch per step
+])
+def test_whole_sequence_launches(mode, I, H, L, bidir, T, B, states):
+    test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states)
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_not_a_number_states_end(mode):
+    """A state of any NaN, the pattern that marks an element as not yet written among them, gives NaN results."""
+    T, B, I, H = 5, 3, 4, 32
+    x = torch.ones(T, B, I, device="cuda")
+    w = torch.full((ops.rnn_param_count(I, H, 1, mode, False),), 0.1, device="cuda")
+    hx = torch.full((1, B, H), -1, dtype=torch.int32, device="cuda").view(torch.float32)
+    y, hy, cy, reserve = ops.rnn(x, hx, None, w, H, 1, mode, False)
+    dy = torch.full((T, B, H), -1, dtype=torch.int32, device="cuda").view(torch.float32)
+    dx, _, _, dw = ops.rnn_backward(x, w, reserve, H, 1, mode, False, dy)
+    assert mode == ops.RNN_RELU or bool(torch.isnan(y).all())      # (NaN > 0 is false: ReLU gives 0)
+    assert bool(torch.isnan(dw).any()) and dx.shape == x.shape
+
+
+def test_two_streams_at_once():
+    """Sequences issued on two streams without waiting for each other give what they give alone."""
+    T, B, I, H = 30, 32, 64, 512
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    w = torch.randn(ops.rnn_param_count(I, H, 1, ops.RNN_LSTM, True), device="cuda", generator=gen) / H ** 0.5
+    xs = [torch.randn(T, B, I, device="cuda", generator=gen) for _ in range(2)]
+    dy = torch.randn(T, B, 2 * H, device="cuda", generator=gen)
+
+    def run(x):
+        y, hy, cy, reserve = ops.rnn(x, None, None, w, H, 1, ops.RNN_LSTM, True)
+        return (y,) + tuple(t for t in ops.rnn_backward(x, w, reserve, H, 1, ops.RNN_LSTM, True, dy) if t is not None)
+
+    alone = [run(x) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    got = [[], []]
+    for _ in range(3):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(run(xs[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for res in got[i]:
+            assert all(torch.equal(a, b) for a, b in zip(res, alone[i]))
+
+
 def _random_configs(n, seed):
     rng = np.random.default_rng(seed)
     out = []
