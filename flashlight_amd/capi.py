@@ -97,6 +97,7 @@ SYMBOLS = {
     "flhip_matmul": (C.c_int, [_VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int32, C.c_int, C.c_int, _VP,
                                C.c_int, _VP]),
     "flhip_matmul_workspace_bytes": (C.c_size_t, [C.c_int32, C.c_int32, C.c_int32, C.c_int, C.c_int, C.c_int]),
+    "flhip_matmul_slices_bytes": (C.c_size_t, [C.c_int32, C.c_int32, C.c_int32, C.c_int, C.c_int, C.c_int]),
     "flhip_matmul_ws": (C.c_int, [_VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int32, C.c_int, C.c_int, _VP,
                                   C.c_int, _VP, C.c_size_t, _VP]),
     "flhip_sum_columns": (C.c_int, [_VP, _VP, C.c_int32, C.c_int32, C.c_int, _VP]),

@@ -945,8 +945,15 @@ extern "C" size_t flhip_matmul_workspace_bytes(int32_t M, int32_t N, int32_t K, 
   if (options().matmul_valu) return 0;
   if (is_lo16(dtype)) return options().matmul_fp32_cores ? 0 : mfma_gemm16_ws_bytes(dtype, 2, M, N, K);
   if (dtype != FLHIP_F32) return 0;
+  if (const size_t n = gemm32_ws_bytes(2, M, N, K)) return n;
   const int ns = nt_slices(M, N, K);
   return ns > 1 ? (size_t)ns * M * N * sizeof(float) : 0;
+}
+
+extern "C" size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || (trans_a && trans_b)) return 0;
+  if (trans_b || dtype != FLHIP_F32 || options().matmul_valu) return flhip_matmul_workspace_bytes(M, N, K, trans_a, trans_b, dtype);
+  return gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K);
 }
 
 extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
@@ -965,7 +972,18 @@ extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M,
   FLHIP_REQUIRE(A && B && C, "matmul: null argument");
   FLHIP_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "matmul: unknown dtype");
-  // thin products (a batch of feature vectors through fl::linear): the kernels made for them
+  // fp32 on the kernels of gemm_f32.hip.  A thin product (a batch of feature vectors through fl::linear) is few tiles and
+  // takes them only with the workspace to cut its contraction (1024 x 64 x 3136: 12 us; the thin kernels 42, one slice 100)
+  const bool thin = N <= 128 && !trans_b;
+  if (dtype == FLHIP_F32 && !(trans_a && trans_b) && !options().matmul_valu && options().matmul_planes < 0) {
+    const int mode = trans_a ? 1 : trans_b ? 2 : 0;
+    if (!thin || (ws ? ws_bytes : 0) >= gemm32_ws_bytes(mode, M, N, K)) {
+      const int rc = gemm32(mode, static_cast<const float*>(A), static_cast<const float*>(B), static_cast<float*>(C), M, N, K,
+                            bias_rows, ws, ws_bytes, as_stream(stream));
+      if (rc >= 0) return rc;
+    }
+  }
+  // the other thin products: the kernels made for them
   if (N <= 128 && !trans_b && !options().matmul_valu) {
     hipStream_t s = as_stream(stream);
     if (!trans_a) {

@@ -1,0 +1,350 @@
+// fp32 matrix products on the matrix cores (v_mfma_f32_32x32x2_f32), column-major:
+//   mode 0  C [M x N] = A [M x K]   * B [K x N]
+//   mode 1  C [M x N] = A [K x M]^T * B [K x N]
+//   mode 2  C [M x N] = A [M x K]   * B [N x K]^T            (+ bias[m])
+// the three products of fl::linear, and those of the recurrent layers over all time steps.
+//
+// A workgroup (4 waves, 2 x 2) owns a TM x TN tile of C, a wave TM/2 x TN/2 of it: RT x CT instruction tiles of 32 x 32.
+// The contraction runs in stages of 16; both operands' stages are copied to LDS by the loads themselves (buffer loads with
+// the LDS modifier: no registers, no vector instructions - on these cores those would wait for the matrix pipe), RING - 1
+// stages ahead of their use, one barrier per stage.
+//
+// An operand is contiguous either along the contraction ("k rows": B of modes 0 and 1, A of mode 1) or along the surviving
+// dimension ("m rows").  The lane of an instruction holds one row and, by lane half h, one of two contraction indexes; the
+// order of the indexes is free as long as both operands have it, and step e of group j takes k = 8 j + 4 h + e:
+//   k rows  LDS [row][4 pieces of 4 k]: a 16-byte read is a lane's operand of four steps.  Piece p of row r lies at slot
+//           p ^ ((r >> 2) & 3), so that the 16 lanes of a read pass touch distinct banks; four neighbouring lanes of a
+//           load still cover 64 contiguous bytes.
+//   m rows  LDS [k][row]: with RT = 2 a lane reads two neighbouring rows at once, which are its rows of the two instruction
+//           tiles (tile t of a wave has the rows 2 r + t).
+// Two workgroups fit a compute unit (64 KB of LDS each at 128 x 128), so one wave multiplies while its neighbour waits.
+//
+// What bounds it is the matrix pipe, and the last round of tiles that does not fill the chip (128 x 128 tiles: 2048 x 6400 is
+// 3.1 tiles per compute unit, so at most 78 % of the pipe's 153 TFLOP/s).  Measured, us (before: the 1x1 convolution kernels
+// with a matrix as one image's plane, A * B^T on 64 x 64 tiles staged through registers, thin products on the vector ALUs):
+//   mode 0  2000 x 4000 x 2000  286 -> 244 (131 TFLOP/s)    1024 x 6400 x 2048  286 -> 264    1024 x 64 x 3136  42 -> 12
+//   mode 1  2000 x 4000 x 2000  268 -> 239                  3072 x 6400 x 1024  353 -> 314    3136 x 64 x 1024  30 -> 11
+//   mode 2  2000 x 2000 x 4000  287 -> 243                  512 x 2048 x 6400   187 -> 112    80 x 2048 x 6400  58 -> 32
+#include <algorithm>
+
+#include "conv2d.h"
+#include "conv2d_mfma.h"
+#include "lds_direct.h"
+
+namespace flhip {
+namespace {
+
+constexpr int KC = 16, RING = 4, GTHREADS = 256;
+constexpr int G32_OOB = (int)0x80000000;
+
+struct Gemm32 {
+  int M, N, K;
+  int mtiles, ntiles;
+  int nstages, sps;            // stages of the contraction, stages per slice
+  unsigned a_bytes, b_bytes;
+  size_t slice;                // elements between the partial results of consecutive slices
+};
+
+// One operand's share of a stage: INSTR load instructions per wave, each 64 lanes x 16 bytes.
+template <bool KROWS, int T>
+struct Side {
+  static constexpr int INSTR = T * KC * 4 / 1024 / 4;
+  static constexpr int BYTES = T * KC * 4;
+  int off[INSTR];              // byte offset of a lane's piece at stage 0 (or out of range)
+  int kidx[INSTR];             // contraction index of that piece within a stage
+  int step;                    // bytes from a stage to the next
+
+  __device__ __forceinline__ void init(int r0, int R, int K, int wave, int lane) {
+#pragma unroll
+    for (int i = 0; i < INSTR; ++i) {
+      const int ii = wave * INSTR + i;
+      if (KROWS) {
+        const int row = ii * 16 + (lane >> 2), p = (lane & 3) ^ ((row >> 2) & 3);
+        kidx[i] = 4 * p;
+        off[i] = r0 + row < R ? ((r0 + row) * K + 4 * p) * 4 : G32_OOB;
+      } else {
+        const int piece = ii * 64 + lane, k = piece / (T / 4), m = 4 * (piece % (T / 4));
+        kidx[i] = k;
+        off[i] = r0 + m < R ? (k * R + r0 + m) * 4 : G32_OOB;
+      }
+    }
+    step = KROWS ? KC * 4 : KC * R * 4;
+  }
+  // the stage at byte offset `at` of every row, to the ring slot at lds (workgroup address).  CHECKED: only its first
+  // `left` contraction indexes exist (none of them, or fewer), the others read zero
+  template <bool CHECKED>
+  __device__ __forceinline__ void load(intx4_t rsrc, unsigned lds, int at, int left, int wave) const {
+#pragma unroll
+    for (int i = 0; i < INSTR; ++i)
+      pd_load_lds(rsrc, lds + (wave * INSTR + i) * 1024, CHECKED && kidx[i] >= left ? G32_OOB : off[i], at);
+  }
+};
+
+// the operands of one group of 8 contraction indexes: v[t][e] for instruction tile t and step e
+template <bool KROWS, int T, int NT>
+__device__ __forceinline__ void read_group(const float* lds, int j, int w, int fr, int h, float (&v)[NT][4]) {
+  if constexpr (KROWS) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int row = w * 32 * NT + t * 32 + fr;
+      const float4 f = *reinterpret_cast<const float4*>(lds + row * KC + 4 * ((2 * j + h) ^ ((row >> 2) & 3)));
+      v[t][0] = f.x; v[t][1] = f.y; v[t][2] = f.z; v[t][3] = f.w;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float* at = lds + (8 * j + 4 * h + e) * T + w * 32 * NT + NT * fr;
+      if constexpr (NT == 2) {
+        const float2 f = *reinterpret_cast<const float2*>(at);
+        v[0][e] = f.x; v[1][e] = f.y;
+      } else {
+        v[0][e] = *at;
+      }
+    }
+  }
+}
+
+template <int MODE, int TM, int TN>
+__global__ void __launch_bounds__(GTHREADS, 2)
+gemm32_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias,
+              const float* addend, float* C) {
+  constexpr bool AK = MODE == 1, BK = MODE != 2;
+  constexpr int RT = TM / 64, CT = TN / 64;
+  typedef Side<AK, TM> SA;
+  typedef Side<BK, TN> SB;
+  constexpr int STAGE = SA::BYTES + SB::BYTES;
+  extern __shared__ __align__(16) float g32_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  // consecutive workgroups go to the eight dies in turn: each die takes one run of tiles, and within a run the tiles of
+  // a column block follow each other, so that a die's cache holds what its workgroups share
+  const int tiles = p.mtiles * p.ntiles, per = tiles >> 3, rem = tiles & 7, die = blockIdx.x & 7;
+  const int tile = die * per + min(die, rem) + (blockIdx.x >> 3);
+  const int m0 = (tile % p.mtiles) * TM, n0 = (tile / p.mtiles) * TN;
+  const int s0 = blockIdx.y * p.sps, send = min(p.nstages, s0 + p.sps);
+
+  SA sa;
+  SB sb;
+  sa.init(m0, p.M, p.K, wave, lane);
+  sb.init(n0, p.N, p.K, wave, lane);
+  const intx4_t ar = pd_rsrc(A, p.a_bytes), br = pd_rsrc(B, p.b_bytes);
+  const unsigned lds0 = pd_lds_addr(g32_lds);
+  // stages from `send` on are not fetched, but every stage counts the same number of loads
+  auto stage_in = [&](auto checked, int slot, int s) __attribute__((always_inline)) {
+    constexpr bool CHECKED = decltype(checked)::value;
+    const int left = s < send ? p.K - s * KC : 0, at = CHECKED && s >= send ? 0 : s;
+    const unsigned lds = lds0 + (unsigned)slot * STAGE;
+    sa.template load<CHECKED>(ar, lds, at * sa.step, left, wave);
+    sb.template load<CHECKED>(br, lds + SA::BYTES, at * sb.step, left, wave);
+  };
+  constexpr std::integral_constant<bool, true> checked{};
+  constexpr std::integral_constant<bool, false> whole{};
+  floatx16 acc[RT][CT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s) stage_in(checked, s, s0 + s);
+  auto stage = [&](auto checked_, int slot, int s) __attribute__((always_inline)) {
+    // this stage has landed when at most the two behind it are still in flight
+    if constexpr (SA::INSTR + SB::INSTR == 4) PD_WAIT_VM(8);
+    else if constexpr (SA::INSTR + SB::INSTR == 3) PD_WAIT_VM(6);
+    else PD_WAIT_VM(4);
+    __syncthreads();                         // ... for every wave, and every wave is done with the slot of stage s - 1
+    const float* la = g32_lds + slot * (STAGE / 4);
+    const float* lb = la + SA::BYTES / 4;
+    float a[KC / 8][RT][4], b[KC / 8][CT][4];
+#pragma unroll
+    for (int j = 0; j < KC / 8; ++j) {
+      read_group<AK, TM, RT>(la, j, wm, fr, h, a[j]);
+      read_group<BK, TN, CT>(lb, j, wn, fr, h, b[j]);
+      if (j == 0) stage_in(checked_, (slot + RING - 1) % RING, s + RING - 1);
+    }
+#pragma unroll
+    for (int j = 0; j < KC / 8; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int c = 0; c < CT; ++c)
+            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j][i][e], b[j][c][e], acc[i][c], 0, 0, 0);
+  };
+  int s = s0;
+  // rounds of the ring whose look-ahead is whole stages
+  const int sfull = min(send, p.K / KC) - (RING - 1);
+  for (; s + RING <= sfull; s += RING) {
+#pragma unroll
+    for (int x = 0; x < RING; ++x) stage(whole, x, s + x);
+  }
+  for (; s < send; s += RING) {
+#pragma unroll
+    for (int x = 0; x < RING; ++x)
+      if (s + x < send) stage(checked, x, s + x);
+  }
+  PD_WAIT_VM(0);                             // nothing may land in LDS after the workgroup has ended
+
+  // element r of a lane: row 8 (r / 4) + 4 h + r % 4, column fr of the instruction tile
+  float* out = C + (size_t)blockIdx.y * p.slice;
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const int n = n0 + wn * 32 * CT + (BK ? c * 32 + fr : CT * fr + c);
+    if (n >= p.N) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = 8 * q + 4 * h;
+      if constexpr (AK || RT == 1) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const int m = m0 + wm * 32 * RT + i * 32 + row;
+          if (m >= p.M) continue;
+          float v[4];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = acc[i][c][4 * q + x] + (bias && m + x < p.M ? bias[m + x] : 0.f);
+          float* at = out + (size_t)n * p.M + m;
+          if (addend) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              if (m + x < p.M) v[x] += addend[(size_t)n * p.M + m + x];
+          }
+          if (!AK || (p.M & 3) == 0) {
+            *reinterpret_cast<float4*>(at) = make_float4(v[0], v[1], v[2], v[3]);
+          } else {
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              if (m + x < p.M) at[x] = v[x];
+          }
+        }
+      } else {                               // rows 2 r + t: eight neighbours of the two tiles (M is a multiple of 4)
+        const int m = m0 + wm * 64 + 2 * row;
+#pragma unroll
+        for (int x2 = 0; x2 < 2; ++x2) {
+          const int mm = m + 4 * x2;
+          if (mm >= p.M) continue;
+          float v[4];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = acc[x & 1][c][4 * q + 2 * x2 + (x >> 1)] + (bias ? bias[mm + x] : 0.f);
+          if (addend) {
+            const float4 f = *reinterpret_cast<const float4*>(addend + (size_t)n * p.M + mm);
+            v[0] += f.x; v[1] += f.y; v[2] += f.z; v[3] += f.w;
+          }
+          *reinterpret_cast<float4*>(out + (size_t)n * p.M + mm) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+      }
+    }
+  }
+}
+
+// out = sum of the slices (+ bias[row]) (+ addend, which may be out); rows of M4 pieces, M a multiple of 4 where there is
+// a bias
+__global__ void __launch_bounds__(256) gemm32_sum_kernel(const float4* __restrict__ part, const float* __restrict__ bias,
+                                                         const float4* addend, float4* out, size_t n4, int M4, int slices) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
+    float4 v = part[i];
+#pragma unroll 4
+    for (int k = 1; k < slices; ++k) {       // loads in flight together, sums in slice order
+      const float4 w = part[(size_t)k * n4 + i];
+      v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+    }
+    if (bias) {
+      const float* b = bias + 4 * (i % (size_t)M4);
+      v.x += b[0]; v.y += b[1]; v.z += b[2]; v.w += b[3];
+    }
+    if (addend) {
+      const float4 f = addend[i];
+      v.x += f.x; v.y += f.y; v.z += f.z; v.w += f.w;
+    }
+    out[i] = v;
+  }
+}
+
+struct Gemm32Plan {
+  Gemm32 p;
+  int tm, tn, slices;
+};
+
+// The tile and the number of contraction slices with the least estimated time: rounds of workgroups over the compute units
+// times a tile's stages, in units of a 128 x 128 stage (2048 matrix cycles); a smaller tile reads more LDS per product
+// (measured: 64 x 64 tiles reach about 0.85 of the rate of 128 x 128); slices cost their partial results' traffic.
+bool gemm32_plan(int mode, int M, int N, int K, bool sliced, Gemm32Plan* best) {
+  const bool ak = mode == 1, bk = mode != 2;
+  if ((ak ? K : M) % 4 != 0 || (bk ? K : N) % 4 != 0) return false;      // rows of whole 16-byte pieces
+  const long long ab = (long long)M * K * 4, bb = (long long)N * K * 4;
+  if (ab >= (1ll << 31) || bb >= (1ll << 31) || (long long)M * N >= (1ll << 31)) return false;
+  const int cus = mfma_num_cus(), nst = (K + KC - 1) / KC;
+  double best_cost = 1e30;
+  for (int tm : {128, 64})
+    for (int tn : {128, 64}) {
+      const int mt = (M + tm - 1) / tm, nt = (N + tn - 1) / tn;
+      const double rate = tm * tn == 128 * 128 ? 1.0 : tm * tn == 128 * 64 ? 0.93 : 0.85;
+      for (int ns = 1; ns <= (sliced ? 16 : 1); ++ns) {
+        if (ns > 1 && (nst / ns < 8 || ((size_t)M * N) % 4 != 0)) break;
+        const int sps = (nst + ns - 1) / ns;
+        if ((nst + sps - 1) / sps != ns) continue;
+        const long long wgs = (long long)mt * nt * ns, rounds = (wgs + cus - 1) / cus;
+        // a workgroup alone on its unit has nobody to hide its waits behind
+        const double alone = wgs <= cus ? 1.25 : 1.0;
+        double cost = (double)rounds * (sps + 6) * (tm * tn / 16384.0) / rate * alone;
+        if (ns > 1) cost += (double)(ns + 1) * M * N * 4 / 4e12 / (2048.0 / 2.4e9) + 3.0;
+        if (cost < best_cost) {
+          best_cost = cost;
+          best->tm = tm; best->tn = tn; best->slices = ns;
+          best->p.mtiles = mt; best->p.ntiles = nt; best->p.sps = sps;
+        }
+      }
+    }
+  best->p.M = M; best->p.N = N; best->p.K = K;
+  best->p.nstages = nst;
+  best->p.a_bytes = (unsigned)ab; best->p.b_bytes = (unsigned)bb;
+  best->p.slice = (size_t)M * N;
+  return true;
+}
+
+template <int MODE, int TM, int TN>
+int gemm32_go(const Gemm32Plan& pl, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
+  constexpr size_t lds = (size_t)RING * (TM + TN) * KC * 4;
+  auto kernel = gemm32_kernel<MODE, TM, TN>;
+  if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return -1;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(pl.p.mtiles * pl.p.ntiles), (unsigned)pl.slices), dim3(GTHREADS), lds, s, pl.p, A, B,
+                     bias, addend, C);
+  return check_launch("matmul (fp32)");
+}
+template <int MODE>
+int gemm32_tile(const Gemm32Plan& pl, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
+  if (pl.tm == 128) return pl.tn == 128 ? gemm32_go<MODE, 128, 128>(pl, A, B, bias, addend, C, s) : gemm32_go<MODE, 128, 64>(pl, A, B, bias, addend, C, s);
+  return pl.tn == 128 ? gemm32_go<MODE, 64, 128>(pl, A, B, bias, addend, C, s) : gemm32_go<MODE, 64, 64>(pl, A, B, bias, addend, C, s);
+}
+
+}  // namespace
+
+// bytes of workspace with which gemm32 may cut the contraction (0: it does not, or declines)
+size_t gemm32_ws_bytes(int mode, int M, int N, int K) {
+  Gemm32Plan pl{};
+  if (!gemm32_plan(mode, M, N, K, true, &pl) || pl.slices == 1) return 0;
+  return (size_t)pl.slices * M * N * sizeof(float);
+}
+
+int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int K, const float* bias, void* ws, size_t ws_bytes,
+           hipStream_t s, const float* addend) {
+  Gemm32Plan pl{};
+  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) |
+       reinterpret_cast<uintptr_t>(addend)) % 16 != 0)
+    return -1;
+  if (!gemm32_plan(mode, M, N, K, ws != nullptr && (!bias || M % 4 == 0), &pl)) return -1;
+  if (pl.slices > 1 && ws_bytes < (size_t)pl.slices * M * N * sizeof(float) && !gemm32_plan(mode, M, N, K, false, &pl)) return -1;
+  float* dst = pl.slices > 1 ? static_cast<float*>(ws) : C;
+  const float *b = pl.slices > 1 ? nullptr : bias, *a = pl.slices > 1 ? nullptr : addend;
+  const int rc = mode == 0 ? gemm32_tile<0>(pl, A, B, b, a, dst, s) : mode == 1 ? gemm32_tile<1>(pl, A, B, b, a, dst, s)
+                                                                              : gemm32_tile<2>(pl, A, B, b, a, dst, s);
+  if (rc || pl.slices == 1) return rc;
+  const size_t n4 = (size_t)M * N / 4;
+  hipLaunchKernelGGL(gemm32_sum_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, s,
+                     reinterpret_cast<const float4*>(ws), bias,
+                     reinterpret_cast<const float4*>(addend), reinterpret_cast<float4*>(C), n4, M / 4, pl.slices);
+  return check_launch("matmul (fp32, slices added)");
+}
+
+}  // namespace flhip

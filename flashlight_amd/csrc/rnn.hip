@@ -24,8 +24,11 @@
 
 extern "C" int flhip_matmul(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
                             int trans_a, int trans_b, const float* bias_rows, int dtype, void* stream);
-extern "C" int flhip_sum_columns(const void* x, float* out, int32_t rows, int32_t cols, int dtype,
-                                 void* stream);
+extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K, int trans_a,
+                               int trans_b, const float* bias_rows, int dtype, void* ws, size_t ws_bytes, void* stream);
+extern "C" int flhip_sum_columns_ws(const void* x, float* out, int32_t rows, int32_t cols, int dtype, void* ws,
+                                    size_t ws_bytes, void* stream);
+extern "C" size_t flhip_sum_columns_workspace_bytes(int32_t rows, int32_t cols, int dtype);
 
 namespace flhip {
 namespace {
@@ -140,9 +143,15 @@ int wgrad_slices(size_t M, size_t N, size_t K) {
   return (int)((chunks + cps - 1) / cps);
 }
 
+// the products over all time steps and the column sums may use the scratch at the end of the workspace
+struct Scratch {
+  void* p = nullptr;
+  size_t bytes = 0;
+};
+
 int mm(const float* A, const float* B, float* C, size_t M, size_t N, size_t K, int ta, int tb,
-       const float* bias, hipStream_t s) {
-  return flhip_matmul(A, B, C, (int32_t)M, (int32_t)N, (int32_t)K, ta, tb, bias, FLHIP_F32, s);
+       const float* bias, hipStream_t s, Scratch w = Scratch()) {
+  return flhip_matmul_ws(A, B, C, (int32_t)M, (int32_t)N, (int32_t)K, ta, tb, bias, FLHIP_F32, w.p, w.bytes, s);
 }
 
 // C = op(A) B in `*slices` partial products at C + k*M*N (see step_slices)
@@ -178,14 +187,26 @@ size_t wgrad_scratch_offset(const RnnGeom& g) {
          (size_t)(g.D - 1) * (2 * TB * g.GH + 3 * g.BH);
 }
 
-size_t workspace_floats(const RnnGeom& g) {
+size_t workspace_core(const RnnGeom& g) {
   const size_t TB = (size_t)g.T * g.B;
   int k;
   const size_t sf = step_slices(g.GH, g.B, g.H, &k);
   const size_t fwd = std::max(TB * g.GH + sf * g.B * g.GH + g.GH, (size_t)g.D * (TB * g.GH + g.GH));
   const size_t bwd = wgrad_scratch_offset(g) + wgrad_scratch(g);
-  return std::max(fwd, bwd) + 64;
+  return (std::max(fwd, bwd) + 67) & ~(size_t)3;
 }
+Scratch scratch_of(const RnnGeom& g, float* ws) {
+  const int TB = g.T * g.B, GH = (int)g.GH;
+  size_t n = flhip_sum_columns_workspace_bytes(GH, TB, FLHIP_F32);
+  for (int in : {g.I, g.D * g.H}) {
+    n = std::max(n, gemm32_ws_bytes(1, GH, TB, in));
+    n = std::max(n, gemm32_ws_bytes(0, in, TB, GH));
+    n = std::max(n, gemm32_ws_bytes(2, in, GH, TB));
+  }
+  n = std::max(n, gemm32_ws_bytes(2, g.H, GH, TB));
+  return Scratch{ws + workspace_core(g), (n + 15) & ~(size_t)15};
+}
+size_t workspace_bytes(const RnnGeom& g) { return workspace_core(g) * sizeof(float) + scratch_of(g, nullptr).bytes; }
 
 // the fused step kernels tile the hidden state by 16 and hold at most 64 batch columns
 bool fused_applies(const RnnGeom& g) {
@@ -944,13 +965,32 @@ __global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
 inline unsigned nblocks(size_t n) { return (unsigned)((n + 255) / 256); }
 
 // dst [M x N] = A [M x K] * B^T, through `scratch` when the contraction is cut into slices
-int mm_nt(const float* A, const float* B, float* dst, size_t M, size_t N, size_t K, float* scratch, hipStream_t s) {
+int mm_nt(const float* A, const float* B, float* dst, size_t M, size_t N, size_t K, float* scratch, Scratch w, hipStream_t s) {
+  if (const int rc = gemm32(2, A, B, dst, (int)M, (int)N, (int)K, nullptr, w.p, w.bytes, s); rc >= 0) return rc;
   const int ns = wgrad_slices(M, N, K);
   if (ns <= 1) return gemm_nt(FLHIP_F32, A, B, dst, (int)M, (int)N, (int)K, 1, s);
   if (const int rc = gemm_nt(FLHIP_F32, A, B, scratch, (int)M, (int)N, (int)K, ns, s)) return rc;
   hipLaunchKernelGGL(rnn_add2_kernel, dim3(nblocks(M * N)), dim3(256), 0, s, (const float*)nullptr, scratch, ns, dst,
                      M * N);
   return FLHIP_OK;
+}
+
+// dW [GH][in] row-major = column-major in x GH = IN [in x TB] * dGW^T; dR likewise with the states before each step; the
+// bias gradients are the row sums (one sum for both but for the GRU: its n gate's recurrent side differs)
+int weight_gradients(const RnnGeom& g, const Offsets& o, const float* in, size_t inl, const float* HP, const float* dGW,
+                     const float* dGR, float* dw, float* ws, hipStream_t s) {
+  const size_t TB = (size_t)g.T * g.B;
+  float* scratch = ws + wgrad_scratch_offset(g);
+  const Scratch w = scratch_of(g, ws);
+  if (const int rc = mm_nt(in, dGW, dw + o.W, inl, g.GH, TB, scratch, w, s)) return rc;
+  if (const int rc = mm_nt(HP, dGR, dw + o.R, g.H, g.GH, TB, scratch, w, s)) return rc;
+  if (const int rc = flhip_sum_columns_ws(dGW, dw + o.bW, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, w.p, w.bytes, s)) return rc;
+  if (g.mode == RNN_GRU) {
+    if (const int rc = flhip_sum_columns_ws(dGR, dw + o.bR, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, w.p, w.bytes, s)) return rc;
+  } else {
+    hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.GH)), dim3(256), 0, s, dw + o.bW, dw + o.bR, g.GH);
+  }
+  return check_launch("rnn_bwd");
 }
 
 template <int MODE>
@@ -971,7 +1011,7 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
   hipLaunchKernelGGL(rnn_bias_kernel, dim3(nblocks(g.GH)), dim3(256), 0, s, w + o.bW, w + o.bR, bsum,
                      (int)g.GH, g.H, g.mode);
   // XP [GH x TB] = W [GH x in] (row-major = a column-major in x GH matrix, transposed) * IN [in x TB]
-  if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s)) return rc;
+  if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws))) return rc;
   hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, hx ? hx + (size_t)pl * g.BH : nullptr,
                      HP, g.BH);
   if (MODE == RNN_LSTM)
@@ -1107,7 +1147,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
     hipLaunchKernelGGL(rnn_seq_init_kernel, dim3(std::max(1u, blocks), g.D), dim3(256), 0, s, ip);
     for (int dir = 0; dir < g.D; ++dir)
       if (const int rc = mm(w + offsets(g, l * g.D + dir).W, in, const_cast<float*>(p.d[dir].xp), g.GH, TB, inl, 1, 0,
-                            ip.d[dir].bsum, s))
+                            ip.d[dir].bsum, s, scratch_of(g, ws)))
         return rc;
     const int rc = seq_fwd<MODE>(g, p, s);
     if (rc != FLHIP_DECLINED) return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
@@ -1120,7 +1160,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
     float* bsum = ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH;
     hipLaunchKernelGGL(rnn_bias_kernel, dim3(nblocks(g.GH)), dim3(256), 0, s, w + o.bW, w + o.bR, bsum,
                        (int)g.GH, g.H, g.mode);
-    if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s)) return rc;
+    if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws))) return rc;
     hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s,
                        hx ? hx + (size_t)pl * g.BH : nullptr, res + (size_t)pl * r.per_pl + r.hp, g.BH);
     if (MODE == RNN_LSTM)
@@ -1212,17 +1252,10 @@ int backward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const flo
     hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, dc, dcx + (size_t)pl * g.BH, g.BH);
   // gradient of the layer input: gin [in x TB] (+)= W^T [in x GH] * dGW [GH x TB]
   float* gdst = first_dir ? gin : tmp;
-  if (const int rc = mm(w + o.W, dGW, gdst, inl, TB, g.GH, 0, 0, nullptr, s)) return rc;
+  if (const int rc = mm(w + o.W, dGW, gdst, inl, TB, g.GH, 0, 0, nullptr, s, scratch_of(g, ws))) return rc;
   if (!first_dir)
     hipLaunchKernelGGL(rnn_add2_kernel, dim3(nblocks(TB * inl)), dim3(256), 0, s, gin, tmp, 1, gin, TB * inl);
-  // dW [GH][in] row-major = column-major in x GH = IN [in x TB] * dGW^T; dR likewise with the
-  // states before each step; the bias gradients are the row sums
-  float* scratch = ws + wgrad_scratch_offset(g);
-  if (const int rc = mm_nt(in, dGW, dw + o.W, inl, g.GH, TB, scratch, s)) return rc;
-  if (const int rc = mm_nt(HP, dGR, dw + o.R, g.H, g.GH, TB, scratch, s)) return rc;
-  if (const int rc = flhip_sum_columns(dGW, dw + o.bW, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, s)) return rc;
-  if (const int rc = flhip_sum_columns(dGR, dw + o.bR, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, s)) return rc;
-  return check_launch("rnn_bwd");
+  return weight_gradients(g, o, in, inl, HP, dGW, dGR, dw, ws, s);
 }
 
 template <int MODE, int NBT>
@@ -1325,19 +1358,21 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
       hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, dc[dir],
                          dcx + (size_t)(l * g.D + dir) * g.BH, g.BH);
   }
+  const Scratch sc = scratch_of(g, ws);
   for (int dir = 0; dir < g.D; ++dir) {
     const int pl = l * g.D + dir;
     const Offsets o = offsets(g, pl);
     const float* HP = res + (size_t)pl * r.per_pl + r.hp;
-    float* gdst = dir == 0 ? gin : tmp;
-    if (const int rc = mm(w + o.W, dGW[dir], gdst, inl, TB, g.GH, 0, 0, nullptr, s)) return rc;
-    if (dir)
-      hipLaunchKernelGGL(rnn_add2_kernel, dim3(nblocks(TB * inl)), dim3(256), 0, s, gin, tmp, 1, gin, TB * inl);
-    float* scratch = ws + wgrad_scratch_offset(g);
-    if (const int rc = mm_nt(in, dGW[dir], dw + o.W, inl, g.GH, TB, scratch, s)) return rc;
-    if (const int rc = mm_nt(HP, dGR[dir], dw + o.R, g.H, g.GH, TB, scratch, s)) return rc;
-    if (const int rc = flhip_sum_columns(dGW[dir], dw + o.bW, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, s)) return rc;
-    if (const int rc = flhip_sum_columns(dGR[dir], dw + o.bR, (int32_t)g.GH, (int32_t)TB, FLHIP_F32, s)) return rc;
+    // gradient of the layer input, the second direction's added to the first's
+    int rc = dir == 0 ? -1 : gemm32(0, w + o.W, dGW[dir], gin, (int)inl, (int)TB, (int)g.GH, nullptr, sc.p, sc.bytes, s, gin);
+    if (rc > 0) return rc;
+    if (rc < 0) {
+      float* gdst = dir == 0 ? gin : tmp;
+      if ((rc = mm(w + o.W, dGW[dir], gdst, inl, TB, g.GH, 0, 0, nullptr, s, sc))) return rc;
+      if (dir)
+        hipLaunchKernelGGL(rnn_add2_kernel, dim3(nblocks(TB * inl)), dim3(256), 0, s, gin, tmp, 1, gin, TB * inl);
+    }
+    if ((rc = weight_gradients(g, o, in, inl, HP, dGW[dir], dGR[dir], dw, ws, s))) return rc;
   }
   return check_launch("rnn_bwd");
 }
@@ -1357,7 +1392,7 @@ extern "C" size_t flhip_rnn_reserve_bytes(const flhip_rnn_desc* d) {
 }
 extern "C" size_t flhip_rnn_workspace_bytes(const flhip_rnn_desc* d) {
   RnnGeom g;
-  return make_geom(d, &g) == FLHIP_OK ? workspace_floats(g) * sizeof(float) : 0;
+  return make_geom(d, &g) == FLHIP_OK ? workspace_bytes(g) : 0;
 }
 
 extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void* hx, const void* cx,

@@ -586,8 +586,10 @@ def linear(input, weight, bias=None):
             raise ValueError("linear: bias must have one element per output feature")
         b = _dev(bias, "bias").float().contiguous()
     y = torch.empty(tuple(x.shape[:-1]) + (fout,), dtype=x.dtype, device=x.device)
-    capi.check(capi.lib().flhip_matmul(_ptr(w), _ptr(x), _ptr(y), fout, frames, fin, 0, 0, _ptr(b),
-                                       _dtype_tag(x), _stream()))
+    nws = capi.lib().flhip_matmul_slices_bytes(fout, frames, fin, 0, 0, _dtype_tag(x))
+    ws = torch.empty((nws,), dtype=torch.uint8, device=x.device) if nws else None
+    capi.check(capi.lib().flhip_matmul_ws(_ptr(w), _ptr(x), _ptr(y), fout, frames, fin, 0, 0, _ptr(b), _dtype_tag(x),
+                                          _ptr(ws) if nws else None, nws, _stream()))
     return y
 
 
@@ -599,10 +601,12 @@ def linear_backward(grad_output, input, weight, want_bias=True):
     frames = x.numel() // fin
     tag = _dtype_tag(x)
     dx = torch.empty_like(x)
-    capi.check(capi.lib().flhip_matmul(_ptr(w), _ptr(g), _ptr(dx), fin, frames, fout, 1, 0, None, tag,
-                                       _stream()))
+    nws = capi.lib().flhip_matmul_slices_bytes(fin, frames, fout, 1, 0, tag)
+    ws = torch.empty((nws,), dtype=torch.uint8, device=x.device) if nws else None
+    capi.check(capi.lib().flhip_matmul_ws(_ptr(w), _ptr(g), _ptr(dx), fin, frames, fout, 1, 0, None, tag,
+                                          _ptr(ws) if nws else None, nws, _stream()))
     dw = torch.empty_like(w)
-    nws = capi.lib().flhip_matmul_workspace_bytes(fout, fin, frames, 0, 1, tag)
+    nws = capi.lib().flhip_matmul_slices_bytes(fout, fin, frames, 0, 1, tag)
     ws = torch.empty((nws,), dtype=torch.uint8, device=x.device) if nws else None
     capi.check(capi.lib().flhip_matmul_ws(_ptr(g), _ptr(x), _ptr(dw), fout, fin, frames, 0, 1, None, tag,
                                           _ptr(ws) if nws else None, nws, _stream()))

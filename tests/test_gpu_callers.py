@@ -205,6 +205,42 @@ def test_matmul_fp32_with_a_matrix_as_one_plane(M, N, K, ta, tb, planes):
         capi.set_option("MATMUL_PLANES", None)
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K,bias", [
+    (4, 4, 4, True),              # one piece of everything: three stages of the ring are never fetched
+    (64, 64, 16, False),          # one tile, one stage
+    (132, 68, 20, True),          # tiles with one piece of rows, a last stage of one piece
+    (128, 256, 112, False),       # as many stages as the unrolled loop takes in one round, and those behind it
+    (260, 132, 148, True),        # rounds of the ring, a ragged end
+    (64, 60, 4000, False),        # a long contraction in slices
+    (1024, 4, 3136, True),        # a thin product: slices, the bias added with them
+    (516, 1540, 64, True),        # more tiles than dies, not a multiple of them
+])
+def test_matmul_fp32_tiles(mode, M, N, K, bias):
+    """The fp32 products with and without a workspace, against float64.  A sum of K rounded products in any order differs
+    by about sqrt(K) units of 2^-24 in the 2-norm; allowed are twice that, and one more unit for the bias."""
+    import ctypes as C
+
+    from flashlight_amd import capi
+    rng = np.random.default_rng(M + N + K + mode)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    b = rng.standard_normal(M).astype(np.float32) if bias else None
+    ref = A.astype(np.float64) @ B.astype(np.float64) + (0 if b is None else b[:, None].astype(np.float64))
+    Ad, Bd = dev(np.ascontiguousarray(A if mode == 1 else A.T)), dev(np.ascontiguousarray(B if mode == 2 else B.T))
+    bd = dev(b) if bias else None
+    L, st = capi.lib(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    P = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None
+    need = L.flhip_matmul_slices_bytes(M, N, K, int(mode == 1), int(mode == 2), capi.F32)
+    for nws in {0, need}:
+        out = torch.full((N, M), float("nan"), device="cuda")
+        ws = torch.full((max(nws // 4, 4),), float("nan"), device="cuda")
+        capi.check(L.flhip_matmul_ws(P(Ad), P(Bd), P(out), M, N, K, int(mode == 1), int(mode == 2), P(bd), capi.F32,
+                                     P(ws) if nws else None, nws, st))
+        got = host(out).T.astype(np.float64)
+        assert rel_l2(got, ref) <= 2 * (np.sqrt(K) + 1) * 2.0 ** -24, (nws, rel_l2(got, ref))
+
+
 def test_matmul_fp32_at_the_size_of_a_speech_model():
     """2000 x 2000 weights against 4000 frames in fp32 (the plane mapping by shape), against numpy's float64 product."""
     M, N, K = 2000, 4000, 2000
