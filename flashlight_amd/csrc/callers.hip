@@ -499,7 +499,7 @@ matmul_tn_skinny(const T* __restrict__ A, const T* __restrict__ B, T* __restrict
   if (mi < M && nj < N) st(C, (size_t)nj * M + mi, mine);
 }
 
-// ---- logSoftmax over dimension 0 of a C x X matrix (Functions.cpp:1044-1070) ----
+// ---- logSoftmax over dimension 0 of a C x X matrix (Functions.cpp:1044-1070), columns too long for registers (rows.hip) ----
 // one wave per column
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -535,15 +535,15 @@ logsoftmax_bwd_kernel(const T* __restrict__ dy, const T* __restrict__ y, T* __re
 // ---- categorical cross-entropy on log-probabilities (Functions.cpp:1078-1154) ----
 // stats[0] = sum over counted columns of -x[target, col], stats[1] = counted columns,
 // stats[2] = columns whose target is neither in [0, C) nor the ignore index,
-// stats[3] = stats[0] / stats[1] (the MEAN reduction).  One block; columns are added
-// in a fixed order.
+// stats[3] = stats[0] / stats[1] (the MEAN reduction).  One block, one round of latencies per 1024 columns;
+// columns are added in a fixed order.
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(1024)
 cce_fwd_kernel(const T* __restrict__ x, const int32_t* __restrict__ target, float* __restrict__ stats,
                float* __restrict__ per_col, int Cn, int X, int ignore) {
-  __shared__ float red[4];
+  __shared__ float red[16];
   float s = 0.f, cnt = 0.f, bad = 0.f;
-  for (int i = threadIdx.x; i < X; i += 256) {
+  for (int i = threadIdx.x; i < X; i += 1024) {
     const int t = target[i];
     float v = 0.f;
     if (t == ignore) {
@@ -556,35 +556,14 @@ cce_fwd_kernel(const T* __restrict__ x, const int32_t* __restrict__ target, floa
     if (per_col) per_col[i] = v;
     s += v;
   }
-  s = block_sum(s, red);
-  cnt = block_sum(cnt, red);
-  bad = block_sum(bad, red);
+  s = block_sum<16>(s, red);
+  cnt = block_sum<16>(cnt, red);
+  bad = block_sum<16>(bad, red);
   if (threadIdx.x == 0) {
     stats[0] = s;
     stats[1] = cnt;
     stats[2] = bad;
     stats[3] = s / cnt;
-  }
-}
-
-// dx[c, col] = -(g_col) where c == target[col] and the column counts, else 0;
-// g_col = grad[0] / count (mean), grad[0] (sum) or grad[col] (none)
-template <typename T>
-__global__ void __launch_bounds__(256)
-cce_bwd_kernel(const float* __restrict__ grad, const int32_t* __restrict__ target,
-               const float* __restrict__ stats, T* __restrict__ dx, int Cn, int X, int reduction,
-               int ignore) {
-  const size_t total = (size_t)Cn * X;
-  const size_t stride = (size_t)gridDim.x * 256;
-  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += stride) {
-    const int col = (int)(e / Cn), c = (int)(e - (size_t)col * Cn);
-    const int t = target[col];
-    float v = 0.f;
-    if (t != ignore && c == t) {
-      const float g = reduction == 0 ? grad[col] : reduction == 1 ? grad[0] / stats[1] : grad[0];
-      v = -g;
-    }
-    st(dx, e, v);
   }
 }
 
@@ -1168,6 +1147,7 @@ extern "C" int flhip_logsoftmax_fwd(const void* x, void* y, int32_t classes, int
   FLHIP_REQUIRE(x && y, "logsoftmax: null argument");
   FLHIP_REQUIRE(classes > 0 && cols > 0, "logsoftmax: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "logsoftmax: unknown dtype");
+  if (rows_logsoftmax_fwd(x, y, classes, cols, dtype, as_stream(stream))) return check_launch("logsoftmax");
   const dim3 grid((unsigned)((cols + 3) / 4));
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
@@ -1182,6 +1162,7 @@ extern "C" int flhip_logsoftmax_bwd(const void* dy, const void* y, void* dx, int
   FLHIP_REQUIRE(dy && y && dx, "logsoftmax_bwd: null argument");
   FLHIP_REQUIRE(classes > 0 && cols > 0, "logsoftmax_bwd: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "logsoftmax_bwd: unknown dtype");
+  if (rows_logsoftmax_bwd(dy, y, dx, classes, cols, dtype, as_stream(stream))) return check_launch("logsoftmax_bwd");
   const dim3 grid((unsigned)((cols + 3) / 4));
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
@@ -1199,7 +1180,7 @@ extern "C" int flhip_cce_fwd(const void* logp, const int32_t* target, float* sta
   FLHIP_REQUIRE(dtype_ok(dtype), "cce: unknown dtype");
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
-    hipLaunchKernelGGL((cce_fwd_kernel<T>), dim3(1), dim3(256), 0, as_stream(stream),
+    hipLaunchKernelGGL((cce_fwd_kernel<T>), dim3(1), dim3(1024), 0, as_stream(stream),
                        (const T*)logp, target, stats, per_column, classes, cols, ignore_index);
   });
   return check_launch("cce");
@@ -1212,13 +1193,7 @@ extern "C" int flhip_cce_bwd(const float* grad, const int32_t* target, const flo
   FLHIP_REQUIRE(classes > 0 && cols > 0, "cce_bwd: sizes must be positive");
   FLHIP_REQUIRE(reduction >= 0 && reduction <= 2, "cce_bwd: unknown reduction");
   FLHIP_REQUIRE(dtype_ok(dtype), "cce_bwd: unknown dtype");
-  const size_t total = (size_t)classes * cols;
-  by_dtype(dtype, [&](auto* t_) {
-    using T = FLHIP_T_OF(t_);
-    hipLaunchKernelGGL((cce_bwd_kernel<T>), dim3(blocks_for(total)), dim3(256), 0,
-                       as_stream(stream), grad, target, stats, (T*)dx, classes, cols, reduction,
-                       ignore_index);
-  });
+  rows_cce_bwd(grad, target, stats, dx, classes, cols, reduction, ignore_index, dtype, as_stream(stream));
   return check_launch("cce_bwd");
 }
 

@@ -301,6 +301,12 @@ struct Options {
 };
 const Options& options();
 
+// rows.hip: rows held in registers (false: the row does not fit)
+bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hipStream_t s);
+bool rows_logsoftmax_bwd(const void* dy, const void* y, void* dx, int n, int rows, int dtype, hipStream_t s);
+void rows_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx, int n, int rows, int reduction,
+                  int ignore, int dtype, hipStream_t s);
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline bool dtype_ok(int32_t dt) { return dt == FLHIP_F32 || dt == FLHIP_BF16 || dt == FLHIP_F16; }

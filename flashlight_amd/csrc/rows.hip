@@ -1,0 +1,569 @@
+// Operations along contiguous rows: log-softmax and its gradient, the gradient of the categorical cross-entropy, and layer
+// norm over the leading dimensions with its scale and shift, forward and backward.
+//
+// All are bound by memory: what each cannot do without is every tensor once.  A row is therefore read once into registers
+// (raw 16-byte pieces, whatever the element type) and everything follows from there: one wave to a row of at most 64 NP
+// pieces (four rows to a workgroup), one workgroup of 256 to a longer one; NP pieces per thread, 1 .. 8.  Rows need not start
+// on 16-byte boundaries (9998 classes in bf16: every other row is 4 bytes off): the elements before the first and
+// behind the last whole piece of a row are handled one per thread.
+#include <algorithm>
+
+#include "common.h"
+
+namespace flhip {
+namespace {
+
+template <typename T> struct Piece { static constexpr int N = 16 / (int)sizeof(T); };
+
+// element e of a raw piece, and a raw piece of elements
+template <typename T>
+__device__ __forceinline__ void unpack(const uintx4_t& r, float (&v)[Piece<T>::N]) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(r[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (std::is_same<T, f16_t>::value) {
+        v[2 * i] = f16lo(r[i]); v[2 * i + 1] = f16hi(r[i]);
+      } else {
+        v[2 * i] = __uint_as_float(r[i] << 16); v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
+      }
+    }
+  }
+}
+template <typename T>
+__device__ __forceinline__ uintx4_t packed(const float (&v)[Piece<T>::N]) {
+  uintx4_t r;
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __float_as_uint(v[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      r[i] = std::is_same<T, f16_t>::value ? pack_f16(v[2 * i], v[2 * i + 1]) : pack_bf16(v[2 * i], v[2 * i + 1]);
+  }
+  return r;
+}
+
+// The split of a row of n elements: `head` single ones, `body` whole pieces, single ones again.  The single elements
+// (fewer than two pieces together) belong to the threads 0 .. in order.
+template <typename T>
+struct RowSplit {
+  int head, body, singles;
+  __device__ __forceinline__ RowSplit(const T* row, int n) {
+    constexpr int N = Piece<T>::N;
+    head = (int)((16 - (reinterpret_cast<uintptr_t>(row) & 15)) & 15) / (int)sizeof(T);
+    if (head > n) head = n;
+    body = (n - head) / N;
+    singles = n - body * N;
+  }
+  // element index of single i
+  __device__ __forceinline__ int at(int i) const { return i < head ? i : i + body * Piece<T>::N; }
+};
+
+template <int THREADS>
+__device__ __forceinline__ float row_sum(float v, float* smem) {
+  if constexpr (THREADS == 64) return wave_sum(v);
+  else return block_sum<THREADS / 64>(v, smem);
+}
+template <int THREADS>
+__device__ __forceinline__ float row_max(float v, float* smem) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  if constexpr (THREADS > 64) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = smem[0];
+#pragma unroll
+    for (int i = 1; i < THREADS / 64; ++i) v = fmaxf(v, smem[i]);
+  }
+  return v;
+}
+
+// ---- log-softmax over rows (Functions.cpp:1044-1070) --------------------------------------------------------------------
+// 4000 rows of 9998 in bf16 (160 MB): 137 -> 29 us (before: one wave to a row, element by element, three times over).
+template <typename T, int THREADS, int NP>
+__global__ void __launch_bounds__(256) logsoftmax_rows_fwd(const T* __restrict__ x, T* __restrict__ y, int n, int rows) {
+  constexpr int N = Piece<T>::N;
+  __shared__ float smem[4];
+  const int row = THREADS == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
+  if (THREADS == 64 && row >= rows) return;
+  const T* xr = x + (size_t)row * n;
+  T* yr = y + (size_t)row * n;
+  const RowSplit<T> sp(xr, n);
+  const uintx4_t* xb = reinterpret_cast<const uintx4_t*>(xr + sp.head);
+  uintx4_t r[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) r[i] = xb[t + i * THREADS];
+  const bool has1 = t < sp.singles;
+  const float one = has1 ? ld(xr, sp.at(t)) : -INFINITY;
+  float mx = one;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      float v[N];
+      unpack<T>(r[i], v);
+#pragma unroll
+      for (int e = 0; e < N; ++e) mx = fmaxf(mx, v[e]);
+    }
+  mx = row_max<THREADS>(mx, smem);
+  float s = has1 ? expf(one - mx) : 0.f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      float v[N];
+      unpack<T>(r[i], v);
+#pragma unroll
+      for (int e = 0; e < N; ++e) s += expf(v[e] - mx);
+    }
+  s = row_sum<THREADS>(s, smem);
+  const float lse = logf(s) + mx;
+  uintx4_t* yb = reinterpret_cast<uintx4_t*>(yr + sp.head);
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      float v[N];
+      unpack<T>(r[i], v);
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] -= lse;
+      yb[t + i * THREADS] = packed<T>(v);
+    }
+  if (has1) st(yr, sp.at(t), one - lse);
+}
+
+// dx = dy - exp(y) * sum of dy: 4000 rows of 9998 in bf16 (240 MB): 113 -> 44 us
+template <typename T, int THREADS, int NP>
+__global__ void __launch_bounds__(256)
+logsoftmax_rows_bwd(const T* __restrict__ dy, const T* __restrict__ y, T* __restrict__ dx, int n, int rows) {
+  constexpr int N = Piece<T>::N;
+  __shared__ float smem[4];
+  const int row = THREADS == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
+  if (THREADS == 64 && row >= rows) return;
+  const size_t o = (size_t)row * n;
+  const RowSplit<T> sp(dy + o, n);
+  const uintx4_t* gb = reinterpret_cast<const uintx4_t*>(dy + o + sp.head);
+  const uintx4_t* yb = reinterpret_cast<const uintx4_t*>(y + o + sp.head);
+  uintx4_t g[NP], p[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      g[i] = gb[t + i * THREADS];
+      p[i] = yb[t + i * THREADS];
+    }
+  const bool has1 = t < sp.singles;
+  const float g1 = has1 ? ld(dy + o, sp.at(t)) : 0.f, y1 = has1 ? ld(y + o, sp.at(t)) : 0.f;
+  float s = g1;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      float v[N];
+      unpack<T>(g[i], v);
+#pragma unroll
+      for (int e = 0; e < N; ++e) s += v[e];
+    }
+  s = row_sum<THREADS>(s, smem);
+  uintx4_t* xb = reinterpret_cast<uintx4_t*>(dx + o + sp.head);
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (t + i * THREADS < sp.body) {
+      float v[N], q[N];
+      unpack<T>(g[i], v);
+      unpack<T>(p[i], q);
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] -= expf(q[e]) * s;
+      xb[t + i * THREADS] = packed<T>(v);
+    }
+  if (has1) st(dx + o, sp.at(t), g1 - expf(y1) * s);
+}
+
+// ---- gradient of the categorical cross-entropy (Functions.cpp:1128-1150) ----------------------------------------------
+// dx[c, col] = -(g_col) where c == target[col] and the column counts, else 0; g_col = grad[0] / count (mean), grad[0] (sum)
+// or grad[col] (none).  A store stream of one row per workgroup: 4000 x 9998 in bf16 (80 MB): 35 -> 13 us.
+template <typename T>
+__global__ void __launch_bounds__(256)
+cce_rows_bwd(const float* __restrict__ grad, const int32_t* __restrict__ target, const float* __restrict__ stats,
+             T* __restrict__ dx, int n, int rows, int reduction, int ignore) {
+  constexpr int N = Piece<T>::N;
+  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+    const int tg = target[row];
+    const float g = tg == ignore ? 0.f : -(reduction == 0 ? grad[row] : reduction == 1 ? grad[0] / stats[1] : grad[0]);
+    T* xr = dx + (size_t)row * n;
+    const RowSplit<T> sp(xr, n);
+    uintx4_t* xb = reinterpret_cast<uintx4_t*>(xr + sp.head);
+    for (int i = threadIdx.x; i < sp.body; i += 256) {
+      float v[N];
+      const int c0 = sp.head + i * N;
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] = c0 + e == tg ? g : 0.f;
+      xb[i] = packed<T>(v);
+    }
+    if ((int)threadIdx.x < sp.singles) {
+      const int c = sp.at(threadIdx.x);
+      st(xr, c, c == tg ? g : 0.f);
+    }
+  }
+}
+
+// ---- layer norm over rows, with scale and shift (nn/modules/LayerNorm.cpp:42-131) --------------------------------------
+// y = w * (x - mean) / sqrt(var + eps) + b, statistics per row; w, b per element of the row (or one each), fp32, rounded to
+// the storage type first as the composed form has it.  Composed of a batch norm and a broadcast the forward pass moved
+// every element five times and the backward pass eight, the sums for dw and db with a stride of a row between lanes:
+// 4000 rows of 2000 in bf16: forward 21 + 20 -> 11 us, backward 155 + 5 + 25 -> 20 + 6 us.
+template <typename T>
+__device__ __forceinline__ float as_stored(float v) {
+  T t[1];
+  st(t, 0, v);
+  return ld(t, 0);
+}
+
+// WHOLE: rows of whole pieces on 16-byte boundaries; a thread then keeps its scales and shifts in registers from row to row
+// (fetched again for every row, element by element, they are most of the loads: 35 us).
+// the fp32 parameters of a piece's elements (all of them exist, or none)
+template <typename T>
+__device__ __forceinline__ void load_params(const float* p, int c0, int n, int pstride, float (&v)[Piece<T>::N]) {
+#pragma unroll
+  for (int e = 0; e < Piece<T>::N; e += 4) {
+    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (c0 < n) f = pstride ? *reinterpret_cast<const float4*>(p + c0 + e) : make_float4(p[0], p[0], p[0], p[0]);
+    v[e] = as_stored<T>(f.x); v[e + 1] = as_stored<T>(f.y); v[e + 2] = as_stored<T>(f.z); v[e + 3] = as_stored<T>(f.w);
+  }
+}
+
+template <typename T, int THREADS, int NP, bool WHOLE>
+__global__ void __launch_bounds__(256)
+layernorm_rows_fwd(const T* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, T* __restrict__ y,
+                   float* __restrict__ mean, float* __restrict__ invstd, int n, int rows, int pstride, float eps) {
+  constexpr int N = Piece<T>::N, RPB = 256 / THREADS;
+  __shared__ float smem[4];
+  const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
+  float wv[WHOLE ? NP : 1][N], bv[WHOLE ? NP : 1][N];
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      load_params<T>(w, (t + i * THREADS) * N, n, pstride, wv[i]);
+      load_params<T>(b, (t + i * THREADS) * N, n, pstride, bv[i]);
+    }
+  }
+  for (int row = blockIdx.x * RPB + (THREADS == 64 ? threadIdx.x >> 6 : 0); row < rows; row += gridDim.x * RPB) {
+    const T* xr = x + (size_t)row * n;
+    T* yr = y + (size_t)row * n;
+    const RowSplit<T> sp(xr, n);
+    const uintx4_t* xb = reinterpret_cast<const uintx4_t*>(xr + sp.head);
+    uintx4_t r[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) r[i] = xb[t + i * THREADS];
+    const bool has1 = !WHOLE && t < sp.singles;
+    const float one = has1 ? ld(xr, sp.at(t)) : 0.f;
+    float s = one;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) s += v[e];
+      }
+    const float m = row_sum<THREADS>(s, smem) / (float)n;
+    float q = has1 ? (one - m) * (one - m) : 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) q += (v[e] - m) * (v[e] - m);
+      }
+    const float is = 1.f / sqrtf(row_sum<THREADS>(q, smem) / (float)n + eps);
+    if (t == 0) {
+      mean[row] = m;
+      invstd[row] = is;
+    }
+    uintx4_t* yb = reinterpret_cast<uintx4_t*>(yr + sp.head);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+        const int c0 = sp.head + (t + i * THREADS) * N;
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          const int c = pstride * (c0 + e);
+          const float we = WHOLE ? wv[WHOLE ? i : 0][e] : as_stored<T>(w[c]), be = WHOLE ? bv[WHOLE ? i : 0][e] : as_stored<T>(b[c]);
+          v[e] = we * ((v[e] - m) * is) + be;
+        }
+        yb[t + i * THREADS] = packed<T>(v);
+      }
+    if (has1) {
+      const int c = sp.at(t);
+      st(yr, c, as_stored<T>(w[pstride * c]) * ((one - m) * is) + as_stored<T>(b[pstride * c]));
+    }
+  }
+}
+
+// dx = invstd * (g - mean(g) - xhat * mean(g * xhat)), g = w * dy, and over slice blockIdx.x of the rows the sums of
+// dy * xhat and dy per element of the row: part[slice][2][n].  Here the pieces of a row always start at its first element
+// (a thread keeps its elements' sums from row to row), so rows of whole pieces are the fast case; a row that is not reads
+// and writes single elements.
+template <typename T, int NP, bool WHOLE>
+__global__ void __launch_bounds__(256)
+layernorm_rows_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __restrict__ w,
+                   const float* __restrict__ mean, const float* __restrict__ invstd, T* __restrict__ dx,
+                   float* __restrict__ part, int n, int rows, int rps, int pstride) {
+  constexpr int N = Piece<T>::N;
+  __shared__ float smem[8];
+  const int t = threadIdx.x, r0 = blockIdx.x * rps, r1 = min(rows, r0 + rps);
+  float sw[NP][N], sb[NP][N], wv[NP][N];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if constexpr (WHOLE) load_params<T>(w, (t + i * 256) * N, n, pstride, wv[i]);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const int c = (t + i * 256) * N + e;
+      sw[i][e] = sb[i][e] = 0.f;
+      if (!WHOLE) wv[i][e] = c < n ? as_stored<T>(w[pstride * c]) : 0.f;
+    }
+  }
+  for (int row = r0; row < r1; ++row) {
+    const size_t o = (size_t)row * n;
+    float g[NP][N], xh[NP][N];
+    const float m = mean[row], is = invstd[row];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int c0 = (t + i * 256) * N;
+      if (WHOLE) {
+        uintx4_t a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+        if (c0 < n) {
+          a = *reinterpret_cast<const uintx4_t*>(dy + o + c0);
+          b = *reinterpret_cast<const uintx4_t*>(x + o + c0);
+        }
+        unpack<T>(a, g[i]);
+        unpack<T>(b, xh[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          g[i][e] = c0 + e < n ? ld(dy + o, c0 + e) : 0.f;
+          xh[i][e] = c0 + e < n ? ld(x + o, c0 + e) : 0.f;
+        }
+      }
+    }
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        if ((t + i * 256) * N + e < n) xh[i][e] = (xh[i][e] - m) * is;
+        sw[i][e] += g[i][e] * xh[i][e];
+        sb[i][e] += g[i][e];
+        g[i][e] *= wv[i][e];
+        s1 += g[i][e];
+        s2 += g[i][e] * xh[i][e];
+      }
+    block_sum2<4>(s1, s2, smem);
+    s1 /= (float)n;
+    s2 /= (float)n;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int c0 = (t + i * 256) * N;
+      float v[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] = is * (g[i][e] - s1 - xh[i][e] * s2);
+      if (WHOLE) {
+        if (c0 < n) *reinterpret_cast<uintx4_t*>(dx + o + c0) = packed<T>(v);
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          if (c0 + e < n) st(dx + o, c0 + e, v[e]);
+      }
+    }
+  }
+  float* out = part + (size_t)blockIdx.x * 2 * n;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const int c = (t + i * 256) * N + e;
+      if (c < n) {
+        out[c] = sw[i][e];
+        out[n + c] = sb[i][e];
+      }
+    }
+}
+
+// dw[c], db[c] = sums over the slices of part[slice][2][n]: a workgroup adds 64 columns, its 16 waves every 16th slice
+__global__ void __launch_bounds__(1024)
+layernorm_fold(const float* __restrict__ part, float* __restrict__ dw, float* __restrict__ db, int n, int slices) {
+  __shared__ float red[16][65];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;      // of 2 n
+  float s = 0.f;
+  if (c < 2 * n)
+#pragma unroll 4
+    for (int k = wave; k < slices; k += 16) s += part[(size_t)k * 2 * n + c];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && c < 2 * n) {
+#pragma unroll
+    for (int k = 1; k < 16; ++k) s += red[k][lane];
+    if (c < n) dw[c] = s;
+    else db[c - n] = s;
+  }
+}
+// one parameter element for the whole row: the sums over its columns
+__global__ void __launch_bounds__(256)
+layernorm_fold_scalar(const float* __restrict__ cols, float* __restrict__ dw, float* __restrict__ db, int n) {
+  __shared__ float smem[8];
+  float a = 0.f, b = 0.f;
+  for (int i = threadIdx.x; i < n; i += 256) {
+    a += cols[i];
+    b += cols[n + i];
+  }
+  block_sum2<4>(a, b, smem);
+  if (threadIdx.x == 0) {
+    dw[0] = a;
+    db[0] = b;
+  }
+}
+
+// f(threads tag, pieces tag) for rows of n elements; false: too long for registers
+template <typename T, typename F>
+bool by_row(int n, F&& f) {
+  const int pieces = (n + Piece<T>::N - 1) / Piece<T>::N;
+  using std::integral_constant;
+  integral_constant<int, 64> wave;
+  integral_constant<int, 256> wg;
+  integral_constant<int, 1> n1;
+  integral_constant<int, 2> n2;
+  integral_constant<int, 4> n4;
+  integral_constant<int, 8> n8;
+  if (pieces <= 64) f(wave, n1);
+  else if (pieces <= 128) f(wave, n2);
+  else if (pieces <= 256) f(wg, n1);
+  else if (pieces <= 512) f(wg, n2);
+  else if (pieces <= 1024) f(wg, n4);
+  else if (pieces <= 2048) f(wg, n8);
+  else return false;
+  return true;
+}
+
+bool same_offset(const void* a, const void* b, const void* c = nullptr) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a) & 15;
+  return x == (reinterpret_cast<uintptr_t>(b) & 15) && (!c || x == (reinterpret_cast<uintptr_t>(c) & 15));
+}
+
+// slices of the rows for the backward pass: about two workgroups per compute unit
+int ln_slices(int rows) { return std::max(1, std::min(512, rows / 4)); }
+
+}  // namespace
+
+// -> false where the row does not fit (the caller's element-wise kernels take it)
+bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hipStream_t s) {
+  if (!same_offset(x, y)) return false;
+  return by_dtype(dtype, [&](auto* t_) {
+    using T = FLHIP_T_OF(t_);
+    return by_row<T>(n, [&](auto th, auto np) {
+      const dim3 grid((unsigned)(th.value == 64 ? (rows + 3) / 4 : rows));
+      hipLaunchKernelGGL((logsoftmax_rows_fwd<T, th.value, np.value>), grid, dim3(256), 0, s, (const T*)x, (T*)y, n, rows);
+    });
+  });
+}
+
+bool rows_logsoftmax_bwd(const void* dy, const void* y, void* dx, int n, int rows, int dtype, hipStream_t s) {
+  if (!same_offset(dy, y, dx)) return false;
+  return by_dtype(dtype, [&](auto* t_) {
+    using T = FLHIP_T_OF(t_);
+    return by_row<T>(n, [&](auto th, auto np) {
+      const dim3 grid((unsigned)(th.value == 64 ? (rows + 3) / 4 : rows));
+      hipLaunchKernelGGL((logsoftmax_rows_bwd<T, th.value, np.value>), grid, dim3(256), 0, s, (const T*)dy, (const T*)y, (T*)dx,
+                         n, rows);
+    });
+  });
+}
+
+void rows_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx, int n, int rows, int reduction,
+                  int ignore, int dtype, hipStream_t s) {
+  by_dtype(dtype, [&](auto* t_) {
+    using T = FLHIP_T_OF(t_);
+    hipLaunchKernelGGL((cce_rows_bwd<T>), dim3((unsigned)std::min(rows, 16384)), dim3(256), 0, s, grad, target, stats, (T*)dx, n,
+                       rows, reduction, ignore);
+  });
+}
+
+}  // namespace flhip
+
+using namespace flhip;
+
+extern "C" int flhip_layernorm_applies(int64_t n, int64_t rows, int dtype) {
+  if (n <= 0 || rows <= 0 || rows > 0x7fffffffll || !dtype_ok(dtype)) return 0;
+  return n <= 1024 * 16 / (int64_t)dtype_size(dtype);      // four pieces per thread (the backward pass's registers)
+}
+
+extern "C" int flhip_layernorm_fwd(const void* x, const float* w, const float* b, void* y, float* mean, float* invstd,
+                                   int64_t n, int64_t rows, int scalar_params, double epsilon, int dtype, void* stream) {
+  FLHIP_REQUIRE(x && w && b && y && mean && invstd, "layernorm: null argument");
+  FLHIP_REQUIRE(dtype_ok(dtype), "layernorm: unknown dtype");
+  FLHIP_REQUIRE(flhip_layernorm_applies(n, rows, dtype), "layernorm: row length not supported");
+  FLHIP_REQUIRE(same_offset(x, y), "layernorm: x and y must be aligned alike");
+  by_dtype(dtype, [&](auto* t_) {
+    using T = FLHIP_T_OF(t_);
+    const bool whole = n % Piece<T>::N == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                                                 reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+    by_row<T>((int)n, [&](auto th, auto np) {
+      const int64_t blocks = th.value == 64 ? (rows + 3) / 4 : rows;
+      auto go = [&](auto kernel, int64_t most) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(blocks, most)), dim3(256), 0, as_stream(stream), (const T*)x, w, b, (T*)y,
+                           mean, invstd, (int)n, (int)rows, scalar_params ? 0 : 1, (float)epsilon);
+      };
+      if (whole) go(layernorm_rows_fwd<T, th.value, np.value, true>, 1024);
+      else go(layernorm_rows_fwd<T, th.value, np.value, false>, 65536);
+    });
+  });
+  return check_launch("layernorm_fwd");
+}
+
+extern "C" size_t flhip_layernorm_bwd_workspace_bytes(int64_t n, int64_t rows, int dtype) {
+  if (!flhip_layernorm_applies(n, rows, dtype)) return 0;
+  return (size_t)(ln_slices((int)rows) + 1) * 2 * (size_t)n * sizeof(float);
+}
+
+extern "C" int flhip_layernorm_bwd(const void* dy, const void* x, const float* w, const float* mean, const float* invstd,
+                                   void* dx, float* dw, float* db, int64_t n, int64_t rows, int scalar_params, int dtype,
+                                   void* ws, size_t ws_bytes, void* stream) {
+  FLHIP_REQUIRE(dy && x && w && mean && invstd && dx && dw && db, "layernorm_bwd: null argument");
+  FLHIP_REQUIRE(dtype_ok(dtype), "layernorm_bwd: unknown dtype");
+  FLHIP_REQUIRE(flhip_layernorm_applies(n, rows, dtype), "layernorm_bwd: row length not supported");
+  FLHIP_REQUIRE(ws && ws_bytes >= flhip_layernorm_bwd_workspace_bytes(n, rows, dtype), "layernorm_bwd: workspace too small");
+  hipStream_t s = as_stream(stream);
+  const int want = ln_slices((int)rows), rps = (int)((rows + want - 1) / want), slices = (int)((rows + rps - 1) / rps);
+  float* part = static_cast<float*>(ws);
+  by_dtype(dtype, [&](auto* t_) {
+    using T = FLHIP_T_OF(t_);
+    constexpr int N = Piece<T>::N;
+    const bool whole = n % N == 0 && ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) |
+                                       reinterpret_cast<uintptr_t>(dx) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+    const int pieces = (int)((n + N - 1) / N);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)slices), dim3(256), 0, s, (const T*)dy, (const T*)x, w, mean, invstd, (T*)dx, part,
+                         (int)n, (int)rows, rps, scalar_params ? 0 : 1);
+    };
+    if (whole) {
+      if (pieces <= 256) go(layernorm_rows_bwd<T, 1, true>);
+      else if (pieces <= 512) go(layernorm_rows_bwd<T, 2, true>);
+      else go(layernorm_rows_bwd<T, 4, true>);
+    } else {
+      if (pieces <= 256) go(layernorm_rows_bwd<T, 1, false>);
+      else if (pieces <= 512) go(layernorm_rows_bwd<T, 2, false>);
+      else go(layernorm_rows_bwd<T, 4, false>);
+    }
+  });
+  if (const int rc = check_launch("layernorm_bwd")) return rc;
+  float* cols = part + (size_t)slices * 2 * n;
+  hipLaunchKernelGGL(layernorm_fold, dim3((unsigned)((2 * n + 63) / 64)), dim3(1024), 0, s, part, scalar_params ? cols : dw,
+                     scalar_params ? cols + n : db, (int)n, slices);
+  if (scalar_params) hipLaunchKernelGGL(layernorm_fold_scalar, dim3(1), dim3(256), 0, s, cols, dw, db, (int)n);
+  return check_launch("layernorm_bwd (sums)");
+}

@@ -830,6 +830,22 @@ def layer_norm(input, norm_axes, epsilon=1e-5, weight=None, bias=None):
         w4 = [whcn[k] for k in ctx["perm"]]
         bn_axes = list(range(len(norm), 4))
         norm = list(range(len(norm)))
+    if contiguous and weight is not None and bias is not None and norm == list(range(len(norm))):
+        # rows of contiguous elements: statistics, scale and shift in one pass
+        n = 1
+        for k in norm:
+            n *= whcn[k]
+        rows = x.numel() // max(n, 1)
+        L, tag = capi.lib(), _dtype_tag(x)
+        if weight.numel() in (1, n) and bias.numel() == weight.numel() and L.flhip_layernorm_applies(n, rows, tag):
+            w, b = _f32vec(weight, weight.numel(), "weight"), _f32vec(bias, weight.numel(), "bias")
+            y = torch.empty_like(x)
+            sm = torch.empty((rows,), dtype=torch.float32, device=x.device)
+            si = torch.empty((rows,), dtype=torch.float32, device=x.device)
+            capi.check(L.flhip_layernorm_fwd(_ptr(x), _ptr(w), _ptr(b), _ptr(y), _ptr(sm), _ptr(si), n, rows,
+                                             int(weight.numel() == 1 and n > 1), float(epsilon), tag, _stream()))
+            ctx.update({"x4": x4, "sm": sm, "si": si, "comp": comp, "rows": (n, rows)})
+            return y, ctx
     xhat, sm, si = batchnorm(x4, None, None, None, None, bn_axes, True, 0.0, epsilon)
     ctx.update({"x4": x4, "xhat": xhat, "sm": sm, "si": si, "comp": bn_axes})
     out = xhat
@@ -846,6 +862,20 @@ def layer_norm_backward(grad_output, ctx, weight=None):
     """-> (gradInput, gradWeight, gradBias) of `layer_norm` (the last two None without
     parameters)."""
     g = _dev(grad_output, "gradOutput")
+    if "rows" in ctx:
+        (n, rows), x = ctx["rows"], ctx["x4"]
+        if g.numel() != x.numel() or g.dtype != x.dtype:
+            raise ValueError("layerNorm backward: gradOutput must match the input")
+        L, tag = capi.lib(), _dtype_tag(x)
+        w = _f32vec(weight, weight.numel(), "weight")
+        dx = torch.empty_like(x)
+        dw = torch.empty((weight.numel(),), dtype=torch.float32, device=x.device)
+        db = torch.empty_like(dw)
+        nws = L.flhip_layernorm_bwd_workspace_bytes(n, rows, tag)
+        ws = _ws(nws, x.device)
+        capi.check(L.flhip_layernorm_bwd(_ptr(g), _ptr(x), _ptr(w), _ptr(ctx["sm"]), _ptr(ctx["si"]), _ptr(dx), _ptr(dw),
+                                         _ptr(db), n, rows, int(weight.numel() == 1 and n > 1), tag, _ptr(ws), nws, _stream()))
+        return dx.reshape(grad_output.shape), dw, db
     if ctx["perm"] is not None:
         whcn = list(g.shape)[::-1]
         whcn += [1] * (4 - len(whcn))

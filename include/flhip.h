@@ -497,6 +497,19 @@ int flhip_affine_bwd(const void* dy, const void* x, const void* w, void* dx, flo
                      int scalar_params, int dtype, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* fl::LayerNorm::forward (nn/modules/LayerNorm.cpp:42-131) over contiguous rows of n elements (the normalised
+ * dimensions are the leading ones), statistics, scale and shift in one pass: y = w * (x - mean) / sqrt(var + eps) + b
+ * with w, b (fp32, rounded to the storage type in the kernel) of n elements or, scalar_params != 0, one; mean and invstd
+ * (fp32, one per row) feed the backward pass: dx, and dw = sum over rows of dy * xhat, db = sum of dy (fp32).
+ * flhip_layernorm_applies: whether a row fits (16 KiB). */
+int flhip_layernorm_applies(int64_t n, int64_t rows, int dtype);
+int flhip_layernorm_fwd(const void* x, const float* w, const float* b, void* y, float* mean, float* invstd, int64_t n,
+                        int64_t rows, int scalar_params, double epsilon, int dtype, void* stream);
+size_t flhip_layernorm_bwd_workspace_bytes(int64_t n, int64_t rows, int dtype);
+int flhip_layernorm_bwd(const void* dy, const void* x, const float* w, const float* mean, const float* invstd, void* dx,
+                        float* dw, float* db, int64_t n, int64_t rows, int scalar_params, int dtype, void* ws,
+                        size_t ws_bytes, void* stream);
+
 /* fl::embedding (Functions.cpp:1707-1749): y[:, i] = w[:, idx[i]] for n indices (s32 on the device) into a
  * dim x tokens table; an index outside [0, tokens) gives a column of zeros.  Backward (there a CSR matrix of ones
  * times the transposed deltas): dw[:, t] = the sum of dy[:, i] over idx[i] == t, added in the order of i in fp32 and

@@ -295,6 +295,61 @@ def test_logsoftmax(classes, cols, dtype):
     assert np.allclose(host(dx), dx_ref, atol=_tol(dtype) * 10, rtol=_tol(dtype))
 
 
+# rows held in registers: one wave / one workgroup to a row, 1 to 8 pieces of 16 bytes per thread, rows that start off a
+# 16-byte boundary, the longest that fit (8192 / 16384 elements) and the first that do not
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("classes,cols", [(3, 9), (256, 5), (257, 5), (1025, 6), (2049, 3), (4001, 5), (8192, 2), (8193, 3), (9998, 3),
+                                          (16384, 2), (16385, 2)])
+def test_logsoftmax_and_cross_entropy_rows(classes, cols, dtype):
+    rng = np.random.default_rng(classes + cols)
+    x = _round((rng.standard_normal((cols, classes)) * 3).astype(np.float32), dtype)
+    dy = _round(rng.standard_normal((cols, classes)).astype(np.float32), dtype)
+    # one rounding to the storage type (half a unit of 2^-8 / 2^-11), the fp32 sum and exponentials below it
+    half = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    y_ref = flref.logsoftmax_fwd(x)
+    y = host(ops.log_softmax(dev(x, dtype)))
+    assert (np.abs(y - y_ref) <= (half + 1e-5) * np.abs(y_ref) + 2e-6).all()
+    yq = _round(y_ref, dtype)
+    dx_ref = flref.logsoftmax_bwd(dy, yq)
+    dx = host(ops.log_softmax_backward(dev(dy, dtype), dev(yq, dtype)))
+    total = np.abs(dy).sum(1, keepdims=True)       # what the sum of dy is made of: its fp32 error scales exp(y)
+    assert (np.abs(dx - dx_ref) <= (half + 1e-5) * np.abs(dx_ref) + 1e-6 * total * np.exp(yq) + 1e-7).all()
+    t = rng.integers(0, classes, cols).astype(np.int32)
+    t[0], t[-1], t[cols // 2] = 0, classes - 1, -1
+    _, _, _, count, _ = flref.cce_fwd(y_ref, t)
+    loss, stats = ops.categorical_cross_entropy(dev(y_ref), dev(t))
+    g = np.array([1.5], np.float32)
+    got = host(ops.categorical_cross_entropy_backward(dev(g), x.shape, dtype, dev(t), stats))
+    want = flref.cce_bwd(x.shape, g, t, count, ops.REDUCE_MEAN)
+    assert (np.abs(got - want) <= (half + 1e-6) * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("n,rows,scalar", [(1, 7, False), (7, 3, False), (8, 1, True), (512, 9, False), (520, 33, False), (1000, 130, True),
+                                           (2000, 70, False), (2001, 5, False), (4096, 6, False), (8192, 3, False)])
+def test_layer_norm_rows(n, rows, scalar, dtype):
+    """Layer norm over contiguous rows in one pass: one wave / one workgroup to a row, whole pieces and odd lengths, one
+    row to several slices of rows, a single parameter; 8192 elements in fp32 are composed of the general kernels."""
+    rng = np.random.default_rng(n + rows)
+    x = _round((rng.standard_normal((rows, n)) * 1.5 + 0.4).astype(np.float32), dtype)
+    dy = _round(rng.standard_normal((rows, n)).astype(np.float32), dtype)
+    w = _round((1 + 0.2 * rng.standard_normal(1 if scalar else n)).astype(np.float32), dtype)
+    b = _round((0.2 * rng.standard_normal(1 if scalar else n)).astype(np.float32), dtype)
+    whcn = [n, rows, 1, 1]
+    ry, rxhat, rmean, rvar = flref.layer_norm_fwd(x, whcn, (0,), 1e-5, w, b)
+    rdx, rdw, rdb = flref.layer_norm_bwd(dy, x, rxhat, rmean, rvar, whcn, (0,), 1e-5, w)
+    y, ctx = ops.layer_norm(dev(x, dtype), (0,), 1e-5, dev(w), dev(b))
+    dx, dw, db = ops.layer_norm_backward(dev(dy, dtype), ctx, dev(w))
+    tol = _tol(dtype)
+    assert rel_l2(host(y), ry) <= tol
+    if n > 1:
+        assert rel_l2(host(dx), rdx) <= tol
+        assert rel_l2(host(dw), rdw) <= tol
+    assert rel_l2(host(db), rdb) <= 1e-4
+    dx2, dw2, db2 = ops.layer_norm_backward(dev(dy, dtype), ctx, dev(w))
+    assert torch.equal(dx, dx2) and torch.equal(dw, dw2) and torch.equal(db, db2)
+
+
 @pytest.mark.parametrize("reduction", [ops.REDUCE_NONE, ops.REDUCE_MEAN, ops.REDUCE_SUM])
 def test_cross_entropy(reduction):
     rng = np.random.default_rng(70 + reduction)
