@@ -46,6 +46,7 @@ static bool apply_option(Options& o, const char* name, const char* v) {
       if (strstr(v, "tap1d")) m |= Options::SKIP_TAP1D;
       if (strstr(v, "cells")) m |= Options::SKIP_CELLS;
       if (strstr(v, "tap2d")) m |= Options::SKIP_TAP2D;
+      if (strstr(v, "thin")) m |= Options::SKIP_THIN;
     }
     o.conv_skip = m;
     return true;

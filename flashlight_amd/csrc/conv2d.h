@@ -156,6 +156,13 @@ int mfma_tap1d_wgrad(const ConvGeom& g, int dtype, const void* x, const void* dy
 // bytes of channels-last rows that their forward pass leaves at the start of its workspace and the filter gradient
 // takes as `rows` in place of x (0: the two passes do not both apply)
 size_t mfma_tap1d_rows_bytes(const ConvGeom& g, int dtype);
+// few result tiles: the waves of a workgroup share a 32 x 32 tile's contraction (conv2d_mfma_thin.hip); any window of
+// stride 1 without groups, source channels a multiple of 8; weights in mfma_thin_ws() bytes of workspace
+size_t mfma_thin_ws(const ConvGeom& g, int dtype, bool bwd);
+int mfma_thin_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s, void* ws,
+                       size_t ws_bytes);
+int mfma_thin_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx, hipStream_t s, void* ws,
+                            size_t ws_bytes);
 // 3x3 filter gradient with operand rows copied straight to LDS (conv2d_mfma_wgrad_dma_bf16.hip)
 size_t mfma_wgrad_dma16_ws(const ConvGeom& g);
 // tile: 0 = by the measured rule, 32 / 64 = that tile side or decline

@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "conv2d.h"
+#include "conv2d_mfma.h"
 
 // Scratch of flhip_conv2d_bwd_filter_static: lives in the code object, one copy per
 // device the library is loaded on, never freed.  The name is only a host-side handle;
@@ -157,6 +158,26 @@ static bool tap2d_on(const ConvGeom& g, int dtype) {
   return (dtype == FLHIP_BF16 || dtype == FLHIP_F16) && g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
 }
 
+// Few result tiles (of 32 channels x 32 positions): the thin kernels.  `first`: asked before the 3x3 slab and strip kernels, which
+// they beat up to two tiles per compute unit in fp32 (64 channels 56 x 56: 392 tiles 18.1 -> 15.9 us, 784 tiles 18.7 -> 22.3; 13 x 13
+// at batch 48, 508 tiles: 26 -> 18) and one in 16-bit storage (196 tiles 10.9 -> 9.0, 784 tiles 11.3 -> 13.0).  Not first: windows
+// those two do not take, where the tapped GEMM (64 x 64 tiles, fp32 arithmetic) lost at every size measured, 16-bit storage
+// by 2.5 to 9 (128 channels 28 x 28, one image: 68 -> 10 us; 256 channels 14 x 14 at batch 33: 176 -> 47), fp32 by 1.02 to 4 (5x5 over
+// 14 x 14, 64 -> 32 channels, backward-data: batch 1 62 -> 18, batch 512 253 -> 142).  1x1 windows: fp32 with few tiles for their contraction (2048 -> 512
+// over 7 x 7, 32 tiles: 52 -> 31, 112 tiles 54 -> 33; but 512 -> 2048, 128 tiles 17.6 -> 21.6).
+// Strided windows stay where they were: their forward pass leaves its gathered input to the filter gradient (16-bit storage) or
+// gives the same bits with and without a workspace (fp32).  So do fp32 forward passes of more than 9 taps (the small convnets'
+// 5x5): their bits, and with them the choices of the max pools behind them, stay what they were (36 -> 32 us at 784 tiles).
+static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
+  if (force_direct() || skip(Options::SKIP_THIN) || algo_is(Options::ALGO_TAPPED)) return false;
+  const bool lo = dtype != FLHIP_F32;
+  if (g.sy != 1 || g.sx != 1 || (lo && (skip(SK_BF16) || algo_is(Options::ALGO_CONVERT)))) return false;
+  const long long pos = (long long)g.N * (bwd ? g.H * g.W : g.OH * g.OW), tiles = (pos + 31) / 32 * (((bwd ? g.C : g.K) + 31) / 32);
+  if (g.KH * g.KW == 1) return first && !lo && tiles <= (bwd ? g.K : g.C) / 8;
+  if (!lo && !bwd && g.KH * g.KW > 9) return false;
+  return !first || tiles <= (lo ? 1 : 2) * (long long)mfma_num_cus();
+}
+
 static bool long_rows(const ConvGeom& g, int dtype, bool bwd, size_t ws_bytes) {
   if (algo_is(Options::ALGO_TAPPED)) return false;
   const size_t need = mfma_tapped_ws(g, dtype, bwd);
@@ -230,7 +251,9 @@ extern "C" size_t flhip_conv2d_workspace_bytes(const flhip_conv_desc* d, int pas
     const size_t a = mfma_tapped_ws(g, d->dtype, pass == FLHIP_CONV_BWD_DATA);
     const size_t b = is_lo16(d->dtype) ? mfma_pointwise16_lattice_ws(g, pass == FLHIP_CONV_BWD_DATA)
                                             : pass == FLHIP_CONV_BWD_DATA ? mfma_pointwise_split_ws(g, d->dtype, true) : 0;
-    const size_t c = mfma_tap1d_conv_ws(g, d->dtype, pass == FLHIP_CONV_BWD_DATA);
+    const bool bwd = pass == FLHIP_CONV_BWD_DATA;
+    size_t c = mfma_tap1d_conv_ws(g, d->dtype, bwd);
+    if (bwd || thin_on(g, d->dtype, bwd, true) || thin_on(g, d->dtype, bwd, false)) c = std::max(c, mfma_thin_ws(g, d->dtype, bwd));
     // (the stacked-plane kernels: where their rule takes the geometry, and for every plane of at most 32 x 32 positions so
     // that a caller can try them by plan number; beyond that their copy of the input is tens of megabytes nobody asked for)
     const size_t c2 = (tap2d_on(g, d->dtype) || g.H * g.W <= 1024) ? mfma_tap2d_conv_ws(g, d->dtype, pass == FLHIP_CONV_BWD_DATA) : 0;
@@ -258,6 +281,7 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_FIRST) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_first16_conv_fwd(g, x, w, bias, y, s, d->dtype);
     if (r < 0 && !skip(Options::SKIP_CELLS)) r = mfma_cells_conv_fwd(g, d->dtype, x, w, bias, y, s);
+    if (r < 0 && thin_on(g, d->dtype, false, true)) r = mfma_thin_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_STRIP) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_strip16_conv_fwd(g, x, w, bias, y, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
@@ -265,6 +289,8 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
     if (r < 0 && !skip(SK_GEMM)) r = mfma_pointwise_conv_fwd(g, d->dtype, x, w, bias, y, s);
     if (r < 0 && algo_is(Options::ALGO_TAPPED)) r = mfma_tapped_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && !skip(SK_SLAB)) r = mfma_slab_conv_fwd(g, d->dtype, x, w, bias, y, s);
+    if (r < 0 && !long_rows(g, d->dtype, false, ws ? ws_bytes : 0) && thin_on(g, d->dtype, false, false))
+      r = mfma_thin_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && !skip(SK_TAPPED) && !long_rows(g, d->dtype, false, ws ? ws_bytes : 0))
       r = mfma_tapped_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0) r = mfma_conv_fwd(g, d->dtype, x, w, bias, y, s);
@@ -287,11 +313,11 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
 static const char* const kBwdDataPlans[] = {"bf16 1x1, tiles loaded straight to LDS", "bf16 1x1 / gathered taps", "bf16 3x3 strip",
                                             "bf16 slab", "1x1 GEMM, split contraction", "1x1 GEMM", "slab", "tapped GEMM",
                                             "gather", "direct", "one-row windows", "stride-2 window over few channels, 2 x 2 cells",
-                                            "3x3 windows over stacked planes"};
+                                            "3x3 windows over stacked planes", "few tiles, contraction shared by the waves"};
 static const char* const kBwdFilterPlans[] = {"bf16 3x3 rows straight to LDS, 32 x 32 tiles", "bf16 3x3 rows straight to LDS, 64 x 64 tiles",
                                               "bf16 1x1 / gathered taps", "bf16 first layer", "bf16 3x3 rows", "1x1 GEMM", "row slab",
                                               "tapped GEMM", "gather", "direct", "one-row windows"};
-constexpr int kNumDataPlans = 13, kNumFilterPlans = 11;
+constexpr int kNumDataPlans = 14, kNumFilterPlans = 11;
 
 static int bwd_data_direct(const flhip_conv_desc* d, const ConvGeom& g, const void* dy, const void* w, void* dx, hipStream_t s) {
   const size_t total = (size_t)g.N * g.C * g.H * g.W;
@@ -330,6 +356,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
       case 9: r = bwd_data_direct(d, g, dy, w, dx, s); break;
       case 10: r = mfma_tap1d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes); break;
       case 11: r = mfma_cells_conv_bwd_data(g, d->dtype, dy, w, dx, s); break;
+      case 13: r = mfma_thin_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes); break;
       default: r = mfma_tap2d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     }
     return r < 0 ? FLHIP_DECLINED : r;
@@ -343,6 +370,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
       r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pointwise16_conv_bwd_data(g, dy, w, dx, s, ws, ws_bytes, d->dtype);
+    if (r < 0 && thin_on(g, d->dtype, true, true)) r = mfma_thin_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_STRIP) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_strip16_conv_bwd_data(g, dy, w, dx, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
@@ -351,6 +379,8 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
     if (r < 0 && !skip(SK_GEMM)) r = mfma_pointwise_conv_bwd_data(g, d->dtype, dy, w, dx, s);
     if (r < 0 && algo_is(Options::ALGO_TAPPED)) r = mfma_tapped_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && !skip(SK_SLAB)) r = mfma_slab_conv_bwd_data(g, d->dtype, dy, w, dx, s);
+    if (r < 0 && !long_rows(g, d->dtype, true, ws ? ws_bytes : 0) && thin_on(g, d->dtype, true, false))
+      r = mfma_thin_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && !skip(SK_TAPPED) && !long_rows(g, d->dtype, true, ws ? ws_bytes : 0))
       r = mfma_tapped_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0) r = mfma_conv_bwd_data(g, d->dtype, dy, w, dx, s);

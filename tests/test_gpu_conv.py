@@ -245,6 +245,47 @@ def test_conv_bf16_with_family_switched_off(family, case):
         capi.set_option("CONV_SKIP", None)
 
 
+# Few result tiles, the contraction shared by a workgroup's waves: channel counts off the units of 16 and the blocks of
+# 32, positions off the tiles of 32 and tiles across images, windows of up to 16 taps and more (the weights' copy goes 16
+# taps at a time), dilation, fewer units than waves; then every split: 16, 8 and 4 waves of one block of
+# channels, 8 and 4 waves of two.
+THIN_CASES = [
+    ((1, 8, 5, 7), (33, 8, 3, 3), (1, 1), (1, 1), (1, 1), 1),
+    ((3, 24, 11, 11), (70, 24, 3, 3), (1, 1), (0, 2), (1, 1), 1),
+    ((2, 40, 9, 13), (32, 40, 5, 5), (1, 1), (2, 2), (1, 1), 1),
+    ((2, 16, 12, 10), (48, 16, 4, 4), (1, 1), (3, 1), (2, 1), 1),
+    ((1, 128, 14, 14), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1), 1),
+    ((1, 1024, 7, 7), (40, 1024, 1, 1), (1, 1), (0, 0), (1, 1), 1),
+    ((16, 32, 28, 28), (32, 32, 5, 5), (1, 1), (2, 2), (1, 1), 1),
+    ((33, 32, 28, 28), (24, 32, 5, 5), (1, 1), (2, 2), (1, 1), 1),
+    ((24, 64, 28, 28), (64, 64, 5, 5), (1, 1), (2, 2), (1, 1), 1),
+    ((33, 64, 28, 28), (64, 64, 5, 5), (1, 1), (2, 2), (1, 1), 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", THIN_CASES)
+def test_conv_few_tiles(case, dtype):
+    """Sums in fp32, results rounded once: 2^-9 relative in bf16, 2^-12 in f16."""
+    for name, (got, ref) in _run(case, 61, dtype).items():
+        tight = 1e-4 if name in ("dw", "db") or dtype == torch.float32 else 4e-3 if dtype == torch.bfloat16 else 1e-3
+        assert rel_l2(got, ref) <= tight, (name, rel_l2(got, ref))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", MORE)
+def test_conv_with_few_tiles_on_the_other_families(case, dtype):
+    """The small shapes that the kernels above now take, on the kernels that larger batches of them run on."""
+    from flashlight_amd import capi
+    capi.set_option("CONV_SKIP", "thin")
+    try:
+        for name, (got, ref) in _run(case, 62, dtype).items():
+            tight = 1e-4 if name in ("dw", "db") or dtype == torch.float32 else 4e-3 if dtype == torch.bfloat16 else 1e-3
+            assert rel_l2(got, ref) <= tight, (name, rel_l2(got, ref))
+    finally:
+        capi.set_option("CONV_SKIP", None)
+
+
 # fp32 slab kernels over rows of whole 16-byte units (the 16-byte loaders) and over other rows (the element-wise
 # loaders): strides, dilation, groups, a filter tail, rows of 8 to 60 columns, a 5x1 and a 1x3 window, whole 7x7 planes.
 F32_SLAB_CASES = [
