@@ -986,7 +986,11 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   }
   p.tsplit = (g.OW + p.TL - 1) / p.TL;
   p.units = p.rows * p.tsplit;
-  p.upw = std::max(1, p.units / std::max(1, want));
+  // ranges per workgroup.  16-bit storage: never more workgroups than compute units, since each more range writes its
+  // partial tiles (6.3 MB over 250 -> 250 channels) and the reduction reads them (7 x 1111 frames, 448 -> 224 workgroups: 76 -> 66 us,
+  // 24 x 400 frames of 128 channels, 384 -> 192: 41 -> 36; but 16 x 1500 of 128 channels, 256 -> 128: 42 -> 52).  fp32 is bound by the
+  // matrix pipe, and rather has a last round that is half full than workgroups of twice the length
+  p.upw = esz == 2 ? (p.units - 1) / std::max(1, mfma_num_cus() / tiles) + 1 : std::max(1, p.units / std::max(1, want));
   pl->nsplit = (p.units + p.upw - 1) / p.upw;
   const long long rb = (long long)p.rows * p.TS * p.Cs * esz;
   const long long yb = (long long)g.N * g.K * g.H * g.OW * esz;
