@@ -1054,7 +1054,9 @@ bool seq_applies(const RnnGeom& g, hipStream_t s) {
   return st == hipStreamCaptureStatusNone;
 }
 
-// FLHIP_DECLINED where the device does not hold the launch (nothing has run then)
+// FLHIP_DECLINED where the runtime refuses the first launch (nothing has run then): the device does not hold it, or the
+// process has no cooperative launches to give (a program on the system's runtime and the default stream is told 'illegal
+// state' where torch's runtime launches)
 template <typename P>
 int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s) {
   if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return FLHIP_DECLINED;
@@ -1066,7 +1068,8 @@ int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s)
                                                     (unsigned)lds, s);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      if (p.cluster0 == 0 && e == hipErrorCooperativeLaunchTooLarge) return FLHIP_DECLINED;
+      if (p.cluster0 == 0 && (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorIllegalState || e == hipErrorNotSupported))
+        return FLHIP_DECLINED;
       return fail(FLHIP_RUNTIME_ERROR, std::string("rnn: ") + hipGetErrorString(e));
     }
   }
