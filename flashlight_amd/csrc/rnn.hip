@@ -1043,9 +1043,10 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
 }
 
 // ---- launching whole sequences: the hidden size a multiple of 4 (16-byte pieces of the state) and at most 1024
-// (registers), a stream that is not being captured (a cooperative launch is not recorded)
+// (registers), a step's gates within what a buffer load addresses (2 GiB: an LSTM of 1024 units up to 131071
+// columns), a stream that is not being captured (a cooperative launch is not recorded)
 bool seq_applies(const RnnGeom& g, hipStream_t s) {
-  if (options().rnn_unfused || g.H % 4 != 0 || g.H > 1024) return false;
+  if (options().rnn_unfused || g.H % 4 != 0 || g.H > 1024 || (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31)) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
