@@ -867,8 +867,8 @@ def layer_norm_backward(grad_output, ctx, weight=None):
     g = _dev(grad_output, "gradOutput")
     if "rows" in ctx:
         (n, rows), x = ctx["rows"], ctx["x4"]
-        if g.numel() != x.numel() or g.dtype != x.dtype:
-            raise ValueError("layerNorm backward: gradOutput must match the input")
+        if g.numel() != x.numel() or g.dtype != x.dtype or weight is None or weight.numel() not in (1, n):
+            raise ValueError("layerNorm backward: gradOutput and weight must match the input")
         L, tag = capi.lib(), _dtype_tag(x)
         w = _f32vec(weight, weight.numel(), "weight")
         dx = torch.empty_like(x)

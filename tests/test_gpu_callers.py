@@ -501,6 +501,15 @@ def test_layer_norm(whcn, norm, params, dtype):
         assert rel_l2(host(dw), rdw) <= tol and rel_l2(host(db), rdb) <= tol
 
 
+def test_layer_norm_rows_refuse_what_does_not_match():
+    """The backward pass reads the weight and the gradient by the forward pass's sizes."""
+    _, ctx = ops.layer_norm(dev(np.ones((3, 8), np.float32)), (0,), 1e-5, dev(np.ones(8, np.float32)), dev(np.zeros(8, np.float32)))
+    g = np.ones((3, 8), np.float32)
+    for bad_g, bad_w in ((g, None), (g, np.ones(4, np.float32)), (g[:2], np.ones(8, np.float32))):
+        with pytest.raises(ValueError):
+            ops.layer_norm_backward(dev(bad_g), ctx, None if bad_w is None else dev(bad_w))
+
+
 def test_layer_norm_argument_errors():
     with pytest.raises(ValueError):
         ops.layer_norm(dev(np.zeros((2, 2, 2, 2, 2), np.float32)), (0,))
