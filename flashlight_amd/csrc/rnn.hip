@@ -1056,8 +1056,8 @@ bool seq_applies(const RnnGeom& g, hipStream_t s) {
 }
 
 // FLHIP_DECLINED where the runtime refuses the first launch (nothing has run then): the device does not hold it, or the
-// process has no cooperative launches to give (a program on the system's runtime and the default stream is told 'illegal
-// state' where torch's runtime launches)
+// process gets no cooperative queue (a program started by a process that had launched cooperatively on the same card was
+// told 'illegal state'; by itself it launches)
 template <typename P>
 int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s) {
   if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return FLHIP_DECLINED;
@@ -1120,9 +1120,10 @@ void launch_step_fwd(const StepFwd& p, int D, hipStream_t s) {
 // sequence (seq), or one per time step for both directions
 template <int MODE>
 int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, const float* w, const float* hx,
-                        const float* cx, float* out, float* hy, float* cy, float* res, float* ws, bool seq, hipStream_t s) {
+                        const float* cx, float* out, float* hy, float* cy, float* res, float* ws, bool& seq, hipStream_t s) {
   const Reserve r = reserve_layout(g);
   const size_t TB = (size_t)g.T * g.B;
+  bool prepared = false;      // the initial states and the input projections are in place
   if (seq) {
     SeqInit ip{};
     SeqFwd p{};
@@ -1155,9 +1156,11 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
         return rc;
     const int rc = seq_fwd<MODE>(g, p, s);
     if (rc != FLHIP_DECLINED) return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
+    seq = false;              // nor the layers that follow
     if (!fused_applies(g)) return FLHIP_DECLINED;
+    prepared = true;
   }
-  for (int dir = 0; dir < g.D; ++dir) {
+  for (int dir = 0; dir < g.D && !prepared; ++dir) {
     const int pl = l * g.D + dir;
     const Offsets o = offsets(g, pl);
     float* XP = ws + (size_t)dir * TB * g.GH;
@@ -1270,7 +1273,7 @@ void launch_step_bwd(const StepBwd& p, int D, hipStream_t s) {
 template <int MODE>
 int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, const float* w, const float* gout,
                          const float* dhy, const float* dcy, float* gin, float* dhx, float* dcx, float* dw,
-                         const float* res, float* ws, bool seq, hipStream_t s) {
+                         const float* res, float* ws, bool& seq, hipStream_t s) {
   const Reserve r = reserve_layout(g);
   const size_t TB = (size_t)g.T * g.B, inmax = widest_input(g);
   int kdummy;
@@ -1303,9 +1306,9 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
     }
     hipLaunchKernelGGL(rnn_seq_init_kernel, dim3((unsigned)std::min<size_t>((ip.n / 4 + 255) / 256, 2048), g.D), dim3(256), 0, s, ip);
     const int rc = seq_bwd<MODE>(g, p, s);
-    if (rc == FLHIP_DECLINED && !fused_applies(g)) return FLHIP_DECLINED;
     if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
     seq = rc == FLHIP_OK;
+    if (!seq && !fused_applies(g)) return FLHIP_DECLINED;
   }
   if (!seq) {
   if (MODE == RNN_LSTM)
@@ -1413,7 +1416,7 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
-  const bool seq = seq_applies(g, s);
+  bool seq = seq_applies(g, s);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     float* out = l == g.L - 1 ? static_cast<float*>(y) : res + r.acts + (size_t)l * act;
@@ -1477,7 +1480,7 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   float* goutbuf = wsf + 2 * TB * g.GH;
   float* ginbuf = goutbuf + act;
   const float* gout = static_cast<const float*>(dy);   // gradient of the top layer's output (may be null)
-  const bool seq = seq_applies(g, s);
+  bool seq = seq_applies(g, s);
   for (int l = g.L - 1; l >= 0; --l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;
