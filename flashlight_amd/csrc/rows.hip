@@ -221,61 +221,78 @@ __device__ __forceinline__ float as_stored(float v) {
   return ld(t, 0);
 }
 
-// WHOLE: rows of whole pieces on 16-byte boundaries; a thread then keeps its scales and shifts in registers from row to row
-// (fetched again for every row, element by element, they are most of the loads: 35 us).
-// the fp32 parameters of a piece's elements (all of them exist, or none)
-template <typename T>
-__device__ __forceinline__ void load_params(const float* p, int c0, int n, int pstride, float (&v)[Piece<T>::N]) {
+// A thread has the same N elements at col + i * THREADS * N in every row, and keeps their scales and shifts in registers from
+// row to row (fetched again for every row they are most of the loads: 35 us for those 4000 rows of 2000).  N is a piece of 16
+// bytes where the rows are of whole pieces on 16-byte boundaries, or else one: neighbouring threads then read neighbouring
+// elements wherever a row, of x or of y, starts (10000 rows of 2001 in bf16: 78 -> 27 us against pieces with single elements around
+// them and parameters per row; composed 57).
+template <typename T, int N>
+struct Elements {                  // N elements of T as they are held
+  typename std::conditional<N == 1, float, uintx4_t>::type raw;
+  __device__ __forceinline__ void load(const T* p) {
+    if constexpr (N == 1) raw = ld(p, 0);
+    else raw = *reinterpret_cast<const uintx4_t*>(p);
+  }
+  __device__ __forceinline__ void get(float (&v)[N]) const {
+    if constexpr (N == 1) v[0] = raw;
+    else unpack<T>(raw, v);
+  }
+  static __device__ __forceinline__ void store(T* p, const float (&v)[N]) {
+    if constexpr (N == 1) st(p, 0, v[0]);
+    else *reinterpret_cast<uintx4_t*>(p) = packed<T>(v);
+  }
+};
+// their fp32 parameters
+template <typename T, int N>
+__device__ __forceinline__ void load_params(const float* p, int c, int n, int pstride, float (&v)[N]) {
+  if constexpr (N == 1) {
+    v[0] = c < n ? as_stored<T>(p[pstride * c]) : 0.f;
+  } else {
 #pragma unroll
-  for (int e = 0; e < Piece<T>::N; e += 4) {
-    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c0 < n) f = pstride ? *reinterpret_cast<const float4*>(p + c0 + e) : make_float4(p[0], p[0], p[0], p[0]);
-    v[e] = as_stored<T>(f.x); v[e + 1] = as_stored<T>(f.y); v[e + 2] = as_stored<T>(f.z); v[e + 3] = as_stored<T>(f.w);
+    for (int e = 0; e < N; e += 4) {
+      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (c < n) f = pstride ? *reinterpret_cast<const float4*>(p + c + e) : make_float4(p[0], p[0], p[0], p[0]);
+      v[e] = as_stored<T>(f.x); v[e + 1] = as_stored<T>(f.y); v[e + 2] = as_stored<T>(f.z); v[e + 3] = as_stored<T>(f.w);
+    }
   }
 }
 
-template <typename T, int THREADS, int NP, bool WHOLE>
+template <typename T, int THREADS, int NP, int N>
 __global__ void __launch_bounds__(256)
 layernorm_rows_fwd(const T* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, T* __restrict__ y,
                    float* __restrict__ mean, float* __restrict__ invstd, int n, int rows, int pstride, float eps) {
-  constexpr int N = Piece<T>::N, RPB = 256 / THREADS;
+  constexpr int RPB = 256 / THREADS;
   __shared__ float smem[4];
   const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
-  float wv[WHOLE ? NP : 1][N], bv[WHOLE ? NP : 1][N];
-  if constexpr (WHOLE) {
+  auto col = [&](int i) { return (t + i * THREADS) * N; };
+  float wv[NP][N], bv[NP][N];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      load_params<T>(w, (t + i * THREADS) * N, n, pstride, wv[i]);
-      load_params<T>(b, (t + i * THREADS) * N, n, pstride, bv[i]);
-    }
+  for (int i = 0; i < NP; ++i) {
+    load_params<T>(w, col(i), n, pstride, wv[i]);
+    load_params<T>(b, col(i), n, pstride, bv[i]);
   }
   for (int row = blockIdx.x * RPB + (THREADS == 64 ? threadIdx.x >> 6 : 0); row < rows; row += gridDim.x * RPB) {
     const T* xr = x + (size_t)row * n;
     T* yr = y + (size_t)row * n;
-    const RowSplit<T> sp(xr, n);
-    const uintx4_t* xb = reinterpret_cast<const uintx4_t*>(xr + sp.head);
-    uintx4_t r[NP];
+    Elements<T, N> r[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      if (t + i * THREADS < sp.body) r[i] = xb[t + i * THREADS];
-    const bool has1 = !WHOLE && t < sp.singles;
-    const float one = has1 ? ld(xr, sp.at(t)) : 0.f;
-    float s = one;
+      if (col(i) < n) r[i].load(xr + col(i));
+    float s = 0.f, q = 0.f;
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      if (t + i * THREADS < sp.body) {
+      if (col(i) < n) {
         float v[N];
-        unpack<T>(r[i], v);
+        r[i].get(v);
 #pragma unroll
         for (int e = 0; e < N; ++e) s += v[e];
       }
     const float m = row_sum<THREADS>(s, smem) / (float)n;
-    float q = has1 ? (one - m) * (one - m) : 0.f;
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      if (t + i * THREADS < sp.body) {
+      if (col(i) < n) {
         float v[N];
-        unpack<T>(r[i], v);
+        r[i].get(v);
 #pragma unroll
         for (int e = 0; e < N; ++e) q += (v[e] - m) * (v[e] - m);
       }
@@ -284,25 +301,15 @@ layernorm_rows_fwd(const T* __restrict__ x, const float* __restrict__ w, const f
       mean[row] = m;
       invstd[row] = is;
     }
-    uintx4_t* yb = reinterpret_cast<uintx4_t*>(yr + sp.head);
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      if (t + i * THREADS < sp.body) {
+      if (col(i) < n) {
         float v[N];
-        unpack<T>(r[i], v);
-        const int c0 = sp.head + (t + i * THREADS) * N;
+        r[i].get(v);
 #pragma unroll
-        for (int e = 0; e < N; ++e) {
-          const int c = pstride * (c0 + e);
-          const float we = WHOLE ? wv[WHOLE ? i : 0][e] : as_stored<T>(w[c]), be = WHOLE ? bv[WHOLE ? i : 0][e] : as_stored<T>(b[c]);
-          v[e] = we * ((v[e] - m) * is) + be;
-        }
-        yb[t + i * THREADS] = packed<T>(v);
+        for (int e = 0; e < N; ++e) v[e] = wv[i][e] * ((v[e] - m) * is) + bv[i][e];
+        Elements<T, N>::store(yr + col(i), v);
       }
-    if (has1) {
-      const int c = sp.at(t);
-      st(yr, c, as_stored<T>(w[pstride * c]) * ((one - m) * is) + as_stored<T>(b[pstride * c]));
-    }
   }
 }
 
@@ -321,7 +328,7 @@ layernorm_rows_bwd(const T* __restrict__ dy, const T* __restrict__ x, const floa
   float sw[NP][N], sb[NP][N], wv[NP][N];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    if constexpr (WHOLE) load_params<T>(w, (t + i * 256) * N, n, pstride, wv[i]);
+    if constexpr (WHOLE) load_params<T, N>(w, (t + i * 256) * N, n, pstride, wv[i]);
 #pragma unroll
     for (int e = 0; e < N; ++e) {
       const int c = (t + i * 256) * N + e;
@@ -450,6 +457,22 @@ bool by_row(int n, F&& f) {
   return true;
 }
 
+// the same with the elements of a row (at most 8192) dealt out one by one
+template <typename F>
+void by_element(int n, F&& f) {
+  using std::integral_constant;
+  integral_constant<int, 64> wave;
+  integral_constant<int, 256> wg;
+  if (n <= 64) f(wave, integral_constant<int, 1>{});
+  else if (n <= 128) f(wave, integral_constant<int, 2>{});
+  else if (n <= 256) f(wave, integral_constant<int, 4>{});
+  else if (n <= 512) f(wave, integral_constant<int, 8>{});
+  else if (n <= 1024) f(wave, integral_constant<int, 16>{});
+  else if (n <= 2048) f(wg, integral_constant<int, 8>{});
+  else if (n <= 4096) f(wg, integral_constant<int, 16>{});
+  else f(wg, integral_constant<int, 32>{});
+}
+
 bool same_offset(const void* a, const void* b, const void* c = nullptr) {
   const uintptr_t x = reinterpret_cast<uintptr_t>(a) & 15;
   return x == (reinterpret_cast<uintptr_t>(b) & 15) && (!c || x == (reinterpret_cast<uintptr_t>(c) & 15));
@@ -507,20 +530,19 @@ extern "C" int flhip_layernorm_fwd(const void* x, const float* w, const float* b
   FLHIP_REQUIRE(x && w && b && y && mean && invstd, "layernorm: null argument");
   FLHIP_REQUIRE(dtype_ok(dtype), "layernorm: unknown dtype");
   FLHIP_REQUIRE(flhip_layernorm_applies(n, rows, dtype), "layernorm: row length not supported");
-  FLHIP_REQUIRE(same_offset(x, y), "layernorm: x and y must be aligned alike");
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
-    const bool whole = n % Piece<T>::N == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
-                                                 reinterpret_cast<uintptr_t>(b)) & 15) == 0;
-    by_row<T>((int)n, [&](auto th, auto np) {
-      const int64_t blocks = th.value == 64 ? (rows + 3) / 4 : rows;
-      auto go = [&](auto kernel, int64_t most) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(blocks, most)), dim3(256), 0, as_stream(stream), (const T*)x, w, b, (T*)y,
-                           mean, invstd, (int)n, (int)rows, scalar_params ? 0 : 1, (float)epsilon);
-      };
-      if (whole) go(layernorm_rows_fwd<T, th.value, np.value, true>, 1024);
-      else go(layernorm_rows_fwd<T, th.value, np.value, false>, 65536);
-    });
+    const bool whole = n % Piece<T>::N == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
+                                                 reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+    auto go = [&](auto th, auto np, auto ne) {
+      // up to eight workgroups for each compute unit (with four, 10000 rows of 2001 in bf16 take 42 us instead of 27)
+      const int64_t blocks = std::min<int64_t>(th.value == 64 ? (rows + 3) / 4 : rows, 2048);
+      hipLaunchKernelGGL((layernorm_rows_fwd<T, th.value, np.value, ne.value>), dim3((unsigned)blocks), dim3(256), 0,
+                         as_stream(stream), (const T*)x, w, b, (T*)y, mean, invstd, (int)n, (int)rows, scalar_params ? 0 : 1,
+                         (float)epsilon);
+    };
+    if (whole) by_row<T>((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, Piece<T>::N>{}); });
+    else by_element((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, 1>{}); });
   });
   return check_launch("layernorm_fwd");
 }

@@ -350,6 +350,25 @@ def test_layer_norm_rows(n, rows, scalar, dtype):
     assert torch.equal(dx, dx2) and torch.equal(dw, dw2) and torch.equal(db, db2)
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("n", [6, 8, 29, 512, 520, 2000, 2001])
+def test_layer_norm_of_views(n, dtype):
+    """Contiguous views that start anywhere (a slice of the frames, or of a larger buffer) give what their copies give, up to
+    the order of a row's sums, forward and backward."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    rows = 5
+    buf = torch.randn(2, rows * n + 8, device="cuda", generator=gen).to(dtype)
+    w, b = torch.randn(n, device="cuda", generator=gen), torch.randn(n, device="cuda", generator=gen)
+    for shift in range(8):
+        x, dy = (t[shift:shift + rows * n].view(rows, n) for t in buf)
+        (y, ctx), (want, ctx2) = ops.layer_norm(x, (0,), 1e-5, w, b), ops.layer_norm(x.clone(), (0,), 1e-5, w, b)
+        # (the row's sums are taken piece by piece from its first 16-byte boundary: another start, another order)
+        tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+        assert rel_l2(host(y), host(want)) <= tol, shift
+        got, ref = ops.layer_norm_backward(dy, ctx, w), ops.layer_norm_backward(dy.clone(), ctx2, w)
+        assert all(rel_l2(host(a), host(r)) <= tol for a, r in zip(got, ref)), shift
+
+
 @pytest.mark.parametrize("reduction", [ops.REDUCE_NONE, ops.REDUCE_MEAN, ops.REDUCE_SUM])
 def test_cross_entropy(reduction):
     rng = np.random.default_rng(70 + reduction)
