@@ -314,92 +314,92 @@ layernorm_rows_fwd(const T* __restrict__ x, const float* __restrict__ w, const f
 }
 
 // dx = invstd * (g - mean(g) - xhat * mean(g * xhat)), g = w * dy, and over slice blockIdx.x of the rows the sums of
-// dy * xhat and dy per element of the row: part[slice][2][n].  Here the pieces of a row always start at its first element
-// (a thread keeps its elements' sums from row to row), so rows of whole pieces are the fast case; a row that is not reads
-// and writes single elements.
-template <typename T, int NP, bool WHOLE>
+// dy * xhat and dy per element of the row: part[slice][2][n].  A thread has the same elements in every row, as above, and
+// keeps their sums from row to row.  A row of one wave takes no barrier, and the four waves of a workgroup each have a row in
+// flight.  (100000 rows in bf16, before, a workgroup to every row and runs of 8 elements per thread: 29 elements 359 -> 31 us, 100
+// elements 429 -> 53, 256 elements 190 -> 51, 257 elements 433 -> 104; composed 168, 482, 1194 and 790.)
+template <typename T, int THREADS, int NP, int N>
 __global__ void __launch_bounds__(256)
 layernorm_rows_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __restrict__ w,
                    const float* __restrict__ mean, const float* __restrict__ invstd, T* __restrict__ dx,
                    float* __restrict__ part, int n, int rows, int rps, int pstride) {
-  constexpr int N = Piece<T>::N;
+  constexpr int RPB = 256 / THREADS;
   __shared__ float smem[8];
-  const int t = threadIdx.x, r0 = blockIdx.x * rps, r1 = min(rows, r0 + rps);
+  const int wave = threadIdx.x >> 6, t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
+  const int r0 = blockIdx.x * rps, r1 = min(rows, r0 + rps);
+  auto col = [&](int i) { return (t + i * THREADS) * N; };
   float sw[NP][N], sb[NP][N], wv[NP][N];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    if constexpr (WHOLE) load_params<T, N>(w, (t + i * 256) * N, n, pstride, wv[i]);
+    load_params<T>(w, col(i), n, pstride, wv[i]);
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const int c = (t + i * 256) * N + e;
-      sw[i][e] = sb[i][e] = 0.f;
-      if (!WHOLE) wv[i][e] = c < n ? as_stored<T>(w[pstride * c]) : 0.f;
-    }
+    for (int e = 0; e < N; ++e) sw[i][e] = sb[i][e] = 0.f;
   }
-  for (int row = r0; row < r1; ++row) {
+  for (int row = r0 + (THREADS == 64 ? wave : 0); row < r1; row += RPB) {
     const size_t o = (size_t)row * n;
+    Elements<T, N> rg[NP] = {}, rx[NP] = {};
     float g[NP][N], xh[NP][N];
     const float m = mean[row], is = invstd[row];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int c0 = (t + i * 256) * N;
-      if (WHOLE) {
-        uintx4_t a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
-        if (c0 < n) {
-          a = *reinterpret_cast<const uintx4_t*>(dy + o + c0);
-          b = *reinterpret_cast<const uintx4_t*>(x + o + c0);
-        }
-        unpack<T>(a, g[i]);
-        unpack<T>(b, xh[i]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < N; ++e) {
-          g[i][e] = c0 + e < n ? ld(dy + o, c0 + e) : 0.f;
-          xh[i][e] = c0 + e < n ? ld(x + o, c0 + e) : 0.f;
-        }
+    for (int i = 0; i < NP; ++i)
+      if (col(i) < n) {
+        rg[i].load(dy + o + col(i));
+        rx[i].load(x + o + col(i));
       }
-    }
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int i = 0; i < NP; ++i)
+    for (int i = 0; i < NP; ++i) {             // (elements that do not exist are zeros)
+      rg[i].get(g[i]);
+      rx[i].get(xh[i]);
 #pragma unroll
       for (int e = 0; e < N; ++e) {
-        if ((t + i * 256) * N + e < n) xh[i][e] = (xh[i][e] - m) * is;
+        if (col(i) < n) xh[i][e] = (xh[i][e] - m) * is;
         sw[i][e] += g[i][e] * xh[i][e];
         sb[i][e] += g[i][e];
         g[i][e] *= wv[i][e];
         s1 += g[i][e];
         s2 += g[i][e] * xh[i][e];
       }
-    block_sum2<4>(s1, s2, smem);
+    }
+    if constexpr (THREADS == 64) {
+      s1 = wave_sum(s1);
+      s2 = wave_sum(s2);
+    } else {
+      block_sum2<4>(s1, s2, smem);
+    }
     s1 /= (float)n;
     s2 /= (float)n;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int c0 = (t + i * 256) * N;
       float v[N];
 #pragma unroll
       for (int e = 0; e < N; ++e) v[e] = is * (g[i][e] - s1 - xh[i][e] * s2);
-      if (WHOLE) {
-        if (c0 < n) *reinterpret_cast<uintx4_t*>(dx + o + c0) = packed<T>(v);
-      } else {
-#pragma unroll
-        for (int e = 0; e < N; ++e)
-          if (c0 + e < n) st(dx + o, c0 + e, v[e]);
-      }
+      if (col(i) < n) Elements<T, N>::store(dx + o + col(i), v);
     }
   }
   float* out = part + (size_t)blockIdx.x * 2 * n;
+  if constexpr (THREADS == 64) {               // the four waves' sums meet in LDS, added in wave order
+    __shared__ float comb[4][64 * NP * N];
 #pragma unroll
-  for (int i = 0; i < NP; ++i)
+    for (int which = 0; which < 2; ++which) {
+      __syncthreads();
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const int c = (t + i * 256) * N + e;
-      if (c < n) {
-        out[c] = sw[i][e];
-        out[n + c] = sb[i][e];
-      }
+      for (int i = 0; i < NP; ++i)
+#pragma unroll
+        for (int e = 0; e < N; ++e) comb[wave][col(i) + e] = which ? sb[i][e] : sw[i][e];
+      __syncthreads();
+      for (int c = threadIdx.x; c < n; c += 256) out[which * n + c] = comb[0][c] + comb[1][c] + comb[2][c] + comb[3][c];
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (col(i) < n)
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          out[col(i) + e] = sw[i][e];
+          out[n + col(i) + e] = sb[i][e];
+        }
+  }
 }
 
 // dw[c], db[c] = sums over the slices of part[slice][2][n]: a workgroup adds 64 columns, its 16 waves every 16th slice
@@ -522,6 +522,9 @@ using namespace flhip;
 
 extern "C" int flhip_layernorm_applies(int64_t n, int64_t rows, int dtype) {
   if (n <= 0 || rows <= 0 || rows > 0x7fffffffll || !dtype_ok(dtype)) return 0;
+  // a row of one element has nothing to sum: with many of them the general kernels are faster (forward / backward, 100000
+  // rows: 35 / 42 us there, 23 / 29 here; 1000000 rows: 35 / 68 there, 160 / 230 here)
+  if (n == 1 && rows > (1 << 17)) return 0;
   return n <= 1024 * 16 / (int64_t)dtype_size(dtype);      // four pieces per thread (the backward pass's registers)
 }
 
@@ -564,23 +567,14 @@ extern "C" int flhip_layernorm_bwd(const void* dy, const void* x, const float* w
   float* part = static_cast<float*>(ws);
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
-    constexpr int N = Piece<T>::N;
-    const bool whole = n % N == 0 && ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) |
-                                       reinterpret_cast<uintptr_t>(dx) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
-    const int pieces = (int)((n + N - 1) / N);
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)slices), dim3(256), 0, s, (const T*)dy, (const T*)x, w, mean, invstd, (T*)dx, part,
-                         (int)n, (int)rows, rps, scalar_params ? 0 : 1);
+    const bool whole = n % Piece<T>::N == 0 && ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) |
+                                                 reinterpret_cast<uintptr_t>(dx) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+    auto go = [&](auto th, auto np, auto ne) {
+      hipLaunchKernelGGL((layernorm_rows_bwd<T, th.value, np.value, ne.value>), dim3((unsigned)slices), dim3(256), 0, s, (const T*)dy,
+                         (const T*)x, w, mean, invstd, (T*)dx, part, (int)n, (int)rows, rps, scalar_params ? 0 : 1);
     };
-    if (whole) {
-      if (pieces <= 256) go(layernorm_rows_bwd<T, 1, true>);
-      else if (pieces <= 512) go(layernorm_rows_bwd<T, 2, true>);
-      else go(layernorm_rows_bwd<T, 4, true>);
-    } else {
-      if (pieces <= 256) go(layernorm_rows_bwd<T, 1, false>);
-      else if (pieces <= 512) go(layernorm_rows_bwd<T, 2, false>);
-      else go(layernorm_rows_bwd<T, 4, false>);
-    }
+    if (whole) by_row<T>((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, Piece<T>::N>{}); });
+    else by_element((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, 1>{}); });
   });
   if (const int rc = check_launch("layernorm_bwd")) return rc;
   float* cols = part + (size_t)slices * 2 * n;
