@@ -57,6 +57,17 @@ def test_convert_many_launch_split():
     assert plan([1 << 40])[0] == -1           # refused, like the call itself
 
 
+def test_layernorm_row_limits():
+    """Rows that the row kernels take: up to 16 KiB, and no more of them than their int row counters can step past."""
+    applies = capi.lib().flhip_layernorm_applies
+    assert applies(4096, 1, capi.F32) and not applies(4097, 1, capi.F32)
+    assert applies(8192, 1, capi.BF16) and not applies(8193, 1, capi.F16)
+    assert applies(2, 1 << 30, capi.BF16) and not applies(2, (1 << 30) + 1, capi.BF16)
+    assert not applies(2, (1 << 31) - 1, capi.BF16)
+    assert applies(1, 1 << 17, capi.F32) and not applies(1, (1 << 17) + 1, capi.F32)
+    assert not applies(0, 4, capi.F32) and not applies(4, 0, capi.F32) and not applies(4, 4, 17)
+
+
 def test_conv_out_dims_and_errors():
     lib = capi.lib()
     oh, ow = C.c_int32(), C.c_int32()
