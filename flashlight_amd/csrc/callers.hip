@@ -499,7 +499,7 @@ matmul_tn_skinny(const T* __restrict__ A, const T* __restrict__ B, T* __restrict
   if (mi < M && nj < N) st(C, (size_t)nj * M + mi, mine);
 }
 
-// ---- logSoftmax over dimension 0 of a C x X matrix (Functions.cpp:1044-1070), columns too long for registers (rows.hip) ----
+// ---- logSoftmax over dimension 0 of a C x X matrix (Functions.cpp:1044-1070), columns that rows.hip leaves ----
 // one wave per column
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -564,6 +564,27 @@ cce_fwd_kernel(const T* __restrict__ x, const int32_t* __restrict__ target, floa
     stats[1] = cnt;
     stats[2] = bad;
     stats[3] = s / cnt;
+  }
+}
+
+// columns of few classes (rows.hip takes the others): dx[c, col] = -(g_col) where c == target[col] and the column counts, else 0;
+// g_col = grad[0] / count (mean), grad[0] (sum) or grad[col] (none)
+template <typename T>
+__global__ void __launch_bounds__(256)
+cce_bwd_kernel(const float* __restrict__ grad, const int32_t* __restrict__ target,
+               const float* __restrict__ stats, T* __restrict__ dx, int Cn, int X, int reduction,
+               int ignore) {
+  const size_t total = (size_t)Cn * X;
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += stride) {
+    const int col = (int)(e / Cn), c = (int)(e - (size_t)col * Cn);
+    const int t = target[col];
+    float v = 0.f;
+    if (t != ignore && c == t) {
+      const float g = reduction == 0 ? grad[col] : reduction == 1 ? grad[0] / stats[1] : grad[0];
+      v = -g;
+    }
+    st(dx, e, v);
   }
 }
 
@@ -1193,7 +1214,14 @@ extern "C" int flhip_cce_bwd(const float* grad, const int32_t* target, const flo
   FLHIP_REQUIRE(classes > 0 && cols > 0, "cce_bwd: sizes must be positive");
   FLHIP_REQUIRE(reduction >= 0 && reduction <= 2, "cce_bwd: unknown reduction");
   FLHIP_REQUIRE(dtype_ok(dtype), "cce_bwd: unknown dtype");
-  rows_cce_bwd(grad, target, stats, dx, classes, cols, reduction, ignore_index, dtype, as_stream(stream));
+  if (!rows_cce_bwd(grad, target, stats, dx, classes, cols, reduction, ignore_index, dtype, as_stream(stream))) {
+    const size_t total = (size_t)classes * cols;
+    by_dtype(dtype, [&](auto* t_) {
+      using T = FLHIP_T_OF(t_);
+      hipLaunchKernelGGL((cce_bwd_kernel<T>), dim3(blocks_for(total)), dim3(256), 0, as_stream(stream), grad, target, stats, (T*)dx,
+                         classes, cols, reduction, ignore_index);
+    });
+  }
   return check_launch("cce_bwd");
 }
 

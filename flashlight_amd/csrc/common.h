@@ -301,10 +301,10 @@ struct Options {
 };
 const Options& options();
 
-// rows.hip: rows held in registers (false: the row does not fit)
+// rows.hip: rows held in registers (false: the row does not fit, or is so short that a lane per element is faster)
 bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hipStream_t s);
 bool rows_logsoftmax_bwd(const void* dy, const void* y, void* dx, int n, int rows, int dtype, hipStream_t s);
-void rows_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx, int n, int rows, int reduction,
+bool rows_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx, int n, int rows, int reduction,
                   int ignore, int dtype, hipStream_t s);
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }

@@ -325,6 +325,13 @@ def test_logsoftmax_and_cross_entropy_rows(classes, cols, dtype):
 
 
 @pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("classes", [79, 80, 159, 160, 383, 384])
+def test_logsoftmax_and_cross_entropy_between_elements_and_pieces(classes, dtype):
+    """The shortest rows that are held as pieces, and the longest that are not."""
+    test_logsoftmax_and_cross_entropy_rows(classes, 35, dtype)
+
+
+@pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("n,rows,scalar", [(1, 7, False), (7, 3, False), (8, 1, True), (512, 9, False), (520, 33, False), (1000, 130, True),
                                            (2000, 70, False), (2001, 5, False), (4096, 6, False), (8192, 3, False)])
 def test_layer_norm_rows(n, rows, scalar, dtype):
