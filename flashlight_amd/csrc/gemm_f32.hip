@@ -22,9 +22,12 @@
 // What bounds it is the matrix pipe, and the last round of tiles that does not fill the chip (128 x 128 tiles: 2048 x 6400 is
 // 3.1 tiles per compute unit, so at most 78 % of the pipe's 153 TFLOP/s).  Measured, us (before: the 1x1 convolution kernels
 // with a matrix as one image's plane, A * B^T on 64 x 64 tiles staged through registers, thin products on the vector ALUs):
-//   mode 0  2000 x 4000 x 2000  286 -> 244 (131 TFLOP/s)    1024 x 6400 x 2048  286 -> 264    1024 x 64 x 3136  42 -> 12
-//   mode 1  2000 x 4000 x 2000  268 -> 239                  3072 x 6400 x 1024  353 -> 314    3136 x 64 x 1024  30 -> 11
-//   mode 2  2000 x 2000 x 4000  287 -> 243                  512 x 2048 x 6400   187 -> 112    80 x 2048 x 6400  58 -> 32
+//   mode 0  2000 x 4000 x 2000  286 -> 240 (133 TFLOP/s)    1024 x 6400 x 2048  286 -> 237    1024 x 64 x 3136  42 -> 12
+//   mode 1  2000 x 4000 x 2000  268 -> 235                  3072 x 6400 x 1024  353 -> 297    3136 x 64 x 1024  30 -> 10
+//   mode 2  2000 x 2000 x 4000  287 -> 240                  512 x 2048 x 6400   187 -> 103    80 x 2048 x 6400  58 -> 31
+// Over a short contraction it is the stores of C: with lanes along C's contiguous dimension they are whole cache lines
+// wherever a column starts (lanes along the other one, 16 bytes each: mode 1, 9998 x 2000 x 64 81 -> 35 us, 2048 x 6000 x 64
+// 30 -> 21, 4002 x 132 x 20 5.9 -> 4.4; the 1x1 kernels: 40, 24, 4.5).
 #include <algorithm>
 
 #include "conv2d.h"
@@ -171,7 +174,7 @@ gemm32_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B
         for (int i = 0; i < RT; ++i)
 #pragma unroll
           for (int c = 0; c < CT; ++c)
-            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j][i][e], b[j][c][e], acc[i][c], 0, 0, 0);
+            acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][c][e], a[j][i][e], acc[i][c], 0, 0, 0);
   };
   int s = s0;
   // rounds of the ring whose look-ahead is whole stages
@@ -187,55 +190,51 @@ gemm32_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B
   }
   PD_WAIT_VM(0);                             // nothing may land in LDS after the workgroup has ended
 
-  // element r of a lane: row 8 (r / 4) + 4 h + r % 4, column fr of the instruction tile
-  float* out = C + (size_t)blockIdx.y * p.slice;
+  // B's columns are the rows of the instruction's tiles, so that the lanes of a store are neighbours along C's contiguous
+  // dimension, wherever its columns start: element r of a lane is column 8 (r / 4) + 4 h + r % 4 and row fr of C's tile
+  // (M is below 2^22: a tile's columns lie within 2 GiB.  A store past the last column is out of the buffer's range, one past the
+  // last row is put there, and so neither needs a branch around it.)
+  const int m = m0 + wm * 32 * RT + (AK ? fr : RT * fr);      // and 32 (AK) or one row further for the second tile
+  constexpr int MSTEP = AK ? 32 : 1;
+  const int nl = wn * 32 * CT + (BK ? 4 * h : CT * 4 * h);
+  const size_t origin = (size_t)n0 * p.M, left = ((size_t)(p.N - n0) * p.M) * 4;
+  const unsigned range = left < 0x7fffffffu ? (unsigned)left : 0x7fffffffu;
+  const __amdgpu_buffer_rsrc_t orsrc = make_rsrc(C + (size_t)blockIdx.y * p.slice + origin, range);
+  int at[RT];
+  float bv[RT];
 #pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int n = n0 + wn * 32 * CT + (BK ? c * 32 + fr : CT * fr + c);
-    if (n >= p.N) continue;
+  for (int i = 0; i < RT; ++i) {
+    const bool in = m + i * MSTEP < p.M;
+    at[i] = in ? (nl * p.M + m + i * MSTEP) * 4 : G32_OOB;
+    bv[i] = bias && in ? bias[m + i * MSTEP] : 0.f;
+  }
+  auto store = [&](auto added) __attribute__((always_inline)) {
+    constexpr bool ADD = decltype(added)::value;
+    const __amdgpu_buffer_rsrc_t arsrc = make_rsrc(ADD ? addend + origin : nullptr, range);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 8 * q + 4 * h;
-      if constexpr (AK || RT == 1) {
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          const int m = m0 + wm * 32 * RT + i * 32 + row;
-          if (m >= p.M) continue;
-          float v[4];
-#pragma unroll
-          for (int x = 0; x < 4; ++x) v[x] = acc[i][c][4 * q + x] + (bias && m + x < p.M ? bias[m + x] : 0.f);
-          float* at = out + (size_t)n * p.M + m;
-          if (addend) {
-#pragma unroll
-            for (int x = 0; x < 4; ++x)
-              if (m + x < p.M) v[x] += addend[(size_t)n * p.M + m + x];
+      for (int r = 0; r < 16; ++r) {
+        const int col = 8 * (r >> 2) + (r & 3), o = (BK ? c * 32 + col : CT * col + c) * p.M * 4;
+        if constexpr (RT == 2 && !AK) {          // (M is a multiple of 4)
+          float2 v = make_float2(acc[0][c][r] + bv[0], acc[1][c][r] + bv[1]);
+          if (ADD) {
+            const uintx2_t f = __builtin_amdgcn_raw_buffer_load_b64(arsrc, at[0] + o, 0, 0);
+            v.x += __uint_as_float(f.x); v.y += __uint_as_float(f.y);
           }
-          if (!AK || (p.M & 3) == 0) {
-            *reinterpret_cast<float4*>(at) = make_float4(v[0], v[1], v[2], v[3]);
-          } else {
+          __builtin_amdgcn_raw_buffer_store_b64(uintx2_t{__float_as_uint(v.x), __float_as_uint(v.y)}, orsrc, at[0] + o, 0, 0);
+        } else {
 #pragma unroll
-            for (int x = 0; x < 4; ++x)
-              if (m + x < p.M) at[x] = v[x];
+          for (int i = 0; i < RT; ++i) {
+            float v = acc[i][c][r] + bv[i];
+            if (ADD) v += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(arsrc, at[i] + o, 0, 0));
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), orsrc, at[i] + o, 0, 0);
           }
-        }
-      } else {                               // rows 2 r + t: eight neighbours of the two tiles (M is a multiple of 4)
-        const int m = m0 + wm * 64 + 2 * row;
-#pragma unroll
-        for (int x2 = 0; x2 < 2; ++x2) {
-          const int mm = m + 4 * x2;
-          if (mm >= p.M) continue;
-          float v[4];
-#pragma unroll
-          for (int x = 0; x < 4; ++x) v[x] = acc[x & 1][c][4 * q + 2 * x2 + (x >> 1)] + (bias ? bias[mm + x] : 0.f);
-          if (addend) {
-            const float4 f = *reinterpret_cast<const float4*>(addend + (size_t)n * p.M + mm);
-            v[0] += f.x; v[1] += f.y; v[2] += f.z; v[3] += f.w;
-          }
-          *reinterpret_cast<float4*>(out + (size_t)n * p.M + mm) = make_float4(v[0], v[1], v[2], v[3]);
         }
       }
-    }
-  }
+  };
+  if (addend) store(std::true_type{});
+  else store(std::false_type{});
 }
 
 // out = sum of the slices (+ bias[row]) (+ addend, which may be out); rows of M4 pieces, M a multiple of 4 where there is
@@ -273,7 +272,7 @@ bool gemm32_plan(int mode, int M, int N, int K, bool sliced, Gemm32Plan* best) {
   const bool ak = mode == 1, bk = mode != 2;
   if ((ak ? K : M) % 4 != 0 || (bk ? K : N) % 4 != 0) return false;      // rows of whole 16-byte pieces
   const long long ab = (long long)M * K * 4, bb = (long long)N * K * 4;
-  if (ab >= (1ll << 31) || bb >= (1ll << 31) || (long long)M * N >= (1ll << 31)) return false;
+  if (ab >= (1ll << 31) || bb >= (1ll << 31) || (long long)M * N >= (1ll << 31) || M >= 1 << 22) return false;
   const int cus = mfma_num_cus(), nst = (K + KC - 1) / KC;
   double best_cost = 1e30;
   for (int tm : {128, 64})

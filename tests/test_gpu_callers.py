@@ -241,6 +241,29 @@ def test_matmul_fp32_tiles(mode, M, N, K, bias):
         assert rel_l2(got, ref) <= 2 * (np.sqrt(K) + 1) * 2.0 ** -24, (nws, rel_l2(got, ref))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 129, 4), (3, 130, 20), (65, 132, 64), (130, 257, 128), (501, 300, 36), (127, 4, 2048), (1001, 133, 256)])
+def test_matmul_fp32_tiles_with_odd_rows(M, N, K):
+    """A^T * B where C's columns do not start on 16-byte boundaries."""
+    test_matmul_fp32_tiles(1, M, N, K, True)
+
+
+@pytest.mark.parametrize("M", [(1 << 22) - 4, 1 << 22])
+def test_matmul_fp32_of_very_many_rows(M):
+    """The most rows whose tiles' columns lie within 2 GiB, and one piece more."""
+    import ctypes as C
+
+    from flashlight_amd import capi
+    N, K = 8, 4
+    A, B = torch.randn(K, M, device="cuda"), torch.randn(K, N, device="cuda")
+    out = torch.full((N, M), float("nan"), device="cuda")
+    P = lambda t: C.c_void_p(t.data_ptr())
+    capi.check(capi.lib().flhip_matmul_ws(P(A), P(B), P(out), M, N, K, 0, 1, None, capi.F32, None, 0,
+                                          C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    # four products and their sum: at most 4 units of 2^-24 of the sum of their magnitudes
+    want, mag = (B.double().t() @ A.double()), B.abs().double().t() @ A.abs().double()
+    assert bool(((out.double() - want).abs() <= 4 * 2.0 ** -24 * mag).all())
+
+
 def test_matmul_fp32_at_the_size_of_a_speech_model():
     """2000 x 2000 weights against 4000 frames in fp32 (the plane mapping by shape), against numpy's float64 product."""
     M, N, K = 2000, 4000, 2000
