@@ -950,10 +950,23 @@ extern "C" size_t flhip_matmul_workspace_bytes(int32_t M, int32_t N, int32_t K, 
   return ns > 1 ? (size_t)ns * M * N * sizeof(float) : 0;
 }
 
+// A thin product A * B (N <= 128) in fp32: on gemm_f32.hip, in one slice or several, or on matmul_nn_skinny?  A round of
+// that kernel's workgroups over the chip takes about 4 us and 10.5 more per 1000 of the contraction, however few rows there are.
+// One slice of gemm_f32.hip: 512 x 64, K 64 / 128 / 256: 3.8 / 4.7 / 6.7 us (4.7 / 5.0 / 5.5); from a second round on it is the
+// faster one at every K (4096 x 64 x 256: 6.9, 7.3; 4096 x 128 x 256: 7.1, 12).  Slices: 512 x 64, K 512 / 768 / 1024: 7.4 / 7.3 / 8.0
+// (8.5 / 11.4 / 14.5), but the second launch and the workspace cost the host some 4 us, so that calls in a row come every 14 us
+// where this kernel's come every 11.5: worth it from where its rounds take longer than that (a little later for a single block of
+// columns: 12.8 us at K 1024).
+static bool thin_on_gemm32(int M, int N, int K, bool slices) {
+  const long long rounds = ((long long)((M + 63) / 64) * ((N + SK_NT - 1) / SK_NT) + 255) / 256;
+  return slices ? K >= (N <= SK_NT ? 1152 : 1024) || rounds * K >= 1408 : K <= 128 || rounds > 1;
+}
+
 extern "C" size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || (trans_a && trans_b)) return 0;
   if (trans_b || dtype != FLHIP_F32 || options().matmul_valu) return flhip_matmul_workspace_bytes(M, N, K, trans_a, trans_b, dtype);
-  return gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K);
+  const size_t need = gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K);
+  return !trans_a && N <= 128 && !thin_on_gemm32(M, N, K, need > 0) ? 0 : need;
 }
 
 extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
@@ -972,16 +985,15 @@ extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M,
   FLHIP_REQUIRE(A && B && C, "matmul: null argument");
   FLHIP_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "matmul: unknown dtype");
-  // fp32 on the kernels of gemm_f32.hip.  A thin product (a batch of feature vectors through fl::linear) is few tiles and
-  // takes them only with the workspace to cut its contraction (1024 x 64 x 3136: 12 us; the thin kernels 42, one slice 100)
+  // fp32 on the kernels of gemm_f32.hip.  A thin product (a batch of feature vectors through fl::linear) is few tiles: where
+  // these would cut its contraction, it takes them only with the workspace for that (1024 x 64 x 3136: 12 us; the thin kernels
+  // 42, one slice 100)
   const bool thin = N <= 128 && !trans_b;
   if (dtype == FLHIP_F32 && !(trans_a && trans_b) && !options().matmul_valu && options().matmul_planes < 0) {
-    const int mode = trans_a ? 1 : trans_b ? 2 : 0;
-    if (!thin || (ws ? ws_bytes : 0) >= gemm32_ws_bytes(mode, M, N, K)) {
-      const int rc = gemm32(mode, static_cast<const float*>(A), static_cast<const float*>(B), static_cast<float*>(C), M, N, K,
-                            bias_rows, ws, ws_bytes, as_stream(stream));
-      if (rc >= 0) return rc;
-    }
+    const int rc = gemm32(trans_a ? 1 : trans_b ? 2 : 0, static_cast<const float*>(A), static_cast<const float*>(B),
+                          static_cast<float*>(C), M, N, K, bias_rows, ws, ws_bytes, as_stream(stream), nullptr,
+                          !thin ? nullptr : trans_a ? [](int, int, int, bool) { return true; } : thin_on_gemm32);
+    if (rc >= 0) return rc;
   }
   // the other thin products: the kernels made for them
   if (N <= 128 && !trans_b && !options().matmul_valu) {

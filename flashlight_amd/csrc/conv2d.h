@@ -72,10 +72,11 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
                 const float* bias_rows, hipStream_t s, void* ws, size_t ws_bytes);
 size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K);
 // the three products in fp32 (gemm_f32.hip), + bias[row] + addend (C's layout, may be C), their contraction cut into slices
-// where gemm32_ws_bytes() of workspace are there; -1 where rows are not whole 16-byte pieces or a tensor is too large
+// where gemm32_ws_bytes() of workspace are there; -1 where rows are not whole 16-byte pieces or a tensor is too large, and,
+// with `take`, where the workspace is short or take(M, N, K, more than one slice) is false
 size_t gemm32_ws_bytes(int mode, int M, int N, int K);
 int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int K, const float* bias, void* ws,
-           size_t ws_bytes, hipStream_t s, const float* addend = nullptr);
+           size_t ws_bytes, hipStream_t s, const float* addend = nullptr, bool (*take)(int, int, int, bool) = nullptr);
 // column-major C = A * B^T on a kernel of its own (both operands contiguous along the
 // surviving dimension); slices > 1 (f32): partial products M * N floats apart
 int gemm_nt(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int slices, hipStream_t s);

@@ -26,8 +26,8 @@
 //   mode 1  2000 x 4000 x 2000  268 -> 235                  3072 x 6400 x 1024  353 -> 297    3136 x 64 x 1024  30 -> 10
 //   mode 2  2000 x 2000 x 4000  287 -> 240                  512 x 2048 x 6400   187 -> 103    80 x 2048 x 6400  58 -> 31
 // Over a short contraction it is the stores of C: with lanes along C's contiguous dimension they are whole cache lines
-// wherever a column starts (lanes along the other one, 16 bytes each: mode 1, 9998 x 2000 x 64 81 -> 35 us, 2048 x 6000 x 64
-// 30 -> 21, 4002 x 132 x 20 5.9 -> 4.4; the 1x1 kernels: 40, 24, 4.5).
+// wherever a column starts (lanes along the other one, 16 bytes each: mode 1, 9998 x 2000 x 64 81 -> 34 us, 2048 x 6000 x 64
+// 30 -> 21, 4002 x 132 x 20 5.8 -> 3.9; the 1x1 kernels: 40, 24, 4.5).
 #include <algorithm>
 
 #include "conv2d.h"
@@ -327,13 +327,16 @@ size_t gemm32_ws_bytes(int mode, int M, int N, int K) {
 }
 
 int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int K, const float* bias, void* ws, size_t ws_bytes,
-           hipStream_t s, const float* addend) {
+           hipStream_t s, const float* addend, bool (*take)(int, int, int, bool)) {
   Gemm32Plan pl{};
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) |
        reinterpret_cast<uintptr_t>(addend)) % 16 != 0)
     return -1;
-  if (!gemm32_plan(mode, M, N, K, ws != nullptr && (!bias || M % 4 == 0), &pl)) return -1;
-  if (pl.slices > 1 && ws_bytes < (size_t)pl.slices * M * N * sizeof(float) && !gemm32_plan(mode, M, N, K, false, &pl)) return -1;
+  const bool can = ws != nullptr && (!bias || M % 4 == 0);
+  if (!gemm32_plan(mode, M, N, K, can || take, &pl)) return -1;
+  const bool fits = can && ws_bytes >= (size_t)pl.slices * M * N * sizeof(float);
+  if (take && ((pl.slices > 1 && !fits) || !take(M, N, K, pl.slices > 1))) return -1;
+  if (pl.slices > 1 && !fits && !gemm32_plan(mode, M, N, K, false, &pl)) return -1;
   float* dst = pl.slices > 1 ? static_cast<float*>(ws) : C;
   const float *b = pl.slices > 1 ? nullptr : bias, *a = pl.slices > 1 ? nullptr : addend;
   const int rc = mode == 0 ? gemm32_tile<0>(pl, A, B, b, a, dst, s) : mode == 1 ? gemm32_tile<1>(pl, A, B, b, a, dst, s)

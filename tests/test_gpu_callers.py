@@ -247,6 +247,13 @@ def test_matmul_fp32_tiles_with_odd_rows(M, N, K):
     test_matmul_fp32_tiles(1, M, N, K, True)
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 64, 128), (512, 64, 132), (64, 8, 1148), (64, 8, 1152), (64, 9, 1020), (64, 9, 1024), (4096, 32, 132), (4096, 33, 132),
+                                   (4096, 64, 700), (4096, 64, 704)])
+def test_matmul_fp32_thin(M, N, K):
+    """Both sides of the lines between the kernels for few columns."""
+    test_matmul_fp32_tiles(0, M, N, K, True)
+
+
 @pytest.mark.parametrize("M", [(1 << 22) - 4, 1 << 22])
 def test_matmul_fp32_of_very_many_rows(M):
     """The most rows whose tiles' columns lie within 2 GiB, and one piece more."""
