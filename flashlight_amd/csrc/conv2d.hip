@@ -158,13 +158,28 @@ static bool tap2d_on(const ConvGeom& g, int dtype) {
   return (dtype == FLHIP_BF16 || dtype == FLHIP_F16) && g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
 }
 
+// 1x1 windows in fp32 with few tiles for their contraction: the thin kernels take about 8 us + 6 per 1000 source channels + 10 per million
+// weights (their copy), the 1x1 kernels 4 + 24 per 1000 source channels forward (3 + 21 over planes of whole 16-byte pieces) and
+// 5 + 31 (4 + 22) backward, where they do not cut the contraction, which the forward pass never does.  Measured, us, 1x1 kernels /
+// thin: forward over 7 x 7 256 -> 64 channels 10.6 / 8.9, 512 -> 1024 17.0 / 15.2, 2048 -> 512 52.6 / 31.3; over 4 x 4 256 -> 64 8.5 /
+// 8.6, 512 -> 1024 13.8 / 13.9, 1024 -> 512 24.0 / 16.9, 1024 -> 2048 25.8 / 32.3; backward over 7 x 7 from 256 to 64 channels 12.5 /
+// 8.8, from 512 to 1024 20.7 / 14.9, from 128 to 512 8.5 / 9.0 (1 x 1), and cut, from 1024 to 512 16.4 / 18.5, from 2048 to 512
+// 23.3 / 31.1.  Over more than 24 planes of one position a tile's loads touch as many cache lines (2048 -> 1000, 24 / 33 images:
+// 53.6 / 49.0, 54.0 / 61.2; 1024 -> 512, 33: 29.1 / 27.2).
+static bool thin_1x1(const ConvGeom& g, bool bwd, long long tiles) {
+  const long long src = bwd ? g.K : g.C, dst = bwd ? g.C : g.K;
+  if (tiles > src / 8 || src < 256 || dst > 2048) return false;
+  if (bwd) return mfma_pointwise_split_ws(g, FLHIP_F32, true) == 0;
+  if (g.H * g.W == 1 && g.N > 24 && dst > 512) return false;
+  return g.H * g.W % 4 ? src * (1830 - dst) > 400000 : src * (1500 - dst) > 530000;
+}
+
 // Few result tiles (of 32 channels x 32 positions): the thin kernels.  `first`: asked before the 3x3 slab and strip kernels, which
 // they beat up to two tiles per compute unit in fp32 (64 channels 56 x 56: 392 tiles 18.1 -> 15.9 us, 784 tiles 18.7 -> 22.3; 13 x 13
 // at batch 48, 508 tiles: 26 -> 18) and one in 16-bit storage (196 tiles 10.9 -> 9.0, 784 tiles 11.3 -> 13.0).  Not first: windows
 // those two do not take, where the tapped GEMM (64 x 64 tiles, fp32 arithmetic) lost at every size measured, 16-bit storage
 // by 2.5 to 9 (128 channels 28 x 28, one image: 68 -> 10 us; 256 channels 14 x 14 at batch 33: 176 -> 47), fp32 by 1.02 to 4 (5x5 over
-// 14 x 14, 64 -> 32 channels, backward-data: batch 1 62 -> 18, batch 512 253 -> 142).  1x1 windows: fp32 with few tiles for their contraction (2048 -> 512
-// over 7 x 7, 32 tiles: 52 -> 31, 112 tiles 54 -> 33; but 512 -> 2048, 128 tiles 17.6 -> 21.6).
+// 14 x 14, 64 -> 32 channels, backward-data: batch 1 62 -> 18, batch 512 253 -> 142).
 // Strided windows stay where they were: their forward pass leaves its gathered input to the filter gradient (16-bit storage) or
 // gives the same bits with and without a workspace (fp32).  So do fp32 forward passes of more than 9 taps (the small convnets'
 // 5x5): their bits, and with them the choices of the max pools behind them, stay what they were (36 -> 32 us at 784 tiles).
@@ -173,7 +188,7 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
   const bool lo = dtype != FLHIP_F32;
   if (g.sy != 1 || g.sx != 1 || (lo && (skip(SK_BF16) || algo_is(Options::ALGO_CONVERT)))) return false;
   const long long pos = (long long)g.N * (bwd ? g.H * g.W : g.OH * g.OW), tiles = (pos + 31) / 32 * (((bwd ? g.C : g.K) + 31) / 32);
-  if (g.KH * g.KW == 1) return first && !lo && tiles <= (bwd ? g.K : g.C) / 8;
+  if (g.KH * g.KW == 1) return first && !lo && thin_1x1(g, bwd, tiles);
   if (!lo && !bwd && g.KH * g.KW > 9) return false;
   return !first || tiles <= (lo ? 1 : 2) * (long long)mfma_num_cus();
 }

@@ -77,6 +77,15 @@ def test_thin_products_cut_only_long_contractions():
     assert ws(512, 64, 512, 1, 0, capi.F32) > 0                                                   # A^T * B: always the faster one
 
 
+@pytest.mark.parametrize("n,c,k,plane,thin", [(1, 256, 64, 7, True), (1, 256, 64, 4, False), (1, 2048, 512, 7, True), (1, 128, 512, 4, False),
+                                              (2, 512, 1024, 7, True), (2, 512, 1024, 4, False), (24, 2048, 1000, 1, True),
+                                              (25, 2048, 1000, 1, False), (1, 1024, 2048, 4, False)])
+def test_1x1_windows_with_few_tiles(n, c, k, plane, thin):
+    """Which fp32 forward passes of 1x1 windows take the kernels for few tiles (they copy the weights to the workspace)."""
+    d = capi.ConvDesc(n, c, plane, plane, k, 1, 1, 1, 1, 0, 0, 1, 1, 1, capi.F32)
+    assert (capi.lib().flhip_conv2d_workspace_bytes(C.byref(d), capi.CONV_FWD) > 0) == thin
+
+
 def test_conv_out_dims_and_errors():
     lib = capi.lib()
     oh, ow = C.c_int32(), C.c_int32()
