@@ -78,7 +78,7 @@ def test_thin_products_cut_only_long_contractions():
 
 
 @pytest.mark.parametrize("n,c,k,plane,thin", [(1, 256, 64, 7, True), (1, 256, 64, 4, False), (1, 2048, 512, 7, True), (1, 128, 512, 4, False),
-                                              (2, 512, 1024, 7, True), (2, 512, 1024, 4, False), (24, 2048, 1000, 1, True),
+                                              (1, 512, 1024, 7, True), (1, 512, 1024, 4, False), (24, 2048, 1000, 1, True),
                                               (25, 2048, 1000, 1, False), (1, 1024, 2048, 4, False)])
 def test_1x1_windows_with_few_tiles(n, c, k, plane, thin):
     """Which fp32 forward passes of 1x1 windows take the kernels for few tiles (they copy the weights to the workspace)."""
