@@ -369,9 +369,10 @@ __global__ void __launch_bounds__(256) rnn_cell_fwd(CellFwd a, int B, int H) {
 // One time step of up to two directions in one launch: recurrent product and gate math.
 // A workgroup owns four hidden units (blockIdx.x) of one direction (blockIdx.y): its
 // 16-row matrix-core tile is {gate g, unit hh} = row 4*g + hh of the recurrent
-// matrices, its columns are the batch (NBT tiles of 16, batch <= 64), and the eight
-// waves split the contraction over the hidden state in interleaved chunks of 16 (as the sequence
-// kernels do: a captured launch sequence and an eager one add in the same order).  A
+// matrices, its columns are the batch (NBT tiles of 16, batch <= 64), and the contraction
+// over the hidden state is split over eight groups in interleaved chunks of 16, whether four waves
+// or eight hold them (as the sequence kernels do: a captured launch sequence and an eager one add
+// in the same order).  A
 // lane's 16-byte load supplies the operands of four 16x16x4 products (the k index of a
 // lane group is permuted the same way on both operands).  The partial tiles meet in
 // LDS, then one thread per (batch, unit) applies the gates; those threads issue the
@@ -381,12 +382,13 @@ struct StepFwd {
   CellFwd d[2];
   int B, H;
 };
-constexpr int STEP_WAVES = 8;
+constexpr int STEP_GROUPS = 8;
+constexpr int step_fwd_chunks(int nbt) { return nbt == 4 ? 4 : 8; }      // in flight per wave
 
-template <int MODE, int NBT>
-__global__ void __launch_bounds__(64 * STEP_WAVES) rnn_step_fwd(StepFwd p) {
-  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16, W = STEP_WAVES;
-  __shared__ float red[W][16][NB + 1];
+template <int MODE, int NBT, int W>
+__global__ void __launch_bounds__(64 * W) rnn_step_fwd(StepFwd p) {
+  constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16, S = STEP_GROUPS / W;
+  __shared__ float red[STEP_GROUPS][16][NB + 1];
   const CellFwd& a = p.d[blockIdx.y];
   const int H = p.H, B = p.B, h0 = blockIdx.x * 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
@@ -405,12 +407,14 @@ __global__ void __launch_bounds__(64 * STEP_WAVES) rnn_step_fwd(StepFwd p) {
     bv[nt] = b < B;
     bp[nt] = a.hp + (size_t)(bv[nt] ? b : 0) * H + 4 * fg;
   }
-  floatx4_t acc[NBT];
+  floatx4_t acc[S][NBT];                  // group wave + W * s of the contraction: every S-th of the wave's chunks
 #pragma unroll
-  for (int nt = 0; nt < NBT; ++nt) acc[nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int nt = 0; nt < NBT; ++nt) acc[s][nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
   // U chunks are in flight per wave at a time: the loop is bound by the latency of
   // its loads, not by the products
-  constexpr int U = NBT == 4 ? 4 : 8;
+  constexpr int U = step_fwd_chunks(NBT);
   const int chunks = H >> 4;
   const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int c0 = wave; c0 < chunks; c0 += W * U) {
@@ -438,14 +442,17 @@ __global__ void __launch_bounds__(64 * STEP_WAVES) rnn_step_fwd(StepFwd p) {
       for (int nt = 0; nt < NBT; ++nt) {
         const float bv4[4] = {rb[u][nt].x, rb[u][nt].y, rb[u][nt].z, rb[u][nt].w};
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av4[m], bv4[m], acc[nt], 0, 0, 0);
+        for (int m = 0; m < 4; ++m)
+          acc[u % S][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av4[m], bv4[m], acc[u % S][nt], 0, 0, 0);
       }
     }
   }
 #pragma unroll
-  for (int nt = 0; nt < NBT; ++nt)
+  for (int s = 0; s < S; ++s)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[wave][4 * fg + r][nt * 16 + fr] = acc[nt][r];
+    for (int nt = 0; nt < NBT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave + W * s][4 * fg + r][nt * 16 + fr] = acc[s][nt][r];
   __syncthreads();
   if (cell) {
     const int hh = tid & 3;
@@ -454,7 +461,7 @@ __global__ void __launch_bounds__(64 * STEP_WAVES) rnn_step_fwd(StepFwd p) {
     for (int gq = 0; gq < G; ++gq) {
       float v = 0.f;
 #pragma unroll
-      for (int wv = 0; wv < W; ++wv) v += red[wv][gq * 4 + hh][cb];
+      for (int k = 0; k < STEP_GROUPS; ++k) v += red[k][gq * 4 + hh][cb];
       rp[gq] = v;
     }
     cell_fwd_finish<MODE>(a, cb, ch, H, cin, rp);
@@ -575,13 +582,13 @@ struct StepBwd {
   CellBwd d[2];
   int B, H;
 };
-constexpr int step_bwd_waves(int nbt) { return nbt == 4 ? 2 * STEP_WAVES : STEP_WAVES; }
+constexpr int step_bwd_waves(int nbt) { return nbt == 4 ? 2 * STEP_GROUPS : STEP_GROUPS; }
 
 template <int MODE, int NBT>
 __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, NB = NBT * 16;
   constexpr int NW = NBT == 4 ? 2 : NBT;      // batch tiles per wave
-  constexpr int KG = STEP_WAVES;              // wave groups along the contraction
+  constexpr int KG = STEP_GROUPS;             // wave groups along the contraction
   __shared__ float red[KG][16][NB + 1];
   const CellBwd& a = p.d[blockIdx.y];
   const int H = p.H, B = p.B, h0 = blockIdx.x * 16, GH = G * H;
@@ -675,7 +682,7 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 // All workgroups of the launch have to be resident at once: the launch is cooperative, and a launch covers as many
 // clusters as the compute units hold, the rest follow in further launches.  A wait that does not end (it would take a
 // device that lost workgroups) stops after RNN_SPINS loads; the wave then goes on with NaN, which reaches every output.
-constexpr int SEQ_WAVES = STEP_WAVES, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
+constexpr int SEQ_WAVES = STEP_GROUPS, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
 constexpr int RNN_SPINS = 1 << 22;
 constexpr int RNN_OOB = (int)0x80000000;
 constexpr int AUX_AGENT = 16;      // buffer loads: sc1, agent scope
@@ -1111,9 +1118,23 @@ int seq_bwd(const RnnGeom& g, SeqBwd& p, hipStream_t s) {
   return FLHIP_DECLINED;
 }
 
+// Four or eight waves to a workgroup of rnn_step_fwd: as many chunks are asked for as fill whole rounds of the workgroup (past
+// the last one, again), so the number with the smaller rounds wins where the other's ask for more (20 steps of an LSTM in a
+// captured graph, us with 4 / 8 waves: 512 units, 32 columns 164 / 221, two directions 192 / 246; 1536 units 33 % more with 8;
+// 640 units, 64 columns 17 % more).  Equal rounds: eight where they need only one and the chip holds a workgroup to a compute unit
+// (1024 units, 1 column 143 / 135, two directions 199 / 227; 512 units, 64 columns 238 / 225), else four.
+template <int NBT>
+bool step_fwd_eight(int H, int D) {
+  constexpr int U = step_fwd_chunks(NBT);
+  const int chunks = H / 16, four = (chunks + 4 * U - 1) / (4 * U), eight = (chunks + 8 * U - 1) / (8 * U);
+  return four == 2 * eight && eight == 1 && (NBT == 4 || D * H <= 1024);
+}
+
 template <int MODE, int NBT>
 void launch_step_fwd(const StepFwd& p, int D, hipStream_t s) {
-  hipLaunchKernelGGL((rnn_step_fwd<MODE, NBT>), dim3(p.H / 4, D), dim3(64 * STEP_WAVES), 0, s, p);
+  const dim3 grid(p.H / 4, D);
+  if (step_fwd_eight<NBT>(p.H, D)) hipLaunchKernelGGL((rnn_step_fwd<MODE, NBT, 8>), grid, dim3(512), 0, s, p);
+  else hipLaunchKernelGGL((rnn_step_fwd<MODE, NBT, 4>), grid, dim3(256), 0, s, p);
 }
 
 // one layer, all directions: per direction the input projection of all steps, then the recurrence: one launch for the whole

@@ -63,6 +63,48 @@ def test_capture_and_replay_matches_eager():
         assert torch.equal(rm_g, rm_e) and torch.equal(rv_g, rv_e)
 
 
+def _rnn_eager_and_captured(mode, H, L, bidir, B, T=5, I=24):
+    gen = torch.Generator(device="cuda").manual_seed(H + B)
+    D = 2 if bidir else 1
+    x = torch.randn(T, B, I, device="cuda", generator=gen)
+    w = torch.randn(ops.rnn_param_count(I, H, L, mode, bidir), device="cuda", generator=gen) / H ** 0.5
+    dy = torch.randn(T, B, D * H, device="cuda", generator=gen)
+    hx = torch.randn(L * D, B, H, device="cuda", generator=gen)
+    cx = torch.randn(L * D, B, H, device="cuda", generator=gen) if mode == ops.RNN_LSTM else None
+
+    def seq():
+        y, hy, cy, reserve = ops.rnn(x, hx, cx, w, H, L, mode, bidir)
+        return [t for t in (y, hy, cy) + tuple(ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)) if t is not None]
+
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        seq()
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = seq()
+    for it in range(3):
+        x.copy_(torch.randn(T, B, I, device="cuda", generator=gen))
+        want = [t.clone() for t in seq()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        yield want, outs
+
+
+@pytest.mark.parametrize("mode,H,bidir,B", [(ops.RNN_LSTM, 512, True, 33),     # four waves to a step's workgroup, three column tiles
+                                            (ops.RNN_GRU, 640, False, 16),     # eight waves
+                                            (ops.RNN_TANH, 320, True, 64),     # eight waves, four column tiles
+                                            (ops.RNN_RELU, 1024, True, 1),     # four waves, two rounds
+                                            (ops.RNN_LSTM, 16, False, 2)])     # one chunk
+def test_rnn_step_kernels_add_as_the_sequence_kernels_do(mode, H, bidir, B):
+    """Captured (a launch per step) and eager (a launch per sequence) give the same bits where the step kernels apply."""
+    for want, outs in _rnn_eager_and_captured(mode, H, 1, bidir, B):
+        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
 def test_rnn_capture_and_replay_matches_eager():
     dev = torch.device("cuda:0")
     gen = torch.Generator(device="cuda").manual_seed(9)
