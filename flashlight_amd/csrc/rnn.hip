@@ -17,6 +17,7 @@
 // Layouts follow Flashlight: x [input, B, T] column-major = memory [T][B][input], etc.
 // fp32 only; no dropout between layers (the closure's dropProb must be 0).
 #include <algorithm>
+#include <atomic>
 
 #include "common.h"
 #include "conv2d.h"
@@ -1053,7 +1054,7 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
 // (registers), a step's gates within what a buffer load addresses (2 GiB: an LSTM of 1024 units up to 131071
 // columns), a stream that is not being captured (a cooperative launch is not recorded)
 bool seq_applies(const RnnGeom& g, hipStream_t s) {
-  if (options().rnn_unfused || g.H % 4 != 0 || g.H > 1024 || (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31)) return false;
+  if (options().rnn_unfused || options().rnn_sequences == Options::SEQ_NEVER || g.H % 4 != 0 || g.H > 1024 || (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31)) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -1062,11 +1063,14 @@ bool seq_applies(const RnnGeom& g, hipStream_t s) {
   return st == hipStreamCaptureStatusNone;
 }
 
+std::atomic<uint64_t> g_seq_launches{0};
+
 // FLHIP_DECLINED where the runtime refuses the first launch (nothing has run then): the device does not hold it, or the
 // process gets no cooperative queue (a program started by a process that had launched cooperatively on the same card was
 // told 'illegal state'; by itself it launches)
 template <typename P>
 int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s) {
+  if (options().rnn_sequences == Options::SEQ_REFUSED) return FLHIP_DECLINED;
   if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return FLHIP_DECLINED;
   const int per = std::max(1, mfma_num_cus() / p.nwg);
   for (p.cluster0 = 0; p.cluster0 < clusters; p.cluster0 += per) {
@@ -1080,6 +1084,7 @@ int seq_launch(void (*kernel)(P), P& p, int clusters, size_t lds, hipStream_t s)
         return FLHIP_DECLINED;
       return fail(FLHIP_RUNTIME_ERROR, std::string("rnn: ") + hipGetErrorString(e));
     }
+    g_seq_launches.fetch_add(1, std::memory_order_relaxed);
   }
   return FLHIP_OK;
 }
@@ -1409,6 +1414,8 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
 }  // namespace flhip
 
 using namespace flhip;
+
+extern "C" uint64_t flhip_rnn_sequence_launches(void) { return g_seq_launches.load(std::memory_order_relaxed); }
 
 extern "C" size_t flhip_rnn_param_count(const flhip_rnn_desc* d) {
   RnnGeom g;

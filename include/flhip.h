@@ -126,9 +126,10 @@ const char* flhip_arch(void);
  * (value NULL restores the default; the FLHIP_ prefix on `name` is optional).  Not to be
  * called while another thread is inside the library.  Results stay within the stated
  * tolerances under every setting; the switches only choose between kernels.
- *   CONV_ALGO = direct | gather | tapped | convert | auto    CONV_SKIP = bf16,gemm1x1,slab,tapped,strip,first,wgrad128,pwdma,wd32,tap1d,cells,tap2d
+ *   CONV_ALGO = direct | gather | tapped | convert | auto    CONV_SKIP = bf16,gemm1x1,slab,tapped,strip,first,wgrad128,pwdma,wd32,tap1d,cells,tap2d,thin
  *   PW_PT = 2 | 4 | 8    PW16_PF = 0 | 1 | 2 | 4 | 8    CONV_STACK = 0 | 1 | 2 | 4 | 8    BN_ALGO = split | resident | auto
- *   SLAB_WAVES = 0 | 4 | 8
+ *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = never | refused | auto (a layer's recurrence in one launch: not tried | as if the runtime
+ *                   refused the launch | by shape)
  *   PW16_NO_TAPS, TAPPED_NO_REORDER, MATMUL_VALU, MATMUL_FP32_CORES, RNN_UNFUSED, TAP2D_ALL = 1 | 0
  *   MATMUL_PLANES = 0..7 (bit m: the fp32 product of form m - 0: A B, 1: A^T B, 2: A B^T - takes a matrix as one
  *                   image's plane whatever its shape; 0: never; unset: by shape)
@@ -595,6 +596,8 @@ int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void* w, const v
                   const void* dhy, const void* dcy, const void* reserve, size_t reserve_bytes,
                   void* dx, void* dhx, void* dcx, void* dw, void* workspace,
                   size_t workspace_bytes, void* stream);
+/* how many launches that hold a layer's whole recurrence this process has made so far */
+uint64_t flhip_rnn_sequence_launches(void);
 
 #ifdef __cplusplus
 }

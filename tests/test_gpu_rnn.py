@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from flashlight_amd import ops
+from flashlight_amd import capi, ops
 from gpu_util import dev, host
 from oracle import flref
 from refmath import rel_l2
@@ -78,7 +78,51 @@ def test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states):
     (flref.RNN_GRU, 6, 1028, 1, False, 2, 3, True),        # too wide: a launch per step
 ])
 def test_whole_sequence_launches(mode, I, H, L, bidir, T, B, states):
+    before = capi.lib().flhip_rnn_sequence_launches()
     test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states)
+    launches = capi.lib().flhip_rnn_sequence_launches() - before
+    clusters = (2 if bidir else 1) * -(-B // 16)
+    assert launches >= 2 * L if H <= 1024 else launches == 0
+    if (H, clusters) == (1000, 5):      # 63 workgroups each: four to the first launch, forward and backward
+        assert launches == 4
+
+
+@pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
+    (flref.RNN_LSTM, 12, 48, 3, True, 4, 20, True),        # the step kernels follow on the projections already made
+    (flref.RNN_GRU, 12, 512, 2, False, 3, 33, True),
+    (flref.RNN_RELU, 8, 64, 2, True, 5, 16, False),
+    (flref.RNN_TANH, 8, 16, 2, True, 1, 1, True),
+    (flref.RNN_LSTM, 7, 20, 2, True, 4, 9, True),          # a hidden size off 16, more than 64 columns: the two-kernel steps
+    (flref.RNN_GRU, 9, 500, 2, False, 3, 18, True),
+    (flref.RNN_LSTM, 5, 32, 2, True, 3, 70, True),
+    (flref.RNN_RELU, 8, 4, 2, False, 4, 5, False),
+])
+def test_refused_sequence_launches(mode, I, H, L, bidir, T, B, states):
+    """What runs where the runtime refuses a cooperative launch, after the initial states and the input projections have been
+    put in place for it: forward alone, backward alone, and both."""
+    before = capi.lib().flhip_rnn_sequence_launches()
+    try:
+        capi.set_option("RNN_SEQUENCES", "refused")
+        test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states)
+        assert capi.lib().flhip_rnn_sequence_launches() == before
+        x = torch.randn(T, B, I, device="cuda")
+        w = torch.randn(ops.rnn_param_count(I, H, L, mode, bidir), device="cuda") / H ** 0.5
+        dy = torch.randn(T, B, (2 if bidir else 1) * H, device="cuda")
+        run = {}
+        for fwd in ("refused", "auto"):
+            for bwd in ("refused", "auto"):
+                capi.set_option("RNN_SEQUENCES", fwd)
+                y, hy, cy, reserve = ops.rnn(x, None, None, w, H, L, mode, bidir)
+                capi.set_option("RNN_SEQUENCES", bwd)
+                run[fwd, bwd] = [t for t in (y, hy, cy) + tuple(ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)) if t is not None]
+        for got in run.values():
+            for a, b in zip(got, run["auto", "auto"]):
+                # the same sums in another order, through a few steps
+                assert rel_l2(host(a), host(b)) <= 1e-5
+                if H % 16 == 0 and B <= 64:
+                    assert torch.equal(a, b)
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
 
 
 @pytest.mark.parametrize("mode", MODES)
