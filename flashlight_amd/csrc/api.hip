@@ -90,6 +90,7 @@ static bool apply_option(Options& o, const char* name, const char* v) {
   if (!strcmp(name, "RNN_UNFUSED")) return flag(&o.rnn_unfused);
   if (!strcmp(name, "RNN_SEQUENCES")) {
     if (!v || !*v || !strcmp(v, "auto")) o.rnn_sequences = Options::SEQ_AUTO;
+    else if (!strcmp(v, "always")) o.rnn_sequences = Options::SEQ_ALWAYS;
     else if (!strcmp(v, "never")) o.rnn_sequences = Options::SEQ_NEVER;
     else if (!strcmp(v, "refused")) o.rnn_sequences = Options::SEQ_REFUSED;
     else return false;

@@ -7,8 +7,8 @@
 // GRU r, z, n with n = tanh(W_n x + b_Wn + r * (R_n h + b_Rn)), h' = (1-z)*n + z*h.
 //
 // Structure: the input projections of all time steps of a pseudo-layer are one matrix
-// product; the recurrence is one launch per layer where the hidden size allows, else a loop over
-// time of (recurrent product, gate kernel).
+// product; the recurrence is one launch per layer where the hidden size allows and the sequence
+// is long enough to gain by it, else a launch per step, or a loop over time of (recurrent product, gate kernel).
 // The products go through flhip_matmul (matrix cores where the shapes allow).  The
 // forward pass keeps, per pseudo-layer and in step order, the state before every step,
 // the gate activations and (GRU) R_n h + b_Rn in the reserve buffer; the backward pass
@@ -217,15 +217,6 @@ bool fused_applies(const RnnGeom& g) {
 __device__ __forceinline__ float sigm(float v) {
 #pragma clang fp contract(off)
   return 1.f / (1.f + expf(-v));
-}
-
-// bsum[q] = bW[q] + bR[q], except the GRU n gate, whose recurrent bias stays inside
-// r * (R_n h + b_Rn)
-__global__ void __launch_bounds__(256) rnn_bias_kernel(const float* __restrict__ bW, const float* __restrict__ bR,
-                                                       float* __restrict__ bsum, int GH, int H, int mode) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= GH) return;
-  bsum[q] = (mode == RNN_GRU && q >= 2 * H) ? bW[q] : bW[q] + bR[q];
 }
 
 // Dropout between layers: x[i] *= keep(i) / (1 - p) over the output sequence of `layer`, with the
@@ -946,8 +937,9 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   if (cell && MODE == RNN_LSTM && q.dcx) q.dcx[e] = dc;
 }
 
-// What a sequence launch finds in place: forward, per direction (blockIdx.y), the initial states, RNN_UNSET in the rows of
-// all steps' states, and the biases as rnn_bias_kernel makes them; backward, RNN_UNSET in all rows of dGR.
+// What a recurrence finds in place: forward, per direction (blockIdx.y), the initial states and the summed biases (the GRU's
+// n gate apart, whose recurrent bias stays inside r * (R_n h + b_Rn)), and for a sequence launch RNN_UNSET in the rows of all
+// steps' states; backward, RNN_UNSET in all rows of dGR.
 struct SeqInit {
   struct Dir {
     const float *hx, *cx, *bW, *bR;
@@ -968,6 +960,12 @@ __global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
   }
   for (size_t i = i0; i < (size_t)p.GH; i += stride)
     q.bsum[i] = (p.mode == RNN_GRU && i >= (size_t)2 * p.H) ? q.bW[i] : q.bW[i] + q.bR[i];
+}
+
+// one launch for all directions
+void launch_init(const SeqInit& p, int D, hipStream_t s) {
+  const size_t most = std::max<size_t>(std::max<size_t>(p.n / 4, p.BH), p.GH);
+  hipLaunchKernelGGL(rnn_seq_init_kernel, dim3((unsigned)std::min<size_t>((most + 255) / 256, 2048), D), dim3(256), 0, s, p);
 }
 
 inline unsigned nblocks(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -1016,15 +1014,12 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
   float* RP = XP + TB * g.GH;
   int kdummy;
   float* bsum = RP + (size_t)step_slices(g.GH, g.B, g.H, &kdummy) * g.B * g.GH;
-  hipLaunchKernelGGL(rnn_bias_kernel, dim3(nblocks(g.GH)), dim3(256), 0, s, w + o.bW, w + o.bR, bsum,
-                     (int)g.GH, g.H, g.mode);
+  SeqInit ip{};
+  ip.BH = g.BH; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+  ip.d[0] = {hx ? hx + (size_t)pl * g.BH : nullptr, cx ? cx + (size_t)pl * g.BH : nullptr, w + o.bW, w + o.bR, HP, CP, bsum};
+  launch_init(ip, 1, s);
   // XP [GH x TB] = W [GH x in] (row-major = a column-major in x GH matrix, transposed) * IN [in x TB]
   if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws))) return rc;
-  hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s, hx ? hx + (size_t)pl * g.BH : nullptr,
-                     HP, g.BH);
-  if (MODE == RNN_LSTM)
-    hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s,
-                       cx ? cx + (size_t)pl * g.BH : nullptr, CP, g.BH);
   for (int st = 0; st < g.T; ++st) {
     const int t = dir ? g.T - 1 - st : st;
     int nrp = 1;
@@ -1050,11 +1045,48 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
   return check_launch("rnn_fwd");
 }
 
+// hidden units per workgroup of rnn_seq_fwd: the fewest for which a layer's clusters fit the compute units
+int seq_units(const RnnGeom& g) {
+  const int clusters = g.D * ((g.B + SEQ_COLS - 1) / SEQ_COLS), cus = mfma_num_cus();
+  if (g.mode == RNN_LSTM || g.mode == RNN_GRU) {
+    if (clusters * ((g.H + 3) / 4) <= cus) return 4;
+    if (clusters * ((g.H + 7) / 8) <= cus) return 8;
+  }
+  return 16;
+}
+
+// Does a pass gain by sequence launches?  One costs some 20 us more than a step's launch does (the cooperative queue, on both
+// sides), and saves on each step, the more so the more a step has to do.  Sequence / steps, of the time:
+//   Against the step kernels, over 4 / 6 / 8 steps: LSTM of 128 units forward 1.07, 0.93, 0.80 with 16 columns, 0.94, 0.76, 0.65
+//   with 32, 0.92, 0.75, 0.64 with 64; of 512 units, two directions, 1.01, 1.00, 0.91 with 16, 0.86, 0.73, 0.66 with 64; of 1024 units,
+//   two directions, 32 columns, over 2 / 4 steps 0.99 and 0.80; GRU of 512 units, training, 16 columns 1.27, 1.09, 0.99.
+//   Against the two-kernel steps (two launches per step and direction), over 2 / 4 steps: LSTM of 512 units, 128 columns 0.71, 0.47;
+//   of 200 units 1.08, 0.84, ReLU of 200 units 1.13, 0.85; of 128 units, two directions 0.77, 0.56.
+//   Clusters beyond the compute units go in further launches, so that with many columns the estimates (us per step, from 32 to
+//   1024 units, ReLU to LSTM) decide: LSTM of 512 units over 20 steps, 256 columns (2 launches) 0.77, 512 columns (4) 1.19; 1024
+//   units, 256 columns (4) 1.23, backward 0.8.
+bool seq_pays(const RnnGeom& g, bool bwd) {
+  const int tiles = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+  if (fused_applies(g)) {
+    const int weight = g.D * g.H * tiles * (g.G == 1 ? 5 : 2 * g.G + 2) / 10;
+    return g.T >= (weight >= 3500 ? 3 : weight >= 1500 ? 4 : g.B > 32 ? 5 : weight >= 700 || g.B > 16 ? 6 : 8);
+  }
+  const int units = bwd ? 16 : seq_units(g), nwg = (g.H + units - 1) / units, per = std::max(1, mfma_num_cus() / nwg);
+  const int launches = (g.D * tiles + per - 1) / per;
+  if (launches == 1) return g.T >= (g.D == 2 || g.GH >= 1000 ? 2 : 3);
+  const double H = g.H, step = bwd ? 5.5 + H * (0.006 + 0.016 * g.G * (1.0 + g.B / 750.0)) : 5.0 + H * (0.012 + 0.0053 * g.G);
+  const double seq = bwd ? 1.6 + H * (0.0048 * g.G - 0.0003) : 1.1 + H * (0.0015 + 0.0019 * g.G);
+  return g.T * (g.D * step - launches * seq) > 22.0 * launches;
+}
+
 // ---- launching whole sequences: the hidden size a multiple of 4 (16-byte pieces of the state) and at most 1024
 // (registers), a step's gates within what a buffer load addresses (2 GiB: an LSTM of 1024 units up to 131071
 // columns), a stream that is not being captured (a cooperative launch is not recorded)
-bool seq_applies(const RnnGeom& g, hipStream_t s) {
-  if (options().rnn_unfused || options().rnn_sequences == Options::SEQ_NEVER || g.H % 4 != 0 || g.H > 1024 || (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31)) return false;
+bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
+  const int asked = options().rnn_sequences;
+  if (options().rnn_unfused || asked == Options::SEQ_NEVER || g.H % 4 != 0 || g.H > 1024 ||
+      (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31) || (asked == Options::SEQ_AUTO && !seq_pays(g, bwd)))
+    return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -1102,9 +1134,9 @@ int seq_fwd_hu(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
 template <int MODE>
 int seq_fwd(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
   if constexpr (MODE == RNN_LSTM || MODE == RNN_GRU) {
-    const int cus = mfma_num_cus(), clusters = g.D * p.groups;
-    if (clusters * ((g.H + 3) / 4) <= cus) return seq_fwd_hu<MODE, 4>(g, p, s);
-    if (clusters * ((g.H + 7) / 8) <= cus) return seq_fwd_hu<MODE, 8>(g, p, s);
+    const int units = seq_units(g);
+    if (units == 4) return seq_fwd_hu<MODE, 4>(g, p, s);
+    if (units == 8) return seq_fwd_hu<MODE, 8>(g, p, s);
   }
   return seq_fwd_hu<MODE, 16>(g, p, s);
 }
@@ -1149,56 +1181,36 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
                         const float* cx, float* out, float* hy, float* cy, float* res, float* ws, bool& seq, hipStream_t s) {
   const Reserve r = reserve_layout(g);
   const size_t TB = (size_t)g.T * g.B;
-  bool prepared = false;      // the initial states and the input projections are in place
+  // the initial states and the input projections
+  SeqInit ip{};
+  SeqFwd p{};
+  p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
+  p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+  ip.BH = g.BH; ip.n = seq ? (size_t)g.T * g.BH : 0; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+  for (int dir = 0; dir < g.D; ++dir) {
+    const int pl = l * g.D + dir;
+    const Offsets o = offsets(g, pl);
+    float* base = res + (size_t)pl * r.per_pl;
+    SeqFwd::Dir& q = p.d[dir];
+    q.xp = ws + (size_t)dir * TB * g.GH;
+    q.R = w + o.R; q.bRn = w + o.bR + 2 * g.H;
+    q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
+    q.out = out + (size_t)dir * g.H;
+    q.hy = hy + (size_t)pl * g.BH;
+    q.cy = cy && MODE == RNN_LSTM ? cy + (size_t)pl * g.BH : nullptr;
+    ip.d[dir] = {hx ? hx + (size_t)pl * g.BH : nullptr, cx ? cx + (size_t)pl * g.BH : nullptr, w + o.bW, w + o.bR, q.HP, q.CP,
+                 ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH};
+  }
+  launch_init(ip, g.D, s);
+  for (int dir = 0; dir < g.D; ++dir)
+    if (const int rc = mm(w + offsets(g, l * g.D + dir).W, in, const_cast<float*>(p.d[dir].xp), g.GH, TB, inl, 1, 0,
+                          ip.d[dir].bsum, s, scratch_of(g, ws)))
+      return rc;
   if (seq) {
-    SeqInit ip{};
-    SeqFwd p{};
-    p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
-    p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
-    ip.BH = g.BH; ip.n = (size_t)g.T * g.BH; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
-    for (int dir = 0; dir < g.D; ++dir) {
-      const int pl = l * g.D + dir;
-      const Offsets o = offsets(g, pl);
-      float* base = res + (size_t)pl * r.per_pl;
-      SeqFwd::Dir& q = p.d[dir];
-      q.xp = ws + (size_t)dir * TB * g.GH;
-      q.R = w + o.R; q.bRn = w + o.bR + 2 * g.H;
-      q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
-      q.out = out + (size_t)dir * g.H;
-      q.hy = hy + (size_t)pl * g.BH;
-      q.cy = cy && MODE == RNN_LSTM ? cy + (size_t)pl * g.BH : nullptr;
-      SeqInit::Dir& i = ip.d[dir];
-      i.hx = hx ? hx + (size_t)pl * g.BH : nullptr;
-      i.cx = cx ? cx + (size_t)pl * g.BH : nullptr;
-      i.bW = w + o.bW; i.bR = w + o.bR;
-      i.HP = q.HP; i.CP = q.CP;
-      i.bsum = ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH;
-    }
-    const unsigned blocks = (unsigned)std::min<size_t>((ip.n / 4 + 255) / 256, 2048);
-    hipLaunchKernelGGL(rnn_seq_init_kernel, dim3(std::max(1u, blocks), g.D), dim3(256), 0, s, ip);
-    for (int dir = 0; dir < g.D; ++dir)
-      if (const int rc = mm(w + offsets(g, l * g.D + dir).W, in, const_cast<float*>(p.d[dir].xp), g.GH, TB, inl, 1, 0,
-                            ip.d[dir].bsum, s, scratch_of(g, ws)))
-        return rc;
     const int rc = seq_fwd<MODE>(g, p, s);
     if (rc != FLHIP_DECLINED) return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
     seq = false;              // nor the layers that follow
     if (!fused_applies(g)) return FLHIP_DECLINED;
-    prepared = true;
-  }
-  for (int dir = 0; dir < g.D && !prepared; ++dir) {
-    const int pl = l * g.D + dir;
-    const Offsets o = offsets(g, pl);
-    float* XP = ws + (size_t)dir * TB * g.GH;
-    float* bsum = ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH;
-    hipLaunchKernelGGL(rnn_bias_kernel, dim3(nblocks(g.GH)), dim3(256), 0, s, w + o.bW, w + o.bR, bsum,
-                       (int)g.GH, g.H, g.mode);
-    if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws))) return rc;
-    hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s,
-                       hx ? hx + (size_t)pl * g.BH : nullptr, res + (size_t)pl * r.per_pl + r.hp, g.BH);
-    if (MODE == RNN_LSTM)
-      hipLaunchKernelGGL(rnn_init_kernel, dim3(nblocks(g.BH)), dim3(256), 0, s,
-                         cx ? cx + (size_t)pl * g.BH : nullptr, res + (size_t)pl * r.per_pl + r.cp, g.BH);
   }
   for (int st = 0; st < g.T; ++st) {
     StepFwd p{};
@@ -1330,7 +1342,7 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
       q.dcx = dcx ? dcx + (size_t)pl * g.BH : nullptr;
       ip.d[dir].HP = dGR[dir];
     }
-    hipLaunchKernelGGL(rnn_seq_init_kernel, dim3((unsigned)std::min<size_t>((ip.n / 4 + 255) / 256, 2048), g.D), dim3(256), 0, s, ip);
+    launch_init(ip, g.D, s);
     const int rc = seq_bwd<MODE>(g, p, s);
     if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
     seq = rc == FLHIP_OK;
@@ -1444,7 +1456,7 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
-  bool seq = seq_applies(g, s);
+  bool seq = seq_applies(g, false, s);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     float* out = l == g.L - 1 ? static_cast<float*>(y) : res + r.acts + (size_t)l * act;
@@ -1508,7 +1520,7 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   float* goutbuf = wsf + 2 * TB * g.GH;
   float* ginbuf = goutbuf + act;
   const float* gout = static_cast<const float*>(dy);   // gradient of the top layer's output (may be null)
-  bool seq = seq_applies(g, s);
+  bool seq = seq_applies(g, true, s);
   for (int l = g.L - 1; l >= 0; --l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;

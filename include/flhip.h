@@ -128,8 +128,8 @@ const char* flhip_arch(void);
  * tolerances under every setting; the switches only choose between kernels.
  *   CONV_ALGO = direct | gather | tapped | convert | auto    CONV_SKIP = bf16,gemm1x1,slab,tapped,strip,first,wgrad128,pwdma,wd32,tap1d,cells,tap2d,thin
  *   PW_PT = 2 | 4 | 8    PW16_PF = 0 | 1 | 2 | 4 | 8    CONV_STACK = 0 | 1 | 2 | 4 | 8    BN_ALGO = split | resident | auto
- *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = never | refused | auto (a layer's recurrence in one launch: not tried | as if the runtime
- *                   refused the launch | by shape)
+ *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = always | never | refused | auto (a layer's recurrence in one launch: wherever it can be |
+ *                   not tried | as if the runtime refused the launch | where it is the faster one)
  *   PW16_NO_TAPS, TAPPED_NO_REORDER, MATMUL_VALU, MATMUL_FP32_CORES, RNN_UNFUSED, TAP2D_ALL = 1 | 0
  *   MATMUL_PLANES = 0..7 (bit m: the fp32 product of form m - 0: A B, 1: A^T B, 2: A B^T - takes a matrix as one
  *                   image's plane whatever its shape; 0: never; unset: by shape)

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import flashlight_amd as fa
-from flashlight_amd import ops
+from flashlight_amd import capi, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -101,8 +101,12 @@ def _rnn_eager_and_captured(mode, H, L, bidir, B, T=5, I=24):
                                             (ops.RNN_LSTM, 16, False, 2)])     # one chunk
 def test_rnn_step_kernels_add_as_the_sequence_kernels_do(mode, H, bidir, B):
     """Captured (a launch per step) and eager (a launch per sequence) give the same bits where the step kernels apply."""
-    for want, outs in _rnn_eager_and_captured(mode, H, 1, bidir, B):
-        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+    capi.set_option("RNN_SEQUENCES", "always")       # (also over a few steps)
+    try:
+        for want, outs in _rnn_eager_and_captured(mode, H, 1, bidir, B):
+            assert all(torch.equal(a, b) for a, b in zip(outs, want))
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
 
 
 def test_rnn_capture_and_replay_matches_eager():

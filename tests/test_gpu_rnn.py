@@ -79,7 +79,11 @@ def test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states):
 ])
 def test_whole_sequence_launches(mode, I, H, L, bidir, T, B, states):
     before = capi.lib().flhip_rnn_sequence_launches()
-    test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states)
+    capi.set_option("RNN_SEQUENCES", "always")       # (also where the sequence is too short to gain by them)
+    try:
+        test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states)
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
     launches = capi.lib().flhip_rnn_sequence_launches() - before
     clusters = (2 if bidir else 1) * -(-B // 16)
     assert launches >= 2 * L if H <= 1024 else launches == 0
@@ -109,20 +113,53 @@ def test_refused_sequence_launches(mode, I, H, L, bidir, T, B, states):
         w = torch.randn(ops.rnn_param_count(I, H, L, mode, bidir), device="cuda") / H ** 0.5
         dy = torch.randn(T, B, (2 if bidir else 1) * H, device="cuda")
         run = {}
-        for fwd in ("refused", "auto"):
-            for bwd in ("refused", "auto"):
+        for fwd in ("refused", "always"):
+            for bwd in ("refused", "always"):
                 capi.set_option("RNN_SEQUENCES", fwd)
                 y, hy, cy, reserve = ops.rnn(x, None, None, w, H, L, mode, bidir)
                 capi.set_option("RNN_SEQUENCES", bwd)
                 run[fwd, bwd] = [t for t in (y, hy, cy) + tuple(ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)) if t is not None]
         for got in run.values():
-            for a, b in zip(got, run["auto", "auto"]):
+            for a, b in zip(got, run["always", "always"]):
                 # the same sums in another order, through a few steps
                 assert rel_l2(host(a), host(b)) <= 1e-5
                 if H % 16 == 0 and B <= 64:
                     assert torch.equal(a, b)
     finally:
         capi.set_option("RNN_SEQUENCES", None)
+
+
+@pytest.mark.parametrize("H,B,bidir,T,fwd,bwd", [
+    (64, 16, False, 7, 0, 0), (64, 16, False, 8, 1, 1), (64, 32, True, 5, 0, 0), (64, 32, True, 6, 1, 1),
+    (64, 33, False, 4, 0, 0), (64, 33, False, 5, 1, 1),
+    (512, 16, True, 5, 0, 0), (512, 16, True, 6, 1, 1), (1024, 20, True, 2, 0, 0), (1024, 20, True, 3, 1, 1),     # against a launch per step
+    (64, 65, False, 2, 0, 0), (64, 65, False, 3, 1, 1), (20, 4, True, 1, 0, 0), (20, 4, True, 2, 1, 1),
+    (512, 512, False, 4, 0, 0), (512, 512, False, 8, 0, 4),                    # four launches: backward alone
+])
+def test_where_sequence_launches_pay(H, B, bidir, T, fwd, bwd):
+    """Launches of the two passes on both sides of the lines between the kernels, and what they give against each other."""
+    gen = torch.Generator(device="cuda").manual_seed(H + B + T)
+    x = torch.randn(T, B, 16, device="cuda", generator=gen)
+    w = torch.randn(ops.rnn_param_count(16, H, 1, ops.RNN_LSTM, bidir), device="cuda", generator=gen) / H ** 0.5
+    dy = torch.randn(T, B, (2 if bidir else 1) * H, device="cuda", generator=gen)
+    count = capi.lib().flhip_rnn_sequence_launches
+
+    def run():
+        n = [count()]
+        y, hy, cy, reserve = ops.rnn(x, None, None, w, H, 1, ops.RNN_LSTM, bidir)
+        n.append(count())
+        out = (y, hy, cy) + tuple(ops.rnn_backward(x, w, reserve, H, 1, ops.RNN_LSTM, bidir, dy))
+        return out, n[1] - n[0], count() - n[1]
+    got, nf, nb = run()
+    assert (nf, nb) == (fwd, bwd)
+    try:
+        capi.set_option("RNN_SEQUENCES", "never" if fwd or bwd else "always")
+        want, nf, nb = run()
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
+    assert (nf > 0) == (fwd == bwd == 0)
+    for a, b in zip(got, want):
+        assert rel_l2(host(a), host(b)) <= 1e-5          # the same sums in another order
 
 
 @pytest.mark.parametrize("mode", MODES)
