@@ -96,13 +96,14 @@ static bool apply_option(Options& o, const char* name, const char* v) {
     else return false;
     return true;
   }
+  if (!strcmp(name, "RNN_WAIT")) { o.rnn_wait = v ? atoi(v) : def.rnn_wait; return true; }
   if (!strcmp(name, "TAP2D_ALL")) return flag(&o.tap2d_all);
   return false;
 }
 
 static void options_from_environment() {
   static const char* const names[] = {"CONV_ALGO", "CONV_SKIP", "PW_PT", "PW16_PF", "CONV_STACK", "SLAB_WAVES", "BN_ALGO", "PW16_NO_TAPS",
-                                      "TAPPED_NO_REORDER", "MATMUL_VALU", "MATMUL_FP32_CORES", "MATMUL_PLANES", "RNN_UNFUSED", "RNN_SEQUENCES", "TAP2D_ALL"};
+                                      "TAPPED_NO_REORDER", "MATMUL_VALU", "MATMUL_FP32_CORES", "MATMUL_PLANES", "RNN_UNFUSED", "RNN_SEQUENCES", "RNN_WAIT", "TAP2D_ALL"};
   for (const char* n : names) {
     const std::string var = std::string("FLHIP_") + n;
     if (const char* v = getenv(var.c_str())) apply_option(g_options, n, v);   // unknown values keep the default

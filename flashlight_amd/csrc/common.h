@@ -299,6 +299,8 @@ struct Options {
   enum { SEQ_AUTO = 0, SEQ_ALWAYS, SEQ_NEVER, SEQ_REFUSED };
   int rnn_sequences = SEQ_AUTO;   // RNN_SEQUENCES = auto | always (sequence launches wherever the kernels apply) | never | refused (tried wherever
                                   // they apply, as if the runtime refused each of them)
+  int rnn_wait = 1 << 22;         // RNN_WAIT: loads after which a wait inside a sequence launch gives up; negative: the first workgroup of every
+                                  // cluster gives up at its first wait
   bool tap2d_all = false;         // TAP2D_ALL: the kernel for 3x3 windows over stacked planes takes every geometry it can, not only those of its measured rule
   int bn_algo = 0;                // BN_ALGO = split (1) | resident (2)
 };

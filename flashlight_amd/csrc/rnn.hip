@@ -194,8 +194,10 @@ size_t workspace_core(const RnnGeom& g) {
   const size_t sf = step_slices(g.GH, g.B, g.H, &k);
   const size_t fwd = std::max(TB * g.GH + sf * g.B * g.GH + g.GH, (size_t)g.D * (TB * g.GH + g.GH));
   const size_t bwd = wgrad_scratch_offset(g) + wgrad_scratch(g);
-  return (std::max(fwd, bwd) + 67) & ~(size_t)3;
+  return ((std::max(fwd, bwd) + 67) & ~(size_t)3) + 4;
 }
+// whether a wait inside one of the call's sequence launches has given up (one word before the scratch)
+uint32_t* seq_status(const RnnGeom& g, float* ws) { return reinterpret_cast<uint32_t*>(ws + workspace_core(g) - 4); }
 Scratch scratch_of(const RnnGeom& g, float* ws) {
   const int TB = g.T * g.B, GH = (int)g.GH;
   size_t n = flhip_sum_columns_workspace_bytes(GH, TB, FLHIP_F32);
@@ -293,25 +295,26 @@ __device__ __forceinline__ CellFwdIn<MODE> cell_fwd_load(const CellFwd& a, int b
 
 // Values that another workgroup of the same launch waits for (the sequence kernels below): every element starts as
 // RNN_UNSET, a NaN that no element is stored as, and is written once, past the caches that the readers do not share.
-constexpr uint32_t RNN_UNSET = 0xffffffffu;
-__device__ __forceinline__ float rnn_value(float v) { return __float_as_uint(v) == RNN_UNSET ? __uint_as_float(0x7fc00000u) : v; }
-__device__ __forceinline__ void rnn_publish(float* p, float v) {
-  __hip_atomic_store(p, rnn_value(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// RNN_LOST, another one, is stored by a workgroup that has given up waiting.
+constexpr uint32_t RNN_UNSET = 0xffffffffu, RNN_LOST = 0xfffffffeu;
+__device__ __forceinline__ float rnn_value(float v) { return __float_as_uint(v) >= RNN_LOST ? __uint_as_float(0x7fc00000u) : v; }
+__device__ __forceinline__ void rnn_publish(float* p, float v, bool lost) {
+  __hip_atomic_store(p, lost ? __uint_as_float(RNN_LOST) : rnn_value(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // SEQ: the state goes to the other workgroups of the launch; returns what the element's thread keeps for the next step
-// (LSTM: c, else h)
+// (LSTM: c, else h).  lost (rp is NaN then): so are the state and what follows from it, also where the ReLU of a NaN is zero
 template <int MODE, bool SEQ = false>
 __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h, int H, const CellFwdIn<MODE>& in,
-                                                 const float* rp) {
+                                                 const float* rp, bool lost = false) {
 #pragma clang fp contract(off)
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
   const size_t e = (size_t)b * H + h, q = (size_t)b * G * H + h;
   float hv, keep = 0.f;
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float pre = in.xp[0] + rp[0];
-    hv = MODE == RNN_RELU ? (pre > 0.f ? pre : 0.f) : tanhf(pre);
-    if (SEQ) rnn_publish(a.hn + e, hv);
+    hv = MODE == RNN_RELU ? (pre > 0.f || (SEQ && lost) ? pre : 0.f) : tanhf(pre);
+    if (SEQ) rnn_publish(a.hn + e, hv, lost);
     a.gt[q] = hv;
   } else if (MODE == RNN_LSTM) {
     const float ig = sigm(in.xp[0] + rp[0]), fg = sigm(in.xp[G > 1 ? 1 : 0] + rp[G > 1 ? 1 : 0]);
@@ -319,7 +322,7 @@ __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h,
     const float c = fmaf(fg, in.prev, ig * gg);
     keep = c;
     hv = og * tanhf(c);
-    if (SEQ) rnn_publish(a.hn + e, hv);
+    if (SEQ) rnn_publish(a.hn + e, hv, lost);
     a.cn[e] = c;
     if (a.cy) a.cy[e] = c;
     a.gt[q] = ig; a.gt[q + H] = fg; a.gt[q + 2 * H] = gg; a.gt[q + 3 * H] = og;
@@ -329,7 +332,7 @@ __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h,
     const float ng = tanhf(fmaf(rg, rn, in.xp[G > 2 ? 2 : 0]));
     hv = fmaf(1.f - zg, ng, zg * in.prev);
     keep = hv;
-    if (SEQ) rnn_publish(a.hn + e, hv);
+    if (SEQ) rnn_publish(a.hn + e, hv, lost);
     a.rn[e] = rn;
     a.gt[q] = rg; a.gt[q + H] = zg; a.gt[q + 2 * H] = ng;
   }
@@ -509,13 +512,13 @@ __device__ __forceinline__ CellBwdIn<MODE> cell_bwd_load(const CellBwd& a, int b
 }
 
 // SEQ: the recurrent-side gradients go to the other workgroups of the launch, and what the element's thread hands to its
-// next step stays in *dc and *dir
+// next step stays in *dc and *dir.  lost: as in the forward pass (rec is NaN)
 template <int MODE, bool SEQ = false>
 __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, int H, const CellBwdIn<MODE>& in,
-                                                float rec, float* dc_out = nullptr, float* dir_out = nullptr) {
+                                                float rec, float* dc_out = nullptr, float* dir_out = nullptr, bool lost = false) {
 #pragma clang fp contract(off)
   auto put = [&](size_t i, float v) {
-    if (SEQ) rnn_publish(a.dgr + i, v);
+    if (SEQ) rnn_publish(a.dgr + i, v, lost);
     else a.dgr[i] = v;
   };
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
@@ -524,7 +527,7 @@ __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, 
   float direct = 0.f;
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float hv = in.gt[0];
-    const float gp = MODE == RNN_RELU ? (hv > 0.f ? go : 0.f) : go * fmaf(-hv, hv, 1.f);
+    const float gp = MODE == RNN_RELU ? (hv > 0.f || (SEQ && lost) ? go : 0.f) : go * fmaf(-hv, hv, 1.f);
     put(q, gp);
     a.dgw[q] = gp;
   } else if (MODE == RNN_LSTM) {
@@ -673,9 +676,10 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 //
 // All workgroups of the launch have to be resident at once: the launch is cooperative, and a launch covers as many
 // clusters as the compute units hold, the rest follow in further launches.  A wait that does not end (it would take a
-// device that lost workgroups) stops after RNN_SPINS loads; the wave then goes on with NaN, which reaches every output.
+// device that lost workgroups) stops after RNN_WAIT loads, some seconds.  Its workgroup then goes on with NaN in every mode
+// and stores RNN_LOST for the others, which do the same from their next step on, and sets a word in the workspace with which
+// the launches of the call's other layers begin; so every output that depends on the missing values is NaN.
 constexpr int SEQ_WAVES = STEP_GROUPS, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
-constexpr int RNN_SPINS = 1 << 22;
 constexpr int RNN_OOB = (int)0x80000000;
 constexpr int AUX_AGENT = 16;      // buffer loads: sc1, agent scope
 
@@ -688,6 +692,46 @@ struct SeqFwd {
   int groups;        // of 16 batch columns
   int nwg;           // workgroups of a cluster
   int cluster0;      // first cluster of this launch; cluster = direction * groups + group
+  int wait;          // options().rnn_wait
+  uint32_t* status;  // the layer (from 1) whose launch first gave up
+  uint32_t layer;
+};
+
+// What a wave knows of waits that gave up.  One that has (dead) leaves NaN in its partial sums, and so in all elements of its
+// workgroup and, from the next step on, of its cluster.  ReLU layers turn a NaN sum into zero: there a word per wave in LDS tells
+// the threads of the elements, and RNN_LOST the other workgroups.
+struct SeqLost {
+  int* flags;
+  uint32_t *status, layer;
+  int limit;         // loads of a wait; negative: give up at once
+  // before: *status.  -> whether another layer's launch has given up (what this layer's other clusters do is no matter: they don't
+  // depend on each other, and a word that another layer has set is left as it is)
+  template <bool FLAGS>
+  __device__ __forceinline__ int begin(uint32_t before, bool first) {
+    before = __builtin_amdgcn_readfirstlane(before);
+    const int dead = before != 0 && before != layer;
+    if (limit < 0 && !first) limit = 1 << 22;
+    if (dead) status = nullptr;
+    if (FLAGS) flags[threadIdx.x >> 6] = dead;
+    return dead;
+  }
+  template <bool FLAGS, int N>
+  __device__ __forceinline__ void tell(int dead, floatx4_t (&acc)[N]) const {
+    if (__builtin_expect(dead, 0)) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] = floatx4_t{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+      if (FLAGS) flags[threadIdx.x >> 6] = 1;
+      if (status && (threadIdx.x & 63) == 0) __hip_atomic_store(status, layer, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  template <bool FLAGS>
+  __device__ __forceinline__ bool any() const {
+    int f = 0;
+    if (FLAGS)
+#pragma unroll
+      for (int w = 0; w < SEQ_WAVES; ++w) f |= flags[w];
+    return f != 0;
+  }
 };
 
 // every load so far has arrived: what a loop carries from before it then needs no wait inside it (that wait would be one
@@ -712,19 +756,24 @@ __device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const int (&o
   for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, AUX_AGENT);
 }
 template <int N>
-__device__ __forceinline__ bool seq_unset(const uintx4_t (&v)[N]) {
-  uint32_t m = 0;                    // (RNN_UNSET is the largest word)
+__device__ __forceinline__ uint32_t seq_largest(const uintx4_t (&v)[N]) {
+  uint32_t m = 0;                    // (RNN_UNSET is the largest word, RNN_LOST the next)
 #pragma unroll
   for (int i = 0; i < N; ++i) m = max(max(m, max(v[i].x, v[i].y)), max(v[i].z, v[i].w));
-  return __builtin_amdgcn_ballot_w64(m == RNN_UNSET) != 0;
+  return m;
 }
-// Repeats the loads until every element is set.  -> whether the wave has given up, now or before (dead)
+// Repeats the loads until every element is set.  -> whether the wave goes on without: it has given up, now or before (dead), or
+// the owner of an element has
 template <int N>
-__device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], int dead) {
-  if (__builtin_amdgcn_readfirstlane(dead) || !seq_unset(v)) return dead;
-  for (int spin = 0; spin < RNN_SPINS; ++spin) {
+__device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], int dead, int limit) {
+  if (__builtin_amdgcn_readfirstlane(dead) || limit < 0) return 1;
+  uint32_t m = seq_largest(v);
+  if (__builtin_amdgcn_ballot_w64(m >= RNN_LOST) == 0) return 0;
+  for (int spin = 0; spin < limit; ++spin) {
+    if (__builtin_amdgcn_ballot_w64(m == RNN_UNSET) == 0) return 1;
     seq_load(r, off, v);
-    if (!seq_unset(v)) return 0;
+    m = seq_largest(v);
+    if (__builtin_amdgcn_ballot_w64(m >= RNN_LOST) == 0) return 0;
   }
   return 1;
 }
@@ -736,7 +785,10 @@ __device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const int (&of
 template <int MODE, int HU, int NC>
 __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, RT = (G * HU + 15) / 16, W = SEQ_WAVES;
+  constexpr bool FLAGS = MODE == RNN_RELU;
   extern __shared__ float seq_red[];      // [2][W][16 RT][17]
+  __shared__ int seq_lost[W];
+  const uint32_t status = *p.status;
   const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * HU;
   const int dir = __builtin_amdgcn_readfirstlane(cluster / p.groups), b0 = (cluster - dir * p.groups) * SEQ_COLS;
   const SeqFwd::Dir q = dir ? p.d[1] : p.d[0];
@@ -768,7 +820,8 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   float keep = 0.f;
   if (cell) keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? HP[e] : 0.f;
   seq_drain();
-  int dead = 0;
+  SeqLost lost{seq_lost, p.status, p.layer, p.wait};
+  int dead = lost.begin<FLAGS>(status, h0 == 0);
   for (int sv = 0; sv < T; ++sv) {
     const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
     c.xp = q.xp + (size_t)t * B * GH;
@@ -783,7 +836,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
     const __amdgpu_buffer_rsrc_t r = make_rsrc(HP + st * BH, (unsigned)(BH * 4));
     uintx4_t v[NC];
     seq_load(r, off, v);
-    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v, dead));
+    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v, dead, lost.limit));
     seq_drain();
     floatx4_t acc[RT];
 #pragma unroll
@@ -796,6 +849,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
             acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][i][m], __uint_as_float(v[i][m]), acc[rt], 0, 0, 0);
+    lost.tell<FLAGS>(dead, acc);
     float* red = seq_red + (st & 1) * (W * RT * 16 * 17);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -803,6 +857,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
       for (int x = 0; x < 4; ++x) red[(wave * RT * 16 + rt * 16 + 4 * fg + x) * 17 + fr] = acc[rt][x];
     __syncthreads();
     if (cell) {
+      const bool gone = lost.any<FLAGS>();
       float rp[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -818,7 +873,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
       c.out = q.out + (size_t)t * B * p.ldo;
       c.hy = st == T - 1 ? q.hy : nullptr;
       c.cy = st == T - 1 ? q.cy : nullptr;
-      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp);
+      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp, gone);
     }
   }
 }
@@ -829,7 +884,8 @@ struct SeqBwd {
     float *dGW, *dGR, *dhx, *dcx;
   } d[2];
   int B, H, T, ldo;
-  int groups, nwg, cluster0;
+  int groups, nwg, cluster0, wait;
+  uint32_t *status, layer;
 };
 
 // The same for the backward pass: a workgroup owns 16 hidden units (rows of one tile: columns of the recurrent matrices,
@@ -838,7 +894,10 @@ struct SeqBwd {
 template <int MODE, int NC>
 __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1, W = SEQ_WAVES, U = NC < 8 ? NC : 8, NB = NC / U;
+  constexpr bool FLAGS = MODE == RNN_RELU;
   __shared__ float red2[2][W][16][17];
+  __shared__ int seq_lost[W];
+  const uint32_t status = *p.status;
   const int cl = blockIdx.x / p.nwg, cluster = p.cluster0 + cl, h0 = (blockIdx.x - cl * p.nwg) * 16;
   const int dir = __builtin_amdgcn_readfirstlane(cluster / p.groups), b0 = (cluster - dir * p.groups) * SEQ_COLS;
   const SeqBwd::Dir q = dir ? p.d[1] : p.d[0];
@@ -868,7 +927,9 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   CellBwd c{};
   c.ldo = p.ldo;
   float direct = cell && q.dhy ? q.dhy[e] : 0.f, dc = cell && MODE == RNN_LSTM && q.dcy ? q.dcy[e] : 0.f;
-  int dead = 0;
+  SeqLost lost{seq_lost, p.status, p.layer, p.wait};
+  int dead = lost.begin<FLAGS>(status, h0 == 0);
+  if (dead) direct = __builtin_nanf("");          // (the first step waits for nobody)
   seq_drain();
   for (int sv = T - 1; sv >= (q.dhx ? -1 : 0); --sv) {
     const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
@@ -889,7 +950,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
     if (st < T - 1) {
       seq_pause<8>();
       const __amdgpu_buffer_rsrc_t r = make_rsrc(dGR + (size_t)(st + 1) * B * GH, (unsigned)((size_t)B * GH * 4));
-      floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+      floatx4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
       uintx4_t v[2][U];
       {
         int off[U];
@@ -904,20 +965,22 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
           seq_load(r, off, v[(b + 1) & 1]);
         }
         offsets_of(b, off);
-        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v[b & 1], dead));
+        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v[b & 1], dead, lost.limit));
         if (b == NB - 1) seq_drain();
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if ((wave + W * (b * U + u)) * 16 < GH)
 #pragma unroll
             for (int m = 0; m < 4; ++m)
-              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b * U + u][m], __uint_as_float(v[b & 1][u][m]), acc, 0, 0, 0);
+              acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b * U + u][m], __uint_as_float(v[b & 1][u][m]), acc[0], 0, 0, 0);
       }
+      lost.tell<FLAGS>(dead, acc);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) red[wave][4 * fg + x][fr] = acc[x];
+      for (int x = 0; x < 4; ++x) red[wave][4 * fg + x][fr] = acc[0][x];
       __syncthreads();
     }
     if (cell) {
+      const bool gone = st < T - 1 ? lost.any<FLAGS>() : dead;      // (the flags are there from the first barrier on)
       float rec = 0.f;
       if (st < T - 1) {
 #pragma unroll
@@ -930,7 +993,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
         in.dc = dc;
         c.dgw = q.dGW + (size_t)t * B * GH;
         c.dgr = dGR + (size_t)st * B * GH;
-        cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct);
+        cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct, gone);
       }
     }
   }
@@ -947,11 +1010,13 @@ struct SeqInit {
   } d[2];
   size_t BH, n;       // elements of a state / of the rows to be filled
   int GH, H, mode;
+  uint32_t* status;   // to be cleared, or null
 };
 __global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
   const SeqInit::Dir& q = p.d[blockIdx.y];
   const size_t stride = (size_t)gridDim.x * 256, i0 = (size_t)blockIdx.x * 256 + threadIdx.x;
   const uintx4_t unset = {RNN_UNSET, RNN_UNSET, RNN_UNSET, RNN_UNSET};
+  if (p.status && blockIdx.y == 0 && i0 == 0) *p.status = 0;
   for (size_t i = i0; i < p.n / 4; i += stride) reinterpret_cast<uintx4_t*>(q.HP + p.BH)[i] = unset;
   if (p.BH == 0) return;                      // backward: nothing but the fill
   for (size_t i = i0; i < p.BH; i += stride) {
@@ -1186,7 +1251,9 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
   SeqFwd p{};
   p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
   p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+  p.wait = options().rnn_wait; p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
   ip.BH = g.BH; ip.n = seq ? (size_t)g.T * g.BH : 0; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+  ip.status = l == 0 ? p.status : nullptr;
   for (int dir = 0; dir < g.D; ++dir) {
     const int pl = l * g.D + dir;
     const Offsets o = offsets(g, pl);
@@ -1327,7 +1394,9 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
     SeqBwd p{};
     p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
     p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+    p.wait = options().rnn_wait; p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
     ip.n = TB * g.GH;
+    ip.status = l == g.L - 1 ? p.status : nullptr;
     for (int dir = 0; dir < g.D; ++dir) {
       const int pl = l * g.D + dir;
       const float* base = res + (size_t)pl * r.per_pl;

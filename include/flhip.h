@@ -130,6 +130,8 @@ const char* flhip_arch(void);
  *   PW_PT = 2 | 4 | 8    PW16_PF = 0 | 1 | 2 | 4 | 8    CONV_STACK = 0 | 1 | 2 | 4 | 8    BN_ALGO = split | resident | auto
  *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = always | never | refused | auto (a layer's recurrence in one launch: wherever it can be |
  *                   not tried | as if the runtime refused the launch | where it is the faster one)
+ *   RNN_WAIT = n (loads after which a wait inside such a launch gives up and its results become NaN; negative: the first
+ *                   workgroups give up at once)
  *   PW16_NO_TAPS, TAPPED_NO_REORDER, MATMUL_VALU, MATMUL_FP32_CORES, RNN_UNFUSED, TAP2D_ALL = 1 | 0
  *   MATMUL_PLANES = 0..7 (bit m: the fp32 product of form m - 0: A B, 1: A^T B, 2: A B^T - takes a matrix as one
  *                   image's plane whatever its shape; 0: never; unset: by shape)

@@ -176,6 +176,45 @@ def test_not_a_number_states_end(mode):
     assert bool(torch.isnan(dw).any()) and dx.shape == x.shape
 
 
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("L,bidir", [(1, False), (2, True)])
+def test_a_wait_that_gives_up_ends_in_not_a_number(mode, L, bidir):
+    """The first workgroup of every cluster stops waiting at once (the others run as ever, and all end): every output that
+    depends on what it did not wait for is NaN, in ReLU layers too and in the layers above; the next call is as ever."""
+    T, B, I, H, D = 5, 20, 8, 64, 2 if bidir else 1
+    gen = torch.Generator(device="cuda").manual_seed(mode)
+    x = torch.randn(T, B, I, device="cuda", generator=gen)
+    w = torch.randn(ops.rnn_param_count(I, H, L, mode, bidir), device="cuda", generator=gen) / H ** 0.5
+    dy = torch.randn(T, B, D * H, device="cuda", generator=gen)
+    nan = lambda t: bool(torch.isnan(t).all())
+    fine = lambda t: bool(torch.isfinite(t).all())
+
+    def forward():
+        return ops.rnn(x, None, None, w, H, L, mode, bidir)
+    try:
+        capi.set_option("RNN_SEQUENCES", "always")
+        y0, hy0, _, reserve = forward()
+        d0 = ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)
+        capi.set_option("RNN_WAIT", "-1")
+        y, hy, cy, _ = forward()
+        assert nan(hy) and (cy is None or nan(cy))
+        if L == 1:                                  # the first step of the other workgroups needs nobody else
+            units = torch.isnan(y[0]).all(0)
+            assert 0 < int(units.sum()) < H and bool(units[0]) and fine(y[0][:, ~units]) and nan(y[1:])
+        else:
+            assert nan(y)
+        dx, dhx, dcx, dw = ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)
+        assert nan(dhx) and nan(dw) and (dcx is None or nan(dcx))
+        assert nan(dx[:-1]) if L == 1 else nan(dx)
+        capi.set_option("RNN_WAIT", None)
+        y, hy, _, reserve = forward()
+        d = ops.rnn_backward(x, w, reserve, H, L, mode, bidir, dy)
+        assert torch.equal(y, y0) and torch.equal(hy, hy0) and torch.equal(d[0], d0[0]) and torch.equal(d[3], d0[3])
+    finally:
+        capi.set_option("RNN_WAIT", None)
+        capi.set_option("RNN_SEQUENCES", None)
+
+
 def test_two_streams_at_once():
     """Sequences issued on two streams without waiting for each other give what they give alone."""
     T, B, I, H = 30, 32, 64, 512
