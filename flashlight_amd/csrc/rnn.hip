@@ -270,8 +270,9 @@ struct CellFwd {
   int ldo;
 };
 
-// (The gate math below leaves no choice of fused or separate multiply-adds to the compiler: the step kernels of a captured
-// sequence and the sequence kernels give the same bits.)
+// (The gate math below leaves no choice of fused or separate multiply-adds to the compiler, and the step kernels add in the
+// sequence kernels' order: hidden sizes that are multiples of 16 with at most 64 columns give the same bits captured and eager.
+// The two-kernel steps, which others run on where a sequence launch is not made, add their products in another order.)
 // gate math of one (batch b, hidden h) element, in two halves so that a kernel can issue
 // the loads before it computes the recurrent projections rp (one per gate)
 template <int MODE>

@@ -109,6 +109,20 @@ def test_rnn_step_kernels_add_as_the_sequence_kernels_do(mode, H, bidir, B):
         capi.set_option("RNN_SEQUENCES", None)
 
 
+@pytest.mark.parametrize("mode,H,bidir,B", [(ops.RNN_LSTM, 20, True, 7), (ops.RNN_GRU, 500, False, 18), (ops.RNN_LSTM, 32, True, 70),
+                                            (ops.RNN_RELU, 100, False, 3)])
+def test_rnn_capture_off_the_step_kernels(mode, H, bidir, B):
+    """A hidden size off 16, or more than 64 columns: captured, the two-kernel steps add in another order than the sequence
+    kernels (a few units of 2^-24 per sum, over five steps and their backward pass)."""
+    capi.set_option("RNN_SEQUENCES", "always")
+    try:
+        for want, outs in _rnn_eager_and_captured(mode, H, 2, bidir, B):
+            for a, b in zip(outs, want):
+                assert float((a - b).norm() / b.norm()) <= 1e-5
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
+
+
 def test_rnn_capture_and_replay_matches_eager():
     dev = torch.device("cuda:0")
     gen = torch.Generator(device="cuda").manual_seed(9)
