@@ -994,11 +994,18 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   }
   p.tsplit = (g.OW + p.TL - 1) / p.TL;
   p.units = p.rows * p.tsplit;
-  // ranges per workgroup.  16-bit storage: never more workgroups than compute units, since each more range writes its
-  // partial tiles (6.3 MB over 250 -> 250 channels) and the reduction reads them (7 x 1111 frames, 448 -> 224 workgroups: 76 -> 66 us,
-  // 24 x 400 frames of 128 channels, 384 -> 192: 41 -> 36; but 16 x 1500 of 128 channels, 256 -> 128: 42 -> 52).  fp32 is bound by the
+  // ranges per workgroup.  16-bit storage: no more workgroups than compute units, since each more range writes its
+  // partial tiles (6.3 MB over 250 -> 250 channels and 21 taps) and the reduction reads them (us with more / no more of them: 7 x 1111
+  // frames, 448 / 224 workgroups 67 / 58, 24 x 400 frames of 128 channels, 384 / 192: 38 / 35).  But windows of up to 11 taps have few
+  // partial tiles and leave registers for two workgroups on a compute unit: where all of them run at once, a long range each is
+  // faster than two in a row on half the chip (9 x 1184 frames, 128 -> 200 channels, 6 taps, 288 / 144: 32 / 40; 9 x 1208, 128 ->
+  // 250, 9 taps 28 / 32; 17 x 985 stride 2, 80 -> 384, 8 taps, 306 / 162: 37 / 42), a short one is not (ranges of 208 to 368
+  // frames: 0.88 to 1.04 of the time on no more; from 416 frames on 1.0 to 1.3, at worst 0.93; twice the compute units
+  // exactly, 16 x 549 frames, 250 -> 250, 6 taps: 0.84).  fp32 is bound by the
   // matrix pipe, and rather has a last round that is half full than workgroups of twice the length
-  p.upw = esz == 2 ? (p.units - 1) / std::max(1, mfma_num_cus() / tiles) + 1 : std::max(1, p.units / std::max(1, want));
+  const int cus = mfma_num_cus();
+  const bool two = TQ <= 3 && p.TL > 400 && pl->lds_bytes <= 80 * 1024 && (long long)p.units * tiles < 2 * cus;
+  p.upw = esz == 4 ? std::max(1, p.units / std::max(1, want)) : two ? 1 : (p.units - 1) / std::max(1, cus / tiles) + 1;
   pl->nsplit = (p.units + p.upw - 1) / p.upw;
   const long long rb = (long long)p.rows * p.TS * p.Cs * esz;
   const long long yb = (long long)g.N * g.K * g.H * g.OW * esz;

@@ -686,7 +686,8 @@ def test_one_row_filter_gradient_from_the_forward_pass_rows(shape, dtype):
                                    ((2, 250, 1, 111), (250, 250, 1, 21), 1, 10),   # the speech window, filter and channel tails
                                    ((3, 33, 2, 181), (150, 33, 1, 11), 2, 5),      # two rows per image, stride 2
                                    ((1, 32, 1, 23), (32, 32, 1, 23), 1, 11),       # one row, shorter than a range
-                                   ((2, 96, 1, 998), (40, 96, 1, 16), 1, 8)])      # several ranges per row
+                                   ((2, 96, 1, 998), (40, 96, 1, 16), 1, 8),       # several ranges per row
+                                   ((257, 17, 1, 410), (33, 17, 1, 6), 1, 3)])     # a range per workgroup, more of them than compute units
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_one_row_filter_gradient_over_odd_rows(shape, dtype, shift):
