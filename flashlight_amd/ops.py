@@ -602,6 +602,8 @@ def linear_backward(grad_output, input, weight, want_bias=True):
     g, x, w = _dev(grad_output, "gradOutput"), _dev(input, "input"), _dev(weight, "weight")
     fin, fout = w.shape
     frames = x.numel() // fin
+    if x.numel() != frames * fin or g.numel() != frames * fout or not g.dtype == x.dtype == w.dtype:
+        raise ValueError("linear backward: gradOutput [.., out], input [.., in] and weight [in, out] of one type expected")
     tag = _dtype_tag(x)
     dx = torch.empty_like(x)
     nws = capi.lib().flhip_matmul_slices_bytes(fin, frames, fout, 1, 0, tag)

@@ -54,6 +54,16 @@ def test_linear(fin, fout, batch, dtype):
     assert rel_l2(host(db), flref.sum_columns(fout, batch, dy)) <= 1e-5
 
 
+def test_linear_backward_refuses_operands_that_do_not_belong_together():
+    """Raised on the host, before anything is launched: the products would read past the smaller operand."""
+    z = lambda *s, dt=torch.float32: torch.zeros(s, device="cuda", dtype=dt)
+    for g, x, w in ((z(5, 232), z(5, 692), z(232, 692)),                       # the weight as [out, in]
+                    (z(4, 232), z(5, 692), z(692, 232)), (z(5, 231), z(5, 692), z(692, 232)),
+                    (z(5, 232), z(5, 691), z(692, 232)), (z(5, 232, dt=torch.bfloat16), z(5, 692), z(692, 232))):
+        with pytest.raises(ValueError):
+            ops.linear_backward(g, x, w)
+
+
 @pytest.mark.parametrize("M,N,K", [(5, 7, 3), (64, 64, 16), (70, 33, 129), (1, 9, 200), (130, 67, 300)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("with_bias", [False, True])
