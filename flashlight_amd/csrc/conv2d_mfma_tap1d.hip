@@ -39,6 +39,8 @@
 // Positions are the rows of the instruction tile: a lane holds 4 consecutive positions of one
 // result channel (8 with two phases), stored as one piece.
 #include <algorithm>
+#include <cmath>
+#include <cmath>
 #include <cstring>
 
 #include "conv2d_mfma.h"
@@ -980,36 +982,61 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   if (!p.Cs) return false;
   p.K = g.K; p.C = g.C; p.KW = g.KW; p.px = g.px;
   p.ktiles = (g.K + 63) / 64; p.ctiles = (g.C + 31) / 32;
-  const int tiles = p.ktiles * p.ctiles;
-  const int PC = esz == 2 ? (g.sx == 1 ? 6 : 5) : 9;
-  // ranges: enough workgroups for the chip; a range's slab must fit in LDS
-  const int want = (mfma_num_cus() + tiles - 1) / tiles;
-  int tsplit = std::max(1, (want + p.rows - 1) / p.rows);
-  for (;; ++tsplit) {
-    p.TL = ((g.OW + tsplit - 1) / tsplit + 15) / 16 * 16;
-    p.SRW = (p.TL - 1) * g.sx + 4 * TQ;
-    pl->lds_bytes = (size_t)(((long long)p.SRW * PC + 63) / 64) * 1024;
-    if (pl->lds_bytes <= 150 * 1024) break;
-    if (p.TL <= 16) return false;
-  }
-  p.tsplit = (g.OW + p.TL - 1) / p.TL;
-  p.units = p.rows * p.tsplit;
-  // ranges per workgroup.  16-bit storage: no more workgroups than compute units, since each more range writes its
-  // partial tiles (6.3 MB over 250 -> 250 channels and 21 taps) and the reduction reads them (us with more / no more of them: 7 x 1111
-  // frames, 448 / 224 workgroups 67 / 58, 24 x 400 frames of 128 channels, 384 / 192: 38 / 35).  But windows of up to 11 taps have few
-  // partial tiles and leave registers for two workgroups on a compute unit: where all of them run at once, a long range each is
-  // faster than two in a row on half the chip (9 x 1184 frames, 128 -> 200 channels, 6 taps, 288 / 144: 32 / 40; 9 x 1208, 128 ->
-  // 250, 9 taps 28 / 32; 17 x 985 stride 2, 80 -> 384, 8 taps, 306 / 162: 37 / 42), a short one is not (ranges of 208 to 368
-  // frames: 0.88 to 1.04 of the time on no more; from 416 frames on 1.0 to 1.3, at worst 0.93; twice the compute units
-  // exactly, 16 x 549 frames, 250 -> 250, 6 taps: 0.84).  fp32 is bound by the
-  // matrix pipe, and rather has a last round that is half full than workgroups of twice the length
-  const int cus = mfma_num_cus();
-  const bool two = TQ <= 3 && p.TL > 400 && pl->lds_bytes <= 80 * 1024 && (long long)p.units * tiles < 2 * cus;
-  p.upw = esz == 4 ? std::max(1, p.units / std::max(1, want)) : two ? 1 : (p.units - 1) / std::max(1, cus / tiles) + 1;
-  pl->nsplit = (p.units + p.upw - 1) / p.upw;
   const long long rb = (long long)p.rows * p.TS * p.Cs * esz;
   const long long yb = (long long)g.N * g.K * g.H * g.OW * esz;
   if (rb >= (1ll << 31) || yb >= (1ll << 31)) return false;
+  const int tiles = p.ktiles * p.ctiles;
+  const int PC = esz == 2 ? (g.sx == 1 ? 6 : 5) : 9;
+  const int cus = mfma_num_cus();
+  // ranges of ceil(OW / tsplit) positions; false: the slab of one does not fit in LDS
+  auto split = [&](int tsplit) {
+    p.TL = ((g.OW + tsplit - 1) / tsplit + 15) / 16 * 16;
+    p.SRW = (p.TL - 1) * g.sx + 4 * TQ;
+    pl->lds_bytes = (size_t)(((long long)p.SRW * PC + 63) / 64) * 1024;
+    p.tsplit = (g.OW + p.TL - 1) / p.TL;
+    p.units = p.rows * p.tsplit;
+    return pl->lds_bytes <= 150 * 1024;
+  };
+  if (esz == 4) {
+    // fp32 is bound by the matrix pipe: enough workgroups for the chip, rather with a last round that is half full than of
+    // twice the length
+    const int want = (cus + tiles - 1) / tiles;
+    for (int tsplit = std::max(1, (want + p.rows - 1) / p.rows); !split(tsplit); ++tsplit)
+      if (p.TL <= 16) return false;
+    p.upw = std::max(1, p.units / want);
+  } else {
+    // 16-bit storage is bound by what surrounds the products.  The length of a range and the ranges per workgroup with the least
+    // estimated time: a workgroup's ranges follow each other, about 1 us each and 0.012 + 0.002 per four taps for a position; its partial
+    // tiles (TQ times 32 KB, written and read) take 0.013 us per four taps of the whole, and the reduction 0.05 for each that it adds.
+    // No more workgroups than compute units, but for windows of up to 11 taps, whose registers leave room for two on a unit:
+    // up to twice as many with one range each, of which those that share a unit take 1.2 times as long.  (Constants fitted to
+    // 14292 times of 1175 random geometries; taking the estimate's choice costs 1 % over the best of those measured, at worst 15.
+    // Filling the chip whatever the partial tiles cost, as before, 19 %, at worst 126: 16 -> 64 channels over 31 x 193 frames, 7 taps,
+    // 27 -> 13 us; 64 -> 40 over 4 x 1017, 15 taps, stride 2, 30 -> 14; 250 -> 250 over 7 x 1111, 21 taps, 57.)
+    double best = 1e30;
+    int best_split = 0, best_upw = 0;
+    const double set = 0.013 * TQ * tiles + 0.05;
+    for (int tsplit = 1;; tsplit += std::max(1, tsplit / 4)) {
+      const bool fits = split(tsplit);
+      const double each = 1.0 + p.TL * (0.012 + 0.002 * TQ);
+      auto consider = [&](int upw, double slower) {
+        const double cost = (double)((p.units + upw - 1) / upw) * set + upw * each * slower;
+        if (cost < best) { best = cost; best_split = tsplit; best_upw = upw; }
+      };
+      if (fits) {
+        const int least = (p.units - 1) / std::max(1, cus / tiles) + 1;
+        const int upw = (int)std::sqrt(p.units * set / each);
+        consider(std::max(least, upw), 1.0);
+        consider(std::max(least, upw + 1), 1.0);
+        if (TQ <= 3 && pl->lds_bytes <= 80 * 1024 && least == 2 && (long long)p.units * tiles < 2 * cus) consider(1, 1.2);
+      }
+      if (p.TL <= 16) break;
+    }
+    if (!best_split) return false;
+    split(best_split);
+    p.upw = best_upw;
+  }
+  pl->nsplit = (p.units + p.upw - 1) / p.upw;
   p.src_bytes = (unsigned)rb; p.dy_bytes = (unsigned)yb;
   pl->rows_bytes = ((size_t)rb + 255) & ~(size_t)255;
   pl->part_bytes = (size_t)pl->nsplit * tiles * (4 * TQ) * 2048 * sizeof(float);

@@ -87,13 +87,16 @@ def test_1x1_windows_with_few_tiles(n, c, k, plane, thin):
 
 
 @pytest.mark.parametrize("n,c,t,k,kw,stride,dtype,parts", [
-    (9, 160, 1031, 200, 8, 1, capi.BF16, 360), (9, 128, 1208, 250, 9, 1, capi.F16, 288), (17, 80, 985, 384, 8, 2, capi.BF16, 306),
-    (9, 64, 603, 100, 9, 1, capi.BF16, 144), (7, 250, 1111, 250, 21, 1, capi.BF16, 224), (16, 128, 1500, 128, 21, 1, capi.BF16, 256)])
+    (31, 16, 193, 64, 7, 1, capi.BF16, 31), (4, 64, 1017, 40, 15, 2, capi.F16, 32), (9, 64, 603, 100, 9, 1, capi.BF16, 72),
+    (17, 97, 400, 193, 6, 1, capi.F16, 272), (17, 80, 985, 384, 8, 2, capi.BF16, 306), (7, 250, 1111, 250, 21, 1, capi.BF16, 224),
+    (16, 128, 1500, 128, 21, 1, capi.BF16, 256), (7, 80, 200, 250, 21, 1, capi.F32, 336)])
 def test_one_row_filter_gradient_partial_tiles(n, c, t, k, kw, stride, dtype, parts):
     """How many partial tiles (one per workgroup) the filter gradient of one-row windows leaves in its workspace, behind the
-    channels-last rows: more than the 256 compute units only for long ranges and few taps."""
+    channels-last rows: as many as their own cost is worth, in 16-bit storage more than the 256 compute units only for long
+    ranges and few taps."""
     d = capi.ConvDesc(n, c, 1, t, k, 1, kw, 1, stride, 0, kw // 2, 1, 1, 1, dtype)
-    rows = (n * t * (96 if c == 80 else 64 if c == 64 else 128 if c == 128 else 256) * 2 + 255) // 256 * 256
+    cs = min(v for v in (32, 64, 96, 128, 256) if c <= v)
+    rows = (n * t * cs * (4 if dtype == capi.F32 else 2) + 255) // 256 * 256
     tile = (kw + 4) // 4 * 4 * 2048 * 4
     assert capi.lib().flhip_conv2d_workspace_bytes(C.byref(d), capi.CONV_BWD_FILTER) == rows + parts * tile
 

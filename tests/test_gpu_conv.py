@@ -687,7 +687,8 @@ def test_one_row_filter_gradient_from_the_forward_pass_rows(shape, dtype):
                                    ((3, 33, 2, 181), (150, 33, 1, 11), 2, 5),      # two rows per image, stride 2
                                    ((1, 32, 1, 23), (32, 32, 1, 23), 1, 11),       # one row, shorter than a range
                                    ((2, 96, 1, 998), (40, 96, 1, 16), 1, 8),       # several ranges per row
-                                   ((257, 17, 1, 410), (33, 17, 1, 6), 1, 3)])     # a range per workgroup, more of them than compute units
+                                   ((17, 97, 1, 400), (193, 97, 1, 6), 1, 3),      # a range per workgroup, more of them than compute units
+                                   ((31, 16, 1, 193), (64, 16, 1, 7), 1, 3)])      # ranges of whole rows, few partial tiles
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_one_row_filter_gradient_over_odd_rows(shape, dtype, shift):
