@@ -68,6 +68,13 @@ def test_layernorm_row_limits():
     assert not applies(0, 4, capi.F32) and not applies(4, 0, capi.F32) and not applies(4, 4, 17)
 
 
+def test_layernorm_backward_slices():
+    """Partial sums of the backward pass (and one more row of them): a workgroup to each of few long rows."""
+    ws = capi.lib().flhip_layernorm_bwd_workspace_bytes
+    for n, rows, slices in ((6590, 5, 5), (2000, 4000, 512), (1025, 30, 30), (1024, 30, 7), (29, 3, 1)):
+        assert ws(n, rows, capi.F16) == (slices + 1) * 2 * n * 4, (n, rows)
+
+
 def test_thin_products_cut_only_long_contractions():
     """Workspace for the slices of A * B with few columns: only where a second launch pays for itself."""
     ws = capi.lib().flhip_matmul_slices_bytes
