@@ -962,6 +962,15 @@ static bool thin_on_gemm32(int M, int N, int K, bool slices) {
   return slices ? K >= (N <= SK_NT ? 1152 : 1024) || rounds * K >= 1408 : K <= 128 || rounds > 1;
 }
 
+// The same for A^T * B and matmul_tn_skinny.  Slices, and one slice where it is short, always win; but a C of M * N elements that are
+// not whole 16-byte pieces is not cut, and one slice then takes 3 us and 15 per 1000 of the contraction, that kernel 7 us, 3.5 per
+// 1000 and the more the larger C is (us here / there: 23 x 9 x 384 8.4 / 8.2, x 512 10.6 / 9.2, x 1024 18 / 11; 2049 x 127 x 512
+// 11 / 27; 1043 x 63 x 640 12.7 / 14.2, x 1024 18.8 / 18.7; 1043 x 2 x 2128 30 / 13).
+static bool thin_tn_on_gemm32(int M, int N, int K, bool slices) {
+  const long long mn = (long long)M * N;
+  return slices || mn % 4 == 0 || K <= 384 + mn / 200;
+}
+
 extern "C" size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || (trans_a && trans_b)) return 0;
   if (trans_b || dtype != FLHIP_F32 || options().matmul_valu) return flhip_matmul_workspace_bytes(M, N, K, trans_a, trans_b, dtype);
@@ -992,7 +1001,7 @@ extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M,
   if (dtype == FLHIP_F32 && !(trans_a && trans_b) && !options().matmul_valu && options().matmul_planes < 0) {
     const int rc = gemm32(trans_a ? 1 : trans_b ? 2 : 0, static_cast<const float*>(A), static_cast<const float*>(B),
                           static_cast<float*>(C), M, N, K, bias_rows, ws, ws_bytes, as_stream(stream), nullptr,
-                          !thin ? nullptr : trans_a ? [](int, int, int, bool) { return true; } : thin_on_gemm32);
+                          !thin ? nullptr : trans_a ? thin_tn_on_gemm32 : thin_on_gemm32);
     if (rc >= 0) return rc;
   }
   // the other thin products: the kernels made for them

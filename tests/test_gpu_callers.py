@@ -36,7 +36,7 @@ def test_relu(dtype, n):
 
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("fin,fout,batch", [(3136, 1024, 16), (1024, 10, 64), (37, 21, 9), (5, 130, 1), (200, 1, 70),
-                                             (96, 80, 300), (130, 67, 1000)])
+                                             (96, 80, 300), (130, 67, 1000), (1043, 2128, 2), (23, 396, 3)])
 def test_linear(fin, fout, batch, dtype):
     rng = np.random.default_rng(fin + fout + batch)
     x = _round(rng.standard_normal((batch, fin)).astype(np.float32), dtype)
