@@ -1012,7 +1012,7 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
     // up to twice as many with one range each, of which those that share a unit take 1.2 times as long.  (Constants fitted to
     // 14292 times of 1175 random geometries; taking the estimate's choice costs 1 % over the best of those measured, at worst 15.
     // Filling the chip whatever the partial tiles cost, as before, 19 %, at worst 126: 16 -> 64 channels over 31 x 193 frames, 7 taps,
-    // 27 -> 13 us; 64 -> 40 over 4 x 1017, 15 taps, stride 2, 30 -> 14; 250 -> 250 over 7 x 1111, 21 taps, 57.)
+    // 27 -> 14 us; 64 -> 40 over 4 x 1017, 15 taps, stride 2, 26 -> 12; 250 -> 250 over 7 x 1111, 21 taps, 56 -> 55.)
     double best = 1e30;
     int best_split = 0, best_upw = 0;
     const double set = 0.013 * TQ * tiles + 0.05;
