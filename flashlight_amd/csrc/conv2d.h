@@ -29,6 +29,7 @@ int mfma_slab_wgrad(const ConvGeom& g, int dtype, const void* x, const void* dy,
                     float* db, void* ws, size_t ws_bytes, hipStream_t s);
 size_t mfma_slab_wgrad_ws(const ConvGeom& g, int dtype);
 bool mfma_slab_wgrad_applies(const ConvGeom& g);
+bool mfma_slab_takes(const ConvGeom& g, bool bwd);      // windows of stride 1 whose operands are aligned
 int mfma_slab_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx,
                             hipStream_t s);
 
@@ -129,6 +130,7 @@ int mfma_pwd16_wgrad(const ConvGeom& g, const void* x, const void* dy, float* dw
 int mfma_strip16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y,
                           hipStream_t s, int dtype);
 int mfma_strip16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, void* dx, hipStream_t s, int dtype);
+bool mfma_slab16_takes(const ConvGeom& g, bool bwd);    // the same in 16-bit storage
 int mfma_slab16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y,
                          hipStream_t s, int dtype);
 int mfma_slab16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, void* dx,

@@ -176,7 +176,11 @@ static bool thin_1x1(const ConvGeom& g, bool bwd, long long tiles) {
 
 // Few result tiles (of 32 channels x 32 positions): the thin kernels.  `first`: asked before the 3x3 slab and strip kernels, which
 // they beat up to two tiles per compute unit in fp32 (64 channels 56 x 56: 392 tiles 18.1 -> 15.9 us, 784 tiles 18.7 -> 22.3; 13 x 13
-// at batch 48, 508 tiles: 26 -> 18) and one in 16-bit storage (196 tiles 10.9 -> 9.0, 784 tiles 11.3 -> 13.0).  Not first: windows
+// at batch 48, 508 tiles: 26 -> 18) and one in 16-bit storage (196 tiles 10.9 -> 9.0, 784 tiles 11.3 -> 13.0).  But over few source
+// channels the copy of the weights and its launch take longer than a slab kernel's one launch where that takes the window (56 x 56,
+// us slab / thin: fp32 8 channels 6.5 / 8.2, 16 8.5 / 8.2 and over 392 tiles 8.9 / 9.2, 40 13.1 / 10.2 and 13.6 / 14.4; 32 x 32, 10 images,
+// 8 channels 6.5 / 9.6; 16-bit storage 16 channels 6.4 / 7.5, 32 6.6 / 8.7, 40 8.4 / 8.7, 64 -> 24 8.6 / 9.3 forward, 10.1 / 8.9
+// backward).  Not first: windows
 // those two do not take, where the tapped GEMM (64 x 64 tiles, fp32 arithmetic) lost at every size measured, 16-bit storage
 // by 2.5 to 9 (128 channels 28 x 28, one image: 68 -> 10 us; 256 channels 14 x 14 at batch 33: 176 -> 47), fp32 by 1.02 to 4 (5x5 over
 // 14 x 14, 64 -> 32 channels, backward-data: batch 1 62 -> 18, batch 512 253 -> 142).
@@ -190,7 +194,12 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
   const long long pos = (long long)g.N * (bwd ? g.H * g.W : g.OH * g.OW), tiles = (pos + 31) / 32 * (((bwd ? g.C : g.K) + 31) / 32);
   if (g.KH * g.KW == 1) return first && !lo && thin_1x1(g, bwd, tiles);
   if (!lo && !bwd && g.KH * g.KW > 9) return false;
-  return !first || tiles <= (lo ? 1 : 2) * (long long)mfma_num_cus();
+  if (!first) return true;
+  const long long cus = mfma_num_cus();
+  if (tiles > (lo ? 1 : 2) * cus) return false;
+  const int src = bwd ? g.K : g.C, dst = bwd ? g.C : g.K;
+  const bool few = lo ? src <= 40 || (!bwd && src <= 64 && dst <= 32) : src <= 24 || (src <= 40 && tiles > cus);
+  return !few || !(lo ? mfma_slab16_takes(g, bwd) : mfma_slab_takes(g, bwd));
 }
 
 static bool long_rows(const ConvGeom& g, int dtype, bool bwd, size_t ws_bytes) {

@@ -642,21 +642,44 @@ int launch(SlabParams& p, const void* src, const void* wgt, const float* bias, v
   return check_launch("conv2d (mfma slab)");
 }
 
+void fill_fwd(const ConvGeom& g, SlabParams* p) {
+  p->N = g.N; p->SC = g.C; p->SH = g.H; p->SW = g.W; p->DC = g.K; p->DH = g.OH; p->DW = g.OW;
+  p->KH = g.KH; p->KW = g.KW; p->KHW = g.KH * g.KW; p->dly = g.dly; p->dlx = g.dlx;
+  p->sh0 = -g.py; p->sw0 = -g.px; p->shs = g.dly; p->sws = g.dlx;
+  p->min_sh = -g.py; p->min_sw = -g.px;
+  p->psh = g.sy; p->psw = g.sx;
+  p->groups = g.groups; p->SCg = g.Cg; p->DCg = g.Kg;
+  p->a_mstride = g.Cg * p->KHW; p->a_cstride = p->KHW; p->w_group_stride = g.Kg * g.Cg * p->KHW;
+  p->mtiles = (g.Kg + BM - 1) / BM;
+}
+
+void fill_bwd(const ConvGeom& g, SlabParams* p) {
+  p->N = g.N; p->SC = g.K; p->SH = g.OH; p->SW = g.OW; p->DC = g.C; p->DH = g.H; p->DW = g.W;
+  p->KH = g.KH; p->KW = g.KW; p->KHW = g.KH * g.KW; p->dly = g.dly; p->dlx = g.dlx;
+  p->sh0 = g.py; p->sw0 = g.px; p->shs = -g.dly; p->sws = -g.dlx;
+  p->min_sh = g.py - (g.KH - 1) * g.dly; p->min_sw = g.px - (g.KW - 1) * g.dlx;
+  p->psh = 1; p->psw = 1;
+  p->groups = g.groups; p->SCg = g.Kg; p->DCg = g.Cg;
+  p->a_mstride = p->KHW; p->a_cstride = g.Cg * p->KHW; p->w_group_stride = g.Kg * g.Cg * p->KHW;
+  p->mtiles = (g.Cg + BM - 1) / BM;
+}
+
 }  // namespace
+
+bool mfma_slab_takes(const ConvGeom& g, bool bwd) {
+  SlabParams p{};
+  if (bwd) fill_bwd(g, &p);
+  else fill_fwd(g, &p);
+  size_t shmem = 0;
+  return plan(&p, &shmem, bwd, true);
+}
 
 int mfma_slab_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w,
                        const float* bias, void* y, hipStream_t s) {
   // strides: results step through the slab; 1x1 windows with a stride are left to the GEMM kernels
   if ((g.sy != 1 || g.sx != 1) && g.KH * g.KW == 1) return -1;
   SlabParams p{};
-  p.N = g.N; p.SC = g.C; p.SH = g.H; p.SW = g.W; p.DC = g.K; p.DH = g.OH; p.DW = g.OW;
-  p.KH = g.KH; p.KW = g.KW; p.KHW = g.KH * g.KW; p.dly = g.dly; p.dlx = g.dlx;
-  p.sh0 = -g.py; p.sw0 = -g.px; p.shs = g.dly; p.sws = g.dlx;
-  p.min_sh = -g.py; p.min_sw = -g.px;
-  p.psh = g.sy; p.psw = g.sx;
-  p.groups = g.groups; p.SCg = g.Cg; p.DCg = g.Kg;
-  p.a_mstride = g.Cg * p.KHW; p.a_cstride = p.KHW; p.w_group_stride = g.Kg * g.Cg * p.KHW;
-  p.mtiles = (g.Kg + BM - 1) / BM;
+  fill_fwd(g, &p);
   return by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
     return launch<T, false>(p, x, w, bias, y, s);
@@ -667,14 +690,7 @@ int mfma_slab_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const 
                             hipStream_t s) {
   if (g.sy != 1 || g.sx != 1) return -1;
   SlabParams p{};
-  p.N = g.N; p.SC = g.K; p.SH = g.OH; p.SW = g.OW; p.DC = g.C; p.DH = g.H; p.DW = g.W;
-  p.KH = g.KH; p.KW = g.KW; p.KHW = g.KH * g.KW; p.dly = g.dly; p.dlx = g.dlx;
-  p.sh0 = g.py; p.sw0 = g.px; p.shs = -g.dly; p.sws = -g.dlx;
-  p.min_sh = g.py - (g.KH - 1) * g.dly; p.min_sw = g.px - (g.KW - 1) * g.dlx;
-  p.psh = 1; p.psw = 1;
-  p.groups = g.groups; p.SCg = g.Kg; p.DCg = g.Cg;
-  p.a_mstride = p.KHW; p.a_cstride = g.Cg * p.KHW; p.w_group_stride = g.Kg * g.Cg * p.KHW;
-  p.mtiles = (g.Cg + BM - 1) / BM;
+  fill_bwd(g, &p);
   return by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
     return launch<T, true>(p, dy, w, nullptr, dx, s);

@@ -780,6 +780,14 @@ long long mfma_slab16_conv_fwd_workgroups(const ConvGeom& g) {
   return (long long)(p.VS > 1 ? (p.N + p.VS - 1) / p.VS : p.N * p.tiles_per_image) * p.mtiles * p.groups;
 }
 
+bool mfma_slab16_takes(const ConvGeom& g, bool bwd) {
+  Slab16Params p{};
+  if (bwd) fill_bwd(g, &p);
+  else fill_fwd(g, &p);
+  size_t shmem = 0;
+  return plan(&p, &shmem);
+}
+
 int mfma_slab16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y,
                          hipStream_t s, int dtype) {
   // strides: results step through the slab; 1x1 windows with a stride are left to the GEMM kernels

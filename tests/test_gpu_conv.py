@@ -294,6 +294,23 @@ def test_conv_with_few_tiles_on_the_other_families(case, dtype):
         capi.set_option("CONV_SKIP", None)
 
 
+@pytest.mark.parametrize("dtype,n,c,k,plane", [(torch.float32, 2, 8, 8, 56), (torch.float32, 10, 8, 8, 32), (torch.float32, 2, 40, 128, 56),
+                                               (torch.bfloat16, 1, 16, 24, 56), (torch.float16, 2, 32, 32, 56), (torch.bfloat16, 2, 64, 16, 56)])
+def test_few_tiles_over_few_channels_stay_on_the_slab_kernels(dtype, n, c, k, plane):
+    """Forward passes whose weights' copy costs more than the kernel for few tiles gains: the same bits as without it."""
+    from flashlight_amd import capi
+    rng = np.random.default_rng(63)
+    x = dev(rng.standard_normal((n, c, plane, plane)).astype(np.float32)).to(dtype)
+    w = dev((rng.standard_normal((k, c, 3, 3)) / 8).astype(np.float32)).to(dtype)
+    y = fa.conv2d(x, w, None, px=1, py=1)
+    capi.set_option("CONV_SKIP", "thin")
+    try:
+        want = fa.conv2d(x, w, None, px=1, py=1)
+    finally:
+        capi.set_option("CONV_SKIP", None)
+    assert torch.equal(y, want)
+
+
 # fp32 slab kernels over rows of whole 16-byte units (the 16-byte loaders) and over other rows (the element-wise
 # loaders): strides, dilation, groups, a filter tail, rows of 8 to 60 columns, a 5x1 and a 1x3 window, whole 7x7 planes.
 F32_SLAB_CASES = [
