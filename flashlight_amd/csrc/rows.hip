@@ -85,9 +85,9 @@ __device__ __forceinline__ float row_max(float v, float* smem) {
 // ---- log-softmax over rows (Functions.cpp:1044-1070) --------------------------------------------------------------------
 // 4000 rows of 9998 in bf16 (160 MB): 137 -> 29 us (before: one wave to a row, element by element, three times over).
 template <typename T, int THREADS, int NP>
-__global__ void __launch_bounds__(256) logsoftmax_rows_fwd(const T* __restrict__ x, T* __restrict__ y, int n, int rows) {
+__global__ void __launch_bounds__(THREADS == 64 ? 256 : THREADS) logsoftmax_rows_fwd(const T* __restrict__ x, T* __restrict__ y, int n, int rows) {
   constexpr int N = Piece<T>::N;
-  __shared__ float smem[4];
+  __shared__ float smem[8];
   const int row = THREADS == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
   if (THREADS == 64 && row >= rows) return;
@@ -135,12 +135,14 @@ __global__ void __launch_bounds__(256) logsoftmax_rows_fwd(const T* __restrict__
   if (has1) st(yr, sp.at(t), one - lse);
 }
 
-// dx = dy - exp(y) * sum of dy: 4000 rows of 9998 in bf16 (240 MB): 113 -> 44 us
+// dx = dy - exp(y) * sum of dy: 4000 rows of 9998 in bf16 (240 MB): 113 -> 44 us.  Rows of more than 16 KB have 512 threads: 8 pieces
+// of both operands in each of 256 do not fit the registers (8032 rows of 4917 in fp32 219 us, one wave to a row 130; 8760 of 5127
+// 258 -> 99 with 512 threads)
 template <typename T, int THREADS, int NP>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(THREADS == 64 ? 256 : THREADS)
 logsoftmax_rows_bwd(const T* __restrict__ dy, const T* __restrict__ y, T* __restrict__ dx, int n, int rows) {
   constexpr int N = Piece<T>::N;
-  __shared__ float smem[4];
+  __shared__ float smem[8];
   const int row = THREADS == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
   if (THREADS == 64 && row >= rows) return;
@@ -446,13 +448,12 @@ bool by_row(int n, F&& f) {
   integral_constant<int, 1> n1;
   integral_constant<int, 2> n2;
   integral_constant<int, 4> n4;
-  integral_constant<int, 8> n8;
   if (pieces <= 64) f(wave, n1);
   else if (pieces <= 128) f(wave, n2);
   else if (pieces <= 256) f(wg, n1);
   else if (pieces <= 512) f(wg, n2);
   else if (pieces <= 1024) f(wg, n4);
-  else if (pieces <= 2048) f(wg, n8);
+  else if (pieces <= 2048) f(integral_constant<int, 512>{}, n4);
   else return false;
   return true;
 }
@@ -498,7 +499,7 @@ bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hip
     using T = FLHIP_T_OF(t_);
     return by_row<T>(n, [&](auto th, auto np) {
       const dim3 grid((unsigned)(th.value == 64 ? (rows + 3) / 4 : rows));
-      hipLaunchKernelGGL((logsoftmax_rows_fwd<T, th.value, np.value>), grid, dim3(256), 0, s, (const T*)x, (T*)y, n, rows);
+      hipLaunchKernelGGL((logsoftmax_rows_fwd<T, th.value, np.value>), grid, dim3(std::max(256, th.value)), 0, s, (const T*)x, (T*)y, n, rows);
     });
   });
 }
@@ -509,7 +510,7 @@ bool rows_logsoftmax_bwd(const void* dy, const void* y, void* dx, int n, int row
     using T = FLHIP_T_OF(t_);
     return by_row<T>(n, [&](auto th, auto np) {
       const dim3 grid((unsigned)(th.value == 64 ? (rows + 3) / 4 : rows));
-      hipLaunchKernelGGL((logsoftmax_rows_bwd<T, th.value, np.value>), grid, dim3(256), 0, s, (const T*)dy, (const T*)y, (T*)dx,
+      hipLaunchKernelGGL((logsoftmax_rows_bwd<T, th.value, np.value>), grid, dim3(std::max(256, th.value)), 0, s, (const T*)dy, (const T*)y, (T*)dx,
                          n, rows);
     });
   });
@@ -558,7 +559,9 @@ extern "C" int flhip_layernorm_fwd(const void* x, const float* w, const float* b
     };
     // 1024 threads to a row that 256 would hold with 32 elements, scales and shifts each: registers for three such rows on a compute
     // unit hide too little (3261 rows of 6147 in f16: 85 us, composed 63; with 1024 threads 3405 rows of 6463 54, composed 70)
-    if (whole) by_row<T>((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, Piece<T>::N>{}); });
+    if (whole) by_row<T>((int)n, [&](auto th, auto np) {
+      if constexpr (th.value <= 256) go(th, np, std::integral_constant<int, Piece<T>::N>{});      // (no longer ones apply)
+    });
     else if (n > 4096) go(std::integral_constant<int, 1024>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
     else by_element((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, 1>{}); });
   });
@@ -588,7 +591,9 @@ extern "C" int flhip_layernorm_bwd(const void* dy, const void* x, const float* w
       hipLaunchKernelGGL((layernorm_rows_bwd<T, th.value, np.value, ne.value>), dim3((unsigned)slices), dim3(256), 0, s, (const T*)dy,
                          (const T*)x, w, mean, invstd, (T*)dx, part, (int)n, (int)rows, rps, scalar_params ? 0 : 1);
     };
-    if (whole) by_row<T>((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, Piece<T>::N>{}); });
+    if (whole) by_row<T>((int)n, [&](auto th, auto np) {
+      if constexpr (th.value <= 256) go(th, np, std::integral_constant<int, Piece<T>::N>{});      // (no longer ones apply)
+    });
     else by_element((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, 1>{}); });
   });
   if (const int rc = check_launch("layernorm_bwd")) return rc;

@@ -335,10 +335,10 @@ def test_logsoftmax(classes, cols, dtype):
     assert np.allclose(host(dx), dx_ref, atol=_tol(dtype) * 10, rtol=_tol(dtype))
 
 
-# rows held in registers: one wave / one workgroup to a row, 1 to 8 pieces of 16 bytes per thread, rows that start off a
+# rows held in registers: one wave / one workgroup to a row, 1 to 4 pieces of 16 bytes per thread, rows that start off a
 # 16-byte boundary, the longest that fit (8192 / 16384 elements) and the first that do not
 @pytest.mark.parametrize("dtype", DT)
-@pytest.mark.parametrize("classes,cols", [(3, 9), (256, 5), (257, 5), (1025, 6), (2049, 3), (4001, 5), (8192, 2), (8193, 3), (9998, 3),
+@pytest.mark.parametrize("classes,cols", [(3, 9), (256, 5), (257, 5), (1025, 6), (2049, 3), (4001, 5), (4096, 3), (4099, 7), (8192, 2), (8193, 3), (9998, 3),
                                           (16384, 2), (16385, 2)])
 def test_logsoftmax_and_cross_entropy_rows(classes, cols, dtype):
     rng = np.random.default_rng(classes + cols)
