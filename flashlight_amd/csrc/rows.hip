@@ -489,12 +489,17 @@ int ln_slices(int n, int rows) { return std::max(1, std::min(512, n > 1024 ? row
 // Rows of less than 320 bytes leave most of a wave's lanes without a piece, and the single elements around the pieces cost
 // more than they save: a lane per element is faster then (100000 rows, us by elements / by pieces: bf16 forward 29 elements 20.7 / 33.0,
 // 128 31.5 / 32.5, 192 43.1 / 32.8, backward 16.4 / 31.8, 24.4 / 27.5, 33.4 / 27.8; fp32 forward 29 elements 22.0 / 25.3, 64 23.7 /
-// 25.1, 100 33.3 / 25.5, backward 17.7 / 22.5, 19.8 / 19.5, 27.1 / 21.3).
-bool short_row(int n, int dtype) { return n < 320 / (int)dtype_size(dtype); }
+// 25.1, 100 33.3 / 25.5, backward 17.7 / 22.5, 19.8 / 19.5, 27.1 / 21.3).  Backward the line lies at 352 bytes, and at 400 where rows are
+// not whole pieces (152202 rows of 182 in f16 48.9 / 55.2, 14592 6.5 / 8.5, 8518 of 178 in bf16 5.1 / 5.7; but 105143 of 176 33.9 / 30.1,
+// 45584 of 219 in f16 21.8 / 20.3).
+bool short_row(int n, int dtype, bool bwd) {
+  const int bytes = n * (int)dtype_size(dtype);
+  return bytes < (!bwd ? 320 : bytes % 16 ? 400 : 352);
+}
 
 // -> false where the row does not fit (the caller's element-wise kernels take it)
 bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hipStream_t s) {
-  if (short_row(n, dtype) || !same_offset(x, y)) return false;
+  if (short_row(n, dtype, false) || !same_offset(x, y)) return false;
   return by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
     return by_row<T>(n, [&](auto th, auto np) {
@@ -505,7 +510,7 @@ bool rows_logsoftmax_fwd(const void* x, void* y, int n, int rows, int dtype, hip
 }
 
 bool rows_logsoftmax_bwd(const void* dy, const void* y, void* dx, int n, int rows, int dtype, hipStream_t s) {
-  if (short_row(n, dtype) || !same_offset(dy, y, dx)) return false;
+  if (short_row(n, dtype, true) || !same_offset(dy, y, dx)) return false;
   return by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
     return by_row<T>(n, [&](auto th, auto np) {

@@ -365,7 +365,7 @@ def test_logsoftmax_and_cross_entropy_rows(classes, cols, dtype):
 
 
 @pytest.mark.parametrize("dtype", DT)
-@pytest.mark.parametrize("classes", [79, 80, 159, 160, 383, 384])
+@pytest.mark.parametrize("classes", [79, 80, 87, 88, 99, 101, 159, 160, 175, 176, 199, 201, 383, 384])
 def test_logsoftmax_and_cross_entropy_between_elements_and_pieces(classes, dtype):
     """The shortest rows that are held as pieces, and the longest that are not."""
     test_logsoftmax_and_cross_entropy_rows(classes, 35, dtype)
