@@ -540,9 +540,9 @@ using namespace flhip;
 
 extern "C" int flhip_layernorm_applies(int64_t n, int64_t rows, int dtype) {
   if (n <= 0 || rows <= 0 || rows > 1 << 30 || !dtype_ok(dtype)) return 0;      // (a grid's stride past the last row stays an int)
-  // a row of one element has nothing to sum: with many of them the general kernels are faster (forward / backward, 100000
-  // rows: 35 / 42 us there, 23 / 29 here; 1000000 rows: 35 / 68 there, 160 / 230 here)
-  if (n == 1 && rows > (1 << 17)) return 0;
+  // a row of one element has nothing to sum: with many of them the general kernels are faster (forward / backward in f16, 123245
+  // rows: 11 / 19 us there, 23 / 35 here; 59588: 10.5 / 15.7, 13.2 / 21.4; 33092: backward 14.3, 15.8)
+  if (n == 1 && rows > (1 << 14)) return 0;
   return n <= 1024 * 16 / (int64_t)dtype_size(dtype);      // four pieces per thread (the backward pass's registers)
 }
 

@@ -64,7 +64,7 @@ def test_layernorm_row_limits():
     assert applies(8192, 1, capi.BF16) and not applies(8193, 1, capi.F16)
     assert applies(2, 1 << 30, capi.BF16) and not applies(2, (1 << 30) + 1, capi.BF16)
     assert not applies(2, (1 << 31) - 1, capi.BF16)
-    assert applies(1, 1 << 17, capi.F32) and not applies(1, (1 << 17) + 1, capi.F32)
+    assert applies(1, 1 << 14, capi.F32) and not applies(1, (1 << 14) + 1, capi.F32)
     assert not applies(0, 4, capi.F32) and not applies(4, 0, capi.F32) and not applies(4, 4, 17)
 
 
