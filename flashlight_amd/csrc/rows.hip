@@ -422,16 +422,18 @@ layernorm_fold(const float* __restrict__ part, float* __restrict__ dw, float* __
     else db[c - n] = s;
   }
 }
-// one parameter element for the whole row: the sums over its columns
-__global__ void __launch_bounds__(256)
+// one parameter element for the whole row: the sums over its columns (16 waves: with four, a row of 5000 columns takes 20 rounds
+// of loads one after the other)
+__global__ void __launch_bounds__(1024)
 layernorm_fold_scalar(const float* __restrict__ cols, float* __restrict__ dw, float* __restrict__ db, int n) {
-  __shared__ float smem[8];
+  __shared__ float smem[32];
   float a = 0.f, b = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) {
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 1024) {
     a += cols[i];
     b += cols[n + i];
   }
-  block_sum2<4>(a, b, smem);
+  block_sum2<16>(a, b, smem);
   if (threadIdx.x == 0) {
     dw[0] = a;
     db[0] = b;
@@ -605,6 +607,6 @@ extern "C" int flhip_layernorm_bwd(const void* dy, const void* x, const float* w
   float* cols = part + (size_t)slices * 2 * n;
   hipLaunchKernelGGL(layernorm_fold, dim3((unsigned)((2 * n + 63) / 64)), dim3(1024), 0, s, part, scalar_params ? cols : dw,
                      scalar_params ? cols + n : db, (int)n, slices);
-  if (scalar_params) hipLaunchKernelGGL(layernorm_fold_scalar, dim3(1), dim3(256), 0, s, cols, dw, db, (int)n);
+  if (scalar_params) hipLaunchKernelGGL(layernorm_fold_scalar, dim3(1), dim3(1024), 0, s, cols, dw, db, (int)n);
   return check_launch("layernorm_bwd (sums)");
 }
