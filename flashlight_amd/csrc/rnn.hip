@@ -1136,7 +1136,7 @@ int seq_units(const RnnGeom& g) {
 int seq_pause_fwd(const RnnGeom& g, int units) {
   const double V = (double)g.D * ((g.H + units - 1) / units) * g.B * g.H * 4e-6;      // MB
   if (g.G == 1) return g.H <= 384 ? 3 : g.H <= 512 ? 4 : V < 1 ? 4 : g.H <= 768 ? 6 : 7;
-  if (g.H <= 256) return V < 2 ? 4 : 5;
+  if (g.H <= 256) return V < 1 ? 4 : 5;
   if (g.H <= 512) return g.H <= 448 || V < 4 ? 5 : 6;
   return (int)(units == 4 ? 5.5 + V / 4 : units == 8 ? 6.5 + 0.6 * V : 5.5 + 0.4 * V);
 }
@@ -1153,6 +1153,8 @@ int seq_pause_bwd(const RnnGeom& g) {
 //   two directions, 32 columns, over 2 / 4 steps 0.99 and 0.80; GRU of 512 units, training, 16 columns 1.27, 1.09, 0.99.
 //   Against the two-kernel steps (two launches per step and direction), over 2 / 4 steps: LSTM of 512 units, 128 columns 0.71, 0.47;
 //   of 200 units 1.08, 0.84, ReLU of 200 units 1.13, 0.85; of 128 units, two directions 0.77, 0.56.
+//   Backward the steps cost more: GRU of 768 units, 3 layers, 51 columns, over 3 steps 0.81; against the two-kernel steps, one step, LSTM
+//   of 768 units, 70 columns 0.75, of 1000 units, 1 column 0.83, GRU of 768 units, 2 layers, 66 columns 0.87.
 //   Clusters beyond the compute units go in further launches, so that with many columns the estimates (us per step, from 32 to
 //   1024 units, ReLU to LSTM) decide: LSTM of 512 units over 20 steps, 256 columns (2 launches) 0.77, 512 columns (4) 1.19; 1024
 //   units, 256 columns (4) 1.23, backward 0.8.
@@ -1160,11 +1162,11 @@ bool seq_pays(const RnnGeom& g, bool bwd) {
   const int tiles = (g.B + SEQ_COLS - 1) / SEQ_COLS;
   if (fused_applies(g)) {
     const int weight = g.D * g.H * tiles * (g.G == 1 ? 5 : 2 * g.G + 2) / 10;
-    return g.T >= (weight >= 3500 ? 3 : weight >= 1500 ? 4 : g.B > 32 ? 5 : weight >= 700 || g.B > 16 ? 6 : 8);
+    return g.T >= (weight >= (bwd ? 2000 : 3500) ? 3 : weight >= 1500 ? 4 : g.B > 32 ? 5 : weight >= 600 || g.B > 16 ? 6 : 8);
   }
   const int units = bwd ? 16 : seq_units(g), nwg = (g.H + units - 1) / units, per = std::max(1, mfma_num_cus() / nwg);
   const int launches = (g.D * tiles + per - 1) / per;
-  if (launches == 1) return g.T >= (g.D == 2 || g.GH >= 1000 ? 2 : 3);
+  if (launches == 1) return g.T >= (bwd && g.GH >= 2000 ? 1 : g.D == 2 || g.GH >= 1000 ? 2 : 3);
   const double H = g.H, step = bwd ? 5.5 + H * (0.006 + 0.016 * g.G * (1.0 + g.B / 750.0)) : 5.0 + H * (0.012 + 0.0053 * g.G);
   const double seq = bwd ? 1.6 + H * (0.0048 * g.G - 0.0003) : 1.1 + H * (0.0015 + 0.0019 * g.G);
   return g.T * (g.D * step - launches * seq) > 22.0 * launches;
