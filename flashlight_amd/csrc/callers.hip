@@ -955,11 +955,11 @@ extern "C" size_t flhip_matmul_workspace_bytes(int32_t M, int32_t N, int32_t K, 
 // One slice of gemm_f32.hip: 512 x 64, K 64 / 128 / 256: 3.8 / 4.7 / 6.7 us (4.7 / 5.0 / 5.5); from a second round on it is the
 // faster one at every K (4096 x 64 x 256: 6.9, 7.3; 4096 x 128 x 256: 7.1, 12).  Slices: 512 x 64, K 512 / 768 / 1024: 7.4 / 7.3 / 8.0
 // (8.5 / 11.4 / 14.5), but the second launch and the workspace cost the host some 4 us, so that calls in a row come every 14 us
-// where this kernel's come every 11.5: worth it from where its rounds take longer than that (a little later for a single block of
-// columns: 12.8 us at K 1024).
+// where this kernel's come every 11: worth it from where its rounds take longer than that (7 x 940 -> 60 8.1 / 13.9,
+// 4 x 1072 -> 52 7.9 / 16.0, 45 x 552 -> 3996, two rounds, 10.3 / 21.7).
 static bool thin_on_gemm32(int M, int N, int K, bool slices) {
   const long long rounds = ((long long)((M + 63) / 64) * ((N + SK_NT - 1) / SK_NT) + 255) / 256;
-  return slices ? K >= (N <= SK_NT ? 1152 : 1024) || rounds * K >= 1408 : K <= 128 || rounds > 1;
+  return slices ? rounds * K >= 704 : K <= 128 || rounds > 1;
 }
 
 // The same for A^T * B and matmul_tn_skinny.  Slices, and one slice where it is short, always win; but a C of M * N elements that are

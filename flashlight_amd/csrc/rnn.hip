@@ -153,7 +153,7 @@ struct Scratch {
 int mm(const float* A, const float* B, float* C, size_t M, size_t N, size_t K, int ta, int tb,
        const float* bias, hipStream_t s, Scratch w = Scratch()) {
   // A thin product A * B that gemm_f32.hip cuts into slices is faster there from the shortest such contraction on (512 x 64 x 512 7.4 /
-  // 8.5 us).  flhip_matmul_ws leaves it to the other kernel up to a contraction of 1024 for the second launch's host time,
+  // 8.5 us).  flhip_matmul_ws leaves it to the other kernel up to a contraction of 704 for the second launch's host time,
   // which a layer's queued launches hide: GRU of 320 units, 3 layers, backward over 13 steps, 7 columns 321 -> 272 us.
   if (!ta && !tb && N <= 128 && !options().matmul_valu && options().matmul_planes < 0) {
     const int rc = gemm32(0, A, B, C, (int)M, (int)N, (int)K, bias, w.p, w.bytes, s, nullptr,
