@@ -315,6 +315,66 @@ layernorm_rows_fwd(const T* __restrict__ x, const float* __restrict__ w, const f
   }
 }
 
+// Rows that are not of whole pieces, with one scale and shift: pieces on 16-byte boundaries and single elements around them, as
+// the log-softmax takes them, since there are no parameters per element to fetch (8558 rows of 2113 in f16: 44 us element by
+// element, 21 so; x and y have to start alike).
+template <typename T, int THREADS, int NP>
+__global__ void __launch_bounds__(256)
+layernorm_ragged_fwd(const T* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, T* __restrict__ y,
+                     float* __restrict__ mean, float* __restrict__ invstd, int n, int rows, float eps) {
+  constexpr int N = Piece<T>::N, RPB = 256 / THREADS;
+  __shared__ float smem[4];
+  const int t = THREADS == 64 ? threadIdx.x & 63 : threadIdx.x;
+  const float we = as_stored<T>(w[0]), be = as_stored<T>(b[0]);
+  for (int row = blockIdx.x * RPB + (THREADS == 64 ? threadIdx.x >> 6 : 0); row < rows; row += gridDim.x * RPB) {
+    const T* xr = x + (size_t)row * n;
+    T* yr = y + (size_t)row * n;
+    const RowSplit<T> sp(xr, n);
+    const uintx4_t* xb = reinterpret_cast<const uintx4_t*>(xr + sp.head);
+    uintx4_t r[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) r[i] = xb[t + i * THREADS];
+    const bool has1 = t < sp.singles;
+    const float one = has1 ? ld(xr, sp.at(t)) : 0.f;
+    float s = one;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) s += v[e];
+      }
+    const float m = row_sum<THREADS>(s, smem) / (float)n;
+    float q = has1 ? (one - m) * (one - m) : 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) q += (v[e] - m) * (v[e] - m);
+      }
+    const float is = 1.f / sqrtf(row_sum<THREADS>(q, smem) / (float)n + eps);
+    if (t == 0) {
+      mean[row] = m;
+      invstd[row] = is;
+    }
+    uintx4_t* yb = reinterpret_cast<uintx4_t*>(yr + sp.head);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (t + i * THREADS < sp.body) {
+        float v[N];
+        unpack<T>(r[i], v);
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = we * ((v[e] - m) * is) + be;
+        yb[t + i * THREADS] = packed<T>(v);
+      }
+    if (has1) st(yr, sp.at(t), we * ((one - m) * is) + be);
+  }
+}
+
 // dx = invstd * (g - mean(g) - xhat * mean(g * xhat)), g = w * dy, and over slice blockIdx.x of the rows the sums of
 // dy * xhat and dy per element of the row: part[slice][2][n].  A thread has the same elements in every row, as above, and
 // keeps their sums from row to row.  A row of one wave takes no barrier, and the four waves of a workgroup each have a row in
@@ -568,6 +628,12 @@ extern "C" int flhip_layernorm_fwd(const void* x, const float* w, const float* b
     // unit hide too little (3261 rows of 6147 in f16: 85 us, composed 63; with 1024 threads 3405 rows of 6463 54, composed 70)
     if (whole) by_row<T>((int)n, [&](auto th, auto np) {
       if constexpr (th.value <= 256) go(th, np, std::integral_constant<int, Piece<T>::N>{});      // (no longer ones apply)
+    });
+    else if (scalar_params && n >= 256 && same_offset(x, y)) by_row<T>((int)n, [&](auto th, auto np) {
+      if constexpr (th.value <= 256)
+        hipLaunchKernelGGL((layernorm_ragged_fwd<T, th.value, np.value>),
+                           dim3((unsigned)std::min<int64_t>(th.value == 64 ? (rows + 3) / 4 : rows, 2048)), dim3(256), 0, as_stream(stream),
+                           (const T*)x, w, b, (T*)y, mean, invstd, (int)n, (int)rows, (float)epsilon);
     });
     else if (n > 4096) go(std::integral_constant<int, 1024>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
     else by_element((int)n, [&](auto th, auto np) { go(th, np, std::integral_constant<int, 1>{}); });

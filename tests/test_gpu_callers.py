@@ -400,7 +400,8 @@ def test_layer_norm_rows(n, rows, scalar, dtype):
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("n,rows,scalar", [(64, 21, False), (65, 3, True), (128, 2050, False), (129, 6, False), (257, 37, False), (513, 5, True),
                                            (1024, 21, False), (1025, 21, False), (2049, 9, False), (4095, 5, False), (4097, 3, False),
-                                           (1025, 515, False), (4097, 515, False), (8191, 2, True)])
+                                           (1025, 515, False), (4097, 515, False), (8191, 2, True),
+                                           (255, 9, True), (257, 2050, True), (1025, 21, True), (2051, 5, True), (4095, 7, True)])
 def test_layer_norm_rows_at_the_edges(n, rows, scalar, dtype):
     """One element more or less than a wave or a workgroup takes per thread, and rows that leave waves without one."""
     test_layer_norm_rows(n, rows, scalar, dtype)
