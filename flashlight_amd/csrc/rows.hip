@@ -543,8 +543,9 @@ bool same_offset(const void* a, const void* b, const void* c = nullptr) {
 
 // slices of the rows for the backward pass: about two workgroups per compute unit.  A workgroup goes through its rows one after the
 // other (four at a time, where a wave has a row of its own), so few long rows get one each: with four to a workgroup, 5 rows of 6590
-// in f16 took 46 us, 12 of 6803 42 (composed 17 and 18); with one each, 4 rows of 6789 13 and 22 of 6897 14 (composed 20 and 21)
-int ln_slices(int n, int rows) { return std::max(1, std::min(512, n > 1024 ? rows : rows / 4)); }
+// in f16 took 46 us, 12 of 6803 42 (composed 17 and 18); with one each, 4 rows of 6789 13 and 22 of 6897 14 (composed 20 and 21).
+// More rows have more partial sums for the fold to read: 843 of 8104 in bf16 27 us with four to a workgroup, 35 with 512 workgroups
+int ln_slices(int n, int rows) { return std::max(n > 1024 ? std::min(rows, 128) : 1, std::min(512, rows / 4)); }
 
 }  // namespace
 
