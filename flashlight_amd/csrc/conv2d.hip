@@ -164,12 +164,13 @@ static bool tap2d_on(const ConvGeom& g, int dtype) {
 // thin: forward over 7 x 7 256 -> 64 channels 10.6 / 8.9, 512 -> 1024 17.0 / 15.2, 2048 -> 512 52.6 / 31.3; over 4 x 4 256 -> 64 8.5 /
 // 8.6, 512 -> 1024 13.8 / 13.9, 1024 -> 512 24.0 / 16.9, 1024 -> 2048 25.8 / 32.3; backward over 7 x 7 from 256 to 64 channels 12.5 /
 // 8.8, from 512 to 1024 20.7 / 14.9, from 128 to 512 8.5 / 9.0 (1 x 1), and cut, from 1024 to 512 16.4 / 18.5, from 2048 to 512
-// 23.3 / 31.1.  Over more than 24 planes of one position a tile's loads touch as many cache lines (2048 -> 1000, 24 / 33 images:
+// 23.3 / 31.1; cut over ragged planes to few channels from 1024 to 64 over 7 x 7 15.2 / 13.4, 25 images 16.8 / 14.1, from 1000 to 32 over
+// 13 x 13, 11 images, 16.4 / 13.6.  Over more than 24 planes of one position a tile's loads touch as many cache lines (2048 -> 1000, 24 / 33 images:
 // 53.6 / 49.0, 54.0 / 61.2; 1024 -> 512, 33: 29.1 / 27.2).
 static bool thin_1x1(const ConvGeom& g, bool bwd, long long tiles) {
   const long long src = bwd ? g.K : g.C, dst = bwd ? g.C : g.K;
   if (tiles > src / 8 || src < 256 || dst > 2048) return false;
-  if (bwd) return mfma_pointwise_split_ws(g, FLHIP_F32, true) == 0;
+  if (bwd) return mfma_pointwise_split_ws(g, FLHIP_F32, true) == 0 || (g.H * g.W % 4 != 0 && src <= 1024 && dst <= 128);
   if (g.H * g.W == 1 && g.N > 24 && dst > 512) return false;
   return g.H * g.W % 4 ? src * (1830 - dst) > 400000 : src * (1500 - dst) > 530000;
 }

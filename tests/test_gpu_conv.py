@@ -274,7 +274,8 @@ def test_conv_few_tiles(case, dtype):
 
 @pytest.mark.parametrize("case", [((1, 256, 7, 7), (64, 256, 1, 1), (1, 1), (0, 0), (1, 1), 1), ((1, 256, 4, 4), (64, 256, 1, 1), (1, 1), (0, 0), (1, 1), 1),
                                   ((2, 512, 7, 7), (256, 512, 1, 1), (1, 1), (0, 0), (1, 1), 1), ((25, 512, 1, 1), (520, 512, 1, 1), (1, 1), (0, 0), (1, 1), 1),
-                                  ((3, 128, 4, 4), (512, 128, 1, 1), (1, 1), (0, 0), (1, 1), 1)])
+                                  ((3, 128, 4, 4), (512, 128, 1, 1), (1, 1), (0, 0), (1, 1), 1), ((2, 64, 5, 5), (1000, 64, 1, 1), (1, 1), (0, 0), (1, 1), 1),
+                                  ((1, 129, 7, 7), (1024, 129, 1, 1), (1, 1), (0, 0), (1, 1), 1)])
 def test_conv_few_tiles_1x1(case):
     """1x1 windows on both sides of the lines between the kernels."""
     test_conv_few_tiles(case, torch.float32)
