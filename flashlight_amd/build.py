@@ -11,7 +11,7 @@ LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "_obj")
 LIB = os.path.join(LIBDIR, "libflhip.so")
 
-SOURCES = ["api.hip", "callers.hip", "gemm_f32.hip", "rows.hip", "rnn.hip", "pool2d.hip", "batchnorm.hip", "conv2d.hip", "conv2d_mfma_gather.hip", "conv2d_mfma_wgrad.hip",
+SOURCES = ["api.hip", "callers.hip", "gemm_f32.hip", "gemm_f32_split.hip", "rows.hip", "rnn.hip", "pool2d.hip", "batchnorm.hip", "conv2d.hip", "conv2d_mfma_gather.hip", "conv2d_mfma_wgrad.hip",
            "conv2d_mfma_slab.hip", "conv2d_mfma_pointwise.hip", "conv2d_mfma_pointwise_bf16.hip", "conv2d_mfma_wgrad_slab.hip", "conv2d_mfma_slab_bf16.hip",
            "conv2d_mfma_wgrad_slab_bf16.hip", "conv2d_mfma_strip_bf16.hip", "conv2d_mfma_first_bf16.hip", "conv2d_mfma_cells.hip",
            "conv2d_mfma_pointwise_dma_bf16.hip", "conv2d_mfma_wgrad_dma_bf16.hip", "conv2d_mfma_tap1d.hip", "conv2d_mfma_thin.hip"]

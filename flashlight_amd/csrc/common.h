@@ -294,7 +294,7 @@ struct Options {
   bool matmul_valu = false;       // MATMUL_VALU: flhip_matmul stays off the matrix cores
   int matmul_planes = -1;         // MATMUL_PLANES: bit m set = fp32 product of mode m (0: A B, 1: A^T B, 2: A B^T) with a
                                   // matrix as one image's plane whatever its shape; 0: never; -1: by shape
-  bool matmul_fp32_cores = false; // MATMUL_FP32_CORES: 16-bit products stay on the fp32 matrix instructions
+  bool matmul_fp32_cores = false; // MATMUL_FP32_CORES: 16-bit products stay on the fp32 matrix instructions, fp32 ones too
   bool rnn_unfused = false;       // RNN_UNFUSED: two-kernel rnn steps
   enum { SEQ_AUTO = 0, SEQ_ALWAYS, SEQ_NEVER, SEQ_REFUSED };
   int rnn_sequences = SEQ_AUTO;   // RNN_SEQUENCES = auto | always (sequence launches wherever the kernels apply) | never | refused (tried wherever

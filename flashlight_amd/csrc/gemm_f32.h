@@ -1,0 +1,29 @@
+// What the two kernels for fp32 matrix products share.
+#pragma once
+#include <stddef.h>
+#include <hip/hip_runtime.h>
+
+namespace flhip {
+
+constexpr int G32_KC = 16;          // contraction indexes per stage
+
+struct Gemm32 {
+  int M, N, K;
+  int mtiles, ntiles;
+  int nstages, sps;            // stages of the contraction, stages per slice
+  unsigned a_bytes, b_bytes;
+  size_t slice;                // elements between the partial results of consecutive slices
+};
+
+// consecutive workgroups go to the eight dies in turn: each die takes one run of tiles, and within a run the tiles of
+// a column block follow each other, so that a die's cache holds what its workgroups share
+__device__ __forceinline__ int gemm32_tile_of(int wg, int tiles) {
+  const int per = tiles >> 3, rem = tiles & 7, die = wg & 7;
+  return die * per + (die < rem ? die : rem) + (wg >> 3);
+}
+
+// gemm_f32_split.hip: mode and tile tm x tn (128 x 128, 128 x 64 or 64 x 128); -1 where the tile has no kernel
+int gemm32_split(int mode, int tm, int tn, int slices, const Gemm32& p, const float* A, const float* B, const float* bias,
+                 const float* addend, float* C, hipStream_t s);
+
+}  // namespace flhip

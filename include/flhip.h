@@ -440,7 +440,7 @@ int flhip_pad_bwd(const void* dy, void* dx, const int64_t* dims, const int32_t* 
 /* C (M x N) = op(A) (M x K) * op(B) (K x N), fp32 accumulate, one rounding to the element
  * type; trans_a: A is stored K x M, trans_b: B is stored N x K.  bias_rows (fp32[M], may be
  * NULL) is added to every column.  bf16 / f16 products of more than 128 columns run on the
- * 16-bit matrix instructions (option MATMUL_FP32_CORES: on the fp32 ones).  Serves fl::linear (Functions.cpp:1255-1309): forward
+ * 16-bit matrix instructions (option MATMUL_FP32_CORES: on the fp32 ones, fp32 products too).  Serves fl::linear (Functions.cpp:1255-1309): forward
  * matmul(weight, input) + tile(bias), backward matmulTN(weight, gradOutput) and
  * matmulNT(gradOutput, input). */
 int flhip_matmul(const void* A, const void* B, void* C, int32_t M, int32_t N,

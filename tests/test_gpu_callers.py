@@ -257,6 +257,41 @@ def test_matmul_fp32_tiles_with_odd_rows(M, N, K):
     test_matmul_fp32_tiles(1, M, N, K, True)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (2396, 1292, 16), (2700, 1092, 20), (2744, 76, 1584), (68, 2720, 1380),            # 128 x 64: whole stages, a last one of 4, slices of either
+    (2460, 1656, 32), (2480, 1604, 20), (180, 2732, 1232), (132, 2720, 1220),          # 64 x 128
+    (2540, 2516, 80), (2528, 2492, 68), (520, 2544, 1120)])                            # 128 x 128
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_matmul_fp32_in_three_parts(mode, M, N, K):
+    """The tiles whose operands are taken apart into bf16 parts, the bias with them."""
+    test_matmul_fp32_tiles(mode, M, N, K, True)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_matmul_fp32_in_three_parts_keeps_what_bf16_cannot_hold(mode):
+    """Infinities, NaN and values that round to infinity in bf16 give what they give in fp32; the rows and columns without
+    them stay as precise.  (Large values times small ones: their sums are finite.)"""
+    M, N, K = 2528, 2492, 68
+    rng = np.random.default_rng(mode)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    B[7] = 1.0 + rng.random(N, dtype=np.float32)
+    A[3, 7], A[700, 7], A[701, 5], A[2527, 7] = np.inf, -np.inf, np.nan, 3.4e38
+    B[7] *= 1e-3
+    B[40, 9], B[67, 2491] = np.inf, np.nan
+    A[1000, 66], B[66, :] = 0.0, B[66, :] * 1e-30
+    with np.errstate(all="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+    got = _matmul_through_c_abi(A if mode == 1 else A.T.copy(), B if mode == 2 else B.T.copy(), M, N, K, mode == 1, mode == 2, None,
+                                torch.float32).T.astype(np.float64)
+    assert (np.isnan(got) == np.isnan(ref)).all() and (np.isinf(got) == np.isinf(ref)).all()
+    inf = np.isinf(ref)
+    assert inf.any() and (got[inf] == ref[inf]).all()
+    for rows in (slice(2527, 2528), slice(704, 2527)):
+        ok = np.isfinite(ref[rows])
+        assert rel_l2(got[rows][ok], ref[rows][ok]) <= 2 * np.sqrt(K) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 64, 128), (512, 64, 132), (64, 8, 1148), (64, 8, 1152), (64, 9, 1020), (64, 9, 1024), (4096, 32, 132), (4096, 33, 132),
                                    (4096, 64, 700), (4096, 64, 704)])
 def test_matmul_fp32_thin(M, N, K):
