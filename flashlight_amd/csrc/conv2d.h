@@ -143,6 +143,18 @@ int mfma_tap1d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void*
                         void* ws, size_t ws_bytes);
 int mfma_tap1d_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx, hipStream_t s, void* ws,
                              size_t ws_bytes);
+// the same windows in fp32, and windows of several rows, stride 1 and a result of the same size over stacked planes, operands in
+// three bf16 parts
+// (conv2d_mfma_tap_split.hip); the one-row forward pass leaves its channels-last rows at the start of its workspace
+size_t mfma_tap1d_split_ws(const ConvGeom& g, bool bwd, size_t* rows_bytes);
+int mfma_tap1d_split(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, void* dst, hipStream_t s, void* ws,
+                     size_t ws_bytes);
+bool mfma_tap2d_split_pays(const ConvGeom& g, bool bwd);
+size_t mfma_tap2d_split_ws(const ConvGeom& g, bool bwd);
+int mfma_tap2d_split(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, void* dst, hipStream_t s, void* ws,
+                     size_t ws_bytes);
+int mfma_tap1d_cs(int C, int esz);
+void mfma_tap1d_rows_f32(const float* x, float* xr, int C, int H, int T, int Cs, int rows, hipStream_t s);
 // 3x3 windows of stride 1 and padding 1 over small planes on the same kernels: every plane of the batch in one
 // sequence (rows followed by a zero column, planes separated by a zero row), 65 to 512 (fp32: 256) contraction channels;
 // operands in mfma_tap2d_conv_ws() bytes of workspace; -1 when the shape is not theirs or the room is missing

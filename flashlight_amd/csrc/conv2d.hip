@@ -148,14 +148,15 @@ static bool tap1d_on(int dtype) {
   return dtype == FLHIP_F32 || ((dtype == FLHIP_BF16 || dtype == FLHIP_F16) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT));
 }
 
-// 3x3 windows over stacked planes: bf16, planes of at most 64 positions (the 7 x 7 layers) and a sequence of at least
-// 2048 positions.  Measured (batch 64 / 32, forward): 7 x 7 x 512 41.9 / 40.3 us against 62.3 / 54.8 on the slab
-// kernel; 14 x 14 x 256 42.2 / 33.0 against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5 against 25.5 / 19.7, so larger planes
-// stay where they were; fp32 loses at every size (14 x 14 x 256: 221 against 140 us).  TAP2D_ALL lifts the rule.
-static bool tap2d_on(const ConvGeom& g, int dtype) {
+// Windows over stacked planes.  fp32: by the estimate of conv2d_mfma_tap_split.hip.  16-bit storage: 3x3 windows over planes of at
+// most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.  Measured (batch 64 / 32, forward): 7 x 7 x 512
+// 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0 against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5
+// against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts both rules.
+static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
   if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
   if (options().tap2d_all) return true;
-  return (dtype == FLHIP_BF16 || dtype == FLHIP_F16) && g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
+  if (dtype == FLHIP_F32) return mfma_tap2d_split_pays(g, bwd);
+  return g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
 }
 
 // 1x1 windows in fp32 with few tiles for their contraction: the thin kernels take about 8 us + 6 per 1000 source channels + 10 per million
@@ -280,8 +281,8 @@ extern "C" size_t flhip_conv2d_workspace_bytes(const flhip_conv_desc* d, int pas
     size_t c = mfma_tap1d_conv_ws(g, d->dtype, bwd);
     if (bwd || thin_on(g, d->dtype, bwd, true) || thin_on(g, d->dtype, bwd, false)) c = std::max(c, mfma_thin_ws(g, d->dtype, bwd));
     // (the stacked-plane kernels: where their rule takes the geometry, and for every plane of at most 32 x 32 positions so
-    // that a caller can try them by plan number; beyond that their copy of the input is tens of megabytes nobody asked for)
-    const size_t c2 = (tap2d_on(g, d->dtype) || g.H * g.W <= 1024) ? mfma_tap2d_conv_ws(g, d->dtype, pass == FLHIP_CONV_BWD_DATA) : 0;
+    // that a caller can try them by plan number; beyond that their copy of the input is tens of megabytes nobody asked for; fp32 copies the weights alone)
+    const size_t c2 = (tap2d_on(g, d->dtype, bwd) || g.H * g.W <= 1024) ? mfma_tap2d_conv_ws(g, d->dtype, pass == FLHIP_CONV_BWD_DATA) : 0;
     return std::max(std::max(a, c2), std::max(b, c));
   }
   return 0;
@@ -298,7 +299,7 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
   if (!force_direct()) {
     int r = -1;
     if (tap1d_on(d->dtype)) r = mfma_tap1d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
-    if (r < 0 && tap2d_on(g, d->dtype)) r = mfma_tap2d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
+    if (r < 0 && tap2d_on(g, d->dtype, false)) r = mfma_tap2d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pwd16_conv_fwd(g, x, w, bias, y, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
@@ -389,7 +390,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
   if (!force_direct()) {
     int r = -1;
     if (tap1d_on(d->dtype)) r = mfma_tap1d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
-    if (r < 0 && tap2d_on(g, d->dtype)) r = mfma_tap2d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
+    if (r < 0 && tap2d_on(g, d->dtype, true)) r = mfma_tap2d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && !skip(Options::SKIP_CELLS)) r = mfma_cells_conv_bwd_data(g, d->dtype, dy, w, dx, s);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype);

@@ -470,11 +470,12 @@ struct Tap1Plan {
   int C, H, T;           // of the source tensor, for the rows pass
 };
 
-// channels of the channels-last rows: the count padded to one the convolution kernels are compiled for
-int tap1d_cs(int C) {
+// channels of the channels-last rows: the count padded to one the 16-bit convolution kernels are compiled for (the fp32 ones take
+// any whole chunk)
+int tap1d_cs(int C, int esz) {
   for (int c : {32, 64, 96, 128, 256})
     if (C <= c) return c;
-  return 0;
+  return esz == 4 && C <= 512 ? (C + 31) / 32 * 32 : 0;
 }
 
 // taps per unrolled group of the bf16 kernels (fp32: 1)
@@ -487,7 +488,7 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
   if (g.OH != g.H || (long long)g.N * g.H > 65535) return false;
   const int Cc = bwd ? g.K : g.C, Mo = bwd ? g.C : g.K;
   // contraction channels padded to a count the kernel is compiled for
-  const int Cs = tap1d_cs(Cc);
+  const int Cs = tap1d_cs(Cc, esz);
   if (!Cs || Cc < 16) return false;
   const int cell = 16 / esz;
   const int KS = Cs / (2 * cell), DT = esz == 2 ? dt_of(KS) : 1;
@@ -978,7 +979,7 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   pl->TQ = TQ; pl->SS = g.sx;
   pl->odd = esz == 2 && g.OW % 2 != 0;
   p.rows = g.N * g.H; p.H = g.H; p.OW = g.OW; p.TS = g.W;
-  p.Cs = tap1d_cs(g.C);
+  p.Cs = tap1d_cs(g.C, esz);
   if (!p.Cs) return false;
   p.K = g.K; p.C = g.C; p.KW = g.KW; p.px = g.px;
   p.ktiles = (g.K + 63) / 64; p.ctiles = (g.C + 31) / 32;
@@ -1089,14 +1090,20 @@ int esz_of(int dtype) { return dtype == FLHIP_F32 ? 4 : dtype == FLHIP_BF16 || d
 
 }  // namespace
 
+int mfma_tap1d_cs(int C, int esz) { return tap1d_cs(C, esz); }
+void mfma_tap1d_rows_f32(const float* x, float* xr, int C, int H, int T, int Cs, int rows, hipStream_t s) {
+  launch_rows(x, xr, C, H, T, Cs, rows, s);
+}
+
 size_t mfma_tap1d_conv_ws(const ConvGeom& g, int dtype, bool bwd) {
+  if (dtype == FLHIP_F32) return mfma_tap1d_split_ws(g, bwd, nullptr);
   Tap1Plan pl;
   return esz_of(dtype) && tap1d_plan(g, bwd, esz_of(dtype), &pl) ? pl.rows_bytes + pl.w_bytes : 0;
 }
 
 int mfma_tap1d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
                         void* ws, size_t ws_bytes) {
-  if (dtype == FLHIP_F32) return run_conv<float>(g, false, x, w, bias, y, s, ws, ws_bytes);
+  if (dtype == FLHIP_F32) return mfma_tap1d_split(g, false, x, w, bias, y, s, ws, ws_bytes);
   if (dtype == FLHIP_BF16) return run_conv<bf16_t>(g, false, x, w, bias, y, s, ws, ws_bytes);
   if (dtype == FLHIP_F16) return run_conv<f16_t>(g, false, x, w, bias, y, s, ws, ws_bytes);
   return -1;
@@ -1104,20 +1111,21 @@ int mfma_tap1d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void*
 
 int mfma_tap1d_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx, hipStream_t s, void* ws,
                              size_t ws_bytes) {
-  if (dtype == FLHIP_F32) return run_conv<float>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
+  if (dtype == FLHIP_F32) return mfma_tap1d_split(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   if (dtype == FLHIP_BF16) return run_conv<bf16_t>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   if (dtype == FLHIP_F16) return run_conv<f16_t>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   return -1;
 }
 
 size_t mfma_tap2d_conv_ws(const ConvGeom& g, int dtype, bool bwd) {
+  if (dtype == FLHIP_F32) return mfma_tap2d_split_ws(g, bwd);
   Tap1Plan pl;
   return esz_of(dtype) && tap2d_plan(g, bwd, esz_of(dtype), &pl) ? pl.rows_bytes + pl.w_bytes : 0;
 }
 
 int mfma_tap2d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
                         void* ws, size_t ws_bytes) {
-  if (dtype == FLHIP_F32) return run_conv2d<float>(g, false, x, w, bias, y, s, ws, ws_bytes);
+  if (dtype == FLHIP_F32) return mfma_tap2d_split(g, false, x, w, bias, y, s, ws, ws_bytes);
   if (dtype == FLHIP_BF16) return run_conv2d<bf16_t>(g, false, x, w, bias, y, s, ws, ws_bytes);
   if (dtype == FLHIP_F16) return run_conv2d<f16_t>(g, false, x, w, bias, y, s, ws, ws_bytes);
   return -1;
@@ -1125,7 +1133,7 @@ int mfma_tap2d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void*
 
 int mfma_tap2d_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx, hipStream_t s, void* ws,
                              size_t ws_bytes) {
-  if (dtype == FLHIP_F32) return run_conv2d<float>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
+  if (dtype == FLHIP_F32) return mfma_tap2d_split(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   if (dtype == FLHIP_BF16) return run_conv2d<bf16_t>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   if (dtype == FLHIP_F16) return run_conv2d<f16_t>(g, true, dy, w, nullptr, dx, s, ws, ws_bytes);
   return -1;
@@ -1140,6 +1148,10 @@ size_t mfma_tap1d_rows_bytes(const ConvGeom& g, int dtype) {
   Tap1Plan f;
   Tap1WPlan w;
   const int esz = esz_of(dtype);
+  if (dtype == FLHIP_F32) {
+    size_t rows = 0;
+    return mfma_tap1d_split_ws(g, false, &rows) && tap1d_wgrad_plan(g, esz, &w) && rows == w.rows_bytes ? rows : 0;
+  }
   return esz && tap1d_plan(g, false, esz, &f) && tap1d_wgrad_plan(g, esz, &w) && f.rows_bytes == w.rows_bytes ? w.rows_bytes : 0;
 }
 

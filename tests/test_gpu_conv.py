@@ -557,6 +557,85 @@ def test_forward_and_backward_data_without_workspace(shape):
     assert torch.equal(y0, y) and torch.equal(dx0, dx)
 
 
+# (planes, weights, stride): a tile's blocks 1 to 4 of 32 positions, 128 or 64 result channels, one or two slab rows per thread
+PARTS_CASES = [
+    ((1, 16, 1, 33), (32, 16, 1, 2), 1),            # the smallest of everything, one chunk
+    ((2, 320, 1, 70), (40, 320, 1, 5), 2),          # more channels than the 16-bit kernels take; phases of 3 and 2 taps
+    ((1, 17, 3, 200), (40, 17, 1, 32), 1),          # a second chunk of one channel, the most taps, rows of an image
+    ((16, 33, 1, 1500), (256, 33, 1, 5), 1),
+    ((16, 256, 1, 700), (200, 256, 1, 3), 2),
+    ((24, 130, 1, 900), (250, 130, 1, 21), 2),
+    ((24, 256, 1, 1500), (320, 256, 1, 2), 1),      # two slab rows per thread
+    ((1, 32, 4, 4), (32, 32, 3, 3), 1),             # planes smaller than a tile
+    ((2, 48, 1, 30), (40, 48, 3, 3), 1),
+    ((3, 512, 7, 7), (104, 512, 3, 3), 1),
+    ((40, 32, 56, 56), (130, 32, 3, 3), 1),         # wide rows: slabs of more than 256 rows
+    ((2, 33, 14, 9), (64, 33, 5, 5), 1),
+    ((1, 32, 9, 70), (40, 32, 3, 1), 1),            # no zero column
+    ((1, 40, 20, 100), (33, 40, 5, 7), 1),          # 35 taps
+    ((64, 64, 28, 28), (128, 64, 3, 3), 1),
+    ((64, 128, 20, 20), (40, 128, 5, 3), 1),
+]
+
+
+@pytest.mark.parametrize("xs,ws,stride", PARTS_CASES)
+def test_fp32_windows_in_three_parts(xs, ws, stride):
+    """fp32 windows whose operands are taken apart into bf16 parts, forward (with a bias) and backward-data, against float64.  Sums of
+    n rounded products in any order differ by about sqrt(n) units of 2^-24 in the 2-norm; allowed are twice that."""
+    import torch.nn.functional as F
+    from flashlight_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(sum(xs) + sum(ws))
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    pad = (ws[2] // 2, ws[3] // 2)
+    kw = dict(sx=stride, sy=1, px=pad[1], py=pad[0])
+    x, w, b = r(*xs), r(*ws), r(ws[0])
+    capi.set_option("TAP2D_ALL", "1")
+    try:
+        y = fa.conv2d(x, w, b, **kw)
+        dy = r(*y.shape)
+        dx = fa.conv2d_backward_data(dy, xs, w, **kw)
+    finally:
+        capi.set_option("TAP2D_ALL", None)
+    w2, geo = w.double().view(ws[0], -1), dict(kernel_size=ws[2:], padding=pad, stride=(1, stride))
+    want = torch.matmul(w2, F.unfold(x.double(), **geo)).view(y.shape) + b.double().view(1, -1, 1, 1)
+    back = F.fold(torch.matmul(w2.t().contiguous(), dy.double().flatten(2)), xs[2:], **geo)
+    for got, ref, n in ((y, want, w2.shape[1]), (dx, back, ws[0] * ws[2] * ws[3])):
+        err = float((got.double() - ref).norm() / ref.norm())
+        assert err <= 2 * (n ** 0.5 + 1) * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("xs,ws,stride", [((2, 80, 1, 300), (70, 80, 1, 9), 1), ((2, 80, 1, 300), (70, 80, 1, 9), 2), ((3, 64, 14, 14), (70, 64, 3, 3), 1)])
+def test_fp32_windows_in_three_parts_keep_what_bf16_cannot_hold(xs, ws, stride):
+    """Infinities, NaN and values that round to infinity in bf16 reach the results that they reach in fp32, and no others."""
+    import torch.nn.functional as F
+    from flashlight_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, w = torch.rand(*xs, generator=g, device="cuda") + 0.5, torch.rand(*ws, generator=g, device="cuda") + 0.5
+    x[0, 3, 0, 7], x[1, 9, 0, 2], x[0, 20, 0, 11], x[1, 1, 0, 5] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[5, 2] = 0.0
+    w[:, 1] *= 1e-3
+    pad = (ws[2] // 2, ws[3] // 2)
+    kw = dict(sx=stride, sy=1, px=pad[1], py=pad[0])
+    capi.set_option("TAP2D_ALL", "1")
+    try:
+        y = fa.conv2d(x, w, None, **kw)
+        dy = torch.rand(*y.shape, generator=g, device="cuda") + 0.5
+        dy[0, 1, 0, 3], dy[1, 2, 0, 4], dy[1, 69, 0, 9] = float("inf"), float("nan"), 3.4e38
+        dx = fa.conv2d_backward_data(dy, xs, w, **kw)
+    finally:
+        capi.set_option("TAP2D_ALL", None)
+    xc, wc = x.double().cpu().requires_grad_(), w.double().cpu()
+    want = F.conv2d(xc, wc, stride=(1, stride), padding=pad)
+    want.backward(dy.double().cpu())
+    for got, ref in ((y, want.detach()), (dx, xc.grad)):
+        got = got.double().cpu()
+        ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+        assert bool((got.isnan() == ref.isnan()).all()) and bool((got.isinf() == ref.isinf()).all())
+        inf, ok = ref.isinf(), ref.isfinite()
+        assert bool((got[inf] == ref[inf]).all()) and bool(ref.isnan().any()) and bool(inf.any())
+        assert float(((got[ok] - ref[ok]).abs() / ref[ok].abs()).max()) <= 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
