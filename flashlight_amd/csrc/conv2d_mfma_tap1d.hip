@@ -1,7 +1,7 @@
 // Convolutions with one-row windows (KH = 1, KW taps along the contiguous axis: the 21 x 1
 // windows of a wav2letter-style speech stack) on the matrix cores, forward, backward-data and
-// filter gradient, column stride 1 or 2; bf16 storage on v_mfma_f32_32x32x16_bf16 and fp32 on
-// v_mfma_f32_32x32x2_f32 (the same kernels compiled for either element type).
+// filter gradient, column stride 1 or 2; 16-bit storage on v_mfma_f32_32x32x16 (bf16 and IEEE half), and the filter gradient in fp32
+// too (its forward and backward-data: conv2d_mfma_tap_split.hip).
 //
 //   forward        y[m][o]  = sum_c sum_j w[m][c][j]  x[c][o*s + j - p]   (+ bias[m])
 //   backward-data  dx[c][u] = sum_m sum_j w[m][c][j] dy[m][(u + p - j) / s]   where s divides
@@ -12,13 +12,11 @@
 // boundary.  So two small passes first bring the operands into the order the instruction reads:
 //   rows     xr[sequence][position][Cs]: the source with its channels last, Cs = the channel
 //            count padded with zeros (tap1d_rows_kernel; a sequence is one (image, row) pair); a
-//            tap then shifts whole 16-byte cells (8 bf16 or 4 fp32 channels of one position);
+//            tap then shifts whole 16-byte cells (8 channels of one position);
 //   weights  wf[block of 32 result channels][tap][stage of 2 cells][lane][cell]: the fragment
 //            of every (tap, stage) exactly as the 64 lanes hold it, in the order the kernel walks
 //            (tap1d_weights_kernel); padded channels and taps are zero.
-// A stage is 16 bf16 channels (one matrix instruction per block) or 8 fp32 channels (four
-// instructions of 2 channels each: lane half h holds channels 4 h .. 4 h + 3 of the stage and
-// instruction e multiplies element e of both operands, so the four cover the stage).
+// A stage is 16 channels, one matrix instruction per block.
 // Backward-data over a stride of 2 is two interleaved stride-1 problems (the results of even
 // and of odd index take the taps of one parity each): "phases" of one workgroup, which
 // writes both so that its stores cover whole runs of dx.
@@ -35,7 +33,7 @@
 //     contiguous memory, fetched straight into registers RW stages ahead of its use.  No other
 //     wave needs it, so the main loop has no barrier.
 //   * Per stage a wave reads NB position fragments from LDS (two stages ahead of their use) and
-//     issues NB (bf16) or 4 NB (fp32) matrix instructions.
+//     issues NB matrix instructions.
 // Positions are the rows of the instruction tile: a lane holds 4 consecutive positions of one
 // result channel (8 with two phases), stored as one piece.
 #include <algorithm>
@@ -45,6 +43,7 @@
 
 #include "conv2d_mfma.h"
 #include "lds_direct.h"
+#include "split_f32.h"
 
 namespace flhip {
 namespace {
@@ -77,12 +76,6 @@ __device__ __forceinline__ void tap1d_mma(floatx16& acc, const uintx4_t& a, cons
 // two results rounded to the storage type, the first in the low half
 __device__ __forceinline__ uint32_t tap1d_pack(float a, float b, const bf16_t*) { return pack_bf16(a, b); }
 __device__ __forceinline__ uint32_t tap1d_pack(float a, float b, const f16_t*) { return pack_f16(a, b); }
-__device__ __forceinline__ uint32_t tap1d_pack(float, float, const float*) { return 0u; }   // (fp32 results are not packed)
-__device__ __forceinline__ void tap1d_mma(floatx16& acc, const uintx4_t& a, const uintx4_t& w, const float*) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[e]), __uint_as_float(w[e]), acc, 0, 0, 0);
-}
 
 struct Tap1Params {
   int rows, H;           // sequences (images x rows), rows per image
@@ -219,7 +212,7 @@ tap_weights_by_tap_kernel(const T* __restrict__ w, uintx4_t* __restrict__ wf, Ta
 
 // ---- the convolution ---------------------------------------------------------------------
 // KS stages per tap; DT taps per unrolled group; RW stages between a weight fragment's load and its use (RW divides
-// DT * KS; a bf16 stage is one matrix instruction per block, an fp32 stage four longer ones); SS source stride;
+// DT * KS); SS source stride;
 // NPH phases; NB blocks of 32 positions.
 // TD: the taps form a two-dimensional window over planes stacked in one sequence (see tap2d_plan); only the slab
 // offset of a tap and the addresses of the results differ.
@@ -371,7 +364,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   const int n = row / p.H, h = row - n * p.H;
   const long long rbase = (((long long)n * p.Mo + m) * p.H + h) * p.TOu;     // element offset of the result row
   const __amdgpu_buffer_rsrc_t drs = make_rsrc(dst, p.dst_bytes);
-  const bool aligned = ESZ == 4 || (rbase & 1) == 0;     // pieces start on 4-byte boundaries
+  const bool aligned = (rbase & 1) == 0;     // pieces start on 4-byte boundaries
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -385,11 +378,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
       const int u = o * NPH;
       if (aligned && u + 4 * NPH <= p.TOu) {      // (u is a multiple of 4)
         const int at = (int)((rbase + u) * ESZ);
-        if (ESZ == 4) {
-          __builtin_amdgcn_raw_buffer_store_b128(uintx4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, drs, at, 0, 0);
-          if (NPH == 2)
-            __builtin_amdgcn_raw_buffer_store_b128(uintx4_t{__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])}, drs, at + 16, 0, 0);
-        } else if (NPH == 1) {
+        if (NPH == 1) {
           const T* const tt = nullptr;
           const uintx2_t t = {tap1d_pack(v[0], v[1], tt), tap1d_pack(v[2], v[3], tt)};
           __builtin_amdgcn_raw_buffer_store_b64(t, drs, at, 0, 0);
@@ -478,11 +467,12 @@ int tap1d_cs(int C, int esz) {
   return esz == 4 && C <= 512 ? (C + 31) / 32 * 32 : 0;
 }
 
-// taps per unrolled group of the bf16 kernels (fp32: 1)
+// taps per unrolled group 
 int dt_of(int KS) { return KS >= 16 ? 1 : KS >= 8 ? 2 : KS == 6 ? 2 : KS == 4 ? 4 : KS == 2 ? 8 : 0; }
 
-// bwd = false: forward; true: backward-data.  esz: bytes per element (2: bf16, 4: fp32)
-bool tap1d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
+// bwd = false: forward; true: backward-data.
+bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
+  constexpr int esz = 2;
   if (g.KH != 1 || g.py != 0 || g.sy != 1 || g.dlx != 1 || g.groups != 1) return false;
   if (g.KW < 2 || g.KW > 32 || (g.sx != 1 && g.sx != 2)) return false;
   if (g.OH != g.H || (long long)g.N * g.H > 65535) return false;
@@ -490,8 +480,7 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
   // contraction channels padded to a count the kernel is compiled for
   const int Cs = tap1d_cs(Cc, esz);
   if (!Cs || Cc < 16) return false;
-  const int cell = 16 / esz;
-  const int KS = Cs / (2 * cell), DT = esz == 2 ? dt_of(KS) : 1;
+  const int KS = Cs / 16, DT = dt_of(KS);
   Tap1Params& p = pl->p;
   Tap1Weights& w = pl->w;
   std::memset(&p, 0, sizeof p);
@@ -541,12 +530,12 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
     span = std::max(span, p.d0[q] + p.nreal[q]);
   }
   const int CPR = 2 * KS + 1;
-  // three blocks of positions per wave; two where the slab of three does not fit (fp32, 256 channels, forward stride 2)
-  // 16-bit storage: two also where the workgroups of two still fit the compute units at once, so that more of the chip works on
+  // three blocks of positions per wave; two
+  // where the workgroups of two still fit the compute units at once, so that more of the chip works on
   // shorter tiles (250 -> 250 channels over 7 x 1111 frames, 168 -> 252 workgroups, with the copies: 49.7 -> 46.2 us, stride 2
   // 84 -> 126: 45.8 -> 41.6; but 12 x 900 frames, 240 -> 360: 47.5 -> 51.6)
   p.mtiles = (Mo + T1_BM - 1) / T1_BM;
-  const bool few = esz == 2 && (long long)p.rows * ((p.TO + 63) / 64) * p.mtiles <= mfma_num_cus();
+  const bool few = (long long)p.rows * ((p.TO + 63) / 64) * p.mtiles <= mfma_num_cus();
   pl->NB = 0;
   for (int nb = few ? 2 : 3; nb >= 2 && !pl->NB; --nb) {
     const int tp = 32 * nb;
@@ -558,7 +547,7 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
       p.SR = 2 * p.half;
     }
     pl->lds_bytes = (size_t)(((long long)p.SR * CPR + 63) / 64) * 1024;
-    if (pl->lds_bytes <= 160 * 1024 && (nb == 3 || esz == 2 || (KS == 32 && pl->SS == 2))) pl->NB = nb;
+    if (pl->lds_bytes <= 160 * 1024) pl->NB = nb;
   }
   if (!pl->NB) return false;
   p.ptiles = (p.TO + 32 * pl->NB - 1) / (32 * pl->NB);
@@ -585,12 +574,8 @@ int launch_conv(const Tap1Plan& pl, const T* xr, const uintx4_t* wf, const float
     return check_launch("conv2d (one-row windows)");
   };
   if (pl.NB == 2) {
-    if constexpr (sizeof(T) == 4 && KS == 32) return go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 2>);
-    if constexpr (sizeof(T) == 2) {
-      if (pl.p.nph == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 1, 2, 2>);
-      return pl.SS == 2 ? go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 2>) : go(tap1d_conv_kernel<T, KS, DT, RW, 1, 1, 2>);
-    }
-    return -1;
+    if (pl.p.nph == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 1, 2, 2>);
+    return pl.SS == 2 ? go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 2>) : go(tap1d_conv_kernel<T, KS, DT, RW, 1, 1, 2>);
   }
   if (pl.p.nph == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 1, 2, 3>);
   if (pl.SS == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 3>);
@@ -601,7 +586,7 @@ template <typename T>
 int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, void* dst, hipStream_t s,
              void* ws, size_t ws_bytes) {
   Tap1Plan pl;
-  if (!tap1d_plan(g, bwd, (int)sizeof(T), &pl)) return -1;
+  if (!tap1d_plan(g, bwd, &pl)) return -1;
   if (!ws || ws_bytes < pl.rows_bytes + pl.w_bytes) return -1;
   T* xr = static_cast<T*>(ws);
   uintx4_t* wf = reinterpret_cast<uintx4_t*>(static_cast<char*>(ws) + pl.rows_bytes);
@@ -613,22 +598,12 @@ int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const 
   }
   if (const int rc = check_launch("conv2d (one-row windows, operand passes)")) return rc;
   T* out = static_cast<T*>(dst);
-  if constexpr (sizeof(T) == 2) {
-    switch (pl.p.KS) {
-      case 2: return launch_conv<T, 2, 8, 16>(pl, xr, wf, bias, out, s);
-      case 4: return launch_conv<T, 4, 4, 16>(pl, xr, wf, bias, out, s);
-      case 6: return launch_conv<T, 6, 2, 12>(pl, xr, wf, bias, out, s);
-      case 8: return launch_conv<T, 8, 2, 16>(pl, xr, wf, bias, out, s);
-      default: return launch_conv<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
-    }
-  } else {
-    switch (pl.p.KS) {
-      case 4: return launch_conv<T, 4, 1, 4>(pl, xr, wf, bias, out, s);
-      case 8: return launch_conv<T, 8, 1, 4>(pl, xr, wf, bias, out, s);
-      case 12: return launch_conv<T, 12, 1, 4>(pl, xr, wf, bias, out, s);
-      case 16: return launch_conv<T, 16, 1, 4>(pl, xr, wf, bias, out, s);
-      default: return launch_conv<T, 32, 1, 4>(pl, xr, wf, bias, out, s);
-    }
+  switch (pl.p.KS) {
+    case 2: return launch_conv<T, 2, 8, 16>(pl, xr, wf, bias, out, s);
+    case 4: return launch_conv<T, 4, 4, 16>(pl, xr, wf, bias, out, s);
+    case 6: return launch_conv<T, 6, 2, 12>(pl, xr, wf, bias, out, s);
+    case 8: return launch_conv<T, 8, 2, 16>(pl, xr, wf, bias, out, s);
+    default: return launch_conv<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
   }
 }
 
@@ -639,17 +614,17 @@ int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const 
 // tap 3 r + s sits r P + s rows into it.  Backward-data is the same walk over dy with the taps in reverse order and
 // the roles of the two channel counts exchanged.  (H + 1)(W + 1) / (H W) of the positions are computed: 1.15 for
 // 14 x 14 planes, 1.31 for 7 x 7.
-bool tap2d_plan(const ConvGeom& g, bool bwd, int esz, Tap1Plan* pl) {
+bool tap2d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
+  constexpr int esz = 2;
   if (g.KH != 3 || g.KW != 3 || g.sy != 1 || g.sx != 1 || g.py != 1 || g.px != 1 || g.dly != 1 || g.dlx != 1 || g.groups != 1)
     return false;
   const int Cc = bwd ? g.K : g.C, Mo = bwd ? g.C : g.K;
   // contraction channels padded to a count the two-dimensional kernel is compiled for
   int Cs = 0;
   for (int c : {128, 256, 512})
-    if (!Cs && Cc <= c && (esz == 2 || c <= 256)) Cs = c;
+    if (!Cs && Cc <= c) Cs = c;
   if (!Cs || Cc <= Cs / 2) return false;
-  const int cell = 16 / esz;
-  const int KS = Cs / (2 * cell), DT = esz == 2 ? dt_of(KS) : 1;
+  const int KS = Cs / 16, DT = dt_of(KS);
   Tap1Params& p = pl->p;
   Tap1Weights& w = pl->w;
   std::memset(&p, 0, sizeof p);
@@ -709,7 +684,7 @@ template <typename T>
 int run_conv2d(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, void* dst, hipStream_t s,
                void* ws, size_t ws_bytes) {
   Tap1Plan pl;
-  if (!tap2d_plan(g, bwd, (int)sizeof(T), &pl)) return -1;
+  if (!tap2d_plan(g, bwd, &pl)) return -1;
   if (!ws || ws_bytes < pl.rows_bytes + pl.w_bytes) return -1;
   T* xr = static_cast<T*>(ws);
   uintx4_t* wf = reinterpret_cast<uintx4_t*>(static_cast<char*>(ws) + pl.rows_bytes);
@@ -723,14 +698,10 @@ int run_conv2d(const ConvGeom& g, bool bwd, const void* src, const void* w, cons
   }
   if (const int rc = check_launch("conv2d (3x3 windows over stacked planes, operand passes)")) return rc;
   T* out = static_cast<T*>(dst);
-  if constexpr (sizeof(T) == 2) {
-    switch (pl.p.KS) {
-      case 8: return launch_conv2d<T, 8, 2, 16>(pl, xr, wf, bias, out, s);
-      case 16: return launch_conv2d<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
-      default: return launch_conv2d<T, 32, 1, 16>(pl, xr, wf, bias, out, s);
-    }
-  } else {
-    return pl.p.KS == 16 ? launch_conv2d<T, 16, 1, 4>(pl, xr, wf, bias, out, s) : launch_conv2d<T, 32, 1, 4>(pl, xr, wf, bias, out, s);
+  switch (pl.p.KS) {
+    case 8: return launch_conv2d<T, 8, 2, 16>(pl, xr, wf, bias, out, s);
+    case 16: return launch_conv2d<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
+    default: return launch_conv2d<T, 32, 1, 16>(pl, xr, wf, bias, out, s);
   }
 }
 
@@ -774,12 +745,10 @@ template <typename T, int TQ, int SS, bool ODD>
 __global__ void __launch_bounds__(256, 1)
 tap1d_wgrad_kernel(Tap1WParams p, const T* __restrict__ xr, const T* __restrict__ dy, float* __restrict__ part) {
   extern __shared__ uintx4_t t1_slab[];
-  constexpr int CELL = Tap1Elem<T>::CELL;
-  constexpr int ESZ = (int)sizeof(T);
-  constexpr bool LO = ESZ == 2;
+  constexpr int CELL = 8, ESZ = 2;
   constexpr int STEP = 2 * CELL;                // positions per step: a lane half holds CELL consecutive ones
   constexpr int RC = 32 / CELL;                 // cells of a slab row in use (32 channels)
-  constexpr int PC = LO ? (SS == 1 ? 6 : 5) : RC + 1;   // cells per slab row
+  constexpr int PC = SS == 1 ? 6 : 5;           // cells per slab row
   constexpr int PE = PC * CELL;                 // the same in elements
   constexpr int RD = 4;                         // steps between a dy fragment's load and its use
   const int tid = threadIdx.x, lane = tid & 63;
@@ -802,15 +771,14 @@ tap1d_wgrad_kernel(Tap1WParams p, const T* __restrict__ xr, const T* __restrict_
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][t][r] = 0.f;
   // a tile of ones for the bias slot
-  const uint32_t one = !LO ? 0x3f800000u : std::is_same<T, f16_t>::value ? 0x3c003c00u : 0x3f803f80u;
+  const uint32_t one = std::is_same<T, f16_t>::value ? 0x3c003c00u : 0x3f803f80u;
   const uintx4_t ones = {one, one, one, one};
   const int bias_slot = p.KW - wave * TQ;       // this wave's slot index of the bias gradient (outside 0 .. TQ - 1: none)
 
-  // this lane's first read of a step at the wave's first tap.  bf16: transposing reads, row SS * (fs / 4) (+ 8 SS fg),
-  // channels 16 fq + 4 (fs % 4) .. + 3.  fp32: four 4-byte reads, rows SS * (4 fg + e), channel fr.
+  // this lane's first (transposing) read of a step at the wave's first tap: row SS * (fs / 4) (+ 8 SS fg), channels
+  // 16 fq + 4 (fs % 4) .. + 3
   const T* const slabT = reinterpret_cast<const T*>(t1_slab);
-  const int blane = LO ? ((8 * fg + (fs >> 2)) * SS + wave * TQ) * PE + 16 * fq + 4 * (fs & 3)
-                       : (4 * fg * SS + wave * TQ) * PE + fr;
+  const int blane = ((8 * fg + (fs >> 2)) * SS + wave * TQ) * PE + 16 * fq + 4 * (fs & 3);
 
   const int u0 = split * p.upw, u1 = min(u0 + p.upw, p.units);
   for (int u = u0; u < u1; ++u) {
@@ -855,7 +823,7 @@ tap1d_wgrad_kernel(Tap1WParams p, const T* __restrict__ xr, const T* __restrict_
       const int cnt = tailn ? tailn - CELL * fg : CELL;
 #pragma unroll
       for (int d = 0; d < 4; ++d)
-        tmask[d] = LO ? (cnt >= 2 * d + 2 ? 0xffffffffu : cnt == 2 * d + 1 ? 0x0000ffffu : 0u) : (cnt > d ? 0xffffffffu : 0u);
+        tmask[d] = cnt >= 2 * d + 2 ? 0xffffffffu : cnt == 2 * d + 1 ? 0x0000ffffu : 0u;
     }
     uintx4_t aq[RD][2];
     uint32_t ax[ODD ? RD : 1][2];                 // ODD: the word behind each fragment
@@ -883,16 +851,10 @@ tap1d_wgrad_kernel(Tap1WParams p, const T* __restrict__ xr, const T* __restrict_
     // the slab fragment of slot t + 1 is read while slot t is multiplied (the first slot of a step behind the last
     // of the step before)
     auto bread = [&](const T* at) __attribute__((always_inline)) {
-      if constexpr (LO) {
-        const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)at);
-        const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + 4 * SS * PE));
-        const uintx2_t l2 = __builtin_bit_cast(uintx2_t, lo), h2 = __builtin_bit_cast(uintx2_t, hi);
-        return uintx4_t{l2.x, l2.y, h2.x, h2.y};
-      } else {
-        lds_f1 f = (lds_f1)at;
-        return uintx4_t{__float_as_uint(f[0]), __float_as_uint(f[SS * PE]), __float_as_uint(f[2 * SS * PE]),
-                        __float_as_uint(f[3 * SS * PE])};
-      }
+      const shortx4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)at);
+      const shortx4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + 4 * SS * PE));
+      const uintx2_t l2 = __builtin_bit_cast(uintx2_t, lo), h2 = __builtin_bit_cast(uintx2_t, hi);
+      return uintx4_t{l2.x, l2.y, h2.x, h2.y};
     };
     uintx4_t bnext = bread(slabT + blane);
 #define T1W_STEP(I)                                                                                       \
@@ -933,6 +895,152 @@ tap1d_wgrad_kernel(Tap1WParams p, const T* __restrict__ xr, const T* __restrict_
         const int kl = a * 32 + (r >> 2) * 8 + fg * 4 + (r & 3);
         out[t * 2048 + kl * 32 + fr] = acc[a][t][r];
       }
+  }
+}
+
+// The same in fp32: dy and the rows in three bf16 parts (split_f32.h), six products in place of one, two accumulators.
+// A workgroup owns one of the tile's two blocks of 32 filters (TQ slots per wave: 32 TQ registers of accumulators, and two workgroups
+// still share a compute unit, so that one multiplies while the other brings in its slab).  The slab's rows are taken apart when
+// they go to LDS, [row][part][32 channels] - 12 cells a row, 14 for stride 2, which keeps the four rows of a transposing read on
+// distinct banks - and dy in registers, by each wave for itself (44 vector instructions to 6 TQ products).
+// Measured, us with the sum of the tiles (before: v_mfma_f32_32x32x2_f32, 0.7 of its pipe), 21 taps: 250 -> 250 channels, 16 x 1500 frames
+// 592 -> 363, stride 2 315 -> 197, 80 -> 250 318 -> 163; error in the 2-norm 9.8e-7 -> 3.4e-7.
+constexpr int t1ws_cells(int SS) { return SS == 1 ? 12 : 14; }
+
+template <int TQ, int SS>
+__global__ void __launch_bounds__(256, 2)
+tap1d_wgrad_split_kernel(Tap1WParams p, const float* __restrict__ xr, const float* __restrict__ dy, float* __restrict__ part) {
+  extern __shared__ uintx4_t t1_slab[];
+  constexpr int ROW = t1ws_cells(SS) * 16;      // bytes
+  constexpr int RD = 2;                         // steps between a dy fragment's load and its use
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int split = blockIdx.x, tile = blockIdx.y >> 1, fb = blockIdx.y & 1;
+  const int kt = tile / p.ctiles, ct = tile - kt * p.ctiles;
+  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(xr, p.src_bytes), drs = make_rsrc(dy, p.dy_bytes);
+  const int fr = lane & 31, fg = lane >> 5, fq = (lane >> 4) & 1, fs = lane & 15;
+  if (kt * 64 + fb * 32 >= p.K) return;         // (nobody reads that half of the tile)
+  const int k = kt * 64 + fb * 32 + fr;
+
+  floatx16 big[TQ], small[TQ];
+#pragma unroll
+  for (int t = 0; t < TQ; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) big[t][r] = small[t][r] = 0.f;
+  const int bias_slot = p.KW - wave * TQ;
+  char* const slab = reinterpret_cast<char*>(t1_slab);
+  // this lane's first read of a step at the wave's first tap: row SS * (fs / 4) (+ 8 SS fg), channels 16 fq + 4 (fs % 4) .. + 3
+  const int blane = ((8 * fg + (fs >> 2)) * SS + wave * TQ) * ROW + 32 * fq + 8 * (fs & 3);
+
+  const int u0 = split * p.upw, u1 = min(u0 + p.upw, p.units);
+  for (int u = u0; u < u1; ++u) {
+    const int seq = u / p.tsplit, tr = u - seq * p.tsplit;
+    const int t0 = tr * p.TL, oend = min(p.OW, t0 + p.TL);
+    if (t0 >= oend) continue;
+    const int nsteps = (oend - t0 + 15) / 16, tailn = (oend - t0) % 16;
+    const int n = seq / p.H, h = seq - n * p.H;
+    const int aoff = k < p.K ? ((((n * p.K + k) * p.H + h) * p.OW) + t0 + 8 * fg) * 4 : T1_OOB;
+    uintx4_t raw[RD][2];
+    auto dy_load = [&](int i, int st) __attribute__((always_inline)) {
+      const int off = st < nsteps ? aoff : T1_OOB;
+      raw[i][0] = __builtin_amdgcn_raw_buffer_load_b128(drs, off, st * 64, 0);
+      raw[i][1] = __builtin_amdgcn_raw_buffer_load_b128(drs, off, st * 64 + 16, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < RD; ++i) dy_load(i, i);
+    if (u != u0) __syncthreads();                // every wave is done with the previous slab
+    // ---- slab: row R holds source position t0 * SS - px + R, channels 32 ct .. + 31; a thread takes 8 channels of a row
+    for (int i = tid; i < p.SRW * 4; i += 256) {
+      const int R = i >> 2, c = i & 3, sp = t0 * SS - p.px + R;
+      const int off = (unsigned)sp < (unsigned)p.TS ? ((seq * p.TS + sp) * p.Cs + ct * 32 + 8 * c) * 4 : T1_OOB;
+      const uintx4_t v0 = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0), v1 = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 16, 0);
+      const Split2 s0 = split2(__uint_as_float(v0.x), __uint_as_float(v0.y)), s1 = split2(__uint_as_float(v0.z), __uint_as_float(v0.w));
+      const Split2 s2 = split2(__uint_as_float(v1.x), __uint_as_float(v1.y)), s3 = split2(__uint_as_float(v1.z), __uint_as_float(v1.w));
+      char* const at = slab + R * ROW + 16 * c;
+      *reinterpret_cast<uintx4_t*>(at) = uintx4_t{s0.h, s1.h, s2.h, s3.h};
+      *reinterpret_cast<uintx4_t*>(at + 64) = uintx4_t{s0.m, s1.m, s2.m, s3.m};
+      *reinterpret_cast<uintx4_t*>(at + 128) = uintx4_t{s0.l, s1.l, s2.l, s3.l};
+    }
+    __syncthreads();
+    const char* bp = slab + blane;
+    for (int st0 = 0; st0 < nsteps; st0 += RD) {
+#pragma unroll
+      for (int i = 0; i < RD; ++i) {
+        const int st = st0 + i;                  // (a step past the last: dy reads zero there, the rows are those of the last)
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(raw[i][e >> 2][e & 3]);
+        if (tailn && st == nsteps - 1) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = 8 * fg + e < tailn ? v[e] : 0.f;
+        }
+        uintx4_t a[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const Split2 s = split2(v[2 * e], v[2 * e + 1]);
+          a[0][e] = s.h; a[1][e] = s.m; a[2][e] = s.l;
+        }
+        dy_load(i, st + RD);
+#pragma unroll
+        for (int t = 0; t < TQ; ++t) {
+          uintx4_t b[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const char* const at = bp + t * ROW + 64 * q;
+            const uintx2_t lo = __builtin_bit_cast(uintx2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)at));
+            const uintx2_t hi = __builtin_bit_cast(uintx2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + 4 * SS * ROW)));
+            b[q] = uintx4_t{lo.x, lo.y, hi.x, hi.y};
+          }
+          if (t == bias_slot) {                  // dy times ones
+            b[0] = uintx4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+            b[1] = b[2] = uintx4_t{0u, 0u, 0u, 0u};
+          }
+          split_mma(big[t], small[t], a, b);
+        }
+        if (st + 1 < nsteps) bp += 16 * SS * ROW;
+      }
+    }
+  }
+
+  bool bad = false;
+#pragma unroll
+  for (int t = 0; t < TQ; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      big[t][r] += small[t][r];
+      bad |= not_finite(big[t][r]);
+    }
+  if (__builtin_amdgcn_ballot_w64(bad)) {          // once more with the operands as they are
+#pragma unroll
+    for (int t = 0; t < TQ; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) big[t][r] = 0.f;
+#pragma unroll 1
+    for (int u = u0; u < u1; ++u) {
+      const int seq = u / p.tsplit, t0 = (u - seq * p.tsplit) * p.TL, oend = min(p.OW, t0 + p.TL);
+      const int n = seq / p.H, h = seq - n * p.H;
+#pragma unroll 1
+      for (int o = t0 + fg; o < oend + fg; o += 2) {
+        const bool in = o < oend;
+        const float a = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, in && k < p.K ? (((n * p.K + k) * p.H + h) * p.OW + o) * 4 : T1_OOB, 0, 0));
+#pragma unroll
+        for (int t = 0; t < TQ; ++t) {
+          const int sp = o * SS - p.px + wave * TQ + t;
+          const float x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              xrs, in && (unsigned)sp < (unsigned)p.TS ? ((seq * p.TS + sp) * p.Cs + ct * 32 + fr) * 4 : T1_OOB, 0, 0));
+          big[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, t == bias_slot ? 1.f : x, big[t], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  // ---- the tile: element r of slot t: filter 32 fb + 8 (r / 4) + 4 fg + r % 4, channel fr
+  float* out = part + ((size_t)(split * (p.ktiles * p.ctiles) + tile) * (4 * TQ) + wave * TQ) * 2048;
+#pragma unroll
+  for (int t = 0; t < TQ; ++t) {
+    if (wave * TQ + t > p.KW) continue;          // an unused slot
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[t * 2048 + (fb * 32 + (r >> 2) * 8 + fg * 4 + (r & 3)) * 32 + fr] = big[t][r];
   }
 }
 
@@ -987,7 +1095,7 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   const long long yb = (long long)g.N * g.K * g.H * g.OW * esz;
   if (rb >= (1ll << 31) || yb >= (1ll << 31)) return false;
   const int tiles = p.ktiles * p.ctiles;
-  const int PC = esz == 2 ? (g.sx == 1 ? 6 : 5) : 9;
+  const int PC = esz == 2 ? (g.sx == 1 ? 6 : 5) : t1ws_cells(g.sx), most = esz == 2 ? 150 * 1024 : 80 * 1024;
   const int cus = mfma_num_cus();
   // ranges of ceil(OW / tsplit) positions; false: the slab of one does not fit in LDS
   auto split = [&](int tsplit) {
@@ -996,11 +1104,11 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
     pl->lds_bytes = (size_t)(((long long)p.SRW * PC + 63) / 64) * 1024;
     p.tsplit = (g.OW + p.TL - 1) / p.TL;
     p.units = p.rows * p.tsplit;
-    return pl->lds_bytes <= 150 * 1024;
+    return pl->lds_bytes <= (size_t)most;
   };
   if (esz == 4) {
-    // fp32 is bound by the matrix pipe: enough workgroups for the chip, rather with a last round that is half full than of
-    // twice the length
+    // fp32 is bound by the matrix pipe: enough workgroups for the chip (a tile is two of them, and two share a compute unit), rather
+    // with a last round that is half full than of twice the length
     const int want = (cus + tiles - 1) / tiles;
     for (int tsplit = std::max(1, (want + p.rows - 1) / p.rows); !split(tsplit); ++tsplit)
       if (p.TL <= 16) return false;
@@ -1052,10 +1160,18 @@ int launch_wgrad(const Tap1WPlan& pl, const T* xr, const T* dy, float* part, hip
     hipLaunchKernelGGL(kernel, grid, dim3(256), pl.lds_bytes, s, pl.p, xr, dy, part);
     return check_launch("conv2d_bwd_filter (one-row windows)");
   };
-  if constexpr (sizeof(T) == 2) {
+  if constexpr (sizeof(T) == 4) {
+    const dim3 halves(grid.x, 2 * grid.y);
+    auto go32 = [&](auto kernel) {
+      if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), pl.lds_bytes)) return -1;
+      hipLaunchKernelGGL(kernel, halves, dim3(256), pl.lds_bytes, s, pl.p, xr, dy, part);
+      return check_launch("conv2d_bwd_filter (one-row windows, fp32 in three parts)");
+    };
+    return pl.SS == 2 ? go32(tap1d_wgrad_split_kernel<TQ, 2>) : go32(tap1d_wgrad_split_kernel<TQ, 1>);
+  } else {
     if (pl.odd) return pl.SS == 2 ? go(tap1d_wgrad_kernel<T, TQ, 2, true>) : go(tap1d_wgrad_kernel<T, TQ, 1, true>);
+    return pl.SS == 2 ? go(tap1d_wgrad_kernel<T, TQ, 2, false>) : go(tap1d_wgrad_kernel<T, TQ, 1, false>);
   }
-  return pl.SS == 2 ? go(tap1d_wgrad_kernel<T, TQ, 2, false>) : go(tap1d_wgrad_kernel<T, TQ, 1, false>);
 }
 
 template <typename T>
@@ -1098,7 +1214,7 @@ void mfma_tap1d_rows_f32(const float* x, float* xr, int C, int H, int T, int Cs,
 size_t mfma_tap1d_conv_ws(const ConvGeom& g, int dtype, bool bwd) {
   if (dtype == FLHIP_F32) return mfma_tap1d_split_ws(g, bwd, nullptr);
   Tap1Plan pl;
-  return esz_of(dtype) && tap1d_plan(g, bwd, esz_of(dtype), &pl) ? pl.rows_bytes + pl.w_bytes : 0;
+  return esz_of(dtype) && tap1d_plan(g, bwd, &pl) ? pl.rows_bytes + pl.w_bytes : 0;
 }
 
 int mfma_tap1d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
@@ -1120,7 +1236,7 @@ int mfma_tap1d_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const
 size_t mfma_tap2d_conv_ws(const ConvGeom& g, int dtype, bool bwd) {
   if (dtype == FLHIP_F32) return mfma_tap2d_split_ws(g, bwd);
   Tap1Plan pl;
-  return esz_of(dtype) && tap2d_plan(g, bwd, esz_of(dtype), &pl) ? pl.rows_bytes + pl.w_bytes : 0;
+  return esz_of(dtype) && tap2d_plan(g, bwd, &pl) ? pl.rows_bytes + pl.w_bytes : 0;
 }
 
 int mfma_tap2d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
@@ -1152,7 +1268,7 @@ size_t mfma_tap1d_rows_bytes(const ConvGeom& g, int dtype) {
     size_t rows = 0;
     return mfma_tap1d_split_ws(g, false, &rows) && tap1d_wgrad_plan(g, esz, &w) && rows == w.rows_bytes ? rows : 0;
   }
-  return esz && tap1d_plan(g, false, esz, &f) && tap1d_wgrad_plan(g, esz, &w) && f.rows_bytes == w.rows_bytes ? w.rows_bytes : 0;
+  return esz && tap1d_plan(g, false, &f) && tap1d_wgrad_plan(g, esz, &w) && f.rows_bytes == w.rows_bytes ? w.rows_bytes : 0;
 }
 
 int mfma_tap1d_wgrad(const ConvGeom& g, int dtype, const void* x, const void* dy, float* dw, float* db, void* ws, size_t ws_bytes,

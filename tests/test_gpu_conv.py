@@ -636,6 +636,46 @@ def test_fp32_windows_in_three_parts_keep_what_bf16_cannot_hold(xs, ws, stride):
         assert float(((got[ok] - ref[ok]).abs() / ref[ok].abs()).max()) <= 1e-5
 
 
+@pytest.mark.parametrize("xs,k,kw,stride", [
+    ((1, 16, 1, 16), 32, 6, 1),          # one step of one range; half of a tile's filters
+    ((2, 33, 2, 47), 33, 7, 2),          # the other half with one filter, rows of an image, a last step of 8 positions
+    ((3, 320, 1, 131), 70, 11, 1),       # more channels than the 16-bit kernels' rows
+    ((5, 40, 1, 700), 96, 15, 2),        # several ranges, an odd number of steps
+    ((7, 64, 1, 1601), 130, 19, 1),
+    ((9, 100, 1, 500), 64, 23, 1),       # every slot of six in use, the bias gradient in the last
+])
+@pytest.mark.parametrize("special", [False, True])
+def test_fp32_one_row_filter_gradient_in_three_parts(xs, k, kw, stride, special):
+    """Against float64; sums of n rounded products differ by about sqrt(n) units of 2^-24, allowed are twice that.  special: infinities,
+    NaN and values that bf16 cannot hold reach the gradients that they reach in fp32, and no others."""
+    import torch.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(kw)
+    x = torch.randn(*xs, generator=g, device="cuda")
+    geo = dict(sx=stride, sy=1, px=kw // 2, py=0)
+    to = (xs[3] + 2 * (kw // 2) - kw) // stride + 1
+    dy = torch.randn(xs[0], k, xs[2], to, generator=g, device="cuda")
+    if special:
+        x, dy = x.abs() + 0.5, dy.abs() + 0.5
+        x[0, 3, 0, 5], x[0, 7, 0, 9], x[0, 9, 0, 1] = float("inf"), float("nan"), 3.4e38
+        dy[0, :, 0, :13] = 0.5               # (times 3.4e38: no product of finite values overflows but the one of two such)
+        dy[0, 2, 0, 1], dy[0, 30, 0, 2], dy[:, 1] = float("-inf"), 3.4e38, 1e-3
+    ws = (k, xs[1], 1, kw)
+    dw, db = fa.conv2d_backward_filter_bias(dy, x, ws, True, **geo)
+    cols = F.unfold(x.double().transpose(1, 2).reshape(-1, xs[1], 1, xs[3]), (1, kw), padding=(0, kw // 2), stride=(1, stride))
+    d2 = dy.double().transpose(1, 2).reshape(-1, k, to)
+    n = cols.shape[0] * to
+    want = d2.transpose(0, 1).reshape(k, n) @ cols.permute(0, 2, 1).reshape(n, -1).contiguous()
+    for got, ref in ((dw.double().reshape(k, -1), want), (db.double(), d2.sum((0, 2)))):
+        if special:
+            ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+            assert bool((got.isnan() == ref.isnan()).all()) and bool((got.isinf() == ref.isinf()).all())
+            assert bool((got[ref.isinf()] == ref[ref.isinf()]).all())
+            got, ref = got[ref.isfinite()], ref[ref.isfinite()]
+            assert float(((got - ref).abs() / ref.abs()).max()) <= 1e-5
+        else:
+            assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
