@@ -127,6 +127,12 @@ size_t mfma_pwd16_wgrad_ws(const ConvGeom& g);
 long long mfma_slab16_conv_fwd_workgroups(const ConvGeom& g);
 int mfma_pwd16_wgrad(const ConvGeom& g, const void* x, const void* dy, float* dw, void* ws, size_t ws_bytes, hipStream_t s,
                      int dtype = FLHIP_BF16);
+// large products on tiles of 256 (conv2d_mfma_big_lo16.hip)
+int mfma_big16_halves(bool conv, long long images, int Kc, int Mo, int P);
+int mfma_big16(int dtype, bool bwd, long long images, int Kc, int Mo, int P, const void* src, const void* w, const float* bias,
+               const float* pos_bias, void* dst, const void* addend, int halves, hipStream_t s);
+bool mfma_big16_nt_pays(int M, int C);
+int mfma_big16_nt(int dtype, int M, int C, int K, const void* a, const void* b, const float* bias, void* out, hipStream_t s);
 int mfma_strip16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y,
                           hipStream_t s, int dtype);
 int mfma_strip16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, void* dx, hipStream_t s, int dtype);

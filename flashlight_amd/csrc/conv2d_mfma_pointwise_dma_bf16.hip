@@ -354,15 +354,21 @@ int pwd16_bm(const PwdParams& p) {
   return small ? 64 : PD_BM;
 }
 
-// grid and kernel variant for a filled-in PwdParams (Kc, Mo, P, Pc, ncells, nstages, ctiles and the byte sizes)
+// conv: a convolution (else a matrix product).  grid and kernel variant for a filled-in PwdParams (Kc, Mo, P, Pc, ncells, nstages, ctiles and the byte sizes)
 // slices > 1 (matrix products): the contraction in that many slices at most, their fp32 partial products at p.part
 template <typename E, bool BWD>
 int pwd16_go(PwdParams p, const void* src, const void* w, const float* bias, void* dst, const void* addend,
-             hipStream_t s, const char* what, int* slices = nullptr) {
+             hipStream_t s, const char* what, bool conv, int* slices = nullptr) {
   // tiles of 64 result channels when tiles of 128 would leave half of the CUs without a workgroup (7x7 planes
   // with 512 result channels at batch 64: 112 workgroups of 64 stages); the deep ring for grids of at most one
   // workgroup per CU.  FLHIP_PW16_PF = 1 / 4 forces the shallow / deep ring with tiles of 128, 2 / 8 with tiles of 64.
   const int cus = mfma_num_cus(), pf = options().pw16_pf;
+  const long long images = p.ncells / p.Pc;
+  const int halves = pf ? -1 : mfma_big16_halves(conv, images, p.Kc, p.Mo, p.P);
+  if (halves >= 0) {
+    if (slices) *slices = 1;
+    return mfma_big16(Lo16<E>::TAG, BWD, images, p.Kc, p.Mo, p.P, src, w, bias, p.pos_bias, dst, addend, halves, s);
+  }
   const int bm = pwd16_bm(p);
   const bool small = bm == 64;
   p.mtiles = (p.Mo + bm - 1) / bm;
@@ -417,7 +423,7 @@ int launch_pwd16(const ConvGeom& g, const void* src, const void* w, const float*
   p.P = g.H * g.W;
   if (!pwd16_sizes(&p, g.N)) return -1;
   return pwd16_go<E, BWD>(p, src, w, bias, dst, addend, s,
-                          BWD ? "conv2d_bwd_data 1x1 (bf16 mfma, direct-to-LDS)" : "conv2d_fwd 1x1 (bf16 mfma, direct-to-LDS)");
+                          BWD ? "conv2d_bwd_data 1x1 (bf16 mfma, direct-to-LDS)" : "conv2d_fwd 1x1 (bf16 mfma, direct-to-LDS)", true);
 }
 
 
@@ -743,6 +749,7 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
     p.dup = (8 - K % 8) % 8;
     const long long xb = (long long)M * K * 2, db = (long long)N * K * 2;
     if (xb >= (1ll << 31) || db >= (1ll << 31)) return -1;
+    if (!options().pw16_pf && mfma_big16_nt_pays(N, M)) return mfma_big16_nt(dtype, N, M, K, B, A, bias_rows, C, s);
     p.x_bytes = (unsigned)xb;
     p.dy_bytes = (unsigned)db;
     p.ncells = p.Pc;
@@ -768,12 +775,12 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
   p.pos_bias = bias_rows;
   return by_lo16(dtype, [&](auto* e_) {
     using E = FLHIP_T_OF(e_);
-    if (mode == 0) return pwd16_go<E, false>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B, 16-bit mfma)");
+    if (mode == 0) return pwd16_go<E, false>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B, 16-bit mfma)", false);
     const size_t per = (size_t)M * N * sizeof(float);
     int slices = ws ? (int)std::min<size_t>(ws_bytes / per, 32) : 1;
-    if (slices <= 1) return pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)");
+    if (slices <= 1) return pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false);
     p.part = static_cast<float*>(ws);
-    const int rc = pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", &slices);
+    const int rc = pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false, &slices);
     if (rc != 0 || slices <= 1) return rc;
     const size_t n = (size_t)M * N;
     hipLaunchKernelGGL(gemm16_sum_slices_kernel<E>, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,

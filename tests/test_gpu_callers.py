@@ -334,6 +334,32 @@ def test_matmul_fp32_at_the_size_of_a_speech_model():
         assert not bad.any(), (ta, tb, int(bad.sum()), np.argwhere(bad)[:4].tolist())
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (3083, 2570, 264),          # 143 tiles of 256 x 256; rows of no whole cells, a last stage of 8
+    (4100, 4106, 40),           # 289: the last 33 in halves, some of those past the last row
+    (3330, 2826, 32),           # one stage: fewer than the ring holds
+    (3080, 2564, 127),          # a last cell that repeats one element
+    (7000, 1290, 1001)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_matmul_in_16_bit_storage_on_large_tiles(M, N, K, mode, dtype):
+    """Products of many tiles, against the fp32 product of the same operands: one rounding per element, and sums in another order."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    B = torch.randn(K, N, generator=g, device="cuda").to(dtype)
+    b = torch.randn(M, generator=g, device="cuda") if mode < 2 else None
+    import ctypes as C
+    from flashlight_amd import capi
+    Ad, Bd = (A if mode == 1 else A.t()).contiguous(), (B if mode == 2 else B.t()).contiguous()
+    out = torch.full((N, M), float("nan"), device="cuda", dtype=dtype)
+    P = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None
+    capi.check(capi.lib().flhip_matmul(P(Ad), P(Bd), P(out), M, N, K, int(mode == 1), int(mode == 2), P(b), capi.BF16 if dtype == torch.bfloat16 else capi.F16,
+                                       C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    want = (A.float() @ B.float()).t() + (b if b is not None else 0)
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert bool(((out.float() - want).abs() <= unit * want.abs() + 1e-4 * K ** 0.5).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_matmul_in_16_bit_storage_at_the_size_of_a_speech_model(dtype):
     """2000 x 2000 weights against 4000 frames, the three products of a layer's step; checked against numpy's

@@ -557,6 +557,27 @@ def test_forward_and_backward_data_without_workspace(shape):
     assert torch.equal(y0, y) and torch.equal(dx0, dx)
 
 
+@pytest.mark.parametrize("xs,k", [((120, 544, 7, 7), 2040), ((64, 1024, 14, 14), 1000), ((100, 576, 20, 20), 1016)])    # 216, 200, 628 tiles of 256
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_1x1_windows_on_large_tiles(xs, k, dtype):
+    """Large 1x1 layers, forward with a bias and backward-data with an addend, against the fp32 products of the same operands."""
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(k, xs[1], 1, 1, generator=g, device="cuda") / xs[1] ** 0.5).to(dtype)
+    b = torch.randn(k, generator=g, device="cuda")
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    y = ops.conv2d(x, w, b)
+    want = torch.matmul(w.float().view(k, -1), x.float().flatten(2)).view(y.shape) + b.view(1, -1, 1, 1)
+    assert bool(((y.float() - want).abs() <= unit * want.abs() + 1e-4).all())
+    wt = (torch.randn(xs[1], k, 1, 1, generator=g, device="cuda") / xs[1] ** 0.5).to(dtype)      # the same product as a gradient
+    add = torch.randn(*y.shape, generator=g, device="cuda").to(dtype)
+    dx = ops.conv2d_backward_data(x, tuple(y.shape), wt, addend=add)
+    want = torch.matmul(wt.float().view(xs[1], k).t().contiguous(), x.float().flatten(2)).view(y.shape)
+    total = want + add.float()      # the product is rounded, its sum with the addend once more: unit |p| + unit (|p + a| + unit |p|)
+    assert bool(((dx.float() - total).abs() <= unit * ((1 + unit) * want.abs() + total.abs()) + 1e-4).all())
+
+
 # (planes, weights, stride): a tile's blocks 1 to 4 of 32 positions, 128 or 64 result channels, one or two slab rows per thread
 PARTS_CASES = [
     ((1, 16, 1, 33), (32, 16, 1, 2), 1),            # the smallest of everything, one chunk
