@@ -204,6 +204,11 @@ size_t workspace_core(const RnnGeom& g) {
   const size_t bwd = wgrad_scratch_offset(g) + wgrad_scratch(g);
   return ((std::max(fwd, bwd) + 67) & ~(size_t)3) + 4;
 }
+// whether whole sequences may be launched: 16-byte pieces of the state, recurrent matrices in registers
+bool seq_holds(const RnnGeom& g) { return g.H % 4 == 0 && g.H <= 1024; }
+// floats of a step of the exchange, and the exchange of the call's sequence launches (behind the scratch; the layers use it in turn)
+size_t seq_row(const RnnGeom& g, size_t K) { return (size_t)g.B * ((K + 15) & ~(size_t)15); }
+
 // whether a wait inside one of the call's sequence launches has given up (one word before the scratch)
 uint32_t* seq_status(const RnnGeom& g, float* ws) { return reinterpret_cast<uint32_t*>(ws + workspace_core(g) - 4); }
 Scratch scratch_of(const RnnGeom& g, float* ws) {
@@ -217,7 +222,14 @@ Scratch scratch_of(const RnnGeom& g, float* ws) {
   n = std::max(n, gemm32_ws_bytes(2, g.H, GH, TB));
   return Scratch{ws + workspace_core(g), (n + 15) & ~(size_t)15};
 }
-size_t workspace_bytes(const RnnGeom& g) { return workspace_core(g) * sizeof(float) + scratch_of(g, nullptr).bytes; }
+float* seq_exchange(const RnnGeom& g, float* ws) {
+  const Scratch w = scratch_of(g, ws);
+  return static_cast<float*>(w.p) + w.bytes / sizeof(float);
+}
+size_t workspace_bytes(const RnnGeom& g) {
+  const size_t exchange = seq_holds(g) ? (size_t)g.D * g.T * seq_row(g, g.GH) : 0;
+  return (workspace_core(g) + exchange) * sizeof(float) + scratch_of(g, nullptr).bytes;
+}
 
 // the fused step kernels tile the hidden state by 16 and hold at most 64 batch columns
 bool fused_applies(const RnnGeom& g) {
@@ -259,6 +271,30 @@ __global__ void __launch_bounds__(256) rnn_add2_kernel(const float* a, const flo
     for (int k = 0; k < nb; ++k) v += b[(size_t)k * n + i];
   out[i] = v;
 }
+
+constexpr int SEQ_COLS = 16;
+constexpr int RNN_OOB = (int)0x80000000;
+// Where the values of a step are that the workgroups of a cluster hand to each other (the state, the gate gradients): a
+// buffer of its own, in chunks of 16 contraction indexes, and in a chunk in the order of the lanes that read it, [4][columns][4], so
+// that a wave's load is one piece of 1 KB.  Read from the rows of the reserve buffer / workspace it was 16 pieces of 64 bytes, a
+// row apart (8 KB: all in one channel of the caches): the 128 KB of a step of an LSTM of 512 units' backward pass took 10000 cycles of
+// its 13600.
+struct SeqRow {
+  int K, nc;            // contraction, columns of the cluster
+  int lane;             // byte offset of this lane's piece in a chunk, or RNN_OOB
+  size_t step;          // floats between steps
+  float* base;
+  __device__ __forceinline__ SeqRow(float* X, int K, int B, int b0) : K(K), nc(min(SEQ_COLS, B - b0)) {
+    const int Kp = (K + 15) & ~15, fr = threadIdx.x & 15, fg = threadIdx.x >> 4 & 3;
+    lane = fr < nc ? (fg * nc + fr) * 16 : RNN_OOB;
+    step = (size_t)B * Kp;
+    base = X + (size_t)b0 * Kp;
+  }
+  __device__ __forceinline__ int at(int k, int col) const { return (k >> 4) * (nc * 16) + ((k >> 2 & 3) * nc + col) * 4 + (k & 3); }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int st) const {
+    return make_rsrc(base + st * step, (unsigned)(K * nc * 4));      // (the last chunk's pieces beyond K are the buffer's end)
+  }
+};
 
 struct CellFwd {
   const float* xp;    // [B][GH] input projection (+ biases) of this time step
@@ -315,7 +351,7 @@ __device__ __forceinline__ void rnn_publish(float* p, float v, bool lost) {
 // (LSTM: c, else h).  lost (rp is NaN then): so are the state and what follows from it, also where the ReLU of a NaN is zero
 template <int MODE, bool SEQ = false>
 __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h, int H, const CellFwdIn<MODE>& in,
-                                                 const float* rp, bool lost = false) {
+                                                 const float* rp, bool lost = false, float* pub = nullptr) {
 #pragma clang fp contract(off)
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
   const size_t e = (size_t)b * H + h, q = (size_t)b * G * H + h;
@@ -323,7 +359,7 @@ __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h,
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float pre = in.xp[0] + rp[0];
     hv = MODE == RNN_RELU ? (pre > 0.f || (SEQ && lost) ? pre : 0.f) : tanhf(pre);
-    if (SEQ) rnn_publish(a.hn + e, hv, lost);
+    if (SEQ && pub) rnn_publish(pub, hv, lost);
     a.gt[q] = hv;
   } else if (MODE == RNN_LSTM) {
     const float ig = sigm(in.xp[0] + rp[0]), fg = sigm(in.xp[G > 1 ? 1 : 0] + rp[G > 1 ? 1 : 0]);
@@ -331,7 +367,7 @@ __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h,
     const float c = fmaf(fg, in.prev, ig * gg);
     keep = c;
     hv = og * tanhf(c);
-    if (SEQ) rnn_publish(a.hn + e, hv, lost);
+    if (SEQ && pub) rnn_publish(pub, hv, lost);
     a.cn[e] = c;
     if (a.cy) a.cy[e] = c;
     a.gt[q] = ig; a.gt[q + H] = fg; a.gt[q + 2 * H] = gg; a.gt[q + 3 * H] = og;
@@ -341,11 +377,11 @@ __device__ __forceinline__ float cell_fwd_finish(const CellFwd& a, int b, int h,
     const float ng = tanhf(fmaf(rg, rn, in.xp[G > 2 ? 2 : 0]));
     hv = fmaf(1.f - zg, ng, zg * in.prev);
     keep = hv;
-    if (SEQ) rnn_publish(a.hn + e, hv, lost);
+    if (SEQ && pub) rnn_publish(pub, hv, lost);
     a.rn[e] = rn;
     a.gt[q] = rg; a.gt[q + H] = zg; a.gt[q + 2 * H] = ng;
   }
-  if (!SEQ) a.hn[e] = hv;
+  a.hn[e] = hv;
   a.out[(size_t)b * a.ldo + h] = hv;
   if (a.hy) a.hy[e] = hv;
   return keep;
@@ -524,11 +560,11 @@ __device__ __forceinline__ CellBwdIn<MODE> cell_bwd_load(const CellBwd& a, int b
 // next step stays in *dc and *dir.  lost: as in the forward pass (rec is NaN)
 template <int MODE, bool SEQ = false>
 __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, int H, const CellBwdIn<MODE>& in,
-                                                float rec, float* dc_out = nullptr, float* dir_out = nullptr, bool lost = false) {
+                                                float rec, float* dc_out = nullptr, float* dir_out = nullptr, bool lost = false,
+                                                float* pub = nullptr, const SeqRow* row = nullptr, int col = 0) {
 #pragma clang fp contract(off)
-  auto put = [&](size_t i, float v) {
-    if (SEQ) rnn_publish(a.dgr + i, v, lost);
-    else a.dgr[i] = v;
+  auto put = [&](int g, float v) {
+    if (SEQ) rnn_publish(pub + row->at(g * H + h, col), v, lost);
   };
   constexpr int G = MODE == RNN_LSTM ? 4 : MODE == RNN_GRU ? 3 : 1;
   const size_t e = (size_t)b * H + h, q = (size_t)b * G * H + h;
@@ -537,7 +573,8 @@ __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, 
   if (MODE == RNN_RELU || MODE == RNN_TANH) {
     const float hv = in.gt[0];
     const float gp = MODE == RNN_RELU ? (hv > 0.f || (SEQ && lost) ? go : 0.f) : go * fmaf(-hv, hv, 1.f);
-    put(q, gp);
+    put(0, gp);
+    a.dgr[q] = gp;
     a.dgw[q] = gp;
   } else if (MODE == RNN_LSTM) {
     const float ig = in.gt[0], fg = in.gt[G > 1 ? 1 : 0], gg = in.gt[G > 2 ? 2 : 0], og = in.gt[G > 3 ? 3 : 0];
@@ -545,7 +582,8 @@ __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, 
     const float dc = fmaf(go * og, fmaf(-tc, tc, 1.f), in.dc);
     const float v0 = dc * gg * ig * (1.f - ig), v1 = dc * in.cp * fg * (1.f - fg);
     const float v2 = dc * ig * fmaf(-gg, gg, 1.f), v3 = go * tc * og * (1.f - og);
-    put(q, v0); put(q + H, v1); put(q + 2 * H, v2); put(q + 3 * H, v3);
+    put(0, v0); put(1, v1); put(2, v2); put(3, v3);
+    a.dgr[q] = v0; a.dgr[q + H] = v1; a.dgr[q + 2 * H] = v2; a.dgr[q + 3 * H] = v3;
     a.dgw[q] = v0; a.dgw[q + H] = v1; a.dgw[q + 2 * H] = v2; a.dgw[q + 3 * H] = v3;
     if (SEQ) *dc_out = dc * fg;
     else a.dc[e] = dc * fg;
@@ -553,7 +591,8 @@ __device__ __forceinline__ void cell_bwd_finish(const CellBwd& a, int b, int h, 
     const float rg = in.gt[0], zg = in.gt[G > 1 ? 1 : 0], ng = in.gt[G > 2 ? 2 : 0], rn = in.rn;
     const float dn = go * (1.f - zg) * fmaf(-ng, ng, 1.f);
     const float v0 = dn * rn * rg * (1.f - rg), v1 = go * (in.hp - ng) * zg * (1.f - zg);
-    put(q, v0); put(q + H, v1); put(q + 2 * H, dn * rg);
+    put(0, v0); put(1, v1); put(2, dn * rg);
+    a.dgr[q] = v0; a.dgr[q + H] = v1; a.dgr[q + 2 * H] = dn * rg;
     a.dgw[q] = v0; a.dgw[q + H] = v1; a.dgw[q + 2 * H] = dn;
     direct = go * zg;
   }
@@ -672,30 +711,30 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 // recurrent matrices from the caches per step (LSTM of 512 units, two directions, 32 columns: 8.2 us forward, 12.4 us
 // backward per step, where the products need 0.9 and 1.7).  Here the workgroups stay: each keeps its part of the
 // recurrent matrices in registers for all steps, and only the state (forward) or the pre-activation gradients (backward)
-// of a step travel between workgroups.  Per step, forward / backward: that LSTM 8.2 -> 3.1 / 12.4 -> 5.9 us; GRU of 1024
-// units, 64 columns 16.2 -> 6.3 / 29.7 -> 7.3 us (products 2.6, exchange of 64 / 192 KB per workgroup); LSTM of 320 units,
-// 5 columns 5.1 -> 1.9 us forward.  What bounds them is the exchange's trip and its volume.  Batch columns do not depend on each other: a cluster of workgroups is one
-// direction of 16 columns, and clusters never wait for one another.
+// of a step travel between workgroups.  Per step, forward / backward: that LSTM 8.2 -> 2.8 / 12.4 -> 4.6 us; GRU of 1024
+// units, 64 columns 16.2 -> 5.1 / 29.7 -> 5.8 us (products 2.6, exchange of 64 / 192 KB per workgroup); LSTM of 320 units,
+// 5 columns 5.1 -> 1.8 us forward.  What bounds them: the products (fp32 matrix pipe), the exchange's trip and volume, and the
+// gates' math between two barriers (0.6 us of the LSTM's step).  Batch columns do not depend on each other: a cluster of workgroups
+// is one direction of 16 columns, and clusters never wait for one another.
 //
-// The exchange needs no flags and no barrier over the grid: the step's rows in the reserve buffer / workspace (which the
-// later products read anyway) are filled with RNN_UNSET before the launch, the owner of an element stores it once with
+// The exchange needs no flags and no barrier over the grid: its buffer (SeqRow; a row for every step, none is used twice) is filled with
+// RNN_UNSET before the launch, the owner of an element stores it once with
 // agent scope, and a reader repeats its 16-byte loads (agent scope as well: they pass by the caches that the eight dies
-// do not share) until none of its elements is unset.  Measured alone, 64 workgroups exchanging 32 / 128 KB per step:
-// 1.9 / 3.4 us, of which a load's trip is about 1.
+// do not share) until none of its elements is unset.  (A cluster's workgroups on one die, found by its number, with loads and stores that its
+// cache answers, gained nothing on that: LSTM of 512 units, two directions, 32 columns over 200 steps backward 1167 -> 1219 us.)
 //
 // All workgroups of the launch have to be resident at once: the launch is cooperative, and a launch covers as many
 // clusters as the compute units hold, the rest follow in further launches.  A wait that does not end (it would take a
 // device that lost workgroups) stops after RNN_WAIT loads, some seconds.  Its workgroup then goes on with NaN in every mode
 // (RNN_LOST in ReLU layers), which is what the others' next steps read, and sets a word in the workspace with which the launches
 // of the call's other layers begin; so every output that depends on the missing values is NaN.
-constexpr int SEQ_WAVES = STEP_GROUPS, SEQ_THREADS = 64 * SEQ_WAVES, SEQ_COLS = 16;
-constexpr int RNN_OOB = (int)0x80000000;
+constexpr int SEQ_WAVES = STEP_GROUPS, SEQ_THREADS = 64 * SEQ_WAVES;
 constexpr int AUX_AGENT = 16;      // buffer loads: sc1, agent scope
 
 struct SeqFwd {
   struct Dir {
     const float *xp, *R, *bRn;
-    float *HP, *CP, *GT, *RN, *out, *hy, *cy;
+    float *HP, *CP, *GT, *RN, *out, *hy, *cy, *X;
   } d[2];
   int B, H, T, ldo;
   int groups;        // of 16 batch columns
@@ -736,17 +775,6 @@ struct SeqLost {
     }
   }
 };
-// whether one of the partial sums part[i * stride] or of the n words at row is RNN_LOST
-__device__ __forceinline__ bool seq_lost(const float* part, int stride, const float* row, int n) {
-  bool lost = false;
-#pragma unroll 1
-  for (int w = 0; w < STEP_GROUPS; ++w) lost |= __float_as_uint(part[w * stride]) == RNN_LOST;
-#pragma unroll 1
-  for (int k = 0; k < n && !lost; ++k)
-    lost = __float_as_uint(__hip_atomic_load(row + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == RNN_LOST;
-  return lost;
-}
-
 // every load so far has arrived: what a loop carries from before it then needs no wait inside it (that wait would be one
 // for the stores of the step before)
 __device__ __forceinline__ void seq_drain() { __builtin_amdgcn_s_waitcnt(0x0f70); }
@@ -759,12 +787,16 @@ __device__ __forceinline__ void seq_pause(int n) {
   for (; n > 0; --n) __builtin_amdgcn_s_sleep(2);
 }
 
-// N 16-byte loads per lane at off[i].  (A lane's load that does not exist is out of the buffer's range and reads zero.)
+// 16 bytes per lane of each of the chunks c0, c0 + SEQ_WAVES, ...: N of them.  What does not exist is out of the buffer's
+// range and reads zero.
 template <int N>
-__device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N]) {
-  asm volatile("" ::: "memory");       // memory may have changed since the last load
+__device__ __forceinline__ void seq_load(__amdgpu_buffer_rsrc_t r, const SeqRow& row, int c0, uintx4_t (&v)[N]) {
+  int lane = row.lane;
+  asm volatile("" : "+v"(lane) : : "memory");      // memory may have changed since the last load; and N sums in each step cost less
+                                                   // than registers that hold them over all steps
 #pragma unroll
-  for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, AUX_AGENT);
+  for (int i = 0; i < N; ++i)
+    v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, lane + (c0 + SEQ_WAVES * i) * (row.nc * 64), 0, AUX_AGENT);
 }
 template <int N>
 __device__ __forceinline__ bool seq_unset(const uintx4_t (&v)[N]) {
@@ -777,13 +809,24 @@ __device__ __forceinline__ bool seq_unset(const uintx4_t (&v)[N]) {
 // loop: where it looked for RNN_LOST too the compiler kept a second copy of v, whose moves every step paid for (LSTM of 1024
 // units over 156 steps, 4 columns, forward 479 -> 585 us).  RNN_LOST goes through the products by itself.
 template <int N>
-__device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const int (&off)[N], uintx4_t (&v)[N], int dead, int limit) {
+__device__ __forceinline__ int seq_wait(__amdgpu_buffer_rsrc_t r, const SeqRow& row, int c0, uintx4_t (&v)[N], int dead, int limit) {
   if (__builtin_amdgcn_readfirstlane(dead) || !seq_unset(v)) return dead;
   for (int spin = 0; spin < limit; ++spin) {
-    seq_load(r, off, v);
+    seq_load(r, row, c0, v);
     if (!seq_unset(v)) return 0;
   }
   return 1;
+}
+
+// whether one of the partial sums part[i * stride] or of column col of the row is RNN_LOST
+__device__ __forceinline__ bool seq_lost(const float* part, int stride, const SeqRow& row, int st, int col) {
+  bool lost = false;
+#pragma unroll 1
+  for (int w = 0; w < STEP_GROUPS; ++w) lost |= __float_as_uint(part[w * stride]) == RNN_LOST;
+#pragma unroll 1
+  for (int k = 0; k < row.K && !lost; ++k)
+    lost = __float_as_uint(__hip_atomic_load(row.base + st * row.step + row.at(k, col), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == RNN_LOST;
+  return lost;
 }
 
 // A workgroup owns HU hidden units of its cluster: row gate * HU + unit of its RT tiles of 16 rows.  The eight waves split
@@ -800,11 +843,11 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   const SeqFwd::Dir q = dir ? p.d[1] : p.d[0];
   float* const HP = q.HP;
   const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const SeqRow row(q.X, H, B, b0);
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   float a[RT][NC][4];
-  int off[NC];
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int k = (wave + W * i) * 16 + 4 * fg;
@@ -815,7 +858,6 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
       if (gate < G && h < H && k < H) v = *reinterpret_cast<const float4*>(q.R + ((size_t)gate * H + h) * H + k);
       a[rt][i][0] = v.x; a[rt][i][1] = v.y; a[rt][i][2] = v.z; a[rt][i][3] = v.w;
     }
-    off[i] = (b0 + fr < B && k < H) ? ((b0 + fr) * H + k) * 4 : RNN_OOB;
   }
   const int unit = tid % HU, col = tid / HU, ch = h0 + unit, cb = b0 + col;
   const bool cell = tid < HU * SEQ_COLS && cb < B && ch < H;
@@ -839,10 +881,10 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
       in.prev = keep;
     }
     if (st > 0) seq_pause(p.pause);
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(HP + st * BH, (unsigned)(BH * 4));
+    const __amdgpu_buffer_rsrc_t r = row.rsrc(st);
     uintx4_t v[NC];
-    seq_load(r, off, v);
-    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v, dead, lost.limit));
+    seq_load(r, row, wave, v);
+    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, row, wave, v, dead, lost.limit));
     seq_drain();
     floatx4_t acc[RT];
 #pragma unroll
@@ -872,15 +914,16 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
         rp[g] = sum;
       }
       const bool gone = MODE == RNN_RELU && __builtin_expect(rp[0] != rp[0], 0) &&
-                        seq_lost(red + unit * 17 + col, RT * 16 * 17, HP + st * BH + (size_t)cb * H, H);
+                        seq_lost(red + unit * 17 + col, RT * 16 * 17, row, st, col);
       c.hn = HP + (st + 1) * BH;
+      float* const pub = st + 1 < T ? row.base + (st + 1) * row.step + row.at(ch, col) : nullptr;
       c.cn = q.CP + (st + 1) * BH;
       c.gt = q.GT + (size_t)st * B * GH;
       c.rn = q.RN + st * BH;
       c.out = q.out + (size_t)t * B * p.ldo;
       c.hy = st == T - 1 ? q.hy : nullptr;
       c.cy = st == T - 1 ? q.cy : nullptr;
-      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp, gone);
+      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp, gone, pub);
     }
   }
 }
@@ -888,7 +931,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
 struct SeqBwd {
   struct Dir {
     const float *gout, *dhy, *dcy, *R, *HP, *CP, *GT, *RN;
-    float *dGW, *dGR, *dhx, *dcx;
+    float *dGW, *dGR, *dhx, *dcx, *X;
   } d[2];
   int B, H, T, ldo;
   int groups, nwg, cluster0, wait, pause;
@@ -897,6 +940,9 @@ struct SeqBwd {
 
 // The same for the backward pass: a workgroup owns 16 hidden units (rows of one tile: columns of the recurrent matrices,
 // 4 NC registers) and reads the gate gradients of all units of its cluster, U chunks in flight while U are multiplied.
+// What the next step needs of the reserve buffer is asked for as soon as this step's exchange has arrived: asked for at the step's
+// begin, from HBM, it held up the exchange's loads behind it (LSTM of 512 units, two directions, 32 columns over 200 steps 1289 -> 1167 us;
+// forward, with fewer such loads, the registers' moves cost more than that gained, 706 -> 745).
 // After the last step the gradient of the initial state is one more product.
 template <int MODE, int NC>
 __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
@@ -908,6 +954,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   const SeqBwd::Dir q = dir ? p.d[1] : p.d[0];
   float* const dGR = q.dGR;
   const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const SeqRow row(q.X, GH, B, b0);
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -918,14 +965,6 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) a[i][m] = (h0 + fr < H && k < GH) ? q.R[(size_t)(k + m) * H + h0 + fr] : 0.f;
   }
-  const int brow = b0 + fr < B ? (b0 + fr) * GH * 4 : RNN_OOB;
-  auto offsets_of = [&](int b, int (&off)[U]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (wave + W * (b * U + u)) * 16 + 4 * fg;
-      off[u] = k < GH ? brow + k * 4 : RNN_OOB;      // (brow out of range: so is the sum)
-    }
-  };
   const int unit = tid & 15, col = tid >> 4, ch = h0 + unit, cb = b0 + col;
   const bool cell = tid < 16 * SEQ_COLS && cb < B && ch < H;
   const size_t BH = (size_t)B * H, e = (size_t)cb * H + ch;
@@ -936,42 +975,40 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   int dead = lost.begin(status, h0 == 0);
   if (dead) direct = __builtin_nanf("");          // (the first step waits for nobody)
   seq_drain();
-  for (int sv = T - 1; sv >= (q.dhx ? -1 : 0); --sv) {
-    const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
-    CellBwdIn<MODE> in{};
+  CellBwdIn<MODE> nx{};
+  auto fetch = [&](int st) __attribute__((always_inline)) {
     if (cell && st >= 0) {
       const size_t qe = (size_t)cb * GH + ch;
-      in.go = q.gout ? q.gout[((size_t)t * B + cb) * p.ldo + ch] : 0.f;
+      nx.go = q.gout ? q.gout[((size_t)(dir ? T - 1 - st : st) * B + cb) * p.ldo + ch] : 0.f;
 #pragma unroll
-      for (int g = 0; g < G; ++g) in.gt[g] = q.GT[(size_t)st * B * GH + qe + (size_t)g * H];
+      for (int g = 0; g < G; ++g) nx.gt[g] = q.GT[(size_t)st * B * GH + qe + (size_t)g * H];
       if (MODE == RNN_LSTM) {
-        in.cn = q.CP[(st + 1) * BH + e]; in.cp = q.CP[st * BH + e];
+        nx.cn = q.CP[(st + 1) * BH + e]; nx.cp = q.CP[st * BH + e];
       }
       if (MODE == RNN_GRU) {
-        in.hp = q.HP[st * BH + e]; in.rn = q.RN[st * BH + e];
+        nx.hp = q.HP[st * BH + e]; nx.rn = q.RN[st * BH + e];
       }
     }
+  };
+  fetch(T - 1);
+  for (int sv = T - 1; sv >= (q.dhx ? -1 : 0); --sv) {
+    const int st = __builtin_amdgcn_readfirstlane(sv), t = dir ? T - 1 - st : st;
+    CellBwdIn<MODE> in = nx;
     float (*red)[16][17] = red2[st & 1];
     if (st < T - 1) {
       seq_pause(p.pause);
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(dGR + (size_t)(st + 1) * B * GH, (unsigned)((size_t)B * GH * 4));
+      const __amdgpu_buffer_rsrc_t r = row.rsrc(st + 1);
       floatx4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
       uintx4_t v[2][U];
-      {
-        int off[U];
-        offsets_of(0, off);
-        seq_load(r, off, v[0]);
-      }
+      seq_load(r, row, wave, v[0]);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        int off[U];
-        if (b + 1 < NB) {
-          offsets_of(b + 1, off);
-          seq_load(r, off, v[(b + 1) & 1]);
+        if (b + 1 < NB) seq_load(r, row, wave + W * (b + 1) * U, v[(b + 1) & 1]);
+        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, row, wave + W * b * U, v[b & 1], dead, lost.limit));
+        if (b == NB - 1) {
+          seq_drain();
+          fetch(st - 1);
         }
-        offsets_of(b, off);
-        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, off, v[b & 1], dead, lost.limit));
-        if (b == NB - 1) seq_drain();
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if ((wave + W * (b * U + u)) * 16 < GH)
@@ -983,6 +1020,8 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
 #pragma unroll
       for (int x = 0; x < 4; ++x) red[wave][4 * fg + x][fr] = acc[0][x];
       __syncthreads();
+    } else {
+      fetch(st - 1);
     }
     if (cell) {
       float rec = 0.f;
@@ -995,12 +1034,12 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
       } else {
         bool gone = st == T - 1 && dead;
         if (MODE == RNN_RELU && __builtin_expect(rec != rec, 0))
-          gone = seq_lost(&red[0][unit][col], 16 * 17, dGR + (size_t)(st + 1) * B * GH + (size_t)cb * GH, GH);
+          gone = seq_lost(&red[0][unit][col], 16 * 17, row, st + 1, col);
         in.go += direct;
         in.dc = dc;
         c.dgw = q.dGW + (size_t)t * B * GH;
         c.dgr = dGR + (size_t)st * B * GH;
-        cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct, gone);
+        cell_bwd_finish<MODE, true>(c, cb, ch, H, in, rec, &dc, &direct, gone, row.base + st * row.step, &row, col);
       }
     }
   }
@@ -1008,14 +1047,15 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
 }
 
 // What a recurrence finds in place: forward, per direction (blockIdx.y), the initial states and the summed biases (the GRU's
-// n gate apart, whose recurrent bias stays inside r * (R_n h + b_Rn)), and for a sequence launch RNN_UNSET in the rows of all
-// steps' states; backward, RNN_UNSET in all rows of dGR.
+// n gate apart, whose recurrent bias stays inside r * (R_n h + b_Rn)), and for a sequence launch the initial state and
+// RNN_UNSET in the exchange; backward, RNN_UNSET in all of it.
 struct SeqInit {
   struct Dir {
     const float *hx, *cx, *bW, *bR;
-    float *HP, *CP, *bsum;
+    float *HP, *CP, *bsum, *X;
   } d[2];
-  size_t BH, n;       // elements of a state / of the rows to be filled
+  size_t BH, n;       // elements of a state / of the exchange to be filled
+  int B;
   int GH, H, mode;
   uint32_t* status;   // to be cleared, or null
 };
@@ -1024,10 +1064,17 @@ __global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
   const size_t stride = (size_t)gridDim.x * 256, i0 = (size_t)blockIdx.x * 256 + threadIdx.x;
   const uintx4_t unset = {RNN_UNSET, RNN_UNSET, RNN_UNSET, RNN_UNSET};
   if (p.status && blockIdx.y == 0 && i0 == 0) *p.status = 0;
-  for (size_t i = i0; i < p.n / 4; i += stride) reinterpret_cast<uintx4_t*>(q.HP + p.BH)[i] = unset;
+  const size_t first = p.BH ? (size_t)p.B * ((p.H + 15) & ~15) : 0;     // forward: the initial state, below
+  for (size_t i = i0 + first / 4; i < p.n / 4; i += stride) reinterpret_cast<uintx4_t*>(q.X)[i] = unset;
   if (p.BH == 0) return;                      // backward: nothing but the fill
   for (size_t i = i0; i < p.BH; i += stride) {
-    q.HP[i] = q.hx ? rnn_value(q.hx[i]) : 0.f;
+    const float h = q.hx ? rnn_value(q.hx[i]) : 0.f;
+    q.HP[i] = h;
+    if (p.n) {
+      const int b = (int)(i / p.H), k = (int)(i - (size_t)b * p.H), b0 = b & ~(SEQ_COLS - 1);
+      const SeqRow row(q.X, p.H, p.B, b0);
+      row.base[row.at(k, b - b0)] = h;
+    }
     if (p.mode == RNN_LSTM) q.CP[i] = q.cx ? q.cx[i] : 0.f;
   }
   for (size_t i = i0; i < (size_t)p.GH; i += stride)
@@ -1127,24 +1174,18 @@ int seq_units(const RnnGeom& g) {
   return 16;
 }
 
-// The pause of seq_pause.  Too short costs up to a third of a step, too long some 20 ns per step and unit, so each is a little more
-// than what was best.  Forward it follows from what all workgroups of a layer ask for in a step (V), and from how much a workgroup
-// asks for at once (NC loads per lane) and does with it (HU).  Measured, 60 steps, us with pauses of 3 / 5 / 8 / 16: LSTM of 200 units,
-// 32 columns 133 / 137 / 146 / 171; of 512 units, 32 columns 218 / 191 / 196 / 219; of 1024 units, 2 columns 212 / 183 / 190 / 216, 12
-// 306 / 287 / 242 / 262, 32 385 / 381 / 369 / 335, 64 502 / 497 / 481 / 467 (12: 456); GRU of 768 units, 32 columns 320 / 313 / 294 / 280
-// (10: 273); ReLU of 256 units, 12 columns 111 / 112 / 122 / 146, of 1024, 64 columns 284 / 270 / 243 / 265.
+// The pause of seq_pause.  Too short costs up to a tenth of a step, too long some 60 ns per step and unit.  Forward it follows from
+// what all workgroups of a layer ask for in a step (V, MB).  Measured, us with pauses of 2 / 4 / 6 / 8: LSTM of 320 units, 5 columns over
+// 100 steps (V 0.5) 214 / 218 / 228 / 238; GRU of 256 units, two directions, 20 columns (2.6) 204 / 208 / 216 / 228; tanh of 384 units, two
+// directions, 64 columns (4.7) 231 / 215 / 227 / 233; LSTM of 512 units, two directions, 32 columns over 200 steps (8.4) 686 / 642 / 639 /
+// 648; GRU of 1024 units, 64 columns (16.8) 580 / 568 / 572 / 583.
 int seq_pause_fwd(const RnnGeom& g, int units) {
-  const double V = (double)g.D * ((g.H + units - 1) / units) * g.B * g.H * 4e-6;      // MB
-  if (g.G == 1) return g.H <= 384 ? 3 : g.H <= 512 ? 4 : V < 1 ? 4 : g.H <= 768 ? 6 : 7;
-  if (g.H <= 256) return V < 1 ? 4 : 5;
-  if (g.H <= 512) return g.H <= 448 || V < 4 ? 5 : 6;
-  return (int)(units == 4 ? 5.5 + V / 4 : units == 8 ? 6.5 + 0.6 * V : 5.5 + 0.4 * V);
+  const double V = (double)g.D * ((g.H + units - 1) / units) * g.B * g.H * 4e-6;
+  return V < 4 ? 2 : 4;
 }
-// Backward the loads come in several rounds, and 1 to 3 is best everywhere (LSTM of 512 units, two directions, 32 columns, of the
-// best: 1 / 2 / 3 / 8 1.02, 1.01, 1.00, 1.03; GRU of 1024 units, 12 columns 1.06, 1.03, 1.01, 1.02; LSTM of 128 units, 2 columns 1.00, 1.02, 1.03, 1.14).
-int seq_pause_bwd(const RnnGeom& g) {
-  return g.G > 1 && (double)g.D * ((g.H + 15) / 16) * g.B * g.GH * 4e-6 >= 3 ? 3 : 2;
-}
+// Backward a step has more to load and to do between its stores and the next step's loads: 0 / 1 / 2 / 4 1372 / 1375 / 1382 / 1405 us
+// (that LSTM of 512 units), 338 / 337 / 343 / 352 (LSTM of 128 units, 16 columns over 100 steps).
+constexpr int SEQ_PAUSE_BWD = 1;
 
 // Does a pass gain by sequence launches?  One costs some 20 us more than a step's launch does (the cooperative queue, on both
 // sides), and saves on each step, the more so the more a step has to do.  Sequence / steps, of the time:
@@ -1177,7 +1218,7 @@ bool seq_pays(const RnnGeom& g, bool bwd) {
 // columns), a stream that is not being captured (a cooperative launch is not recorded)
 bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
   const int asked = options().rnn_sequences;
-  if (options().rnn_unfused || asked == Options::SEQ_NEVER || g.H % 4 != 0 || g.H > 1024 ||
+  if (options().rnn_unfused || asked == Options::SEQ_NEVER || !seq_holds(g) ||
       (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31) || (asked == Options::SEQ_AUTO && !seq_pays(g, bwd)))
     return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -1280,7 +1321,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
   p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
   p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
   p.wait = options().rnn_wait; p.pause = seq_pause_fwd(g, seq_units(g)); p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
-  ip.BH = g.BH; ip.n = seq ? (size_t)g.T * g.BH : 0; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+  ip.BH = g.BH; ip.n = seq ? (size_t)g.T * seq_row(g, g.H) : 0; ip.B = g.B; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
   ip.status = l == 0 ? p.status : nullptr;
   for (int dir = 0; dir < g.D; ++dir) {
     const int pl = l * g.D + dir;
@@ -1291,10 +1332,11 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
     q.R = w + o.R; q.bRn = w + o.bR + 2 * g.H;
     q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
     q.out = out + (size_t)dir * g.H;
+    q.X = seq_exchange(g, ws) + (size_t)dir * g.T * seq_row(g, g.H);
     q.hy = hy + (size_t)pl * g.BH;
     q.cy = cy && MODE == RNN_LSTM ? cy + (size_t)pl * g.BH : nullptr;
     ip.d[dir] = {hx ? hx + (size_t)pl * g.BH : nullptr, cx ? cx + (size_t)pl * g.BH : nullptr, w + o.bW, w + o.bR, q.HP, q.CP,
-                 ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH};
+                 ws + (size_t)g.D * TB * g.GH + (size_t)dir * g.GH, q.X};
   }
   launch_init(ip, g.D, s);
   for (int dir = 0; dir < g.D; ++dir)
@@ -1422,8 +1464,8 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
     SeqBwd p{};
     p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
     p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
-    p.wait = options().rnn_wait; p.pause = seq_pause_bwd(g); p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
-    ip.n = TB * g.GH;
+    p.wait = options().rnn_wait; p.pause = SEQ_PAUSE_BWD; p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
+    ip.n = (size_t)g.T * seq_row(g, g.GH);
     ip.status = l == g.L - 1 ? p.status : nullptr;
     for (int dir = 0; dir < g.D; ++dir) {
       const int pl = l * g.D + dir;
@@ -1437,7 +1479,8 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
       q.dGW = dGW[dir]; q.dGR = dGR[dir];
       q.dhx = dhx ? dhx + (size_t)pl * g.BH : nullptr;
       q.dcx = dcx ? dcx + (size_t)pl * g.BH : nullptr;
-      ip.d[dir].HP = dGR[dir];
+      q.X = seq_exchange(g, ws) + (size_t)dir * g.T * seq_row(g, g.GH);
+      ip.d[dir].X = q.X;
     }
     launch_init(ip, g.D, s);
     const int rc = seq_bwd<MODE>(g, p, s);
