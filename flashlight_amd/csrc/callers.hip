@@ -453,6 +453,51 @@ matmul_nn_skinny(const T* __restrict__ A, const T* __restrict__ B, T* __restrict
   }
 }
 
+// The same with few rows: there most of the lanes above have none, and their chain of staging and steps is as long as ever.  A
+// workgroup owns SR_M rows of two columns, and its threads stride over the contraction: B is read in whole lines, A's lines by
+// neighbouring threads.  What bounds it is the latency of a thread's few loads.  us (the kernel above / this one): 10 rows, 64
+// columns, K 64 / 256 / 1024 / 4096 4.8 / 3.7, 5.6 / 4.3, 14 / 6.7, 48 / 17; 64 rows, 128 columns in bf16 5.1 / 4.0, 6.0 / 5.6, 15 / 14.5, 52 / 46:
+// up to SR_MAX rows it is the faster one for every K and N <= 128.
+constexpr int SR_NT = 2, SR_M = 16, SR_MAX = 64;
+template <typename T>
+__global__ void __launch_bounds__(256)
+matmul_nn_rows(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, int M, int N, int K,
+               const float* __restrict__ bias) {
+  constexpr int V = SR_NT * SR_M;
+  __shared__ float part[V][257];
+  const int tid = threadIdx.x, n0 = blockIdx.x * SR_NT, m0 = blockIdx.y * SR_M;
+  float acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = 0.f;
+  const T* b[SR_NT];
+#pragma unroll
+  for (int j = 0; j < SR_NT; ++j) b[j] = B + (size_t)min(n0 + j, N - 1) * K;
+#pragma unroll 2
+  for (int k = tid; k < K; k += 256) {
+    float a[SR_M], v[SR_NT];
+#pragma unroll
+    for (int r = 0; r < SR_M; ++r) a[r] = ld(A, (size_t)k * M + min(m0 + r, M - 1));
+#pragma unroll
+    for (int j = 0; j < SR_NT; ++j) v[j] = ld(b[j], (size_t)k);
+#pragma unroll
+    for (int j = 0; j < SR_NT; ++j)
+#pragma unroll
+      for (int r = 0; r < SR_M; ++r) acc[j * SR_M + r] += a[r] * v[j];
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) part[i][tid] = acc[i];
+  __syncthreads();
+  // eight threads add up a result: every eighth partial sum each, then across
+  const int i = tid >> 3;
+  float s = 0.f;
+#pragma unroll
+  for (int u = 0; u < 32; ++u) s += part[i][(tid & 7) + 8 * u];
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  const int n = n0 + i / SR_M, r = m0 + i % SR_M;
+  if ((tid & 7) == 0 && r < M && n < N) st(C, (size_t)n * M + r, s + (bias ? bias[r] : 0.f));
+}
+
 // C (M x N) = A^T * B with A stored K x M: both operands are contiguous along the contraction.  A wave
 // owns 8 x 8 results; its lanes stride over k and the 64 sums are reduced across the wave at the end.
 template <typename T>
@@ -1011,8 +1056,12 @@ extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M,
       const dim3 grid((unsigned)((M + 63) / 64), (unsigned)((N + SK_NT - 1) / SK_NT));
       by_dtype(dtype, [&](auto* t_) {
         using T = FLHIP_T_OF(t_);
-        hipLaunchKernelGGL((matmul_nn_skinny<T>), grid, dim3(1024), 0, s, (const T*)A, (const T*)B,
-                           (T*)C, M, N, K, bias_rows);
+        const dim3 cols((unsigned)((N + SR_NT - 1) / SR_NT), (unsigned)((M + SR_M - 1) / SR_M));
+        if (M <= SR_MAX)
+          hipLaunchKernelGGL((matmul_nn_rows<T>), cols, dim3(256), 0, s, (const T*)A, (const T*)B, (T*)C, M, N, K, bias_rows);
+        else
+          hipLaunchKernelGGL((matmul_nn_skinny<T>), grid, dim3(1024), 0, s, (const T*)A, (const T*)B,
+                             (T*)C, M, N, K, bias_rows);
       });
       return check_launch("matmul (thin, A * B)");
     }

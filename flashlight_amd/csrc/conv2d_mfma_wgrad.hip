@@ -14,7 +14,14 @@
 // walked in chunks of 16 positions through double-buffered LDS tiles stored
 // [row][position] with pitch 17.  What a column j means (channel offset, window
 // shift) is decoded once per kernel; every thread keeps the entries of its own
-// columns in registers.  Padding is fetched as out-of-range buffer loads (zero).
+// columns in registers: eight at most (with sixteen, and twice the tile, the kernel kept 162 registers in memory).  Padding
+// is fetched as out-of-range buffer loads (zero).
+//
+// What bounds it: the gather's address arithmetic and single-element loads beside the fp32 matrix pipe (0.41 of its rate at 512
+// images, 5 x 5, 32 -> 64 channels over 14 x 14), and with few positions the chain of chunks, so that a split goes down to four of them.
+// With the partial sums' reduction, us (sixteen columns, splits of at least 256 positions / now): 5 x 5, 32 -> 64 channels over 14 x 14, 1 / 8 / 64 / 512
+// images 49 -> 13, 55 -> 16, 71 -> 38, 229 -> 164; 1 -> 32 over 28 x 28, 64 images 25 -> 18; 7 x 7 stride 2, 3 -> 64 over 224 x 224, 32 images
+// 144 -> 134.  Four chunks in registers instead of two: no gain; 8 waves and chunks of 32 positions: 45 at 64 images.
 #include "conv2d_mfma.h"
 
 namespace flhip {
@@ -24,7 +31,7 @@ constexpr int THREADS = 256;    // 4 waves
 constexpr int BM = MFMA_BM;
 constexpr int WKC = 16;         // positions per K-chunk
 constexpr int WKP = 17;         // LDS pitch of both tiles (positions contiguous)
-constexpr int WNT_MAX = 8;      // 16-column blocks per wave
+constexpr int WNT_MAX = 4;      // 16-column blocks per wave
 constexpr int WNB_MAX = 2 * WNT_MAX;
 constexpr int WCL_MAX = WNB_MAX;        // columns gathered per thread (16 per block / 16 lanes)
 constexpr int WAR = BM / 16;            // dy rows per thread
@@ -231,11 +238,7 @@ wgrad_kernel(WgradParams p, const T* __restrict__ x, const T* __restrict__ dy,
     case 1: run(std::integral_constant<int, 1>{}); break;
     case 2: run(std::integral_constant<int, 2>{}); break;
     case 3: run(std::integral_constant<int, 3>{}); break;
-    case 4: run(std::integral_constant<int, 4>{}); break;
-    case 5: run(std::integral_constant<int, 5>{}); break;
-    case 6: run(std::integral_constant<int, 6>{}); break;
-    case 7: run(std::integral_constant<int, 7>{}); break;
-    default: run(std::integral_constant<int, 8>{}); break;
+    default: run(std::integral_constant<int, 4>{}); break;
   }
 
   if (do_db && tid < min(m_lim, BM)) {
@@ -394,7 +397,7 @@ bool wgrad_split(WgradParams* p, const ConvGeom& g) {
   const long long base_wgs = (long long)p->ntiles_n * p->mtiles * g.groups;
   if (p->ntiles_n * p->mtiles > 65535 || g.groups > 65535) return false;
   long long ns = 2 * mfma_num_cus() / base_wgs;
-  const long long max_ns = (p->Ptotal + 255) / 256;
+  const long long max_ns = (p->Ptotal + 63) / 64;
   if (ns > max_ns) ns = max_ns;
   if (ns < 1) ns = 1;
   long long pps = (p->Ptotal + ns - 1) / ns;

@@ -292,6 +292,20 @@ def test_matmul_fp32_in_three_parts_keeps_what_bf16_cannot_hold(mode):
         assert rel_l2(got[rows][ok], ref[rows][ok]) <= 2 * np.sqrt(K) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (10, 64, 1024), (17, 3, 255), (33, 127, 257), (63, 128, 700), (65, 9, 300)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_matmul_few_rows(M, N, K, dtype):
+    """Blocks of 16 rows and pairs of columns with remainders, contractions around the 256 threads', both sides of 64 rows."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(N, K, device="cuda", generator=gen).to(dtype)
+    w = torch.randn(K, M, device="cuda", generator=gen).to(dtype)
+    b = torch.randn(M, device="cuda", generator=gen)
+    want = host(x).astype(np.float64) @ host(w).astype(np.float64) + host(b)
+    # fp32 sums in runs of K / 256 and a tree; one rounding to the storage type
+    bound = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert rel_l2(host(ops.linear(x, w, b)), want) <= bound
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 64, 128), (512, 64, 132), (64, 8, 1148), (64, 8, 1152), (64, 9, 1020), (64, 9, 1024), (4096, 32, 132), (4096, 33, 132),
                                    (4096, 64, 700), (4096, 64, 704)])
 def test_matmul_fp32_thin(M, N, K):
