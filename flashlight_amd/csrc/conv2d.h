@@ -61,6 +61,11 @@ size_t mfma_pointwise16_gathered_bytes(const ConvGeom& g);
 size_t mfma_pointwise_split_ws(const ConvGeom& g, int dtype, bool bwd);
 int mfma_pointwise_conv_split(const ConvGeom& g, int dtype, bool bwd, const void* src, const void* w,
                               const float* bias, void* dst, void* ws, size_t ws_bytes, hipStream_t s);
+// 1x1 windows in fp32 in three bf16 parts (gemm_f32_split.hip): forward (strided too), backward-data (+ addend, or null) and filter
+// gradient of stride 1; -1 where the general kernels are the faster ones, a shape is not theirs or the room is missing
+int mfma_pointwise_parts(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, const void* addend, void* dst,
+                         hipStream_t s);
+int mfma_pointwise_parts_wgrad(const ConvGeom& g, const void* x, const void* dy, float* dw, void* ws, size_t ws_bytes, hipStream_t s);
 // column-major C = op(A) op(B) on the 1x1 kernels (mode 0: A B, 1: A^T B, 2: A B^T);
 // -1 when it does not apply
 int mfma_gemm(int dtype, int mode, const void* A, const void* B, void* C, int M, int N, int K,

@@ -312,6 +312,7 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
       r = mfma_strip16_conv_fwd(g, x, w, bias, y, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_slab16_conv_fwd(g, x, w, bias, y, s, d->dtype);
+    if (r < 0 && d->dtype == FLHIP_F32 && !skip(SK_GEMM)) r = mfma_pointwise_parts(g, false, x, w, bias, nullptr, y, s);
     if (r < 0 && !skip(SK_GEMM)) r = mfma_pointwise_conv_fwd(g, d->dtype, x, w, bias, y, s);
     if (r < 0 && algo_is(Options::ALGO_TAPPED)) r = mfma_tapped_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && !skip(SK_SLAB)) r = mfma_slab_conv_fwd(g, d->dtype, x, w, bias, y, s);
@@ -357,9 +358,10 @@ static int bwd_data_direct(const flhip_conv_desc* d, const ConvGeom& g, const vo
   return check_launch("conv2d_bwd_data");
 }
 
-// plan < 0: the default rule; otherwise that family alone (FLHIP_DECLINED when it does not take the geometry)
+// plan < 0: the default rule; otherwise that family alone (FLHIP_DECLINED when it does not take the geometry).  With an addend:
+// *added is set where the kernel has added it
 static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w, void* dx, void* ws, size_t ws_bytes,
-                         int plan, void* stream) {
+                         int plan, void* stream, const void* addend = nullptr, bool* added = nullptr) {
   FLHIP_REQUIRE(d && dy && w && dx, "conv2d_bwd_data: null argument");
   ConvGeom g;
   const int rc = make_geom(d, &g);
@@ -401,6 +403,10 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
       r = mfma_strip16_conv_bwd_data(g, dy, w, dx, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_slab16_conv_bwd_data(g, dy, w, dx, s, d->dtype);
+    if (r < 0 && d->dtype == FLHIP_F32 && !skip(SK_GEMM)) {
+      r = mfma_pointwise_parts(g, true, dy, w, nullptr, addend, dx, s);
+      if (r >= 0 && addend) *added = true;
+    }
     if (r < 0 && !skip(SK_GEMM)) r = mfma_pointwise_conv_split(g, d->dtype, true, dy, w, nullptr, dx, ws, ws_bytes, s);
     if (r < 0 && !skip(SK_GEMM)) r = mfma_pointwise_conv_bwd_data(g, d->dtype, dy, w, dx, s);
     if (r < 0 && algo_is(Options::ALGO_TAPPED)) r = mfma_tapped_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
@@ -453,8 +459,9 @@ extern "C" int flhip_conv2d_bwd_data_add(const flhip_conv_desc* d, const void* d
     if (r >= 0) return r;
   }
   // every other kernel: the plain pass, then the element-wise sum
-  const int r = flhip_conv2d_bwd_data(d, dy, w, dx, ws, ws_bytes, stream);
-  if (r != FLHIP_OK) return r;
+  bool added = false;
+  const int r = bwd_data_impl(d, dy, w, dx, ws, ws_bytes, -1, stream, addend, &added);
+  if (r != FLHIP_OK || added) return r;
   return flhip_add(dx, addend, dx, (size_t)g.N * g.C * g.H * g.W, d->dtype, stream);
 }
 
@@ -523,6 +530,7 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
       r = mfma_first16_wgrad(g, x, dy, dw, db, ws, ws_bytes, s, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_wgrad16(g, x, dy, dw, db, ws, ws_bytes, s, d->dtype);
+    if (r < 0 && dw && !db && d->dtype == FLHIP_F32 && !skip(SK_GEMM)) r = mfma_pointwise_parts_wgrad(g, x, dy, dw, ws, ws_bytes, s);
     if (r < 0 && !skip(SK_GEMM))
       r = mfma_pointwise_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, algo_is(Options::ALGO_TAPPED), s);
     if (r < 0 && !skip(SK_SLAB)) r = mfma_slab_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, s);

@@ -33,6 +33,7 @@
 // lane's four accumulator values are four consecutive positions of one channel and
 // leave as one 16-byte store.
 #include "conv2d_mfma.h"
+#include "gemm_f32.h"
 
 namespace flhip {
 namespace {
@@ -1181,6 +1182,104 @@ int mfma_gemm_slices(int K, int ksplit) {
   if (ksplit <= 1) return 1;
   const int cps = (chunks + ksplit - 1) / ksplit;
   return (chunks + cps - 1) / cps;
+}
+
+// ---- 1x1 windows in fp32 in three bf16 parts (gemm_f32_split.hip) --------------------------------------------------
+namespace {
+
+struct PwParts {
+  Gemm32 p;
+  int tm, tn, slices;
+};
+
+// Which products run there, by 67 geometries of 0.1 to 40 GFLOP, with batch norm's planes and ragged ones, us general kernel / there:
+//   forward, backward-data: 128 positions x 64 channels, from three tiles to two compute units on.  More than that were
+//     faster throughout (0.62 to 0.91 of the time): 64 -> 256 channels over 56 x 56, 32 images 50 / 39 and back 48 / 36, 1024 -> 256 over
+//     14 x 14, 64 images 80 / 61, 2048 channels from 512 over 7 x 7, 33 images 46 / 33; fewer leave the chip to one round of workgroups that
+//     take 1.5 times as long per step of the contraction: 256 tiles 1024 -> 256 50 / 53, 200 43 / 47, 100 16 / 26.  With an addend the
+//     general kernel's sum is a pass of its own, which is worth three tiles to four units over up to 256 channels: 200 tiles 16 / 13, 296
+//     18 / 11, 128 positions of it 10 / 8.5, but 256 of 1024 channels 54 / 53, 172 15 / 12 and 112 of 1024 33 / 48.
+//   filter gradient: from 600 million multiply-adds on (1.2 GFLOP; below, the tiles of 64 x 64 have the shorter start: 530 million 20.9 /
+//     23.3 and 21.2 / 22.3, 460 20.1 / 18.8, 150 to 200 13.4 / 14.8; above, 670 26 / 23, 640 25 / 21).  256 x 256 tiles' worth of channels or more on tiles of 128 x 128, 256 workgroups:
+//     1024 x 256 over 14 x 14, 64 images 70 / 51; fewer on 128 x 64, 256 workgroups up to 820 million (256 x 128 over 17408 positions
+//     24.2 / 19.1, 512 workgroups 19.4), 512 beyond (over 40960 35.6 / 28.5, 256 31.3; 256 x 64 over 100352 47 / 39, 256 45).  The contraction's slices
+//     are at most the general kernel's, so that no caller needs more room.
+bool pw_parts_plan(const ConvGeom& g, int mode, bool added, PwParts* pl) {
+  if (!pw_applies(g)) return false;
+  const bool unit = g.sy == 1 && g.sx == 1 && g.OH == g.H && g.OW == g.W;
+  if (mode != 0 && !unit) return false;
+  const long long xb = (long long)g.N * g.C * g.H * g.W * 4, yb = (long long)g.N * g.K * g.OH * g.OW * 4, wb = (long long)g.K * g.C * 4;
+  const long long most = (1ll << 31) - std::max(xb, yb) / g.N;     // (a load ahead of the contraction's end: one image on)
+  if (xb >= most || yb >= most || wb >= (1ll << 31)) return false;
+  Gemm32& p = pl->p;
+  const int P = g.OH * g.OW, SP = g.H * g.W, cus = mfma_num_cus();
+  p.M = mode == 1 ? g.C : g.N * P;
+  p.N = mode == 2 ? g.C : g.K;
+  p.K = mode == 0 ? g.C : mode == 2 ? g.K : g.N * SP;
+  if (mode == 0 && g.C % 4 != 0) return false;       // the weights are read in 16-byte pieces of a filter ...
+  if (mode == 1 && (SP % 4 != 0 || SP < G32_KC)) return false;     // ... here both operands in pieces of a plane
+  if (p.K < G32_KC) return false;
+  p.P = P; p.SP = mode == 2 ? P : SP; p.OW = g.OW;
+  p.rowstep = mode == 0 ? g.sy * g.W : g.OW;
+  p.colstep = mode == 0 ? g.sx : 1;
+  p.a_bytes = (unsigned)(mode == 2 ? yb : xb);
+  p.b_bytes = (unsigned)(mode == 1 ? yb : wb);
+  p.nstages = (p.K + G32_KC - 1) / G32_KC;
+  p.sps = p.nstages;
+  pl->tm = 128; pl->tn = 64;
+  pl->slices = 1;
+  if (mode != 1) {
+    const long long tiles = (long long)((p.M + 127) / 128) * ((p.N + 63) / 64);
+    if (2 * tiles <= 3ll * cus && !(added && 4 * tiles >= 3ll * cus && p.K <= 256)) return false;
+    if (tiles >= 1ll << 31) return false;
+  } else {
+    const long long macs = (long long)p.M * p.N * p.K;
+    if (macs < 600000000) return false;
+    if ((long long)p.M * p.N >= 256 * 1024) pl->tn = 128;
+    else if (p.M <= 64) pl->tm = 64, pl->tn = 128;
+  }
+  p.mtiles = (p.M + pl->tm - 1) / pl->tm;
+  p.ntiles = (p.N + pl->tn - 1) / pl->tn;
+  if (mode == 1) {
+    const long long tiles = (long long)p.mtiles * p.ntiles;
+    PwWgradParams q{};
+    if (!pw_wgrad_plan(g, &q)) return false;
+    const bool twice = pl->tm * pl->tn < 128 * 128 && (long long)p.M * p.N * p.K >= 820000000;
+    long long ns = std::min((long long)q.nsplit, (twice ? 2 : 1) * cus / tiles);
+    if (ns > 8) ns -= ns % 8;
+    ns = std::max(1ll, ns);
+    p.sps = (int)((p.nstages + ns - 1) / ns);
+    pl->slices = (p.nstages + p.sps - 1) / p.sps;
+    p.slice = (size_t)p.M * p.N;
+  }
+  p.slices = pl->slices;
+  return true;
+}
+
+bool aligned16(const void* a, const void* b) { return (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 16 == 0; }
+
+}  // namespace
+
+int mfma_pointwise_parts(const ConvGeom& g, bool bwd, const void* src, const void* w, const float* bias, const void* addend, void* dst,
+                         hipStream_t s) {
+  PwParts pl{};
+  const int mode = bwd ? 2 : 0;
+  if (!pw_parts_plan(g, mode, addend != nullptr, &pl) || !aligned16(src, w)) return -1;
+  return gemm32_split_planes(mode, pl.tm, pl.tn, 1, pl.p, static_cast<const float*>(src), static_cast<const float*>(w), bias,
+                             static_cast<const float*>(addend), static_cast<float*>(dst), s);
+}
+
+int mfma_pointwise_parts_wgrad(const ConvGeom& g, const void* x, const void* dy, float* dw, void* ws, size_t ws_bytes, hipStream_t s) {
+  PwParts pl{};
+  if (!pw_parts_plan(g, 1, false, &pl) || !aligned16(x, dy)) return -1;
+  const size_t E = (size_t)g.K * g.C;
+  if (pl.slices > 1 && (!ws || ws_bytes < pl.slices * E * sizeof(float))) return -1;
+  float* const out = pl.slices > 1 ? static_cast<float*>(ws) : dw;
+  const int rc = gemm32_split_planes(1, pl.tm, pl.tn, pl.slices, pl.p, static_cast<const float*>(x), static_cast<const float*>(dy), nullptr,
+                                     nullptr, out, s);
+  if (rc || pl.slices == 1) return rc;
+  wgrad_reduce_launch(out, pl.slices, (int)E, 0, 0, dw, nullptr, s);
+  return check_launch("conv2d_bwd_filter 1x1 (reduce)");
 }
 
 }  // namespace flhip

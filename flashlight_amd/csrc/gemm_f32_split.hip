@@ -21,6 +21,12 @@
 //   mode 0  2000 x 4000 x 2000  256 -> 157 (204 TFLOP/s)  8.0e-7 -> 2.7e-7    1024 x 6400 x 3072  312 -> 205
 //   mode 1  2000 x 4000 x 2000  256 -> 160                8.0e-7 -> 2.7e-7    2048 x 6400 x 512   113 -> 82
 //   mode 2  2000 x 2000 x 4000  265 -> 164 (2 slices)     1.1e-6 -> 2.7e-7    1024 x 2048 x 6400  200 -> 135 (4 slices)
+//
+// Layers of 1x1 windows are the same products with the positions of all images as A's and C's rows (modes 0 and 2) or as the contraction
+// (mode 1): only where a thread's values lie differs (PL), a position being looked up once per workgroup.  Over large planes memory bounds
+// them: four small tiles to a compute unit (128 registers; three at 129; A^T B on 64 x 128 tiles needs 132) and tiles that share positions one after the other on one
+// die, us: 64 -> 256 channels over 56 x 56, 32 images 47 -> 39 (129 MB), the addend's loads in front of the stores 70 -> 38; filter
+// gradient of 256 x 64, a slice's tiles on one die, 45 -> 39.  (The general kernels' times stand at the rule, conv2d_mfma_pointwise.hip.)
 #include <algorithm>
 
 #include "conv2d.h"
@@ -65,6 +71,37 @@ struct SplitSide {
       rowstep = R * 4;
     }
   }
+  // rows that are positions of planes (contiguous along the rows): where the first value of position r0 + row lies
+  __device__ __forceinline__ void init_positions(int r0, const Gemm32& p, int tid) {
+    init(r0, p.M, p.K, tid);
+    if constexpr (!KROWS) {
+      const int r = r0 + tid % T, img = r / p.P, pos = r - img * p.P, row = pos / p.OW;
+      if (r < p.M) off[0] = ((img * p.K + k0) * p.SP + row * p.rowstep + (pos - row * p.OW) * p.colstep) * 4;
+      step = G32_KC * p.SP * 4;
+      rowstep = p.SP * 4;
+    }
+  }
+  // rows that are channels, the contraction their positions, one image after the other: pieces of 4 positions, which a plane
+  // holds whole.  (Past the last image a piece lies past the tensor.)
+  int piece, pieces, jump;
+  __device__ __forceinline__ void init_channels(int r0, int R, const Gemm32& p, int s0, int tid) {
+    init(r0, R, p.SP, tid);
+    pieces = p.SP / 4;
+    jump = (R - 1) * p.SP * 4;
+    const int at0 = s0 * (G32_KC / 4) + (tid & 3), img = at0 / pieces;
+    piece = at0 - img * pieces;
+#pragma unroll
+    for (int i = 0; i < (KROWS ? EL / 4 : 1); ++i)
+      if (off[i] != S_OOB) off[i] += (img * R * p.SP + 4 * piece - k0) * 4;
+  }
+  __device__ __forceinline__ void load_next(float (&v)[EL], __amdgpu_buffer_rsrc_t rsrc) {
+    load<false>(v, rsrc, 0, G32_KC);
+    piece += G32_KC / 4;
+    const int by = G32_KC * 4 + (piece >= pieces ? jump : 0);
+    if (piece >= pieces) piece -= pieces;
+#pragma unroll
+    for (int i = 0; i < (KROWS ? EL / 4 : 1); ++i) off[i] += by;       // (a row that is none: past every tensor all the same)
+  }
   // the stage at byte offset `stage` of every row.  CHECKED: only its first `left` contraction indexes exist, the others read
   // zero
   template <bool CHECKED>
@@ -107,8 +144,8 @@ struct SplitSide {
   }
 };
 
-template <int MODE, int TM, int TN>
-__global__ void __launch_bounds__(ST, 2)
+template <int MODE, int TM, int TN, bool PL>
+__global__ void __launch_bounds__(ST, PL && TM * TN < 128 * 128 && !(MODE == 1 && TM == 64) ? 4 : 2)
 gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias,
                     const float* addend, float* C) {
   constexpr bool AK = MODE == 1, BK = MODE != 2;
@@ -123,18 +160,45 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
   __shared__ __align__(16) char lds[2 * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
-  const int tile = gemm32_tile_of(blockIdx.x, p.mtiles * p.ntiles);
-  const int m0 = (tile % p.mtiles) * TM, n0 = (tile / p.mtiles) * TN;
-  const int s0 = blockIdx.y * p.sps, send = min(p.nstages, s0 + p.sps);
+  int tile, slice = blockIdx.y;
+  if constexpr (PL && MODE == 1) {
+    // the tiles of a slice follow each other on one die, whose cache holds the slice's rows (slices past the last full eight: as they come)
+    const int tiles = p.mtiles * p.ntiles, at = blockIdx.x, full8 = p.slices / 8 * 8;
+    if (at < full8 * tiles) {
+      tile = (at >> 3) % tiles;
+      slice = (at >> 3) / tiles * 8 + (at & 7);
+    } else {
+      tile = at % tiles;
+      slice = at / tiles;
+    }
+  } else {
+    tile = gemm32_tile_of(blockIdx.x, p.mtiles * p.ntiles);
+  }
+  // (over planes the weights are the small operand: the tiles that share positions follow each other)
+  const bool nfast = PL && MODE != 1;
+  const int m0 = (nfast ? tile / p.ntiles : tile % p.mtiles) * TM, n0 = (nfast ? tile % p.ntiles : tile / p.mtiles) * TN;
+  const int s0 = slice * p.sps, send = min(p.nstages, s0 + p.sps);
 
   SA sa;
   SB sb;
-  sa.init(m0, p.M, p.K, tid);
-  sb.init(n0, p.N, p.K, tid);
+  if constexpr (PL && MODE == 1) {
+    sa.init_channels(m0, p.M, p, s0, tid);
+    sb.init_channels(n0, p.N, p, s0, tid);
+  } else {
+    if constexpr (PL) sa.init_positions(m0, p, tid);
+    else sa.init(m0, p.M, p.K, tid);
+    sb.init(n0, p.N, p.K, tid);
+  }
   const __amdgpu_buffer_rsrc_t ar = make_rsrc(A, p.a_bytes), br = make_rsrc(B, p.b_bytes);
   float va[SA::EL], vb[SB::EL];
-  const int full = min(send, p.K / G32_KC);    // end of the slice's whole stages (there is one at least)
+  // end of the slice's whole stages (there is one at least; of planes every stage is one: what lies past them reads zero)
+  const int full = PL && MODE == 1 ? send : min(send, p.K / G32_KC);
   auto stage_in = [&](int s) __attribute__((always_inline)) {
+    if constexpr (PL && MODE == 1) {
+      sa.load_next(va, ar);
+      sb.load_next(vb, br);
+      return;
+    }
     s = min(s, full - 1);
     sa.template load<false>(va, ar, s * sa.step, G32_KC);
     sb.template load<false>(vb, br, s * sb.step, G32_KC);
@@ -215,18 +279,31 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
 #pragma unroll
         for (int r = 0; r < 16; ++r) big[i][c][r] = 0.f;
     const int kend = min(p.K, send * G32_KC);
+    size_t arow[RT];                           // positions of planes: a row's first value
+    if constexpr (PL && MODE != 1) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int m = m0 + wm * 32 * RT + 32 * i + fr, img = m / p.P, pos = m - img * p.P;
+        arow[i] = (size_t)img * p.K * p.SP + pos / p.OW * p.rowstep + pos % p.OW * p.colstep;
+      }
+    }
+    auto index = [&](int img, int pos, int row, int rows) { return ((size_t)img * rows + row) * p.SP + pos; };
 #pragma unroll 1
     for (int k = s0 * G32_KC + h; k < ((kend + 1) & ~1); k += 2) {
       float a[RT], b[CT];
+      const int img = PL && MODE == 1 ? k / p.SP : 0, pos = PL && MODE == 1 ? k - img * p.SP : 0;
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
         const int m = m0 + wm * 32 * RT + 32 * i + fr;
-        a[i] = k < kend && m < p.M ? A[AK ? (size_t)m * p.K + k : (size_t)k * p.M + m] : 0.f;
+        const size_t at = !PL ? (AK ? (size_t)m * p.K + k : (size_t)k * p.M + m)
+                        : MODE == 1 ? index(img, pos, m, p.M) : arow[i] + (size_t)k * p.SP;
+        a[i] = k < kend && m < p.M ? A[at] : 0.f;
       }
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
         const int n = n0 + wn * 32 * CT + 32 * c + fr;
-        b[c] = k < kend && n < p.N ? B[BK ? (size_t)n * p.K + k : (size_t)k * p.N + n] : 0.f;
+        const size_t at = PL && MODE == 1 ? index(img, pos, n, p.N) : BK ? (size_t)n * p.K + k : (size_t)k * p.N + n;
+        b[c] = k < kend && n < p.N ? B[at] : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < RT; ++i)
@@ -239,48 +316,64 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
   // dimension: element r of a lane is column 8 (r / 4) + 4 h + r % 4 and row fr of C's tile.  (A store past the last column is
   // out of the buffer's range, one past the last row is put there.)
   const int m = m0 + wm * 32 * RT + fr, nl = wn * 32 * CT + 4 * h;
-  const size_t origin = (size_t)n0 * p.M, left = ((size_t)(p.N - n0) * p.M) * 4;
+  constexpr bool PC = PL && MODE != 1;         // C in planes: columns P apart, a column past the last is looked for (the next image is there)
+  const int ldc = PC ? p.P : p.M, cols = p.N - n0 - nl;
+  const size_t origin = (size_t)n0 * ldc, left = ((size_t)(PC ? p.M / p.P * p.N : p.N) * ldc - origin) * 4;
   const unsigned range = left < 0x7fffffffu ? (unsigned)left : 0x7fffffffu;
-  const __amdgpu_buffer_rsrc_t orsrc = make_rsrc(C + (size_t)blockIdx.y * p.slice + origin, range);
+  const __amdgpu_buffer_rsrc_t orsrc = make_rsrc(C + (size_t)slice * p.slice + origin, range);
   int at[RT];
   float bv[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
     const bool in = m + i * 32 < p.M;
-    at[i] = in ? (nl * p.M + m + i * 32) * 4 : S_OOB;
-    bv[i] = bias && in ? bias[m + i * 32] : 0.f;
+    const int img = PC ? (m + i * 32) / p.P : 0;
+    at[i] = !in ? S_OOB : (PC ? (img * p.N + nl) * p.P + m + i * 32 - img * p.P : nl * p.M + m + i * 32) * 4;
+    bv[i] = bias && !PC && in ? bias[m + i * 32] : 0.f;
   }
-  auto store = [&](auto added) __attribute__((always_inline)) {
-    constexpr bool ADD = decltype(added)::value;
-    const __amdgpu_buffer_rsrc_t arsrc = make_rsrc(ADD ? addend + origin : nullptr, range);
+  // f(element, byte offset, whether the column exists) over the lane's elements
+  auto each = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int o = (c * 32 + 8 * (r >> 2) + (r & 3)) * p.M * 4;
+        const int col = c * 32 + 8 * (r >> 2) + (r & 3);
+        const bool is = !PC || col < cols;
+        const float bc = PC && bias && is ? bias[n0 + nl + col] : 0.f;
 #pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          float v = big[i][c][r] + bv[i];
-          if (ADD) v += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(arsrc, at[i] + o, 0, 0));
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), orsrc, at[i] + o, 0, 0);
-        }
+        for (int i = 0; i < RT; ++i) f(big[i][c][r], PC ? bc : bv[i], is ? at[i] + col * ldc * 4 : S_OOB);
       }
   };
-  if (addend) store(std::true_type{});
-  else store(std::false_type{});
+  if (addend) {                  // (all of its loads before the first store, behind which they could not move)
+    const __amdgpu_buffer_rsrc_t arsrc = make_rsrc(addend + origin, range);
+    float add[RT * CT * 16];
+    int e = 0;
+    each([&](float, float, int o) { add[e++] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(arsrc, o, 0, 0)); });
+    e = 0;
+    each([&](float v, float b, int o) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v + b + add[e++]), orsrc, o, 0, 0); });
+  } else {
+    each([&](float v, float b, int o) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v + b), orsrc, o, 0, 0); });
+  }
 }
 
-template <int MODE, int TM, int TN>
+template <int MODE, int TM, int TN, bool PL>
 int split_go(const Gemm32& p, int slices, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
-  hipLaunchKernelGGL((gemm32_split_kernel<MODE, TM, TN>), dim3((unsigned)(p.mtiles * p.ntiles), (unsigned)slices), dim3(ST), 0, s, p, A, B,
+  hipLaunchKernelGGL((gemm32_split_kernel<MODE, TM, TN, PL>), PL && MODE == 1 ? dim3((unsigned)(p.mtiles * p.ntiles * slices)) : dim3((unsigned)(p.mtiles * p.ntiles), (unsigned)slices), dim3(ST), 0, s, p, A, B,
                      bias, addend, C);
   return check_launch("matmul (fp32 in three parts)");
 }
-template <int MODE>
+template <int MODE, bool PL>
 int split_tile(int tm, int tn, const Gemm32& p, int slices, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
-  if (tm == 128 && tn == 128) return split_go<MODE, 128, 128>(p, slices, A, B, bias, addend, C, s);
-  if (tm == 128) return split_go<MODE, 128, 64>(p, slices, A, B, bias, addend, C, s);
-  return split_go<MODE, 64, 128>(p, slices, A, B, bias, addend, C, s);
+  if constexpr (!PL || MODE == 1) {
+    if (tm == 128 && tn == 128) return split_go<MODE, 128, 128, PL>(p, slices, A, B, bias, addend, C, s);
+    if (tm == 64) return split_go<MODE, 64, 128, PL>(p, slices, A, B, bias, addend, C, s);
+  }
+  return split_go<MODE, 128, 64, PL>(p, slices, A, B, bias, addend, C, s);
+}
+template <bool PL>
+int split_mode(int mode, int tm, int tn, const Gemm32& p, int slices, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
+  return mode == 0 ? split_tile<0, PL>(tm, tn, p, slices, A, B, bias, addend, C, s)
+       : mode == 1 ? split_tile<1, PL>(tm, tn, p, slices, A, B, bias, addend, C, s)
+                   : split_tile<2, PL>(tm, tn, p, slices, A, B, bias, addend, C, s);
 }
 
 }  // namespace
@@ -288,9 +381,11 @@ int split_tile(int tm, int tn, const Gemm32& p, int slices, const float* A, cons
 int gemm32_split(int mode, int tm, int tn, int slices, const Gemm32& p, const float* A, const float* B, const float* bias,
                  const float* addend, float* C, hipStream_t s) {
   if (tm * tn < 128 * 64) return -1;
-  return mode == 0 ? split_tile<0>(tm, tn, p, slices, A, B, bias, addend, C, s)
-       : mode == 1 ? split_tile<1>(tm, tn, p, slices, A, B, bias, addend, C, s)
-                   : split_tile<2>(tm, tn, p, slices, A, B, bias, addend, C, s);
+  return split_mode<false>(mode, tm, tn, p, slices, A, B, bias, addend, C, s);
+}
+int gemm32_split_planes(int mode, int tm, int tn, int slices, const Gemm32& p, const float* A, const float* B, const float* bias,
+                        const float* addend, float* C, hipStream_t s) {
+  return split_mode<true>(mode, tm, tn, p, slices, A, B, bias, addend, C, s);
 }
 
 }  // namespace flhip

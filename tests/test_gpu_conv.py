@@ -697,6 +697,55 @@ def test_fp32_one_row_filter_gradient_in_three_parts(xs, k, kw, stride, special)
             assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,stride", [
+    ((7, 36, 31, 33), 1100, 1),          # a last stage of 4 channels, positions and filters that fill no tile
+    ((61, 64, 7, 7), 1030, 1),           # tiles over several images
+    ((9, 20, 61, 45), 500, 2),           # every other position of an odd plane
+    ((4, 512, 28, 28), 64, 1),           # with an addend, one round of tiles
+    ((64, 96, 14, 14), 600, 1),          # filter gradient: planes of 12 stages and a quarter, tiles of 128 x 64
+    ((60, 60, 24, 24), 300, 1),          # 64 x 128
+    ((17, 700, 12, 12), 420, 1),         # 128 x 128
+    ((25, 100, 40, 40), 260, 1),         # slices for two workgroups to a compute unit
+])
+@pytest.mark.parametrize("special", [False, True])
+def test_fp32_1x1_windows_in_three_parts(xs, k, stride, special):
+    """Forward with a bias, backward-data with and without an addend and filter gradient against float64; sums of n rounded products
+    differ by about sqrt(n) units of 2^-24 in the 2-norm, allowed are twice that.  special: infinities, NaN and values that bf16 cannot hold
+    reach the results that they reach in fp32, and no others."""
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k)
+    r = (lambda *s: torch.rand(*s, generator=g, device="cuda") + 0.5) if special else (lambda *s: torch.randn(*s, generator=g, device="cuda"))
+    x, w, b = r(*xs), r(k, xs[1], 1, 1), r(k)
+    dy = r(xs[0], k, (xs[2] - 1) // stride + 1, (xs[3] - 1) // stride + 1)
+    addend = r(*xs)
+    if special:
+        w[:, 5] *= 1e-3
+        x[0, 3, 0, 2], x[1, 9, 2, 4], x[0, 11, 0, 0], x[1, 5, 4, 4] = float("inf"), float("-inf"), float("nan"), 3.4e38
+        dy[0, 2, 0, 1], dy[1, 30, 1, 2] = float("inf"), float("nan")
+    geo = dict(sx=stride, sy=stride)
+    y = ops.conv2d(x, w, b, **geo)
+    dx = ops.conv2d_backward_data(dy, xs, w, **geo)
+    dxa = ops.conv2d_backward_data(dy, xs, w, addend=addend, **geo)
+    dw = ops.conv2d_backward_filter_bias(dy, x, tuple(w.shape), False, **geo)[0]
+    xl = x.double()[:, :, ::stride, ::stride].flatten(2)
+    w2, d2 = w.double().view(k, -1), dy.double().flatten(2)
+    back = torch.zeros(xs, dtype=torch.float64, device="cuda")
+    back[:, :, ::stride, ::stride] = torch.matmul(w2.t().contiguous(), d2).view(xs[0], xs[1], *dy.shape[2:])
+    rows = lambda t: t.transpose(0, 1).reshape(t.shape[1], -1)
+    for name, got, ref, n in (("y", y, torch.matmul(w2, xl).view(dy.shape) + b.double().view(1, -1, 1, 1), xs[1]), ("dx", dx, back, k),
+                              ("dx + addend", dxa, back + addend.double(), k),
+                              ("dw", dw, (rows(d2) @ rows(xl).t().contiguous()).view(w.shape), d2.shape[0] * d2.shape[2])):
+        got = got.double()
+        if special:
+            ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+            assert bool((got.isnan() == ref.isnan()).all()) and bool((got.isinf() == ref.isinf()).all()), name
+            assert bool((got[ref.isinf()] == ref[ref.isinf()]).all()) and bool(ref.isnan().any()), name
+            ok = ref.isfinite()
+            assert float(((got[ok] - ref[ok]).abs() / ref[ok].abs().clamp(min=1e-3)).max()) <= 1e-5, name
+        else:
+            assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24, name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
