@@ -397,7 +397,8 @@ bool wgrad_split(WgradParams* p, const ConvGeom& g) {
   const long long base_wgs = (long long)p->ntiles_n * p->mtiles * g.groups;
   if (p->ntiles_n * p->mtiles > 65535 || g.groups > 65535) return false;
   long long ns = 2 * mfma_num_cus() / base_wgs;
-  const long long max_ns = (p->Ptotal + 63) / 64;
+  // (windows of one row have kernels of their own, and no more room is asked for on their account)
+  const long long max_ns = g.KH > 1 ? (p->Ptotal + 63) / 64 : (p->Ptotal + 255) / 256;
   if (ns > max_ns) ns = max_ns;
   if (ns < 1) ns = 1;
   long long pps = (p->Ptotal + ns - 1) / ns;
