@@ -121,11 +121,13 @@ int mfma_cells_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void*
 // bf16 3x3 stride-1 pad-1 over 64 source channels, whole contraction per workgroup (conv2d_mfma_strip_bf16.hip)
 // bf16 1x1 stride-1 convolutions with operand tiles copied to LDS by the loads themselves
 // (conv2d_mfma_pointwise_dma_bf16.hip); -1 when the shape is not theirs.  addend (or null): added
-// to the rounded input gradient.
-int mfma_pwd16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
-                        int dtype = FLHIP_BF16);
+// to the rounded input gradient.  With mfma_pwd16_conv_ws() bytes of workspace (0: never) a long contraction over few tiles is cut
+// into slices.
+size_t mfma_pwd16_conv_ws(const ConvGeom& g, bool bwd);
+int mfma_pwd16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y, hipStream_t s, int dtype, void* ws,
+                        size_t ws_bytes);
 int mfma_pwd16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, const void* addend, void* dx,
-                             hipStream_t s, int dtype);
+                             hipStream_t s, int dtype, void* ws, size_t ws_bytes);
 // their filter gradient (no bias gradient; at least 128 channels on both sides); partial tiles in ws
 size_t mfma_pwd16_wgrad_ws(const ConvGeom& g);
 // workgroups the bf16 slab kernel's forward pass would launch (0: not its shape)

@@ -301,7 +301,7 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
     if (tap1d_on(d->dtype)) r = mfma_tap1d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && tap2d_on(g, d->dtype, false)) r = mfma_tap2d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
-      r = mfma_pwd16_conv_fwd(g, x, w, bias, y, s, d->dtype);
+      r = mfma_pwd16_conv_fwd(g, x, w, bias, y, s, d->dtype, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pointwise16_conv_fwd(g, x, w, bias, y, s, ws, ws_bytes, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_FIRST) && !algo_is(Options::ALGO_CONVERT))
@@ -372,7 +372,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
     const bool lo = is_lo16(d->dtype);
     int r = -1;
     switch (plan) {
-      case 0: if (lo) r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype); break;
+      case 0: if (lo) r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype, ws, ws_bytes); break;
       case 1: if (lo) r = mfma_pointwise16_conv_bwd_data(g, dy, w, dx, s, ws, ws_bytes, d->dtype); break;
       case 2: if (lo) r = mfma_strip16_conv_bwd_data(g, dy, w, dx, s, d->dtype); break;
       case 3: if (lo) r = mfma_slab16_conv_bwd_data(g, dy, w, dx, s, d->dtype); break;
@@ -395,7 +395,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
     if (r < 0 && tap2d_on(g, d->dtype, true)) r = mfma_tap2d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && !skip(Options::SKIP_CELLS)) r = mfma_cells_conv_bwd_data(g, d->dtype, dy, w, dx, s);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
-      r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype);
+      r = mfma_pwd16_conv_bwd_data(g, dy, w, nullptr, dx, s, d->dtype, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pointwise16_conv_bwd_data(g, dy, w, dx, s, ws, ws_bytes, d->dtype);
     if (r < 0 && thin_on(g, d->dtype, true, true)) r = mfma_thin_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
@@ -454,7 +454,7 @@ extern "C" int flhip_conv2d_bwd_data_add(const flhip_conv_desc* d, const void* d
   // write dx before they read addend
   FLHIP_REQUIRE(dx != addend, "conv2d_bwd_data_add: dx aliases addend");
   if (!force_direct() && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT)) {
-    int r = skip(Options::SKIP_PWDMA) ? -1 : mfma_pwd16_conv_bwd_data(g, dy, w, addend, dx, s, d->dtype);
+    int r = skip(Options::SKIP_PWDMA) ? -1 : mfma_pwd16_conv_bwd_data(g, dy, w, addend, dx, s, d->dtype, ws, ws_bytes);
     if (r < 0) r = mfma_pointwise16_conv_bwd_data_add(g, dy, w, addend, dx, s, d->dtype);
     if (r >= 0) return r;
   }

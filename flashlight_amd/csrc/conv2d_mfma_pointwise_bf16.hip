@@ -1006,11 +1006,18 @@ bool pw16_taps_forward(const ConvGeom& g, const ConvGeom& c) {
 
 }  // namespace
 
+static size_t part_offset(const ConvGeom& c) { return (lattice_bytes(c) + 255) / 256 * 256; }
+static size_t compact_ws(const ConvGeom& c, bool bwd) {
+  const size_t part = mfma_pwd16_conv_ws(c, bwd);
+  return part ? part_offset(c) + part : lattice_bytes(c);
+}
+
+// (the compact tensor and, where the product's contraction is cut into slices, their partial results; 1x1 layers of stride 1: these alone)
 size_t mfma_pointwise16_lattice_ws(const ConvGeom& g, bool bwd) {
   ConvGeom c;
-  if (pw16_strided_plan(g, &c)) return lattice_bytes(c);
-  if (!options().pw16_no_taps && pw16_taps_plan(g, &c) && (bwd || pw16_taps_forward(g, c))) return lattice_bytes(c);
-  return 0;
+  if (pw16_strided_plan(g, &c)) return compact_ws(c, bwd);
+  if (!options().pw16_no_taps && pw16_taps_plan(g, &c) && (bwd || pw16_taps_forward(g, c))) return compact_ws(c, bwd);
+  return mfma_pwd16_conv_ws(g, bwd);
 }
 
 // Bytes of the gathered input that the forward pass of this geometry leaves at the start of its workspace and
@@ -1030,10 +1037,13 @@ size_t mfma_pointwise16_gathered_bytes(const ConvGeom& g) {
 // the compact 1x1 problem of a strided layer: on the kernels that load straight to LDS where those
 // are ahead, else on the ones above
 template <typename E, bool BWD>
-int launch_compact(const ConvGeom& c, const void* src, const void* w, const float* bias, void* dst, hipStream_t s) {
+int launch_compact(const ConvGeom& c, const void* src, const void* w, const float* bias, void* dst, hipStream_t s, void* ws, size_t ws_bytes) {
   if (!(options().conv_skip & Options::SKIP_PWDMA)) {
-    const int r = BWD ? mfma_pwd16_conv_bwd_data(c, src, w, nullptr, dst, s, Lo16<E>::TAG)
-                      : mfma_pwd16_conv_fwd(c, src, w, bias, dst, s, Lo16<E>::TAG);
+    // (behind the compact tensor: room for the contraction's slices)
+    const size_t lat = part_offset(c);
+    void* const part = ws_bytes > lat ? static_cast<char*>(ws) + lat : nullptr;
+    const int r = BWD ? mfma_pwd16_conv_bwd_data(c, src, w, nullptr, dst, s, Lo16<E>::TAG, part, part ? ws_bytes - lat : 0)
+                      : mfma_pwd16_conv_fwd(c, src, w, bias, dst, s, Lo16<E>::TAG, part, part ? ws_bytes - lat : 0);
     if (r >= 0) return r;
   }
   return launch_pw16<E, BWD>(c, src, w, bias, dst, s);
@@ -1046,11 +1056,11 @@ static int pointwise16_conv_fwd_impl(const ConvGeom& g, const void* x, const voi
   if (pw16_strided_plan(g, &c)) {
     if (!ws || ws_bytes < lattice_bytes(c)) return -1;
     lattice_gather(g, x, ws, s);
-    return launch_compact<E, false>(c, ws, w, bias, y, s);
+    return launch_compact<E, false>(c, ws, w, bias, y, s, ws, ws_bytes);
   }
   if (!options().pw16_no_taps && pw16_taps_plan(g, &c) && pw16_taps_forward(g, c) && ws && ws_bytes >= lattice_bytes(c) &&
       taps_gather(g, x, ws, s))
-    return launch_compact<E, false>(c, ws, w, bias, y, s);
+    return launch_compact<E, false>(c, ws, w, bias, y, s, ws, ws_bytes);
   if (!pw16_applies(g)) return -1;
   return launch_pw16<E, false>(g, x, w, bias, y, s);
 }
@@ -1061,14 +1071,14 @@ static int pointwise16_conv_bwd_data_impl(const ConvGeom& g, const void* dy, con
   ConvGeom c;
   if (pw16_strided_plan(g, &c)) {
     if (!ws || ws_bytes < lattice_bytes(c)) return -1;
-    const int rc = launch_compact<E, true>(c, dy, w, nullptr, ws, s);
+    const int rc = launch_compact<E, true>(c, dy, w, nullptr, ws, s, ws, ws_bytes);
     if (rc != FLHIP_OK) return rc;
     lattice_scatter(g, ws, dx, s);
     return check_launch("conv2d_bwd_data strided 1x1 (bf16 mfma)");
   }
   if (!options().pw16_no_taps && pw16_taps_plan(g, &c)) {
     if (!ws || ws_bytes < lattice_bytes(c)) return -1;
-    const int rc = launch_compact<E, true>(c, dy, w, nullptr, ws, s);
+    const int rc = launch_compact<E, true>(c, dy, w, nullptr, ws, s, ws, ws_bytes);
     if (rc != FLHIP_OK) return rc;
     if (!taps_spread<E>(g, ws, dx, s)) return fail(FLHIP_RUNTIME_ERROR, "conv2d_bwd_data: plane too wide for the spread kernel");
     return check_launch("conv2d_bwd_data strided window (bf16 mfma)");

@@ -68,11 +68,11 @@ struct PwdParams {
   int nstages, mtiles, ctiles;
   unsigned src_bytes, w_bytes, dst_bytes;
   const float* pos_bias;   // one value per position, added to every result channel (matrix products: one image), or null
-  // matrix products with the contraction cut into slices (blockIdx.y): sps stages per slice (nstages: one slice), and
-  // where slice k leaves its fp32 partial product, [result channel][position], Mo * P floats per slice (null: one slice,
-  // results in the element type at dst)
-  int sps;
+  // the contraction cut into `slices`: sps stages per slice (nstages: one slice), and where slice k leaves its fp32
+  // partial product, [image][result channel][position], `slice` floats per slice (null: one slice, results in the element type at dst)
+  int sps, slices;
   float* part;
+  size_t slice;
 };
 
 // rows r0 .. r0+7 of column c0 + s of a 16-bit tile stored [row][column] (see the 1x1 kernels
@@ -125,10 +125,13 @@ pwd16_conv_kernel(PwdParams p, const E* __restrict__ src, const E* __restrict__ 
   static_assert(PD_NS == 4 || PD_NS == 8, "the ring slot is the stage number modulo a power of two");
 
   // consecutive workgroups go to different XCDs: the channel tiles that share a source tile
-  // run back to back on one XCD
+  // run back to back on one XCD; the slices of a source tile, which share nothing, go to different ones (with a slice's source
+  // tiles on the XCDs that the slice before had, layers of one or two source tiles ran on as many XCDs: 2048 channels from 512 over
+  // 7 x 7, one image, two slices 12.8 us, one slice 8.2)
   const int id = blockIdx.x, xcd = id & 7, seq = id >> 3;
-  const int mtile = seq % p.mtiles, ctile = (seq / p.mtiles) * 8 + xcd;
-  if (ctile >= p.ctiles) return;
+  const int mtile = seq % p.mtiles, unit = (seq / p.mtiles) * 8 + xcd;
+  if (unit >= p.ctiles * p.slices) return;
+  const int slice = p.slices > 1 ? unit / p.ctiles : 0, ctile = unit - slice * p.ctiles;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = mtile * BM, cell0 = ctile * PD_CELLS;
@@ -168,7 +171,7 @@ pwd16_conv_kernel(PwdParams p, const E* __restrict__ src, const E* __restrict__ 
     }
   }
   const bool fourth = wave + 12 < NI, fifth = wave + 16 < NI;
-  const int sbeg = blockIdx.y * p.sps;      // this slice's first stage
+  const int sbeg = slice * p.sps;      // this slice's first stage
   const int n = min(p.nstages - sbeg, p.sps), n2 = (n + 1) & ~1;
   // stages are multiplied in pairs: with an odd number the stage past the contraction fetches nothing and fills its
   // slot with zeros (both operands: it adds 0)
@@ -256,24 +259,25 @@ pwd16_conv_kernel(PwdParams p, const E* __restrict__ src, const E* __restrict__ 
 #undef PD_READ
 
   if (p.part) {
-    // a slice's partial product leaves in fp32 straight from the accumulators (one image): a lane's four consecutive
+    // a slice's partial product leaves in fp32 straight from the accumulators: a lane's four consecutive
     // positions of a result channel; the positions a plane's last cell repeats are written twice with the same value
-    float* const part = p.part + (size_t)blockIdx.y * p.Mo * p.P;
+    // (16 bytes per store, from any element on)
+    const __amdgpu_buffer_rsrc_t prs = make_rsrc(p.part + slice * p.slice, (unsigned)(p.slice * 4));
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int ch = m0 + mw0 + j * 32 + fr;
-      if (ch >= p.Mo) continue;
+    for (int i = 0; i < NA; ++i)
 #pragma unroll
-      for (int i = 0; i < NA; ++i)
+      for (int g = 0; g < 4; ++g) {
+        const int cell = cell0 + (pos0 + i * 32) / 8 + g;
+        if (cell >= p.ncells) continue;
+        const int img = cell / p.Pc, at = min(8 * (cell - img * p.Pc), p.P - 8) + fh * 4;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int cell = cell0 + (pos0 + i * 32) / 8 + g;
-          if (cell >= p.ncells) continue;
-          float* q = part + (size_t)ch * p.P + min(8 * cell, p.P - 8) + fh * 4;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) q[e] = acc[i][j][4 * g + e];
+        for (int j = 0; j < 2; ++j) {
+          const int ch = m0 + mw0 + j * 32 + fr;
+          if (ch >= p.Mo) continue;
+          const floatx4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4_t, v), prs, ((img * p.Mo + ch) * p.P + at) * 4, 0, 0);
         }
-    }
+      }
     return;
   }
   __syncthreads();      // every wave has read its last fragments: the ring becomes the staging tile
@@ -355,7 +359,7 @@ int pwd16_bm(const PwdParams& p) {
 }
 
 // conv: a convolution (else a matrix product).  grid and kernel variant for a filled-in PwdParams (Kc, Mo, P, Pc, ncells, nstages, ctiles and the byte sizes)
-// slices > 1 (matrix products): the contraction in that many slices at most, their fp32 partial products at p.part
+// slices > 1: the contraction in that many slices at most, their fp32 partial products at p.part
 template <typename E, bool BWD>
 int pwd16_go(PwdParams p, const void* src, const void* w, const float* bias, void* dst, const void* addend,
              hipStream_t s, const char* what, bool conv, int* slices = nullptr) {
@@ -372,8 +376,6 @@ int pwd16_go(PwdParams p, const void* src, const void* w, const float* bias, voi
   const int bm = pwd16_bm(p);
   const bool small = bm == 64;
   p.mtiles = (p.Mo + bm - 1) / bm;
-  const long long grid = (long long)((p.ctiles + 7) / 8) * 8 * p.mtiles;
-  if (grid > 0x7fffffffll) return -1;
   int ns = 1;
   p.sps = p.nstages;
   if (slices) {
@@ -381,8 +383,11 @@ int pwd16_go(PwdParams p, const void* src, const void* w, const float* bias, voi
     *slices = ns;
     if (ns <= 1) p.part = nullptr;
   }
+  p.slices = ns;
+  const long long grid = ((long long)p.ctiles * ns + 7) / 8 * 8 * p.mtiles;
+  if (grid > 0x7fffffffll) return -1;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)ns), dim3(256), 0, s, p, static_cast<const E*>(src),
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, s, p, static_cast<const E*>(src),
                        static_cast<const E*>(w), bias, static_cast<E*>(dst), static_cast<const E*>(addend));
   };
   bool deep = (long long)p.ctiles * p.mtiles * ns <= (long long)cus;
@@ -413,17 +418,83 @@ bool pwd16_sizes(PwdParams* p, long long images) {
   return images * p->Pc <= 0x7fffffffll;
 }
 
+bool pwd16_conv_plan(const ConvGeom& g, bool bwd, PwdParams* p) {
+  if (!pwd16_applies(g, bwd)) return false;
+  p->Kc = bwd ? g.K : g.C;
+  p->Mo = bwd ? g.C : g.K;
+  p->P = g.H * g.W;
+  return pwd16_sizes(p, g.N);
+}
+
+// Slices of a layer's contraction: few tiles of many stages leave most of the chip idle behind one chain of stages.  A stage takes
+// 0.24 us or more, over planes of an odd number of positions 0.34; cutting costs 3 us (the second launch), 0.2 per slice and 1.9 per
+// slice and million results (written in fp32 and read back), and it has to be worth another 4, the second launch's time on the host,
+// which small batches wait for.  Fitted to 0.01 to 1 million results over 16 to 279 stages, 1 / 2 / 4 / 8 slices, us: 8 tiles of 64 stages
+// 17.7 / 13.0 / 9.5 / 8.4, 40 tiles (2048 -> 512 channels over 7 x 7, 10 images) 24.2 / 17.6 / 13.4 / 14.2, 120 tiles (33 images) 25 /
+// 20.7, of 144 stages (3 x 3 of stride 2 to 512 channels) 65 / 48; not where it loses: 96 tiles of 32 stages 11.6 / 13.3, 128 of 16 8.4 /
+// 12.6, or gains little: 8 of 32 11.2 / 9.7 / 8.0.
+int pwd16_conv_slices(const ConvGeom& g, const PwdParams& p) {
+  if (p.nstages < 40 || options().pw16_pf) return 1;      // (fewer never make up for it; asked for on every call)
+  const int bm = pwd16_bm(p), tiles = p.ctiles * ((p.Mo + bm - 1) / bm);
+  const int most = std::min(8, std::min(p.nstages / 8, mfma_num_cus() / tiles));
+  if (most < 2 || mfma_big16_halves(true, g.N, p.Kc, p.Mo, p.P) >= 0) return 1;
+  const double million = 1e-6 * g.N * p.Mo * p.P, stage = p.P % 2 ? 0.34 : 0.24;
+  double best = stage * p.nstages;
+  int slices = 1;
+  for (int ns = 2; ns <= most; ++ns) {
+    const int sps = (p.nstages + ns - 1) / ns;
+    const double t = stage * sps + 7 + 0.2 * ns + 1.9 * ns * million;
+    if (t < best) best = t, slices = (p.nstages + sps - 1) / sps;
+  }
+  return slices;
+}
+
+// dst = the sum of `slices` fp32 partial products, n floats apart, added in slice order, + bias[channel], rounded once, + addend, rounded
+// once more; eight elements per thread (n is a multiple of 8: so is the number of result channels)
+template <typename E>
+__global__ void __launch_bounds__(256)
+pwd16_sum_kernel(const float* __restrict__ part, const float* __restrict__ bias, const E* __restrict__ addend, E* __restrict__ dst, unsigned bytes,
+                 unsigned n, int slices, int P, int Mo) {
+  const unsigned i = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= n) return;
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < slices; ++k) {
+    const float4* q = reinterpret_cast<const float4*>(part + (size_t)k * n + i);
+    const float4 a = q[0], b = q[1];
+    v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+    v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+  }
+  if (bias)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += bias[(i + e) / P % Mo];
+  uintx4_t o = {Lo16<E>::pack(v[0], v[1]), Lo16<E>::pack(v[2], v[3]), Lo16<E>::pack(v[4], v[5]), Lo16<E>::pack(v[6], v[7])};
+  if (addend) {
+    const uintx4_t a = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(addend, bytes), i * 2, 0, 0);
+    o = uintx4_t{pd_add_x2<E>(o.x, a.x), pd_add_x2<E>(o.y, a.y), pd_add_x2<E>(o.z, a.z), pd_add_x2<E>(o.w, a.w)};
+  }
+  __builtin_amdgcn_raw_buffer_store_b128(o, make_rsrc(dst, bytes), i * 2, 0, 0);
+}
+
 template <typename E, bool BWD>
 int launch_pwd16(const ConvGeom& g, const void* src, const void* w, const float* bias, void* dst, const void* addend,
-                 hipStream_t s) {
-  if (!pwd16_applies(g, BWD)) return -1;
+                 hipStream_t s, void* ws, size_t ws_bytes) {
   PwdParams p{};
-  p.Kc = BWD ? g.K : g.C;
-  p.Mo = BWD ? g.C : g.K;
-  p.P = g.H * g.W;
-  if (!pwd16_sizes(&p, g.N)) return -1;
-  return pwd16_go<E, BWD>(p, src, w, bias, dst, addend, s,
-                          BWD ? "conv2d_bwd_data 1x1 (bf16 mfma, direct-to-LDS)" : "conv2d_fwd 1x1 (bf16 mfma, direct-to-LDS)", true);
+  if (!pwd16_conv_plan(g, BWD, &p)) return -1;
+  const char* const what = BWD ? "conv2d_bwd_data 1x1 (bf16 mfma, direct-to-LDS)" : "conv2d_fwd 1x1 (bf16 mfma, direct-to-LDS)";
+  const size_t n = (size_t)g.N * p.Mo * p.P;
+  int slices = pwd16_conv_slices(g, p);
+  if (slices <= 1 || !ws || ws_bytes < slices * n * sizeof(float) || reinterpret_cast<uintptr_t>(ws) % 16 != 0)
+    return pwd16_go<E, BWD>(p, src, w, bias, dst, addend, s, what, true);
+  p.part = static_cast<float*>(ws);
+  p.slice = n;
+  const int rc = pwd16_go<E, BWD>(p, src, w, nullptr, dst, nullptr, s, what, true, &slices);
+  if (rc) return rc;
+  hipLaunchKernelGGL((pwd16_sum_kernel<E>), dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, p.part, bias, static_cast<const E*>(addend),
+                     static_cast<E*>(dst), p.dst_bytes, (unsigned)n, slices, p.P, p.Mo);
+  return check_launch("conv2d 1x1 (slices added)");
 }
 
 
@@ -652,13 +723,22 @@ bool pwd16_wgrad_plan(const ConvGeom& g, PwdWgradParams* p) {
 
 }  // namespace
 
-int mfma_pwd16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y, hipStream_t s, int dtype) {
-  return by_lo16(dtype, [&](auto* e_) { return launch_pwd16<FLHIP_T_OF(e_), false>(g, x, w, bias, y, nullptr, s); });
+// bytes of workspace with which a 1x1 layer's contraction is cut into slices (0: it is not, or not these kernels')
+size_t mfma_pwd16_conv_ws(const ConvGeom& g, bool bwd) {
+  PwdParams p{};
+  if (!pwd16_conv_plan(g, bwd, &p)) return 0;
+  const int slices = pwd16_conv_slices(g, p);
+  return slices > 1 ? (size_t)slices * g.N * p.Mo * p.P * sizeof(float) : 0;
+}
+
+int mfma_pwd16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const float* bias, void* y, hipStream_t s, int dtype, void* ws,
+                        size_t ws_bytes) {
+  return by_lo16(dtype, [&](auto* e_) { return launch_pwd16<FLHIP_T_OF(e_), false>(g, x, w, bias, y, nullptr, s, ws, ws_bytes); });
 }
 
 int mfma_pwd16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, const void* addend, void* dx,
-                             hipStream_t s, int dtype) {
-  return by_lo16(dtype, [&](auto* e_) { return launch_pwd16<FLHIP_T_OF(e_), true>(g, dy, w, nullptr, dx, addend, s); });
+                             hipStream_t s, int dtype, void* ws, size_t ws_bytes) {
+  return by_lo16(dtype, [&](auto* e_) { return launch_pwd16<FLHIP_T_OF(e_), true>(g, dy, w, nullptr, dx, addend, s, ws, ws_bytes); });
 }
 
 }  // namespace flhip
@@ -780,6 +860,7 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
     int slices = ws ? (int)std::min<size_t>(ws_bytes / per, 32) : 1;
     if (slices <= 1) return pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false);
     p.part = static_cast<float*>(ws);
+    p.slice = (size_t)M * N;
     const int rc = pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false, &slices);
     if (rc != 0 || slices <= 1) return rc;
     const size_t n = (size_t)M * N;

@@ -578,6 +578,51 @@ def test_1x1_windows_on_large_tiles(xs, k, dtype):
     assert bool(((dx.float() - total).abs() <= unit * ((1 + unit) * want.abs() + total.abs()) + 1e-4).all())
 
 
+@pytest.mark.parametrize("xs,ws,stride", [
+    ((1, 2048, 7, 7), (512, 2048, 1, 1), 1),       # eight slices; rows of odd planes in pieces of 8 that overlap
+    ((3, 1824, 6, 6), (72, 1824, 1, 1), 1),        # 57 stages: slices of different lengths, a tile of 8 channels
+    ((9, 512, 7, 7), (2048, 512, 1, 1), 1),        # backward-data: 64 stages, 32 tiles
+    ((2, 512, 14, 14), (512, 512, 3, 3), 2),       # gathered taps, partial results behind them
+    ((3, 2048, 9, 11), (136, 2048, 1, 1), 2),      # every other position, a plane of 30
+    ((2, 1312, 3, 3), (2048, 1312, 1, 1), 1),      # planes of 9 positions
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_1x1_windows_with_the_contraction_in_slices(xs, ws, stride, dtype):
+    """Forward with a bias, backward-data with and without an addend, against fp32 products of the same operands; run to run the same bits;
+    with less workspace than asked for, the same results in one slice."""
+    import ctypes as C
+    import torch.nn.functional as F
+    from flashlight_amd import capi, ops
+    g = torch.Generator(device="cuda").manual_seed(ws[0])
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    pad = ws[2] // 2
+    geo = dict(sx=stride, sy=stride, px=pad, py=pad)
+    n = ws[1] * ws[2] * ws[3]
+    x, w, b = r(*xs).to(dtype), (r(*ws) / n ** 0.5).to(dtype), r(ws[0])
+    y = ops.conv2d(x, w, b, **geo)
+    dy, add = r(*y.shape).to(dtype), r(*xs).to(dtype)
+    dx, dxa = ops.conv2d_backward_data(dy, xs, w, **geo), ops.conv2d_backward_data(dy, xs, w, addend=add, **geo)
+    assert torch.equal(y, ops.conv2d(x, w, b, **geo)) and torch.equal(dx, ops.conv2d_backward_data(dy, xs, w, **geo))
+    w2, un = w.float().view(ws[0], -1), dict(kernel_size=ws[2:], padding=pad, stride=stride)
+    want = torch.matmul(w2, F.unfold(x.float(), **un)).view(y.shape) + b.view(1, -1, 1, 1)
+    taps = torch.matmul(w2.t().contiguous(), dy.float().flatten(2))
+    back = F.fold(taps, xs[2:], **un)
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    # (windows of several taps: each tap's product is rounded before the sum of those that reach a position)
+    each = F.fold(taps.abs(), xs[2:], **un) if ws[2] > 1 else 0 * back
+    assert bool(((y.float() - want).abs() <= unit * want.abs() + 1e-4).all())
+    assert bool(((dx.float() - back).abs() <= unit * (back.abs() + (1 + unit) * each) + 1e-4).all())
+    total = back + add.float()
+    assert bool(((dxa.float() - total).abs() <= unit * ((1 + unit) * (back.abs() + each) + total.abs()) + 1e-4).all())
+    cd = capi.ConvDesc(*xs, ws[0], ws[2], ws[3], stride, stride, pad, pad, 1, 1, 1, ops._dtype_tag(x))
+    nws = capi.lib().flhip_conv2d_workspace_bytes(C.byref(cd), capi.CONV_FWD) // 2
+    if stride == 1 and nws:
+        short, y1 = torch.empty(nws, dtype=torch.uint8, device="cuda"), torch.empty_like(y)
+        capi.check(capi.lib().flhip_conv2d_fwd(C.byref(cd), x.data_ptr(), w.data_ptr(), b.data_ptr(), y1.data_ptr(), short.data_ptr(), nws, None))
+        torch.cuda.synchronize()
+        assert bool(((y1.float() - want).abs() <= unit * want.abs() + 1e-4).all())
+
+
 # (planes, weights, stride): a tile's blocks 1 to 4 of 32 positions, 128 or 64 result channels, one or two slab rows per thread
 PARTS_CASES = [
     ((1, 16, 1, 33), (32, 16, 1, 2), 1),            # the smallest of everything, one chunk
