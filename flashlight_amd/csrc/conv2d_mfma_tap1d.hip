@@ -11,11 +11,11 @@
 // (channel-major rows of positions) a shifted 16-byte fragment would start on any element
 // boundary.  So two small passes first bring the operands into the order the instruction reads:
 //   rows     xr[sequence][position][Cs]: the source with its channels last, Cs = the channel
-//            count padded with zeros (tap1d_rows_kernel; a sequence is one (image, row) pair); a
+//            count padded with zeros (tap1d_rows_block; a sequence is one (image, row) pair); a
 //            tap then shifts whole 16-byte cells (8 channels of one position);
 //   weights  wf[block of 32 result channels][tap][stage of 2 cells][lane][cell]: the fragment
 //            of every (tap, stage) exactly as the 64 lanes hold it, in the order the kernel walks
-//            (tap1d_weights_kernel); padded channels and taps are zero.
+//            (tap1d_weights_block); padded channels and taps are zero.
 // A stage is 16 channels, one matrix instruction per block.
 // Backward-data over a stride of 2 is two interleaved stride-1 problems (the results of even
 // and of odd index take the taps of one parity each): "phases" of one workgroup, which
@@ -57,6 +57,7 @@ typedef const uintx4_t* lds_cell_t;
 #endif
 
 constexpr int T1_BM = 128;       // result channels per workgroup
+constexpr int T1_KW = 32;        // taps of a window
 constexpr int T1_MAXTAPS = 64;   // taps over both phases, padding included
 constexpr int T1_OOB = (int)0x80000000;
 
@@ -97,24 +98,30 @@ struct Tap1Params {
 };
 
 // ---- operand passes ------------------------------------------------------------------------
+// two neighbouring 16-bit values from any address, the second one only where it exists
+struct __attribute__((packed, aligned(2))) Pair16 {
+  uint32_t v;
+};
+template <typename T>
+__device__ __forceinline__ uint32_t pair_at(const T* p, int left) {
+  return left >= 2 ? reinterpret_cast<const Pair16*>(p)->v : left == 1 ? (uint32_t)__builtin_bit_cast(uint16_t, *p) : 0u;
+}
+
 // x[n][c][h][t] -> xr[n * H + h][t][Cs], channels c >= C zero.  A block transposes 64 channels x 64
-// positions through LDS: (bf16: pairs of positions in, where rows of an even length start on 4-byte
-// boundaries;) whole 16-byte cells out.
-template <typename T, bool PAIRS>
-__global__ void __launch_bounds__(256)
-tap1d_rows_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int Tn, int Cs) {
+// positions through LDS: (16-bit storage: pairs of positions in;) whole 16-byte cells out.
+template <typename T>
+__device__ __forceinline__ void tap1d_rows_block(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int Tn, int Cs, int bx, int by,
+                                                 int row, void* lds) {
   constexpr int CELL = Tap1Elem<T>::CELL;
-  __shared__ T tile[64][sizeof(T) == 2 ? 66 : 65];
-  const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64, row = blockIdx.z;
+  T(*tile)[sizeof(T) == 2 ? 66 : 65] = reinterpret_cast<T(*)[sizeof(T) == 2 ? 66 : 65]>(lds);
+  const int t0 = bx * 64, c0 = by * 64;
   const int n = row / H, h = row - n * H;
-  if (PAIRS && sizeof(T) == 2) {
+  if constexpr (sizeof(T) == 2) {
     const int tp = threadIdx.x & 31, cy = threadIdx.x >> 5;      // pair of positions, channel (+ 8 i)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int c = c0 + cy + 8 * i, t = t0 + 2 * tp;
-      uint32_t v = 0u;
-      if (c < C && t < Tn) v = *reinterpret_cast<const uint32_t*>(x + (((size_t)n * C + c) * H + h) * Tn + t);   // (Tn is even)
-      *reinterpret_cast<uint32_t*>(&tile[cy + 8 * i][2 * tp]) = v;
+      *reinterpret_cast<uint32_t*>(&tile[cy + 8 * i][2 * tp]) = pair_at(x + (((size_t)n * C + c) * H + h) * Tn + t, c < C ? Tn - t : 0);
     }
   } else {
     const int tx = threadIdx.x & 63, cy = threadIdx.x >> 6;
@@ -140,12 +147,17 @@ tap1d_rows_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int
 }
 
 template <typename T>
+__global__ void __launch_bounds__(256)
+tap1d_rows_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int Tn, int Cs) {
+  __shared__ __align__(16) T tile[64][sizeof(T) == 2 ? 66 : 65];
+  tap1d_rows_block(x, xr, C, H, Tn, Cs, blockIdx.x, blockIdx.y, blockIdx.z, tile);
+}
+
+static dim3 rows_grid(int Tn, int Cs, int rows) { return dim3((unsigned)((Tn + 63) / 64), (unsigned)((Cs + 63) / 64), (unsigned)rows); }
+
+template <typename T>
 static void launch_rows(const T* x, T* xr, int C, int H, int Tn, int Cs, int rows, hipStream_t s) {
-  const dim3 grid((unsigned)((Tn + 63) / 64), (unsigned)((Cs + 63) / 64), (unsigned)rows);
-  if (sizeof(T) == 2 && Tn % 2 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0)
-    hipLaunchKernelGGL((tap1d_rows_kernel<T, true>), grid, dim3(256), 0, s, x, xr, C, H, Tn, Cs);
-  else
-    hipLaunchKernelGGL((tap1d_rows_kernel<T, false>), grid, dim3(256), 0, s, x, xr, C, H, Tn, Cs);
+  hipLaunchKernelGGL((tap1d_rows_kernel<T>), rows_grid(Tn, Cs, rows), dim3(256), 0, s, x, xr, C, H, Tn, Cs);
 }
 
 struct Tap1Weights {
@@ -157,29 +169,63 @@ struct Tap1Weights {
   signed char tapj[T1_MAXTAPS];   // weight tap of stored tap i (-1: padding)
 };
 
+// The fragments of 32 result channels x 16 contraction channels, every tap: 32 (or, over the filters, 16) runs of 16 (32) channels'
+// taps come in as pairs of neighbours and leave LDS tap by tap.
+template <typename T>
+__device__ __forceinline__ void tap1d_weights_block(const T* __restrict__ w, uintx4_t* __restrict__ wf, const Tap1Weights& p, int block, T* lds) {
+  const int mblk = block / p.KS, ks = block - mblk * p.KS, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = mblk * 32, c0 = ks * 16;
+  // a row of the runs: its threads, pairs between two of a thread, the source's first element and how many follow in range
+  const int per = p.bwd ? 16 : 8, r = tid / per, q = tid % per, pitch = (p.bwd ? 34 : 16) * p.KW + 2;
+  // (neighbouring lanes read elements KW apart over the filters: two unused ones after every 32 keep even KW off one bank)
+  const auto at = [&](int e) { return p.bwd ? e + 2 * (e >> 5) : e; };
+  const int first = (p.bwd ? m0 : c0) * p.KW, row = (p.bwd ? c0 : m0) + r;
+  const int left = row < (p.bwd ? p.Cc : p.Mo) ? p.Cw * p.KW - first : 0;
+  const T* const src = w + (size_t)(left > 0 ? row : 0) * p.Cw * p.KW + first;
+  uint32_t in[T1_KW];                     // (all of a thread's loads before the first value is waited for)
+#pragma unroll
+  for (int k = 0; k < T1_KW; ++k) {
+    const int e = 2 * (q + per * k);
+    if (k < p.KW) in[k] = pair_at(src + e, left - e);
+  }
+#pragma unroll
+  for (int k = 0; k < T1_KW; ++k)
+    if (k < p.KW) *reinterpret_cast<uint32_t*>(lds + r * pitch + at(2 * (q + per * k))) = in[k];
+  __syncthreads();
+  const int fr = lane & 31, fh = lane >> 5;
+  const T* const mine = lds + (p.bwd ? 8 * fh : fr) * pitch;
+  const int run = (p.bwd ? fr : 8 * fh) * p.KW, step = p.bwd ? pitch : p.KW;
+#pragma unroll 4
+  for (int tap = wave; tap < p.taps_total; tap += 4) {
+    const int j = p.tapj[tap];
+    const T* const from = mine + at(run + max(j, 0));
+    __attribute__((aligned(16))) T v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = from[e * step];
+    if (j < 0)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = T{};
+    wf[(((size_t)mblk * p.taps_total + tap) * p.KS + ks) * 64 + lane] = *reinterpret_cast<const uintx4_t*>(v);
+  }
+}
+
+// Both operands of a layer in 16-bit storage in one launch: neither pass fills the chip, and each is a few microseconds of latency
+// (loads, LDS, stores).  The first blocks take the rows, the others the weights.  Rows one element at a time where they are odd, and
+// weights gathered fragment by fragment (every line met once per tap) in a launch of their own: 8.2 + 8.8 us for 250 -> 250 channels, 21 taps
+// over 7 x 1111 frames, and a launch more for the host; the layer's passes replayed from a graph 48.6 -> 44.6 and 45.5 -> 44.2; 120 random layers in bf16 and f16 0.87 of the time forward, 0.89 backward, the
+// slowest 1.09 (over 29 filters, 13.0 -> 14.2 us: 16 blocks of weights).
 template <typename T>
 __global__ void __launch_bounds__(256)
-tap1d_weights_kernel(const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p) {
-  constexpr int CELL = Tap1Elem<T>::CELL;
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long total = (long long)p.mblocks * p.taps_total * p.KS * 64;
-  if (idx >= total) return;
-  const int lane = (int)(idx & 63);
-  const long long st = idx >> 6;
-  const int per_block = p.taps_total * p.KS;
-  const int mblk = (int)(st / per_block), s = (int)(st - (long long)mblk * per_block);
-  const int tap = s / p.KS, ks = s - tap * p.KS;
-  const int m = mblk * 32 + (lane & 31), c0 = (2 * ks + (lane >> 5)) * CELL;
-  const int j = p.tapj[tap];
-  __attribute__((aligned(16))) T v[CELL];
-#pragma unroll
-  for (int e = 0; e < CELL; ++e) {
-    const int c = c0 + e;
-    v[e] = T{};
-    if (j >= 0 && m < p.Mo && c < p.Cc)
-      v[e] = w[p.bwd ? ((size_t)c * p.Cw + m) * p.KW + j : ((size_t)m * p.Cw + c) * p.KW + j];
+tap1d_operands_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int Tn, int Cs, int tblocks, int cblocks, int rblocks,
+                      const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p) {
+  extern __shared__ uintx4_t t1_operands[];
+  const int b = blockIdx.x;
+  if (b < rblocks) {
+    const int t = b / tblocks;
+    tap1d_rows_block(x, xr, C, H, Tn, Cs, b - t * tblocks, t % cblocks, t / cblocks, t1_operands);
+  } else {
+    tap1d_weights_block(w, wf, p, b - rblocks, reinterpret_cast<T*>(t1_operands));
   }
-  wf[idx] = *reinterpret_cast<const uintx4_t*>(v);
 }
 
 // The same fragments with the tap as the index that changes fastest after the lane: the four waves of a block then read
@@ -590,11 +636,12 @@ int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const 
   if (!ws || ws_bytes < pl.rows_bytes + pl.w_bytes) return -1;
   T* xr = static_cast<T*>(ws);
   uintx4_t* wf = reinterpret_cast<uintx4_t*>(static_cast<char*>(ws) + pl.rows_bytes);
-  launch_rows(static_cast<const T*>(src), xr, pl.C, pl.H, pl.T, pl.p.Cs, pl.p.rows, s);
   {
-    const long long total = (long long)pl.w.mblocks * pl.w.taps_total * pl.w.KS * 64;
-    hipLaunchKernelGGL(tap1d_weights_kernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const T*>(w), wf, pl.w);
+    const dim3 rg = rows_grid(pl.T, pl.p.Cs, pl.p.rows);
+    const size_t rblocks = (size_t)rg.x * rg.y * rg.z, blocks = rblocks + (size_t)pl.w.mblocks * pl.w.KS;
+    const size_t lds = std::max<size_t>(64 * 66 * sizeof(T), (544 * (size_t)pl.w.KW + 64) * sizeof(T));
+    hipLaunchKernelGGL((tap1d_operands_kernel<T>), dim3((unsigned)blocks), dim3(256), lds, s, static_cast<const T*>(src), xr, pl.C, pl.H, pl.T,
+                       pl.p.Cs, (int)rg.x, (int)rg.y, (int)rblocks, static_cast<const T*>(w), wf, pl.w);
   }
   if (const int rc = check_launch("conv2d (one-row windows, operand passes)")) return rc;
   T* out = static_cast<T*>(dst);
