@@ -249,27 +249,19 @@ static int static_scratch(void** out) {
 
 using namespace flhip;
 
+// bytes of workspace of the filter gradient: the largest of its plans, so any kernel can run; one_row: with the one-row windows' kernels
+static size_t filter_ws(const ConvGeom& g, int dtype, bool one_row) {
+  size_t a = std::max(mfma_conv_bwd_filter_ws(g, dtype), mfma_slab_wgrad_ws(g, dtype));
+  if (is_lo16(dtype))
+    a = std::max({a, mfma_wgrad16_ws(g), mfma_wgrad_dma16_ws(g), mfma_pointwise16_wgrad_ws(g), mfma_first16_wgrad_ws(g)});
+  a = std::max(a, mfma_pointwise_wgrad_ws(g));
+  return one_row ? std::max(a, mfma_tap1d_wgrad_ws(g, dtype)) : a;
+}
+
 extern "C" size_t flhip_conv2d_workspace_bytes(const flhip_conv_desc* d, int pass) {
   ConvGeom g;
   if (make_geom(d, &g) != FLHIP_OK) return 0;
-  if (pass == FLHIP_CONV_BWD_FILTER) {
-    // the larger of the two filter-gradient plans, so either kernel can run
-    size_t a = mfma_conv_bwd_filter_ws(g, d->dtype);
-    const size_t b = mfma_slab_wgrad_ws(g, d->dtype);
-    size_t c = is_lo16(d->dtype) ? mfma_wgrad16_ws(g) : 0;
-    const size_t c2 = is_lo16(d->dtype) ? mfma_wgrad_dma16_ws(g) : 0;
-    if (c2 > c) c = c2;
-    const size_t e = mfma_pointwise_wgrad_ws(g);
-    const size_t f = is_lo16(d->dtype) ? mfma_pointwise16_wgrad_ws(g) : 0;
-    const size_t h = is_lo16(d->dtype) ? mfma_first16_wgrad_ws(g) : 0;
-    const size_t t1 = mfma_tap1d_wgrad_ws(g, d->dtype);
-    if (h > a) a = h;
-    if (t1 > a) a = t1;
-    if (b > a) a = b;
-    if (e > a) a = e;
-    if (f > a) a = f;
-    return c > a ? c : a;
-  }
+  if (pass == FLHIP_CONV_BWD_FILTER) return filter_ws(g, d->dtype, true);
   // forward / backward-data: the kernels for windows with several taps read reordered
   // weights when the caller brings room for them (they run without it, slower)
   // (bf16: strided 1x1 windows gather the input's lattice points / spread a compact gradient)
@@ -486,7 +478,7 @@ static int bwd_filter_direct(const flhip_conv_desc* d, const ConvGeom& g, const 
 }
 
 static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* dy, float* dw, float* db, void* ws,
-                           size_t ws_bytes, int plan, void* stream) {
+                           size_t ws_bytes, int plan, void* stream, bool one_row = true) {
   FLHIP_REQUIRE(d && dy, "conv2d_bwd_filter: null argument");
   FLHIP_REQUIRE(dw || db, "conv2d_bwd_filter: nothing to compute");
   FLHIP_REQUIRE(!dw || x, "conv2d_bwd_filter: filter gradient needs the input");
@@ -516,12 +508,12 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
     return r < 0 ? FLHIP_DECLINED : r;
   }
   if (!force_direct()) {
-    const size_t need = flhip_conv2d_workspace_bytes(d, FLHIP_CONV_BWD_FILTER);
+    const size_t need = filter_ws(g, d->dtype, one_row);
     FLHIP_REQUIRE(ws_bytes >= need && (ws || need == 0), "conv2d_bwd_filter: workspace too small");
     int r = -1;
     // (3x3 stride 1 with rows copied straight to LDS first: it also takes the 7x7 planes that would otherwise go
     // through gathered taps below)
-    if (dw && tap1d_on(d->dtype)) r = mfma_tap1d_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, s);
+    if (dw && one_row && tap1d_on(d->dtype)) r = mfma_tap1d_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, s);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_wgrad_dma16(g, x, dy, dw, db, ws, ws_bytes, s, 0, d->dtype);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
@@ -590,7 +582,10 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   ConvGeom g;
   const int rc = make_geom(d, &g);
   if (rc != FLHIP_OK) return rc;
-  const size_t need = flhip_conv2d_workspace_bytes(d, FLHIP_CONV_BWD_FILTER);
+  // (fp32 one-row windows of more than 256 channels: their own kernels' copy of the input and partial tiles, or, where those do not fit, the
+  // general kernels, which ask for less)
+  const bool one_row = !(d->dtype == FLHIP_F32 && g.C > 256) || filter_ws(g, d->dtype, true) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
+  const size_t need = filter_ws(g, d->dtype, one_row);
   if (need > (size_t)FLHIP_STATIC_SCRATCH_BYTES)
     return fail(FLHIP_INVALID_ARGUMENT,
                 "conv2d_bwd_filter_static: this geometry needs " + std::to_string(need) +
@@ -602,5 +597,5 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   if (rs != FLHIP_OK) return rs;
   // same plan as the workspace entry point given exactly `need` bytes: every partial
   // the reduction reads is written by this call first, so nothing has to be cleared
-  return flhip_conv2d_bwd_filter(d, x, dy, dw, db, ptr, need, stream);
+  return bwd_filter_impl(d, x, dy, dw, db, ptr, need, -1, stream, one_row);
 }

@@ -791,6 +791,30 @@ def test_fp32_1x1_windows_in_three_parts(xs, k, stride, special):
             assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24, name
 
 
+@pytest.mark.parametrize("xs,k,kw,dtype", [((2, 512, 17, 17), 250, 22, torch.float32), ((4, 512, 14, 14), 250, 17, torch.float32)])
+def test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dtype):
+    """fp32 one-row windows of more than 256 channels, whose own kernels ask for more than the static buffer holds, run on the general
+    ones; against float64, allowed is twice sqrt(n) units of 2^-24."""
+    import ctypes as C
+    import torch.nn.functional as F
+    from flashlight_amd import capi, ops
+    g = torch.Generator(device="cuda").manual_seed(kw)
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    to = xs[3] + 2 * (kw // 2) - kw + 1
+    dy = torch.randn(xs[0], k, xs[2], to, generator=g, device="cuda").to(dtype)
+    cd = capi.ConvDesc(*xs, k, 1, kw, 1, 1, 0, kw // 2, 1, 1, 1, ops._dtype_tag(x))
+    assert capi.lib().flhip_conv2d_workspace_bytes(C.byref(cd), capi.CONV_BWD_FILTER) > capi.STATIC_SCRATCH_BYTES
+    dw = torch.empty(k, xs[1], 1, kw, device="cuda")
+    ops.conv2d_backward_filter_bias_static(dy, x, dw, None, px=kw // 2)
+    want = torch.zeros(k, xs[1], kw, dtype=torch.float64, device="cuda")
+    xp = F.pad(x.double(), (kw // 2, kw // 2))
+    d2 = dy.double().transpose(0, 1).reshape(k, -1)
+    for j in range(kw):
+        want[:, :, j] = d2 @ xp[..., j:j + to].transpose(0, 1).reshape(xs[1], -1).t().contiguous()
+    n = d2.shape[1]
+    assert float((dw.double().view(k, xs[1], kw) - want).norm() / want.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
