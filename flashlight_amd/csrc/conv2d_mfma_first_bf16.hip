@@ -212,8 +212,10 @@ first16_conv_kernel(First16Params p, const bf16_t* __restrict__ src, const bf16_
 // part of the 64 x 192 tile in registers over all its bands; the partial tiles are added in a
 // fixed order by first16_wgrad_reduce.
 constexpr int FW_RB = 4;            // result rows per band
-constexpr int FW_CP = 232;          // elements per row copy (two copies per row)
-constexpr int FW_DP = 120;          // dy row pitch (elements)
+// elements per row copy (two copies per row) and dy row pitch, for results of up to 112 positions a row and for up to 128 (256 columns of the
+// image: 64 images of 3 channels 599 us on the general kernel -> 75, one image 53 -> 17)
+constexpr int fw_cp(bool wide) { return wide ? 264 : 232; }
+constexpr int fw_dp(bool wide) { return wide ? 136 : 120; }
 constexpr int FW_NJ = 192;          // columns of the tile
 
 struct First16WgradParams {
@@ -227,10 +229,11 @@ struct First16WgradParams {
 
 // KS = steps of 16 positions per result row when known at compile time (the loop is then
 // unrolled and its fragment reads run ahead of the matrix instructions), 0 = any
-template <typename E, int KS>
+template <typename E, int KS, bool WIDE>
 __global__ void __launch_bounds__(256, 2)
 first16_wgrad_kernel(First16WgradParams p, const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy,
                      float* __restrict__ partial) {
+  constexpr int FW_CP = fw_cp(WIDE), FW_DP = fw_dp(WIDE);
   extern __shared__ uint16_t lds_first[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -305,6 +308,10 @@ first16_wgrad_kernel(First16WgradParams p, const bf16_t* __restrict__ x, const b
   const int xcp = tid >= xcdw ? 1 : 0;
   const int xsd = tid - xcp * xcdw + xcp - shd;        // source dword of this thread's dword of a row
   const bool xcol_ok = tid < 2 * xcdw && (unsigned)xsd < (unsigned)hw;
+  // (WIDE: the second copy's last dwords, past the 256 threads, go to the first ones as well)
+  constexpr int xmore = 2 * xcdw > 256 ? 2 * xcdw - 256 : 0;
+  const int ysd = tid + 256 - xcdw + 1 - shd;
+  const bool ycol_ok = tid < xmore && (unsigned)ysd < (unsigned)hw;
 
   for (int band = blockIdx.x; band < p.total_bands; band += gridDim.x) {
     int bi;
@@ -339,6 +346,19 @@ first16_wgrad_kernel(First16WgradParams p, const bf16_t* __restrict__ x, const b
 #pragma unroll
         for (int k = 0; k < 8; ++k)
           if (tid < 2 * xcdw && rl0 + k < p.NR) xs32[(c * p.NR + rl0 + k) * (2 * xcdw) + tid] = v[k];
+        if constexpr (xmore > 0) {
+          if (tid < xmore) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const int ih = oh0 * p.sy - p.py + rl0 + k;
+              v[k] = (ycol_ok && rl0 + k < p.NR && (unsigned)ih < (unsigned)p.H)
+                         ? x32[(((size_t)n * p.C + c) * p.H + ih) * hw + ysd] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (rl0 + k < p.NR) xs32[(c * p.NR + rl0 + k) * (2 * xcdw) + 256 + tid] = v[k];
+          }
+        }
       }
     store_dy(0);
     __syncthreads();
@@ -418,7 +438,8 @@ bool first16_wgrad_plan(const ConvGeom& g, First16WgradParams* p, int* nwg, size
   const int sh = g.px & 1;
   if (g.KW + sh > 8 || g.C > 4 || g.KH > 15) return false;
   if (g.C * g.KH + 1 > FW_NJ / 8) return false;
-  if (g.OW % 16 != 0 || g.OW > 112 || g.K % 32 != 0) return false;
+  if (g.OW % 16 != 0 || g.OW > 128 || g.K % 32 != 0) return false;
+  if (g.OW > 112 && g.K > 64) return false;      // (its partial tiles would ask for more room than the general kernel's)
   if ((long long)g.N * g.K * g.OH * g.OW * 2 >= (1ll << 31) || (long long)g.N * g.C * g.H * g.W * 2 >= (1ll << 31)) return false;
   p->N = g.N; p->C = g.C; p->H = g.H; p->W = g.W; p->K = g.K; p->OH = g.OH; p->OW = g.OW;
   p->KH = g.KH; p->KW = g.KW; p->sy = g.sy; p->py = g.py; p->px = g.px;
@@ -428,7 +449,8 @@ bool first16_wgrad_plan(const ConvGeom& g, First16WgradParams* p, int* nwg, size
   p->total_bands = g.N * p->bands_per_image;
   p->mtiles = (g.K + 63) / 64;
   *nwg = std::min(p->total_bands, 2 * mfma_num_cus());
-  *shmem = ((size_t)(g.C * p->NR + 2) * 2 * FW_CP + 2 * 64 * FW_DP) * sizeof(uint16_t);
+  const bool wide = g.OW > 112;
+  *shmem = ((size_t)(g.C * p->NR + 2) * 2 * fw_cp(wide) + 2 * 64 * fw_dp(wide)) * sizeof(uint16_t);
   return *shmem <= 80 * 1024;
 }
 
@@ -455,7 +477,7 @@ int mfma_first16_wgrad(const ConvGeom& g, const void* x, const void* dy, float* 
   float* partial = static_cast<float*>(ws);
   const int rc = by_lo16(dtype, [&](auto* e_) {
     using E = FLHIP_T_OF(e_);
-    auto kernel = g.OW == 112 ? first16_wgrad_kernel<E, 7> : first16_wgrad_kernel<E, 0>;
+    auto kernel = g.OW == 112 ? first16_wgrad_kernel<E, 7, false> : g.OW == 128 ? first16_wgrad_kernel<E, 8, true> : first16_wgrad_kernel<E, 0, false>;
     if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), shmem)) return -1;
     hipLaunchKernelGGL(kernel, dim3((unsigned)nwg, (unsigned)p.mtiles), dim3(256), shmem, s, p,
                        static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(dy), partial);

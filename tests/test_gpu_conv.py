@@ -815,6 +815,27 @@ def test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dt
     assert float((dw.double().view(k, xs[1], kw) - want).norm() / want.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,win,pad", [((2, 3, 256, 256), 64, 7, 3), ((5, 4, 41, 256), 32, 5, 2), ((3, 1, 30, 258), 64, 7, 2), ((40, 3, 64, 256), 64, 7, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_first_layer_filter_gradient_over_rows_of_128(xs, k, win, pad, dtype):
+    """First layers whose results are 128 positions wide, filter and bias gradient, against float64: fp32 sums of n exact products differ by
+    about sqrt(n) units of 2^-24 in the 2-norm, allowed are twice that."""
+    import torch.nn.functional as F
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k + win)
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    oh, ow = (xs[2] + 2 * pad - win) // 2 + 1, (xs[3] + 2 * pad - win) // 2 + 1
+    assert ow == 128
+    dy = torch.randn(xs[0], k, oh, ow, generator=g, device="cuda").to(dtype)
+    dw, db = ops.conv2d_backward_filter_bias(dy, x, (k, xs[1], win, win), True, sx=2, sy=2, px=pad, py=pad)
+    cols = F.unfold(x.double(), (win, win), padding=pad, stride=2)
+    d2 = dy.double().flatten(2).transpose(0, 1).reshape(k, -1)
+    want = d2 @ cols.permute(0, 2, 1).reshape(-1, cols.shape[1]).contiguous()
+    n = d2.shape[1]
+    for got, ref in ((dw.double().view(k, -1), want), (db.double(), d2.sum(1))):
+        assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
