@@ -1019,7 +1019,7 @@ static bool thin_tn_on_gemm32(int M, int N, int K, bool slices) {
 extern "C" size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || (trans_a && trans_b)) return 0;
   if (trans_b || dtype != FLHIP_F32 || options().matmul_valu) return flhip_matmul_workspace_bytes(M, N, K, trans_a, trans_b, dtype);
-  const size_t need = gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K);
+  const size_t need = gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K, !trans_a);
   return !trans_a && N <= 128 && !thin_on_gemm32(M, N, K, need > 0) ? 0 : need;
 }
 
@@ -1033,9 +1033,15 @@ extern "C" int flhip_matmul(const void* A, const void* B, void* C, int32_t M, in
   return flhip_matmul_ws(A, B, C, M, N, K, trans_a, trans_b, bias_rows, dtype, nullptr, 0, stream);
 }
 
+// (A * B is the forward product of fl::linear)
 extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
                                int trans_a, int trans_b, const float* bias_rows, int dtype, void* ws,
                                size_t ws_bytes, void* stream) {
+  return matmul(A, B, C, M, N, K, trans_a, trans_b, bias_rows, dtype, ws, ws_bytes, stream, !trans_a && !trans_b);
+}
+
+int flhip::matmul(const void* A, const void* B, void* C, int M, int N, int K, int trans_a, int trans_b, const float* bias_rows, int dtype,
+                  void* ws, size_t ws_bytes, void* stream, bool fp32_sums) {
   FLHIP_REQUIRE(A && B && C, "matmul: null argument");
   FLHIP_REQUIRE(M > 0 && N > 0 && K > 0, "matmul: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "matmul: unknown dtype");
@@ -1046,7 +1052,7 @@ extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M,
   if (dtype == FLHIP_F32 && !(trans_a && trans_b) && !options().matmul_valu && options().matmul_planes < 0) {
     const int rc = gemm32(trans_a ? 1 : trans_b ? 2 : 0, static_cast<const float*>(A), static_cast<const float*>(B),
                           static_cast<float*>(C), M, N, K, bias_rows, ws, ws_bytes, as_stream(stream), nullptr,
-                          !thin ? nullptr : trans_a ? thin_tn_on_gemm32 : thin_on_gemm32);
+                          !thin ? nullptr : trans_a ? thin_tn_on_gemm32 : thin_on_gemm32, fp32_sums);
     if (rc >= 0) return rc;
   }
   // the other thin products: the kernels made for them

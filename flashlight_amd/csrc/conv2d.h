@@ -79,10 +79,20 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
 size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K);
 // the three products in fp32 (gemm_f32.hip), + bias[row] + addend (C's layout, may be C), their contraction cut into slices
 // where gemm32_ws_bytes() of workspace are there; -1 where rows are not whole 16-byte pieces or a tensor is too large, and,
-// with `take`, where the workspace is short or take(M, N, K, more than one slice) is false
-size_t gemm32_ws_bytes(int mode, int M, int N, int K);
+// with `take`, where the workspace is short or take(M, N, K, more than one slice) is false.
+// fp32_sums (modes 0 and 1): on the fp32 instruction whatever the size, none in three bf16 parts.  For the products in front of a ReLU
+// whose choices the same step's gradients hang on (fl::linear's forward product, the input product of ReLU recurrent layers): the parts'
+// sums are nearer to 64 bits, but not the same ones, and an input within their rounding of zero then falls on the other side, with a
+// whole row of gradients.  In parts, against these: linear of 1200 to 2000 features over 3000 to 6000 frames, ReLU, layer norm,
+// classifier, gradients up to 1e-3 in the 2-norm and 9e-2 of their rms at most (without such a choice 1e-6 and 1e-5); a ReLU layer of
+// 512 units over 200 steps of 64 columns 1e-3 and 0.2.
+size_t gemm32_ws_bytes(int mode, int M, int N, int K, bool fp32_sums = false);
 int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int K, const float* bias, void* ws,
-           size_t ws_bytes, hipStream_t s, const float* addend = nullptr, bool (*take)(int, int, int, bool) = nullptr);
+           size_t ws_bytes, hipStream_t s, const float* addend = nullptr, bool (*take)(int, int, int, bool) = nullptr,
+           bool fp32_sums = false);
+// flhip_matmul_ws; fp32_sums: fp32 products as above
+int matmul(const void* A, const void* B, void* C, int M, int N, int K, int trans_a, int trans_b, const float* bias_rows, int dtype, void* ws,
+           size_t ws_bytes, void* stream, bool fp32_sums);
 // column-major C = A * B^T on a kernel of its own (both operands contiguous along the
 // surviving dimension); slices > 1 (f32): partial products M * N floats apart
 int gemm_nt(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int slices, hipStream_t s);

@@ -148,14 +148,19 @@ static bool tap1d_on(int dtype) {
   return dtype == FLHIP_F32 || ((dtype == FLHIP_BF16 || dtype == FLHIP_F16) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT));
 }
 
-// Windows over stacked planes.  fp32: by the estimate of conv2d_mfma_tap_split.hip.  16-bit storage: 3x3 windows over planes of at
-// most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.  Measured (batch 64 / 32, forward): 7 x 7 x 512
-// 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0 against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5
-// against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts both rules.
+// Windows over stacked planes.  fp32: by the estimate of conv2d_mfma_tap_split.hip, but the forward pass of windows larger than 3x3
+// stays on the fp32 instruction: they are the layers of small convnets, whose ReLU and pool decide on its last bits, and the same
+// step's gradients hang on those.  (With the parts' sums, nearer to 64 bits as they are, the gradients of a step over 300 to 512 images of
+// 28 x 28 through two 5x5 layers were up to 3e-3 apart from these in the 2-norm, else 1e-6; the second layer over 64 / 512 images 38 / 145 us,
+// in parts 18 / 65.)
+// 16-bit storage: 3x3 windows over planes of at most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.
+// Measured (batch 64 / 32, forward): 7 x 7 x 512 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0
+// against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5 against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts both
+// rules.
 static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
   if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
   if (options().tap2d_all) return true;
-  if (dtype == FLHIP_F32) return mfma_tap2d_split_pays(g, bwd);
+  if (dtype == FLHIP_F32) return (bwd || g.KH * g.KW <= 9) && mfma_tap2d_split_pays(g, bwd);
   return g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
 }
 

@@ -3,6 +3,7 @@
 //   mode 0  C [M x N] = A [M x K]   * B [K x N]
 //   mode 1  C [M x N] = A [K x M]^T * B [K x N]
 //   mode 2  C [M x N] = A [M x K]   * B [N x K]^T
+// (Products whose fp32 sums have to stay, gemm32's fp32_sums, run on gemm_f32.hip whatever their size: 2000 x 4000 x 2000 forward 232 us, here 160.)
 //
 // A workgroup (4 waves, 2 x 2) owns a TM x TN tile of C, a wave RT x CT instruction tiles of 32 x 32 with two accumulators each.
 // The contraction runs in stages of 16.  A stage's values pass through registers, where they are taken apart: loaded two stages

@@ -23,10 +23,6 @@
 #include "conv2d.h"
 #include "conv2d_mfma.h"
 
-extern "C" int flhip_matmul(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K,
-                            int trans_a, int trans_b, const float* bias_rows, int dtype, void* stream);
-extern "C" int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N, int32_t K, int trans_a,
-                               int trans_b, const float* bias_rows, int dtype, void* ws, size_t ws_bytes, void* stream);
 extern "C" int flhip_sum_columns_ws(const void* x, float* out, int32_t rows, int32_t cols, int dtype, void* ws,
                                     size_t ws_bytes, void* stream);
 extern "C" size_t flhip_sum_columns_workspace_bytes(int32_t rows, int32_t cols, int dtype);
@@ -151,7 +147,7 @@ struct Scratch {
 };
 
 int mm(const float* A, const float* B, float* C, size_t M, size_t N, size_t K, int ta, int tb,
-       const float* bias, hipStream_t s, Scratch w = Scratch()) {
+       const float* bias, hipStream_t s, Scratch w = Scratch(), bool fp32_sums = false) {
   // A thin product A * B that gemm_f32.hip cuts into slices is faster there from the shortest such contraction on (512 x 64 x 512 7.4 /
   // 8.5 us).  flhip_matmul_ws leaves it to the other kernel up to a contraction of 704 for the second launch's host time,
   // which a layer's queued launches hide: GRU of 320 units, 3 layers, backward over 13 steps, 7 columns 321 -> 272 us.
@@ -160,7 +156,7 @@ int mm(const float* A, const float* B, float* C, size_t M, size_t N, size_t K, i
                           [](int, int, int, bool slices) { return slices; });
     if (rc >= 0) return rc;
   }
-  return flhip_matmul_ws(A, B, C, (int32_t)M, (int32_t)N, (int32_t)K, ta, tb, bias, FLHIP_F32, w.p, w.bytes, s);
+  return matmul(A, B, C, (int)M, (int)N, (int)K, ta, tb, bias, FLHIP_F32, w.p, w.bytes, s, fp32_sums);
 }
 
 // C = op(A) B in `*slices` partial products at C + k*M*N (see step_slices)
@@ -215,7 +211,7 @@ Scratch scratch_of(const RnnGeom& g, float* ws) {
   const int TB = g.T * g.B, GH = (int)g.GH;
   size_t n = flhip_sum_columns_workspace_bytes(GH, TB, FLHIP_F32);
   for (int in : {g.I, g.D * g.H}) {
-    n = std::max(n, gemm32_ws_bytes(1, GH, TB, in));
+    n = std::max(n, gemm32_ws_bytes(1, GH, TB, in, g.mode == RNN_RELU));
     n = std::max(n, gemm32_ws_bytes(0, in, TB, GH));
     n = std::max(n, gemm32_ws_bytes(2, in, GH, TB));
   }
@@ -1138,7 +1134,7 @@ int forward_pl(const RnnGeom& g, int pl, const float* in, size_t inl, const floa
   ip.d[0] = {hx ? hx + (size_t)pl * g.BH : nullptr, cx ? cx + (size_t)pl * g.BH : nullptr, w + o.bW, w + o.bR, HP, CP, bsum};
   launch_init(ip, 1, s);
   // XP [GH x TB] = W [GH x in] (row-major = a column-major in x GH matrix, transposed) * IN [in x TB]
-  if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws))) return rc;
+  if (const int rc = mm(w + o.W, in, XP, g.GH, TB, inl, 1, 0, bsum, s, scratch_of(g, ws), MODE == RNN_RELU)) return rc;
   for (int st = 0; st < g.T; ++st) {
     const int t = dir ? g.T - 1 - st : st;
     int nrp = 1;
@@ -1341,7 +1337,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
   launch_init(ip, g.D, s);
   for (int dir = 0; dir < g.D; ++dir)
     if (const int rc = mm(w + offsets(g, l * g.D + dir).W, in, const_cast<float*>(p.d[dir].xp), g.GH, TB, inl, 1, 0,
-                          ip.d[dir].bsum, s, scratch_of(g, ws)))
+                          ip.d[dir].bsum, s, scratch_of(g, ws), MODE == RNN_RELU))
       return rc;
   if (seq) {
     const int rc = seq_fwd<MODE>(g, p, s);

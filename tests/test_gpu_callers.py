@@ -292,6 +292,23 @@ def test_matmul_fp32_in_three_parts_keeps_what_bf16_cannot_hold(mode):
         assert rel_l2(got[rows][ok], ref[rows][ok]) <= 2 * np.sqrt(K) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("M,N,K", [(1200, 3001, 1200), (2700, 1092, 20), (512, 2544, 1120), (1024, 300, 3136)])
+def test_matmul_forward_keeps_the_sums_of_the_fp32_instruction(M, N, K):
+    """fl::linear's forward product, in front of a ReLU on whose choices the same step's gradients hang: the bits of the fp32
+    instruction, also where the backward products run in three bf16 parts."""
+    from flashlight_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w, b = (torch.randn(*s, generator=g, device="cuda") for s in ((N, K), (K, M), (M,)))
+    y = ops.linear(x, w, b)
+    capi.set_option("MATMUL_FP32_CORES", "1")
+    try:
+        want = ops.linear(x, w, b)
+    finally:
+        capi.set_option("MATMUL_FP32_CORES", None)
+    assert torch.equal(y, want)
+    assert rel_l2(host(y), host(x).astype(np.float64) @ host(w).astype(np.float64) + host(b)) <= 2 * np.sqrt(K) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (10, 64, 1024), (17, 3, 255), (33, 127, 257), (63, 128, 700), (65, 9, 300)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_matmul_few_rows(M, N, K, dtype):

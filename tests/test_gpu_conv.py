@@ -702,6 +702,22 @@ def test_fp32_windows_in_three_parts_keep_what_bf16_cannot_hold(xs, ws, stride):
         assert float(((got[ok] - ref[ok]).abs() / ref[ok].abs()).max()) <= 1e-5
 
 
+@pytest.mark.parametrize("n", [33, 300])
+def test_forward_of_large_windows_keeps_the_sums_of_the_fp32_instruction(n):
+    """Windows larger than 3x3 in front of a ReLU and a pool on whose choices the same step's gradients hang: the forward pass has the bits of
+    the kernels on the fp32 instruction."""
+    from flashlight_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w, b = (torch.randn(*s, generator=g, device="cuda") for s in ((n, 32, 14, 14), (64, 32, 5, 5), (64,)))
+    y = fa.conv2d(x, w, b, px=2, py=2)
+    capi.set_option("CONV_SKIP", "tap2d")
+    try:
+        want = fa.conv2d(x, w, b, px=2, py=2)
+    finally:
+        capi.set_option("CONV_SKIP", None)
+    assert torch.equal(y, want)
+
+
 @pytest.mark.parametrize("xs,k,kw,stride", [
     ((1, 16, 1, 16), 32, 6, 1),          # one step of one range; half of a tile's filters
     ((2, 33, 2, 47), 33, 7, 2),          # the other half with one filter, rows of an image, a last step of 8 positions

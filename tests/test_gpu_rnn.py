@@ -64,6 +64,23 @@ def test_rnn_forward_backward(mode, I, H, L, bidir, T, B, states):
         assert rel_l2(host(dcx), rdcx) <= 2e-4
 
 
+def test_relu_layers_keep_the_sums_of_the_fp32_instruction():
+    """The input products of ReLU layers, on whose choices the same step's gradients hang: the bits of the fp32 instruction in every layer,
+    also where the other modes' run in three bf16 parts."""
+    I, H, L, T, B = 512, 512, 2, 200, 64
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(T, B, I, generator=g, device="cuda")
+    for mode, same in ((flref.RNN_RELU, True), (flref.RNN_TANH, False)):
+        w = torch.randn(ops.rnn_param_count(I, H, L, mode, False), generator=g, device="cuda") / H ** 0.5
+        y = ops.rnn(x, None, None, w, H, L, mode, False)[0]
+        capi.set_option("MATMUL_FP32_CORES", "1")
+        try:
+            want = ops.rnn(x, None, None, w, H, L, mode, False)[0]
+        finally:
+            capi.set_option("MATMUL_FP32_CORES", None)
+        assert torch.equal(y, want) == same
+
+
 @pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
     # whole sequences in one launch: hidden sizes that are multiples of 4 up to 1024.  4, 8 and 16 units per workgroup,
     # a last workgroup with units to spare, a last contraction chunk with columns to spare, more waves than chunks
