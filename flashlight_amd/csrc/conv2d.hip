@@ -600,7 +600,7 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   void* ptr = nullptr;
   const int rs = static_scratch(&ptr);
   if (rs != FLHIP_OK) return rs;
-  // same plan as the workspace entry point given exactly `need` bytes: every partial
-  // the reduction reads is written by this call first, so nothing has to be cleared
+  // the same plan as the workspace entry point's given exactly `need` bytes (but for the windows above that do not fit): every
+  // partial the reduction reads is written by this call first, so nothing has to be cleared
   return bwd_filter_impl(d, x, dy, dw, db, ptr, need, -1, stream, one_row);
 }

@@ -212,6 +212,8 @@ int flhip_conv2d_bwd_filter_gathered(const flhip_conv_desc* d, const void* gathe
  * hipMalloc / hipFree or other allocating call is made.  Geometries whose
  * flhip_conv2d_workspace_bytes(d, FLHIP_CONV_BWD_FILTER) exceeds that size are refused
  * with FLHIP_INVALID_ARGUMENT.  Results are bit-identical to flhip_conv2d_bwd_filter.
+ * One exception to both: fp32 windows of one row over more than 256 channels that exceed it run on the
+ * general kernels, which need less; their sums are in another order than flhip_conv2d_bwd_filter's.
  * The device of `stream` must be the current device.  All calls on one GPU share the
  * buffer: calls that overlap in time on one GPU (different streams, or threads) race. */
 #define FLHIP_STATIC_SCRATCH_BYTES (40u << 20)

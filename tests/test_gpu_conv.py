@@ -831,6 +831,30 @@ def test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dt
     assert float((dw.double().view(k, xs[1], kw) - want).norm() / want.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,kw,stride", [((5, 88, 1, 2139), 188, 12, 2), ((9, 39, 1, 1911), 318, 12, 1), ((4, 250, 1, 1100), 250, 9, 1),
+                                            ((11, 80, 1, 1134), 250, 15, 1), ((8, 80, 1, 1529), 250, 11, 2)])
+def test_static_filter_gradient_of_long_one_row_windows(xs, k, kw, stride):
+    """fp32 one-row windows whose rows and partial tiles fit the static buffer when the partial tiles are no more than it takes to fill the
+    chip: accepted, the bits of the workspace entry point, and against float64 within twice sqrt(n) units of 2^-24."""
+    import torch.nn.functional as F
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(kw)
+    pad = kw // 2
+    x = torch.randn(*xs, generator=g, device="cuda")
+    to = (xs[3] + 2 * pad - kw) // stride + 1
+    dy = torch.randn(xs[0], k, 1, to, generator=g, device="cuda")
+    dw, db = torch.empty(k, xs[1], 1, kw, device="cuda"), torch.empty(k, device="cuda")
+    ops.conv2d_backward_filter_bias_static(dy, x, dw, db, sx=stride, px=pad)
+    dw2, db2 = ops.conv2d_backward_filter_bias(dy, x, tuple(dw.shape), True, sx=stride, px=pad)
+    assert torch.equal(dw, dw2) and torch.equal(db, db2)
+    xp = F.pad(x.double(), (pad, pad))
+    d2 = dy.double().transpose(0, 1).reshape(k, -1)
+    want = torch.stack([d2 @ xp[..., j:j + stride * (to - 1) + 1:stride].transpose(0, 1).reshape(xs[1], -1).t().contiguous() for j in range(kw)], -1)
+    n = d2.shape[1]
+    for got, ref in ((dw.double().view(want.shape), want), (db.double(), d2.sum(1))):
+        assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("xs,k,win,pad", [((2, 3, 256, 256), 64, 7, 3), ((5, 4, 41, 256), 32, 5, 2), ((3, 1, 30, 258), 64, 7, 2), ((40, 3, 64, 256), 64, 7, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_first_layer_filter_gradient_over_rows_of_128(xs, k, win, pad, dtype):
