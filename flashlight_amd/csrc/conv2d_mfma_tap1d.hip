@@ -1155,46 +1155,50 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
     return pl->lds_bytes <= (size_t)most;
   };
   if (esz == 4) {
-    // No more partial tiles than the kernel on the fp32 instruction asked for, whose slab had 9 cells a row and 150 KB: ranges for about
-    // `want` workgroups and tile, or as many as it takes for their slab to fit, rounded down to whole ranges per workgroup.  (Shorter ranges
-    // at that many per workgroup made up to twice as many tiles, and geometries that fit the static buffer no longer did: 250 -> 250
-    // channels over 4 x 1100 frames, 9 taps 31.5 -> 42.3 MB; 80 -> 250 over 11 x 1134, 15 taps 39.4 -> 56.7.)
+    // fp32 is bound by the matrix pipe: enough workgroups for the chip (a tile is two of them, and two share a compute unit), rather
+    // with a last round that is half full than of twice the length ...
     const int want = (cus + tiles - 1) / tiles;
-    int most_splits = 0;
-    for (int tsplit = std::max(1, (want + p.rows - 1) / p.rows); !most_splits; ++tsplit) {
+    auto fill = [&](auto fits) {
+      for (int tsplit = std::max(1, (want + p.rows - 1) / p.rows); !fits(tsplit); ++tsplit)
+        if (p.TL <= 16) return 0;
+      p.upw = std::max(1, p.units / want);
+      return (p.units + p.upw - 1) / p.upw;
+    };
+    // ... but no more partial tiles than with a slab of 9 cells a row and 150 KB, the fp32 instruction's kernel: the parts' smaller one makes
+    // ranges shorter, as many of them per workgroup then up to twice the tiles, and geometries that fit the static buffer no longer did
+    // (250 -> 250 channels over 4 x 1100 frames, 9 taps 31.5 -> 42.3 MB; 80 -> 250 over 11 x 1134, 15 taps 39.4 -> 56.7).
+    const int most_splits = fill([&](int tsplit) {
       split(tsplit);
-      if (((long long)p.SRW * 9 + 63) / 64 * 1024 <= 150 * 1024) {
-        const int upw = std::max(1, p.units / want);
-        most_splits = (p.units + upw - 1) / upw;
-      } else if (p.TL <= 16) {
-        return false;
-      }
-    }
-    // Under that bound the range's length and ranges per workgroup with the least estimated time: 1.8 us and 0.021 per four taps
-    // and position for a range, 0.7 of it where a workgroup has its compute unit for itself (a tile is two workgroups, and two share a
-    // unit), rounds of 512 workgroups, 0.01 per four taps and tile and 0.11 for each set of partial tiles.  Fitted to 5900 times of 220
-    // random geometries (1 to 24 x 100 to 2200 frames, 16 to 320 channels, 7 to 21 taps); 150 others take 0.85 of their time
-    // with ranges that fill the chip (3 x 128 -> 250 channels, 173 frames, 12 taps 34 -> 21 us; 8 x 250 -> 250, 1248 frames, 21 taps
-    // 101 -> 101), the slowest 1.04.
-    double best = 1e30;
-    int best_split = 0, best_upw = 0;
-    const double set = 0.01 * TQ * tiles + 0.11;
-    for (int tsplit = 1;; tsplit += std::max(1, tsplit / 4)) {
-      if (split(tsplit)) {
-        const double each = 1.8 + 0.021 * TQ * p.TL;
-        const int even = (int)(p.units / std::max(1.0, std::sqrt(p.units * set / each)));
-        for (int n : {most_splits, cus / tiles, cus / tiles / 2, even}) {
-          const int upw = (p.units - 1) / std::max(1, std::min(n, most_splits)) + 1, ns = (p.units + upw - 1) / upw;
-          const int wgs = 2 * tiles * ns, rounds = (wgs + 2 * cus - 1) / (2 * cus);
-          const double cost = rounds * upw * each * (wgs <= cus ? 0.7 : 1.0) + ns * set;
-          if (cost < best) { best = cost; best_split = tsplit; best_upw = upw; }
+      return ((long long)p.SRW * 9 + 63) / 64 * 1024 <= 150 * 1024;
+    });
+    const int splits = fill(split);
+    if (!most_splits || !splits) return false;
+    // Where it would be more, the range's length and ranges per workgroup with the least estimated time under that bound: 1.8 us and
+    // 0.021 per four taps and position for a range, 0.7 of it where a workgroup has its compute unit for itself, rounds of 512
+    // workgroups, 0.01 per four taps and tile and 0.11 for each set of partial tiles.  Fitted to 5900 times of 220 random geometries (1 to 24 x
+    // 100 to 2200 frames, 16 to 320 channels, 7 to 21 taps); of 150 others those that the bound reaches take 0.86 to 1.00 of their time
+    // without it (17 x 39 -> 250 channels, 1993 frames, 15 taps 120 -> 104 us; 2 x 250 -> 256, 1624 frames, 21 taps 91 -> 81).
+    if (splits > most_splits) {
+      double best = 1e30;
+      int best_split = 0, best_upw = 0;
+      const double set = 0.01 * TQ * tiles + 0.11;
+      for (int tsplit = 1;; tsplit += std::max(1, tsplit / 4)) {
+        if (split(tsplit)) {
+          const double each = 1.8 + 0.021 * TQ * p.TL;
+          const int even = (int)(p.units / std::max(1.0, std::sqrt(p.units * set / each)));
+          for (int n : {most_splits, cus / tiles, cus / tiles / 2, even}) {
+            const int upw = (p.units - 1) / std::max(1, std::min(n, most_splits)) + 1, ns = (p.units + upw - 1) / upw;
+            const int wgs = 2 * tiles * ns, rounds = (wgs + 2 * cus - 1) / (2 * cus);
+            const double cost = rounds * upw * each * (wgs <= cus ? 0.7 : 1.0) + ns * set;
+            if (cost < best) { best = cost; best_split = tsplit; best_upw = upw; }
+          }
         }
+        if (p.TL <= 16) break;
       }
-      if (p.TL <= 16) break;
+      if (!best_split) return false;
+      split(best_split);
+      p.upw = best_upw;
     }
-    if (!best_split) return false;
-    split(best_split);
-    p.upw = best_upw;
   } else {
     // 16-bit storage is bound by what surrounds the products.  The length of a range and the ranges per workgroup with the least
     // estimated time: a workgroup's ranges follow each other, about 1 us each and 0.012 + 0.002 per four taps for a position; its partial
