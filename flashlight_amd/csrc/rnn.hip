@@ -202,7 +202,7 @@ size_t workspace_core(const RnnGeom& g) {
 }
 // whether whole sequences may be launched: 16-byte pieces of the state, recurrent matrices in registers
 bool seq_holds(const RnnGeom& g) { return g.H % 4 == 0 && g.H <= 1024; }
-// floats of a step of the exchange, and the exchange of the call's sequence launches (behind the scratch; the layers use it in turn)
+// floats of a step of the exchange
 size_t seq_row(const RnnGeom& g, size_t K) { return (size_t)g.B * ((K + 15) & ~(size_t)15); }
 
 // whether a wait inside one of the call's sequence launches has given up (one word before the scratch)
@@ -218,15 +218,6 @@ Scratch scratch_of(const RnnGeom& g, float* ws) {
   n = std::max(n, gemm32_ws_bytes(2, g.H, GH, TB));
   return Scratch{ws + workspace_core(g), (n + 15) & ~(size_t)15};
 }
-float* seq_exchange(const RnnGeom& g, float* ws) {
-  const Scratch w = scratch_of(g, ws);
-  return static_cast<float*>(w.p) + w.bytes / sizeof(float);
-}
-size_t workspace_bytes(const RnnGeom& g) {
-  const size_t exchange = seq_holds(g) ? (size_t)g.D * g.T * seq_row(g, g.GH) : 0;
-  return (workspace_core(g) + exchange) * sizeof(float) + scratch_of(g, nullptr).bytes;
-}
-
 // the fused step kernels tile the hidden state by 16 and hold at most 64 batch columns
 bool fused_applies(const RnnGeom& g) {
   return !options().rnn_unfused && g.H % 16 == 0 && g.B <= 64;
@@ -270,8 +261,8 @@ __global__ void __launch_bounds__(256) rnn_add2_kernel(const float* a, const flo
 
 constexpr int SEQ_COLS = 16;
 constexpr int RNN_OOB = (int)0x80000000;
-// Where the values of a step are that the workgroups of a cluster hand to each other (the state, the gate gradients): a
-// buffer of its own, in chunks of 16 contraction indexes, and in a chunk in the order of the lanes that read it, [4][columns][4], so
+// Where the values of a step are that the workgroups of a cluster hand to each other (the state, the gate gradients): an exchange
+// (where it lies: seq_place), in chunks of 16 contraction indexes, and in a chunk in the order of the lanes that read it, [4][columns][4], so
 // that a wave's load is one piece of 1 KB.  Read from the rows of the reserve buffer / workspace it was 16 pieces of 64 bytes, a
 // row apart (8 KB: all in one channel of the caches): the 128 KB of a step of an LSTM of 512 units' backward pass took 10000 cycles of
 // its 13600.
@@ -1211,18 +1202,83 @@ bool seq_pays(const RnnGeom& g, bool bwd) {
 
 // ---- launching whole sequences: the hidden size a multiple of 4 (16-byte pieces of the state) and at most 1024
 // (registers), a step's gates within what a buffer load addresses (2 GiB: an LSTM of 1024 units up to 131071
-// columns), a stream that is not being captured (a cooperative launch is not recorded)
-bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
+// columns) ...
+bool seq_asked(const RnnGeom& g, bool bwd) {
   const int asked = options().rnn_sequences;
-  if (options().rnn_unfused || asked == Options::SEQ_NEVER || !seq_holds(g) ||
-      (size_t)g.B * g.GH * 4 >= ((size_t)1 << 31) || (asked == Options::SEQ_AUTO && !seq_pays(g, bwd)))
-    return false;
+  return !options().rnn_unfused && asked != Options::SEQ_NEVER && seq_holds(g) && (size_t)g.B * g.GH * 4 < ((size_t)1 << 31) &&
+         (asked != Options::SEQ_AUTO || seq_pays(g, bwd));
+}
+// ... and a stream that is not being captured (a cooperative launch is not recorded)
+bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
+  if (!seq_asked(g, bwd)) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
   return st == hipStreamCaptureStatusNone;
+}
+
+// Where the exchange of a layer's sequence launch lies in the workspace, in floats (the layers use it in turn): in what the pass leaves idle
+// while the launch runs, so that it costs nothing but for the lower ones of stacked GRU layers, which need 3 H per position and direction where 2 H to 4 H are idle
+// (3 layers of 512 units, 64 columns over 100 steps 144 -> 159 MiB).
+//   forward   behind the projections and biases: the backward pass' buffers
+//   backward  not GRU, forward direction: in place of dGR[0], which is dGW[0] there (the same values in the same order; rows of whole
+//             chunks only); else gin, tmp and the step kernels' buffers behind them (the topmost layer: gout in front of them too, it reads
+//             the caller's); else the weight gradients' scratch, or behind everything from the products' scratch on
+// (A buffer of its own in every call: LSTM of 512 units, 2 x 2 layers, 32 columns over 200 steps 324 -> 424 MiB of workspace.)
+struct SeqPlace {
+  size_t at[2];
+  size_t end;          // floats of workspace that it takes
+  bool shared;         // dGR[0] is dGW[0]
+};
+SeqPlace seq_place(const RnnGeom& g, bool bwd, bool top) {
+  const size_t TB = (size_t)g.T * g.B, core = workspace_core(g), need = (size_t)g.T * seq_row(g, bwd ? g.GH : g.H);
+  SeqPlace p{};
+  size_t from[2] = {}, to[2] = {}, behind = core;
+  if (bwd) {
+    const size_t gout = 2 * TB * g.GH, scratch = wgrad_scratch_offset(g);
+    from[0] = top ? gout : gout + TB * g.D * g.H;
+    to[0] = g.D == 1 ? scratch + wgrad_scratch(g) : scratch - 2 * TB * g.GH - 3 * g.BH;
+    from[1] = scratch;
+    to[1] = g.D == 1 ? scratch : scratch + wgrad_scratch(g);
+  } else {
+    from[0] = (size_t)g.D * (TB * g.GH + g.GH);
+    to[0] = core - 4;
+    behind += scratch_of(g, nullptr).bytes / sizeof(float);       // (the projections use the scratch after the exchange is filled)
+  }
+  for (int dir = 0; dir < g.D; ++dir) {
+    if (bwd && dir == 0 && g.mode != RNN_GRU && g.GH % 16 == 0) {
+      p.at[0] = TB * g.GH;
+      p.shared = true;
+      continue;
+    }
+    bool placed = false;
+    for (int i = 0; i < 2 && !placed; ++i) {
+      const size_t at = (from[i] + 63) & ~(size_t)63;
+      if (at + need > to[i]) continue;
+      p.at[dir] = at;
+      from[i] = at + need;
+      placed = true;
+    }
+    if (placed) continue;
+    p.at[dir] = behind;
+    behind += need;
+    p.end = behind;
+  }
+  return p;
+}
+
+// what a call cannot do without, and with what its sequence launches take where they may be launched
+size_t base_bytes(const RnnGeom& g) { return workspace_core(g) * sizeof(float) + scratch_of(g, nullptr).bytes; }
+size_t workspace_bytes(const RnnGeom& g) {
+  size_t end = 0;
+  if (seq_asked(g, false)) end = seq_place(g, false, true).end;
+  if (seq_asked(g, true)) {
+    end = std::max(end, seq_place(g, true, true).end);
+    if (g.L > 1) end = std::max(end, seq_place(g, true, false).end);
+  }
+  return std::max(base_bytes(g), end * sizeof(float));
 }
 
 std::atomic<uint64_t> g_seq_launches{0};
@@ -1314,6 +1370,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
   // the initial states and the input projections
   SeqInit ip{};
   SeqFwd p{};
+  const SeqPlace place = seq ? seq_place(g, false, true) : SeqPlace{};
   p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
   p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
   p.wait = options().rnn_wait; p.pause = seq_pause_fwd(g, seq_units(g)); p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
@@ -1328,7 +1385,7 @@ int forward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, co
     q.R = w + o.R; q.bRn = w + o.bR + 2 * g.H;
     q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
     q.out = out + (size_t)dir * g.H;
-    q.X = seq_exchange(g, ws) + (size_t)dir * g.T * seq_row(g, g.H);
+    q.X = ws + place.at[dir];
     q.hy = hy + (size_t)pl * g.BH;
     q.cy = cy && MODE == RNN_LSTM ? cy + (size_t)pl * g.BH : nullptr;
     ip.d[dir] = {hx ? hx + (size_t)pl * g.BH : nullptr, cx ? cx + (size_t)pl * g.BH : nullptr, w + o.bW, w + o.bR, q.HP, q.CP,
@@ -1458,6 +1515,7 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
   if (seq) {
     SeqInit ip{};
     SeqBwd p{};
+    const SeqPlace place = seq_place(g, true, l == g.L - 1);
     p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
     p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
     p.wait = options().rnn_wait; p.pause = SEQ_PAUSE_BWD; p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
@@ -1472,10 +1530,10 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
       q.dcy = dcy ? dcy + (size_t)pl * g.BH : nullptr;
       q.R = w + offsets(g, pl).R;
       q.HP = base + r.hp; q.CP = base + r.cp; q.GT = base + r.gt; q.RN = base + r.rn;
-      q.dGW = dGW[dir]; q.dGR = dGR[dir];
+      q.dGW = dGW[dir]; q.dGR = place.shared && dir == 0 ? dGW[0] : dGR[dir];
       q.dhx = dhx ? dhx + (size_t)pl * g.BH : nullptr;
       q.dcx = dcx ? dcx + (size_t)pl * g.BH : nullptr;
-      q.X = seq_exchange(g, ws) + (size_t)dir * g.T * seq_row(g, g.GH);
+      q.X = ws + place.at[dir];
       ip.d[dir].X = q.X;
     }
     launch_init(ip, g.D, s);
@@ -1483,6 +1541,7 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
     if (rc != FLHIP_OK && rc != FLHIP_DECLINED) return rc;
     seq = rc == FLHIP_OK;
     if (!seq && !fused_applies(g)) return FLHIP_DECLINED;
+    if (seq && place.shared) dGR[0] = dGW[0];
   }
   if (!seq) {
   if (MODE == RNN_LSTM)
@@ -1586,13 +1645,13 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   if (rc0 != FLHIP_OK) return rc0;
   FLHIP_REQUIRE(x && w && y && hy, "rnn_fwd: null argument");
   FLHIP_REQUIRE(reserve && reserve_bytes >= flhip_rnn_reserve_bytes(d), "rnn_fwd: reserve buffer too small");
-  FLHIP_REQUIRE(ws && ws_bytes >= flhip_rnn_workspace_bytes(d), "rnn_fwd: workspace too small");
+  FLHIP_REQUIRE(ws && ws_bytes >= base_bytes(g), "rnn_fwd: workspace too small");
   hipStream_t s = as_stream(stream);
   const Reserve r = reserve_layout(g);
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
-  bool seq = seq_applies(g, false, s);
+  bool seq = seq_applies(g, false, s) && ws_bytes >= workspace_bytes(g);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     float* out = l == g.L - 1 ? static_cast<float*>(y) : res + r.acts + (size_t)l * act;
@@ -1646,7 +1705,7 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   FLHIP_REQUIRE(x && w && dx && dw, "rnn_bwd: null argument");
   FLHIP_REQUIRE(reserve && reserve_bytes >= flhip_rnn_reserve_bytes(d),
                 "rnn_bwd: needs the reserve buffer of the forward pass");
-  FLHIP_REQUIRE(ws && ws_bytes >= flhip_rnn_workspace_bytes(d), "rnn_bwd: workspace too small");
+  FLHIP_REQUIRE(ws && ws_bytes >= base_bytes(g), "rnn_bwd: workspace too small");
   hipStream_t s = as_stream(stream);
   const Reserve r = reserve_layout(g);
   const float* res = static_cast<const float*>(reserve);
@@ -1656,7 +1715,7 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   float* goutbuf = wsf + 2 * TB * g.GH;
   float* ginbuf = goutbuf + act;
   const float* gout = static_cast<const float*>(dy);   // gradient of the top layer's output (may be null)
-  bool seq = seq_applies(g, true, s);
+  bool seq = seq_applies(g, true, s) && ws_bytes >= workspace_bytes(g);
   for (int l = g.L - 1; l >= 0; --l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;

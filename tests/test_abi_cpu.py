@@ -23,6 +23,18 @@ def test_header_symbols_are_exported_and_bound():
     assert declared == set(capi.SYMBOLS)
 
 
+@pytest.mark.parametrize("I,H,L,bidir,mode,T,B", [(512, 512, 2, 1, 2, 200, 32), (1024, 1024, 2, 1, 2, 1000, 64), (320, 512, 1, 0, 1, 400, 64),
+                                                  (1024, 1024, 1, 0, 3, 100, 64)])
+def test_sequence_launches_take_no_workspace_of_their_own(I, H, L, bidir, mode, T, B):
+    """What the backward pass of a recurrent layer holds: the gate gradients twice per direction, the gradients of the output and (two
+    buffers) of the widest input, for every step; beyond that at most twice 16 partial products of the largest weights' gradient and 1 MiB."""
+    d = capi.RnnDesc(I, H, L, bidir, mode, T, B, capi.F32)
+    D, G = 1 + bidir, {1: 1, 2: 4, 3: 3}[mode]
+    widest = max(I, D * H)
+    held = T * B * (2 * D * G * H + D * H + 2 * widest)
+    assert 4 * held <= capi.lib().flhip_rnn_workspace_bytes(C.byref(d)) <= 4 * (held + 2 * 16 * G * H * widest) + (1 << 20)
+
+
 def test_version_and_arch():
     text = open(os.path.join(ROOT, "include", "flhip.h")).read()
     declared = int(re.search(r"#define\s+FLHIP_VERSION\s+(\d+)", text).group(1))

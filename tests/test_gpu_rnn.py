@@ -1,6 +1,8 @@
 """GPU parity of rnn / rnnBackward through the C ABI against oracle/flref.c (which is
 pinned against PyTorch's RNN / LSTM / GRU in tests/test_oracle_rnn.py): all four modes,
 stacked, bidirectional, with and without initial states and output gradients."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -106,6 +108,47 @@ def test_whole_sequence_launches(mode, I, H, L, bidir, T, B, states):
     assert launches >= 2 * L if H <= 1024 else launches == 0
     if (H, clusters) == (1000, 5):      # 63 workgroups each: four to the first launch, forward and backward
         assert launches == 4
+
+
+@pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
+    # where the exchange of a sequence launch lies: in place of the first direction's gate gradients, in idle buffers (the topmost layer
+    # has one more), behind everything
+    (flref.RNN_LSTM, 9, 20, 3, True, 6, 18, True),         # whole chunks: shared, and idle buffers
+    (flref.RNN_LSTM, 70, 16, 1, False, 9, 33, True),
+    (flref.RNN_TANH, 5, 20, 2, True, 6, 18, True),         # a last chunk of 4: both directions in idle buffers
+    (flref.RNN_RELU, 3, 12, 2, False, 9, 5, True),         # chunks larger than the state
+    (flref.RNN_GRU, 12, 48, 1, False, 7, 17, True),        # one layer, the topmost
+    (flref.RNN_GRU, 12, 48, 3, False, 7, 17, True),        # lower layers: behind everything
+    (flref.RNN_GRU, 200, 32, 2, True, 5, 40, True),        # a wide input
+    (flref.RNN_GRU, 6, 20, 3, True, 6, 9, True),
+])
+def test_whole_sequence_launches_in_what_the_pass_leaves_idle(mode, I, H, L, bidir, T, B, states):
+    test_whole_sequence_launches(mode, I, H, L, bidir, T, B, states)
+
+
+def test_whole_sequences_without_room_for_their_exchange():
+    """A workspace of the size without sequence launches is accepted, and the steps run instead."""
+    I, H, L, T, B = 12, 48, 3, 40, 17
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(T, B, I, generator=g, device="cuda")
+    w = torch.randn(ops.rnn_param_count(I, H, L, ops.RNN_GRU, False), generator=g, device="cuda") / H ** 0.5
+    dy = torch.randn(T, B, H, generator=g, device="cuda")
+    y, _, _, reserve = ops.rnn(x, None, None, w, H, L, ops.RNN_GRU, False)
+    want = ops.rnn_backward(x, w, reserve, H, L, ops.RNN_GRU, False, dy)
+    d = capi.RnnDesc(I, H, L, 0, ops.RNN_GRU, T, B, capi.F32)
+    full = capi.lib().flhip_rnn_workspace_bytes(C.byref(d))
+    capi.set_option("RNN_SEQUENCES", "never")
+    try:
+        least = capi.lib().flhip_rnn_workspace_bytes(C.byref(d))
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
+    assert least < full
+    count, P = capi.lib().flhip_rnn_sequence_launches, lambda t: C.c_void_p(t.data_ptr())
+    before = count()
+    ws, dx, dw = torch.empty(least, dtype=torch.uint8, device="cuda"), torch.empty_like(x), torch.empty_like(w)
+    capi.check(capi.lib().flhip_rnn_bwd(C.byref(d), P(x), P(w), P(dy), None, None, P(reserve), reserve.numel() * reserve.element_size(), P(dx), None,
+                                        None, P(dw), P(ws), least, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert count() == before and rel_l2(host(dx), host(want[0])) <= 1e-5 and rel_l2(host(dw), host(want[3])) <= 1e-5
 
 
 @pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
