@@ -1055,7 +1055,7 @@ tap1d_wgrad_split_kernel(Tap1WParams p, const float* __restrict__ xr, const floa
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       big[t][r] += small[t][r];
-      bad |= not_finite(big[t][r]);
+      bad |= split_redo(big[t][r]);
     }
   if (__builtin_amdgcn_ballot_w64(bad)) {          // once more with the operands as they are
 #pragma unroll

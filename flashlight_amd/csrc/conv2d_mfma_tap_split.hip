@@ -226,7 +226,7 @@ tap_split_kernel(TapSplit p, const float* __restrict__ xr, const uintx4_t* __res
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       big[b][r] += small[b][r];
-      bad |= not_finite(big[b][r]);
+      bad |= split_redo(big[b][r]);
     }
   const int mrow = mtile * BM + wm * 32, ob = o0 + wp * (32 * NB) + fr;
   if (__builtin_amdgcn_ballot_w64(bad)) {          // once more with the operands as they are

@@ -269,7 +269,7 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         big[i][c][r] += small[i][c][r];
-        bad |= not_finite(big[i][c][r]);
+        bad |= split_redo(big[i][c][r]);
       }
   // once more with the operands as they are (rows, columns and contraction indexes past the last as zero)
   if (__builtin_amdgcn_ballot_w64(bad)) {

@@ -1,7 +1,8 @@
 // fp32 operands on the 16-bit matrix cores: x = h + m + l, three bf16 parts, each the rounded remainder of those before it
 // (8 + 8 + 8 significant bits: nothing is left of a 24-bit significand), and
 //   a b = ah bh + (ah bm + am bh + am bm + ah bl + al bh),
-// six exact products per pair; what is left out (am bl, al bm, al bl) is below 2^-26 of the product.  The first sum and that of
+// six exact products per pair; what is left out (am bl, al bm, al bl) is below 2^-24.1 of the product, 2^-27.5 in the mean (a sum of one
+// product is off by up to 0.97 units in the last place, rounded once by 0.5; sums gain, see below).  The first sum and that of
 // the five small terms have an accumulator each: the small ones' roundings then fall 2^-8 below those of the first, which has one
 // rounding per 16 contraction indexes where v_mfma_f32_32x32x2_f32 has one per 2.  Measured against 64 bits, relative 2-norm, normal
 // operands (the fp32 instruction on the same operands): contraction of 16 3.5e-8 (8.0e-8), 256 9.1e-8 (3.0e-7), 5248 4.6e-7
@@ -9,8 +10,13 @@
 // The matrix pipe takes six such products in 3/8 of the fp32 instruction's time (16 times its rate).
 //
 // Infinities, NaN and magnitudes that round to infinity in bf16 leave NaN in a part, and so in every result that they
-// reach: the kernels compute tiles with a result that is not finite a second time, on the fp32 instruction.  Magnitudes below
-// 2^-110 lose their last bits to the parts' underflow (2^-134 absolute).
+// reach.  Magnitudes below 2^-110 lose their last bits to the parts' underflow: 2^-134 absolute (subnormal parts are kept),
+// times the other operand, which only a small result can feel.  So the kernels compute what a wave holds a second time, on the fp32
+// instruction, where a result is not finite, or not zero and below 2^-90.  What is left of the underflow is below 2^-24 of a result as
+// long as the other operand's magnitudes add up to no more than 2^20 over the contraction.  (Measured before the second condition: operands
+// of 2^-115 1.1e-6, of 2^-126 2.2e-3 in the 2-norm, the fp32 instruction 4e-7.)  It takes 3 to 5 times as long as the first where one
+// infinity reaches every tile, up to 9 times where all results are small: 3 x 3, 256 -> 256 channels over 14 x 14, 64 images 95 us -> 388,
+// 611 in all, 21 taps, 250 -> 250 channels, 16 x 1500 frames 289 -> 1623, 2840.
 #pragma once
 #include "conv2d_mfma.h"
 
@@ -43,6 +49,10 @@ __device__ __forceinline__ void split_mma(floatx16& big, floatx16& small, const 
   big = Lo16<bf16_t>::mma32(a[0], b[0], big);
 }
 
-__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+// whether a result has to be computed a second time
+__device__ __forceinline__ bool split_redo(float v) {
+  const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+  return u >= 0x7f800000u || u - 1u < 0x12800000u - 1u;      // (0x12800000 = 2^-90)
+}
 
 }  // namespace flhip

@@ -807,6 +807,46 @@ def test_fp32_1x1_windows_in_three_parts(xs, k, stride, special):
             assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24, name
 
 
+@pytest.mark.parametrize("small,other", [(-100, 0), (-115, 0), (-130, 0), (-126, 10), (-120, 100), (-130, 100)])
+def test_fp32_in_three_parts_of_small_operands(small, other):
+    """One operand's values around 2^small, of which the third bf16 part keeps fewer bits or none, the other's around 2^other, in every family of
+    kernels that take fp32 operands apart, against float64.  Where the results are below 2^-90 they are those of the fp32 instruction: within
+    2 (sqrt(n) + 1) units of 2^-24 of the sum of the products' magnitudes, and n units of 2^-149 where they are subnormal.  Else a value may be off by
+    2^-134 as well, times the sum of the other operand's magnitudes."""
+    import torch.nn.functional as F
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(-small)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    S, T = 2.0 ** small, 2.0 ** other
+
+    def check(name, got, f, a, b):
+        """got = f(a, b) with a the small operand"""
+        a, b = a.double(), b.double()
+        want, mag, rest, n = f(a, b), f(a.abs(), b.abs()), f(torch.ones_like(a), b.abs()), f(torch.ones_like(a), torch.ones_like(b))
+        allowed = 2 * (n ** 0.5 + 1) * 2.0 ** -24 * mag + n * 2.0 ** -149 + (2.0 ** -134 * rest if other > 50 else 0)
+        assert bool(((got.double() - want).abs() <= allowed).all()), name
+
+    d, x, w = r(2492, 68) * S, r(2492, 2528) * T, r(2528, 68) * T
+    dx, dw, _ = ops.linear_backward(d, x, w, False)
+    check("A^T B", dx, lambda a, b: a @ b.t().contiguous(), d, w)
+    check("A B^T", dw, lambda a, b: b.t().contiguous() @ a, d, x)
+    x, w = r(64, 64, 28, 28) * S, r(256, 64, 1, 1) * T
+    rows = lambda t: t.transpose(0, 1).reshape(t.shape[1], -1)
+    flat = lambda a, b: (b.view(256, 64) @ rows(a)).view(256, 64, 28, 28).transpose(0, 1)
+    check("1x1", ops.conv2d(x, w, None), flat, x, w)
+    dy = r(64, 256, 28, 28) * T
+    check("1x1 gradient", ops.conv2d_backward_filter_bias(dy, x, w.shape, False)[0].view(256, 64), lambda a, b: rows(b) @ rows(a).t().contiguous(), x, dy)
+    for xs, ws in (((4, 80, 1, 300), (70, 80, 1, 9)), ((64, 64, 14, 14), (64, 64, 3, 3))):
+        pad = (ws[2] // 2, ws[3] // 2)
+        kw = dict(px=pad[1], py=pad[0])
+        x, w, dy = r(*xs) * S, r(*ws) * T, r(xs[0], ws[0], *xs[2:]) * T
+        cols = lambda t: F.unfold(t, ws[2:], padding=pad).permute(1, 0, 2).reshape(ws[1] * ws[2] * ws[3], -1)
+        check(str(ws), ops.conv2d(x, w, None, **kw), lambda a, b: (b.view(ws[0], -1) @ cols(a)).view(ws[0], xs[0], *xs[2:]).transpose(0, 1), x, w)
+        if ws[2] == 1:
+            dw = ops.conv2d_backward_filter_bias(dy, x, ws, False, **kw)[0]
+            check(str(ws) + " gradient", dw.view(ws[0], -1), lambda a, b: rows(b) @ cols(a).t().contiguous(), x, dy)
+
+
 @pytest.mark.parametrize("xs,k,kw,dtype", [((2, 512, 17, 17), 250, 22, torch.float32), ((4, 512, 14, 14), 250, 17, torch.float32)])
 def test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dtype):
     """fp32 one-row windows of more than 256 channels, whose own kernels ask for more than the static buffer holds, run on the general
