@@ -10,6 +10,7 @@ memory and of the stream.
 import ctypes as C
 import enum
 import functools
+import operator
 
 import torch
 
@@ -83,11 +84,22 @@ def _conv_desc(x_shape, w_shape, sx, sy, px, py, dx, dy, groups, tag):
     return capi.ConvDesc(N, Cc, H, W, K, KH, KW, sy, sx, py, px, dy, dx, groups, tag)
 
 
+def _conv_plan(x_shape, w_shape, *numbers):
+    """What follows from a layer's geometry (sx, sy, px, py, dx, dy, groups, tag) alone: the descriptor, a reference to it and the
+    output's shape.  Kept per geometry: built anew they were 1.6 of the 11 us that the host took for a 1x1 layer over one image.  By
+    value: whatever else can be an index (an array or a tensor of one element, which may not be kept) becomes a plain int first."""
+    try:
+        return _kept_conv_plan(x_shape, w_shape, *numbers)
+    except TypeError:
+        ints = lambda values: tuple(int(operator.index(v)) for v in values)
+        return _kept_conv_plan(ints(x_shape), ints(w_shape), *ints(numbers))
+
+
 @functools.lru_cache(maxsize=1024, typed=True)
-def _conv_plan(x_shape, w_shape, sx, sy, px, py, dx, dy, groups, tag):
-    """What follows from a layer's geometry alone: the descriptor, a reference to it and the output's shape.  Kept per geometry: built
-    anew they were 1.6 of the 11 us that the host took for a 1x1 layer over one image."""
-    d = _conv_desc(x_shape, w_shape, sx, sy, px, py, dx, dy, groups, tag)
+def _kept_conv_plan(x_shape, w_shape, *numbers):
+    if any(type(v) is not int for v in (*x_shape, *w_shape, *numbers)):
+        raise TypeError("plain ints expected")
+    d = _conv_desc(x_shape, w_shape, *numbers)
     oh, ow = C.c_int32(), C.c_int32()
     capi.check(capi.lib().flhip_conv2d_out_dims(C.byref(d), C.byref(oh), C.byref(ow)))
     return d, C.byref(d), (d.N, d.K, oh.value, ow.value)

@@ -35,6 +35,22 @@ def test_sequence_launches_take_no_workspace_of_their_own(I, H, L, bidir, mode, 
     assert 4 * held <= capi.lib().flhip_rnn_workspace_bytes(C.byref(d)) <= 4 * (held + 2 * 16 * G * H * widest) + (1 << 20)
 
 
+def test_layer_geometry_is_kept_by_value():
+    """Whatever can be an index is taken as one: arrays of one element, which have no hash, and tensors, whose hash is their identity."""
+    import numpy as np
+    import torch
+    from flashlight_amd import ops
+    plan = lambda s, x=(2, 3, 9, 9): ops._conv_plan(x, (4, 3, 3, 3), s, 1, 1, 1, 1, 1, 1, capi.F32)[2]
+    stride = torch.tensor(1)
+    assert plan(2) == plan(np.array(2)) == plan(np.int64(2)) == (2, 4, 9, 5) and plan(stride) == plan(True) == (2, 4, 9, 9)
+    stride.fill_(2)
+    assert plan(stride) == plan(2, tuple(np.array([2, 3, 9, 9]))) == plan(2, tuple(torch.tensor([2, 3, 9, 9]))) == (2, 4, 9, 5)
+    with pytest.raises(TypeError):
+        plan(2.0)
+    with pytest.raises(ValueError):
+        plan(1, (2, 5, 9, 9))
+
+
 def test_version_and_arch():
     text = open(os.path.join(ROOT, "include", "flhip.h")).read()
     declared = int(re.search(r"#define\s+FLHIP_VERSION\s+(\d+)", text).group(1))
