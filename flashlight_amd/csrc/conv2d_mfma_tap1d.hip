@@ -209,20 +209,42 @@ __device__ __forceinline__ void tap1d_weights_block(const T* __restrict__ w, uin
   }
 }
 
+// The same, one wave per fragment (`unit`: the tap fastest, so that a workgroup's waves read the same lines).
+template <typename T>
+__device__ __forceinline__ void tap1d_weights_gather(const T* __restrict__ w, uintx4_t* __restrict__ wf, const Tap1Weights& p, int unit) {
+  const int lane = threadIdx.x & 63, block = unit / p.taps_total, tap = unit - block * p.taps_total, mblk = block / p.KS, ks = block - mblk * p.KS;
+  if (mblk >= p.mblocks) return;
+  const int m = mblk * 32 + (lane & 31), c0 = ks * 16 + 8 * (lane >> 5), j = p.tapj[tap];
+  __attribute__((aligned(16))) T v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int c = c0 + e;
+    v[e] = j >= 0 && m < p.Mo && c < p.Cc ? w[p.bwd ? ((size_t)c * p.Cw + m) * p.KW + j : ((size_t)m * p.Cw + c) * p.KW + j] : T{};
+  }
+  wf[(((size_t)mblk * p.taps_total + tap) * p.KS + ks) * 64 + lane] = *reinterpret_cast<const uintx4_t*>(v);
+}
+// Up to so many blocks of tap1d_weights_block: they leave most of the chip idle, and each is a chain of loads, LDS and its taps.
+// us of a layer (blocks / fragments; before either 15.5, 11.9, 26.9, 46.5, 55.6): 256 channels to 29 over 6 x 491 frames, 29 taps,
+// backward (8 blocks) 15.0 / 12.4; 80 to 28 over 3 x 300, 21 taps, backward (8) 11.5 / 9.4; 80 to 250 over 7 x 1111, 21 taps (48) 22.1 / 21.3;
+// 250 to 250 (128), weights not in the caches, 33.4 / 35.3; 250 to 1000 over 4 x 400 (512) 35.0 / 42.7.
+constexpr int T1_FEW_BLOCKS = 64;
+
 // Both operands of a layer in 16-bit storage in one launch: neither pass fills the chip, and each is a few microseconds of latency
 // (loads, LDS, stores).  The first blocks take the rows, the others the weights.  Rows one element at a time where they are odd, and
 // weights gathered fragment by fragment (every line met once per tap) in a launch of their own: 8.2 + 8.8 us for 250 -> 250 channels, 21 taps
-// over 7 x 1111 frames, and a launch more for the host; the layer's passes replayed from a graph 48.6 -> 44.6 and 45.5 -> 44.2; 120 random layers in bf16 and f16 0.87 of the time forward, 0.89 backward, the
-// slowest 1.09 (over 29 filters, 13.0 -> 14.2 us: 16 blocks of weights).
+// over 7 x 1111 frames, and a launch more for the host; the layer's passes replayed from a graph 48.6 -> 44.6 and 45.5 -> 44.2; 240
+// random layers in bf16 and f16, both passes, 0.82 of the time, the slowest 1.01.
 template <typename T>
 __global__ void __launch_bounds__(256)
 tap1d_operands_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int Tn, int Cs, int tblocks, int cblocks, int rblocks,
-                      const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p) {
+                      const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p, bool gather) {
   extern __shared__ uintx4_t t1_operands[];
   const int b = blockIdx.x;
   if (b < rblocks) {
     const int t = b / tblocks;
     tap1d_rows_block(x, xr, C, H, Tn, Cs, b - t * tblocks, t % cblocks, t / cblocks, t1_operands);
+  } else if (gather) {
+    tap1d_weights_gather(w, wf, p, (b - rblocks) * 4 + (int)(threadIdx.x >> 6));
   } else {
     tap1d_weights_block(w, wf, p, b - rblocks, reinterpret_cast<T*>(t1_operands));
   }
@@ -638,10 +660,12 @@ int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const 
   uintx4_t* wf = reinterpret_cast<uintx4_t*>(static_cast<char*>(ws) + pl.rows_bytes);
   {
     const dim3 rg = rows_grid(pl.T, pl.p.Cs, pl.p.rows);
-    const size_t rblocks = (size_t)rg.x * rg.y * rg.z, blocks = rblocks + (size_t)pl.w.mblocks * pl.w.KS;
-    const size_t lds = std::max<size_t>(64 * 66 * sizeof(T), (544 * (size_t)pl.w.KW + 64) * sizeof(T));
+    const size_t rblocks = (size_t)rg.x * rg.y * rg.z, wblocks = (size_t)pl.w.mblocks * pl.w.KS;
+    const bool gather = wblocks <= T1_FEW_BLOCKS;
+    const size_t blocks = rblocks + (gather ? (wblocks * pl.w.taps_total + 3) / 4 : wblocks);
+    const size_t lds = std::max<size_t>(64 * 66 * sizeof(T), gather ? 0 : (544 * (size_t)pl.w.KW + 64) * sizeof(T));
     hipLaunchKernelGGL((tap1d_operands_kernel<T>), dim3((unsigned)blocks), dim3(256), lds, s, static_cast<const T*>(src), xr, pl.C, pl.H, pl.T,
-                       pl.p.Cs, (int)rg.x, (int)rg.y, (int)rblocks, static_cast<const T*>(w), wf, pl.w);
+                       pl.p.Cs, (int)rg.x, (int)rg.y, (int)rblocks, static_cast<const T*>(w), wf, pl.w, gather);
   }
   if (const int rc = check_launch("conv2d (one-row windows, operand passes)")) return rc;
   T* out = static_cast<T*>(dst);

@@ -916,6 +916,28 @@ def test_first_layer_filter_gradient_over_rows_of_128(xs, k, win, pad, dtype):
         assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,kw,stride", [((2, 17, 1, 40), 16, 2, 1), ((3, 100, 1, 90), 256, 5, 1), ((3, 100, 1, 90), 257, 5, 1),      # 64 and 72 blocks
+                                            ((2, 256, 1, 75), 129, 21, 2), ((2, 90, 1, 75), 300, 32, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_one_row_windows_in_16_bit_storage_by_blocks_of_weights(xs, k, kw, stride, dtype):
+    """Weights in operand order fragment by fragment (few blocks) and block by block, a last block of one filter, phases of unequal taps;
+    against float64: one rounding per result, fp32 sums."""
+    import torch.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(k, xs[1], 1, kw, generator=g, device="cuda") / (xs[1] * kw) ** 0.5).to(dtype)
+    kw_ = dict(sx=stride, px=kw // 2)
+    y = fa.conv2d(x, w, None, **kw_)
+    dy = torch.randn(*y.shape, generator=g, device="cuda").to(dtype)
+    dx = fa.conv2d_backward_data(dy, xs, w, **kw_)
+    xd, wd = x.double().cpu()[:, :, 0].requires_grad_(), w.double().cpu()[:, :, 0]
+    want = F.conv1d(xd, wd, stride=stride, padding=kw // 2)
+    want.backward(dy.double().cpu()[:, :, 0])
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for got, ref in ((y, want.detach()), (dx, xd.grad)):
+        assert bool(((got.double().cpu()[:, :, 0] - ref).abs() <= unit * ref.abs() + 1e-4).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
