@@ -1235,7 +1235,7 @@ struct SeqPlace {
 SeqPlace seq_place(const RnnGeom& g, bool bwd, bool top) {
   const size_t TB = (size_t)g.T * g.B, core = workspace_core(g), need = (size_t)g.T * seq_row(g, bwd ? g.GH : g.H);
   SeqPlace p{};
-  size_t from[2] = {}, to[2] = {}, behind = core;
+  size_t from[2] = {}, to[2] = {};
   if (bwd) {
     const size_t gout = 2 * TB * g.GH, scratch = wgrad_scratch_offset(g);
     from[0] = top ? gout : gout + TB * g.D * g.H;
@@ -1245,7 +1245,6 @@ SeqPlace seq_place(const RnnGeom& g, bool bwd, bool top) {
   } else {
     from[0] = (size_t)g.D * (TB * g.GH + g.GH);
     to[0] = core - 4;
-    behind += scratch_of(g, nullptr).bytes / sizeof(float);       // (the projections use the scratch after the exchange is filled)
   }
   for (int dir = 0; dir < g.D; ++dir) {
     if (bwd && dir == 0 && g.mode != RNN_GRU && g.GH % 16 == 0) {
@@ -1262,22 +1261,24 @@ SeqPlace seq_place(const RnnGeom& g, bool bwd, bool top) {
       placed = true;
     }
     if (placed) continue;
-    p.at[dir] = behind;
-    behind += need;
-    p.end = behind;
+    // (forward the projections use the scratch after the exchange is filled)
+    p.at[dir] = p.end ? p.end : core + (bwd ? 0 : scratch_of(g, nullptr).bytes / sizeof(float));
+    p.end = p.at[dir] + need;
   }
   return p;
+}
+// floats of workspace that the exchanges of a pass end at
+size_t seq_end(const RnnGeom& g, bool bwd) {
+  const size_t top = seq_place(g, bwd, true).end;
+  return bwd && g.L > 1 ? std::max(top, seq_place(g, true, false).end) : top;
 }
 
 // what a call cannot do without, and with what its sequence launches take where they may be launched
 size_t base_bytes(const RnnGeom& g) { return workspace_core(g) * sizeof(float) + scratch_of(g, nullptr).bytes; }
 size_t workspace_bytes(const RnnGeom& g) {
   size_t end = 0;
-  if (seq_asked(g, false)) end = seq_place(g, false, true).end;
-  if (seq_asked(g, true)) {
-    end = std::max(end, seq_place(g, true, true).end);
-    if (g.L > 1) end = std::max(end, seq_place(g, true, false).end);
-  }
+  for (const bool bwd : {false, true})
+    if (seq_asked(g, bwd)) end = std::max(end, seq_end(g, bwd));
   return std::max(base_bytes(g), end * sizeof(float));
 }
 
@@ -1651,7 +1652,7 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
-  bool seq = seq_applies(g, false, s) && ws_bytes >= workspace_bytes(g);
+  bool seq = seq_applies(g, false, s) && ws_bytes >= seq_end(g, false) * sizeof(float);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     float* out = l == g.L - 1 ? static_cast<float*>(y) : res + r.acts + (size_t)l * act;
@@ -1715,7 +1716,7 @@ extern "C" int flhip_rnn_bwd(const flhip_rnn_desc* d, const void* x, const void*
   float* goutbuf = wsf + 2 * TB * g.GH;
   float* ginbuf = goutbuf + act;
   const float* gout = static_cast<const float*>(dy);   // gradient of the top layer's output (may be null)
-  bool seq = seq_applies(g, true, s) && ws_bytes >= workspace_bytes(g);
+  bool seq = seq_applies(g, true, s) && ws_bytes >= seq_end(g, true) * sizeof(float);
   for (int l = g.L - 1; l >= 0; --l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;
     const size_t inl = l == 0 ? g.I : (size_t)g.D * g.H;
