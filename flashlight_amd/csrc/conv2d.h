@@ -158,9 +158,9 @@ int mfma_slab16_conv_fwd(const ConvGeom& g, const void* x, const void* w, const 
                          hipStream_t s, int dtype);
 int mfma_slab16_conv_bwd_data(const ConvGeom& g, const void* dy, const void* w, void* dx,
                               hipStream_t s, int dtype);
-// windows of one row (KH = 1, 2 to 32 taps, column stride 1 or 2, no groups, 16 to 256 contraction channels) in bf16
-// or fp32 storage through channels-last rows and fragment-ordered weights in mfma_tap1d_conv_ws() bytes of workspace
-// (conv2d_mfma_tap1d.hip); -1 when the shape is not theirs or the room is missing
+// windows of one row (KH = 1, 2 to 32 taps, column stride 1 or 2, no groups, 16 to 256 contraction channels, in fp32 to 512) in 16-bit
+// or fp32 storage through channels-last rows (fp32 backward-data: the planes as they lie) and fragment-ordered weights in
+// mfma_tap1d_conv_ws() bytes of workspace (conv2d_mfma_tap1d.hip; fp32: conv2d_mfma_tap_split.hip); -1 when the shape is not theirs or the room is missing
 size_t mfma_tap1d_conv_ws(const ConvGeom& g, int dtype, bool bwd);
 int mfma_tap1d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
                         void* ws, size_t ws_bytes);
@@ -178,9 +178,9 @@ int mfma_tap2d_split(const ConvGeom& g, bool bwd, const void* src, const void* w
                      size_t ws_bytes);
 int mfma_tap1d_cs(int C, int esz);
 void mfma_tap1d_rows_f32(const float* x, float* xr, int C, int H, int T, int Cs, int rows, hipStream_t s);
-// 3x3 windows of stride 1 and padding 1 over small planes on the same kernels: every plane of the batch in one
-// sequence (rows followed by a zero column, planes separated by a zero row), 65 to 512 (fp32: 256) contraction channels;
-// operands in mfma_tap2d_conv_ws() bytes of workspace; -1 when the shape is not theirs or the room is missing
+// Windows of stride 1 that keep the plane's size on the same kernels: every plane of the batch in one sequence (rows followed by
+// zero columns, planes separated by zero rows).  16-bit storage: 3x3, 65 to 512 contraction channels; fp32: any odd window of several
+// rows and up to 64 taps, 16 to 512 contraction channels; operands in mfma_tap2d_conv_ws() bytes of workspace; -1 when the shape is not theirs or the room is missing
 size_t mfma_tap2d_conv_ws(const ConvGeom& g, int dtype, bool bwd);
 int mfma_tap2d_conv_fwd(const ConvGeom& g, int dtype, const void* x, const void* w, const float* bias, void* y, hipStream_t s,
                         void* ws, size_t ws_bytes);

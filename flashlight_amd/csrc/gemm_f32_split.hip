@@ -25,8 +25,8 @@
 //
 // Layers of 1x1 windows are the same products with the positions of all images as A's and C's rows (modes 0 and 2) or as the contraction
 // (mode 1): only where a thread's values lie differs (PL), a position being looked up once per workgroup.  Over large planes memory bounds
-// them: four small tiles to a compute unit (128 registers; three at 129; A^T B on 64 x 128 tiles needs 132) and tiles that share positions one after the other on one
-// die, us: 64 -> 256 channels over 56 x 56, 32 images 47 -> 39 (129 MB), the addend's loads in front of the stores 70 -> 38; filter
+// them: four small tiles to a compute unit (128 registers, A B with one value kept in memory over its loop; three at 129; A^T B on 64 x
+// 128 tiles needs 132) and tiles that share positions one after the other on one die, us: 64 -> 256 channels over 56 x 56, 32 images 47 -> 39 (129 MB), the addend's loads in front of the stores 70 -> 38; filter
 // gradient of 256 x 64, a slice's tiles on one die, 45 -> 39.  (The general kernels' times stand at the rule, conv2d_mfma_pointwise.hip.)
 #include <algorithm>
 
@@ -192,7 +192,8 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
   }
   const __amdgpu_buffer_rsrc_t ar = make_rsrc(A, p.a_bytes), br = make_rsrc(B, p.b_bytes);
   float va[SA::EL], vb[SB::EL];
-  // end of the slice's whole stages (there is one at least; of planes every stage is one: what lies past them reads zero)
+  // end of the slice's whole stages (the contraction has one at least; a last slice may have none, only the stage of fewer indexes, and then
+  // loads one of the slice before it for nobody; of planes every stage is whole: what lies past them reads zero)
   const int full = PL && MODE == 1 ? send : min(send, p.K / G32_KC);
   auto stage_in = [&](int s) __attribute__((always_inline)) {
     if constexpr (PL && MODE == 1) {

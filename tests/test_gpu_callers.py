@@ -260,7 +260,8 @@ def test_matmul_fp32_tiles_with_odd_rows(M, N, K):
 @pytest.mark.parametrize("M,N,K", [
     (2396, 1292, 16), (2700, 1092, 20), (2744, 76, 1584), (68, 2720, 1380),            # 128 x 64: whole stages, a last one of 4, slices of either
     (2460, 1656, 32), (2480, 1604, 20), (180, 2732, 1232), (132, 2720, 1220),          # 64 x 128
-    (2540, 2516, 80), (2528, 2492, 68), (520, 2544, 1120)])                            # 128 x 128
+    (2540, 2516, 80), (2528, 2492, 68), (520, 2544, 1120),                             # 128 x 128
+    (468, 652, 1444)])                                                                  # 11 slices, the last of 4 contraction indexes alone
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_matmul_fp32_in_three_parts(mode, M, N, K):
     """The tiles whose operands are taken apart into bf16 parts, the bias with them."""
@@ -389,6 +390,25 @@ def test_matmul_in_16_bit_storage_on_large_tiles(M, N, K, mode, dtype):
     want = (A.float() @ B.float()).t() + (b if b is not None else 0)
     unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     assert bool(((out.float() - want).abs() <= unit * want.abs() + 1e-4 * K ** 0.5).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(3081, 2565, 127), (4001, 2561, 65), (2561, 3585, 4001), (129, 65, 33)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_matmul_in_16_bit_storage_of_an_odd_number_of_elements(M, N, K, dtype):
+    """A^T B whose operands end half a word into a 4-byte word, on large tiles and small ones: the last row's last elements, and the last
+    row against the fp32 product: one rounding per element, and sums in another order."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A, B = torch.randn(M, K, generator=g, device="cuda").to(dtype), torch.randn(N, K, generator=g, device="cuda").to(dtype)
+    A[-1, -3:], B[-1, -3:] = torch.tensor([8.0, 16.0, 64.0]), torch.tensor([32.0, -16.0, 64.0])
+    import ctypes as C
+    from flashlight_amd import capi
+    out = torch.full((N, M), float("nan"), device="cuda", dtype=dtype)
+    capi.check(capi.lib().flhip_matmul(C.c_void_p(A.data_ptr()), C.c_void_p(B.data_ptr()), C.c_void_p(out.data_ptr()), M, N, K, 1, 0, None,
+                                       capi.BF16 if dtype == torch.bfloat16 else capi.F16, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    want = B.float() @ A.float().t()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert bool(((out.float() - want).abs() <= unit * want.abs() + 1e-4 * K ** 0.5 * 64).all())
+    assert abs(float(out[-1, -1]) - (256.0 - 256.0 + 4096.0)) <= 2 * unit * 4096 + 5 * K ** 0.5
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
