@@ -13,7 +13,8 @@
 // reach.  Magnitudes below 2^-110 lose their last bits to the parts' underflow: 2^-134 absolute (subnormal parts are kept),
 // times the other operand, which only a small result can feel.  So the kernels compute what a wave holds a second time, on the fp32
 // instruction, where a result is not finite, or not zero and below 2^-90.  What is left of the underflow is below 2^-24 of a result as
-// long as the other operand's magnitudes add up to no more than 2^20 over the contraction.  (Measured before the second condition: operands
+// long as the other operand's magnitudes add up to no more than 2^20 over the contraction, and operands below 2^-134 count as zero where all
+// results that they reach are zero with them (zeros alone are not looked at again: masks and padding are full of them).  (Measured before the second condition: operands
 // of 2^-115 1.1e-6, of 2^-126 2.2e-3 in the 2-norm, the fp32 instruction 4e-7.)  It takes 3 to 5 times as long as the first where one
 // infinity reaches every tile, up to 9 times where all results are small: 3 x 3, 256 -> 256 channels over 14 x 14, 64 images 95 us -> 388,
 // 611 in all, 21 taps, 250 -> 250 channels, 16 x 1500 frames 289 -> 1623, 2840.

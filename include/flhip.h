@@ -442,7 +442,8 @@ int flhip_pad_bwd(const void* dy, void* dx, const int64_t* dims, const int32_t* 
 /* C (M x N) = op(A) (M x K) * op(B) (K x N), fp32 accumulate, one rounding to the element
  * type; trans_a: A is stored K x M, trans_b: B is stored N x K.  bias_rows (fp32[M], may be
  * NULL) is added to every column.  bf16 / f16 products of more than 128 columns run on the
- * 16-bit matrix instructions (option MATMUL_FP32_CORES: on the fp32 ones, fp32 products too).  Serves fl::linear (Functions.cpp:1255-1309): forward
+ * 16-bit matrix instructions, and so do large fp32 ones with an operand transposed, in three bf16 parts (option MATMUL_FP32_CORES:
+ * both on the fp32 instructions, as A * B in fp32 always is).  Serves fl::linear (Functions.cpp:1255-1309): forward
  * matmul(weight, input) + tile(bias), backward matmulTN(weight, gradOutput) and
  * matmulNT(gradOutput, input). */
 int flhip_matmul(const void* A, const void* B, void* C, int32_t M, int32_t N,
@@ -587,7 +588,8 @@ typedef struct flhip_rnn_desc {
 /* number of weight elements (cudnnGetRNNParamsSize / element size); 0 for a bad descriptor */
 size_t flhip_rnn_param_count(const flhip_rnn_desc* d);
 /* the reserve buffer carries the forward pass's states and gate activations to the
- * backward pass (cuDNN's reserve space, RNN.cpp:154-160); the workspace is scratch */
+ * backward pass (cuDNN's reserve space, RNN.cpp:154-160); the workspace is scratch.  Its size
+ * follows the option RNN_SEQUENCES; what `never` asks for is always accepted, and the launches that it holds no room for are not made */
 size_t flhip_rnn_reserve_bytes(const flhip_rnn_desc* d);
 size_t flhip_rnn_workspace_bytes(const flhip_rnn_desc* d);
 /* hx, cx may be NULL (zero initial state); cy may be NULL */
