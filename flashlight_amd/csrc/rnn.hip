@@ -986,19 +986,24 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
       seq_pause(p.pause);
       const __amdgpu_buffer_rsrc_t r = row.rsrc(st + 1);
       floatx4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
+      // (more chunks than there are scalar registers for their offsets and for whether they exist: both in each step, not once, where the
+      // compiler moved 37 to 75 of them to vector registers and back; up to 16 chunks once is the faster one, by 2 to 3 %)
+      SeqRow now = row;
+      int rows = GH;
+      if constexpr (NC > 16) asm volatile("" : "+s"(now.nc), "+s"(rows));
       uintx4_t v[2][U];
-      seq_load(r, row, wave, v[0]);
+      seq_load(r, now, wave, v[0]);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        if (b + 1 < NB) seq_load(r, row, wave + W * (b + 1) * U, v[(b + 1) & 1]);
-        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, row, wave + W * b * U, v[b & 1], dead, lost.limit));
+        if (b + 1 < NB) seq_load(r, now, wave + W * (b + 1) * U, v[(b + 1) & 1]);
+        dead = __builtin_amdgcn_readfirstlane(seq_wait(r, now, wave + W * b * U, v[b & 1], dead, lost.limit));
         if (b == NB - 1) {
           seq_drain();
           fetch(st - 1);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if ((wave + W * (b * U + u)) * 16 < GH)
+          if ((wave + W * (b * U + u)) * 16 < rows)
 #pragma unroll
             for (int m = 0; m < 4; ++m)
               acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b * U + u][m], __uint_as_float(v[b & 1][u][m]), acc[0], 0, 0, 0);
@@ -1165,14 +1170,18 @@ int seq_units(const RnnGeom& g) {
 // what all workgroups of a layer ask for in a step (V, MB).  Measured, us with pauses of 2 / 4 / 6 / 8: LSTM of 320 units, 5 columns over
 // 100 steps (V 0.5) 214 / 218 / 228 / 238; GRU of 256 units, two directions, 20 columns (2.6) 204 / 208 / 216 / 228; tanh of 384 units, two
 // directions, 64 columns (4.7) 231 / 215 / 227 / 233; LSTM of 512 units, two directions, 32 columns over 200 steps (8.4) 686 / 642 / 639 /
-// 648; GRU of 1024 units, 64 columns (16.8) 580 / 568 / 572 / 583.
+// 648; GRU of 1024 units, 64 columns (16.8) 580 / 568 / 572 / 583.  With 4 units to a workgroup every workgroup's loads are many for the few
+// columns that this many clusters have; 60 steps, 2 / 3 / 4: LSTM of 1024 units, 1 column 200 / 179 / 177, 2 columns 187 / 177 / 179, of 768,
+// 1 column 185 / 163 / 164, of 512, 8 columns 145 / 145 / 148; GRU of 640, 1 column 162 / 150 / 153; but LSTM of 320 units, 1 column 133 / 132 / 132, 16
+// 135 / 136 / 139, and with 8 units to a workgroup (LSTM of 1024, two directions, 1 column) 241 / 245 / 246.
 int seq_pause_fwd(const RnnGeom& g, int units) {
   const double V = (double)g.D * ((g.H + units - 1) / units) * g.B * g.H * 4e-6;
-  return V < 4 ? 2 : 4;
+  return V >= 4 ? 4 : units == 4 && g.H >= 512 ? 3 : 2;
 }
 // Backward a step has more to load and to do between its stores and the next step's loads: 0 / 1 / 2 / 4 1372 / 1375 / 1382 / 1405 us
-// (that LSTM of 512 units), 338 / 337 / 343 / 352 (LSTM of 128 units, 16 columns over 100 steps).
-constexpr int SEQ_PAUSE_BWD = 1;
+// (that LSTM of 512 units), 338 / 337 / 343 / 352 (LSTM of 128 units, 16 columns over 100 steps).  Over 42 layers of up to 4 columns each 0
+// takes 0.987 of the time with 1 (at worst 1.004), over 5 to 16 columns 0.994 (1.024), over more 1.004.
+int seq_pause_bwd(const RnnGeom& g) { return g.B <= 4 ? 0 : 1; }
 
 // Does a pass gain by sequence launches?  One costs some 20 us more than a step's launch does (the cooperative queue, on both
 // sides), and saves on each step, the more so the more a step has to do.  Sequence / steps, of the time:
@@ -1519,7 +1528,7 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
     const SeqPlace place = seq_place(g, true, l == g.L - 1);
     p.B = g.B; p.H = g.H; p.T = g.T; p.ldo = g.D * g.H;
     p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
-    p.wait = options().rnn_wait; p.pause = SEQ_PAUSE_BWD; p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
+    p.wait = options().rnn_wait; p.pause = seq_pause_bwd(g); p.status = seq_status(g, ws); p.layer = (uint32_t)l + 1;
     ip.n = (size_t)g.T * seq_row(g, g.GH);
     ip.status = l == g.L - 1 ? p.status : nullptr;
     for (int dir = 0; dir < g.D; ++dir) {
