@@ -209,6 +209,17 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
   return !few || !(lo ? mfma_slab16_takes(g, bwd) : mfma_slab_takes(g, bwd));
 }
 
+// One-row windows on their own kernels.  In fp32 over more than 256 contraction channels only where the thin kernels do not take them
+// first: a workgroup walks the whole contraction there, which is a chain of 0.16 us per chunk of 16 channels and tap, and the thin
+// kernels' waves share it.  320 channels, us own / thin: backward to 320 over 1 x 200 frames, 21 taps 76 / 54 and over 4 x 700 (880 tiles) 80 / 169, forward to
+// 32 over 1 x 60, 9 taps 44 / 25, to 256 over 8 x 100, 5 taps 33 / 20 and over 16 x 300, 3 taps (1200 tiles) 40 / 111; forward of more than 9 taps,
+// which thin does not take, 83 / 239.  Of 970 random layers of 272 to 512 channels the choice is 1 % behind the better one in the geometric mean, at
+// worst 1.52.
+static bool row_on_thin(const ConvGeom& g, int dtype, bool bwd) {
+  return g.KH == 1 && g.KW > 1 && dtype == FLHIP_F32 && (bwd ? g.K : g.C) > 256 && thin_on(g, dtype, bwd, true) && mfma_thin_ws(g, dtype, bwd) > 0;
+}
+static bool tap1d_takes(const ConvGeom& g, int dtype, bool bwd) { return tap1d_on(dtype) && !row_on_thin(g, dtype, bwd); }
+
 static bool long_rows(const ConvGeom& g, int dtype, bool bwd, size_t ws_bytes) {
   if (algo_is(Options::ALGO_TAPPED)) return false;
   const size_t need = mfma_tapped_ws(g, dtype, bwd);
@@ -275,7 +286,7 @@ extern "C" size_t flhip_conv2d_workspace_bytes(const flhip_conv_desc* d, int pas
     const size_t b = is_lo16(d->dtype) ? mfma_pointwise16_lattice_ws(g, pass == FLHIP_CONV_BWD_DATA)
                                             : pass == FLHIP_CONV_BWD_DATA ? mfma_pointwise_split_ws(g, d->dtype, true) : 0;
     const bool bwd = pass == FLHIP_CONV_BWD_DATA;
-    size_t c = mfma_tap1d_conv_ws(g, d->dtype, bwd);
+    size_t c = row_on_thin(g, d->dtype, bwd) ? 0 : mfma_tap1d_conv_ws(g, d->dtype, bwd);
     if (bwd || thin_on(g, d->dtype, bwd, true) || thin_on(g, d->dtype, bwd, false)) c = std::max(c, mfma_thin_ws(g, d->dtype, bwd));
     // (the stacked-plane kernels: where their rule takes the geometry, and for every plane of at most 32 x 32 positions so
     // that a caller can try them by plan number; beyond that their copy of the input is tens of megabytes nobody asked for; fp32 copies the weights alone)
@@ -295,7 +306,7 @@ extern "C" int flhip_conv2d_fwd(const flhip_conv_desc* d, const void* x, const v
   hipStream_t s = as_stream(stream);
   if (!force_direct()) {
     int r = -1;
-    if (tap1d_on(d->dtype)) r = mfma_tap1d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
+    if (tap1d_takes(g, d->dtype, false)) r = mfma_tap1d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && tap2d_on(g, d->dtype, false)) r = mfma_tap2d_conv_fwd(g, d->dtype, x, w, bias, y, s, ws, ws_bytes);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_pwd16_conv_fwd(g, x, w, bias, y, s, d->dtype, ws, ws_bytes);
@@ -388,7 +399,7 @@ static int bwd_data_impl(const flhip_conv_desc* d, const void* dy, const void* w
   }
   if (!force_direct()) {
     int r = -1;
-    if (tap1d_on(d->dtype)) r = mfma_tap1d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
+    if (tap1d_takes(g, d->dtype, true)) r = mfma_tap1d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && tap2d_on(g, d->dtype, true)) r = mfma_tap2d_conv_bwd_data(g, d->dtype, dy, w, dx, s, ws, ws_bytes);
     if (r < 0 && !skip(Options::SKIP_CELLS)) r = mfma_cells_conv_bwd_data(g, d->dtype, dy, w, dx, s);
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !skip(Options::SKIP_PWDMA) && !algo_is(Options::ALGO_CONVERT))
@@ -560,7 +571,7 @@ extern "C" size_t flhip_conv2d_gathered_bytes(const flhip_conv_desc* d) {
   ConvGeom g;
   if (!d || make_geom(d, &g) != FLHIP_OK) return 0;
   // one-row windows (bf16 and fp32): the forward pass's channels-last rows (that family runs first where it applies)
-  if (tap1d_on(d->dtype) && mfma_tap1d_conv_ws(g, d->dtype, false) > 0) return mfma_tap1d_rows_bytes(g, d->dtype);
+  if (tap1d_takes(g, d->dtype, false) && mfma_tap1d_conv_ws(g, d->dtype, false) > 0) return mfma_tap1d_rows_bytes(g, d->dtype);
   return gathered_path(d) ? mfma_pointwise16_gathered_bytes(g) : 0;
 }
 
@@ -574,7 +585,7 @@ extern "C" int flhip_conv2d_bwd_filter_gathered(const flhip_conv_desc* d, const 
                 "conv2d_bwd_filter_gathered: this geometry's forward pass leaves no gathered input");
   const size_t need = flhip_conv2d_workspace_bytes(d, FLHIP_CONV_BWD_FILTER);
   FLHIP_REQUIRE(ws_bytes >= need && (ws || need == 0), "conv2d_bwd_filter_gathered: workspace too small");
-  const bool one_row = tap1d_on(d->dtype) && mfma_tap1d_conv_ws(g, d->dtype, false) > 0;
+  const bool one_row = tap1d_takes(g, d->dtype, false) && mfma_tap1d_conv_ws(g, d->dtype, false) > 0;
   const int r = one_row ? mfma_tap1d_wgrad(g, d->dtype, nullptr, dy, dw, db, ws, ws_bytes, as_stream(stream), gathered)
                         : mfma_pointwise16_wgrad(g, nullptr, dy, dw, db, ws, ws_bytes, as_stream(stream), gathered, d->dtype);
   if (r < 0) return fail(FLHIP_INVALID_ARGUMENT, "conv2d_bwd_filter_gathered: no kernel takes the gathered input of this geometry");

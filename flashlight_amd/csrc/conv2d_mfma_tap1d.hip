@@ -1167,6 +1167,10 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   if (rb >= (1ll << 31) || yb >= (1ll << 31)) return false;
   const int tiles = p.ktiles * p.ctiles;
   if (esz == 4 && tiles > 65535 / 2) return false;      // (two workgroups of the grid's second dimension to a tile)
+  // fp32 over more than 256 channels: from 800 million multiply-adds on; below, the general kernel's two launches are ahead of the copy of the
+  // rows, the tiles and their sums.  us general / here: 320 channels, 21 taps over 1 x 200 frames to 80 filters (110 million) 15 / 36, to 320 (430) 40 / 43,
+  // over 1 x 800 (1700) 70 / 64, 4 x 700 183 / 104.  Of 840 random layers 1 % behind the better one in the geometric mean, at worst 1.38.
+  if (esz == 4 && g.C > 256 && (long long)p.rows * g.OW * g.C * g.K * g.KW < 800000000) return false;
   const int PC = esz == 2 ? (g.sx == 1 ? 6 : 5) : t1ws_cells(g.sx), most = esz == 2 ? 150 * 1024 : 80 * 1024;
   const int cus = mfma_num_cus();
   // ranges of ceil(OW / tsplit) positions; false: the slab of one does not fit in LDS

@@ -35,6 +35,17 @@ def test_sequence_launches_take_no_workspace_of_their_own(I, H, L, bidir, mode, 
     assert 4 * held <= capi.lib().flhip_rnn_workspace_bytes(C.byref(d)) <= 4 * (held + 2 * 16 * G * H * widest) + (1 << 20)
 
 
+@pytest.mark.parametrize("C_,W,K,kw,left", [(320, 60, 32, 9, False), (320, 200, 320, 9, False), (320, 1500, 640, 9, True), (256, 60, 32, 9, True),
+                                            (320, 200, 320, 21, False), (320, 1500, 320, 21, True), (260, 1500, 320, 9, True)])
+def test_one_row_layers_that_leave_their_rows(C_, W, K, kw, left):
+    """fp32 layers of one-row windows leave their channels-last rows to the filter gradient, those of more than 256 channels where both passes have the
+    tiles and products for the kernels that use them; no room is asked for otherwise."""
+    d = capi.ConvDesc(1, C_, 1, W, K, 1, kw, 1, 1, 0, kw // 2, 1, 1, 1, capi.F32)
+    rows = capi.lib().flhip_conv2d_gathered_bytes(C.byref(d))
+    assert (rows > 0) == left
+    assert rows <= capi.lib().flhip_conv2d_workspace_bytes(C.byref(d), capi.CONV_FWD)
+
+
 def test_layer_geometry_is_kept_by_value():
     """Whatever can be an index is taken as one: arrays of one element, which have no hash, and tensors, whose hash is their identity."""
     import numpy as np

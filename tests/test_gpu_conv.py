@@ -670,6 +670,38 @@ def test_fp32_windows_in_three_parts(xs, ws, stride):
         assert err <= 2 * (n ** 0.5 + 1) * 2.0 ** -24, err
 
 
+@pytest.mark.parametrize("xs,k,kw,stride", [
+    ((1, 264, 1, 60), 32, 3, 1), ((1, 264, 1, 60), 272, 12, 1), ((1, 257, 1, 60), 257, 5, 1), ((1, 264, 1, 60), 272, 5, 2),     # few tiles; channels that the kernel for them does not take, strides
+    ((1, 264, 1, 1024), 512, 3, 1), ((1, 264, 1, 1024), 520, 3, 1),            # two tiles per compute unit, and one more
+    ((2, 272, 3, 300), 264, 9, 1), ((1, 320, 1, 140), 850, 21, 1), ((1, 320, 1, 139), 850, 21, 1)])      # 800 million multiply-adds, and fewer
+def test_fp32_one_row_windows_of_many_channels(xs, k, kw, stride):
+    """Layers of more than 256 contraction channels on either side of the rules that choose their kernels, the three passes against float64: within
+    twice sqrt(n) units of 2^-24 in the 2-norm; a filter gradient from what the forward pass left has the bits of the one without."""
+    import torch.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(k)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, w, b, ws = r(*xs), r(k, xs[1], 1, kw), r(k), (k, xs[1], 1, kw)
+    geo = dict(sx=stride, px=kw // 2)
+    y, gathered = fa.conv2d(x, w, b, keep_gathered=True, **geo)
+    dy = r(*y.shape)
+    dx = fa.conv2d_backward_data(dy, xs, w, **geo)
+    dw, db = fa.conv2d_backward_filter_bias(dy, x, ws, True, **geo)
+    if gathered is not None:
+        dw2, db2 = fa.conv2d_backward_filter_bias(dy, x, ws, True, gathered=gathered, **geo)
+        assert torch.equal(dw, dw2) and torch.equal(db, db2)
+    xd, wd, d = (t.double().cpu()[:, :, 0] if t.shape[2] == 1 else t.double().cpu() for t in (x, w, dy))
+    conv = F.conv2d if xs[2] > 1 else F.conv1d
+    kw_ = dict(stride=(1, stride), padding=(0, kw // 2)) if xs[2] > 1 else dict(stride=stride, padding=kw // 2)
+    wd = wd.view(k, xs[1], 1, kw) if xs[2] > 1 else wd
+    xd, wd = xd.requires_grad_(), wd.requires_grad_()
+    want = conv(xd, wd, b.double().cpu(), **kw_)
+    want.backward(d)
+    n = dy.numel() // k
+    for got, ref, m in ((y, want.detach(), xs[1] * kw), (dx, xd.grad, k * kw), (dw, wd.grad, n), (db, d.transpose(0, 1).reshape(k, -1).sum(1), n)):
+        got = got.double().cpu().view(ref.shape)
+        assert float((got - ref).norm() / ref.norm()) <= 2 * (m ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("xs,ws,stride", [((2, 80, 1, 300), (70, 80, 1, 9), 1), ((2, 80, 1, 300), (70, 80, 1, 9), 2), ((3, 64, 14, 14), (70, 64, 3, 3), 1)])
 def test_fp32_windows_in_three_parts_keep_what_bf16_cannot_hold(xs, ws, stride):
     """Infinities, NaN and values that round to infinity in bf16 reach the results that they reach in fp32, and no others."""
