@@ -14,14 +14,14 @@
 // walked in chunks of 16 positions through double-buffered LDS tiles stored
 // [row][position] with pitch 17.  What a column j means (channel offset, window
 // shift) is decoded once per kernel; every thread keeps the entries of its own
-// columns in registers: eight at most (with sixteen, and twice the tile, the kernel kept 162 registers in memory).  Padding
+// columns in registers: eight or ten at most (with sixteen, and twice the tile, the kernel kept 162 registers in memory).  Padding
 // is fetched as out-of-range buffer loads (zero).
 //
 // What bounds it: the gather's address arithmetic and single-element loads beside the fp32 matrix pipe (0.41 of its rate at 512
 // images, 5 x 5, 32 -> 64 channels over 14 x 14), and with few positions the chain of chunks, so that a split goes down to four of them.
 // With the partial sums' reduction, us (sixteen columns, splits of at least 256 positions / now): 5 x 5, 32 -> 64 channels over 14 x 14, 1 / 8 / 64 / 512
 // images 49 -> 13, 55 -> 16, 71 -> 38, 229 -> 164; 1 -> 32 over 28 x 28, 64 images 25 -> 18; 7 x 7 stride 2, 3 -> 64 over 224 x 224, 32 images
-// 144 -> 134.  Four chunks in registers instead of two: no gain; 8 waves and chunks of 32 positions: 45 at 64 images.
+// 144 -> 122.  Four chunks in registers instead of two: no gain; 8 waves and chunks of 32 positions: 45 at 64 images.
 #include "conv2d_mfma.h"
 
 namespace flhip {
@@ -31,9 +31,11 @@ constexpr int THREADS = 256;    // 4 waves
 constexpr int BM = MFMA_BM;
 constexpr int WKC = 16;         // positions per K-chunk
 constexpr int WKP = 17;         // LDS pitch of both tiles (positions contiguous)
-constexpr int WNT_MAX = 4;      // 16-column blocks per wave
-constexpr int WNB_MAX = 2 * WNT_MAX;
-constexpr int WCL_MAX = WNB_MAX;        // columns gathered per thread (16 per block / 16 lanes)
+// 16-column blocks per wave at most, of two waves.  Five where the columns are 9 or 10 blocks, which four make two tiles of (whose waves
+// have 3 and 2 blocks each, and dy passes twice), and the products at least 10^9: that many take it for the longer code.  us (up to
+// 8 blocks per wave / 4 / 5): 7 x 7 stride 2, 3 -> 64 over 224 x 224, 64 images 242 / 253 / 221, 16 images (1.9 10^9) 76 / 72 / 69, 8 (0.9)
+// 53 / 43 / 44; 3 x 3, 16 -> 1000 over 28 x 28, 59 images 203 / 234 / 188, 16 -> 64, 64 images (0.5) 39 / 28 / 32.
+constexpr int WNT = 4, WNT_WIDE = 5;
 constexpr int WAR = BM / 16;            // dy rows per thread
 
 struct WgradParams {
@@ -42,6 +44,7 @@ struct WgradParams {
   int groups, Cg, Kg;
   int ncols;        // Cg*KHW
   int NBW;          // 16-column blocks per workgroup tile
+  bool wide;        // up to 2 WNT_WIDE of them
   int ntiles_n, mtiles;
   int nsplit, pps;  // K-splits and positions per split (multiple of WKC)
   int Ptotal, OHW, HW;
@@ -53,12 +56,13 @@ struct WgradParams {
 
 constexpr int COL_INVALID = -(1 << 20);
 
-template <typename T>
+template <typename T, int WNT_MAX>
 __global__ void __launch_bounds__(THREADS, 2)
 wgrad_kernel(WgradParams p, const T* __restrict__ x, const T* __restrict__ dy,
              float* __restrict__ out /* dw when nsplit == 1, else partials */,
              float* __restrict__ db_out) {
   extern __shared__ float lds[];
+  constexpr int WCL_MAX = 2 * WNT_MAX;               // columns gathered per thread (16 per block / 16 lanes)
   const int BNW = p.NBW * 16;
   const int bstride = BNW * WKP, astride = BM * WKP;
   float* Bs = lds;                                   // [2][BNW][WKP]
@@ -238,7 +242,8 @@ wgrad_kernel(WgradParams p, const T* __restrict__ x, const T* __restrict__ dy,
     case 1: run(std::integral_constant<int, 1>{}); break;
     case 2: run(std::integral_constant<int, 2>{}); break;
     case 3: run(std::integral_constant<int, 3>{}); break;
-    default: run(std::integral_constant<int, 4>{}); break;
+    case 4: run(std::integral_constant<int, 4>{}); break;
+    default: if constexpr (WNT_MAX > 4) run(std::integral_constant<int, WNT_MAX>{}); break;
   }
 
   if (do_db && tid < min(m_lim, BM)) {
@@ -369,10 +374,12 @@ bool wgrad_plan(const ConvGeom& g, WgradParams* p) {
   p->groups = g.groups; p->Cg = g.Cg; p->Kg = g.Kg;
   p->ncols = g.Cg * p->KHW;
   const int nblocks = (p->ncols + 15) / 16;
-  p->ntiles_n = (nblocks + WNB_MAX - 1) / WNB_MAX;
+  p->Ptotal = g.N * g.OH * g.OW;
+  p->wide = nblocks > 2 * WNT && nblocks <= 2 * WNT_WIDE && (long long)p->Ptotal * p->ncols * g.Kg * g.groups >= 1000000000;
+  const int most = 2 * (p->wide ? WNT_WIDE : WNT);
+  p->ntiles_n = (nblocks + most - 1) / most;
   p->NBW = (nblocks + p->ntiles_n - 1) / p->ntiles_n;
   p->mtiles = (g.Kg + BM - 1) / BM;
-  p->Ptotal = g.N * g.OH * g.OW;
   p->OHW = g.OH * g.OW; p->HW = g.H * g.W;
   p->E = g.K * p->ncols;
   p->q16 = WKC / g.OW;
@@ -444,7 +451,7 @@ int mfma_conv_bwd_filter(const ConvGeom& g, int dtype, const void* x, const void
   float* out = p.nsplit > 1 ? static_cast<float*>(ws) : dw;
   const int rc_ = by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
-    auto kernel = wgrad_kernel<T>;
+    auto kernel = p.wide ? wgrad_kernel<T, WNT_WIDE> : wgrad_kernel<T, WNT>;
     if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), shmem)) return -1;
     hipLaunchKernelGGL(kernel, grid, dim3(THREADS), shmem, s, p, static_cast<const T*>(x),
                        static_cast<const T*>(dy), out, db);

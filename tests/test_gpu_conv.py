@@ -927,6 +927,29 @@ def test_static_filter_gradient_of_long_one_row_windows(xs, k, kw, stride):
         assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,win,stride,groups", [((64, 16, 40, 40), 72, 3, 1, 1), ((64, 16, 40, 40), 64, 3, 1, 1),          # 9 blocks of columns, 1.06 and 0.94 10^9 products
+                                                    ((40, 3, 113, 111), 65, 7, 2, 1), ((64, 34, 41, 40), 80, 3, 1, 2), ((300, 8, 30, 30), 27, 4, 1, 1)])     # 10, groups; 8
+def test_filter_gradient_on_tiles_of_nine_and_ten_blocks(xs, k, win, stride, groups):
+    """Column counts that one tile of the general kernel holds over many positions and two over few, against float64 within twice sqrt(n) units
+    of 2^-24, with and without a bias."""
+    import torch.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(*xs, generator=g, device="cuda")
+    ws, geo = (k, xs[1] // groups, win, win), dict(sx=stride, sy=stride, px=win // 2, py=win // 2, groups=groups)
+    dy = torch.randn(*fa.conv2d(x, torch.zeros(*ws, device="cuda"), None, **geo).shape, generator=g, device="cuda")
+    dw, db = fa.conv2d_backward_filter_bias(dy, x, ws, True, **geo)
+    assert torch.equal(dw, fa.conv2d_backward_filter_bias(dy, x, ws, False, **geo)[0])
+    want = torch.zeros(*ws, device="cuda", dtype=torch.float64)
+    for i in range(xs[0]):                       # one image at a time: its windows in 64 bits
+        cols = F.unfold(x[i:i + 1].double(), (win, win), padding=win // 2, stride=stride)[0].view(groups, -1, dy.shape[2] * dy.shape[3])
+        d = dy[i].double().view(groups, k // groups, -1)
+        for q in range(groups):
+            want[q * (k // groups):(q + 1) * (k // groups)] += (d[q] @ cols[q].t().contiguous()).view(-1, *ws[1:])
+    n = dy.numel() // k
+    for got, ref in ((dw.double(), want), (db.double(), dy.double().sum((0, 2, 3)))):
+        assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("xs,k,win,pad", [((2, 3, 256, 256), 64, 7, 3), ((5, 4, 41, 256), 32, 5, 2), ((3, 1, 30, 258), 64, 7, 2), ((40, 3, 64, 256), 64, 7, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_first_layer_filter_gradient_over_rows_of_128(xs, k, win, pad, dtype):
