@@ -699,7 +699,7 @@ __global__ void __launch_bounds__(64 * step_bwd_waves(NBT)) rnn_step_bwd(StepBwd
 // backward per step, where the products need 0.9 and 1.7).  Here the workgroups stay: each keeps its part of the
 // recurrent matrices in registers for all steps, and only the state (forward) or the pre-activation gradients (backward)
 // of a step travel between workgroups.  Per step, forward / backward: that LSTM 8.2 -> 2.9 / 12.4 -> 4.1 us; GRU of 1024
-// units, 64 columns 16.2 -> 5.0 / 29.7 -> 6.2 us (products 2.6, exchange of 64 / 192 KB per workgroup); LSTM of 320 units,
+// units, 64 columns 16.2 -> 5.0 / 29.7 -> 5.7 us (products 2.6, exchange of 64 / 192 KB per workgroup); LSTM of 320 units,
 // 5 columns 5.1 -> 1.8 us forward.  What bounds them: the products (fp32 matrix pipe), the exchange's trip and volume, and the
 // gates' math between two barriers (0.6 us of the LSTM's step).  Batch columns do not depend on each other: a cluster of workgroups
 // is one direction of 16 columns, and clusters never wait for one another.
