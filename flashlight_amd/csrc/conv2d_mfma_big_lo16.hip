@@ -43,10 +43,21 @@ __device__ __forceinline__ void bg_wait(bool more) {
   else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(FEW * STAGES) : "memory");
 }
 
+// Tile t of columns x rows tiles, in panels of `panel` columns (the last one maybe fewer), row after row within a panel.  The 32 tiles
+// that a die computes at a time then need 8 + 4 source tiles at once; column after column it was up to 32 + 1.
+// Measured, us (column after column / here), bf16: A B 4000 x 2000 -> 9998 174 / 172, its two backward products 408 / 396 together, of 4096 x
+// 4096 x 4096 285 / 275, forward 124 / 123, 6000 x 1024 -> 4001 67.2 / 65.7.  Panels of 4 to 8 columns are level, 16 are no better than none.
+__device__ __forceinline__ void bg_panel(int t, int columns, int rows, int panel, int& column, int& row) {
+  const int first = t / (panel * rows) * panel, width = min(panel, columns - first), r = t - first * rows;
+  row = r / width;
+  column = first + r - row * width;
+}
+
 struct BigParams {
   int Kc, Mo;           // contraction channels, result channels
   int P, Pc;            // positions and cells per plane
   int ncells, nstages, mtiles, ctiles;
+  int panel;            // channel tiles side by side (bg_panel)
   int halves;           // of the last tiles, computed as two of 128 channels each
   unsigned src_bytes, w_bytes, dst_bytes;
 };
@@ -222,8 +233,8 @@ __device__ __forceinline__ void big16_tile(const BigParams& p, int m0, int cell0
 }
 
 // The tiles in the order in which workgroups start: whole ones (256 channels) first, then `halves` of them as two of 128 channels each,
-// which fill the compute units' last round.  Consecutive workgroups go to the eight dies in turn; a die takes runs of channel
-// tiles that share a source tile.
+// which fill the compute units' last round.  Consecutive workgroups go to the eight dies in turn; a die takes runs of tiles
+// (bg_panel).
 template <typename E, bool BWD>
 __global__ void __launch_bounds__(BG_THREADS, 2)
 big16_conv_kernel(BigParams p, const E* __restrict__ src, const E* __restrict__ wgt, const float* __restrict__ bias,
@@ -232,11 +243,16 @@ big16_conv_kernel(BigParams p, const E* __restrict__ src, const E* __restrict__ 
   auto at = [&](int n, int i) { return (n >> 3) * (i & 7) + min(n & 7, i & 7) + (i >> 3); };       // the i-th of n tiles, run by run
   if (id < whole) {
     const int t = __builtin_amdgcn_readfirstlane(at(whole, id));
-    big16_tile<E, BWD, 256>(p, (t % p.mtiles) * 256, (t / p.mtiles) * BG_CELLS, src, wgt, bias, pos_bias, dst, addend);
+    int mt, ct;
+    bg_panel(t, p.mtiles, p.ctiles, p.panel, mt, ct);
+    big16_tile<E, BWD, 256>(p, mt * 256, ct * BG_CELLS, src, wgt, bias, pos_bias, dst, addend);
   } else {
-    const int h = __builtin_amdgcn_readfirstlane(at(2 * p.halves, id - whole)), t = whole + (h >> 1), m0 = (t % p.mtiles) * 256 + (h & 1) * 128;
+    const int h = __builtin_amdgcn_readfirstlane(at(2 * p.halves, id - whole)), t = whole + (h >> 1);
+    int mt, ct;
+    bg_panel(t, p.mtiles, p.ctiles, p.panel, mt, ct);
+    const int m0 = mt * 256 + (h & 1) * 128;
     if (m0 >= p.Mo) return;
-    big16_tile<E, BWD, 128>(p, m0, (t / p.mtiles) * BG_CELLS, src, wgt, bias, pos_bias, dst, addend);
+    big16_tile<E, BWD, 128>(p, m0, ct * BG_CELLS, src, wgt, bias, pos_bias, dst, addend);
   }
 }
 
@@ -258,7 +274,7 @@ int big16_go(const BigParams& p, const void* src, const void* w, const float* bi
 // zeros, written by the lanes that loaded them between the wait for their loads and the barrier.
 struct BigNtParams {
   int M, C, K, Kcells;
-  int nstages, mtiles, ctiles, dup;
+  int nstages, mtiles, ctiles, panel, dup;
   unsigned a_bytes, b_bytes;
 };
 constexpr int BN_A = 256, BN_B = 128, BN_STAGE = (BN_A + BN_B) * 128, BN_NS = 3;
@@ -272,10 +288,12 @@ big16_nt_kernel(BigNtParams p, const E* __restrict__ a, const E* __restrict__ b,
   char* const ring = reinterpret_cast<char*>(bg_ring);
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, fh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // runs of tiles that share a's rows on one die
+  // runs of tiles on one die
   const int tiles = p.mtiles * p.ctiles, id = blockIdx.x;
   const int t0 = __builtin_amdgcn_readfirstlane((tiles >> 3) * (id & 7) + min(tiles & 7, id & 7) + (id >> 3));
-  const int m0 = (t0 / p.ctiles) * BN_A, c0 = (t0 % p.ctiles) * BN_B;
+  int mt, ct;
+  bg_panel(t0, p.ctiles, p.mtiles, p.panel, ct, mt);
+  const int m0 = mt * BN_A, c0 = ct * BN_B;
   const intx4_t ars = pd_rsrc(a, p.a_bytes), brs = pd_rsrc(b, p.b_bytes);
 
   // ---- load roles: instruction wave + 8 k fills rows 8 (wave + 8 k) .. + 7 (the first AI: a's rows); lane -> row lane / 8, slot lane % 8
@@ -379,6 +397,12 @@ big16_nt_kernel(BigNtParams p, const E* __restrict__ a, const E* __restrict__ b,
 
 }  // namespace
 
+// equal panels of at most eight columns
+static int bg_panel_width(int columns) {
+  const int panels = (columns + 7) / 8;
+  return (columns + panels - 1) / panels;
+}
+
 // Whether the tiles here are the faster ones, and how many of them, the last, should be computed as two halves (< 0: the smaller
 // kernels).  In rounds of the smaller kernels, which compute a tile of 128 x 128 per unit and round: a round of whole tiles takes 2.8
 // (convolutions 3.0), one of at most 128 tiles in halves 2.0 (2.5); the medians over 32473 random products and layers are 2.3 to 2.9
@@ -408,6 +432,7 @@ int mfma_big16(int dtype, bool bwd, long long images, int Kc, int Mo, int P, con
   p.nstages = (Kc + BG_KC - 1) / BG_KC;
   p.ctiles = (p.ncells + BG_CELLS - 1) / BG_CELLS;
   p.mtiles = (Mo + 255) / 256;
+  p.panel = bg_panel_width(p.mtiles);
   p.halves = halves;
   return by_lo16(dtype, [&](auto* e_) {
     using E = FLHIP_T_OF(e_);
@@ -430,6 +455,7 @@ int mfma_big16_nt(int dtype, int M, int C, int K, const void* a, const void* b, 
   p.nstages = (p.Kcells + 7) / 8;
   p.mtiles = (M + BN_A - 1) / BN_A;
   p.ctiles = (C + BN_B - 1) / BN_B;
+  p.panel = bg_panel_width(p.ctiles);
   p.a_bytes = (unsigned)((long long)M * K * 2); p.b_bytes = (unsigned)((long long)C * K * 2);
   return by_lo16(dtype, [&](auto* e_) {
     using E = FLHIP_T_OF(e_);
