@@ -106,6 +106,7 @@ SYMBOLS = {
     "flhip_logsoftmax_fwd": (C.c_int, [_VP, _VP, C.c_int32, C.c_int32, C.c_int, _VP]),
     "flhip_logsoftmax_bwd": (C.c_int, [_VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int, _VP]),
     "flhip_cce_fwd": (C.c_int, [_VP, _VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int32, C.c_int, _VP]),
+    "flhip_cce_fwd_checked": (C.c_int, [_VP, _VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int32, C.c_int, C.POINTER(C.c_int32), _VP]),
     "flhip_cce_bwd": (C.c_int, [_VP, _VP, _VP, _VP, C.c_int32, C.c_int32, C.c_int, C.c_int32, C.c_int,
                                 _VP]),
     "flhip_rnn_param_count": (C.c_size_t, [_VP]),

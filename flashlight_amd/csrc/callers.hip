@@ -6,6 +6,8 @@
 //
 // Matrices are column-major like Flashlight tensors: element (r, c) of an R x C
 // matrix is at r + c*R.
+#include <atomic>
+
 #include "common.h"
 #include "conv2d.h"
 
@@ -580,26 +582,40 @@ logsoftmax_bwd_kernel(const T* __restrict__ dy, const T* __restrict__ y, T* __re
 // ---- categorical cross-entropy on log-probabilities (Functions.cpp:1078-1154) ----
 // stats[0] = sum over counted columns of -x[target, col], stats[1] = counted columns,
 // stats[2] = columns whose target is neither in [0, C) nor the ignore index,
-// stats[3] = stats[0] / stats[1] (the MEAN reduction).  One block, one round of latencies per 1024 columns;
-// columns are added in a fixed order.
+// stats[3] = stats[0] / stats[1] (the MEAN reduction).  One block; what bounds it is the trip to memory, target first, then its
+// element: CCE_AHEAD columns of a thread are fetched together (4000 columns of 9998 classes in bf16: 11.1 -> 9.1 us), and added
+// one after the other.  said, if not null, is host memory: 1 if stats[2] is 0, else 2.  It says nothing of other memory
+// (ordering the store behind the caches' content would write them back).
+constexpr int CCE_AHEAD = 4;
 template <typename T>
 __global__ void __launch_bounds__(1024)
 cce_fwd_kernel(const T* __restrict__ x, const int32_t* __restrict__ target, float* __restrict__ stats,
-               float* __restrict__ per_col, int Cn, int X, int ignore) {
+               float* __restrict__ per_col, int Cn, int X, int ignore, uint32_t* said) {
   __shared__ float red[16];
   float s = 0.f, cnt = 0.f, bad = 0.f;
-  for (int i = threadIdx.x; i < X; i += 1024) {
-    const int t = target[i];
-    float v = 0.f;
-    if (t == ignore) {
-    } else if (t < 0 || t >= Cn) {
-      bad += 1.f;
-    } else {
-      v = -ld(x, (size_t)i * Cn + t);
-      cnt += 1.f;
+  for (int i0 = threadIdx.x; i0 < X; i0 += 1024 * CCE_AHEAD) {
+    int t[CCE_AHEAD];
+    float e[CCE_AHEAD];
+#pragma unroll
+    for (int k = 0; k < CCE_AHEAD; ++k) t[k] = target[min(i0 + 1024 * k, X - 1)];
+#pragma unroll
+    for (int k = 0; k < CCE_AHEAD; ++k)
+      e[k] = ld(x, (size_t)min(i0 + 1024 * k, X - 1) * Cn + (t[k] < 0 || t[k] >= Cn ? 0 : t[k]));
+#pragma unroll
+    for (int k = 0; k < CCE_AHEAD; ++k) {
+      const int i = i0 + 1024 * k;
+      if (i >= X) break;
+      float v = 0.f;
+      if (t[k] == ignore) {
+      } else if (t[k] < 0 || t[k] >= Cn) {
+        bad += 1.f;
+      } else {
+        v = -e[k];
+        cnt += 1.f;
+      }
+      if (per_col) per_col[i] = v;
+      s += v;
     }
-    if (per_col) per_col[i] = v;
-    s += v;
   }
   s = block_sum<16>(s, red);
   cnt = block_sum<16>(cnt, red);
@@ -609,6 +625,7 @@ cce_fwd_kernel(const T* __restrict__ x, const int32_t* __restrict__ target, floa
     stats[1] = cnt;
     stats[2] = bad;
     stats[3] = s / cnt;
+    if (said) __hip_atomic_store(said, bad != 0.f ? 2u : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -1269,18 +1286,105 @@ extern "C" int flhip_logsoftmax_bwd(const void* dy, const void* y, void* dx, int
   return check_launch("logsoftmax_bwd");
 }
 
-extern "C" int flhip_cce_fwd(const void* logp, const int32_t* target, float* stats, float* per_column,
-                             int32_t classes, int32_t cols, int32_t ignore_index, int dtype,
-                             void* stream) {
+static int cce_fwd(const void* logp, const int32_t* target, float* stats, float* per_column, int32_t classes, int32_t cols,
+                   int32_t ignore_index, int dtype, uint32_t* said, void* stream) {
   FLHIP_REQUIRE(logp && target && stats, "cce: null argument");
   FLHIP_REQUIRE(classes > 0 && cols > 0, "cce: sizes must be positive");
   FLHIP_REQUIRE(dtype_ok(dtype), "cce: unknown dtype");
   by_dtype(dtype, [&](auto* t_) {
     using T = FLHIP_T_OF(t_);
     hipLaunchKernelGGL((cce_fwd_kernel<T>), dim3(1), dim3(1024), 0, as_stream(stream),
-                       (const T*)logp, target, stats, per_column, classes, cols, ignore_index);
+                       (const T*)logp, target, stats, per_column, classes, cols, ignore_index, said);
   });
   return check_launch("cce");
+}
+
+extern "C" int flhip_cce_fwd(const void* logp, const int32_t* target, float* stats, float* per_column,
+                             int32_t classes, int32_t cols, int32_t ignore_index, int dtype,
+                             void* stream) {
+  return cce_fwd(logp, target, stats, per_column, classes, cols, ignore_index, dtype, nullptr, stream);
+}
+
+// Words of host memory that a kernel answers in: one page for the process, one word (in a cache line of its own) per call
+// in flight.  A word whose call has failed is not used again: its kernel may still write it.
+namespace {
+class Answers {
+ public:
+  static Answers& get() {
+    static Answers* const a = new Answers;      // (never freed: a kernel of a failed call may outlive everything else)
+    return *a;
+  }
+  // a word set to 0, or null (no host memory, or as many calls in flight as there are words)
+  volatile uint32_t* take() {
+    uint64_t used = used_.load(std::memory_order_relaxed);
+    while (page_ && ~used) {
+      const int k = __builtin_ctzll(~used);
+      if (used_.compare_exchange_weak(used, used | 1ull << k, std::memory_order_acquire)) {
+        volatile uint32_t* const w = page_ + 16 * k;
+        *w = 0;
+        return w;
+      }
+    }
+    return nullptr;
+  }
+  void give(volatile uint32_t* w) { used_.fetch_and(~(1ull << ((w - page_) / 16)), std::memory_order_release); }
+
+ private:
+  Answers() {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, 64 * 64, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess)
+      page_ = static_cast<uint32_t*>(p);
+    else
+      (void)hipGetLastError();
+  }
+  uint32_t* page_ = nullptr;
+  std::atomic<uint64_t> used_{0};
+};
+}  // namespace
+
+// The host looks at the word itself: a copy of the counter and a wait for the stream came later, which the launches
+// behind the loss wait for: a first step of the MNIST network with 64 images 370 -> 345 us, repeated ones 306 -> 299; the tail of an acoustic
+// model, 4000 frames 957 -> 936 and 923 -> 917.
+extern "C" int flhip_cce_fwd_checked(const void* logp, const int32_t* target, float* stats, float* per_column,
+                                     int32_t classes, int32_t cols, int32_t ignore_index, int dtype, int32_t* out_of_range,
+                                     void* stream) {
+  FLHIP_REQUIRE(out_of_range, "cce: null argument");
+  const hipStream_t s = as_stream(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(s, &capture);
+  (void)hipGetLastError();
+  if (capture != hipStreamCaptureStatusNone)
+    return fail(FLHIP_RUNTIME_ERROR, "cce: the targets cannot be checked in a stream that is being captured");
+  volatile uint32_t* const word = Answers::get().take();
+  const int rc = cce_fwd(logp, target, stats, per_column, classes, cols, ignore_index, dtype, const_cast<uint32_t*>(word), stream);
+  if (rc != FLHIP_OK) {                  // (nothing has been launched)
+    if (word) Answers::get().give(word);
+    return rc;
+  }
+  if (!word) {
+    float bad = 0.f;
+    if (hipMemcpyAsync(&bad, stats + 2, sizeof(bad), hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+      return check_launch("cce (checking the targets)");
+    *out_of_range = bad != 0.f;
+    return FLHIP_OK;
+  }
+  // (the stream is asked now and then, so that a kernel that failed ends the wait)
+  for (uint64_t n = 1; *word == 0; ++n) {
+    __builtin_ia32_pause();
+    if (n % (1u << 14)) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    if (*word == 0) {
+      (void)hipGetLastError();
+      return fail(FLHIP_RUNTIME_ERROR, std::string("cce (checking the targets): ") + hipGetErrorString(e));
+    }
+  }
+  *out_of_range = *word == 2;
+  Answers::get().give(word);
+  return FLHIP_OK;
 }
 
 extern "C" int flhip_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx,

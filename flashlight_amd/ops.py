@@ -678,9 +678,10 @@ def categorical_cross_entropy(input, targets, reduction=REDUCE_MEAN, ignore_inde
     cols = t.numel()
     stats = torch.empty((4,), dtype=torch.float32, device=x.device)
     per = torch.empty((cols,), dtype=torch.float32, device=x.device) if reduction == REDUCE_NONE else None
-    capi.check(capi.lib().flhip_cce_fwd(_ptr(x), _ptr(t), _ptr(stats), _ptr(per), classes, cols,
-                                        ignore_index, _dtype_tag(x), _stream()))
-    if float(stats[2].item()) != 0.0:
+    bad = C.c_int32()
+    capi.check(capi.lib().flhip_cce_fwd_checked(_ptr(x), _ptr(t), _ptr(stats), _ptr(per), classes, cols,
+                                                ignore_index, _dtype_tag(x), C.byref(bad), _stream()))
+    if bad.value:
         raise ValueError("target contains elements out of valid range [0, num_categories) "
                          "in categorical cross entropy")
     if reduction == REDUCE_NONE:

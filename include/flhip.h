@@ -116,8 +116,9 @@ const char* flhip_last_error(void);
  * refuse to run when flhip_version() / 100 differs from FLHIP_VERSION / 100 (a layout change).
  * 200: flhip_rnn_desc gained dropout, seed_lo, seed_hi; flhip_bn_workspace_bytes never returns less
  * than 32 bytes per feature.  202: the *_plan entry points and FLHIP_DECLINED.  203: FLHIP_F16.  204: flhip_act_fwd / _bwd, flhip_glu_fwd / _bwd,
- * flhip_dropout, flhip_rownorm, flhip_weightnorm_fwd / _bwd, flhip_pad_fwd / _bwd, flhip_sgd_many, flhip_adam_many.  205: flhip_prelu_fwd / _bwd, FLHIP_ACT_LEAKY, FLHIP_ACT_THRESHOLD. */
-#define FLHIP_VERSION 206
+ * flhip_dropout, flhip_rownorm, flhip_weightnorm_fwd / _bwd, flhip_pad_fwd / _bwd, flhip_sgd_many, flhip_adam_many.  205: flhip_prelu_fwd / _bwd, FLHIP_ACT_LEAKY, FLHIP_ACT_THRESHOLD.
+ * 207: flhip_cce_fwd_checked. */
+#define FLHIP_VERSION 207
 int flhip_version(void);
 const char* flhip_arch(void);
 
@@ -557,6 +558,10 @@ int flhip_logsoftmax_bwd(const void* dy, const void* y, void* dx, int32_t classe
 int flhip_cce_fwd(const void* logp, const int32_t* target, float* stats,
                   float* per_column, int32_t classes, int32_t cols,
                   int32_t ignore_index, int dtype, void* stream);
+/* The same, and waits until the targets have been looked at: *out_of_range = whether there is one outside [0, classes)
+ * that is not ignore_index (stats[2] != 0).  Not for a stream that is being captured. */
+int flhip_cce_fwd_checked(const void* logp, const int32_t* target, float* stats, float* per_column, int32_t classes,
+                          int32_t cols, int32_t ignore_index, int dtype, int32_t* out_of_range, void* stream);
 int flhip_cce_bwd(const float* grad, const int32_t* target, const float* stats, void* dx,
                   int32_t classes, int32_t cols, int reduction, int32_t ignore_index,
                   int dtype, void* stream);

@@ -557,6 +557,59 @@ def test_cross_entropy(reduction):
         ops.categorical_cross_entropy(dev(logp), dev(np.full(300, 10, np.int32)))
 
 
+@pytest.mark.parametrize("cols", [1, 1023, 1025, 4096, 4097, 9001])
+def test_cross_entropy_over_whole_and_part_rounds_of_columns(cols):
+    """Columns a thread fetches together, the last of them missing; targets out of range anywhere among them are refused, also
+    with more calls in flight than there are threads on one stream, and what was counted before a refusal changes nothing after it."""
+    rng = np.random.default_rng(cols)
+    logp = -rng.random((cols, 7)).astype(np.float32)
+    target = rng.integers(-1, 7, cols).astype(np.int32)
+    target[0] = 3
+    per, s, mean, count, bad = flref.cce_fwd(logp, target)
+    x, t = dev(logp), dev(target)
+    got, stats = ops.categorical_cross_entropy(x, t, ops.REDUCE_NONE)
+    assert np.array_equal(host(got), per) and bad == 0
+    assert host(stats)[1] == count
+    # n additions of positive terms below one: n units of 2^-24 of the sum at most
+    assert abs(host(stats)[0] - np.sum(per.astype(np.float64))) <= cols * 2.0 ** -24 * max(s, 1e-30)
+    for at in {0, cols // 2, cols - 1}:
+        for wrong in (7, -2):
+            t2 = target.copy()
+            t2[at] = wrong
+            with pytest.raises(ValueError):
+                ops.categorical_cross_entropy(x, dev(t2))
+
+    import threading
+    failed = []
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for i in range(20):
+                    t2 = t.clone()
+                    if (i + k) % 3 == 0:
+                        t2[cols - 1] = 7
+                        try:
+                            ops.categorical_cross_entropy(x, t2)
+                            failed.append((k, i))
+                        except ValueError:
+                            pass
+                    else:
+                        _, st = ops.categorical_cross_entropy(x, t2)
+                        if host(st)[1] != count:
+                            failed.append((k, i, host(st)))
+        except Exception as e:      # noqa: BLE001 - the thread reports it
+            failed.append((k, repr(e)))
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not failed, failed[:4]
+
+
 def _mnist_params(rng):
     """Conv2D / Linear initialisation of the reference (nn/modules/Conv2D.cpp:177-194,
     Linear.cpp:62-74): Kaiming-uniform weights, bias U(+-sqrt(1/fanIn))."""
