@@ -27,7 +27,9 @@ MORE = [
     ((3, 5, 56, 56), (2, 2), (2, 2), (0, 0)),     # 2x2 stride 2: non-overlapping fast path
     ((2, 3, 6, 260), (2, 2), (2, 2), (0, 0)),     # ... rows wider than a wave
     ((2, 3, 7, 8), (2, 2), (2, 2), (0, 0)),       # odd height: generic kernels
-    ((2, 3, 8, 6), (2, 2), (2, 2), (0, 0)),       # W % 4 != 0: generic kernels
+    ((2, 3, 8, 6), (2, 2), (2, 2), (0, 0)),       # W % 4 != 0: a window per thread
+    ((1, 1, 2, 2), (2, 2), (2, 2), (0, 0)),       # ... one window
+    ((3, 5, 4, 1030), (2, 2), (2, 2), (0, 0)),    # ... rows wider than a workgroup, the last one not full
 ]
 ALL = GEOMS + MORE
 
@@ -60,7 +62,7 @@ def test_pool_f32_bit_exact(geom, mode):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("geom", [ALL[0], MORE[0], MORE[1], MORE[4], MORE[12], MORE[14]])
+@pytest.mark.parametrize("geom", [ALL[0], MORE[0], MORE[1], MORE[4], MORE[12], MORE[14], MORE[-3], MORE[-1]])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_pool_16bit_storage(geom, mode, dtype):
     xs, win, st, pd = geom
