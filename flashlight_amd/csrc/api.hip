@@ -93,6 +93,7 @@ static bool apply_option(Options& o, const char* name, const char* v) {
     else if (!strcmp(v, "always")) o.rnn_sequences = Options::SEQ_ALWAYS;
     else if (!strcmp(v, "never")) o.rnn_sequences = Options::SEQ_NEVER;
     else if (!strcmp(v, "refused")) o.rnn_sequences = Options::SEQ_REFUSED;
+    else if (!strcmp(v, "stacked")) o.rnn_sequences = Options::SEQ_STACKED;
     else return false;
     return true;
   }

@@ -296,9 +296,9 @@ struct Options {
                                   // matrix as one image's plane whatever its shape; 0: never; -1: by shape
   bool matmul_fp32_cores = false; // MATMUL_FP32_CORES: 16-bit products stay on the fp32 matrix instructions, fp32 ones too
   bool rnn_unfused = false;       // RNN_UNFUSED: two-kernel rnn steps
-  enum { SEQ_AUTO = 0, SEQ_ALWAYS, SEQ_NEVER, SEQ_REFUSED };
-  int rnn_sequences = SEQ_AUTO;   // RNN_SEQUENCES = auto | always (sequence launches wherever the kernels apply) | never | refused (tried wherever
-                                  // they apply, as if the runtime refused each of them)
+  enum { SEQ_AUTO = 0, SEQ_ALWAYS, SEQ_NEVER, SEQ_REFUSED, SEQ_STACKED };
+  int rnn_sequences = SEQ_AUTO;   // RNN_SEQUENCES = auto | always (sequence launches, one per layer, wherever the kernels apply) | never | refused (tried
+                                  // wherever they apply, as if the runtime refused each of them) | stacked (as always, but stacked layers in one launch wherever they can be)
   int rnn_wait = 1 << 22;         // RNN_WAIT: loads after which a wait inside a sequence launch gives up; negative: the first workgroup of every
                                   // cluster gives up at its first wait
   bool tap2d_all = false;         // TAP2D_ALL: the kernel for 3x3 windows over stacked planes takes every geometry it can, not only those of its measured rule

@@ -302,7 +302,8 @@ struct CellFwd {
 };
 
 // (The gate math below leaves no choice of fused or separate multiply-adds to the compiler, and the step kernels add in the
-// sequence kernels' order: hidden sizes that are multiples of 16 with at most 64 columns give the same bits captured and eager.
+// sequence kernels' order: hidden sizes that are multiples of 16 with at most 64 columns give the same bits captured and eager, stacked layers
+// of one direction apart (rnn_stack_fwd: their input products are added inside the steps).
 // The two-kernel steps, which others run on where a sequence launch is not made, add their products in another order.)
 // gate math of one (batch b, hidden h) element, in two halves so that a kernel can issue
 // the loads before it computes the recurrent projections rp (one per gate)
@@ -915,6 +916,160 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_fwd(SeqFwd p) {
   }
 }
 
+// Stacked layers of one direction in one launch: clusters of all layers run side by side, and a layer's step waits for the same step of
+// the layer below (its row of the exchange) as it does for its own step before.  So T + L - 1 steps follow each other instead
+// of L T, there is one cooperative launch instead of L, and the products between the layers are part of the steps: the recurrent
+// and the input matrix lie in registers side by side, and add to one tile (GRU, whose W_n x and R_n h stay apart: to one each).  The
+// lowest layer's projections are made before, as ever.
+// Forward, us, a launch per layer / one for all: LSTM of 320 units, 3 layers, 5 columns, over 25 steps 225 / 84, over 100 steps 600 / 215; of
+// 512 units, 2 layers, 16 columns over 50 steps 268 / 147; of 1024 units, 2 layers, 3 columns over 30 steps 224 / 190; of 256 units, 2
+// layers, 64 columns over 60 steps 289 / 167; GRU of 384 units, 2 layers, 64 columns over 40 steps 257 / 187.  The recurrent and the input
+// product have an accumulator each and the waves' sums are added in pairs: against 64 bits the outputs are off by (a launch per layer, whose
+// products between layers may run in three bf16 parts / one for all) 1.2e-7 / 1.0e-7 for the first of these, 2.4e-7 / 1.6e-7 for the second, 1.8e-7 /
+// 1.9e-7 for the GRU, 3.7e-7 / 2.3e-7 for tanh layers of 200 units over 200 steps.
+constexpr int STACK_LAYERS = 4;
+struct SeqStack {
+  struct Layer {
+    const float *xp, *W, *R, *bsum, *bRn;      // xp: the lowest layer's projections; W: the others' input matrix
+    float *HP, *CP, *GT, *RN, *out, *hy, *cy, *X;
+  } d[STACK_LAYERS];
+  int B, H, T, L;
+  int groups, nwg;
+  int cluster0;      // 0: one launch holds them all
+  int wait, pause;
+  uint32_t* status;
+};
+constexpr size_t stack_lds(int mode, int RT) { return (size_t)2 * SEQ_WAVES * (mode == RNN_GRU ? 2 : 1) * RT * 16 * 17 * sizeof(float); }
+
+template <int MODE, int HU, int NC>
+__global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_stack_fwd(SeqStack p) {
+  constexpr int G = gates_of(MODE), RT = (G * HU + 15) / 16, W = SEQ_WAVES;
+  constexpr bool APART = MODE == RNN_GRU;
+  constexpr int TILES = APART ? 2 * RT : RT;
+  extern __shared__ float seq_red[];      // [2][W][16 TILES][17]
+  const uint32_t status = *p.status;
+  const int cluster = blockIdx.x / p.nwg, h0 = (blockIdx.x - cluster * p.nwg) * HU;
+  const int layer = __builtin_amdgcn_readfirstlane(cluster / p.groups), b0 = (cluster - layer * p.groups) * SEQ_COLS;
+  const SeqStack::Layer q = p.d[layer];
+  const bool upper = layer > 0;
+  float* const HP = q.HP;
+  const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const SeqRow row(q.X, H, B, b0), below(upper ? p.d[upper ? layer - 1 : 0].X : q.X, H, B, b0);
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  float a[RT][NC][4], aw[RT][NC][4];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int k = (wave + W * i) * 16 + 4 * fg;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int r = rt * 16 + fr, gate = r / HU, h = h0 + r % HU;
+      float4 v = make_float4(0.f, 0.f, 0.f, 0.f), u = v;
+      if (gate < G && h < H && k < H) {
+        const size_t at = ((size_t)gate * H + h) * H + k;
+        v = *reinterpret_cast<const float4*>(q.R + at);
+        if (upper) u = *reinterpret_cast<const float4*>(q.W + at);
+      }
+      a[rt][i][0] = v.x; a[rt][i][1] = v.y; a[rt][i][2] = v.z; a[rt][i][3] = v.w;
+      aw[rt][i][0] = u.x; aw[rt][i][1] = u.y; aw[rt][i][2] = u.z; aw[rt][i][3] = u.w;
+    }
+  }
+  const int unit = tid % HU, col = tid / HU, ch = h0 + unit, cb = b0 + col;
+  const bool cell = tid < HU * SEQ_COLS && cb < B && ch < H;
+  const size_t BH = (size_t)B * H, e = (size_t)cb * H + ch;
+  CellFwd c{};
+  c.ldo = H;
+  CellFwdIn<MODE> in{};
+  float keep = 0.f, x0[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) x0[g] = 0.f;
+  if (cell) {
+    keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? HP[e] : 0.f;
+    in.bRn = MODE == RNN_GRU ? q.bRn[ch] : 0.f;
+    if (upper)
+#pragma unroll
+      for (int g = 0; g < G; ++g) x0[g] = q.bsum[(size_t)g * H + ch];
+  }
+  seq_drain();
+  const SeqLost lost{p.status, 1u, p.wait};
+  int dead = SeqLost(lost).begin(status, h0 == 0);
+  const int limit = lost.limit < 0 ? 1 << 22 : lost.limit;
+  const bool publish_last = layer + 1 < p.L;      // the layer above reads the last state too
+  for (int sv = 0; sv < T; ++sv) {
+    const int st = __builtin_amdgcn_readfirstlane(sv);
+    const __amdgpu_buffer_rsrc_t r = row.rsrc(st), rb = below.rsrc(st + 1);
+    uintx4_t v[NC], u[NC];
+    if (upper) seq_load(rb, below, wave, u);
+    if (cell) {
+      if (!upper)
+#pragma unroll
+        for (int g = 0; g < G; ++g) x0[g] = q.xp[((size_t)st * B + cb) * GH + (size_t)g * H + ch];
+      in.prev = keep;
+    }
+    if (st > 0) seq_pause(p.pause);
+    seq_load(r, row, wave, v);
+    floatx4_t acc[2 * RT];               // the recurrent products, the input's
+#pragma unroll
+    for (int rt = 0; rt < 2 * RT; ++rt) acc[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const float (&m)[RT][NC][4], const uintx4_t (&x)[NC], int to) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+        if ((wave + W * i) * 16 < H)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+              acc[to + rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[rt][i][k], __uint_as_float(x[i][k]), acc[to + rt], 0, 0, 0);
+    };
+    if (upper) {
+      dead = __builtin_amdgcn_readfirstlane(seq_wait(rb, below, wave, u, dead, limit));
+      multiply(aw, u, RT);
+    }
+    dead = __builtin_amdgcn_readfirstlane(seq_wait(r, row, wave, v, dead, limit));
+    seq_drain();
+    multiply(a, v, 0);
+    lost.tell(dead, acc);
+    if (!APART)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt] += acc[RT + rt];
+    float* red = seq_red + (st & 1) * (W * TILES * 16 * 17);
+#pragma unroll
+    for (int rt = 0; rt < TILES; ++rt)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) red[(wave * TILES * 16 + rt * 16 + 4 * fg + x) * 17 + fr] = acc[rt][x];
+    __syncthreads();
+    if (cell) {
+      float rp[G];
+      auto sum = [&](int row) __attribute__((always_inline)) {
+        float v[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) v[w] = red[(w * TILES * 16 + row) * 17 + col];
+#pragma unroll
+        for (int n = W / 2; n > 0; n /= 2)
+#pragma unroll
+          for (int w = 0; w < n; ++w) v[w] += v[w + n];
+        return v[0];
+      };
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        rp[g] = sum(g * HU + unit);
+        in.xp[g] = x0[g];
+        if (APART && upper) in.xp[g] += sum(RT * 16 + g * HU + unit);
+      }
+      c.hn = HP + (st + 1) * BH;
+      float* const pub = st + 1 < T || publish_last ? row.base + (st + 1) * row.step + row.at(ch, col) : nullptr;
+      c.cn = q.CP + (st + 1) * BH;
+      c.gt = q.GT + (size_t)st * B * GH;
+      c.rn = q.RN + st * BH;
+      c.out = q.out + (size_t)st * BH;
+      c.hy = st == T - 1 ? q.hy : nullptr;
+      c.cy = st == T - 1 ? q.cy : nullptr;
+      keep = cell_fwd_finish<MODE, true>(c, cb, ch, H, in, rp, false, pub);
+    }
+  }
+}
+
 struct SeqBwd {
   struct Dir {
     const float *gout, *dhy, *dcy, *R, *HP, *CP, *GT, *RN;
@@ -1038,14 +1193,14 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_seq_bwd(SeqBwd p) {
   if (cell && MODE == RNN_LSTM && q.dcx) q.dcx[e] = dc;
 }
 
-// What a recurrence finds in place: forward, per direction (blockIdx.y), the initial states and the summed biases (the GRU's
+// What a recurrence finds in place: forward, per direction or stacked layer (blockIdx.y), the initial states and the summed biases (the GRU's
 // n gate apart, whose recurrent bias stays inside r * (R_n h + b_Rn)), and for a sequence launch the initial state and
 // RNN_UNSET in the exchange; backward, RNN_UNSET in all of it.
 struct SeqInit {
   struct Dir {
     const float *hx, *cx, *bW, *bR;
     float *HP, *CP, *bsum, *X;
-  } d[2];
+  } d[STACK_LAYERS];
   size_t BH, n;       // elements of a state / of the exchange to be filled
   int B;
   int GH, H, mode;
@@ -1073,7 +1228,7 @@ __global__ void __launch_bounds__(256) rnn_seq_init_kernel(SeqInit p) {
     q.bsum[i] = (p.mode == RNN_GRU && i >= (size_t)2 * p.H) ? q.bW[i] : q.bW[i] + q.bR[i];
 }
 
-// one launch for all directions
+// one launch for all directions or stacked layers
 void launch_init(const SeqInit& p, int D, hipStream_t s) {
   const size_t most = std::max<size_t>(std::max<size_t>(p.n / 4, p.BH), p.GH);
   hipLaunchKernelGGL(rnn_seq_init_kernel, dim3((unsigned)std::min<size_t>((most + 255) / 256, 2048), D), dim3(256), 0, s, p);
@@ -1218,8 +1373,7 @@ bool seq_asked(const RnnGeom& g, bool bwd) {
          (asked != Options::SEQ_AUTO || seq_pays(g, bwd));
 }
 // ... and a stream that is not being captured (a cooperative launch is not recorded)
-bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
-  if (!seq_asked(g, bwd)) return false;
+bool seq_uncaptured(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -1227,6 +1381,7 @@ bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) {
   }
   return st == hipStreamCaptureStatusNone;
 }
+bool seq_applies(const RnnGeom& g, bool bwd, hipStream_t s) { return seq_asked(g, bwd) && seq_uncaptured(s); }
 
 // Where the exchange of a layer's sequence launch lies in the workspace, in floats (the layers use it in turn): in what the pass leaves idle
 // while the launch runs, so that it costs nothing but for the lower ones of stacked GRU layers, which need 3 H per position and direction where 2 H to 4 H are idle
@@ -1335,6 +1490,75 @@ int seq_fwd(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
     if (units == 8) return seq_fwd_hu<MODE, 8>(g, p, s);
   }
   return seq_fwd_hu<MODE, 16>(g, p, s);
+}
+
+// Hidden units per workgroup of rnn_stack_fwd, or 0: one direction, nothing between the layers, all their clusters in one
+// launch, both matrices' fragments in 128 registers; not ReLU layers, whose input products stay the fp32 instruction's (the same
+// sums in another order put its inputs on the other side of zero).  One launch is the faster one from three steps of a layer on (us, a launch
+// per step / one for all: 2 layers over 1 / 2 / 3 steps, LSTM of 512 units, 16 columns 39 / 36, 46 / 39, 53 / 42, GRU of 256 units, 40 columns 34
+// / 35, 43 / 37, 53 / 40; 3 layers over 1 step, LSTM of 320 units, 5 columns 51 / 38).
+int stack_units(const RnnGeom& g) {
+  const int asked = options().rnn_sequences;
+  if (options().rnn_unfused || (asked != Options::SEQ_AUTO && asked != Options::SEQ_STACKED)) return 0;
+  if (asked == Options::SEQ_AUTO && g.L * g.T < 3) return 0;
+  if (g.D != 1 || g.L < 2 || g.L > STACK_LAYERS || g.mode == RNN_RELU || g.dropout > 0.f || !seq_holds(g)) return 0;
+  const int clusters = g.L * ((g.B + SEQ_COLS - 1) / SEQ_COLS), nc = ((g.H + 15) / 16 + SEQ_WAVES - 1) / SEQ_WAVES;
+  const int chunks = nc <= 2 ? 2 : nc <= 4 ? 4 : 8;
+  for (int units = g.G == 1 ? 16 : 4; units <= 16; units *= 2)
+    if ((long long)clusters * ((g.H + units - 1) / units) <= mfma_num_cus()) return (g.G * units + 15) / 16 * chunks <= 16 ? units : 0;
+  return 0;
+}
+// where the exchanges of the layers lie, (T + 1) steps each (floats into the workspace, behind the projections and biases; 0: no room)
+size_t stack_place(const RnnGeom& g) {
+  const size_t at = ((size_t)g.T * g.B * g.GH + g.L * g.GH + 63) & ~(size_t)63;
+  return at + g.L * (g.T + 1) * seq_row(g, g.H) <= workspace_core(g) - 4 ? at : 0;
+}
+template <int MODE, int HU>
+int stack_fwd_hu(const RnnGeom& g, SeqStack& p, hipStream_t s) {
+  constexpr int RT = (gates_of(MODE) * HU + 15) / 16;
+  p.nwg = (g.H + HU - 1) / HU;
+  const size_t lds = stack_lds(MODE, RT);
+  const int nc = ((g.H + 15) / 16 + SEQ_WAVES - 1) / SEQ_WAVES, clusters = g.L * p.groups;
+  if (nc <= 2) return seq_launch(rnn_stack_fwd<MODE, HU, 2>, p, clusters, lds, s);
+  if (nc <= 4) return seq_launch(rnn_stack_fwd<MODE, HU, 4>, p, clusters, lds, s);
+  if constexpr (RT <= 2) return seq_launch(rnn_stack_fwd<MODE, HU, 8>, p, clusters, lds, s);
+  return FLHIP_DECLINED;
+}
+// all layers of a stack; FLHIP_DECLINED: not run
+template <int MODE>
+int forward_stack(const RnnGeom& g, const float* x, const float* w, const float* hx, const float* cx, float* y, float* hy, float* cy,
+                  float* res, float* ws, hipStream_t s) {
+  const int units = stack_units(g);
+  const size_t place = stack_place(g), TB = (size_t)g.T * g.B, act = TB * g.H;
+  if (!units || !place) return FLHIP_DECLINED;
+  const Reserve r = reserve_layout(g);
+  SeqInit ip{};
+  SeqStack p{};
+  p.B = g.B; p.H = g.H; p.T = g.T; p.L = g.L;
+  p.groups = (g.B + SEQ_COLS - 1) / SEQ_COLS;
+  p.wait = options().rnn_wait; p.pause = 2; p.status = seq_status(g, ws);
+  ip.BH = g.BH; ip.n = (size_t)(g.T + 1) * seq_row(g, g.H); ip.B = g.B; ip.GH = (int)g.GH; ip.H = g.H; ip.mode = g.mode;
+  ip.status = p.status;
+  for (int l = 0; l < g.L; ++l) {
+    const Offsets o = offsets(g, l);
+    float* const base = res + (size_t)l * r.per_pl;
+    float* const bsum = ws + TB * g.GH + l * g.GH;
+    p.d[l] = {ws, w + o.W, w + o.R, bsum, w + o.bR + 2 * g.H, base + r.hp, base + r.cp, base + r.gt, base + r.rn,
+              l == g.L - 1 ? y : res + r.acts + (size_t)l * act, hy + l * g.BH, cy && MODE == RNN_LSTM ? cy + l * g.BH : nullptr,
+              ws + place + l * ip.n};
+    ip.d[l] = {hx ? hx + l * g.BH : nullptr, cx ? cx + l * g.BH : nullptr, w + o.bW, w + o.bR, p.d[l].HP, p.d[l].CP, bsum, p.d[l].X};
+  }
+  launch_init(ip, g.L, s);
+  if (const int rc = mm(w + offsets(g, 0).W, x, ws, g.GH, TB, g.I, 1, 0, ip.d[0].bsum, s, scratch_of(g, ws), false)) return rc;
+  int rc = FLHIP_DECLINED;
+  if constexpr (MODE == RNN_LSTM || MODE == RNN_GRU) {
+    if (units == 4) rc = stack_fwd_hu<MODE, 4>(g, p, s);
+    else if (units == 8) rc = stack_fwd_hu<MODE, 8>(g, p, s);
+    else rc = stack_fwd_hu<MODE, 16>(g, p, s);
+  } else if constexpr (MODE == RNN_TANH) {
+    rc = stack_fwd_hu<MODE, 16>(g, p, s);
+  }
+  return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
 }
 
 template <int MODE>
@@ -1661,6 +1885,14 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
+  if (stack_units(g) && seq_uncaptured(s)) {
+    auto stack = [&](auto fn) {
+      return fn(g, static_cast<const float*>(x), wf, static_cast<const float*>(hx), static_cast<const float*>(cx), static_cast<float*>(y),
+                static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), s);
+    };
+    const int rc = g.mode == RNN_TANH ? stack(forward_stack<RNN_TANH>) : g.mode == RNN_LSTM ? stack(forward_stack<RNN_LSTM>) : stack(forward_stack<RNN_GRU>);
+    if (rc != FLHIP_DECLINED) return rc;
+  }
   bool seq = seq_applies(g, false, s) && ws_bytes >= seq_end(g, false) * sizeof(float);
   for (int l = 0; l < g.L; ++l) {
     const float* in = l == 0 ? static_cast<const float*>(x) : res + r.acts + (size_t)(l - 1) * act;

@@ -129,8 +129,9 @@ const char* flhip_arch(void);
  * tolerances under every setting; the switches only choose between kernels.
  *   CONV_ALGO = direct | gather | tapped | convert | auto    CONV_SKIP = bf16,gemm1x1,slab,tapped,strip,first,wgrad128,pwdma,wd32,tap1d,cells,tap2d,thin
  *   PW_PT = 2 | 4 | 8    PW16_PF = 0 | 1 | 2 | 4 | 8    CONV_STACK = 0 | 1 | 2 | 4 | 8    BN_ALGO = split | resident | auto
- *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = always | never | refused | auto (a layer's recurrence in one launch: wherever it can be |
- *                   not tried | as if the runtime refused the launch | where it is the faster one)
+ *   SLAB_WAVES = 0 | 4 | 8    RNN_SEQUENCES = always | never | refused | stacked | auto (a layer's recurrence in one launch: wherever it
+ *                   can be | not tried | as if the runtime refused the launch | wherever it can be, stacked layers of one direction in one launch
+ *                   together | where it is the faster one)
  *   RNN_WAIT = n (loads after which a wait inside such a launch gives up and its results become NaN; negative: the first
  *                   workgroups give up at once)
  *   PW16_NO_TAPS, TAPPED_NO_REORDER, MATMUL_VALU, MATMUL_FP32_CORES, RNN_UNFUSED, TAP2D_ALL = 1 | 0

@@ -151,6 +151,69 @@ def test_whole_sequences_without_room_for_their_exchange():
     assert count() == before and rel_l2(host(dx), host(want[0])) <= 1e-5 and rel_l2(host(dw), host(want[3])) <= 1e-5
 
 
+@pytest.mark.parametrize("mode,I,H,L,T,B,states,launches", [
+    # stacked layers in one launch: 4, 8 and 16 units per workgroup, two to four layers, last workgroups, chunks and column groups with some to spare
+    (flref.RNN_LSTM, 7, 20, 2, 6, 5, True, 1),
+    (flref.RNN_LSTM, 9, 320, 3, 5, 5, True, 1),            # 4 units
+    (flref.RNN_LSTM, 33, 516, 2, 4, 3, True, 1),           # 8 units, the last workgroup has 4; odd input width
+    (flref.RNN_LSTM, 8, 1024, 2, 3, 16, False, 1),         # the most registers
+    (flref.RNN_LSTM, 8, 256, 4, 3, 64, True, 1),           # 16 units, four layers of four column groups
+    (flref.RNN_LSTM, 8, 1024, 2, 3, 17, False, 2),         # two column groups: more clusters than compute units, a launch per layer
+    (flref.RNN_LSTM, 8, 512, 4, 2, 40, False, 4),
+    (flref.RNN_GRU, 12, 48, 3, 7, 17, True, 1),
+    (flref.RNN_GRU, 5, 256, 2, 4, 50, True, 1),
+    (flref.RNN_GRU, 6, 384, 2, 3, 70, True, 1),            # 16 units, 5 column groups
+    (flref.RNN_TANH, 8, 1020, 2, 3, 5, False, 1),
+    (flref.RNN_LSTM, 3, 16, 4, 8, 1, True, 1),             # one column
+    (flref.RNN_TANH, 3, 4, 4, 1, 1, True, 4),              # no room for the exchanges in what the pass leaves idle
+    (flref.RNN_RELU, 8, 64, 2, 6, 16, True, 2),            # a launch per layer
+    (flref.RNN_TANH, 8, 16, 5, 3, 4, True, 5),             # five layers: a launch per layer
+])
+def test_stacked_layers_in_one_launch(mode, I, H, L, T, B, states, launches):
+    count = capi.lib().flhip_rnn_sequence_launches
+    try:
+        capi.set_option("RNN_SEQUENCES", "stacked")
+        test_rnn_forward_backward(mode, I, H, L, False, T, B, states)
+        x = torch.randn(T, B, I, device="cuda")
+        w = torch.randn(ops.rnn_param_count(I, H, L, mode, False), device="cuda") / H ** 0.5
+        hx = torch.rand(L, B, H, device="cuda")
+        if mode == flref.RNN_GRU:
+            hx[0, 0, 0] = float("inf")      # (an infinite state that a product with zero would lose)
+        cx = torch.randn(L, B, H, device="cuda") if mode == flref.RNN_LSTM else None
+        before = count()
+        got = [t for t in ops.rnn(x, hx, cx, w, H, L, mode, False) if t is not None]
+        assert count() - before == launches
+        capi.set_option("RNN_SEQUENCES", "always")
+        want = [t for t in ops.rnn(x, hx, cx, w, H, L, mode, False) if t is not None]
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
+    for a, b in zip(got, want):             # outputs, last states and all that is kept for the backward pass: the same sums in another order
+        a, b = host(a.view(torch.float32)), host(b.view(torch.float32))
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+        ok = np.isfinite(b)
+        assert rel_l2(a[ok], b[ok]) <= 1e-5
+
+
+def test_a_wait_of_stacked_layers_that_gives_up_ends_in_not_a_number():
+    T, B, I, H, L = 5, 20, 8, 64, 3
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(T, B, I, device="cuda", generator=gen)
+    for mode in (ops.RNN_TANH, ops.RNN_LSTM, ops.RNN_GRU):
+        w = torch.randn(ops.rnn_param_count(I, H, L, mode, False), device="cuda", generator=gen) / H ** 0.5
+        try:
+            capi.set_option("RNN_SEQUENCES", "stacked")
+            want = ops.rnn(x, None, None, w, H, L, mode, False)[:2]
+            capi.set_option("RNN_WAIT", "-1")
+            y, hy, cy, _ = ops.rnn(x, None, None, w, H, L, mode, False)
+            assert all(bool(torch.isnan(t).all()) for t in (y, hy, cy) if t is not None)
+            capi.set_option("RNN_WAIT", None)
+            got = ops.rnn(x, None, None, w, H, L, mode, False)[:2]
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+        finally:
+            capi.set_option("RNN_WAIT", None)
+            capi.set_option("RNN_SEQUENCES", None)
+
+
 @pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
     (flref.RNN_LSTM, 12, 48, 3, True, 4, 20, True),        # the step kernels follow on the projections already made
     (flref.RNN_GRU, 12, 512, 2, False, 3, 33, True),
