@@ -148,22 +148,6 @@ static bool tap1d_on(int dtype) {
   return dtype == FLHIP_F32 || ((dtype == FLHIP_BF16 || dtype == FLHIP_F16) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT));
 }
 
-// Windows over stacked planes.  fp32: by the estimate of conv2d_mfma_tap_split.hip, but the forward pass of windows larger than 3x3
-// stays on the fp32 instruction: they are the layers of small convnets, whose ReLU and pool decide on its last bits, and the same
-// step's gradients hang on those.  (With the parts' sums, nearer to 64 bits as they are, the gradients of a step over 300 to 512 images of
-// 28 x 28 through two 5x5 layers were up to 3e-3 apart from these in the 2-norm, else 1e-6; the second layer over 64 / 512 images 38 / 145 us,
-// in parts 18 / 65.)
-// 16-bit storage: 3x3 windows over planes of at most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.
-// Measured (batch 64 / 32, forward): 7 x 7 x 512 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0
-// against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5 against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts both
-// rules.
-static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
-  if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
-  if (options().tap2d_all) return true;
-  if (dtype == FLHIP_F32) return (bwd || g.KH * g.KW <= 9) && mfma_tap2d_split_pays(g, bwd);
-  return g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048;
-}
-
 // 1x1 windows in fp32 with few tiles for their contraction: the thin kernels take about 8 us + 6 per 1000 source channels + 10 per million
 // weights (their copy), the 1x1 kernels 4 + 24 per 1000 source channels forward (3 + 21 over planes of whole 16-byte pieces) and
 // 5 + 31 (4 + 22) backward, where they do not cut the contraction, which the forward pass never does.  Measured, us, 1x1 kernels /
@@ -207,6 +191,25 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
   const int src = bwd ? g.K : g.C, dst = bwd ? g.C : g.K;
   const bool few = lo ? src <= 40 || (!bwd && src <= 64 && dst <= 32) : src <= 24 || (src <= 40 && tiles > cus);
   return !few || !(lo ? mfma_slab16_takes(g, bwd) : mfma_slab_takes(g, bwd));
+}
+
+// Windows over stacked planes.  fp32: by the estimate of conv2d_mfma_tap_split.hip, but the forward pass of windows larger than 3x3
+// stays on the fp32 instruction: they are the layers of small convnets, whose ReLU and pool decide on its last bits, and the same
+// step's gradients hang on those.  (With the parts' sums, nearer to 64 bits as they are, the gradients of a step over 300 to 512 images of
+// 28 x 28 through two 5x5 layers were up to 3e-3 apart from these in the 2-norm, else 1e-6; the second layer over 64 / 512 images 38 / 145 us,
+// in parts 18 / 65.)
+// 16-bit storage: 3x3 windows over planes of at most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.
+// Measured (batch 64 / 32, forward): 7 x 7 x 512 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0
+// against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5 against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts the
+// rules.  With 512 channels and more on both sides the slab kernel's 16 chunks take longer than these kernels also for fewer images, where the
+// thin kernels do not take them: us, slab / here, 7 x 7 x 512 12 / 20 / 31 images 49 / 36, 57 / 36, 57 / 36, backward 48 / 34, 56 / 34, 56 / 34; 6 x 6
+// x 512 16 / 31 images 49 / 36, 61 / 36; 14 x 14 x 512 6 / 20 / 31 / 48 images 57 / 36, 63 / 55, 65 / 66, 122 / 71 (256 channels: 8 % either way).
+static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
+  if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
+  if (options().tap2d_all) return true;
+  if (dtype == FLHIP_F32) return (bwd || g.KH * g.KW <= 9) && mfma_tap2d_split_pays(g, bwd);
+  if (g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048) return true;
+  return g.H * g.W <= 196 && g.groups == 1 && std::min(g.C, g.K) >= 512 && !thin_on(g, dtype, bwd, true);
 }
 
 // One-row windows on their own kernels.  In fp32 over more than 256 contraction channels only where the thin kernels do not take them

@@ -993,15 +993,18 @@ bool pw16_taps_plan(const ConvGeom& g, ConvGeom* c, bool wgrad = false) {
 // Forward through gathered taps (the gather writes 9/4 of the input for a 3x3 stride-2 window, the product
 // then runs as a 1x1 layer over C * T channels): where the product goes to the kernels that load straight to LDS
 // this beats the slab kernel's strided forward pass (whose loader moves 2.5 times the bytes per product there)
-// when that pass would need two rounds of workgroups or more: the stride-2 3x3 layers of ResNet-50 at batch 64
-// take 110 / 65 / 102 us on the slab kernel and 73 / 58 / 77 us this way; at batch 32 (one round, two for the
-// first) 37 / 33 / 55 against 42 / 45 / 67.
+// when that pass would need two rounds of workgroups or more, or 16 rounds times chunks of 32 channels (a chunk of a round takes
+// it 3.6 us): us, slab / this way, 256 channels to 14 x 14, 28 / 40 / 56 images 33 / 38, 61 / 42, 66 / 56; 512 to 7 x 7, 20 / 33 / 56 images 57
+// / 34, 113 / 46, 106 / 71; to 8 x 8 57 / 29, 114 / 50, 109 / 57.  Beyond 30 million gathered elements the copy costs what that gains
+// (256 channels to 16 x 16, 47 / 56 images 63 / 58, 62 / 65).  128 channels to 28 x 28, 20 / 33 / 47 images 34 / 31, 37 / 45, 54 / 61: on the slab
+// kernel up to two full rounds (its gather serves the filter gradient as well).
 bool pw16_taps_forward(const ConvGeom& g, const ConvGeom& c) {
   if (!((g.sy > 1 || g.sx > 1) && !(options().conv_skip & Options::SKIP_PWDMA) && c.H * c.W <= 1024 && c.K > 64 &&
         c.C % 32 == 0))
     return false;
   const long long slab = mfma_slab16_conv_fwd_workgroups(g);
-  return slab == 0 || slab >= 2 * (long long)mfma_num_cus();
+  const long long cus = mfma_num_cus(), chunks = (g.C + 31) / 32;
+  return slab == 0 || slab >= 2 * cus || ((slab + cus - 1) / cus * chunks >= 16 && (long long)g.N * c.C * c.H * c.W <= 30000000);
 }
 
 }  // namespace

@@ -613,6 +613,10 @@ bool plan(Slab16Params* p, size_t* shmem) {
   const int max_pos = 2 * NT_MAX * 16;
   if (p->DW > max_pos) return false;
   const int cus = mfma_num_cus();
+  // A round of workgroups costs, per chunk, as much before and beside its products (the chunk's weights, its rows, the barrier) as 32
+  // blocks of 16 positions take: 256 channels over 14 x 14 24 us + 0.75 per block, 128 over 28 x 28 15 + 0.35.  (Priced at one block,
+  // batches between two that fill the chip went in two or three rounds of small tiles: us, us here, 256 channels over 14 x 14, 33 / 40
+  // / 47 images 46 / 54 / 82, 34 / 32 / 36; 128 over 28 x 28, 33 / 47 images 33 / 36, 21 / 24; 64 over 64 x 64, 20 / 56 images 43 / 66, 16 / 40.)
   int best_r = 0;
   double best_cost = 1e30;
   for (int R = 1; R <= p->DH && R * p->DW <= max_pos; ++R) {
@@ -623,7 +627,7 @@ bool plan(Slab16Params* p, size_t* shmem) {
     const long long tiles = (long long)p->N * ((p->DH + R - 1) / R) * p->mtiles * p->groups;
     const long long rounds = (tiles + cus - 1) / cus;
     const int nb = (R * p->DW + 15) / 16;
-    const double cost = (double)rounds * ((nb + 1) / 2 + 0.5);
+    const double cost = (double)rounds * ((nb + 1) / 2 + 16);
     if (cost < best_cost - 1e-9) {
       best_cost = cost;
       best_r = R;

@@ -1629,3 +1629,40 @@ def test_backward_passes_by_plan(shape, dtype):
     assert torch.equal(out, dx0)
     assert L.flhip_conv2d_bwd_data_plan(C.byref(cd), P(dyd), P(wd), P(out), P(ws), nws, nd, S) == capi.INVALID_ARGUMENT
     assert L.flhip_conv2d_plan_name(capi.CONV_BWD_DATA, nd) is None
+
+
+@pytest.mark.parametrize("xs,K,stride", [
+    ((33, 256, 12, 12), 256, 1),       # one round of workgroups over whole planes
+    ((23, 256, 14, 14), 200, 1),       # half planes; a last tile of result channels that is not full
+    ((47, 128, 28, 28), 128, 1),
+    ((20, 64, 64, 64), 64, 1),
+    ((13, 512, 7, 7), 512, 1),         # stacked planes: fewer positions than before, more tiles than the thin kernels take
+    ((6, 512, 14, 14), 520, 1),
+    ((20, 512, 16, 16), 512, 2),       # gathered taps within one round of the slab kernel
+    ((33, 256, 24, 24), 256, 2),       # ... within two
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_three_by_three_in_16_bit_storage_between_whole_rounds(xs, K, stride, dtype):
+    """Batches between those that fill the chip, where the choice of tiles and of kernels follows the number of rounds; against the
+    fp32 product of the same operands (one rounding per element: 2^-9 / 2^-12 of a value at most, and fp32 sums)."""
+    import torch.nn.functional as F
+    gen = torch.Generator(device="cuda").manual_seed(xs[0] + K)
+    N, Cc, H, W = xs
+    oh = (H - 1) // stride + 1
+    x = torch.randn(xs, generator=gen, device="cuda").to(dtype)
+    w = (torch.randn(K, Cc, 3, 3, generator=gen, device="cuda") / (9 * Cc) ** 0.5).to(dtype)
+    g = torch.randn(N, K, oh, oh, generator=gen, device="cuda").to(dtype)
+    geo = dict(sx=stride, sy=stride, px=1, py=1)
+    y, gathered = fa.ops.conv2d(x, w, None, keep_gathered=True, **geo)
+    dx = fa.ops.conv2d_backward_data(g, xs, w, **geo)
+    dw, _ = fa.ops.conv2d_backward_filter_bias(g, x, w.shape, False, gathered=gathered, **geo)
+    wf, tol = w.float().reshape(K, -1), 3e-3 if dtype == torch.bfloat16 else 4e-4
+    ry, rdx, rdw = torch.empty(y.shape, device="cuda"), torch.empty(xs, device="cuda"), torch.zeros(K, 9 * Cc, device="cuda")
+    for n in range(N):
+        u = F.unfold(x[n:n + 1].float(), 3, padding=1, stride=stride)[0]
+        gn = g[n].float().reshape(K, -1)
+        ry[n] = (wf @ u).reshape(K, oh, oh)
+        rdx[n] = F.fold((wf.t() @ gn)[None], (H, W), 3, padding=1, stride=stride)[0]
+        rdw += gn @ u.t()
+    rel = lambda a, b: float((a.float() - b).norm() / b.norm())
+    assert rel(y, ry) <= tol and rel(dx, rdx) <= tol and rel(dw.reshape(K, -1), rdw) <= 1e-5
