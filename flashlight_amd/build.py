@@ -55,6 +55,8 @@ HOST_LIB = os.path.join(LIBDIR, "libflhip_host.so")
 STEP_BENCH = os.path.join(LIBDIR, "flhip_step_bench")
 HOST_SOURCES = ["HipTensor.cpp", "HipAutogradExtension.cpp", "Functions.cpp", "Modules.cpp", "Optimizers.cpp", "Resnet.cpp",
                 "SequentialBuilder.cpp"]
+BIND = os.path.join(HERE, "bind", "flhip_torch.cpp")
+BIND_LIB = os.path.join(LIBDIR, "flhip_torch.so")
 TESTS_DIR = os.path.join(ROOT, "tests", "cpp")
 TESTS_BIN = os.path.join(TESTS_DIR, "bin")
 # test program -> links the CPU checker?
@@ -84,6 +86,25 @@ def build_host(verbose=True):
     if verbose:
         print("built", HOST_LIB, "and", STEP_BENCH)
     return HOST_LIB
+
+
+def build_bind(verbose=True):
+    """flhip_torch.so: the Python module through which ops.py reaches libflhip.so in one native call per operator."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi()), "-I" + os.path.join(ROOT, "include")]
+    for d in cpp_extension.include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", d]
+    cmd += ["-o", BIND_LIB, BIND, "-L" + LIBDIR, "-lflhip", "-L" + torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+            "-Wl,-rpath,$ORIGIN"]
+    subprocess.check_call(cmd)
+    if verbose:
+        print("built", BIND_LIB)
+    return BIND_LIB
 
 
 def build_tests(verbose=True):
@@ -120,7 +141,9 @@ def build(verbose=True):
         if _host_pass_notes:
             print("note: the x86-64 host pass of hipcc ignored the device-only feature flag "
                   "-packed-fp32-ops (%d notices); the gfx950 pass applies it" % _host_pass_notes)
-    build_host(verbose)
+    with ThreadPoolExecutor(max_workers=2) as ex:
+        for f in [ex.submit(build_host, verbose), ex.submit(build_bind, verbose)]:
+            f.result()
     return LIB
 
 

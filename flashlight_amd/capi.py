@@ -4,6 +4,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libflhip.so")
+BIND_PATH = os.path.join(_HERE, "lib", "flhip_torch.so")
 
 OK, INVALID_ARGUMENT, RUNTIME_ERROR, DECLINED = 0, 1, 2, 3
 F32, BF16, F16 = 0, 1, 2
@@ -153,6 +154,27 @@ def lib():
             f.argtypes = args
         _lib = h
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The module flhip_torch (bind/flhip_torch.cpp); there is no fallback when it has not been built."""
+    global _native
+    if _native is None:
+        if not os.path.exists(BIND_PATH):
+            raise RuntimeError(
+                "flashlight_amd: %s is missing; build it with "
+                "`python -m flashlight_amd.build`" % BIND_PATH)
+        lib()
+        import importlib.machinery
+        import importlib.util
+        loader = importlib.machinery.ExtensionFileLoader("flhip_torch", BIND_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("flhip_torch", loader))
+        loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def check(rc):

@@ -24,6 +24,17 @@ class PoolingMode(enum.IntEnum):
     AVG_EXCLUDE_PADDING = 2
 
 
+_native = None
+
+
+def _n():
+    """The native module, whose functions return None for what they leave to the code behind the call."""
+    global _native
+    if _native is None:
+        _native = capi.native()
+    return _native
+
+
 def derive_padding(in_size, filter_size, stride, pad, dilation=1):
     """fl::derivePadding (flashlight/fl/nn/Utils.cpp:87-100); pad == -1 is SAME."""
     if pad == -1:
@@ -44,6 +55,7 @@ def _dtype_tag(t):
 
 
 _TAG_OF = {torch.float32: capi.F32, torch.bfloat16: capi.BF16, torch.float16: capi.F16}
+_TYPE_INDEX = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}      # of the native module's astype_many
 
 
 def _dev(t, name):
@@ -114,6 +126,9 @@ def conv2d(input, weights, bias, sx=1, sy=1, px=0, py=0, dx=1, dy=1, groups=1, k
     keep_gathered: returns (output, gathered) - what the closure's payload carries to the backward pass:
     the gathered input that the forward pass of a strided bf16 layer leaves in its workspace (None for
     geometries that gather nothing), to be given to conv2d_backward_filter_bias(gathered=...)."""
+    out = _n().conv2d(input, weights, bias, sx, sy, px, py, dx, dy, groups, keep_gathered)
+    if out is not None:
+        return out
     x, w = _dev(input, "input"), _dev(weights, "weights")
     if x.dim() != 4 or w.dim() != 4:
         raise ValueError("conv2d: input and weights must have 4 dimensions")
@@ -142,6 +157,9 @@ def conv2d_backward_data(grad_output, input_shape, weights, sx=1, sy=1, px=0, py
     """AutogradExtension::conv2dBackwardData; only the input's shape is needed
     (onednn/Conv2D.cpp:285).  addend: a gradient the input already holds; the result is then
     addend + the pass's result (Variable::addGrad), in one pass where the kernel allows it."""
+    out = _n().conv2d_backward_data(grad_output, input_shape, weights, sx, sy, px, py, dx, dy, groups, addend)
+    if out is not None:
+        return out
     g, w = _dev(grad_output, "gradOutput"), _dev(weights, "weights")
     tag = _dtype_tag(g)
     _, ref, shape = _conv_plan(tuple(input_shape), w.shape, sx, sy, px, py, dx, dy, groups, tag)
@@ -167,6 +185,9 @@ def conv2d_backward_filter_bias(grad_output, input, weights_shape, want_bias, sx
     Gradients are fp32 (the master-weight precision) for both storage types.
     gathered: what conv2d(keep_gathered=True) returned for this layer (the payload); the pass then
     skips gathering the input again."""
+    out = _n().conv2d_backward_filter_bias(grad_output, input, weights_shape, want_bias, sx, sy, px, py, dx, dy, groups, gathered)
+    if out is not None:
+        return out
     g, x = _dev(grad_output, "gradOutput"), _dev(input, "input")
     tag = _dtype_tag(x)
     d, ref, shape = _conv_plan(x.shape, tuple(weights_shape), sx, sy, px, py, dx, dy, groups, tag)
@@ -215,6 +236,9 @@ def pool2d(input, wx, wy, sx, sy, px, py, mode=PoolingMode.MAX, train=True):
     window-relative index per output) is returned for MAX when train is set —
     the reference keeps the equivalent oneDNN workspace in its payload only when
     a payload exists (onednn/Pool2D.cpp:88-92,150-161)."""
+    out = _n().pool2d(input, wx, wy, sx, sy, px, py, mode, train)
+    if out is not None:
+        return out
     x = _dev(input, "input")
     s4 = _as4(x)
     d = _pool_desc(s4, wx, wy, sx, sy, px, py, mode, _dtype_tag(x))
@@ -233,6 +257,9 @@ def pool2d_backward(grad_output, input_shape, argmax, wx, wy, sx, sy, px, py,
                     mode=PoolingMode.MAX):
     """AutogradExtension::pool2dBackward.  The result has the type of
     gradOutput."""
+    out = _n().pool2d_backward(grad_output, input_shape, argmax, wx, wy, sx, sy, px, py, mode)
+    if out is not None:
+        return out
     g = _dev(grad_output, "gradOutput")
     s4 = (1,) * (4 - len(input_shape)) + tuple(input_shape)
     d = _pool_desc(s4, wx, wy, sx, sy, px, py, mode, _dtype_tag(g))
@@ -289,6 +316,10 @@ def batchnorm(input, weight, bias, running_mean, running_var, axes, train, momen
     Train mode: batch statistics; running_mean/running_var (fp32, updated in
     place) follow the rule documented at flhip_bn_fwd_train.  Inference: uses the
     running statistics and returns (output, None, None)."""
+    if train is False:
+        y = _n().batchnorm_infer(input, weight, bias, running_mean, running_var, axes, epsilon)
+        if y is not None:
+            return y, None, None
     x = _dev(input, "input")
     _, ref, Cc, _ = _bn_plan(x.shape, tuple(map(int, axes)), _dtype_tag(x))
     g, b = _f32vec(weight, Cc, "weight"), _f32vec(bias, Cc, "bias")
@@ -316,6 +347,9 @@ def batchnorm(input, weight, bias, running_mean, running_var, axes, train, momen
 
 def batchnorm_backward(grad_output, input, weight, save_mean, save_invstd, axes):
     """AutogradExtension::batchnormBackward -> (gradInput, gradWeight, gradBias)."""
+    out = _n().batchnorm_backward(grad_output, input, weight, save_mean, save_invstd, axes)
+    if out is not None:
+        return out
     g, x = _dev(grad_output, "gradOutput"), _dev(input, "input")
     if g.dtype != x.dtype or g.shape != x.shape:
         raise ValueError("batchnormBackward: gradOutput must match the input")
@@ -340,6 +374,9 @@ def batchnorm_relu(input, weight, bias, running_mean, running_var, axes, momentu
     the tensor -> (output, saveMean, saveInvStd).  residual is optional.  want_mask: through
     flhip_bn_act_fwd_train_mask, with a fourth result, the ReLU's mask as bytes (one per 4
     elements) for batchnorm_relu_backward; rows must hold a multiple of 4 elements."""
+    out = _n().batchnorm_relu(input, weight, bias, running_mean, running_var, axes, momentum, epsilon, residual, relu, want_mask)
+    if out is not None:
+        return out
     x = _dev(input, "input")
     _, ref, Cc, _ = _bn_plan(x.shape, tuple(map(int, axes)), _dtype_tag(x))
     g, b = _f32vec(weight, Cc, "weight"), _f32vec(bias, Cc, "bias")
@@ -373,6 +410,9 @@ def batchnorm_relu_backward(grad_output, input, output, weight, save_mean, save_
     gradient passes the ReLU mask of `output` (the forward result), then batchnormBackward.
     With `mask` (the fourth result of batchnorm_relu(want_mask=True)) the call goes through
     flhip_bn_act_bwd_mask and `output` is not read (it may be None)."""
+    out = _n().batchnorm_relu_backward(grad_output, input, output, weight, save_mean, save_invstd, axes, want_residual_grad, mask)
+    if out is not None:
+        return out
     g, x, y = _dev(grad_output, "gradOutput"), _dev(input, "input"), _dev(output, "output")
     if g.dtype != x.dtype or g.shape != x.shape:
         raise ValueError("batchnormReluBackward: gradOutput must match the input")
@@ -415,6 +455,10 @@ def astype(input, dtype):
 
 def astype_many(inputs, dtype):
     """The same conversion of a list of tensors of one type, in one launch per 64 of them."""
+    if dtype in _TAG_OF:
+        outs = _n().astype_many(inputs, _TYPE_INDEX[dtype])
+        if outs is not None:
+            return outs
     xs = [_dev(t, "input") for t in inputs]
     if not xs:
         return []
@@ -431,6 +475,9 @@ def astype_many(inputs, dtype):
 
 def relu(input):
     """fl::relu (Functions.cpp:1787-1789)."""
+    y = _n().relu(input)
+    if y is not None:
+        return y
     x = _dev(input, "input")
     y = torch.empty_like(x)
     capi.check(capi.lib().flhip_relu_fwd(_ptr(x), _ptr(y), x.numel(), _dtype_tag(x), _stream()))
@@ -438,6 +485,9 @@ def relu(input):
 
 
 def relu_backward(grad_output, input):
+    dx = _n().relu_backward(grad_output, input)
+    if dx is not None:
+        return dx
     g, x = _dev(grad_output, "gradOutput"), _dev(input, "input")
     if g.shape != x.shape or g.dtype != x.dtype:
         raise ValueError("relu backward: gradOutput must match the input")
@@ -569,6 +619,8 @@ def padding_backward(grad_output, dims, before, after):
 
 def sgd_step(params, grads, velocities, lr, momentum=0.0, weight_decay=0.0, nesterov=False):
     """fl::SGDOptimizer::step (optim/SGDOptimizer.cpp:38-68) over lists of tensors of one dtype, in place."""
+    if _n().sgd_step(params, grads, velocities, lr, momentum, weight_decay, nesterov):
+        return
     ps = [_dev(p, "param") for p in params]
     gs = [_dev(g, "grad") for g in grads]
     vs = [_dev(v, "velocity") for v in velocities] if velocities is not None else None
@@ -598,6 +650,9 @@ def adam_step(params, grads, first, second, lr, beta1, beta2, epsilon, weight_de
 def linear(input, weight, bias=None):
     """fl::linear (Functions.cpp:1255-1309): input [..., in] (Flashlight [in, ...]), weight
     torch [in, out] (Flashlight [out, in]), bias [out] or None -> [..., out]."""
+    y = _n().linear(input, weight, bias)
+    if y is not None:
+        return y
     x, w = _dev(input, "input"), _dev(weight, "weight")
     if w.dim() != 2 or x.shape[-1] != w.shape[0] or x.dtype != w.dtype:
         raise ValueError("linear: input [.., in] and weight [in, out] of one type expected")
@@ -619,6 +674,9 @@ def linear(input, weight, bias=None):
 def linear_backward(grad_output, input, weight, want_bias=True):
     """-> (gradInput, gradWeight, gradBias or None), the three branches of the gradient
     closure of fl::linear (Functions.cpp:1276-1303)."""
+    out = _n().linear_backward(grad_output, input, weight, want_bias)
+    if out is not None:
+        return out
     g, x, w = _dev(grad_output, "gradOutput"), _dev(input, "input"), _dev(weight, "weight")
     fin, fout = w.shape
     frames = x.numel() // fin
@@ -647,6 +705,9 @@ def linear_backward(grad_output, input, weight, want_bias=True):
 
 def log_softmax(input):
     """fl::logSoftmax over Flashlight dimension 0 (Functions.cpp:1044-1070): torch [..., classes]."""
+    y = _n().log_softmax(input)
+    if y is not None:
+        return y
     x = _dev(input, "input")
     y = torch.empty_like(x)
     classes = x.shape[-1]
@@ -656,6 +717,9 @@ def log_softmax(input):
 
 
 def log_softmax_backward(grad_output, output):
+    dx = _n().log_softmax_backward(grad_output, output)
+    if dx is not None:
+        return dx
     g, y = _dev(grad_output, "gradOutput"), _dev(output, "output")
     dx = torch.empty_like(y)
     classes = y.shape[-1]
