@@ -29,6 +29,9 @@ int mfma_slab_wgrad(const ConvGeom& g, int dtype, const void* x, const void* dy,
                     float* db, void* ws, size_t ws_bytes, hipStream_t s);
 size_t mfma_slab_wgrad_ws(const ConvGeom& g, int dtype);
 bool mfma_slab_wgrad_applies(const ConvGeom& g);
+// 3x3 windows of stride 1 and padding 1 in fp32, filter gradient in three bf16 parts (conv2d_mfma_wgrad_split.hip); no bias gradient
+int mfma_wgrad3_split(const ConvGeom& g, const float* x, const float* dy, float* dw, void* ws, size_t ws_bytes, hipStream_t s);
+size_t mfma_wgrad3_split_ws(const ConvGeom& g);
 bool mfma_slab_takes(const ConvGeom& g, bool bwd);      // windows of stride 1 whose operands are aligned
 int mfma_slab_conv_bwd_data(const ConvGeom& g, int dtype, const void* dy, const void* w, void* dx,
                             hipStream_t s);

@@ -268,12 +268,14 @@ static int static_scratch(void** out) {
 
 using namespace flhip;
 
-// bytes of workspace of the filter gradient: the largest of its plans, so any kernel can run; one_row: with the one-row windows' kernels
-static size_t filter_ws(const ConvGeom& g, int dtype, bool one_row) {
+// bytes of workspace of the filter gradient: the largest of its plans, so any kernel can run; one_row: with the one-row windows' kernels;
+// parts: with the 3x3 windows' in three bf16 parts
+static size_t filter_ws(const ConvGeom& g, int dtype, bool one_row, bool parts = true) {
   size_t a = std::max(mfma_conv_bwd_filter_ws(g, dtype), mfma_slab_wgrad_ws(g, dtype));
   if (is_lo16(dtype))
     a = std::max({a, mfma_wgrad16_ws(g), mfma_wgrad_dma16_ws(g), mfma_pointwise16_wgrad_ws(g), mfma_first16_wgrad_ws(g)});
   a = std::max(a, mfma_pointwise_wgrad_ws(g));
+  if (parts && dtype == FLHIP_F32) a = std::max(a, mfma_wgrad3_split_ws(g));
   return one_row ? std::max(a, mfma_tap1d_wgrad_ws(g, dtype)) : a;
 }
 
@@ -497,7 +499,7 @@ static int bwd_filter_direct(const flhip_conv_desc* d, const ConvGeom& g, const 
 }
 
 static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* dy, float* dw, float* db, void* ws,
-                           size_t ws_bytes, int plan, void* stream, bool one_row = true) {
+                           size_t ws_bytes, int plan, void* stream, bool one_row = true, bool parts = true) {
   FLHIP_REQUIRE(d && dy, "conv2d_bwd_filter: null argument");
   FLHIP_REQUIRE(dw || db, "conv2d_bwd_filter: nothing to compute");
   FLHIP_REQUIRE(!dw || x, "conv2d_bwd_filter: filter gradient needs the input");
@@ -527,7 +529,7 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
     return r < 0 ? FLHIP_DECLINED : r;
   }
   if (!force_direct()) {
-    const size_t need = filter_ws(g, d->dtype, one_row);
+    const size_t need = filter_ws(g, d->dtype, one_row, parts);
     FLHIP_REQUIRE(ws_bytes >= need && (ws || need == 0), "conv2d_bwd_filter: workspace too small");
     int r = -1;
     // (3x3 stride 1 with rows copied straight to LDS first: it also takes the 7x7 planes that would otherwise go
@@ -542,6 +544,8 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
     if (r < 0 && is_lo16(d->dtype) && !skip(SK_BF16) && !algo_is(Options::ALGO_CONVERT))
       r = mfma_wgrad16(g, x, dy, dw, db, ws, ws_bytes, s, d->dtype);
     if (r < 0 && dw && !db && d->dtype == FLHIP_F32 && !skip(SK_GEMM)) r = mfma_pointwise_parts_wgrad(g, x, dy, dw, ws, ws_bytes, s);
+    if (r < 0 && dw && !db && parts && d->dtype == FLHIP_F32 && !skip(SK_SLAB) && !algo_is(Options::ALGO_TAPPED))
+      r = mfma_wgrad3_split(g, static_cast<const float*>(x), static_cast<const float*>(dy), dw, ws, ws_bytes, s);
     if (r < 0 && !skip(SK_GEMM))
       r = mfma_pointwise_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, algo_is(Options::ALGO_TAPPED), s);
     if (r < 0 && !skip(SK_SLAB)) r = mfma_slab_wgrad(g, d->dtype, x, dy, dw, db, ws, ws_bytes, s);
@@ -604,7 +608,9 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   // (fp32 one-row windows of more than 256 channels: their own kernels' copy of the input and partial tiles, or, where those do not fit, the
   // general kernels, which ask for less)
   const bool one_row = !(d->dtype == FLHIP_F32 && g.C > 256) || filter_ws(g, d->dtype, true) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
-  const size_t need = filter_ws(g, d->dtype, one_row);
+  // (3x3 windows in three parts, likewise, where their partial tiles fit)
+  const bool parts = filter_ws(g, d->dtype, one_row) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
+  const size_t need = filter_ws(g, d->dtype, one_row, parts);
   if (need > (size_t)FLHIP_STATIC_SCRATCH_BYTES)
     return fail(FLHIP_INVALID_ARGUMENT,
                 "conv2d_bwd_filter_static: this geometry needs " + std::to_string(need) +
@@ -616,5 +622,5 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   if (rs != FLHIP_OK) return rs;
   // the same plan as the workspace entry point's given exactly `need` bytes (but for the windows above that do not fit): every
   // partial the reduction reads is written by this call first, so nothing has to be cleared
-  return bwd_filter_impl(d, x, dy, dw, db, ptr, need, -1, stream, one_row);
+  return bwd_filter_impl(d, x, dy, dw, db, ptr, need, -1, stream, one_row, parts);
 }

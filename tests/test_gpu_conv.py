@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import flashlight_amd as fa
+from flashlight_amd import capi
 from gpu_util import bf16_round, dev, host, round_to
 from oracle import flref
 from refmath import rel_l2
@@ -1666,3 +1667,50 @@ def test_three_by_three_in_16_bit_storage_between_whole_rounds(xs, K, stride, dt
         rdw += gn @ u.t()
     rel = lambda a, b: float((a.float() - b).norm() / b.norm())
     assert rel(y, ry) <= tol and rel(dx, rdx) <= tol and rel(dw.reshape(K, -1), rdw) <= 1e-5
+
+
+@pytest.mark.parametrize("xs,K", [
+    ((12, 64, 56, 56), 64),       # one row to a stage, seven cells (an odd number); one tile
+    ((16, 120, 48, 44), 125),     # rows whose last cell has four positions; tiles that are not full
+    ((14, 128, 28, 28), 100),
+    ((13, 190, 24, 20), 190),     # two rows to a stage, three cells; an odd number of rows
+    ((11, 256, 14, 14), 264),      # two cells
+    ((11, 448, 7, 7), 512),       # four rows to a stage, one cell
+    ((20, 512, 5, 8), 320),
+])
+def test_filter_gradient_of_3x3_windows_in_three_parts(xs, K):
+    """Against 64 bits: no further off than the fp32 instruction's kernel (which sums one rounding per four positions), and magnitudes and
+    values that three parts do not hold."""
+    import torch.nn.functional as F
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    N, Cc, H, W = xs
+    x = torch.randn(xs, generator=gen, device="cuda")
+    g = torch.randn(N, K, H, W, generator=gen, device="cuda")
+
+    def exact(x, g):
+        out = torch.zeros(K, 9 * Cc, dtype=torch.float64, device="cuda")
+        for n in range(N):
+            out += g[n].double().reshape(K, -1) @ F.unfold(x[n:n + 1].double(), 3, padding=1)[0].t()
+        return out.reshape(K, Cc, 3, 3)
+
+    def run(x, g):
+        return fa.conv2d_backward_filter_bias(g, x, (K, Cc, 3, 3), False, px=1, py=1)[0]
+    rel = lambda a, b: float((a.double() - b).norm() / b.norm())
+    want = exact(x, g)
+    got = run(x, g)
+    capi.set_option("CONV_SKIP", "slab")
+    try:
+        other = run(x, g)                         # (the general kernel, on the fp32 instruction)
+    finally:
+        capi.set_option("CONV_SKIP", None)
+    assert not torch.equal(got, other)
+    assert rel(got, want) <= 1e-6 and rel(got, want) <= 1.2 * rel(other, want), (rel(got, want), rel(other, want))
+    assert rel(run(x * 2.0 ** -115, g), want * 2.0 ** -115) <= 2e-6
+    x2 = x.clone()
+    x2[N - 1, Cc - 1, H - 1, W - 1] = float("inf")
+    ref = exact(x2, g)
+    got = run(x2, g)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert rel(got[fine], ref[fine]) <= 2e-6
+    assert torch.equal(run(torch.zeros_like(x), g), torch.zeros_like(got))
