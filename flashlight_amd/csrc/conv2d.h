@@ -81,7 +81,7 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
                 const float* bias_rows, hipStream_t s, void* ws, size_t ws_bytes);
 size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K);
 // the three products in fp32 (gemm_f32.hip), + bias[row] + addend (C's layout, may be C), their contraction cut into slices
-// where gemm32_ws_bytes() of workspace are there; -1 where rows are not whole 16-byte pieces or a tensor is too large, and,
+// where gemm32_ws_bytes() of workspace are there; -1 where rows that are no whole 16-byte pieces are better left to the others or a tensor is too large, and,
 // with `take`, where the workspace is short or take(M, N, K, more than one slice) is false.
 // fp32_sums (modes 0 and 1): on the fp32 instruction whatever the size, none in three bf16 parts.  For the products in front of a ReLU
 // whose choices the same step's gradients hang on (fl::linear's forward product, the input product of ReLU recurrent layers): the parts'

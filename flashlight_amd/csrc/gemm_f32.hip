@@ -271,9 +271,20 @@ constexpr Gemm32Tile G32_TILES[] = {{64, 64, 0.17, 1.07, 5}, {128, 64, 0.24, 1.4
 // waits behind.
 constexpr Gemm32Tile G32_FP32_TILES[] = {{128, 128, 1.0, 1.25, 6}, {128, 64, 0.5 / 0.93, 1.25, 6}, {64, 128, 0.5 / 0.93, 1.25, 6}, {64, 64, 0.25 / 0.85, 1.25, 6}};
 
+// Rows of no whole pieces: the kernels in three parts alone, which load what is contiguous along the rows one by one and ask a row's
+// last piece for its end.  us, the 1x1 layers' kernels on the fp32 instruction (which stay where the fp32 instruction's sums do) / here: A^T B 2000 x
+// 4000 x 9998 1681 / 856, 2000 x 1500 x 4001 263 / 150, 256 x 500 x 4001 188 / 18, 256 x 150 x 29 5.9 / 5.3; A B^T 9998 x 2000 x 4000 1631 / 921, 4001 x 768
+// x 1500 107 / 69, 1001 x 256 x 500 15 / 13, 130 x 768 x 150 8.9 / 8.7, but 29 x 768 x 150 7.9 / 8.9, 29 x 768 x 4000 16.2 / 17.9.
+bool gemm32_ragged(int mode, int M, int N, int K, bool fp32_sums) {
+  const double macs = (double)M * N * K;
+  if (fp32_sums || options().matmul_fp32_cores || K < KC) return false;
+  return mode == 2 ? macs >= 1e7 && (K <= 3000 || macs >= 2e8) : macs >= 1e6;
+}
+
 bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gemm32Plan* best) {
   const bool ak = mode == 1, bk = mode != 2;
-  if ((ak ? K : M) % 4 != 0 || (bk ? K : N) % 4 != 0) return false;      // rows of whole 16-byte pieces
+  const bool pieces = (ak ? K : M) % 4 == 0 && (bk ? K : N) % 4 == 0;      // rows of whole 16-byte pieces
+  if (!pieces && !gemm32_ragged(mode, M, N, K, fp32_sums)) return false;
   const long long ab = (long long)M * K * 4, bb = (long long)N * K * 4;
   if (ab >= (1ll << 31) || bb >= (1ll << 31) || (long long)M * N >= (1ll << 31) || M >= 1 << 22) return false;
   const int cus = mfma_num_cus(), nst = (K + KC - 1) / KC;
@@ -282,6 +293,7 @@ bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gem
   double best_cost = 1e30;
   for (const Gemm32Tile& t : whole ? G32_FP32_TILES : G32_TILES) {
     if (!whole && t.tm * t.tn > 64 * 64 && (K < KC || options().matmul_fp32_cores)) continue;
+    if (!pieces && t.tm * t.tn == 64 * 64) continue;
     const int mt = (M + t.tm - 1) / t.tm, nt = (N + t.tn - 1) / t.tn;
     for (int ns = 1; ns <= (sliced ? 16 : 1); ++ns) {
       if (ns > 1 && (nst / ns < 8 || ((size_t)M * N) % 4 != 0)) break;
@@ -301,7 +313,7 @@ bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gem
   best->p.nstages = nst;
   best->p.a_bytes = (unsigned)ab; best->p.b_bytes = (unsigned)bb;
   best->p.slice = (size_t)M * N;
-  return true;
+  return best_cost < 1e30;
 }
 
 template <int MODE, int TM, int TN>
@@ -335,6 +347,7 @@ int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C) |
        reinterpret_cast<uintptr_t>(addend)) % 16 != 0)
     return -1;
+  if (take && ((mode == 1 ? K : M) % 4 != 0 || (mode != 2 ? K : N) % 4 != 0)) return -1;      // (a thin product of such rows stays on the kernels for those)
   const bool can = ws != nullptr && (!bias || M % 4 == 0);
   if (!gemm32_plan(mode, M, N, K, can || take, fp32_sums, &pl)) return -1;
   const bool fits = can && ws_bytes >= (size_t)pl.slices * M * N * sizeof(float);

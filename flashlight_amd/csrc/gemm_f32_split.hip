@@ -104,7 +104,7 @@ struct SplitSide {
     for (int i = 0; i < (KROWS ? EL / 4 : 1); ++i) off[i] += by;       // (a row that is none: past every tensor all the same)
   }
   // the stage at byte offset `stage` of every row.  CHECKED: only its first `left` contraction indexes exist, the others read
-  // zero
+  // zero (a piece that the row ends in holds the next row's first values)
   template <bool CHECKED>
   __device__ __forceinline__ void load(float (&v)[EL], __amdgpu_buffer_rsrc_t rsrc, int stage, int left) const {
     if constexpr (KROWS) {
@@ -112,7 +112,7 @@ struct SplitSide {
       for (int i = 0; i < EL / 4; ++i) {
         const uintx4_t f = __builtin_amdgcn_raw_buffer_load_b128(rsrc, CHECKED && k0 >= left ? S_OOB : off[i], stage, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[4 * i + e] = __uint_as_float(f[e]);
+        for (int e = 0; e < 4; ++e) v[4 * i + e] = !CHECKED || k0 + e < left ? __uint_as_float(f[e]) : 0.f;
       }
     } else {
       const int at0 = off[0] + stage;          // (past the last row: still past every tensor)

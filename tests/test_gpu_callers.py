@@ -293,6 +293,25 @@ def test_matmul_fp32_in_three_parts_keeps_what_bf16_cannot_hold(mode):
         assert rel_l2(got[rows][ok], ref[rows][ok]) <= 2 * np.sqrt(K) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("mode,M,N,K,bias", [
+    (1, 129, 131, 61, False), (1, 260, 515, 33, True), (1, 133, 1000, 31, True), (1, 130, 700, 29, False),   # a last stage of 13, 1, 15, 13 contraction indexes
+    (1, 2052, 301, 18, False), (1, 256, 1300, 4001, True), (1, 255, 500, 2403, False), (1, 516, 132, 1999, True),   # two; in slices; N * M no multiple of 4; slices
+    (2, 1001, 257, 61, False), (2, 129, 1300, 64, False), (2, 4001, 70, 50, False), (2, 999, 1000, 19, False),      # A's columns, B's, both odd; C's columns not aligned
+    (2, 130, 1302, 2500, False), (2, 1002, 514, 1603, False), (2, 1001, 513, 1601, False)])                  # slices, the last two of odd lengths; no slices
+def test_matmul_fp32_of_rows_of_no_whole_pieces(mode, M, N, K, bias):
+    """A row's last piece holds the next row's first values: where those are infinities or NaN, only their own rows may show it."""
+    test_matmul_fp32_tiles(mode, M, N, K, bias)
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    rows, cols = [1, M // 2, M - 1], [2, N // 2, N - 1]
+    A[rows, 0], A[rows, 1], A[rows[1], 2], B[0, cols], B[1, cols[0]] = np.inf, np.nan, -np.inf, np.nan, np.inf
+    got = _matmul_through_c_abi(A if mode == 1 else A.T.copy(), B if mode == 2 else B.T.copy(), M, N, K, mode == 1, mode == 2, None,
+                                torch.float32).T.astype(np.float64)
+    assert np.isnan(got[rows]).all() and np.isnan(got[:, cols]).all()
+    A, B, got = np.delete(A, rows, 0).astype(np.float64), np.delete(B, cols, 1).astype(np.float64), np.delete(np.delete(got, rows, 0), cols, 1)
+    assert rel_l2(got, A @ B) <= 2 * (np.sqrt(K) + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M,N,K", [(1200, 3001, 1200), (2700, 1092, 20), (512, 2544, 1120), (1024, 300, 3136)])
 def test_matmul_forward_keeps_the_sums_of_the_fp32_instruction(M, N, K):
     """fl::linear's forward product, in front of a ReLU on whose choices the same step's gradients hang: the bits of the fp32
