@@ -217,9 +217,11 @@ static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
 // kernels' waves share it.  320 channels, us own / thin: backward to 320 over 1 x 200 frames, 21 taps 76 / 54 and over 4 x 700 (880 tiles) 80 / 169, forward to
 // 32 over 1 x 60, 9 taps 44 / 25, to 256 over 8 x 100, 5 taps 33 / 20 and over 16 x 300, 3 taps (1200 tiles) 40 / 111; forward of more than 9 taps,
 // which thin does not take, 83 / 239.  Of 970 random layers of 272 to 512 channels the choice is 1 % behind the better one in the geometric mean, at
-// worst 1.52.
+// worst 1.52.  In 16-bit storage up to 448 channels: 320 to 320, 11 taps over 200 frames 22.3 / 20.7, 21 taps over 60 31.2 / 29.2, 384 to
+// 80 33.2 / 29.7; but 512 to 512 over 200 frames, 11 taps 23.7 / 29.4, and strided windows, which thin does not take.
 static bool row_on_thin(const ConvGeom& g, int dtype, bool bwd) {
-  return g.KH == 1 && g.KW > 1 && dtype == FLHIP_F32 && (bwd ? g.K : g.C) > 256 && thin_on(g, dtype, bwd, true) && mfma_thin_ws(g, dtype, bwd) > 0;
+  const int src = bwd ? g.K : g.C;
+  return g.KH == 1 && g.KW > 1 && src > 256 && (dtype == FLHIP_F32 || src <= 448) && thin_on(g, dtype, bwd, true) && mfma_thin_ws(g, dtype, bwd) > 0;
 }
 static bool tap1d_takes(const ConvGeom& g, int dtype, bool bwd) { return tap1d_on(dtype) && !row_on_thin(g, dtype, bwd); }
 

@@ -23,7 +23,12 @@
 //
 // A workgroup (4 waves) owns 32 NB result positions (per phase; NB = 3, or 2 where the slab of 3
 // would not fit) of one sequence x 128 result channels; wave w owns channels 32 w .. 32 w + 31:
-// NB (2 NB) accumulator blocks of 32 x 32.
+// NB (2 NB) accumulator blocks of 32 x 32.  NB = 1: 64 positions x 64 channels, two waves to either half of both: for layers of so few
+// tiles that a compute unit has one, where a wave's walk over the taps is the whole time.  What that walk waits for is the
+// fragments' way through the vector cache (4 KB a stage and compute unit at some 40 bytes a clock), not the matrix pipe: a
+// stage takes 95 clocks with one block, 103 with two and 135 with three, of which 32, 64 and 96 are matrix instructions.  (Neither the
+// fragments of a stage next to each other for all four waves, nor touching them all for the die's second-level cache first, nor
+// reading positions three or six stages ahead changes it.)
 //   * The source rows the tile needs (its positions + the window's reach, every channel) are
 //     copied to LDS once, by buffer loads with the LDS modifier (no registers, no vector
 //     instructions); a row of the slab is its cells + 1 unused cell, which puts the eight
@@ -56,7 +61,9 @@ typedef __attribute__((address_space(3))) const uintx4_t* lds_cell_t;
 typedef const uintx4_t* lds_cell_t;
 #endif
 
-constexpr int T1_BM = 128;       // result channels per workgroup
+// a workgroup's four waves: blocks of 32 result channels x groups of positions, with NB blocks of 32 positions in a wave
+__host__ __device__ constexpr int t1_wm(int NB) { return NB == 1 ? 2 : 4; }
+__host__ __device__ constexpr int t1_positions(int NB) { return 32 * NB * 4 / t1_wm(NB); }
 constexpr int T1_KW = 32;        // taps of a window
 constexpr int T1_MAXTAPS = 64;   // taps over both phases, padding included
 constexpr int T1_OOB = (int)0x80000000;
@@ -292,9 +299,9 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   constexpr int CELL = Tap1Elem<T>::CELL;
   constexpr int ESZ = (int)sizeof(T);
   constexpr int CPR = 2 * KS + 1;               // cells per slab row
-  constexpr int TP = 32 * NB;
+  constexpr int WM = t1_wm(NB), TP = t1_positions(NB), BM = 32 * WM;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wp = wave / WM;
   const int ptile = __builtin_amdgcn_readfirstlane(blockIdx.x % p.ptiles);
   const int row = __builtin_amdgcn_readfirstlane(blockIdx.x / p.ptiles);
   const int mtile = blockIdx.y;
@@ -323,7 +330,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   constexpr int NS = DT * KS;
   static_assert(NS % 4 == 0 && NS % RW == 0 && KS >= 2, "fragment sets and the weight ring rotate with the unrolled group");
   const __amdgpu_buffer_rsrc_t wrs = make_rsrc(wf, p.w_bytes);
-  const int mblk = mtile * (T1_BM / 32) + wave;
+  const int mblk = mtile * WM + wm;
   int wpos = mblk * p.taps_total * KS * 1024;   // byte offset of the stage RW ahead of the group's first
   const int wlane = lane * 16;
   uintx4_t bq[RW];
@@ -342,7 +349,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   const int fr = lane & 31, fg = lane >> 5;
   lds_cell_t ap[NB];
 #pragma unroll
-  for (int b = 0; b < NB; ++b) ap[b] = (lds_cell_t)t1_slab + ((b * 32 + fr) * CPR + fg);
+  for (int b = 0; b < NB; ++b) ap[b] = (lds_cell_t)t1_slab + (((wp * NB + b) * 32 + fr) * CPR + fg);
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the slab (and the first weight fragments) have landed
   __syncthreads();
@@ -393,14 +400,14 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   if (NPH == 2) run(acc[NPH - 1], 1);
 
   // ---- results: element r of block b: result index o0 + 32 b + 8 (r / 4) + 4 fg + r % 4 of channel m
-  const int m = mtile * T1_BM + wave * 32 + fr;
+  const int m = mtile * BM + wm * 32 + fr;
   if constexpr (TD) {
     // Results through LDS (the slab is done with): every wave parks its 32 channels x 32 NB positions at storage size,
     // then threads walk positions (consecutive lanes = consecutive positions = consecutive addresses inside a plane's
     // row, and across row ends too: the zero column has no address) with the position's plane / row / column worked
     // out once per thread.  Position o of the sequence = row o / pitch (row 0 and every (pH + 1)-th after it are the
     // zero rows between the planes), column o % pitch (the last one of a row is the zero column).
-    constexpr int TPOS = 32 * NB;
+    constexpr int TPOS = TP, CG = 256 / TPOS;     // (CG: groups of threads, a channel each at a time)
     constexpr int SPT = TPOS + 4;                 // staging pitch (elements): 8-byte rows, lanes on distinct banks
     T* const stage = reinterpret_cast<T*>(t1_slab);
     const float bvt = (bias && m < p.Mo) ? bias[m] : 0.f;
@@ -409,22 +416,22 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        T* const at = stage + (wave * 32 + fr) * SPT + b * 32 + g4 * 8 + fg * 4;
+        T* const at = stage + (wm * 32 + fr) * SPT + (wp * NB + b) * 32 + g4 * 8 + fg * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) st(at, e, acc[0][b][4 * g4 + e] + bvt);
       }
     __syncthreads();
-    if (tid >= 2 * TPOS) return;
+    if (tid >= CG * TPOS) return;
     const int pos = tid % TPOS, cg = tid / TPOS;
     const int o = o0 + pos;
     const int P = p.tpitch, H1 = p.pH + 1;
     const int prow = o / P, col = o - prow * P;
     const int n = max(prow - 1, 0) / H1, h = max(prow - 1, 0) - n * H1;
     if (!(prow >= 1 && n < p.pN && h < p.pH && col < p.pW)) return;
-    const int mlim = min(T1_BM, p.Mo - mtile * T1_BM);
+    const int mlim = min(BM, p.Mo - mtile * BM);
     const size_t plane = (size_t)p.pH * p.pW;
-    T* const out = dst + ((size_t)n * p.Mo + mtile * T1_BM) * plane + (size_t)h * p.pW + col;
-    for (int c = cg; c < mlim; c += 2) out[(size_t)c * plane] = stage[c * SPT + pos];
+    T* const out = dst + ((size_t)n * p.Mo + mtile * BM) * plane + (size_t)h * p.pW + col;
+    for (int c = cg; c < mlim; c += CG) out[(size_t)c * plane] = stage[c * SPT + pos];
     return;
   }
   if (m >= p.Mo) return;
@@ -437,7 +444,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const int o = o0 + b * 32 + g4 * 8 + fg * 4;
+      const int o = o0 + (wp * NB + b) * 32 + g4 * 8 + fg * 4;
       float v[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -528,15 +535,22 @@ struct Tap1Plan {
 };
 
 // channels of the channels-last rows: the count padded to one the 16-bit convolution kernels are compiled for (the fp32 ones take
-// any whole chunk)
+// any whole chunk).  Compiled for every 32 up to 256, in 16-bit storage also for every 64 up to 512.  Before, 16-bit layers of more than
+// 256 channels ran on the general kernels (us, 320 -> 320 channels, 21 taps over 4 x 1200 frames, forward / backward / filter gradient
+// 76.7 / 77.4 / 417 -> 38.0 / 38.3 / 56, stride 2 363 / 247 / 216 -> 34.2 / 31.2 / 46), and 200 channels as 256 (3 x 1300 frames 31.9 -> 24.7).
 int tap1d_cs(int C, int esz) {
-  for (int c : {32, 64, 96, 128, 256})
-    if (C <= c) return c;
-  return esz == 4 && C <= 512 ? (C + 31) / 32 * 32 : 0;
+  if (esz == 4) {
+    for (int c : {32, 64, 96, 128, 256})
+      if (C <= c) return c;
+    return C <= 512 ? (C + 31) / 32 * 32 : 0;
+  }
+  return C <= 256 ? (C + 31) / 32 * 32 : C <= 512 ? (C + 63) / 64 * 64 : 0;
 }
 
-// taps per unrolled group 
-int dt_of(int KS) { return KS >= 16 ? 1 : KS >= 8 ? 2 : KS == 6 ? 2 : KS == 4 ? 4 : KS == 2 ? 8 : 0; }
+int t1_mtiles(int Mo, int NB) { return (Mo + 32 * t1_wm(NB) - 1) / (32 * t1_wm(NB)); }
+
+// taps per unrolled group: so that its stages are a multiple of four
+int dt_of(int KS) { return KS % 4 != 0 ? (KS == 2 ? 8 : 2) : KS >= 12 ? 1 : KS == 8 ? 2 : 4; }
 
 // bwd = false: forward; true: backward-data.
 bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
@@ -598,15 +612,15 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
     span = std::max(span, p.d0[q] + p.nreal[q]);
   }
   const int CPR = 2 * KS + 1;
-  // three blocks of positions per wave; two
-  // where the workgroups of two still fit the compute units at once, so that more of the chip works on
-  // shorter tiles (250 -> 250 channels over 7 x 1111 frames, 168 -> 252 workgroups, with the copies: 49.7 -> 46.2 us, stride 2
-  // 84 -> 126: 45.8 -> 41.6; but 12 x 900 frames, 240 -> 360: 47.5 -> 51.6)
-  p.mtiles = (Mo + T1_BM - 1) / T1_BM;
-  const bool few = (long long)p.rows * ((p.TO + 63) / 64) * p.mtiles <= mfma_num_cus();
+  // three blocks of positions per wave; two, or one with half the channels, where the workgroups still fit the compute units at once, so that
+  // more of the chip works on shorter tiles (us of a layer with its copies; three / two: 250 -> 250 channels over 7 x 1111 frames, 168
+  // and 252 workgroups, 49.7 / 46.2, stride 2, 84 and 126, 45.8 / 41.6; but 12 x 900 frames, 240 and 360, 47.5 / 51.6.  Two / one, 21 taps:
+  // 320 -> 320 over 12 x 254, 144 and 240 workgroups, 35.9 / 32.5, over 4 x 1200, stride 2, 37.1 / 34.2, backward 35.4 / 31.2, 250 -> 250 over 7 x
+  // 1111, stride 2, backward 34.7 / 31.1; one where it is more than the compute units: 7 x 1111, 504 workgroups, 38.0 / 43.9)
+  const auto wgs = [&](int nb) { return (long long)p.rows * ((p.TO + t1_positions(nb) - 1) / t1_positions(nb)) * t1_mtiles(Mo, nb); };
   pl->NB = 0;
-  for (int nb = few ? 2 : 3; nb >= 2 && !pl->NB; --nb) {
-    const int tp = 32 * nb;
+  for (int nb = wgs(1) <= mfma_num_cus() ? 1 : wgs(2) <= mfma_num_cus() ? 2 : 3; nb >= 1 && !pl->NB; --nb) {
+    const int tp = t1_positions(nb);
     if (pl->SS == 1) {
       p.SR = tp + span - 1;
       p.half = 0;
@@ -618,16 +632,17 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
     if (pl->lds_bytes <= 160 * 1024) pl->NB = nb;
   }
   if (!pl->NB) return false;
-  p.ptiles = (p.TO + 32 * pl->NB - 1) / (32 * pl->NB);
+  p.ptiles = (p.TO + t1_positions(pl->NB) - 1) / t1_positions(pl->NB);
+  p.mtiles = t1_mtiles(Mo, pl->NB);
   const long long rb = (long long)p.rows * p.TS * Cs * esz;
-  const long long wb = (long long)p.mtiles * (T1_BM / 32) * stored * KS * 1024;
+  const long long wb = (long long)p.mtiles * t1_wm(pl->NB) * stored * KS * 1024;
   const long long db = (long long)g.N * Mo * g.H * p.TOu * esz;
   if (rb >= (1ll << 31) || wb >= (1ll << 31) || db >= (1ll << 31)) return false;
   p.src_bytes = (unsigned)rb; p.w_bytes = (unsigned)wb; p.dst_bytes = (unsigned)db;
   pl->rows_bytes = ((size_t)rb + 255) & ~(size_t)255;
   pl->w_bytes = (size_t)wb;
   w.Mo = Mo; w.Cc = Cc; w.KS = KS; w.taps_total = stored; w.bwd = bwd ? 1 : 0;
-  w.Cw = g.C; w.KW = g.KW; w.mblocks = p.mtiles * (T1_BM / 32);
+  w.Cw = g.C; w.KW = g.KW; w.mblocks = p.mtiles * t1_wm(pl->NB);
   pl->DT = DT;
   pl->C = Cc; pl->H = g.H; pl->T = p.TS;
   return true;
@@ -641,6 +656,10 @@ int launch_conv(const Tap1Plan& pl, const T* xr, const uintx4_t* wf, const float
     hipLaunchKernelGGL(kernel, grid, dim3(256), pl.lds_bytes, s, pl.p, xr, wf, bias, dst);
     return check_launch("conv2d (one-row windows)");
   };
+  if (pl.NB == 1) {
+    if (pl.p.nph == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 1, 2, 1>);
+    return pl.SS == 2 ? go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 1>) : go(tap1d_conv_kernel<T, KS, DT, RW, 1, 1, 1>);
+  }
   if (pl.NB == 2) {
     if (pl.p.nph == 2) return go(tap1d_conv_kernel<T, KS, DT, RW, 1, 2, 2>);
     return pl.SS == 2 ? go(tap1d_conv_kernel<T, KS, DT, RW, 2, 1, 2>) : go(tap1d_conv_kernel<T, KS, DT, RW, 1, 1, 2>);
@@ -674,7 +693,14 @@ int run_conv(const ConvGeom& g, bool bwd, const void* src, const void* w, const 
     case 4: return launch_conv<T, 4, 4, 16>(pl, xr, wf, bias, out, s);
     case 6: return launch_conv<T, 6, 2, 12>(pl, xr, wf, bias, out, s);
     case 8: return launch_conv<T, 8, 2, 16>(pl, xr, wf, bias, out, s);
-    default: return launch_conv<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
+    case 10: return launch_conv<T, 10, 2, 20>(pl, xr, wf, bias, out, s);
+    case 12: return launch_conv<T, 12, 1, 12>(pl, xr, wf, bias, out, s);
+    case 14: return launch_conv<T, 14, 2, 14>(pl, xr, wf, bias, out, s);
+    case 16: return launch_conv<T, 16, 1, 16>(pl, xr, wf, bias, out, s);
+    case 20: return launch_conv<T, 20, 1, 20>(pl, xr, wf, bias, out, s);
+    case 24: return launch_conv<T, 24, 1, 24>(pl, xr, wf, bias, out, s);
+    case 28: return launch_conv<T, 28, 1, 14>(pl, xr, wf, bias, out, s);
+    default: return launch_conv<T, 32, 1, 16>(pl, xr, wf, bias, out, s);
   }
 }
 
@@ -716,26 +742,28 @@ bool tap2d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
   for (int i = 0; i < p.ntaps[0]; ++i) w.tapj[i] = (signed char)(i < 9 ? (bwd ? 8 - i : i) : -1);
   const int CPR = 2 * KS + 1;
   // three blocks of positions per wave; two where three would leave compute units without a workgroup
-  // (7 x 7 x 512 at batch 64: 172 workgroups of three blocks 43.0 / 40.9 us, 256 of two 41.3 / 39.1)
-  const int mt = (Mo + T1_BM - 1) / T1_BM;
+  // (7 x 7 x 512 at batch 64: 172 workgroups of three blocks 43.0 / 40.9 us, 256 of two 41.3 / 39.1); one with half the channels where those
+  // fit the compute units at once (two / one: 20 images 36.2 / 33.1, 8 x 8 x 512, 12 images 36.1 / 32.3, 7 x 7 x 256, 40 images 24.6 / 22.8)
   pl->SS = 1; pl->DT = DT;
-  pl->NB = (long long)((ts - P + 95) / 96) * mt < mfma_num_cus() ? 2 : 3;
-  p.SR = 32 * pl->NB + 2 * P + 2;
-  p.half = 0;
-  // the slab; the results are staged in the same memory afterwards (128 channels x 100 elements)
-  pl->lds_bytes = std::max((size_t)(((long long)p.SR * CPR + 63) / 64) * 1024, (size_t)T1_BM * (32 * pl->NB + 4) * esz);
+  const auto tiles = [&](int nb) { return (ts - P + t1_positions(nb) - 1) / t1_positions(nb); };      // (the last zero row holds no result)
+  pl->NB = tiles(1) * t1_mtiles(Mo, 1) <= mfma_num_cus() ? 1 : tiles(3) * t1_mtiles(Mo, 3) < mfma_num_cus() ? 2 : 3;
+  const int tp = t1_positions(pl->NB);
+  p.SR = tp + 2 * P + 2;
+  // the slab; the results are staged in the same memory afterwards
+  pl->lds_bytes = std::max((size_t)(((long long)p.SR * CPR + 63) / 64) * 1024, (size_t)32 * t1_wm(pl->NB) * (tp + 4) * esz);
   if (pl->lds_bytes > 160 * 1024) return false;
-  p.ptiles = (p.TS - P + 32 * pl->NB - 1) / (32 * pl->NB);      // (the last zero row holds no result)
-  p.mtiles = (Mo + T1_BM - 1) / T1_BM;
+  p.half = 0;
+  p.ptiles = (int)tiles(pl->NB);
+  p.mtiles = t1_mtiles(Mo, pl->NB);
   const long long rb = ts * Cs * esz;
-  const long long wb = (long long)p.mtiles * (T1_BM / 32) * p.taps_total * KS * 1024;
+  const long long wb = (long long)p.mtiles * t1_wm(pl->NB) * p.taps_total * KS * 1024;
   const long long db = (long long)g.N * Mo * g.H * g.W * esz;
   if (rb >= (1ll << 31) || wb >= (1ll << 31) || db >= (1ll << 31)) return false;
   p.src_bytes = (unsigned)rb; p.w_bytes = (unsigned)wb; p.dst_bytes = (unsigned)db;
   pl->rows_bytes = ((size_t)rb + 255) & ~(size_t)255;
   pl->w_bytes = (size_t)wb;
   w.Mo = Mo; w.Cc = Cc; w.KS = KS; w.taps_total = p.taps_total; w.bwd = bwd ? 1 : 0;
-  w.Cw = g.C; w.KW = 9; w.mblocks = p.mtiles * (T1_BM / 32);
+  w.Cw = g.C; w.KW = 9; w.mblocks = p.mtiles * t1_wm(pl->NB);
   pl->C = Cc; pl->H = g.H; pl->T = g.W;
   return true;
 }
@@ -748,6 +776,7 @@ int launch_conv2d(const Tap1Plan& pl, const T* xr, const uintx4_t* wf, const flo
     hipLaunchKernelGGL(kernel, grid, dim3(256), pl.lds_bytes, s, pl.p, xr, wf, bias, dst);
     return check_launch("conv2d (3x3 windows over stacked planes)");
   };
+  if (pl.NB == 1) return go(tap2d_conv_kernel<T, KS, DT, RW, 1>);
   return pl.NB == 2 ? go(tap2d_conv_kernel<T, KS, DT, RW, 2>) : go(tap2d_conv_kernel<T, KS, DT, RW, 3>);
 }
 
@@ -1167,6 +1196,13 @@ bool tap1d_wgrad_plan(const ConvGeom& g, int esz, Tap1WPlan* pl) {
   if (rb >= (1ll << 31) || yb >= (1ll << 31)) return false;
   const int tiles = p.ktiles * p.ctiles;
   if (esz == 4 && tiles > 65535 / 2) return false;      // (two workgroups of the grid's second dimension to a tile)
+  // 16-bit storage over more than 256 channels, the general kernels / here: 320 channels, 21 taps over 60 frames to 32 filters (13 million multiply-adds)
+  // 10.8 / 16.9, 384 to 80 over 200 (129 million) 16.3 / 21.5, over 4 x 300 (774) 52 / 29, 512 to 512, 11 taps over 60 (173) 20 / 27, over 200 (577) 32 /
+  // 30, 320 to 320 over 200 (225) 22.3 / 22.0, to 32 over 4 x 300 (135) 24 / 20.
+  if (esz == 2 && g.C > 256) {
+    const long long pos = (long long)p.rows * g.OW;
+    if (pos < 64 || pos * g.C * g.K * g.KW < (pos >= 512 ? 100000000 : 200000000)) return false;
+  }
   // fp32 over more than 256 channels: from 800 million multiply-adds on; below, the general kernel's two launches are ahead of the copy of the
   // rows, the tiles and their sums.  us general / here: 320 channels, 21 taps over 1 x 200 frames to 80 filters (110 million) 15 / 36, to 320 (430) 40 / 43,
   // over 1 x 800 (1700) 70 / 64, 4 x 700 183 / 104.  Of 840 random layers 1 % behind the better one in the geometric mean, at worst 1.38.

@@ -994,6 +994,41 @@ def test_one_row_windows_in_16_bit_storage_by_blocks_of_weights(xs, k, kw, strid
         assert bool(((got.double().cpu()[:, :, 0] - ref).abs() <= unit * ref.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("xs,k,kw,stride", [
+    ((2, 144, 1, 75), 70, 5, 1), ((2, 180, 1, 75), 33, 6, 2), ((3, 200, 2, 61), 130, 7, 1), ((1, 129, 1, 64), 64, 2, 2),            # one block a wave: 160, 192, 224 channels
+    ((10, 224, 1, 600), 130, 3, 1), ((20, 130, 1, 600), 130, 4, 1), ((10, 190, 1, 1203), 130, 4, 2), ((21, 220, 1, 1203), 129, 6, 2),   # two, three
+    ((3, 257, 1, 701), 160, 7, 1), ((3, 380, 1, 701), 130, 6, 1), ((3, 440, 1, 702), 161, 3, 1), ((2, 500, 1, 203), 96, 9, 1),      # 320, 384, 448, 512
+    ((2, 300, 1, 203), 290, 21, 2), ((2, 330, 2, 101), 96, 22, 2), ((2, 400, 1, 130), 40, 23, 2), ((2, 512, 1, 131), 512, 21, 2),
+    ((12, 320, 1, 700), 256, 3, 1), ((24, 320, 1, 700), 200, 2, 1), ((12, 512, 1, 700), 256, 4, 2), ((30, 450, 1, 450), 257, 3, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_one_row_windows_in_16_bit_storage_of_many_channels(xs, k, kw, stride, dtype):
+    """Every channel count the kernels are compiled for beyond 128, one, two and three blocks of positions to a wave, and the filter gradient:
+    against float64, one rounding per result of fp32 sums."""
+    import torch.nn.functional as F
+    from flashlight_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k + xs[1])
+    pad = kw // 2
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(k, xs[1], 1, kw, generator=g, device="cuda") / (xs[1] * kw) ** 0.5).to(dtype)
+    y = fa.conv2d(x, w, None, sx=stride, px=pad)
+    dy = torch.randn(*y.shape, generator=g, device="cuda").to(dtype)
+    dx = fa.conv2d_backward_data(dy, xs, w, sx=stride, px=pad)
+    dw, db = ops.conv2d_backward_filter_bias(dy, x, tuple(w.shape), True, sx=stride, px=pad)
+    to, xp, d2 = y.shape[-1], F.pad(x.double(), (pad, pad)), dy.double().transpose(0, 1).reshape(k, -1)
+    taps = [xp[..., j:j + stride * (to - 1) + 1:stride].transpose(0, 1).reshape(xs[1], -1) for j in range(kw)]
+    w64 = w.double()[:, :, 0]
+    want = sum(w64[:, :, j].contiguous() @ t for j, t in enumerate(taps)).view(k, xs[0], xs[2], to).transpose(0, 1)
+    wdx = torch.zeros_like(xp)
+    for j in range(kw):
+        wdx[..., j:j + stride * (to - 1) + 1:stride] += (w64[:, :, j].t().contiguous() @ d2).view(xs[1], xs[0], xs[2], to).transpose(0, 1)
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for got, ref in ((y, want), (dx, wdx[..., pad:pad + xs[3]])):
+        assert bool(((got.double() - ref).abs() <= unit * ref.abs() + 1e-4).all())
+    wdw, n = torch.stack([d2 @ t.t().contiguous() for t in taps], -1), d2.shape[1]
+    for got, ref in ((dw.double()[:, :, 0], wdw), (db.double(), d2.sum(1))):
+        assert float((got - ref).norm() / ref.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_row_windows_without_workspace(dtype):
     """One-row windows reach their kernels through channels-last rows and reordered weights in the workspace;
