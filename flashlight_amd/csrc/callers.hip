@@ -1033,8 +1033,20 @@ static bool thin_tn_on_gemm32(int M, int N, int K, bool slices) {
   return slices || mn % 4 == 0 || K <= 384 + mn / 200;
 }
 
+// Thin products in 16-bit storage: the 16-bit matrix instructions but for few rows of C over a short contraction.  us, the thin kernels (sums of widened
+// operands on the vector ALUs) / here: A * B 9998 x 74 x 512 58 / 8.4, 2000 x 1 x 2000 44 / 9.8, 1024 x 64 x 3136 50 / 12, 128 x 24 x 1200 18.6 / 9.1, 512 x 24 x
+// 512 9.1 / 7.8, 32 x 64 x 2000 17.5 / 9.6; 10 x 128 x 512 5.8 / 7.5, 32 x 64 x 128 5.4 / 6.2.
+static bool thin16_on_mfma(int M, int K) { return M > SR_MAX || K >= 1024; }
+// A^T * B 9998 x 128 x 512 89 / 10.8, 2000 x 74 x 2000 32 / 13.7, 1200 x 64 x 128 11.6 / 6.2, 256 x 1 x 256 9.3 / 7.3; 10 x 128 x 512 9.3 / 11.2, 512 x 8 x 29
+// 8.5 / 9.0.
+static bool thin16_tn_on_mfma(int M, int N, int K) { return M > 16 && (N > 16 || K >= 128); }
+
 extern "C" size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || (trans_a && trans_b)) return 0;
+  if (is_lo16(dtype) && !options().matmul_valu && !options().matmul_fp32_cores) {
+    if (N <= 128 && !trans_b && !(trans_a ? thin16_tn_on_mfma(M, N, K) : thin16_on_mfma(M, K))) return 0;
+    return mfma_gemm16_ws_bytes(dtype, trans_a ? 1 : trans_b ? 2 : 0, M, N, K);
+  }
   if (trans_b || dtype != FLHIP_F32 || options().matmul_valu) return flhip_matmul_workspace_bytes(M, N, K, trans_a, trans_b, dtype);
   const size_t need = gemm32_ws_bytes(trans_a ? 1 : 0, M, N, K, !trans_a);
   return !trans_a && N <= 128 && !thin_on_gemm32(M, N, K, need > 0) ? 0 : need;
@@ -1072,6 +1084,13 @@ int flhip::matmul(const void* A, const void* B, void* C, int M, int N, int K, in
                           !thin ? nullptr : trans_a ? thin_tn_on_gemm32 : thin_on_gemm32, fp32_sums);
     if (rc >= 0) return rc;
   }
+  // 16-bit storage: on the 16-bit matrix instructions where the shape allows (MATMUL_FP32_CORES keeps them on the fp32 ones)
+  const bool lo = is_lo16(dtype) && !(trans_a && trans_b) && !options().matmul_valu && !options().matmul_fp32_cores;
+  if (lo && (!thin || (trans_a ? thin16_tn_on_mfma(M, N, K) : thin16_on_mfma(M, K)))) {
+    const int rc = mfma_gemm16(dtype, trans_a ? 1 : trans_b ? 2 : 0, A, B, C, M, N, K, bias_rows, as_stream(stream),
+                               ws, ws_bytes);
+    if (rc >= 0) return rc;
+  }
   // the other thin products: the kernels made for them
   if (N <= 128 && !trans_b && !options().matmul_valu) {
     hipStream_t s = as_stream(stream);
@@ -1100,11 +1119,9 @@ int flhip::matmul(const void* A, const void* B, void* C, int M, int N, int K, in
     }
   }
   // the matrix-core kernels of the 1x1 convolutions take the three products fl::linear
-  // needs; the tiled vector-ALU kernel below covers the rest.  16-bit storage: on the 16-bit
-  // matrix instructions where the shape allows (MATMUL_FP32_CORES keeps them on the fp32 ones).
-  if (is_lo16(dtype) && !(trans_a && trans_b) && !options().matmul_valu && !options().matmul_fp32_cores) {
-    const int rc = mfma_gemm16(dtype, trans_a ? 1 : trans_b ? 2 : 0, A, B, C, M, N, K, bias_rows, as_stream(stream),
-                               ws, ws_bytes);
+  // needs; the tiled vector-ALU kernel below covers the rest.
+  if (lo && thin) {      // (a bias on A^T * B)
+    const int rc = mfma_gemm16(dtype, trans_a ? 1 : 0, A, B, C, M, N, K, bias_rows, as_stream(stream), ws, ws_bytes);
     if (rc >= 0) return rc;
   }
   if (dtype == FLHIP_F32 && !(trans_a && trans_b) && !options().matmul_valu) {

@@ -32,6 +32,7 @@
 // Positions are the rows of the instruction tile: a lane holds 4 consecutive positions of a
 // result channel; results go through LDS and leave as whole cells.
 #include <algorithm>
+#include <type_traits>
 
 #include "conv2d_mfma.h"
 #include "lds_direct.h"
@@ -529,6 +530,10 @@ struct PwdWgradParams {
   unsigned x_bytes, dy_bytes;
 };
 
+struct __attribute__((packed, aligned(4))) Words4 {
+  uint32_t v[4];
+};
+
 // DIRECT (matrix products: one slice): the tile leaves in the element type, at out16, with bias[column] added
 template <typename E, bool DIRECT>
 __global__ void __launch_bounds__(256, 1)
@@ -672,24 +677,45 @@ pwd16_wgrad_kernel(PwdWgradParams p, const E* __restrict__ x, const E* __restric
 #undef PWG_MULT
 #undef PWG_READ
 
-  // element r of acc[i][jj]: row m0 + wm*64 + i*32 + (r/4)*8 + fh*4 + r%4, column c0 + wn*64 + jj*32 + fr
-  float* o = out + (size_t)slice * (p.nsplit > 1 ? (size_t)p.E + p.Mo : 0);
+  // element r of acc[i][jj]: row m0 + wm*64 + i*32 + (r/4)*8 + fh*4 + r%4, column c0 + wn*64 + jj*32 + fr.  Through LDS (the ring is
+  // done with), so that a row leaves in pieces of 16 bytes: one 16-bit element per store and 64 stores a lane took 5 us of the products' 12.5
+  // (256 x 879 x 256 12.5 -> 7.2 us, 512 x 4000 x 128 11.9 -> 6.4, 513 x 300 x 512, odd rows, 14.6 -> 10.7; fp32 partial products level).
+  using Out = std::conditional_t<DIRECT, uint16_t, float>;
+  constexpr int PITCH = PWG_T + 16 / sizeof(Out), EL = 16 / sizeof(Out), LPR = PWG_T / EL;      // elements of a staged row; of a piece; lanes per row
+  Out* const tile = reinterpret_cast<Out*>(ring);
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj) {
-      const int c = c0 + wn * 64 + jj * 32 + fr;
-      if (c >= p.C) continue;
-      const float bv = (DIRECT && bias) ? bias[c] : 0.f;
+      const int cl = wn * 64 + jj * 32 + fr;
+      const float bv = (DIRECT && bias && c0 + cl < p.C) ? bias[c0 + cl] : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3);
-        if (m >= p.Mo) continue;
-        if (DIRECT) out16[(size_t)m * p.C + c] = Lo16<E>::narrow(acc[i][jj][r] + bv);
-        else o[(size_t)m * p.C + c] = acc[i][jj][r];
+        Out* const at = tile + (wm * 64 + i * 32 + (r >> 2) * 8 + fh * 4 + (r & 3)) * PITCH + cl;
+        if constexpr (DIRECT) *at = Lo16<E>::narrow(acc[i][jj][r] + bv);
+        else *at = acc[i][jj][r];
       }
     }
+  __syncthreads();
+  Out* o;
+  if constexpr (DIRECT) o = out16;
+  else o = out + (size_t)slice * (p.nsplit > 1 ? (size_t)p.E + p.Mo : 0);
+  const bool words = !DIRECT || (((reinterpret_cast<uintptr_t>(out16) >> 1) | p.C) & 1) == 0;      // every row starts on a 4-byte boundary
+  const int row0 = tid / LPR, piece = tid % LPR, width = min(PWG_T, p.C - c0);
+#pragma unroll 4
+  for (int row = row0; row < PWG_T; row += 256 / LPR) {
+    if (m0 + row >= p.Mo) break;
+    Out* const to = o + (size_t)(m0 + row) * p.C + c0;
+    const Out* const from = tile + row * PITCH;
+    if (words && (piece + 1) * EL <= width) *reinterpret_cast<Words4*>(to + piece * EL) = *reinterpret_cast<const Words4*>(from + piece * EL);
+    else if (words)
+      for (int e = piece * EL; e < width; ++e) to[e] = from[e];
+    else
+      for (int e = piece; e < width; e += LPR) to[e] = from[e];
+  }
 }
+
 
 bool pwd16_wgrad_plan(const ConvGeom& g, PwdWgradParams* p) {
   if (!(g.KH == 1 && g.KW == 1 && g.py == 0 && g.px == 0 && g.groups == 1 && g.sy == 1 && g.sx == 1 &&
@@ -777,15 +803,23 @@ int mfma_pwd16_wgrad(const ConvGeom& g, const void* x, const void* dy, float* dw
   return check_launch("conv2d_bwd_filter 1x1 (bf16 mfma, direct-to-LDS)");
 }
 
-// out[i] = the sum of `slices` fp32 partial products, n floats apart, added in slice order and rounded once
+// out[i] = the sum of `slices` fp32 partial products, n floats apart, added in slice order, + bias[i % M], rounded once
 template <typename E>
-__global__ void __launch_bounds__(256) gemm16_sum_slices_kernel(const float* __restrict__ part, uint16_t* __restrict__ out,
-                                                                size_t n, int slices) {
+__global__ void __launch_bounds__(256) gemm16_sum_slices_kernel(const float* __restrict__ part, const float* __restrict__ bias, int M,
+                                                                uint16_t* __restrict__ out, size_t n, int slices) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
     float v = part[i];
     for (int k = 1; k < slices; ++k) v += part[(size_t)k * n + i];
+    if (bias) v += bias[i % M];
     out[i] = Lo16<E>::narrow(v);
   }
+}
+template <typename E>
+int gemm16_sum_slices(const void* ws, const float* bias, int M, int N, void* C, int slices, hipStream_t s) {
+  const size_t n = (size_t)M * N;
+  hipLaunchKernelGGL(gemm16_sum_slices_kernel<E>, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
+                     static_cast<const float*>(ws), bias, M, static_cast<uint16_t*>(C), n, slices);
+  return check_launch("matmul (16-bit mfma, slices added)");
 }
 
 bool gemm16_plan(int mode, int M, int N, int K, const float* bias_rows, PwdParams* p) {
@@ -794,13 +828,64 @@ bool gemm16_plan(int mode, int M, int N, int K, const float* bias_rows, PwdParam
   return pwd16_sizes(p, 1);
 }
 
-// bytes of workspace with which A B^T (mode 2) cuts its contraction into slices (0: one slice, or not these kernels')
+// mode 1 as the filter gradient's kernel sees it; false: not its product
+bool gemm16_nt_plan(int M, int N, int K, PwdWgradParams* p) {
+  if (K < 8) return false;
+  p->C = M; p->Mo = N; p->P = K; p->N = 1;
+  p->Pc = (K + 7) / 8;
+  p->dup = (8 - K % 8) % 8;
+  const long long xb = (long long)M * K * 2, db = (long long)N * K * 2;
+  if (xb >= (1ll << 31) || db >= (1ll << 31)) return false;
+  p->x_bytes = (unsigned)xb;
+  p->dy_bytes = (unsigned)db;
+  p->ncells = p->Pc;
+  p->nstages = (p->ncells + PWG_CH - 1) / PWG_CH;
+  p->ctiles = (M + PWG_T - 1) / PWG_T;
+  p->mtiles = (N + PWG_T - 1) / PWG_T;
+  p->E = 0;
+  p->sps = p->nstages;
+  p->nsplit = 1;
+  return (long long)p->ctiles * p->mtiles <= 65535;
+}
+
+// slices of the contraction of modes 0 and 1, us per stage: where the stages that a workgroup is spared take longer than the second launch
+// (3.5 us) and the partial products' way to memory and back.  One slice / so many, us: mode 1 256 x 879 x 9998 104 / 22, 512 x 4000 x 4001 55 / 39, 512 x 2355
+// x 1024 13.9 / 17.3 (not cut); mode 0 1024 x 200 x 2000 17.6 / 12.6, 29 x 700 x 2000 17.4 / 10.3, 1024 x 700 x 512 8.1 / 12.5 (not cut).
+int gemm16_slices(int ctiles, int mtiles, int nstages, double us, double results, int* sps, int cap) {
+  const int most = pwd16_slices(ctiles, mtiles, nstages, sps, cap);
+  int best = 1;
+  double least = us * nstages;
+  for (int n = 2; n <= most; ++n) {
+    const int per = (nstages + n - 1) / n;
+    const double t = us * per + 3.5 + 2e-6 * results * n;
+    if (t < least) least = t, best = n;
+  }
+  *sps = (nstages + best - 1) / best;
+  return (nstages + *sps - 1) / *sps;
+}
+int gemm16_slices(int mode, const PwdParams& p, int* sps, int cap = 32) {
+  const int bm = pwd16_bm(p), mt = (p.Mo + bm - 1) / bm;
+  if (mode == 2) return pwd16_slices(p.ctiles, mt, p.nstages, sps, cap);
+  return gemm16_slices(p.ctiles, mt, p.nstages, 0.4, (double)p.P * p.Mo, sps, cap);
+}
+
+int gemm16_nt_slices(const PwdWgradParams& p, int* sps, int cap = 32) {
+  return gemm16_slices(p.ctiles, p.mtiles, p.nstages, 0.64, (double)p.C * p.Mo, sps, cap);
+}
+
+// bytes of workspace with which a product cuts its contraction into slices (0: one slice, or not these kernels')
 size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K) {
-  PwdParams p{};
-  if (!is_lo16(dtype) || mode != 2 || M <= 0 || N <= 0 || K <= 0 || !gemm16_plan(mode, M, N, K, nullptr, &p)) return 0;
-  const int bm = pwd16_bm(p);
-  int sps;
-  const int ns = pwd16_slices(p.ctiles, (N + bm - 1) / bm, p.nstages, &sps);
+  if (!is_lo16(dtype) || M <= 0 || N <= 0 || K <= 0) return 0;
+  int sps, ns = 1;
+  if (mode == 1) {
+    PwdWgradParams p{};
+    if (!gemm16_nt_plan(M, N, K, &p) || (!options().pw16_pf && mfma_big16_nt_pays(N, M))) return 0;
+    ns = gemm16_nt_slices(p, &sps);
+  } else {
+    PwdParams p{};
+    if (!gemm16_plan(mode, M, N, K, nullptr, &p)) return 0;
+    ns = gemm16_slices(mode, p, &sps);
+  }
   return ns > 1 ? (size_t)ns * M * N * sizeof(float) : 0;
 }
 
@@ -815,39 +900,35 @@ size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K) {
 // of 8 in mode 0 (a 16-byte cell of B would straddle two rows), a bias or an odd number of columns in mode 2 (the
 // range check of a buffer load works on 4-byte words: the word that holds the last element of B's last row would
 // lie half past the tensor and come back as zero), operands of 2 GiB.
-// With a workspace of mfma_gemm16_ws_bytes, A B^T over a long contraction and few tiles (the weight gradient of a
-// layer over many frames) cuts the contraction into slices, one workgroup per tile and slice; their fp32 partial
-// products are added in slice order.
+// With a workspace of mfma_gemm16_ws_bytes, a long contraction over few tiles (the weight gradient of a
+// layer over many frames, the input gradient of a classifier of many classes) is cut into slices, one workgroup per tile and slice; their fp32 partial
+// products are added in slice order, the bias with them.
 int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int M, int N, int K,
                 const float* bias_rows, hipStream_t s, void* ws, size_t ws_bytes) {
   if (!is_lo16(dtype) || M <= 0 || N <= 0 || K <= 0) return -1;
+  const size_t per = (size_t)M * N * sizeof(float);
+  int slices = ws ? (int)std::min<size_t>(ws_bytes / per, 32) : 1;
   if (mode == 1) {
-    if (K < 8) return -1;
     PwdWgradParams p{};
-    p.C = M; p.Mo = N; p.P = K; p.N = 1;
-    p.Pc = (K + 7) / 8;
-    p.dup = (8 - K % 8) % 8;
-    const long long xb = (long long)M * K * 2, db = (long long)N * K * 2;
-    if (xb >= (1ll << 31) || db >= (1ll << 31)) return -1;
+    if (!gemm16_nt_plan(M, N, K, &p)) return -1;
     if (!options().pw16_pf && mfma_big16_nt_pays(N, M)) return mfma_big16_nt(dtype, N, M, K, B, A, bias_rows, C, s);
-    p.x_bytes = (unsigned)xb;
-    p.dy_bytes = (unsigned)db;
-    p.ncells = p.Pc;
-    p.nstages = (p.ncells + PWG_CH - 1) / PWG_CH;
-    p.ctiles = (M + PWG_T - 1) / PWG_T;
-    p.mtiles = (N + PWG_T - 1) / PWG_T;
-    p.E = 0;
-    p.sps = p.nstages;
-    p.nsplit = 1;
-    if ((long long)p.ctiles * p.mtiles > 65535) return -1;
-    by_lo16(dtype, [&](auto* e_) {
+    return by_lo16(dtype, [&](auto* e_) {
       using E = FLHIP_T_OF(e_);
-      hipLaunchKernelGGL((pwd16_wgrad_kernel<E, true>), dim3(1u, (unsigned)(p.ctiles * p.mtiles)), dim3(256), 0, s, p,
-                         static_cast<const E*>(A), static_cast<const E*>(B), (float*)nullptr, static_cast<uint16_t*>(C),
-                         bias_rows);
-      return 0;
+      const unsigned tiles = (unsigned)(p.ctiles * p.mtiles);
+      if (slices > 1) slices = gemm16_nt_slices(p, &p.sps, slices);
+      if (slices <= 1) {
+        p.sps = p.nstages;
+        hipLaunchKernelGGL((pwd16_wgrad_kernel<E, true>), dim3(1u, tiles), dim3(256), 0, s, p, static_cast<const E*>(A),
+                           static_cast<const E*>(B), (float*)nullptr, static_cast<uint16_t*>(C), bias_rows);
+        return check_launch("matmul (A^T * B, 16-bit mfma)");
+      }
+      p.nsplit = slices;
+      p.E = (int)((long long)M * N - N);      // (its slices lie E + N floats apart)
+      hipLaunchKernelGGL((pwd16_wgrad_kernel<E, false>), dim3((unsigned)slices, tiles), dim3(256), 0, s, p, static_cast<const E*>(A),
+                         static_cast<const E*>(B), static_cast<float*>(ws), (uint16_t*)nullptr, (const float*)nullptr);
+      if (const int rc = check_launch("matmul (A^T * B, 16-bit mfma, slices)")) return rc;
+      return gemm16_sum_slices<E>(ws, bias_rows, M, N, C, slices, s);
     });
-    return check_launch("matmul (A^T * B, 16-bit mfma)");
   }
   if (mode != 0 && mode != 2) return -1;
   PwdParams p{};
@@ -855,18 +936,17 @@ int mfma_gemm16(int dtype, int mode, const void* A, const void* B, void* C, int 
   p.pos_bias = bias_rows;
   return by_lo16(dtype, [&](auto* e_) {
     using E = FLHIP_T_OF(e_);
-    if (mode == 0) return pwd16_go<E, false>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B, 16-bit mfma)", false);
-    const size_t per = (size_t)M * N * sizeof(float);
-    int slices = ws ? (int)std::min<size_t>(ws_bytes / per, 32) : 1;
-    if (slices <= 1) return pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false);
+    const auto go = [&](int* sl) {
+      return mode == 0 ? pwd16_go<E, false>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B, 16-bit mfma)", false, sl)
+                       : pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false, sl);
+    };
+    if (slices > 1) slices = gemm16_slices(mode, p, &p.sps, slices);
+    if (slices <= 1 || (!options().pw16_pf && mfma_big16_halves(false, 1, p.Kc, p.Mo, p.P) >= 0)) return go(nullptr);
+    p.pos_bias = nullptr;      // (it joins the sum)
     p.part = static_cast<float*>(ws);
     p.slice = (size_t)M * N;
-    const int rc = pwd16_go<E, true>(p, A, B, nullptr, C, nullptr, s, "matmul (A * B^T, 16-bit mfma)", false, &slices);
-    if (rc != 0 || slices <= 1) return rc;
-    const size_t n = (size_t)M * N;
-    hipLaunchKernelGGL(gemm16_sum_slices_kernel<E>, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
-                       static_cast<const float*>(ws), static_cast<uint16_t*>(C), n, slices);
-    return check_launch("matmul (A * B^T, 16-bit mfma, slices added)");
+    if (const int rc = go(&slices)) return rc;
+    return gemm16_sum_slices<E>(ws, bias_rows, M, N, C, slices, s);
   });
 }
 

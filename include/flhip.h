@@ -462,8 +462,8 @@ int flhip_matmul_ws(const void* A, const void* B, void* C, int32_t M, int32_t N,
                     int32_t K, int trans_a, int trans_b, const float* bias_rows,
                     int dtype, void* ws, size_t ws_bytes, void* stream);
 /* Bytes at ws with which flhip_matmul_ws cuts the contraction of any of the forms: those of
- * flhip_matmul_workspace_bytes for A * B^T, and what fp32 products of the other two over a small
- * batch (fl::linear forward and its input gradient) can use. */
+ * flhip_matmul_workspace_bytes for A * B^T, and what products of the other two with few results over a long
+ * contraction (fl::linear forward over a small batch, its input gradient) can use. */
 size_t flhip_matmul_slices_bytes(int32_t M, int32_t N, int32_t K, int trans_a, int trans_b, int dtype);
 
 /* out[r] (fp32) = sum over c of x[r, c] for a rows x cols matrix: the bias gradient

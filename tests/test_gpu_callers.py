@@ -126,6 +126,45 @@ def test_matmul_in_16_bit_storage(M, N, K, ta, tb, dtype):
         assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4].tolist())
 
 
+# thin products and those of few results over a long contraction: rows and columns around the tiles of 64 and 128 and the pieces of 8, odd rows
+# of C, one column, slices of equal and unequal length and of a partial last stage, contractions the matrix instructions do not take
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ta,M,N,K", [
+    (False, 65, 1, 64), (False, 9998, 3, 512), (False, 29, 33, 1024), (False, 8, 128, 2000), (False, 7, 128, 2000), (False, 1001, 65, 3136),
+    (False, 2000, 64, 1999), (False, 300, 300, 2056), (False, 64, 17, 1016),
+    (True, 17, 1, 129), (True, 127, 128, 64), (True, 129, 127, 67), (True, 1027, 18, 31), (True, 256, 129, 9998), (True, 513, 40, 4001),
+    (True, 130, 300, 2049), (True, 16, 20, 700), (True, 2000, 100, 8200), (True, 134, 16, 130)])
+def test_matmul_in_16_bit_storage_thin_and_in_slices(ta, M, N, K, dtype):
+    """With and without the workspace, with and without a bias, the operands and C on a 4-byte boundary and 2 bytes behind one (with values around
+    C that stay, NaN around the operands), against the exact sum: one rounding, plus what an fp32 accumulation over K terms may add."""
+    import ctypes as C
+    from flashlight_amd import capi
+    rng = np.random.default_rng(M * 7 + N * 5 + K)
+    A = _round(rng.standard_normal((M, K) if ta else (K, M)).astype(np.float32), dtype)
+    B = _round(rng.standard_normal((N, K)).astype(np.float32), dtype)
+    bias = rng.standard_normal(M).astype(np.float32)
+    code = {torch.bfloat16: capi.BF16, torch.float16: capi.F16}[dtype]
+    lib, S, P = capi.lib(), C.c_void_p(torch.cuda.current_stream().cuda_stream), lambda t: C.c_void_p(t.data_ptr()) if t is not None else None
+    def at(a, shift):      # `shift` elements into a buffer of NaN
+        t = torch.full((a.size + 16,), float("nan"), device="cuda", dtype=dtype)
+        t[shift:shift + a.size] = dev(a, dtype).flatten()
+        return t[shift:]
+    bd = dev(bias)
+    need = lib.flhip_matmul_slices_bytes(M, N, K, int(ta), 0, code)
+    want = B.astype(np.float64) @ (A.T if ta else A).astype(np.float64)                       # stored [n][m]
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for b, nws, shift in ((None, need, 0), (bd, need, 1), (bd, 0, 0), (None, 0, 1), (None, need // 2 // 4 * 4, 0)):
+        ws = torch.full((max(nws // 4, 4),), float("nan"), device="cuda")
+        buf = torch.full((M * N + 4,), 7.0, device="cuda", dtype=dtype)
+        out, Ad, Bd = buf[2 + shift:2 + shift + M * N], at(A, 8 + shift), at(B, 8 + shift)
+        capi.check(lib.flhip_matmul_ws(P(Ad), P(Bd), P(out), M, N, K, int(ta), 0, P(b), code, P(ws) if nws else None, nws, S))
+        ref = want if b is None else want + bias
+        bad = np.abs(host(out).astype(np.float64).reshape(N, M) - ref) > 1.01 * half_ulp * np.abs(ref) + 2e-6 * K + 6e-8
+        assert not bad.any(), (nws, shift, int(bad.sum()), np.argwhere(bad)[:4].tolist())
+        rest = torch.cat([buf[:2 + shift], buf[2 + shift + M * N:]])
+        assert bool((rest == 7).all())
+
+
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("M,N,K,part", [(128, 80, 5000, 1.0), (2000, 80, 12000, 1.0), (1024, 1024, 12000, 1.0),
                                         (67, 130, 3001, 1.0), (256, 64, 4096, 0.5), (300, 200, 70, 1.0)])
