@@ -198,18 +198,21 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
 // step's gradients hang on those.  (With the parts' sums, nearer to 64 bits as they are, the gradients of a step over 300 to 512 images of
 // 28 x 28 through two 5x5 layers were up to 3e-3 apart from these in the 2-norm, else 1e-6; the second layer over 64 / 512 images 38 / 145 us,
 // in parts 18 / 65.)
-// 16-bit storage: 3x3 windows over planes of at most 64 positions (the 7 x 7 layers) and a sequence of at least 2048 positions.
-// Measured (batch 64 / 32, forward): 7 x 7 x 512 41.9 / 40.3 us against 62.3 / 54.8 on the slab kernel; 14 x 14 x 256 42.2 / 33.0
-// against 34.6 / 31.0 and 28 x 28 x 128 41.3 / 32.5 against 25.5 / 19.7, so larger planes stay where they were.  TAP2D_ALL lifts the
-// rules.  With 512 channels and more on both sides the slab kernel's 16 chunks take longer than these kernels also for fewer images, where the
-// thin kernels do not take them: us, slab / here, 7 x 7 x 512 12 / 20 / 31 images 49 / 36, 57 / 36, 57 / 36, backward 48 / 34, 56 / 34, 56 / 34; 6 x 6
-// x 512 16 / 31 images 49 / 36, 61 / 36; 14 x 14 x 512 6 / 20 / 31 / 48 images 57 / 36, 63 / 55, 65 / 66, 122 / 71 (256 channels: 8 % either way).
+// 16-bit storage, 3x3 windows.  us, these kernels / the others (slab, or thin where there are few tiles), forward, bf16: 512 channels over 7 x 7, 1 / 4 / 8
+// images 22 / 28, 23 / 32, 26 / 31, over 14 x 14, 1 / 20 / 48 23 / 29, 46 / 63, 61 / 122; 384 channels over 14 x 14, 4 / 26 / 40 27 / 38, 45 / 50, 56 / 48, over 7 x
+// 7, 16 26 / 39; 256 channels over 14 x 14, 4 images (thin) 19.5 / 17.9, 12 / 33 / 48 / 64 22 / 32, 26 / 34, 30 / 33, 36 / 34, over 16 x 16, 8 / 33 / 40 / 48 21 /
+// 24, 31 / 33, 32 / 32, 36 / 32; 224 channels over 14 x 14, 26 / 40 images 24 / 25, 30 / 28; 128 channels over 28 x 28, 4 / 33 images 17 / 18, 29 / 22.
+// Planes of at most 64 positions with 2048 positions and more: 256 channels over 7 x 7, 64 images 20 / 26.  TAP2D_ALL lifts the rules.
 static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
   if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
   if (options().tap2d_all) return true;
   if (dtype == FLHIP_F32) return (bwd || g.KH * g.KW <= 9) && mfma_tap2d_split_pays(g, bwd);
   if (g.H * g.W <= 64 && (long long)g.N * (g.H + 1) * (g.W + 1) >= 2048) return true;
-  return g.H * g.W <= 196 && g.groups == 1 && std::min(g.C, g.K) >= 512 && !thin_on(g, dtype, bwd, true);
+  if (g.groups != 1) return false;
+  const long long positions = (long long)g.N * (g.H + 1) * (g.W + 1);
+  const int least = std::min(g.C, g.K), most = std::max(g.C, g.K);
+  if (least >= 384) return g.H * g.W <= 196 && (least >= 512 || positions <= 7500);
+  return least >= 208 && most <= 256 && g.H * g.W <= 256 && positions <= (least >= 240 ? 10500 : 7500) && !thin_on(g, dtype, bwd, true);
 }
 
 // One-row windows on their own kernels.  In fp32 over more than 256 contraction channels only where the thin kernels do not take them

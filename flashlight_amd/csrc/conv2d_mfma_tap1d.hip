@@ -257,34 +257,6 @@ tap1d_operands_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H,
   }
 }
 
-// The same fragments with the tap as the index that changes fastest after the lane: the four waves of a block then read
-// the same cache lines (a lane's 8 or 4 contraction channels x 9 taps are neighbours in memory), where in the order
-// above - the stage fastest - every line is met once per tap by a different block.
-template <typename T>
-__global__ void __launch_bounds__(256)
-tap_weights_by_tap_kernel(const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p) {
-  constexpr int CELL = Tap1Elem<T>::CELL;
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long total = (long long)p.mblocks * p.taps_total * p.KS * 64;
-  if (idx >= total) return;
-  const int lane = (int)(idx & 63);
-  const long long st = idx >> 6;
-  const int tap = (int)(st % p.taps_total);
-  const long long r2 = st / p.taps_total;
-  const int ks = (int)(r2 % p.KS), mblk = (int)(r2 / p.KS);
-  const int m = mblk * 32 + (lane & 31), c0 = (2 * ks + (lane >> 5)) * CELL;
-  const int j = p.tapj[tap];
-  __attribute__((aligned(16))) T v[CELL];
-#pragma unroll
-  for (int e = 0; e < CELL; ++e) {
-    const int c = c0 + e;
-    v[e] = T{};
-    if (j >= 0 && m < p.Mo && c < p.Cc)
-      v[e] = w[p.bwd ? ((size_t)c * p.Cw + m) * p.KW + j : ((size_t)m * p.Cw + c) * p.KW + j];
-  }
-  wf[(((long long)mblk * p.taps_total + tap) * p.KS + ks) * 64 + lane] = *reinterpret_cast<const uintx4_t*>(v);
-}
-
 // ---- the convolution ---------------------------------------------------------------------
 // KS stages per tap; DT taps per unrolled group; RW stages between a weight fragment's load and its use (RW divides
 // DT * KS); SS source stride;
@@ -479,7 +451,7 @@ tap1d_conv_kernel(Tap1Params p, const T* __restrict__ xr, const uintx4_t* __rest
 
 // 3 x 3 windows of stride 1 over small planes (the 14 x 14 and 7 x 7 layers of a residual network): the same loop
 // over a sequence that holds every plane of the batch, rows pH + 1 apart with a zero row between two planes, a row's
-// pW positions followed by one zero column (tap2d_rows_kernel writes it so) - the window's taps are then nine fixed
+// pW positions followed by one zero column (tap2d_rows_block writes it so) - the window's taps are then nine fixed
 // offsets into the sequence, and the zero row / column are the padding.  Results at the zero positions are not stored.
 template <typename T, int KS, int DT, int RW, int NB>
 __global__ void __launch_bounds__(256, 1)
@@ -491,11 +463,11 @@ tap2d_conv_kernel(Tap1Params p, const T* __restrict__ xr, const uintx4_t* __rest
 // x[n][c][h][w] -> xr[position][Cs] with position = ((n (H + 1) + 1 + h) P + w), P = W + 1; the zero rows, the zero
 // column and channels c >= C are written as zeros.  A block transposes 64 channels x 64 positions through LDS.
 template <typename T>
-__global__ void __launch_bounds__(256)
-tap2d_rows_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int W, int N, int TS, int Cs) {
+__device__ __forceinline__ void tap2d_rows_block(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int W, int N, int TS, int Cs, int bx,
+                                                 int by, void* lds) {
   constexpr int CELL = Tap1Elem<T>::CELL;
-  __shared__ T tile[64][sizeof(T) == 2 ? 66 : 65];
-  const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+  T(*tile)[66] = reinterpret_cast<T(*)[66]>(lds);
+  const int t0 = bx * 64, c0 = by * 64;
   const int P = W + 1, H1 = H + 1;
   {
     const int tx = threadIdx.x & 63, cy = threadIdx.x >> 6;
@@ -523,6 +495,18 @@ tap2d_rows_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int
       *reinterpret_cast<uintx4_t*>(xr + (size_t)t * Cs + c) = *reinterpret_cast<const uintx4_t*>(v);
     }
   }
+}
+
+// Both operands in one launch, the first blocks the positions', the others the weights', through LDS (tap1d_weights_block): two launches, and weights
+// gathered element by element, took 7 us more (512 channels over 7 x 7, 20 images 33.5 -> 26.5 us; 256 channels over 8 x 8, 64 images 27.5 -> 22.9).
+template <typename T>
+__global__ void __launch_bounds__(256)
+tap2d_operands_kernel(const T* __restrict__ x, T* __restrict__ xr, int C, int H, int W, int N, int TS, int Cs, int tblocks, int rblocks,
+                      const T* __restrict__ w, uintx4_t* __restrict__ wf, Tap1Weights p) {
+  extern __shared__ uintx4_t t1_operands[];
+  const int b = blockIdx.x;
+  if (b < rblocks) tap2d_rows_block(x, xr, C, H, W, N, TS, Cs, b % tblocks, b / tblocks, t1_operands);
+  else tap1d_weights_block(w, wf, p, b - rblocks, reinterpret_cast<T*>(t1_operands));
 }
 
 // ---- host side ---------------------------------------------------------------------------
@@ -789,12 +773,10 @@ int run_conv2d(const ConvGeom& g, bool bwd, const void* src, const void* w, cons
   T* xr = static_cast<T*>(ws);
   uintx4_t* wf = reinterpret_cast<uintx4_t*>(static_cast<char*>(ws) + pl.rows_bytes);
   {
-    const dim3 grid((unsigned)((pl.p.TS + 63) / 64), (unsigned)((pl.p.Cs + 63) / 64));
-    hipLaunchKernelGGL(tap2d_rows_kernel<T>, grid, dim3(256), 0, s, static_cast<const T*>(src), xr, pl.C, g.H, g.W, g.N, pl.p.TS,
-                       pl.p.Cs);
-    const long long total = (long long)pl.w.mblocks * pl.w.taps_total * pl.w.KS * 64;
-    hipLaunchKernelGGL(tap_weights_by_tap_kernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const T*>(w), wf, pl.w);
+    const int tblocks = (pl.p.TS + 63) / 64, rblocks = tblocks * ((pl.p.Cs + 63) / 64), wblocks = pl.w.mblocks * pl.w.KS;
+    const size_t lds = std::max<size_t>(64 * 66, 544 * (size_t)pl.w.KW + 64) * sizeof(T);
+    hipLaunchKernelGGL(tap2d_operands_kernel<T>, dim3((unsigned)(rblocks + wblocks)), dim3(256), lds, s, static_cast<const T*>(src), xr, pl.C,
+                       g.H, g.W, g.N, pl.p.TS, pl.p.Cs, tblocks, rblocks, static_cast<const T*>(w), wf, pl.w);
   }
   if (const int rc = check_launch("conv2d (3x3 windows over stacked planes, operand passes)")) return rc;
   T* out = static_cast<T*>(dst);

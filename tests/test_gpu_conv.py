@@ -1674,6 +1674,11 @@ def test_backward_passes_by_plan(shape, dtype):
     ((20, 64, 64, 64), 64, 1),
     ((13, 512, 7, 7), 512, 1),         # stacked planes: fewer positions than before, more tiles than the thin kernels take
     ((6, 512, 14, 14), 520, 1),
+    ((1, 512, 7, 7), 512, 1),          # ... and of few tiles
+    ((2, 513, 14, 14), 512, 1),        # (more channels forward than they are compiled for)
+    ((4, 400, 14, 14), 390, 1), ((16, 384, 6, 6), 500, 1),
+    ((12, 256, 14, 14), 256, 1), ((20, 250, 16, 16), 240, 1), ((9, 208, 13, 13), 224, 1),      # from 208 channels on
+    ((36, 256, 16, 16), 256, 1), ((37, 240, 16, 16), 240, 1),                                  # the last positions they take, and beyond
     ((20, 512, 16, 16), 512, 2),       # gathered taps within one round of the slab kernel
     ((33, 256, 24, 24), 256, 2),       # ... within two
 ])
