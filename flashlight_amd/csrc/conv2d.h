@@ -90,6 +90,8 @@ size_t mfma_gemm16_ws_bytes(int dtype, int mode, int M, int N, int K);
 // classifier, gradients up to 1e-3 in the 2-norm and 9e-2 of their rms at most (without such a choice 1e-6 and 1e-5); a ReLU layer of
 // 512 units over 200 steps of 64 columns 1e-3 and 0.2.
 size_t gemm32_ws_bytes(int mode, int M, int N, int K, bool fp32_sums = false);
+int gemm32_pair(int mode, const float* A, const float* A2, const float* B, const float* B2, float* C, float* C2, int M, int N, int K, const float* bias, const float* bias2,
+                void* ws, size_t ws_bytes, hipStream_t s);
 int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int K, const float* bias, void* ws,
            size_t ws_bytes, hipStream_t s, const float* addend = nullptr, bool (*take)(int, int, int, bool) = nullptr,
            bool fp32_sums = false);

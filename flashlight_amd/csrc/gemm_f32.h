@@ -16,6 +16,9 @@ struct Gemm32 {
   // 1x1 windows, whose positions are rows of A and C (modes 0 and 2) or the contraction (mode 1): positions of an image, of the source's
   // image, of a result row, and the source's step per result row and column
   int P, SP, OW, rowstep, colstep, slices;
+  // the second of two products of one shape in a launch (gemm32_pair): blockIdx.z = 1
+  const float *A2, *B2, *bias2;
+  float* C2;
 };
 
 // consecutive workgroups go to the eight dies in turn: each die takes one run of tiles, and within a run the tiles of

@@ -111,6 +111,7 @@ gemm32_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B
   extern __shared__ __align__(16) float g32_lds[];
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  if (blockIdx.z) A = p.A2, B = p.B2, bias = p.bias2, C = p.C2;
   const int tile = gemm32_tile_of(blockIdx.x, p.mtiles * p.ntiles);
   const int m0 = (tile % p.mtiles) * TM, n0 = (tile / p.mtiles) * TN;
   const int s0 = blockIdx.y * p.sps, send = min(p.nstages, s0 + p.sps);
@@ -227,9 +228,10 @@ gemm32_kernel(Gemm32 p, const float* __restrict__ A, const float* __restrict__ B
 }
 
 // out = sum of the slices (+ bias[row]) (+ addend, which may be out); rows of M4 pieces, M a multiple of 4 where there is
-// a bias
+// a bias.  blockIdx.y = 1: those of a second product behind them, with bias2, to out2
 __global__ void __launch_bounds__(256) gemm32_sum_kernel(const float4* __restrict__ part, const float* __restrict__ bias,
-                                                         const float4* addend, float4* out, size_t n4, int M4, int slices) {
+                                                         const float4* addend, float4* out, size_t n4, int M4, int slices, const float* bias2, float4* out2) {
+  if (blockIdx.y) part += slices * n4, bias = bias2, out = out2;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
     float4 v = part[i];
 #pragma unroll 4
@@ -281,7 +283,8 @@ bool gemm32_ragged(int mode, int M, int N, int K, bool fp32_sums) {
   return mode == 2 ? macs >= 1e7 && (K <= 3000 || macs >= 2e8) : macs >= 1e6;
 }
 
-bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gemm32Plan* best) {
+// pair > 0: for two such products in a launch, whose slices fit `pair` bytes
+bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gemm32Plan* best, size_t pair = 0) {
   const bool ak = mode == 1, bk = mode != 2;
   const bool pieces = (ak ? K : M) % 4 == 0 && (bk ? K : N) % 4 == 0;      // rows of whole 16-byte pieces
   if (!pieces && !gemm32_ragged(mode, M, N, K, fp32_sums)) return false;
@@ -296,12 +299,12 @@ bool gemm32_plan(int mode, int M, int N, int K, bool sliced, bool fp32_sums, Gem
     if (!pieces && t.tm * t.tn == 64 * 64) continue;
     const int mt = (M + t.tm - 1) / t.tm, nt = (N + t.tn - 1) / t.tn;
     for (int ns = 1; ns <= (sliced ? 16 : 1); ++ns) {
-      if (ns > 1 && (nst / ns < 8 || ((size_t)M * N) % 4 != 0)) break;
+      if (ns > 1 && (nst / ns < 8 || ((size_t)M * N) % 4 != 0 || (pair && (size_t)8 * ns * M * N > pair))) break;
       const int sps = (nst + ns - 1) / ns;
       if ((nst + sps - 1) / sps != ns) continue;
-      const long long wgs = (long long)mt * nt * ns, rounds = (wgs + cus - 1) / cus;
+      const long long wgs = (long long)mt * nt * ns * (pair ? 2 : 1), rounds = (wgs + cus - 1) / cus;
       double cost = (double)rounds * (sps + t.more) * t.stage * (rounds == 1 ? t.alone : 1.0);
-      if (ns > 1) cost += (double)(ns + 1) * M * N * 4 / unit + second;
+      if (ns > 1) cost += (double)(ns + 1) * M * N * (pair ? 8 : 4) / unit + second;
       if (cost < best_cost) {
         best_cost = cost;
         best->tm = t.tm; best->tn = t.tn; best->slices = ns; best->parts = !whole && t.tm * t.tn > 64 * 64;
@@ -321,7 +324,7 @@ int gemm32_go(const Gemm32Plan& pl, const float* A, const float* B, const float*
   constexpr size_t lds = (size_t)RING * (TM + TN) * KC * 4;
   auto kernel = gemm32_kernel<MODE, TM, TN>;
   if (!mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return -1;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(pl.p.mtiles * pl.p.ntiles), (unsigned)pl.slices), dim3(GTHREADS), lds, s, pl.p, A, B,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(pl.p.mtiles * pl.p.ntiles), (unsigned)pl.slices, pl.p.C2 ? 2 : 1), dim3(GTHREADS), lds, s, pl.p, A, B,
                      bias, addend, C);
   return check_launch("matmul (fp32)");
 }
@@ -363,8 +366,34 @@ int gemm32(int mode, const float* A, const float* B, float* C, int M, int N, int
   const size_t n4 = (size_t)M * N / 4;
   hipLaunchKernelGGL(gemm32_sum_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, s,
                      reinterpret_cast<const float4*>(ws), bias,
-                     reinterpret_cast<const float4*>(addend), reinterpret_cast<float4*>(C), n4, M / 4, pl.slices);
+                     reinterpret_cast<const float4*>(addend), reinterpret_cast<float4*>(C), n4, M / 4, pl.slices, (const float*)nullptr, (float4*)nullptr);
   return check_launch("matmul (fp32, slices added)");
+}
+
+// gemm32 of two products of one shape in a launch (and one that adds both's slices, where the workspace holds them); -1: gemm32 twice
+int gemm32_pair(int mode, const float* A, const float* A2, const float* B, const float* B2, float* C, float* C2, int M, int N, int K, const float* bias, const float* bias2,
+                void* ws, size_t ws_bytes, hipStream_t s) {
+  Gemm32Plan pl{};
+  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(A2) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(B2) |
+       reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(C2)) % 16 != 0)
+    return -1;
+  if (bias && M % 4 != 0) return -1;
+  if (!gemm32_plan(mode, M, N, K, ws != nullptr, false, &pl, std::max<size_t>(ws_bytes, 1))) return -1;
+  const bool cut = pl.slices > 1;
+  float* const part = static_cast<float*>(ws);
+  pl.p.A2 = A2; pl.p.B2 = B2; pl.p.bias2 = cut ? nullptr : bias2;
+  pl.p.C2 = cut ? part + (size_t)pl.slices * M * N : C2;
+  float* const dst = cut ? part : C;
+  const float* const b = cut ? nullptr : bias;
+  const int rc = pl.parts  ? gemm32_split(mode, pl.tm, pl.tn, pl.slices, pl.p, A, B, b, nullptr, dst, s)
+               : mode == 0 ? gemm32_tile<0>(pl, A, B, b, nullptr, dst, s)
+               : mode == 1 ? gemm32_tile<1>(pl, A, B, b, nullptr, dst, s)
+                           : gemm32_tile<2>(pl, A, B, b, nullptr, dst, s);
+  if (rc || !cut) return rc;
+  const size_t n4 = (size_t)M * N / 4;
+  hipLaunchKernelGGL(gemm32_sum_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096), 2), dim3(256), 0, s, reinterpret_cast<const float4*>(ws),
+                     bias, (const float4*)nullptr, reinterpret_cast<float4*>(C), n4, M / 4, pl.slices, bias2, reinterpret_cast<float4*>(C2));
+  return check_launch("matmul (fp32, two products' slices added)");
 }
 
 }  // namespace flhip

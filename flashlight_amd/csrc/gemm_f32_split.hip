@@ -159,6 +159,7 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
   typedef SplitSide<BK, TN> SB;
   constexpr int STAGE = SA::BYTES + SB::BYTES;
   __shared__ __align__(16) char lds[2 * STAGE];
+  if (!PL && blockIdx.z) A = p.A2, B = p.B2, bias = p.bias2, C = p.C2;
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
   int tile, slice = blockIdx.y;
@@ -359,7 +360,7 @@ gemm32_split_kernel(Gemm32 p, const float* __restrict__ A, const float* __restri
 
 template <int MODE, int TM, int TN, bool PL>
 int split_go(const Gemm32& p, int slices, const float* A, const float* B, const float* bias, const float* addend, float* C, hipStream_t s) {
-  hipLaunchKernelGGL((gemm32_split_kernel<MODE, TM, TN, PL>), PL && MODE == 1 ? dim3((unsigned)(p.mtiles * p.ntiles * slices)) : dim3((unsigned)(p.mtiles * p.ntiles), (unsigned)slices), dim3(ST), 0, s, p, A, B,
+  hipLaunchKernelGGL((gemm32_split_kernel<MODE, TM, TN, PL>), PL && MODE == 1 ? dim3((unsigned)(p.mtiles * p.ntiles * slices)) : dim3((unsigned)(p.mtiles * p.ntiles), (unsigned)slices, !PL && p.C2 ? 2 : 1), dim3(ST), 0, s, p, A, B,
                      bias, addend, C);
   return check_launch("matmul (fp32 in three parts)");
 }

@@ -83,6 +83,18 @@ def test_relu_layers_keep_the_sums_of_the_fp32_instruction():
         assert torch.equal(y, want) == same
 
 
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("I,H,L,T,B", [
+    (40, 32, 2, 64, 16),        # 1024 rows: the bias sums of both directions in one launch, as the weight gradients, in slices
+    (129, 48, 1, 41, 25),       # 1025 rows: not the bias sums; rows of no whole pieces
+    (33, 16, 1, 3, 2),          # fewer rows than a stage
+    (520, 64, 1, 43, 24),       # more input gradients than are added in a launch of their own
+    (6, 20, 2, 30, 40),         # (40 columns: the second layer's input)
+])
+def test_both_directions_share_their_products(mode, I, H, L, T, B):
+    test_rnn_forward_backward(mode, I, H, L, True, T, B, True)
+
+
 @pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
     # whole sequences in one launch: hidden sizes that are multiples of 4 up to 1024.  4, 8 and 16 units per workgroup,
     # a last workgroup with units to spare, a last contraction chunk with columns to spare, more waves than chunks
