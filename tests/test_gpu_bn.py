@@ -124,6 +124,27 @@ def test_inference(shape, axes):
     assert np.allclose(host(y), y_ref, atol=1e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,C,H,W,shift", [(2, 3, 5, 5, 0), (1, 1, 3, 5, 0), (3, 7, 2, 4, 0), (2, 5, 1, 7, 0), (2, 64, 56, 56, 0), (5, 130, 3, 3, 0), (2, 3, 5, 5, 1),
+                                           (1, 300, 33, 31, 0), (40, 256, 28, 28, 0)])
+def test_inference_in_pieces(N, C, H, W, shift, dtype):
+    """Pieces of 16 bytes over planes of any size (the end of one and the start of the next, the last channel's before the next image's first, a last
+    part of one), planes smaller than a piece, tensors that do not start on one; with and without an affine part: an fp32 result within three
+    roundings of float64's terms, a 16-bit one that rounded once more."""
+    g = torch.Generator(device="cuda").manual_seed(C + H)
+    n = N * C * H * W
+    x = torch.randn(n + 8, generator=g, device="cuda").to(dtype)[shift:shift + n].view(N, C, H, W)
+    gm, bt, rm, rv = (torch.rand(C, generator=g, device="cuda") + 0.1 for _ in range(4))
+    col = lambda t: t.double().view(1, C, 1, 1)
+    for a, b in ((gm, bt), (None, None)):
+        y, _, _ = fa.batchnorm(x, a, b, rm, rv, [2], False, 0.0, 1e-5)
+        k = 1 / (col(rv) + 1e-5).sqrt() * (1 if a is None else col(a))
+        want, add = (x.double() - col(rm)) * k, 0 if b is None else col(b)
+        half_ulp = {torch.float32: 0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+        slack = 6 * 2.0 ** -23 * (want.abs() + (col(rm) * k).abs() + abs(add)) + half_ulp * (want + add).abs()
+        assert bool(((y.double() - want - add).abs() <= slack + 6e-8).all())
+
+
 def test_large_mean_small_variance():
     # a shifted-sum variance must survive mean >> std
     rng = np.random.default_rng(55)
