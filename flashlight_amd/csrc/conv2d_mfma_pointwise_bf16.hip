@@ -809,6 +809,44 @@ lattice_scatter_kernel(const bf16_t* __restrict__ dxc, bf16_t* __restrict__ dx, 
   }
 }
 
+// V elements (V / 2 words) from a boundary of as many bytes
+template <int V>
+__device__ __forceinline__ void load_words(uint32_t (&w)[V / 2], const bf16_t* p) {
+  if constexpr (V == 8) {
+    const uintx4_t q = *reinterpret_cast<const uintx4_t*>(p);
+    w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+  } else if constexpr (V == 4) {
+    const uintx2_t q = *reinterpret_cast<const uintx2_t*>(p);
+    w[0] = q.x; w[1] = q.y;
+  } else {
+    w[0] = *reinterpret_cast<const uint32_t*>(p);
+  }
+}
+template <int V>
+__device__ __forceinline__ void store_words(bf16_t* p, const uint32_t (&w)[V / 2]) {
+  if constexpr (V == 8) *reinterpret_cast<uintx4_t*>(p) = uintx4_t{w[0], w[1], w[2], w[3]};
+  else if constexpr (V == 4) *reinterpret_cast<uintx2_t*>(p) = uintx2_t{w[0], w[1]};
+  else *reinterpret_cast<uint32_t*>(p) = w[0];
+}
+
+// The same over strides of 2 in both directions and planes of 2 OH x 2 OW: a thread takes V elements of a row of dxc and writes the 2 V of dx they lie
+// among and the 2 V zeros below them.  (An element of dx decided by itself: 28 x 28 to 56 x 56, 256 channels, 53 images, with the product 55 us, now 33; 14 x 14, 512 channels 41, now 25.)
+template <int V>
+__global__ void __launch_bounds__(256)
+lattice_scatter2_kernel(const bf16_t* __restrict__ dxc, bf16_t* __restrict__ dx, int OH, int OW, uint32_t total) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t per_row = OW / V, row = i / per_row, c = (i - row * per_row) * V;      // (a row of dxc is two of dx)
+  uint32_t in[V / 2], out[V];
+  load_words<V>(in, dxc + (size_t)row * OW + c);
+  const uint32_t zero[V] = {};
+#pragma unroll
+  for (int e = 0; e < V / 2; ++e) out[2 * e] = in[e] & 0xffffu, out[2 * e + 1] = in[e] >> 16;
+  bf16_t* d = dx + (size_t)row * 4 * OW + 2 * c;
+  store_words<2 * V>(d, out);
+  store_words<2 * V>(d + 2 * OW, zero);
+}
+
 // the stride-1 problem over the lattice points, if the kernels above take it
 bool pw16_strided_plan(const ConvGeom& g, ConvGeom* c) {
   if (!(g.KH == 1 && g.KW == 1 && g.py == 0 && g.px == 0 && g.groups == 1 && (g.sy > 1 || g.sx > 1))) return false;
@@ -828,7 +866,21 @@ void lattice_gather(const ConvGeom& g, const void* x, void* xc, hipStream_t s) {
   hipLaunchKernelGGL(lattice_gather_kernel, dim3((total + 255) / 256), dim3(256), 0, s, static_cast<const bf16_t*>(x),
                      static_cast<bf16_t*>(xc), g.H, g.W, g.OH, g.OW, g.sy, g.sx, total);
 }
+// strides of 2 over planes that they halve, elements a thread may take of a row of the smaller one (0: none)
+int halved(const ConvGeom& g, const void* a, const void* b) {
+  if (g.sy != 2 || g.sx != 2 || g.dly != 1 || g.dlx != 1 || g.H != 2 * g.OH || g.W != 2 * g.OW || (((uintptr_t)a | (uintptr_t)b) & 15)) return 0;
+  return g.OW % 4 == 0 ? 4 : g.OW % 2 == 0 ? 2 : 0;
+}
 void lattice_scatter(const ConvGeom& g, const void* dxc, void* dx, hipStream_t s) {
+  if (const int v = halved(g, dxc, dx)) {
+    const uint32_t n = (uint32_t)((size_t)g.N * g.C * g.OH * g.OW / v);
+    auto go2 = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((n + 255) / 256), dim3(256), 0, s, static_cast<const bf16_t*>(dxc), static_cast<bf16_t*>(dx), g.OH, g.OW, n);
+    };
+    if (v == 4) go2(lattice_scatter2_kernel<4>);
+    else go2(lattice_scatter2_kernel<2>);
+    return;
+  }
   const int vec = ((uintptr_t)dx & 15) ? 1 : g.W % 8 == 0 ? 8 : g.W % 4 == 0 ? 4 : g.W % 2 == 0 ? 2 : 1;
   const uint32_t total = (uint32_t)((size_t)g.N * g.C * g.H * g.W / vec);
   auto go = [&](auto kernel) {
@@ -880,6 +932,78 @@ taps_gather_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ xc, ConvGe
       if constexpr (PAIR) *reinterpret_cast<uint32_t*>(o) = v[0] | (v[1] << 16);
       else *o = (bf16_t)v[0];
     }
+  }
+}
+
+// Both for 3 x 3 windows of stride 2 and padding 1 over planes of 2 OH x 2 OW, V columns of the smaller plane to a thread: whole pieces of the three
+// rows that the taps share instead of an element per tap (us with the product, 128 channels, 56 x 56 to 28 x 28, 53 images: gathering, forward, 67 -> 54, spreading, backward, 79 -> 56; 256
+// channels, 24 x 24 to 12 x 12, 46 -> 32, 45 -> 34).
+template <int V>
+__global__ void __launch_bounds__(256)
+taps_gather3_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ xc, int OH, int OW, unsigned planes) {
+  const int ow = threadIdx.x * V, P = OH * OW, W = 2 * OW;
+  const unsigned plane = blockIdx.x * blockDim.z + threadIdx.z;
+  if (ow >= OW || plane >= planes) return;
+  const bf16_t* xp = x + (size_t)plane * 4 * P + 2 * ow;
+  bf16_t* op = xc + (size_t)plane * 9 * P + ow;
+  for (int oh = threadIdx.y; oh < OH; oh += blockDim.y)
+#pragma unroll
+    for (int kh = 0; kh < 3; ++kh) {
+      const int ih = 2 * oh + kh - 1;      // (below 2 OH always)
+      uint32_t w[V] = {}, before = 0;      // columns 2 ow .. 2 ow + 2 V - 1, and 2 ow - 1
+      if (ih >= 0) {
+        load_words<2 * V>(w, xp + ih * W);
+        if (ow > 0) before = xp[ih * W - 1];
+      }
+      uint32_t even[V / 2], odd[V / 2], left[V / 2];
+#pragma unroll
+      for (int e = 0; e < V / 2; ++e) {
+        even[e] = (w[2 * e] & 0xffffu) | (w[2 * e + 1] << 16);
+        odd[e] = (w[2 * e] >> 16) | (w[2 * e + 1] & 0xffff0000u);
+        left[e] = (e == 0 ? before : w[2 * e - 1] >> 16) | (w[2 * e] & 0xffff0000u);
+      }
+      bf16_t* o = op + 3 * kh * P + oh * OW;
+      store_words<V>(o, left);
+      store_words<V>(o + P, even);
+      store_words<V>(o + 2 * P, odd);
+    }
+}
+template <typename E, int V>
+__global__ void __launch_bounds__(256)
+taps_spread3_kernel(const bf16_t* __restrict__ dxc, bf16_t* __restrict__ dx, int OH, int OW, unsigned planes) {
+  const int b = threadIdx.x * V, P = OH * OW, W = 2 * OW;
+  const unsigned plane = blockIdx.x * blockDim.z + threadIdx.z;
+  if (b >= OW || plane >= planes) return;
+  const bf16_t* cp = dxc + (size_t)plane * 9 * P + b;
+  bf16_t* dp = dx + (size_t)plane * 4 * P + 2 * b;
+  const bool more = b + V < OW;
+  // tap t's elements b .. b + V of row a (zero past the plane; the last one for the taps of column 0 alone)
+  auto row = [&](float (&v)[V + 1], int t, int a, bool behind) {
+    uint32_t w[V / 2] = {};
+    uint16_t last = 0;
+    if (a < OH) {
+      load_words<V>(w, cp + t * P + a * OW);
+      if (behind && more) last = cp[t * P + a * OW + V];
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = Lo16<E>::widen((uint16_t)(e & 1 ? w[e / 2] >> 16 : w[e / 2]));
+    v[V] = Lo16<E>::widen(last);
+  };
+  for (int a = threadIdx.y; a < OH; a += blockDim.y) {
+    float c[9][V + 1];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) row(c[t], t, t < 3 ? a + 1 : a, t % 3 == 0);
+    uint32_t up[V], down[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      // (the taps in the order of their rows and columns, from zero on)
+      const float v00 = 0.f + c[4][e], v01 = 0.f + c[3][e + 1] + c[5][e], v10 = 0.f + c[1][e] + c[7][e],
+                  v11 = 0.f + c[0][e + 1] + c[2][e] + c[6][e + 1] + c[8][e];
+      up[e] = (uint32_t)Lo16<E>::narrow(v00) | ((uint32_t)Lo16<E>::narrow(v01) << 16);
+      down[e] = (uint32_t)Lo16<E>::narrow(v10) | ((uint32_t)Lo16<E>::narrow(v11) << 16);
+    }
+    store_words<2 * V>(dp + 2 * a * W, up);
+    store_words<2 * V>(dp + (2 * a + 1) * W, down);
   }
 }
 
@@ -950,7 +1074,20 @@ inline bool plane_block(int cols, int rows, dim3* b) {
   return true;
 }
 
+bool halved3(const ConvGeom& g) { return g.KH == 3 && g.KW == 3 && g.py == 1 && g.px == 1; }
 bool taps_gather(const ConvGeom& g, const void* x, void* xc, hipStream_t s) {
+  if (const int v = halved3(g) ? halved(g, x, xc) : 0) {
+    dim3 blk;
+    if (plane_block(g.OW / v, g.OH, &blk)) {
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((g.N * g.C + blk.z - 1) / blk.z)), blk, 0, s, static_cast<const bf16_t*>(x), static_cast<bf16_t*>(xc),
+                           g.OH, g.OW, (unsigned)(g.N * g.C));
+      };
+      if (v == 4) go(taps_gather3_kernel<4>);
+      else go(taps_gather3_kernel<2>);
+      return true;
+    }
+  }
   const bool pair = g.OW % 2 == 0 && ((uintptr_t)xc & 3) == 0;
   dim3 block;
   if (!plane_block(g.OW / (pair ? 2 : 1), g.OH, &block)) return false;
@@ -961,6 +1098,18 @@ bool taps_gather(const ConvGeom& g, const void* x, void* xc, hipStream_t s) {
 }
 template <typename E>
 bool taps_spread(const ConvGeom& g, const void* dxc, void* dx, hipStream_t s) {
+  if (const int v = halved3(g) ? halved(g, dxc, dx) : 0) {
+    dim3 blk;
+    if (plane_block(g.OW / v, g.OH, &blk)) {
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((g.N * g.C + blk.z - 1) / blk.z)), blk, 0, s, static_cast<const bf16_t*>(dxc), static_cast<bf16_t*>(dx),
+                           g.OH, g.OW, (unsigned)(g.N * g.C));
+      };
+      if (v == 4) go(taps_spread3_kernel<E, 4>);
+      else go(taps_spread3_kernel<E, 2>);
+      return true;
+    }
+  }
   const bool pair = g.W % 2 == 0 && ((uintptr_t)dx & 3) == 0;
   const bool s2 = g.sy == 2 && g.sx == 2 && g.dly == 1 && g.dlx == 1 && g.KH <= 4 && g.KW <= 4;
   dim3 block;

@@ -1667,6 +1667,32 @@ def test_backward_passes_by_plan(shape, dtype):
     assert L.flhip_conv2d_plan_name(capi.CONV_BWD_DATA, nd) is None
 
 
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("xs,K", [((3, 72, 8, 16), 64), ((2, 64, 2, 8), 72), ((5, 64, 12, 12), 136), ((2, 128, 6, 20), 128), ((2, 64, 4, 4), 64),   # pieces of 4 and 2
+                                  ((2, 64, 6, 6), 64), ((3, 64, 7, 8), 64), ((2, 64, 8, 9), 64),                                                 # odd: element by element
+                                  ((4, 128, 56, 56), 128), ((1, 64, 4, 520), 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_strided_16_bit_layers_over_halved_planes(xs, K, k, dtype):
+    """The copies around strided layers move whole pieces of planes that the stride halves; against float64, one rounding per result (two
+    where backward-data keeps a product per tap) and fp32 sums."""
+    import torch.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(xs[2] + K + k)
+    x = torch.randn(xs, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(K, xs[1], k, k, generator=g, device="cuda") / (xs[1] * k * k) ** 0.5).to(dtype)
+    geo = dict(sx=2, sy=2, px=k // 2, py=k // 2)
+    y, kept = fa.ops.conv2d(x, w, None, keep_gathered=True, **geo)
+    dy = torch.randn(y.shape, generator=g, device="cuda").to(dtype)
+    dx = fa.ops.conv2d_backward_data(dy, xs, w, **geo)
+    dw = [fa.ops.conv2d_backward_filter_bias(dy, x, w.shape, False, gathered=q, **geo)[0] for q in (kept, None)]
+    xd, wd = x.double().cpu().requires_grad_(), w.double().cpu().requires_grad_()
+    ref = F.conv2d(xd, wd, stride=2, padding=k // 2)
+    ref.backward(dy.double().cpu())
+    rel = lambda a, b: float((a.double().cpu() - b).norm() / b.norm())
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert rel(y, ref.detach()) <= unit and rel(dx, xd.grad) <= 1.5 * unit
+    assert all(rel(v, wd.grad) <= 1e-5 for v in dw)
+
+
 @pytest.mark.parametrize("xs,K,stride", [
     ((33, 256, 12, 12), 256, 1),       # one round of workgroups over whole planes
     ((23, 256, 14, 14), 200, 1),       # half planes; a last tile of result channels that is not full
