@@ -515,7 +515,7 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
   if (plan >= 0) {
     FLHIP_REQUIRE(plan < kNumFilterPlans, "conv2d_bwd_filter: unknown plan");
     if (plan == 9) return bwd_filter_direct(d, g, x, dy, dw, db, s);
-    const size_t need = flhip_conv2d_workspace_bytes(d, FLHIP_CONV_BWD_FILTER);
+    const size_t need = filter_ws(g, d->dtype, plan == 10 || g.C <= 256 || d->dtype == FLHIP_F32, false);      // (no plan runs the 3x3 windows' parts)
     FLHIP_REQUIRE(ws_bytes >= need && (ws || need == 0), "conv2d_bwd_filter: workspace too small");
     const bool lo = is_lo16(d->dtype);
     int r = -1;
@@ -534,6 +534,9 @@ static int bwd_filter_impl(const flhip_conv_desc* d, const void* x, const void* 
     return r < 0 ? FLHIP_DECLINED : r;
   }
   if (!force_direct()) {
+    // (a workspace of the size that the general kernels ask for runs those)
+    parts = parts && ws_bytes >= filter_ws(g, d->dtype, one_row);
+    one_row = one_row && (g.C <= 256 || d->dtype == FLHIP_F32 || ws_bytes >= filter_ws(g, d->dtype, true, parts));
     const size_t need = filter_ws(g, d->dtype, one_row, parts);
     FLHIP_REQUIRE(ws_bytes >= need && (ws || need == 0), "conv2d_bwd_filter: workspace too small");
     int r = -1;
@@ -610,9 +613,9 @@ extern "C" int flhip_conv2d_bwd_filter_static(const flhip_conv_desc* d, const vo
   ConvGeom g;
   const int rc = make_geom(d, &g);
   if (rc != FLHIP_OK) return rc;
-  // (fp32 one-row windows of more than 256 channels: their own kernels' copy of the input and partial tiles, or, where those do not fit, the
+  // (one-row windows of more than 256 channels: their own kernels' copy of the input and partial tiles, or, where those do not fit, the
   // general kernels, which ask for less)
-  const bool one_row = !(d->dtype == FLHIP_F32 && g.C > 256) || filter_ws(g, d->dtype, true) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
+  const bool one_row = g.C <= 256 || filter_ws(g, d->dtype, true) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
   // (3x3 windows in three parts, likewise, where their partial tiles fit)
   const bool parts = filter_ws(g, d->dtype, one_row) <= (size_t)FLHIP_STATIC_SCRATCH_BYTES;
   const size_t need = filter_ws(g, d->dtype, one_row, parts);

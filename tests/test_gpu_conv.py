@@ -904,6 +904,26 @@ def test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dt
     assert float((dw.double().view(k, xs[1], kw) - want).norm() / want.norm()) <= 2 * (n ** 0.5 + 1) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("xs,k,kw", [((2, 512, 17, 17), 250, 22), ((16, 320, 1, 1500), 320, 21)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_filter_gradient_of_16_bit_one_row_windows_in_little_room(xs, k, kw, dtype):
+    """16-bit one-row windows of more than 256 channels, whose own kernels ask for more than the static buffer holds: there, and with a workspace of that
+    size, the general kernels."""
+    import ctypes as C
+    from flashlight_amd import capi, ops
+    test_static_filter_gradient_of_one_row_windows_that_do_not_fit(xs, k, kw, dtype)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(*xs, generator=g, device="cuda").to(dtype)
+    dy = torch.randn(xs[0], k, xs[2], xs[3] + 2 * (kw // 2) - kw + 1, generator=g, device="cuda").to(dtype)
+    cd = capi.ConvDesc(*xs, k, 1, kw, 1, 1, 0, kw // 2, 1, 1, 1, ops._dtype_tag(x))
+    a, b = (torch.empty(k, xs[1], 1, kw, device="cuda") for _ in range(2))
+    ops.conv2d_backward_filter_bias_static(dy, x, a, None, px=kw // 2)
+    ws = torch.empty(capi.STATIC_SCRATCH_BYTES, dtype=torch.uint8, device="cuda")
+    P = lambda t: C.c_void_p(t.data_ptr())
+    capi.check(capi.lib().flhip_conv2d_bwd_filter(C.byref(cd), P(x), P(dy), P(b), None, P(ws), ws.numel(), C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.isfinite(a).all() and float((a - b).norm() / a.norm()) <= 1e-5
+
+
 @pytest.mark.parametrize("xs,k,kw,stride", [((5, 88, 1, 2139), 188, 12, 2), ((9, 39, 1, 1911), 318, 12, 1), ((4, 250, 1, 1100), 250, 9, 1),
                                             ((11, 80, 1, 1134), 250, 15, 1), ((8, 80, 1, 1529), 250, 11, 2)])
 def test_static_filter_gradient_of_long_one_row_windows(xs, k, kw, stride):
