@@ -251,12 +251,12 @@ bool bn_desc(const Tensor& x, PyObject* axes, flhip_bn_desc* d) {
   }
   return true;
 }
-// fp32 running statistics or None
-bool running(PyObject* o, const Tensor** t) {
+// running statistics, fp32 and one for each of n features (they are updated in place), or none of them
+bool running(PyObject* o, int64_t n, const Tensor** t) {
   *t = nullptr;
   if (o == Py_None) return true;
   *t = plain(o);
-  return *t && (*t)->scalar_type() == at::kFloat;
+  return *t && (*t)->scalar_type() == at::kFloat && ((*t)->numel() == n || (*t)->numel() == 0);
 }
 
 // input, weight, bias, running mean, running var, axes, epsilon
@@ -285,8 +285,8 @@ PyObject* batchnorm_relu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   flhip_bn_desc d;
   double momentum, eps;
   bool relu, want;
-  if (!x || tag_of(*x) < 0 || !bn_desc(*x, a[5], &d) || !vector(a[1], d.C, &g) || !vector(a[2], d.C, &b) || !running(a[3], &m) ||
-      !running(a[4], &v) || !number(a[6], &momentum) || !number(a[7], &eps) || !truth(a[9], &relu) || !truth(a[10], &want))
+  if (!x || tag_of(*x) < 0 || !bn_desc(*x, a[5], &d) || !vector(a[1], d.C, &g) || !vector(a[2], d.C, &b) || !running(a[3], d.C, &m) ||
+      !running(a[4], d.C, &v) || !number(a[6], &momentum) || !number(a[7], &eps) || !truth(a[9], &relu) || !truth(a[10], &want))
     return none();
   if (a[8] != Py_None) {
     r = plain(a[8]);

@@ -380,6 +380,9 @@ def batchnorm_relu(input, weight, bias, running_mean, running_var, axes, momentu
     x = _dev(input, "input")
     _, ref, Cc, _ = _bn_plan(x.shape, tuple(map(int, axes)), _dtype_tag(x))
     g, b = _f32vec(weight, Cc, "weight"), _f32vec(bias, Cc, "bias")
+    for t, name in ((running_mean, "runningMean"), (running_var, "runningVar")):
+        if t is not None and t.numel() > 0 and (t.dtype != torch.float32 or t.numel() != Cc):
+            raise ValueError("batchnormRelu: %s must be fp32 with one element per feature" % name)
     r = _dev(residual, "residual")
     if r is not None and (r.shape != x.shape or r.dtype != x.dtype):
         raise ValueError("batchnormRelu: the residual must match the input")

@@ -62,6 +62,14 @@ def _both(f, declines=False):
     assert seen and any(seen) != declines, seen
 
 
+def _refused(*fs):
+    """Calls that either way refuses on the host, before a kernel could read or write past an operand's end."""
+    for f in fs:
+        _both(f, declines=True)
+        with pytest.raises(ValueError):
+            f()
+
+
 def _r(*shape, dtype=torch.float32):
     g = torch.Generator(device="cuda").manual_seed(sum(shape) + len(shape))
     return torch.randn(*shape, generator=g, device="cuda").to(dtype)
@@ -146,6 +154,22 @@ def test_batch_norm(dtype, shape, axes):
         mask = ops.batchnorm_relu(x, w, b, None, None, axes, 0.1, 1e-5, want_mask=True)[3]
         _both(lambda: ops.batchnorm_relu_backward(g, x, None, w, sm, si, axes, mask=mask))
         _both(lambda: ops.batchnorm_relu_backward(g, x, None, w, sm, si, axes, mask=mask[1:]), declines=True)
+
+
+@pytest.mark.parametrize("want_mask", [False, True])
+def test_running_statistics_that_are_refused(want_mask):
+    """They are updated in place, one of them per feature."""
+    x, m, v = _r(2, 16, 8, 8), _r(16), _r(16).abs()
+    call = lambda m, v: lambda: ops.batchnorm_relu(x, None, None, m, v, [2], 0.1, 1e-5, want_mask=want_mask)
+    _refused(call(m[:15], v), call(m, v[:1]), call(_r(17), v), call(m, _r(32)), call(m.half(), v), call(m, v.double()), call(None, v[:8]))
+
+    def taken(*k):
+        t = [None if s is None else s.clone() for s in k]
+        return ops.batchnorm_relu(x, None, None, *t, [2], 0.1, 1e-5, want_mask=want_mask), t
+    _both(lambda: taken(m, v))
+    _both(lambda: taken(m.reshape(1, 16, 1, 1), v.reshape(4, 4)))
+    _both(lambda: taken(None, None))
+    _both(lambda: taken(m[:0], v[:0]))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
