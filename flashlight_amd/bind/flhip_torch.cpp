@@ -179,7 +179,7 @@ PyObject* conv2d_backward_data(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor *g = plain(a[0]), *w = plain(a[2]), *add = nullptr;
   int32_t xs[4], ws[4], ys[4];
   flhip_conv_desc d;
-  if (!g || !w || tag_of(*g) < 0 || !four(a[1], xs) || !four(*w, ws) || !conv_desc(xs, ws, a + 3, tag_of(*g), &d, ys) || !same(*g, ys))
+  if (!g || !w || tag_of(*g) < 0 || w->scalar_type() != g->scalar_type() || !four(a[1], xs) || !four(*w, ws) || !conv_desc(xs, ws, a + 3, tag_of(*g), &d, ys) || !same(*g, ys))
     return none();
   if (a[10] != Py_None) {
     add = plain(a[10]);
@@ -205,12 +205,12 @@ PyObject* conv2d_backward_filter_bias(PyObject*, PyObject* const* a, Py_ssize_t 
   int32_t xs[4], ws[4], ys[4];
   flhip_conv_desc d;
   bool want_bias;
-  if (!g || !x || tag_of(*x) < 0 || !four(*x, xs) || !four(a[2], ws) || !truth(a[3], &want_bias) ||
+  if (!g || !x || tag_of(*x) < 0 || g->scalar_type() != x->scalar_type() || !four(*x, xs) || !four(a[2], ws) || !truth(a[3], &want_bias) ||
       !conv_desc(xs, ws, a + 4, tag_of(*x), &d, ys) || !same(*g, ys))
     return none();
   if (a[11] != Py_None) {
     kept = plain(a[11]);
-    if (!kept || kept->numel() != (int64_t)flhip_conv2d_gathered_bytes(&d)) return none();
+    if (!kept || kept->scalar_type() != at::kByte || kept->numel() != (int64_t)flhip_conv2d_gathered_bytes(&d)) return none();
   }
   const Tensor dw = sized(ws, x->options().dtype(at::kFloat));
   Tensor db, scratch;

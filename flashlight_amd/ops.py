@@ -161,6 +161,8 @@ def conv2d_backward_data(grad_output, input_shape, weights, sx=1, sy=1, px=0, py
     if out is not None:
         return out
     g, w = _dev(grad_output, "gradOutput"), _dev(weights, "weights")
+    if g.dtype != w.dtype:
+        raise ValueError("conv2dBackwardData: gradOutput and weights must have the same type")
     tag = _dtype_tag(g)
     _, ref, shape = _conv_plan(tuple(input_shape), w.shape, sx, sy, px, py, dx, dy, groups, tag)
     if tuple(g.shape) != shape:
@@ -189,6 +191,8 @@ def conv2d_backward_filter_bias(grad_output, input, weights_shape, want_bias, sx
     if out is not None:
         return out
     g, x = _dev(grad_output, "gradOutput"), _dev(input, "input")
+    if g.dtype != x.dtype:
+        raise ValueError("conv2dBackwardFilterBias: gradOutput and input must have the same type")
     tag = _dtype_tag(x)
     d, ref, shape = _conv_plan(x.shape, tuple(weights_shape), sx, sy, px, py, dx, dy, groups, tag)
     if tuple(g.shape) != shape:
@@ -199,9 +203,10 @@ def conv2d_backward_filter_bias(grad_output, input, weights_shape, want_bias, sx
     nws = lib.flhip_conv2d_workspace_bytes(ref, capi.CONV_BWD_FILTER)
     ws = _ws(nws, x.device) if nws else None
     if gathered is not None:
-        if gathered.numel() != lib.flhip_conv2d_gathered_bytes(ref):
+        k = _dev(gathered, "gathered")
+        if k.dtype != torch.uint8 or k.numel() != lib.flhip_conv2d_gathered_bytes(ref):
             raise ValueError("conv2dBackwardFilterBias: gathered input of another geometry")
-        capi.check(lib.flhip_conv2d_bwd_filter_gathered(ref, _ptr(gathered), _ptr(g), _ptr(dw), _ptr(db), _ptr(ws), nws, _stream()))
+        capi.check(lib.flhip_conv2d_bwd_filter_gathered(ref, _ptr(k), _ptr(g), _ptr(dw), _ptr(db), _ptr(ws), nws, _stream()))
         return dw, db
     capi.check(lib.flhip_conv2d_bwd_filter(ref, _ptr(x), _ptr(g), _ptr(dw), _ptr(db), _ptr(ws), nws, _stream()))
     return dw, db
@@ -214,8 +219,13 @@ def conv2d_backward_filter_bias_static(grad_output, input, dw, db, sx=1, sy=1, p
     results in the library's static buffer.  Neither this wrapper nor the library
     allocates device memory."""
     g, x = _dev(grad_output, "gradOutput"), _dev(input, "input")
+    dw, db = _dev(dw, "gradWeights"), _dev(db, "gradBias")
     if dw.dtype != torch.float32 or (db is not None and db.dtype != torch.float32):
         raise ValueError("conv2dBackwardFilterBias: gradients are fp32")
+    if g.dtype != x.dtype:
+        raise ValueError("conv2dBackwardFilterBias: gradOutput and input must have the same type")
+    if db is not None and 0 < db.numel() < dw.shape[0]:
+        raise ValueError("conv2dBackwardFilterBias: gradBias must have one element per output channel")
     d = _conv_desc(x.shape, tuple(dw.shape), sx, sy, px, py, dx, dy, groups, _dtype_tag(x))
     oh, ow = C.c_int32(), C.c_int32()
     capi.check(capi.lib().flhip_conv2d_out_dims(C.byref(d), C.byref(oh), C.byref(ow)))

@@ -119,6 +119,29 @@ def test_convolutions_that_are_refused():
         _both(f, declines=True)
 
 
+def test_convolutions_of_operands_that_are_refused():
+    """Operands of two types, and a gathered input that is not the forward call's bytes."""
+    geo, xs, ws = dict(sx=2, sy=2), (3, 128, 28, 28), (128, 128, 1, 1)
+    x, w = _r(*xs, dtype=torch.bfloat16), _r(*ws, dtype=torch.bfloat16)
+    y, kept = ops.conv2d(x, w, None, keep_gathered=True, **geo)
+    assert kept is not None and kept.dtype == torch.uint8
+    n, g, dw, db = kept.numel(), _r(*y.shape, dtype=torch.bfloat16), torch.empty(ws, device="cuda"), torch.empty(128, device="cuda")
+    _both(lambda: ops.conv2d_backward_filter_bias(g, x, ws, True, gathered=kept, **geo))
+    data, grads = ops.conv2d_backward_data, ops.conv2d_backward_filter_bias
+    _refused(lambda: data(g, xs, w.float(), **geo), lambda: data(g.float(), xs, w, **geo), lambda: data(g, xs, w.half(), **geo),
+             lambda: data(g, xs, w.to(torch.uint8), **geo), lambda: data(g.half(), xs, w, addend=x.half(), **geo),
+             lambda: grads(g.float(), x, ws, True, **geo), lambda: grads(g, x.float(), ws, True, **geo), lambda: grads(g.half(), x, ws, False, **geo),
+             lambda: grads(g, x, ws, True, gathered=torch.zeros(n, dtype=torch.bool, device="cuda"), **geo),
+             lambda: grads(g, x, ws, True, gathered=torch.zeros(n, device="cuda"), **geo),
+             lambda: grads(g, x, ws, True, gathered=torch.zeros(2 * n, dtype=torch.uint8, device="cuda")[::2], **geo),
+             lambda: grads(g, x, ws, True, gathered=kept.cpu(), **geo))
+    static = ops.conv2d_backward_filter_bias_static
+    for f in (lambda: static(g.float(), x, dw, db, **geo), lambda: static(g, x, dw, db[:127], **geo), lambda: static(g, x, dw.half(), db, **geo),
+              lambda: static(g, x, dw.transpose(0, 1), db, **geo)):
+        with pytest.raises(ValueError):
+            f()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape,axes", [((3, 8, 14, 14), [2]), ((2, 5, 7, 9), (2,)), ((4, 3, 2, 5), [0, 1, 2]), ((6, 10), [0]), ((3, 4, 5), [1, 2])])
 def test_batch_norm(dtype, shape, axes):
