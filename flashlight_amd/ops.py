@@ -276,6 +276,11 @@ def pool2d_backward(grad_output, input_shape, argmax, wx, wy, sx, sy, px, py,
     if int(mode) == PoolingMode.MAX and argmax is None:
         raise ValueError("pool2dBackward: max pooling needs the forward payload")
     am = _dev(argmax, "argmax") if argmax is not None else None
+    oh, ow = C.c_int32(), C.c_int32()
+    capi.check(capi.lib().flhip_pool2d_out_dims(C.byref(d), C.byref(oh), C.byref(ow)))
+    n = s4[0] * s4[1] * oh.value * ow.value
+    if g.numel() < n or (int(mode) == PoolingMode.MAX and (am.dtype != torch.uint8 or am.numel() < n)):
+        raise ValueError("pool2dBackward: gradOutput or the forward payload does not match the geometry")
     out = torch.empty(s4, dtype=g.dtype, device=g.device)
     capi.check(capi.lib().flhip_pool2d_bwd(C.byref(d), _ptr(g), _ptr(am), _ptr(out), _stream()))
     return out
@@ -318,6 +323,16 @@ def _f32vec(t, n, name):
         raise ValueError("batchnorm: %s must have one element per feature" % name)
     t = _dev(t, name)
     return t if t.dtype == torch.float32 else t.float()
+
+
+def _saved(t, n, name):
+    """A statistic that the forward pass saved."""
+    if t is None:
+        raise ValueError("batchnorm: the backward pass needs the forward payload")
+    t = _dev(t, name)
+    if t.dtype != torch.float32 or t.numel() < n:
+        raise ValueError("batchnorm: %s must be fp32 with one element per feature" % name)
+    return t
 
 
 def batchnorm(input, weight, bias, running_mean, running_var, axes, train, momentum, epsilon):
@@ -367,6 +382,7 @@ def batchnorm_backward(grad_output, input, weight, save_mean, save_invstd, axes)
         raise ValueError("batchnormBackward: needs the forward payload")
     _, ref, Cc, _ = _bn_plan(x.shape, tuple(map(int, axes)), _dtype_tag(x))
     w = _f32vec(weight, Cc, "weight")
+    save_mean, save_invstd = _saved(save_mean, Cc, "saveMean"), _saved(save_invstd, Cc, "saveInvStd")
     dx = torch.empty_like(x)
     dg = torch.empty((Cc,), dtype=torch.float32, device=x.device)
     db = torch.empty((Cc,), dtype=torch.float32, device=x.device)
@@ -433,6 +449,7 @@ def batchnorm_relu_backward(grad_output, input, output, weight, save_mean, save_
         raise ValueError("batchnormReluBackward: output must match the input")
     _, ref, Cc, _ = _bn_plan(x.shape, tuple(map(int, axes)), _dtype_tag(x))
     w = _f32vec(weight, Cc, "weight")
+    save_mean, save_invstd = _saved(save_mean, Cc, "saveMean"), _saved(save_invstd, Cc, "saveInvStd")
     dx = torch.empty_like(x)
     dr = torch.empty_like(x) if want_residual_grad else None
     dg = torch.empty((Cc,), dtype=torch.float32, device=x.device)
@@ -640,10 +657,14 @@ def sgd_step(params, grads, velocities, lr, momentum=0.0, weight_decay=0.0, nest
     n = len(ps)
     if n == 0:
         return
+    counts, kinds = [p.numel() for p in ps], {p.dtype for p in ps}
+    for l in (gs, vs):
+        if l is not None and (len(l) != n or any(map(operator.lt, [t.numel() for t in l], counts)) or {t.dtype for t in l} != kinds or len(kinds) > 1):
+            raise ValueError("sgdStep: gradients and velocities that match the parameters expected, all of one type")
     pa = (C.c_void_p * n)(*[p.data_ptr() for p in ps])
     ga = (C.c_void_p * n)(*[g.data_ptr() for g in gs])
     va = (C.c_void_p * n)(*[v.data_ptr() for v in vs]) if vs is not None else None
-    cnt = (C.c_size_t * n)(*[p.numel() for p in ps])
+    cnt = (C.c_size_t * n)(*counts)
     capi.check(capi.lib().flhip_sgd_many(pa, ga, va, cnt, n, float(lr), float(momentum), float(weight_decay),
                                          int(bool(nesterov)), _dtype_tag(ps[0]), _stream()))
 
@@ -734,6 +755,8 @@ def log_softmax_backward(grad_output, output):
     if dx is not None:
         return dx
     g, y = _dev(grad_output, "gradOutput"), _dev(output, "output")
+    if g.dtype != y.dtype or g.numel() < y.numel():
+        raise ValueError("logSoftmax backward: gradOutput must match the output")
     dx = torch.empty_like(y)
     classes = y.shape[-1]
     capi.check(capi.lib().flhip_logsoftmax_bwd(_ptr(g), _ptr(y), _ptr(dx), classes,

@@ -195,6 +195,30 @@ def test_running_statistics_that_are_refused(want_mask):
     _both(lambda: taken(m[:0], v[:0]))
 
 
+def test_other_operands_that_are_refused():
+    """Gradients, saved statistics, payloads and SGD's lists of another type, or fewer than the kernels read."""
+    x, g, w = _r(2, 16, 8, 8), _r(2, 16, 8, 8), _r(16)
+    y, sm, si, mask = ops.batchnorm_relu(x, w, None, None, None, [2], 0.1, 1e-5, want_mask=True)
+    for bad in (sm[:15], sm.half(), sm.double(), sm.cpu(), torch.empty(32, device="cuda")[::2], None):
+        for a, b in ((bad, si), (sm, bad)):
+            _refused(lambda: ops.batchnorm_backward(g, x, w, a, b, [2]), lambda: ops.batchnorm_relu_backward(g, x, y, w, a, b, [2]),
+                     lambda: ops.batchnorm_relu_backward(g, x, None, w, a, b, [2], mask=mask))
+    p, am = ops.pool2d(x, 2, 2, 2, 2, 0, 0)
+    back = lambda g, am, mode=0: lambda: ops.pool2d_backward(g, x.shape, am, 2, 2, 2, 2, 0, 0, mode)
+    _refused(back(p[:1], am), back(p, am[:, 1:].contiguous()), back(p, am.int()), back(p, am.bool()), back(p, None), back(p[:1], None, 1))
+    _both(back(p.reshape(32, 4, 4), am), declines=True)
+    _both(back(p, None, 2))
+    lp = ops.log_softmax(x)
+    _refused(lambda: ops.log_softmax_backward(g.half(), lp), lambda: ops.log_softmax_backward(g[:1], lp), lambda: ops.log_softmax_backward(g, lp.half()))
+    _both(lambda: ops.log_softmax_backward(g.reshape(-1, 8), lp), declines=True)
+    a, b = [_r(3, 5), _r(7)], lambda *f: [h(t) for h, t in zip(f, (_r(3, 5), _r(7)))]
+    own, short, half = (lambda t: t.clone()), (lambda t: t.flatten()[1:].clone()), (lambda t: t.half())
+    for bad in (b(own, short), b(half, half), b(own, half), b(own)):
+        _refused(lambda: ops.sgd_step(a, bad, b(own, own), 0.1, 0.9), lambda: ops.sgd_step(a, b(own, own), bad, 0.1, 0.9),
+                 lambda: ops.sgd_step(a, bad, None, 0.1))
+    _refused(lambda: ops.sgd_step(b(own, half), b(own, half), b(own, half), 0.1, 0.9))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_the_others(dtype):
     x, g = _r(4, 6, 9, 12, dtype=dtype), _r(4, 6, 9, 12, dtype=dtype)
