@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "flhip.h"
+#include "unlocked.h"
 
 namespace {
 
@@ -93,14 +94,6 @@ PyObject* none() { Py_RETURN_NONE; }
 PyObject* failed(int rc) {
   PyErr_SetString(rc == FLHIP_INVALID_ARGUMENT ? PyExc_ValueError : PyExc_RuntimeError, flhip_last_error());
   return nullptr;
-}
-// the launch, other threads running meanwhile
-template <typename F>
-int launched(F f) {
-  PyThreadState* const state = PyEval_SaveThread();
-  const int rc = f();
-  PyEval_RestoreThread(state);
-  return rc;
 }
 PyObject* wrap(const Tensor& t) {
   if (!t.defined()) return none();
