@@ -610,4 +610,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "flhip_torch", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_flhip_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_flhip_torch() {
+  if (flhip_version() / 100 != FLHIP_VERSION / 100)      // (descriptors of another layout)
+    return PyErr_Format(PyExc_ImportError, "flhip_torch: libflhip version %d, compiled against %d", flhip_version(), FLHIP_VERSION);
+  return PyModule_Create(&module);
+}

@@ -6,6 +6,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libflhip.so")
 BIND_PATH = os.path.join(_HERE, "lib", "flhip_torch.so")
 
+VERSION = 207          # of include/flhip.h, whose descriptors are laid out below
 OK, INVALID_ARGUMENT, RUNTIME_ERROR, DECLINED = 0, 1, 2, 3
 F32, BF16, F16 = 0, 1, 2
 CONV_FWD, CONV_BWD_DATA, CONV_BWD_FILTER = 0, 1, 2
@@ -152,6 +153,8 @@ def lib():
             f = getattr(h, name)
             f.restype = res
             f.argtypes = args
+        if h.flhip_version() // 100 != VERSION // 100:      # descriptors of another layout
+            raise RuntimeError("flashlight_amd: %s is version %d, %d expected" % (LIB_PATH, h.flhip_version(), VERSION))
         _lib = h
     return _lib
 
