@@ -1547,7 +1547,7 @@ int seq_fwd(const RnnGeom& g, SeqFwd& p, hipStream_t s) {
 // / 35, 43 / 37, 53 / 40; 3 layers over 1 step, LSTM of 320 units, 5 columns 51 / 38).
 int stack_units(const RnnGeom& g) {
   const int asked = options().rnn_sequences;
-  if (options().rnn_unfused || (asked != Options::SEQ_AUTO && asked != Options::SEQ_STACKED)) return 0;
+  if (options().rnn_unfused || asked == Options::SEQ_ALWAYS || asked == Options::SEQ_NEVER) return 0;
   if (asked == Options::SEQ_AUTO && g.L * g.T < 3) return 0;
   if (g.D != 1 || g.L < 2 || g.L > STACK_LAYERS || g.mode == RNN_RELU || g.dropout > 0.f || !seq_holds(g)) return 0;
   const int clusters = g.L * ((g.B + SEQ_COLS - 1) / SEQ_COLS), nc = ((g.H + 15) / 16 + SEQ_WAVES - 1) / SEQ_WAVES;

@@ -264,6 +264,47 @@ def test_refused_sequence_launches(mode, I, H, L, bidir, T, B, states):
         capi.set_option("RNN_SEQUENCES", None)
 
 
+@pytest.mark.parametrize("mode,I,H,L,T,B", [
+    (flref.RNN_LSTM, 9, 320, 3, 5, 5),           # 4 units per workgroup; the step kernels follow
+    (flref.RNN_GRU, 12, 48, 3, 7, 17),
+    (flref.RNN_TANH, 8, 64, 2, 6, 16),
+    (flref.RNN_LSTM, 7, 20, 2, 6, 5),            # a hidden size off 16, more than 64 columns: the two-kernel steps
+    (flref.RNN_GRU, 6, 128, 2, 6, 70),
+])
+def test_refused_launch_of_stacked_layers(mode, I, H, L, T, B):
+    """What runs where the runtime refuses the one launch of all layers, after their initial states and exchanges and the lowest layer's
+    projections have been put in place for it."""
+    g = torch.Generator(device="cuda").manual_seed(mode + H)
+    x = torch.randn(T, B, I, generator=g, device="cuda")
+    w = torch.randn(ops.rnn_param_count(I, H, L, mode, False), generator=g, device="cuda") / H ** 0.5
+    hx = torch.rand(L, B, H, generator=g, device="cuda")
+    cx = torch.randn(L, B, H, generator=g, device="cuda") if mode == flref.RNN_LSTM else None
+    count, P = capi.lib().flhip_rnn_sequence_launches, lambda t: None if t is None else C.c_void_p(t.data_ptr())
+    before = count()
+    try:
+        capi.set_option("RNN_SEQUENCES", "never")
+        want = ops.rnn(x, hx, cx, w, H, L, mode, False)
+        capi.set_option("RNN_SEQUENCES", "refused")
+        d = capi.RnnDesc(I, H, L, 0, mode, T, B, capi.F32)
+        n = capi.lib().flhip_rnn_workspace_bytes(C.byref(d))
+        ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+        got = [torch.zeros_like(t) if t is not None else None for t in want]
+        y, hy, cy, reserve = got
+        capi.check(capi.lib().flhip_rnn_fwd(C.byref(d), P(x), P(hx), P(cx), P(w), P(y), P(hy), P(cy), P(reserve), reserve.numel() * reserve.element_size(),
+                                            P(ws), n, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    finally:
+        capi.set_option("RNN_SEQUENCES", None)
+    assert count() == before
+    # elements not yet written (-1) of the exchanges of all layers, T rows each; one layer's own leaves T - 1
+    assert int((ws[: n // 4 * 4].view(torch.int32) == -1).sum()) > T * B * ((H + 15) // 16 * 16)
+    for a, b in zip(got[:3], want[:3]):
+        if b is None:
+            continue
+        assert rel_l2(host(a), host(b)) <= 1e-5      # the same sums in another order
+        if H % 16 == 0 and B <= 64:
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("H,B,bidir,T,fwd,bwd", [
     (64, 16, False, 7, 0, 0), (64, 16, False, 8, 1, 1), (64, 32, True, 5, 0, 0), (64, 32, True, 6, 1, 1),
     (64, 33, False, 4, 0, 0), (64, 33, False, 5, 1, 1),
