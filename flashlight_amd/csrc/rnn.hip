@@ -1252,6 +1252,8 @@ struct BiasSums {
   const float* x[4];
   float *a[4], *b[4];      // where a sum goes, and where else (or null)
 };
+// Up to 1024 rows, 32 additions one after the other in a thread: 0.81 to 1.00 of the pass with the column sums' own launches (72 random layers, 0 to 28 us less).
+// (Above it would still be up to 55 us less, GRU of 768 units, two directions, 2 layers, 1379 rows 2311 / 2256, but the chains of additions grow with the rows.)
 constexpr int BIAS_ROWS = 1024;
 __global__ void __launch_bounds__(1024) rnn_bias_kernel(BiasSums p, int GH, int TB) {
   __shared__ float sums[32][33];
@@ -1891,7 +1893,9 @@ int backward_layer_fused(const RnnGeom& g, int l, const float* in, size_t inl, c
   const Scratch sc = scratch_of(g, ws);
   Offsets os[2];
   const float *hps[2], *gws[2], *grs[2];
-  // gradients of the layer input: where they are small and neither is cut into slices, both directions' in a launch and one that adds them
+  // gradients of the layer input: where they are small and neither is cut into slices, both directions' in a launch and one that adds them (of the pass
+  // 0.69 to 1.01; above it is level, us as it is / in one launch: 2873 columns of 512 inputs 1595 / 1596, 4641 of 40 and 1280 1373 / 1381, 4876 of 512
+  // 396 / 388, 2220 of 1024 226 / 219)
   int pair = -1;
   if (g.D == 2 && TB * inl <= 512 * 1024 && gemm32_ws_bytes(0, (int)inl, (int)TB, (int)g.GH) == 0) {
     pair = gemm32_pair(0, w + offsets(g, l * 2).W, w + offsets(g, l * 2 + 1).W, dGW[0], dGW[1], gin, tmp, (int)inl, (int)TB, (int)g.GH, nullptr, nullptr,

@@ -95,6 +95,28 @@ def test_both_directions_share_their_products(mode, I, H, L, T, B):
     test_rnn_forward_backward(mode, I, H, L, True, T, B, True)
 
 
+@pytest.mark.parametrize("option,value", [("MATMUL_VALU", "1"), ("MATMUL_PLANES", "0"), ("MATMUL_PLANES", "7")])
+def test_both_directions_keep_to_the_kernels_that_are_asked_for(option, value):
+    """The projections of two directions under a switch that chooses between the products' kernels: a direction's outputs have the bits of a layer of
+    that direction alone, which makes its projections by itself."""
+    I, H, T, B, G = 40, 64, 10, 16, 4
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn(T, B, I, generator=g, device="cuda")
+    w = torch.randn(ops.rnn_param_count(I, H, 1, ops.RNN_LSTM, True), generator=g, device="cuda") / H ** 0.5
+    mats, biases = G * H * (I + H), 2 * G * H
+    try:
+        capi.set_option("RNN_SEQUENCES", "never")
+        capi.set_option(option, value)
+        y = ops.rnn(x, None, None, w, H, 1, ops.RNN_LSTM, True)[0]
+        for k in (0, 1):
+            one = torch.cat([w[k * mats:(k + 1) * mats], w[2 * mats + k * biases:2 * mats + (k + 1) * biases]])
+            z = ops.rnn(x.flip(0).contiguous() if k else x, None, None, one, H, 1, ops.RNN_LSTM, False)[0]
+            assert torch.equal(y[:, :, k * H:(k + 1) * H], z.flip(0) if k else z)
+    finally:
+        capi.set_option(option, None)
+        capi.set_option("RNN_SEQUENCES", None)
+
+
 @pytest.mark.parametrize("mode,I,H,L,bidir,T,B,states", [
     # whole sequences in one launch: hidden sizes that are multiples of 4 up to 1024.  4, 8 and 16 units per workgroup,
     # a last workgroup with units to spare, a last contraction chunk with columns to spare, more waves than chunks
