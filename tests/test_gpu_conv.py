@@ -1800,3 +1800,42 @@ def test_filter_gradient_of_3x3_windows_in_three_parts(xs, K):
     fine = torch.isfinite(ref)
     assert rel(got[fine], ref[fine]) <= 2e-6
     assert torch.equal(run(torch.zeros_like(x), g), torch.zeros_like(got))
+
+
+def _classes(t):
+    """0 finite, 1 / 2 infinite, 3 NaN"""
+    t = t.double().cpu()
+    return torch.where(t.isnan(), 3, torch.where(t.isposinf(), 1, torch.where(t.isneginf(), 2, 0)))
+
+
+def _taps(xs, ws, stride):
+    """(window row, column, results that the tap has a position for, those positions) of each tap of a window, padding of half its size"""
+    def along(size, k, s, j):
+        p = k // 2
+        o = [i for i in range((size + 2 * p - k) // s + 1) if 0 <= i * s + j - p < size]
+        return slice(o[0], o[-1] + 1), slice(o[0] * s + j - p, o[-1] * s + j - p + 1, s)
+    sy = stride if ws[2] > 1 else 1
+    for i in range(ws[2]):
+        for j in range(ws[3]):
+            (oy, iy), (ox, ix) = along(xs[2], ws[2], sy, i), along(xs[3], ws[3], stride, j)
+            yield i, j, (slice(None), slice(None), oy, ox), (slice(None), slice(None), iy, ix)
+
+
+@pytest.mark.parametrize("xs,k,kw,stride", [((2, 320, 1, 300), 70, 21, 1), ((2, 272, 1, 501), 64, 11, 1), ((4, 384, 1, 402), 80, 9, 2),
+                                            ((3, 48, 1, 101), 40, 8, 1), ((3, 100, 1, 143), 64, 6, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_16_bit_one_row_filter_gradient_of_what_is_not_finite_at_a_rows_end(xs, k, kw, stride, dtype):
+    """Rows that end within a step of 16 positions: what is not finite there reaches the taps that meet it, and no others."""
+    g = torch.Generator(device="cuda").manual_seed(kw)
+    x = (torch.rand(xs, generator=g, device="cuda") + 0.5).to(dtype)
+    x[0, 1, 0, -1], x[1, xs[1] - 1, 0, -2], x[0, 9, 0, -3] = float("inf"), float("-inf"), float("nan")
+    ow = (xs[3] + 2 * (kw // 2) - kw) // stride + 1
+    dy = (torch.rand(xs[0], k, 1, ow, generator=g, device="cuda") + 0.5).to(dtype)
+    got = fa.conv2d_backward_filter_bias(dy, x, (k, xs[1], 1, kw), False, sx=stride, px=kw // 2)[0].double().cpu()
+    want = torch.empty(k, xs[1], 1, kw, dtype=torch.float64)
+    xd, d = x.double().cpu(), dy.double().cpu()
+    for i, j, o, p in _taps(xs, want.shape, stride):
+        want[:, :, i, j] = d[o].transpose(0, 1).reshape(k, -1) @ xd[p].transpose(0, 1).reshape(xs[1], -1).t()
+    assert torch.equal(_classes(got), _classes(want))
+    ok = want.isfinite()
+    assert 0 < int((~ok).sum()) < 4 * k * kw and float(((got - want)[ok] / want[ok]).abs().max()) <= 1e-4      # (fp32 sums of up to 1600 positive terms)
