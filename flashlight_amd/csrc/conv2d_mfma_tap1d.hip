@@ -96,6 +96,7 @@ struct Tap1Params {
   int d0[2];             // source offset of tap 0 of a phase, relative to the slab's first position
   int smin;              // slab's first source position for result 0
   int SR, half;          // slab rows; stride 2: row of the first odd source offset
+  int zcells;            // cells of zeros behind them, for the taps that do not exist (0: there are none)
   int taps_total;        // ntaps[0] + ntaps[1]
   int ptiles, mtiles;
   unsigned src_bytes, w_bytes, dst_bytes;
@@ -284,7 +285,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   {
     const intx4_t xrs = pd_rsrc(xr, p.src_bytes);
     const unsigned base = pd_lds_addr(t1_slab);
-    const int ncell = p.SR * CPR, ninstr = (ncell + 63) >> 6;
+    const int ncell = p.SR * CPR + p.zcells, ninstr = (ncell + 63) >> 6;
     const float inv = 1.0f / (float)CPR;
     for (int ii = wave; ii < ninstr; ii += 4) {
       const int L = ii * 64 + lane;
@@ -319,9 +320,9 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
       for (int r = 0; r < 16; ++r) acc[q][b][r] = 0.f;
 
   const int fr = lane & 31, fg = lane >> 5;
-  lds_cell_t ap[NB];
+  int ap[NB];                                   // this lane's cell of a tap's first row
 #pragma unroll
-  for (int b = 0; b < NB; ++b) ap[b] = (lds_cell_t)t1_slab + (((wp * NB + b) * 32 + fr) * CPR + fg);
+  for (int b = 0; b < NB; ++b) ap[b] = ((wp * NB + b) * 32 + fr) * CPR + fg;
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the slab (and the first weight fragments) have landed
   __syncthreads();
@@ -331,13 +332,18 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   auto run = [&](floatx16 (&ac)[NB], int q) __attribute__((always_inline)) {
     const int groups = p.ntaps[q] / DT;
     const int dq = p.d0[q], last = p.nreal[q] - 1;
-    // slab offset (cells) of a tap's rows; padding taps read the rows of the last tap that exists: finite values
-    // times zero weights
+    // slab offset (cells) of a tap's rows.  Taps that do not exist (DT > 1) read zeros, every lane the same (`rows` takes its place in the slab off):
+    // zero weights times rows that exist would make NaN of an infinity.  (Behind the last group, where nothing is multiplied: any rows.)
+    const int real = p.zcells ? last : 1 << 30;
     auto toff_of = [&](int tap) {
+      if (DT > 1 && tap > real) return p.SR * CPR;
       const int tl = min(tap, last);
       const int d = dq + (TD ? (tl / p.tw) * p.tpitch + tl % p.tw : tl);
       const int trow = SS == 1 ? d : (d & 1) * p.half + (d >> 1);
       return trow * CPR;
+    };
+    auto rows = [&](int b, int off) __attribute__((always_inline)) {
+      return (lds_cell_t)t1_slab + ((DT > 1 && off == p.SR * CPR ? 0 : ap[b]) + off);
     };
     uintx4_t af[4][NB];
     int tcur[DT];
@@ -346,7 +352,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) af[i][b] = ap[b][tcur[i / KS] + 2 * (i % KS)];
+      for (int b = 0; b < NB; ++b) af[i][b] = rows(b, tcur[i / KS])[2 * (i % KS)];
     for (int g = 0; g < groups; ++g) {
       int tnext[DT];
 #pragma unroll
@@ -356,7 +362,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
         const int i2 = i + 2;
         const int o2 = i2 < NS ? tcur[(i2 % NS) / KS] : tnext[(i2 % NS) / KS];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) af[i2 % 4][b] = ap[b][o2 + 2 * ((i2 % NS) % KS)];
+        for (int b = 0; b < NB; ++b) af[i2 % 4][b] = rows(b, o2)[2 * ((i2 % NS) % KS)];
         const uintx4_t w8 = bq[i % RW];
         bq[i % RW] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wlane, wpos + i * 1024, 0);
 #pragma unroll
@@ -594,6 +600,7 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
   for (int q = 0; q < p.nph; ++q) {
     p.d0[q] = soff[q] - p.smin;
     span = std::max(span, p.d0[q] + p.nreal[q]);
+    if (p.ntaps[q] != p.nreal[q]) p.zcells = 2 * KS;
   }
   const int CPR = 2 * KS + 1;
   // three blocks of positions per wave; two, or one with half the channels, where the workgroups still fit the compute units at once, so that
@@ -612,7 +619,7 @@ bool tap1d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
       p.half = ((2 * (tp - 1) + span - 1) >> 1) + 1;
       p.SR = 2 * p.half;
     }
-    pl->lds_bytes = (size_t)(((long long)p.SR * CPR + 63) / 64) * 1024;
+    pl->lds_bytes = (size_t)(((long long)p.SR * CPR + p.zcells + 63) / 64) * 1024;
     if (pl->lds_bytes <= 160 * 1024) pl->NB = nb;
   }
   if (!pl->NB) return false;
@@ -733,8 +740,9 @@ bool tap2d_plan(const ConvGeom& g, bool bwd, Tap1Plan* pl) {
   pl->NB = tiles(1) * t1_mtiles(Mo, 1) <= mfma_num_cus() ? 1 : tiles(3) * t1_mtiles(Mo, 3) < mfma_num_cus() ? 2 : 3;
   const int tp = t1_positions(pl->NB);
   p.SR = tp + 2 * P + 2;
+  if (p.ntaps[0] != p.nreal[0]) p.zcells = 2 * KS;
   // the slab; the results are staged in the same memory afterwards
-  pl->lds_bytes = std::max((size_t)(((long long)p.SR * CPR + 63) / 64) * 1024, (size_t)32 * t1_wm(pl->NB) * (tp + 4) * esz);
+  pl->lds_bytes = std::max((size_t)(((long long)p.SR * CPR + p.zcells + 63) / 64) * 1024, (size_t)32 * t1_wm(pl->NB) * (tp + 4) * esz);
   if (pl->lds_bytes > 160 * 1024) return false;
   p.half = 0;
   p.ptiles = (int)tiles(pl->NB);

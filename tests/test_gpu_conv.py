@@ -1839,3 +1839,31 @@ def test_16_bit_one_row_filter_gradient_of_what_is_not_finite_at_a_rows_end(xs, 
     assert torch.equal(_classes(got), _classes(want))
     ok = want.isfinite()
     assert 0 < int((~ok).sum()) < 4 * k * kw and float(((got - want)[ok] / want[ok]).abs().max()) <= 1e-4      # (fp32 sums of up to 1600 positive terms)
+
+
+@pytest.mark.parametrize("xs,k,kh,kw,stride", [
+    ((2, 200, 1, 300), 224, 1, 21, 1), ((2, 160, 1, 131), 130, 1, 7, 2), ((3, 80, 1, 90), 96, 1, 9, 1), ((2, 60, 1, 333), 64, 1, 13, 2), ((2, 32, 1, 100), 32, 1, 5, 1),
+    ((26, 224, 14, 14), 210, 3, 3, 1), ((40, 64, 7, 7), 90, 3, 3, 1), ((40, 120, 8, 8), 128, 3, 3, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_16_bit_windows_of_what_is_not_finite(xs, k, kh, kw, stride, dtype):
+    """Channel counts whose taps are filled up to whole groups: an infinity reaches the results that it reaches, as one."""
+    g = torch.Generator(device="cuda").manual_seed(xs[1])
+    x = (torch.rand(xs, generator=g, device="cuda") + 0.5).to(dtype)
+    w = (torch.rand(k, xs[1], kh, kw, generator=g, device="cuda") / 64 + 1 / 128).to(dtype)
+    geo = dict(sx=stride, sy=stride if kh > 1 else 1, px=kw // 2, py=kh // 2)
+    x[0, 3, 0, xs[3] // 2], x[1, xs[1] - 1, xs[2] // 2, xs[3] // 2 + 1] = float("inf"), float("-inf")
+    y = fa.conv2d(x, w, None, **geo)
+    dy = (torch.rand(y.shape, generator=g, device="cuda") + 0.5).to(dtype)
+    dy[0, 2, 0, y.shape[3] // 2], dy[1, k - 1, y.shape[2] // 2, y.shape[3] // 2 + 1] = float("-inf"), float("inf")
+    dx = fa.conv2d_backward_data(dy, xs, w, **geo)
+    xd, wd, d = x.double().cpu(), w.double().cpu(), dy.double().cpu()
+    ry, rdx = torch.zeros(y.shape, dtype=torch.float64), torch.zeros(xs, dtype=torch.float64)
+    for i, j, o, p in _taps(xs, w.shape, stride):
+        at, to = xd[p].transpose(0, 1), d[o].transpose(0, 1)
+        ry[o] += (wd[:, :, i, j] @ at.reshape(xs[1], -1)).reshape(k, *at.shape[1:]).transpose(0, 1)
+        rdx[p] += (wd[:, :, i, j].t() @ to.reshape(k, -1)).reshape(xs[1], *to.shape[1:]).transpose(0, 1)
+    for got, want in ((y, ry), (dx, rdx)):
+        assert torch.equal(_classes(got), _classes(want))
+        ok = want.isfinite()
+        unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)                  # (one rounding per result, beside fp32 sums)
+        assert bool((~ok).any()) and float(((got.double().cpu() - want)[ok] / want[ok]).abs().max()) <= unit
