@@ -302,8 +302,8 @@ struct CellFwd {
 };
 
 // (The gate math below leaves no choice of fused or separate multiply-adds to the compiler, and the step kernels add in the
-// sequence kernels' order: hidden sizes that are multiples of 16 with at most 64 columns give the same bits captured and eager, stacked layers
-// of one direction apart (rnn_stack_fwd: their input products are added inside the steps).
+// sequence kernels' order: hidden sizes that are multiples of 16 with at most 64 columns give the same bits captured and eager, as do stacked
+// layers of one direction that rnn_stack_fwd takes, which runs both ways.
 // The two-kernel steps, which others run on where a sequence launch is not made, add their products in another order.)
 // gate math of one (batch b, hidden h) element, in two halves so that a kernel can issue
 // the loads before it computes the recurrent projections rp (one per gate)
@@ -936,6 +936,7 @@ struct SeqStack {
   int B, H, T, L;
   int groups, nwg;
   int cluster0;      // 0: one launch holds them all
+  int diagonal;      // the launch runs step diagonal - l of layer l; -1: all steps
   int wait, pause;
   uint32_t* status;
 };
@@ -954,6 +955,8 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_stack_fwd(SeqStack p) {
   const bool upper = layer > 0;
   float* const HP = q.HP;
   const int H = p.H, B = p.B, GH = G * H, T = p.T;
+  const int first = p.diagonal < 0 ? 0 : p.diagonal - layer, end = p.diagonal < 0 ? T : first + 1;
+  if (first < 0 || end > T) return;       // (the whole workgroup)
   const SeqRow row(q.X, H, B, b0), below(upper ? p.d[upper ? layer - 1 : 0].X : q.X, H, B, b0);
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -985,7 +988,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_stack_fwd(SeqStack p) {
 #pragma unroll
   for (int g = 0; g < G; ++g) x0[g] = 0.f;
   if (cell) {
-    keep = MODE == RNN_LSTM ? q.CP[e] : MODE == RNN_GRU ? HP[e] : 0.f;
+    keep = MODE == RNN_LSTM ? q.CP[first * BH + e] : MODE == RNN_GRU ? HP[first * BH + e] : 0.f;
     in.bRn = MODE == RNN_GRU ? q.bRn[ch] : 0.f;
     if (upper)
 #pragma unroll
@@ -996,7 +999,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_stack_fwd(SeqStack p) {
   int dead = SeqLost(lost).begin(status, h0 == 0);
   const int limit = lost.limit < 0 ? 1 << 22 : lost.limit;
   const bool publish_last = layer + 1 < p.L;      // the layer above reads the last state too
-  for (int sv = 0; sv < T; ++sv) {
+  for (int sv = first; sv < end; ++sv) {
     const int st = __builtin_amdgcn_readfirstlane(sv);
     const __amdgpu_buffer_rsrc_t r = row.rsrc(st), rb = below.rsrc(st + 1);
     uintx4_t v[NC], u[NC];
@@ -1007,7 +1010,7 @@ __global__ void __launch_bounds__(SEQ_THREADS, 2) rnn_stack_fwd(SeqStack p) {
         for (int g = 0; g < G; ++g) x0[g] = q.xp[((size_t)st * B + cb) * GH + (size_t)g * H + ch];
       in.prev = keep;
     }
-    if (st > 0) seq_pause(p.pause);
+    if (st > first) seq_pause(p.pause);
     seq_load(r, row, wave, v);
     floatx4_t acc[2 * RT];               // the recurrent products, the input's
 #pragma unroll
@@ -1563,21 +1566,34 @@ size_t stack_place(const RnnGeom& g) {
   const size_t at = ((size_t)g.T * g.B * g.GH + g.L * g.GH + 63) & ~(size_t)63;
   return at + g.L * (g.T + 1) * seq_row(g, g.H) <= workspace_core(g) - 4 ? at : 0;
 }
+// All steps in one cooperative launch, or, on a stream that is being captured, a launch for each diagonal of layers and steps: what a step waits for is
+// there when it starts, so that such a launch needs none of the others, and the same kernel gives the same bits.  In a graph, forward, us, a launch per
+// layer and step with the products between layers apart / these: LSTM of 320 units, 3 layers, 5 columns, over 25 steps 398 / 158, over 100 steps 1556 / 564; of
+// 512 units, 2 layers, 16 columns over 50 steps 576 / 342; of 256 units, 4 layers, 64 columns over 20 steps 642 / 228; of 768 units, 2 layers, 16 columns over 30
+// steps 494 / 398; GRU of 384 units, 2 layers, 64 columns over 40 steps 800 / 424; tanh of 1020 units, 2 layers, 5 columns over 30 steps 1172 / 266.  LSTM of 1024
+// units, 2 layers, fetches 48 MB of matrices a launch: 16 columns over 4 steps 96 / 95, but 3 columns over 30 steps 433 / 493.
+int stack_launch(void (*kernel)(SeqStack), SeqStack& p, int clusters, size_t lds, bool captured, hipStream_t s) {
+  p.diagonal = -1;
+  if (!captured) return seq_launch(kernel, p, clusters, lds, s);
+  if (options().rnn_sequences == Options::SEQ_REFUSED || !mfma_allow_lds(reinterpret_cast<const void*>(kernel), lds)) return FLHIP_DECLINED;
+  for (p.diagonal = 0; p.diagonal < p.T + p.L - 1; ++p.diagonal) hipLaunchKernelGGL(kernel, dim3((unsigned)(clusters * p.nwg)), dim3(SEQ_THREADS), lds, s, p);
+  return FLHIP_OK;
+}
 template <int MODE, int HU>
-int stack_fwd_hu(const RnnGeom& g, SeqStack& p, hipStream_t s) {
+int stack_fwd_hu(const RnnGeom& g, SeqStack& p, bool captured, hipStream_t s) {
   constexpr int RT = (gates_of(MODE) * HU + 15) / 16;
   p.nwg = (g.H + HU - 1) / HU;
   const size_t lds = stack_lds(MODE, RT);
   const int nc = ((g.H + 15) / 16 + SEQ_WAVES - 1) / SEQ_WAVES, clusters = g.L * p.groups;
-  if (nc <= 2) return seq_launch(rnn_stack_fwd<MODE, HU, 2>, p, clusters, lds, s);
-  if (nc <= 4) return seq_launch(rnn_stack_fwd<MODE, HU, 4>, p, clusters, lds, s);
-  if constexpr (RT <= 2) return seq_launch(rnn_stack_fwd<MODE, HU, 8>, p, clusters, lds, s);
+  if (nc <= 2) return stack_launch(rnn_stack_fwd<MODE, HU, 2>, p, clusters, lds, captured, s);
+  if (nc <= 4) return stack_launch(rnn_stack_fwd<MODE, HU, 4>, p, clusters, lds, captured, s);
+  if constexpr (RT <= 2) return stack_launch(rnn_stack_fwd<MODE, HU, 8>, p, clusters, lds, captured, s);
   return FLHIP_DECLINED;
 }
 // all layers of a stack; FLHIP_DECLINED: not run
 template <int MODE>
 int forward_stack(const RnnGeom& g, const float* x, const float* w, const float* hx, const float* cx, float* y, float* hy, float* cy,
-                  float* res, float* ws, hipStream_t s) {
+                  float* res, float* ws, bool captured, hipStream_t s) {
   const int units = stack_units(g);
   const size_t place = stack_place(g), TB = (size_t)g.T * g.B, act = TB * g.H;
   if (!units || !place) return FLHIP_DECLINED;
@@ -1602,11 +1618,11 @@ int forward_stack(const RnnGeom& g, const float* x, const float* w, const float*
   if (const int rc = mm(w + offsets(g, 0).W, x, ws, g.GH, TB, g.I, 1, 0, ip.d[0].bsum, s, scratch_of(g, ws), false)) return rc;
   int rc = FLHIP_DECLINED;
   if constexpr (MODE == RNN_LSTM || MODE == RNN_GRU) {
-    if (units == 4) rc = stack_fwd_hu<MODE, 4>(g, p, s);
-    else if (units == 8) rc = stack_fwd_hu<MODE, 8>(g, p, s);
-    else rc = stack_fwd_hu<MODE, 16>(g, p, s);
+    if (units == 4) rc = stack_fwd_hu<MODE, 4>(g, p, captured, s);
+    else if (units == 8) rc = stack_fwd_hu<MODE, 8>(g, p, captured, s);
+    else rc = stack_fwd_hu<MODE, 16>(g, p, captured, s);
   } else if constexpr (MODE == RNN_TANH) {
-    rc = stack_fwd_hu<MODE, 16>(g, p, s);
+    rc = stack_fwd_hu<MODE, 16>(g, p, captured, s);
   }
   return rc == FLHIP_OK ? check_launch("rnn_fwd") : rc;
 }
@@ -1956,10 +1972,11 @@ extern "C" int flhip_rnn_fwd(const flhip_rnn_desc* d, const void* x, const void*
   float* res = static_cast<float*>(reserve);
   const float* wf = static_cast<const float*>(w);
   const size_t act = (size_t)g.T * g.B * g.D * g.H;
-  if (stack_units(g) && seq_uncaptured(s)) {
+  if (stack_units(g)) {
+    const bool captured = !seq_uncaptured(s);
     auto stack = [&](auto fn) {
       return fn(g, static_cast<const float*>(x), wf, static_cast<const float*>(hx), static_cast<const float*>(cx), static_cast<float*>(y),
-                static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), s);
+                static_cast<float*>(hy), static_cast<float*>(cy), res, static_cast<float*>(ws), captured, s);
     };
     const int rc = g.mode == RNN_TANH ? stack(forward_stack<RNN_TANH>) : g.mode == RNN_LSTM ? stack(forward_stack<RNN_LSTM>) : stack(forward_stack<RNN_GRU>);
     if (rc != FLHIP_DECLINED) return rc;

@@ -228,6 +228,40 @@ def test_stacked_layers_in_one_launch(mode, I, H, L, T, B, states, launches):
         assert rel_l2(a[ok], b[ok]) <= 1e-5
 
 
+@pytest.mark.parametrize("mode,I,H,L,T,B", [
+    (flref.RNN_LSTM, 9, 320, 3, 5, 5), (flref.RNN_LSTM, 33, 516, 2, 4, 3), (flref.RNN_LSTM, 8, 256, 4, 1, 64), (flref.RNN_LSTM, 8, 1024, 2, 3, 16),
+    (flref.RNN_GRU, 6, 384, 2, 3, 70), (flref.RNN_GRU, 12, 48, 3, 7, 17), (flref.RNN_TANH, 8, 1020, 2, 3, 5), (flref.RNN_LSTM, 3, 16, 2, 9, 1)])
+def test_stacked_layers_captured_and_eager(mode, I, H, L, T, B):
+    """A launch for each diagonal of layers and steps in a graph, one launch for all without: the same bits, in what the forward pass keeps too, in every replay."""
+    count = capi.lib().flhip_rnn_sequence_launches
+    gen = torch.Generator(device="cuda").manual_seed(H + T)
+    x, dy = torch.empty(T, B, I, device="cuda"), torch.randn(T, B, H, generator=gen, device="cuda")
+    w = torch.randn(ops.rnn_param_count(I, H, L, mode, False), generator=gen, device="cuda") / H ** 0.5
+    hx = torch.rand(L, B, H, generator=gen, device="cuda")
+    cx = torch.randn(L, B, H, generator=gen, device="cuda") if mode == flref.RNN_LSTM else None
+    run = lambda: ops.rnn(x, hx, cx, w, H, L, mode, False)
+    keep = lambda out: [t.clone() for t in out[:3] if t is not None] + [t for t in ops.rnn_backward(x, w, out[3], H, L, mode, False, dy) if t is not None]
+    x.zero_()
+    run()
+    torch.cuda.synchronize()
+    before = count()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static = run()
+    assert count() == before
+    for _ in range(3):
+        x.copy_(torch.randn(T, B, I, generator=gen, device="cuda"))
+        before = count()
+        want = keep(run())
+        assert count() > before
+        for t in static:
+            if t is not None:
+                t.zero_()
+        graph.replay()
+        for a, b in zip(keep(static), want):
+            assert torch.equal(a, b) and bool(b.isfinite().all())
+
+
 def test_a_wait_of_stacked_layers_that_gives_up_ends_in_not_a_number():
     T, B, I, H, L = 5, 20, 8, 64, 3
     gen = torch.Generator(device="cuda").manual_seed(5)
