@@ -270,8 +270,8 @@ int big16_go(const BigParams& p, const void* src, const void* w, const float* bi
 // ---- both operands contiguous along the contraction: out[m][c] = sum_k a[m][k] b[c][k] (+ bias[c]) ------------------------------
 // A tile is 256 rows of a x 128 of b, a stage 64 contraction indexes (whole cache lines of a row), a ring of 3.
 // LDS [row][8 cells of 8 k], 128 bytes a row; cell c of row r lies at c ^ (r & 7), so that the rows of a fragment read spread over
-// the banks.  A row's last cell ends at its last element and so repeats up to 7 of the cell before it: in a's tile those become
-// zeros, written by the lanes that loaded them between the wait for their loads and the barrier.
+// the banks.  A row's last cell ends at its last element and so repeats up to 7 of the cell before it: in both tiles those become
+// zeros (an infinity must meet no zero of the other tile), written by the lanes that loaded them between the wait for their loads and the barrier.
 struct BigNtParams {
   int M, C, K, Kcells;
   int nstages, mtiles, ctiles, panel, dup;
@@ -312,11 +312,11 @@ big16_nt_kernel(BigNtParams p, const E* __restrict__ a, const E* __restrict__ b,
     for (int k = 0; k < INSTR; ++k)
       pd_load_lds(k < AI ? ars : brs, base + k * 8192, rowoff[k] == BG_OOB || cell >= p.Kcells ? BG_OOB : rowoff[k] + col, 0);
   };
-  // zeros over what the last cell of this lane's rows of a repeats (its loads have landed)
+  // zeros over what the last cell of this lane's rows repeats (its loads have landed)
   auto fix_tail = [&](int t, int slot) __attribute__((always_inline)) {
     if (p.dup && t == nst - 1 && 8 * t + lcell == p.Kcells - 1) {
 #pragma unroll
-      for (int k = 0; k < AI; ++k) {
+      for (int k = 0; k < INSTR; ++k) {
         uint16_t* const q = reinterpret_cast<uint16_t*>(ring + slot * BN_STAGE + (wave + 8 * k) * 1024 + lane * 16);
         for (int e = 0; e < p.dup; ++e) q[e] = 0;
       }

@@ -511,7 +511,8 @@ int launch_pwd16(const ConvGeom& g, const void* src, const void* w, const float*
 // Planes that are not a multiple of 8 positions: the last cell of a plane ends at its last
 // position and repeats up to 7 positions of the cell before it; in the dy tile those repeated
 // positions are overwritten with zeros (by the lanes that loaded them, between the wait for
-// their loads and the barrier), so every product is counted once.
+// their loads and the barrier), so every product is counted once.  Matrix products, which have one such cell, write
+// them to the x tile too: an infinity there meets no zero (over planes, a cell in seven, that took 3 of the 412 us of a strided block over 7 x 7).
 // Partial tiles go to the workspace and are added in a fixed order by the reduce kernel the other
 // filter-gradient kernels use.  No bias gradient (layers with one take the kernels with register
 // staging, which sum it from the loader's registers).
@@ -527,6 +528,7 @@ struct PwdWgradParams {
   int ctiles, mtiles;
   int E;
   int dup;                            // positions the last cell of a plane repeats (0: planes of 8k positions)
+  int xfix;                           // those of x become zeros too
   unsigned x_bytes, dy_bytes;
 };
 
@@ -588,13 +590,14 @@ pwd16_wgrad_kernel(PwdWgradParams p, const E* __restrict__ x, const E* __restric
       img += 1;
     }
   };
-  // zeros over the repeated positions of the dy cells this lane loaded into ring slot `slot` (its four dy loads
+  // zeros over the repeated positions of the cells this lane loaded into ring slot `slot` (its eight loads
   // have landed): the first p.dup positions of the cell
   auto fix_tail = [&](int slot) {
     if (tailq & (1u << slot)) {
       char* cellp = reinterpret_cast<char*>(ring + slot * PWG_STAGE) + lane * 16;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < 8; ++k) {
+        if (k >= 4 && !p.xfix) break;
         char* q = cellp + (wave + 4 * k) * 1024;
         int d = p.dup, at = 0;
         if (d >= 4) {
@@ -834,6 +837,7 @@ bool gemm16_nt_plan(int M, int N, int K, PwdWgradParams* p) {
   p->C = M; p->Mo = N; p->P = K; p->N = 1;
   p->Pc = (K + 7) / 8;
   p->dup = (8 - K % 8) % 8;
+  p->xfix = 1;
   const long long xb = (long long)M * K * 2, db = (long long)N * K * 2;
   if (xb >= (1ll << 31) || db >= (1ll << 31)) return false;
   p->x_bytes = (unsigned)xb;

@@ -469,6 +469,34 @@ def test_matmul_in_16_bit_storage_of_an_odd_number_of_elements(M, N, K, dtype):
     assert abs(float(out[-1, -1]) - (256.0 - 256.0 + 4096.0)) <= 2 * unit * 4096 + 5 * K ** 0.5
 
 
+@pytest.mark.parametrize("M,N,K", [(1024, 64, 10), (129, 127, 67), (256, 129, 9998), (200, 1, 9), (3081, 2565, 127)])   # thin; odd rows; slices; one column; large tiles
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_matmul_in_16_bit_storage_of_what_is_not_finite_at_a_rows_end(M, N, K, dtype):
+    """A^T B whose rows are no whole cells of 8: what the last cell repeats of the one before it counts for nothing, infinities too."""
+    import ctypes as C
+    from flashlight_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A, B = torch.randn(M, K, generator=g, device="cuda").to(dtype), torch.randn(N, K, generator=g, device="cuda").to(dtype)
+    inf, nan = float("inf"), float("nan")
+    want = torch.zeros(N, M, dtype=torch.float64, device="cuda")
+    at = [(A, 1, K - 1, inf), (A, M // 2, K - 6, -inf), (A, M - 1, K - 3, nan), (B, 0, K - 7, -inf), (B, N - 1, K - 2, inf)]
+    for t, r, k, v in at:
+        t[r, k] = v
+    for t, r, k, v in at:                   # (each in a column of its own, so that what it meets is finite)
+        if t is A:
+            want[:, r] += v * B[:, k].double()
+        else:
+            want[r] += v * A[:, k].double()
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    need = capi.lib().flhip_matmul_slices_bytes(M, N, K, 1, 0, code)
+    ws, out = torch.empty(max(need, 4), dtype=torch.uint8, device="cuda"), torch.zeros(N, M, device="cuda", dtype=dtype)
+    P = lambda t: C.c_void_p(t.data_ptr())
+    capi.check(capi.lib().flhip_matmul_ws(P(A), P(B), P(out), M, N, K, 1, 0, None, code, P(ws) if need else None, need,
+                                          C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    for f in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(f(out), f(want))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_matmul_in_16_bit_storage_at_the_size_of_a_speech_model(dtype):
     """2000 x 2000 weights against 4000 frames, the three products of a layer's step; checked against numpy's
