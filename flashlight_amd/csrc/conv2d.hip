@@ -202,7 +202,8 @@ static bool thin_on(const ConvGeom& g, int dtype, bool bwd, bool first) {
 // images 22 / 28, 23 / 32, 26 / 31, over 14 x 14, 1 / 20 / 48 23 / 29, 46 / 63, 61 / 122; 384 channels over 14 x 14, 4 / 26 / 40 27 / 38, 45 / 50, 56 / 48, over 7 x
 // 7, 16 26 / 39; 256 channels over 14 x 14, 4 images (thin) 19.5 / 17.9, 12 / 33 / 48 / 64 22 / 32, 26 / 34, 30 / 33, 36 / 34, over 16 x 16, 8 / 33 / 40 / 48 21 /
 // 24, 31 / 33, 32 / 32, 36 / 32; 224 channels over 14 x 14, 26 / 40 images 24 / 25, 30 / 28; 128 channels over 28 x 28, 4 / 33 images 17 / 18, 29 / 22.
-// Planes of at most 64 positions with 2048 positions and more: 256 channels over 7 x 7, 64 images 20 / 26.  TAP2D_ALL lifts the rules.
+// Planes of at most 64 positions with 2048 positions and more: 256 channels over 7 x 7, 64 images 20 / 26.  Layers of 257 to 383 channels
+// stay off them: the kernels are compiled for 256 and 512, so that 272 channels cost what 512 do.  TAP2D_ALL lifts the rules.
 static bool tap2d_on(const ConvGeom& g, int dtype, bool bwd) {
   if (!tap1d_on(dtype) || skip(Options::SKIP_TAP2D)) return false;
   if (options().tap2d_all) return true;

@@ -10,7 +10,8 @@
 // stages that read them.  The shifted fragments of kw = 0 and 2 are made from the aligned one and the words beside it.
 //
 // What bounds it is the bf16 matrix pipe (18 instructions per wave and 16 positions, 21 LDS reads and 60 vector instructions beside them).
-// The partial tiles go to the workspace as [slice][tile][tap][64][64] and are added in the order of the slices.
+// The partial tiles go to the workspace as [slice][tile][tap][64][64] and are added in a fixed order: that of the slices up to eight of them, else
+// interleaved runs of slices, and those in pairs.
 // Measured, us, both launches (before: wgrad_slab_kernel on v_mfma_f32_16x16x4_f32): 64 channels over 56 x 56, 32 / 64 images 71 / 131 -> 61 / 100, 128 over
 // 28 x 28 81 / 147 -> 61 / 99, 256 over 14 x 14 97 / 177 -> 56 / 95, 512 over 7 x 7 108 / 208 -> 59 / 103.  Its products and LDS reads alone, 64
 // channels over 56 x 56, take 31 us per 32 images, all of it 37: with every wave bringing in rows behind the last product of a stage it was 47.
@@ -217,7 +218,10 @@ wgrad3_split_kernel(W3Params p, const float* __restrict__ x, const float* __rest
       big[t][r] += small[t][r];
       bad |= split_redo(big[t][r]);
     }
-  if (__builtin_amdgcn_ballot_w64(bad)) {          // once more with the operands as they are
+  // Once more with the operands as they are, loaded element by element.  Both launches, us, plain / one infinity in every tile of one image / of every image / all
+  // results below 2^-90: 256 channels over 14 x 14, 64 images 109 / 419 / 439 / 455, 64 over 56 x 56, 32 images 66 / 335 / 334 / 344, 512 over 7 x 7, 64 images
+  // 104 / 355 / 358 / 357.
+  if (__builtin_amdgcn_ballot_w64(bad)) {
     const int k = kt * W3_T + fb * 32 + fr, c = ct * W3_T + cb * 32 + fr;
 #pragma unroll
     for (int t = 0; t < 3; ++t)
@@ -293,7 +297,7 @@ size_t w3_lds_bytes(const W3Params& p, int R) { return (size_t)16 * 3 * W3_T * (
 
 bool wgrad3_plan(const ConvGeom& g, W3Params* p, int* R, int* slices) {
   if (!(g.KH == 3 && g.KW == 3 && g.sy == 1 && g.sx == 1 && g.py == 1 && g.px == 1 && g.dly == 1 && g.dlx == 1 && g.groups == 1)) return false;
-  if (g.H < 4 || g.W < 4 || g.W > 64 || g.C < 32 || g.K < 32) return false;
+  if (g.H < 4 || g.W < 4 || g.W > 56 || g.C < 32 || g.K < 32) return false;      // (rows of eight cells, with their pitches of 11 and 9, need 186 KB of LDS)
   const long long xb = (long long)g.N * g.C * g.H * g.W * 4, db = (long long)g.N * g.K * g.H * g.W * 4;
   if (xb >= (1ll << 31) || db >= (1ll << 31)) return false;
   p->C = g.C; p->H = g.H; p->W = g.W; p->K = g.K;
