@@ -96,13 +96,13 @@ struct Tap1Params {
   int d0[2];             // source offset of tap 0 of a phase, relative to the slab's first position
   int smin;              // slab's first source position for result 0
   int SR, half;          // slab rows; stride 2: row of the first odd source offset
-  int zcells;            // cells of zeros behind them, for the taps that do not exist (0: there are none)
   int taps_total;        // ntaps[0] + ntaps[1]
   int ptiles, mtiles;
   unsigned src_bytes, w_bytes, dst_bytes;
   // two-dimensional windows over stacked planes (tap2d_*): taps per window row, slab rows per window row = the
   // pitch of a plane's row, and the plane's geometry for the results
   int tw, tpitch, pW, pH, pN;
+  int zcells;            // cells of zeros behind the slab's rows, for the taps that do not exist (0: there are none)
 };
 
 // ---- operand passes ------------------------------------------------------------------------
@@ -285,7 +285,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
   {
     const intx4_t xrs = pd_rsrc(xr, p.src_bytes);
     const unsigned base = pd_lds_addr(t1_slab);
-    const int ncell = p.SR * CPR + p.zcells, ninstr = (ncell + 63) >> 6;
+    const int ncell = p.SR * CPR + (DT > 1 ? p.zcells : 0), ninstr = (ncell + 63) >> 6;
     const float inv = 1.0f / (float)CPR;
     for (int ii = wave; ii < ninstr; ii += 4) {
       const int L = ii * 64 + lane;
@@ -320,9 +320,9 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
       for (int r = 0; r < 16; ++r) acc[q][b][r] = 0.f;
 
   const int fr = lane & 31, fg = lane >> 5;
-  int ap[NB];                                   // this lane's cell of a tap's first row
+  lds_cell_t ap[NB];                            // this lane's cell of a tap's first row
 #pragma unroll
-  for (int b = 0; b < NB; ++b) ap[b] = ((wp * NB + b) * 32 + fr) * CPR + fg;
+  for (int b = 0; b < NB; ++b) ap[b] = (lds_cell_t)t1_slab + (((wp * NB + b) * 32 + fr) * CPR + fg);
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the slab (and the first weight fragments) have landed
   __syncthreads();
@@ -343,7 +343,7 @@ tap_conv_body(const Tap1Params& p, const T* __restrict__ xr, const uintx4_t* __r
       return trow * CPR;
     };
     auto rows = [&](int b, int off) __attribute__((always_inline)) {
-      return (lds_cell_t)t1_slab + ((DT > 1 && off == p.SR * CPR ? 0 : ap[b]) + off);
+      return (DT > 1 && off == p.SR * CPR ? (lds_cell_t)t1_slab : ap[b]) + off;
     };
     uintx4_t af[4][NB];
     int tcur[DT];
