@@ -1867,3 +1867,28 @@ def test_16_bit_windows_of_what_is_not_finite(xs, k, kh, kw, stride, dtype):
         ok = want.isfinite()
         unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)                  # (one rounding per result, beside fp32 sums)
         assert bool((~ok).any()) and float(((got.double().cpu() - want)[ok] / want[ok]).abs().max()) <= unit
+
+
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("xs,K", [((3, 72, 8, 16), 64), ((5, 64, 12, 12), 136), ((2, 64, 6, 6), 64), ((3, 64, 7, 8), 64), ((4, 128, 56, 56), 128)])      # pieces of 4 and 2, elements
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_strided_16_bit_layers_of_what_is_not_finite(xs, K, k, dtype):
+    """The copies around strided layers, which gather taps, spread them and add what they overlap in: an infinity reaches the results that it reaches, as one."""
+    g = torch.Generator(device="cuda").manual_seed(xs[1] + k)
+    x = (torch.rand(xs, generator=g, device="cuda") + 0.5).to(dtype)
+    w = (torch.rand(K, xs[1], k, k, generator=g, device="cuda") / 64 + 1 / 128).to(dtype)
+    geo = dict(sx=2, sy=2, px=k // 2, py=k // 2)
+    x[0, 3, 2, 2], x[1, xs[1] - 1, 4, 3 if k == 3 else 4], x[0, 5, 0, 0] = float("inf"), float("-inf"), float("nan")
+    y = fa.conv2d(x, w, None, **geo)
+    dy = (torch.rand(y.shape, generator=g, device="cuda") + 0.5).to(dtype)
+    dy[0, 2, 1, 2], dy[1, K - 1, y.shape[2] - 2, 1], dy[1, 7, 1, y.shape[3] - 2] = float("-inf"), float("inf"), float("nan")
+    dx = fa.conv2d_backward_data(dy, xs, w, **geo)
+    xd, wd, d = x.double().cpu(), w.double().cpu(), dy.double().cpu()
+    ry, rdx = torch.zeros(y.shape, dtype=torch.float64), torch.zeros(xs, dtype=torch.float64)
+    for i, j, o, q in _taps(xs, w.shape, 2) if k == 3 else [(0, 0, slice(None), (slice(None), slice(None), slice(0, None, 2), slice(0, None, 2)))]:
+        at, to = xd[q].transpose(0, 1), d[o].transpose(0, 1)
+        ry[o] += (wd[:, :, i, j] @ at.reshape(xs[1], -1)).reshape(K, *at.shape[1:]).transpose(0, 1)
+        rdx[q] += (wd[:, :, i, j].t() @ to.reshape(K, -1)).reshape(xs[1], *to.shape[1:]).transpose(0, 1)
+    for got, want in ((y, ry), (dx, rdx)):
+        assert bool(want.isinf().any()) and bool(want.isnan().any())
+        assert torch.equal(_classes(got), _classes(want))
