@@ -1570,8 +1570,10 @@ size_t stack_place(const RnnGeom& g) {
 // there when it starts, so that such a launch needs none of the others, and the same kernel gives the same bits.  In a graph, forward, us, a launch per
 // layer and step with the products between layers apart / these: LSTM of 320 units, 3 layers, 5 columns, over 25 steps 398 / 158, over 100 steps 1556 / 564; of
 // 512 units, 2 layers, 16 columns over 50 steps 576 / 342; of 256 units, 4 layers, 64 columns over 20 steps 642 / 228; of 768 units, 2 layers, 16 columns over 30
-// steps 494 / 398; GRU of 384 units, 2 layers, 64 columns over 40 steps 800 / 424; tanh of 1020 units, 2 layers, 5 columns over 30 steps 1172 / 266.  LSTM of 1024
-// units, 2 layers, fetches 48 MB of matrices a launch: 16 columns over 4 steps 96 / 95, but 3 columns over 30 steps 433 / 493.
+// steps 494 / 398; GRU of 384 units, 2 layers, 64 columns over 40 steps 800 / 424; tanh of 1020 units, 2 layers, 5 columns over 30 steps 1172 / 266.  What bounds
+// large ones is the matrices, fetched in every launch, the input's too: level at 896 units (LSTM, 2 layers, 3 columns over 30 steps 429 / 412, GRU 395 / 386), and the
+// slower ones at 1024 over few columns (48 MB a launch: LSTM, 2 layers over 30 steps, 1 / 8 / 16 columns 414 / 483, 477 / 501, 516 / 524, GRU 1 / 16 columns 378 / 427, 493 /
+// 469).  (With the states asked for before the matrices, and the input product while the recurrent matrix is on its way, nothing.)
 int stack_launch(void (*kernel)(SeqStack), SeqStack& p, int clusters, size_t lds, bool captured, hipStream_t s) {
   p.diagonal = -1;
   if (!captured) return seq_launch(kernel, p, clusters, lds, s);
